@@ -5,9 +5,8 @@
 // Packed layout: [N/16][K/32][quad 0..3][row 0..15][8 elements]; lane (row + 16 * quad) of a wave reads its
 // 16 bytes of piece (n_tile, k_step) at byte offset lane * 16: the A operand of v_mfma_f32_16x16x32_bf16.
 // The product is computed transposed (C^T = W . A^T): the activations are the B operand, 16 rows per tile.
-// A workgroup owns NT tiles of W; its waves (1 to 16, more when W has few rows, so that the GPU is filled)
-// take the k steps in turn and their sums are added in wave order through LDS: the result is the same in
-// every run and does not depend on the other rows of A.
+// A workgroup owns NT tiles of W; its waves (1 to 16, see skinny_waves) take a run of the k steps each and their sums
+// are added in wave order through LDS: the result is the same in every run and does not depend on the other rows of A.
 #include "cache_layout.h"
 #include "common.h"
 #include "microllm_hip.h"
@@ -19,12 +18,26 @@ typedef float floatx4 __attribute__((ext_vector_type(4)));
 typedef unsigned int uintx4 __attribute__((ext_vector_type(4)));
 
 
-constexpr int kChunk = 8;   // k steps a wave takes in a row
+constexpr int kBufferFlags = 0x00027000;   // a raw buffer of 32-bit words
+constexpr int kNonTemporal = 2;
+constexpr int kChunk = 4;     // k steps a wave takes in a row, then skips what the other waves take
 
 union Piece {
     bf16x8 v;
     uintx4 raw;
 };
+
+// The value of the lane ROWS * steps places further on within every 16 lanes, wrapping round.
+template <int ROWS>
+__device__ inline unsigned turn_lanes(unsigned value, int steps) {
+    const int v = static_cast<int>(value);
+    switch (steps) {        // a constant after unrolling; 0x120 + r: row_ror by r lanes
+        case 1: return static_cast<unsigned>(__builtin_amdgcn_update_dpp(0, v, 0x120 + 16 - ROWS, 0xf, 0xf, false));
+        case 2: return static_cast<unsigned>(__builtin_amdgcn_update_dpp(0, v, 0x120 + (2 * ROWS < 16 ? 16 - 2 * ROWS : 1), 0xf, 0xf, false));
+        case 3: return static_cast<unsigned>(__builtin_amdgcn_update_dpp(0, v, 0x120 + (3 * ROWS < 16 ? 16 - 3 * ROWS : 1), 0xf, 0xf, false));
+        default: return value;
+    }
+}
 
 // EPILOGUE: 0 = float32 [M, N]; 1 = bfloat16 [M, N]; 2 = bfloat16 [M, N / 2] = silu(even rows of W) * (odd rows).
 // 3 = the q/k/v projection of an attention layer finished in place: bias, rotation of the position, queries to
@@ -38,27 +51,145 @@ union Piece {
 // W is read past the caches (non-temporal loads): a step reads every weight once, and all of them together are far
 // more than the caches hold. Measured on MI355X inside the decode step, against ordinary loads for weights under 64 MB:
 // 7B sizes +1 % at batch 8, +1.6 % at batch 1, +0.7 % at batch 64; 0.5B sizes +4 % at batch 1, the same otherwise.
-template <int MT, int NT, int EPILOGUE, bool SCALED, bool PAIRED>
+// HALF: a workgroup owns 8 rows of W instead of 16 (half a tile), for weights whose tiles alone would leave compute
+// units idle: a wave's A operand holds the 8 rows at one k step in its first 8 rows and at the next step in its last 8,
+// and the B operand 8 rows of the activations at the first step and again at the next, so that the product's upper left
+// 8 x 8 is the even step's and its lower right 8 x 8 the odd step's; the other two quarters are read by nobody. MT counts
+// 8 rows of the activations then. SPLIT (more than 16 rows): the same sums in the same order with whole tiles.
+template <int MT, int NT, int EPILOGUE, bool SCALED, int GROUP, int HALF, bool SPLIT>
 __global__ __launch_bounds__(1024) void gemm_skinny_kernel(
     const bf16* __restrict__ a, const bf16* __restrict__ w_packed, void* __restrict__ out,
     int m, int n, int k, int n_tiles, int k_steps, MllSkinnyExtras extras) {
     extern __shared__ float reduce_shared[];
     const MllQkvStore& store = extras.store;   // [waves][NT * MT][64 lanes][4]
     const int lane = threadIdx.x % kWave;
-    const int wave = threadIdx.x / kWave;
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave);
     const int waves = blockDim.x / kWave;
     const int col = lane % 16, quad = lane / 16;
-    const int tile0 = blockIdx.x * NT;
+    constexpr int TILE = HALF ? 8 : 16;         // columns of the result a tile has, and rows of A a group of MT
+    const int tile0 = blockIdx.x * NT;          // in halves of tiles with HALF, as is n_tiles
+    const int token = HALF ? col % 8 : col;     // the row of A (of 8 or 16) that the lane's accumulators belong to
+    const bool mine = !HALF || (col < 8 && quad < 2);       // whether they are results
 
-    floatx4 acc[NT][MT];
+    constexpr int SETS = SPLIT ? 2 : 1;         // sums of even and of odd steps apart
+    floatx4 sums[SETS][NT][MT];
 #pragma unroll
-    for (int nt = 0; nt < NT; ++nt)
+    for (int set = 0; set < SETS; ++set)
 #pragma unroll
-        for (int mt = 0; mt < MT; ++mt) acc[nt][mt] = floatx4{0.0f, 0.0f, 0.0f, 0.0f};
+        for (int nt = 0; nt < NT; ++nt)
+#pragma unroll
+            for (int mt = 0; mt < MT; ++mt) sums[set][nt][mt] = floatx4{0.0f, 0.0f, 0.0f, 0.0f};
 
-    // What the epilogue reads beside the product is asked for here, before the streaming begins, so that these
-    // loads are not waited for at the end. The sums of squares for the rows' factors (SCALED) go straight from
-    // memory into LDS, behind the waves' slots: [m][stride] as it lies in memory, 1 KB per wave-wide load.
+    // The waves take runs of kChunk k steps in turn, so that a workgroup reads one stretch of W at a time. Operands come
+    // through buffer descriptors, whose loads give zeros past the end of what they describe: no branch stands between two
+    // loads, so the compiler counts those in flight instead of waiting for all of them. A wave keeps two blocks of loads
+    // on their way; with few steps a wave everything is asked for at once, before the epilogue's own loads.
+    constexpr int kPast = 0x7ffffff0, kPastRow = 0x40000000;       // offsets past the end of every descriptor here
+    constexpr int DEPTH = HALF ? HALF * kChunk / 2 : (MT + NT <= 3) ? 4 : 2;       // loads of W a tile and block
+    __amdgpu_buffer_rsrc_t w_rsrc[NT];
+#pragma unroll
+    for (int nt = 0; nt < NT; ++nt) {
+        const bool live = tile0 + nt < n_tiles;
+        const int whole = (live ? tile0 + nt : tile0) / (HALF ? 2 : 1);
+        w_rsrc[nt] = __builtin_amdgcn_make_buffer_rsrc(const_cast<bf16*>(w_packed) + static_cast<int64_t>(whole) * k_steps * 512, 0,
+                                                       live ? k_steps * 1024 : 0, kBufferFlags);
+    }
+    const __amdgpu_buffer_rsrc_t a_rsrc = __builtin_amdgcn_make_buffer_rsrc(const_cast<bf16*>(a), 0, m * k * 2, kBufferFlags);
+    // Whole tiles and one group of rows: an A load brings GROUP steps of 16 / GROUP rows instead of one step of 16 (rows
+    // of which most may be none): lane `col` of 16 reads row col % (16 / GROUP) at step col / (16 / GROUP) of the group. Step u's
+    // operand is the loaded one turned by u * 16 / GROUP lanes; what then lies in the columns past the rows belongs to
+    // other steps and goes into columns of the product that nobody reads. GROUP 1 (9 to 16 rows): two steps are read at a
+    // time: lanes 0..7 of every 16 read rows 0..7 (then 8..15) at one step and lanes 8..15 the same rows at the next, so
+    // that a load touches whole 128-byte lines of 8 rows instead of half lines of 16; lanes 8 apart then exchange what the
+    // other needs. With HALF that same load is the operand as it is.
+    constexpr bool PAIRED = MT == 1 && GROUP == 1 && !HALF;
+    constexpr int GROUP_ROWS = HALF ? 8 : 16 / GROUP;
+    const bool upper = col >= 8;
+    // Where a lane reads W and A at step 0; for a row that is none, past the end (and with every step's offset added to it).
+    const int w_at = HALF ? (col / 8) * 1024 + quad * 256 + (tile0 % 2) * 128 + (col % 8) * 16 : lane * 16;
+    int a_at[MT == 1 ? 2 : MT];
+    if constexpr (HALF) {
+#pragma unroll
+        for (int mt = 0; mt < MT; ++mt) a_at[mt] = mt * 8 + token < m ? (mt * 8 + token) * k * 2 + (col / 8) * 64 + quad * 16 : kPastRow;
+    } else if constexpr (GROUP > 1) {
+        const int row = col % GROUP_ROWS;
+        a_at[0] = row < m ? row * k * 2 + (col / GROUP_ROWS) * 64 + quad * 16 : kPastRow;
+    } else if constexpr (PAIRED) {
+#pragma unroll
+        for (int half = 0; half < 2; ++half) {
+            const int row = (col & 7) + 8 * half;
+            a_at[half] = row < m ? row * k * 2 + (upper ? 64 : 0) + quad * 16 : kPastRow;
+        }
+    } else {
+#pragma unroll
+        for (int mt = 0; mt < MT; ++mt) a_at[mt] = mt * 16 + col < m ? (mt * 16 + col) * k * 2 + quad * 16 : kPastRow;
+    }
+    const int k_left = k - quad * 8 - (HALF || GROUP > 1 ? col / GROUP_ROWS : (PAIRED && upper)) * 32;     // a lane reads A at steps below this many elements
+
+    auto load = [&](int block, Piece (&w_piece)[DEPTH][NT], Piece (&a_piece)[DEPTH][MT]) {
+#pragma unroll
+        for (int u = 0; u < DEPTH; ++u) {
+            const int run = HALF ? block * HALF + u / (kChunk / 2) : block * DEPTH / kChunk;     // the wave's run of steps, and the step in it
+            const int within = HALF ? u % (kChunk / 2) * 2 : block * DEPTH % kChunk + u;
+            const int step = (run * waves + wave) * kChunk + within;
+#pragma unroll
+            for (int nt = 0; nt < NT; ++nt)
+                w_piece[u][nt].raw = __builtin_amdgcn_raw_buffer_load_b128(w_rsrc[nt], w_at + step * 1024, 0, kNonTemporal);
+            if constexpr (GROUP > 1 && !HALF) {
+                if (u % GROUP == 0)
+                    a_piece[u][0].raw = __builtin_amdgcn_raw_buffer_load_b128(a_rsrc, step * 32 < k_left ? a_at[0] + step * 64 : kPast, 0, 0);
+            } else if constexpr (PAIRED) {
+                // a_piece[u] of an even u: rows 0..7 (both steps of the pair); of the odd u after it: rows 8..15
+                const int pair = step - (u & 1);
+                a_piece[u][0].raw = __builtin_amdgcn_raw_buffer_load_b128(a_rsrc, pair * 32 < k_left ? a_at[u & 1] + pair * 64 : kPast, 0, 0);
+            } else {
+#pragma unroll
+                for (int mt = 0; mt < MT; ++mt)
+                    a_piece[u][mt].raw = __builtin_amdgcn_raw_buffer_load_b128(a_rsrc, step * 32 < k_left ? a_at[mt] + step * 64 : kPast, 0, 0);
+            }
+        }
+    };
+    auto multiply = [&](Piece (&w_piece)[DEPTH][NT], Piece (&a_piece)[DEPTH][MT]) {
+        if constexpr (GROUP > 1 && !HALF) {
+#pragma unroll
+            for (int u = 0; u < DEPTH; ++u)
+                if (u % GROUP != 0) {
+                    const uintx4 loaded = a_piece[u - u % GROUP][0].raw;
+#pragma unroll
+                    for (int i = 0; i < 4; ++i) a_piece[u][0].raw[i] = turn_lanes<GROUP_ROWS>(loaded[i], u % GROUP);
+                }
+        } else if constexpr (PAIRED) {
+            // low = rows 0..7 at the pair's first step (lanes 0..7) and its second (lanes 8..15), high = rows
+            // 8..15 likewise. The first step's operand: own low | the partner's high; the second's: the partner's
+            // low | own high.
+#pragma unroll
+            for (int u = 0; u < DEPTH; u += 2) {
+                const uintx4 low = a_piece[u][0].raw, high = a_piece[u + 1][0].raw;
+                uintx4 low_swapped, high_swapped;
+#pragma unroll
+                for (int i = 0; i < 4; ++i) {
+                    low_swapped[i] = turn_lanes<8>(low[i], 1);
+                    high_swapped[i] = turn_lanes<8>(high[i], 1);
+                }
+                a_piece[u][0].raw = upper ? high_swapped : low;
+                a_piece[u + 1][0].raw = upper ? high : low_swapped;
+            }
+        }
+#pragma unroll
+        for (int u = 0; u < DEPTH; ++u)
+#pragma unroll
+            for (int nt = 0; nt < NT; ++nt)
+#pragma unroll
+                for (int mt = 0; mt < MT; ++mt)
+                    sums[u % SETS][nt][mt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(w_piece[u][nt].v, a_piece[u][mt].v, sums[u % SETS][nt][mt], 0, 0, 0);
+    };
+    Piece w_even[DEPTH][NT], w_odd[DEPTH][NT], a_even[DEPTH][MT], a_odd[DEPTH][MT];
+    load(0, w_even, a_even);
+    load(1, w_odd, a_odd);
+
+    // What the epilogue reads beside the product is on its way while the weight streams. The sums of squares for the
+    // rows' factors (SCALED) go straight from memory into LDS, behind the waves' slots: [m][stride] as it lies in
+    // memory, 1 KB per wave-wide load.
     float* factor_shared = reduce_shared + static_cast<size_t>(waves - 1) * NT * MT * kWave * 4;
     if (SCALED && wave == 0) {
         const int count = m * extras.scale.stride;                  // floats; stride is a multiple of 4
@@ -68,152 +199,165 @@ __global__ __launch_bounds__(1024) void gemm_skinny_kernel(
                 __builtin_amdgcn_global_load_lds(extras.scale.sumsq + index, factor_shared + first, 16, 0, 0);
         }
     }
+    // Epilogue 3: the lane's 4 columns lie in one head (head_dim is a multiple of 16). In a query or key head the weight's
+    // rows were ordered so that columns 2p and 2p + 1 hold dims p and p + n_freq: the two that rotate together. Where
+    // every value goes is worked out here too (a null pointer: nowhere), since divisions by run-time sizes take as long
+    // as the sums after them.
     float bias_first[NT][2], bias_second[NT][2];
-    float2 cos_sin[NT][2];
-    int slot = -1;
-    if (EPILOGUE == 3 && wave == 0 && col < m) {
-        if (extras.store.slot_mapping) slot = extras.store.slot_mapping[col];
+    float2 cos_sin[NT][MT][2];
+    bf16* target_first[NT][MT][2];
+    bf16* target_second[NT][MT][2];
+    bool rotates[NT][2];
+    if (EPILOGUE == 3 && wave == 0) {
+        int slot[MT], page[MT], place[MT];
+#pragma unroll
+        for (int mt = 0; mt < MT; ++mt) {
+            const int row = mt * TILE + token;
+            slot[mt] = store.slot_mapping && row < m ? store.slot_mapping[row] : -1;
+        }
 #pragma unroll
         for (int nt = 0; nt < NT; ++nt) {
-            const int column = (tile0 + nt) * 16 + quad * 4;
-            const int head = column / extras.store.head_dim, within = column % extras.store.head_dim;
-            const bool is_value = head >= extras.store.heads + extras.store.kv_heads;
+            const int column = (tile0 + nt) * TILE + quad * 4;
+            const int head = column / store.head_dim, within = column % store.head_dim;
+            const bool is_query = head < store.heads, is_value = head >= store.heads + store.kv_heads;
+            const bool live = mine && column < n;
+            int first[2], second[2];
 #pragma unroll
             for (int half = 0; half < 2; ++half) {
-                const bool rotate = !is_value && within + 2 * half < 2 * extras.store.n_freq;
+                const bool rotate = !is_value && within + 2 * half < 2 * store.n_freq;
+                rotates[nt][half] = rotate;
                 const int pair = (within + 2 * half) / 2;
-                const int first = rotate ? pair : within + 2 * half;
-                const int second = rotate ? pair + extras.store.n_freq : within + 2 * half + 1;
-                const bool live = column < n;
-                bias_first[nt][half] = (live && extras.store.bias) ? extras.store.bias[head * extras.store.head_dim + first] : 0.0f;
-                bias_second[nt][half] = (live && extras.store.bias) ? extras.store.bias[head * extras.store.head_dim + second] : 0.0f;
-                cos_sin[nt][half] = make_float2(1.0f, 0.0f);
-                if (live && rotate)
-                    cos_sin[nt][half] = reinterpret_cast<const float2*>(extras.store.cos_sin)[static_cast<int64_t>(col) * extras.store.n_freq + pair];
+                first[half] = rotate ? pair : within + 2 * half;
+                second[half] = rotate ? pair + store.n_freq : within + 2 * half + 1;
+                bias_first[nt][half] = (live && store.bias) ? store.bias[head * store.head_dim + first[half]] : 0.0f;
+                bias_second[nt][half] = (live && store.bias) ? store.bias[head * store.head_dim + second[half]] : 0.0f;
+#pragma unroll
+                for (int mt = 0; mt < MT; ++mt) {
+                    const int row = mt * TILE + token;
+                    cos_sin[nt][mt][half] = make_float2(1.0f, 0.0f);
+                    if (live && rotate && row < m)
+                        cos_sin[nt][mt][half] = reinterpret_cast<const float2*>(store.cos_sin)[static_cast<int64_t>(row) * store.n_freq + pair];
+                }
+            }
+            const CacheLayout layout(store.kv_heads, store.page_size, store.head_dim);
+#pragma unroll
+            for (int mt = 0; mt < MT; ++mt) {
+                const int row = mt * TILE + token;
+                if (nt == 0) {
+                    page[mt] = slot[mt] >= 0 ? slot[mt] / store.page_size : 0;
+                    place[mt] = slot[mt] >= 0 ? slot[mt] % store.page_size : 0;
+                }
+                bf16* q_row = static_cast<bf16*>(store.q_out) + (static_cast<int64_t>(row) * store.heads + head) * store.head_dim;
+#pragma unroll
+                for (int half = 0; half < 2; ++half) {
+                    bf16* to_first = nullptr;
+                    bf16* to_second = nullptr;
+                    if (live && row < m) {
+                        if (is_query) {
+                            to_first = q_row + first[half];
+                            to_second = q_row + second[half];
+                        } else if (slot[mt] >= 0 && !is_value) {
+                            bf16* pages = static_cast<bf16*>(store.k_cache);
+                            to_first = pages + layout.k_at(page[mt], head - store.heads, place[mt], first[half]);
+                            to_second = pages + layout.k_at(page[mt], head - store.heads, place[mt], second[half]);
+                        } else if (slot[mt] >= 0) {
+                            bf16* pages = static_cast<bf16*>(store.v_cache);
+                            const int kv_head = head - store.heads - store.kv_heads;
+                            to_first = pages + layout.v_at(page[mt], kv_head, place[mt], first[half]);
+                            to_second = pages + layout.v_at(page[mt], kv_head, place[mt], second[half]);
+                        }
+                    }
+                    target_first[nt][mt][half] = to_first;
+                    target_second[nt][mt][half] = to_second;
+                }
             }
         }
     }
-    float h_before[NT][4], norm_weight[NT][4];
+    float h_before[NT][MT][4], norm_weight[NT][4];
     if (EPILOGUE == 4 && wave == 0) {
 #pragma unroll
         for (int nt = 0; nt < NT; ++nt)
 #pragma unroll
             for (int i = 0; i < 4; ++i) {
-                const int column = (tile0 + nt) * 16 + quad * 4 + i;
-                const bool live = col < m && column < n;
-                h_before[nt][i] = live ? extras.residual.h[static_cast<int64_t>(col) * n + column] : 0.0f;
-                norm_weight[nt][i] = live ? extras.residual.norm_weight[column] : 0.0f;
+                const int column = (tile0 + nt) * TILE + quad * 4 + i;
+                norm_weight[nt][i] = mine && column < n ? extras.residual.norm_weight[column] : 0.0f;
+#pragma unroll
+                for (int mt = 0; mt < MT; ++mt) {
+                    const int row = mt * TILE + token;
+                    h_before[nt][mt][i] = mine && row < m && column < n ? extras.residual.h[static_cast<int64_t>(row) * n + column] : 0.0f;
+                }
             }
     }
 
-    float side[NT][4];
+    float side[NT][MT][4];
     if (EPILOGUE == 6 && wave == 0) {
         const MllSideTable& table = extras.side;
-        const int id = col < m ? table.ids[col] : 0;
-        const bool known = id >= 0 && id < table.vocab;
 #pragma unroll
-        for (int nt = 0; nt < NT; ++nt)
+        for (int mt = 0; mt < MT; ++mt) {
+            const int id = mt * TILE + token < m ? table.ids[mt * TILE + token] : 0;
+            const bool known = id >= 0 && id < table.vocab;
 #pragma unroll
-            for (int i = 0; i < 4; ++i) {
-                const int column = (tile0 + nt) * 16 + quad * 4 + i;
-                const int64_t at = static_cast<int64_t>(id) * table.stride + table.column_at + column;
-                side[nt][i] = known ? 0.0f : NAN;
-                if (known && column < n)
-                    side[nt][i] = table.dtype == kF32 ? static_cast<const float*>(table.rows)[at] : to_float(static_cast<const bf16*>(table.rows)[at]);
-            }
-    }
-
-    const bf16* w_ptr[NT];
-    bool w_live[NT];
+            for (int nt = 0; nt < NT; ++nt)
 #pragma unroll
-    for (int nt = 0; nt < NT; ++nt) {
-        w_live[nt] = tile0 + nt < n_tiles;
-        w_ptr[nt] = w_packed + static_cast<int64_t>(w_live[nt] ? tile0 + nt : tile0) * k_steps * 512 + lane * 8;
-    }
-    const bf16* a_ptr[MT];
-    bool a_live[MT];
-#pragma unroll
-    for (int mt = 0; mt < MT; ++mt) {
-        const int row = mt * 16 + col;
-        a_live[mt] = row < m;
-        a_ptr[mt] = a + static_cast<int64_t>(a_live[mt] ? row : 0) * k + quad * 8;
-    }
-    // PAIRED (one tile of rows, more than two rows): the activations are read two k steps at a time: lanes 0..7 of every 16 read rows
-    // 0..7 (then 8..15) at one step and lanes 8..15 the same rows at the next, so that a load touches whole 128-byte
-    // lines of 8 rows instead of half lines of 16; lanes 8 apart then exchange what the other needs.
-    const bool upper = col >= 8;
-    const bool low_live = (col & 7) < m, high_live = (col & 7) + 8 < m;
-    const bf16* a_low = a + static_cast<int64_t>(low_live ? (col & 7) : 0) * k + quad * 8;
-    const bf16* a_high = a + static_cast<int64_t>(high_live ? (col & 7) + 8 : 0) * k + quad * 8;
-
-    // A wave takes kChunk consecutive k steps at a time, then skips what the other waves take (the last wave
-    // begins, so that wave 0, which also writes the result, never has more chunks than another); which k steps a
-    // wave sums, and in which order, depends on (n, k) alone, not on the number of rows or tiles. The loads of
-    // DEPTH steps are issued before their products, so that a wave keeps several KB of W in flight.
-    constexpr int DEPTH = (MT + NT <= 2) ? 8 : ((MT + NT <= 4) ? 4 : 2);
-    for (int chunk = (waves - 1 - wave) * kChunk; chunk < k_steps; chunk += waves * kChunk) {
-#pragma unroll
-        for (int base = chunk; base < chunk + kChunk; base += DEPTH) {
-            Piece w_piece[DEPTH][NT];
-            Piece a_piece[DEPTH][MT];
-#pragma unroll
-            for (int u = 0; u < DEPTH; ++u) {
-                const int ks = base + u;
-                const bool live = ks < k_steps;
-#pragma unroll
-                for (int nt = 0; nt < NT; ++nt) {
-                    w_piece[u][nt].raw = uintx4{0u, 0u, 0u, 0u};
-                    if (live && w_live[nt])
-                        w_piece[u][nt].raw = __builtin_nontemporal_load(
-                            reinterpret_cast<const uintx4*>(w_ptr[nt] + static_cast<int64_t>(ks) * 512));
+                for (int i = 0; i < 4; ++i) {
+                    const int column = (tile0 + nt) * TILE + quad * 4 + i;
+                    const int64_t at = static_cast<int64_t>(id) * table.stride + table.column_at + column;
+                    side[nt][mt][i] = known ? 0.0f : NAN;
+                    if (known && mine && column < n)
+                        side[nt][mt][i] = table.dtype == kF32 ? static_cast<const float*>(table.rows)[at] : to_float(static_cast<const bf16*>(table.rows)[at]);
                 }
-                if constexpr (PAIRED) {
-                    // a_piece[u] of an even u: rows 0..7 (both steps of the pair); of the odd u after it: rows 8..15
-                    const int own = (ks & ~1) + (upper ? 1 : 0);
-                    const int k_offset = own * 32;
-                    const bool in_k = own < k_steps && k_offset + quad * 8 < k;
-                    const bool rows_live = (u & 1) ? high_live : low_live;
-                    a_piece[u][0].raw = uintx4{0u, 0u, 0u, 0u};
-                    if (rows_live && in_k)
-                        a_piece[u][0].raw = *reinterpret_cast<const uintx4*>(((u & 1) ? a_high : a_low) + k_offset);
-                } else {
-                    const int k_offset = ks * 32;
-                    const bool in_k = live && k_offset + quad * 8 < k;
-#pragma unroll
-                    for (int mt = 0; mt < MT; ++mt) {
-                        a_piece[u][mt].raw = uintx4{0u, 0u, 0u, 0u};
-                        if (a_live[mt] && in_k) a_piece[u][mt].raw = *reinterpret_cast<const uintx4*>(a_ptr[mt] + k_offset);
-                    }
-                }
-            }
-            if constexpr (PAIRED) {
-                // low = rows 0..7 at the pair's first step (lanes 0..7) and its second (lanes 8..15), high = rows
-                // 8..15 likewise. The first step's operand: own low | the partner's high; the second's: the partner's
-                // low | own high.
-#pragma unroll
-                for (int u = 0; u < DEPTH; u += 2) {
-                    const uintx4 low = a_piece[u][0].raw, high = a_piece[u + 1][0].raw;
-                    uintx4 low_swapped, high_swapped;
-#pragma unroll
-                    for (int i = 0; i < 4; ++i) {
-                        low_swapped[i] = static_cast<unsigned>(__builtin_amdgcn_update_dpp(0, static_cast<int>(low[i]), 0x128, 0xf, 0xf, false));
-                        high_swapped[i] = static_cast<unsigned>(__builtin_amdgcn_update_dpp(0, static_cast<int>(high[i]), 0x128, 0xf, 0xf, false));
-                    }
-                    a_piece[u][0].raw = upper ? high_swapped : low;
-                    a_piece[u + 1][0].raw = upper ? high : low_swapped;
-                }
-            }
-#pragma unroll
-            for (int u = 0; u < DEPTH; ++u)
-#pragma unroll
-                for (int nt = 0; nt < NT; ++nt)
-#pragma unroll
-                    for (int mt = 0; mt < MT; ++mt)
-                        acc[nt][mt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(w_piece[u][nt].v, a_piece[u][mt].v, acc[nt][mt], 0, 0, 0);
         }
     }
 
-    // The waves' sums, added in wave order by wave 0.
+    // No branch around a load, for the same reason; a block past the last step costs no memory access.
+    constexpr int kBlockSteps = HALF ? HALF * kChunk : DEPTH;
+    const int blocks = (k_steps + waves * kChunk - 1) / (waves * kChunk) * kChunk;     // steps of the wave with the most, whole runs
+    for (int done = 2 * kBlockSteps; done < blocks; done += 2 * kBlockSteps) {
+        multiply(w_even, a_even);
+        load(done / kBlockSteps, w_even, a_even);
+        __builtin_amdgcn_sched_barrier(0);      // else the loads sink below the next products, behind their waits
+        multiply(w_odd, a_odd);
+        load(done / kBlockSteps + 1, w_odd, a_odd);
+        __builtin_amdgcn_sched_barrier(0);
+    }
+    multiply(w_even, a_even);
+    multiply(w_odd, a_odd);
+
+    floatx4 (&acc)[NT][MT] = sums[0];
+    if constexpr (HALF != 0 || SPLIT) {         // the even steps' sums and the odd ones'
+#pragma unroll
+        for (int nt = 0; nt < NT; ++nt)
+#pragma unroll
+            for (int mt = 0; mt < MT; ++mt)
+#pragma unroll
+                for (int i = 0; i < 4; ++i) acc[nt][mt][i] += SPLIT ? sums[SETS - 1][nt][mt][i] : __shfl(acc[nt][mt][i], (lane + 40) % kWave, kWave);
+    }
+
+    // The factor of row `col`: the four lanes of a row take every fourth run of four sums; the order of the
+    // additions is fixed by the number of sums. Formed while other waves may still be waiting for their weights.
+    float row_factor[MT];
+    if (SCALED && wave == 0) {
+        asm volatile("s_waitcnt vmcnt(0)" ::: "memory");       // the loads into LDS have landed (the wave issued them itself)
+        floatx4 parts = floatx4{0.0f, 0.0f, 0.0f, 0.0f};      // four sums side by side, then the four together
+        if (col < m) {
+            const float* squares = factor_shared + col * extras.scale.stride;
+#pragma unroll 4
+            for (int run = quad; 4 * run < extras.scale.groups; run += 4) {
+                floatx4 four = *reinterpret_cast<const floatx4*>(squares + 4 * run);
+#pragma unroll
+                for (int i = 0; i < 4; ++i)
+                    if (4 * run + i >= extras.scale.groups) four[i] = 0.0f;
+                parts += four;
+            }
+        }
+        float part = (parts[0] + parts[1]) + (parts[2] + parts[3]);
+        part = sum_lanes_16_apart(part);
+        const float factor = 1.0f / sqrtf(part / static_cast<float>(extras.scale.width) + extras.scale.eps);
+#pragma unroll
+        for (int mt = 0; mt < MT; ++mt) row_factor[mt] = HALF ? __shfl(factor, mt * 8 + token, kWave) : factor;
+    }
+
+    // The waves' sums, added in wave order by wave 0; four slots are read at a time.
     if (waves > 1) {
         floatx4* slots = reinterpret_cast<floatx4*>(reduce_shared);
         if (wave > 0) {
@@ -224,85 +368,78 @@ __global__ __launch_bounds__(1024) void gemm_skinny_kernel(
         }
         __syncthreads();
         if (wave > 0) return;
-        for (int other = 0; other < waves - 1; ++other)
+        for (int first = 0; first < waves - 1; first += 4) {
+            floatx4 part[4][NT][MT];
 #pragma unroll
-            for (int nt = 0; nt < NT; ++nt)
+            for (int i = 0; i < 4; ++i) {
+                const int other = min(first + i, waves - 2);
 #pragma unroll
-                for (int mt = 0; mt < MT; ++mt) acc[nt][mt] += slots[(other * NT * MT + nt * MT + mt) * kWave + lane];
-    }
-
-    // The factor of row `col`: the four lanes of a row take every fourth run of four sums; the order of the
-    // additions is fixed by the number of sums.
-    float row_factor = 1.0f;
-    if (SCALED) {
-        asm volatile("s_waitcnt vmcnt(0)" ::: "memory");       // the loads into LDS have landed (the wave issued them itself)
-        floatx4 parts = floatx4{0.0f, 0.0f, 0.0f, 0.0f};      // four sums side by side, then the four together
-        if (col < m) {
-            const float* sums = factor_shared + col * extras.scale.stride;
-#pragma unroll 4
-            for (int run = quad; 4 * run < extras.scale.groups; run += 4) {
-                floatx4 four = *reinterpret_cast<const floatx4*>(sums + 4 * run);
+                for (int nt = 0; nt < NT; ++nt)
 #pragma unroll
-                for (int i = 0; i < 4; ++i)
-                    if (4 * run + i >= extras.scale.groups) four[i] = 0.0f;
-                parts += four;
+                    for (int mt = 0; mt < MT; ++mt) part[i][nt][mt] = slots[(other * NT * MT + nt * MT + mt) * kWave + lane];
             }
+#pragma unroll
+            for (int i = 0; i < 4; ++i)
+                if (first + i < waves - 1) {
+#pragma unroll
+                    for (int nt = 0; nt < NT; ++nt)
+#pragma unroll
+                        for (int mt = 0; mt < MT; ++mt) acc[nt][mt] += part[i][nt][mt];
+                }
         }
-        float part = (parts[0] + parts[1]) + (parts[2] + parts[3]);
-        part = sum_lanes_16_apart(part);
-        row_factor = 1.0f / sqrtf(part / static_cast<float>(extras.scale.width) + extras.scale.eps);
     }
 
-    // acc[nt][mt][i] = C[row mt*16 + col][column (tile0 + nt)*16 + quad*4 + i]
+    // acc[nt][mt][i] = C[row mt * TILE + token][column (tile0 + nt) * TILE + quad * 4 + i] in the lanes that hold results
 #pragma unroll
     for (int nt = 0; nt < NT; ++nt) {
         const int n_tile = tile0 + nt;
         if (n_tile >= n_tiles) continue;       // the same for every lane of the wave
-        float squares = 0.0f;                  // epilogue 4: this lane's share of its row's sum of squares over the tile
+        float squares[MT];                     // epilogue 4: this lane's share of its rows' sums of squares over the tile
 #pragma unroll
         for (int mt = 0; mt < MT; ++mt) {
-            const int row = mt * 16 + col;
-            if (row >= m) continue;
-            if (SCALED) acc[nt][mt] *= row_factor;
+            squares[mt] = 0.0f;
+            const int row = mt * TILE + token;
+            if (row >= m || !mine) continue;
+            if (SCALED) acc[nt][mt] *= row_factor[mt];
             if (EPILOGUE == 4) {
                 const MllResidualNorm& residual = extras.residual;
-                const int column = n_tile * 16 + quad * 4;
+                const int column = n_tile * TILE + quad * 4;
                 float* h_row = residual.h + static_cast<int64_t>(row) * n;
                 bf16* x_row = static_cast<bf16*>(residual.x_out) + static_cast<int64_t>(row) * n;
 #pragma unroll
                 for (int i = 0; i < 4; ++i) {
                     if (column + i >= n) continue;
-                    const float value = h_before[nt][i] + acc[nt][mt][i];
+                    const float value = h_before[nt][mt][i] + acc[nt][mt][i];
                     h_row[column + i] = value;
                     x_row[column + i] = from_float<bf16>(value * norm_weight[nt][i]);
-                    squares += value * value;
+                    squares[mt] += value * value;
                 }
             } else if (EPILOGUE == 0) {
                 float* target = static_cast<float*>(out) + static_cast<int64_t>(row) * n;
 #pragma unroll
                 for (int i = 0; i < 4; ++i) {
-                    const int column = n_tile * 16 + quad * 4 + i;
+                    const int column = n_tile * TILE + quad * 4 + i;
                     if (column < n) target[column] = acc[nt][mt][i];
                 }
             } else if (EPILOGUE == 1) {
                 bf16* target = static_cast<bf16*>(out) + static_cast<int64_t>(row) * n;
 #pragma unroll
                 for (int i = 0; i < 4; ++i) {
-                    const int column = n_tile * 16 + quad * 4 + i;
+                    const int column = n_tile * TILE + quad * 4 + i;
                     if (column < n) target[column] = from_float<bf16>(acc[nt][mt][i]);
                 }
             } else if (EPILOGUE == 6) {
                 bf16* target = static_cast<bf16*>(out) + static_cast<int64_t>(row) * n;
 #pragma unroll
                 for (int i = 0; i < 4; ++i) {
-                    const int column = n_tile * 16 + quad * 4 + i;
-                    if (column < n) target[column] = from_float<bf16>(activate(acc[nt][mt][i], kActGeluTanh) * side[nt][i]);
+                    const int column = n_tile * TILE + quad * 4 + i;
+                    if (column < n) target[column] = from_float<bf16>(activate(acc[nt][mt][i], kActGeluTanh) * side[nt][mt][i]);
                 }
             } else if (EPILOGUE == 7) {
                 bf16* target = static_cast<bf16*>(out) + static_cast<int64_t>(row) * (n / 2);
 #pragma unroll
                 for (int i = 0; i < 4; i += 2) {
-                    const int column = n_tile * 8 + quad * 2 + i / 2;
+                    const int column = n_tile * (TILE / 2) + quad * 2 + i / 2;
                     if (column < n / 2)
                         target[column] = from_float<bf16>(gated_value(acc[nt][mt][i], acc[nt][mt][i + 1], kActClampedGlu, extras.glu_limit, extras.glu_slope));
                 }
@@ -310,94 +447,97 @@ __global__ __launch_bounds__(1024) void gemm_skinny_kernel(
                 bf16* target = static_cast<bf16*>(out) + static_cast<int64_t>(row) * (n / 2);
 #pragma unroll
                 for (int i = 0; i < 4; i += 2) {
-                    const int column = n_tile * 8 + quad * 2 + i / 2;
+                    const int column = n_tile * (TILE / 2) + quad * 2 + i / 2;
                     if (column < n / 2) target[column] = from_float<bf16>(gate_fast<EPILOGUE == 5>(acc[nt][mt][i]) * acc[nt][mt][i + 1]);
                 }
             } else {
-                // The lane's 4 columns lie in one head (head_dim is a multiple of 16). In a query or key head the
-                // weight's rows were ordered so that columns 2p and 2p + 1 hold dims p and p + n_freq: the two that
-                // rotate together.
-                const int column = n_tile * 16 + quad * 4;
-                if (column >= n) continue;
-                const int head = column / store.head_dim, within = column % store.head_dim;
-                const bool is_query = head < store.heads;
-                const bool is_value = head >= store.heads + store.kv_heads;
-                const CacheLayout layout(store.kv_heads, store.page_size, store.head_dim);
-                bf16* q_row = static_cast<bf16*>(store.q_out) + (static_cast<int64_t>(row) * store.heads + head) * store.head_dim;
 #pragma unroll
-                for (int i = 0; i < 4; i += 2) {
-                    const bool rotate = !is_value && within + i < 2 * store.n_freq;
-                    const int pair = (within + i) / 2;
-                    const int first = rotate ? pair : within + i;
-                    const int second = rotate ? pair + store.n_freq : within + i + 1;
-                    const float x1 = acc[nt][mt][i] + bias_first[nt][i / 2], x2 = acc[nt][mt][i + 1] + bias_second[nt][i / 2];
-                    float y1 = x1, y2 = x2;
-                    if (rotate) {
-                        const float c = cos_sin[nt][i / 2].x, sn = cos_sin[nt][i / 2].y;
-                        y1 = rotate_first(x1, x2, c, sn);
-                        y2 = rotate_second(x1, x2, c, sn);
-                    }
-                    if (is_query) {
-                        q_row[first] = from_float<bf16>(y1);
-                        q_row[second] = from_float<bf16>(y2);
-                    } else if (slot >= 0 && !is_value) {
-                        bf16* pages = static_cast<bf16*>(store.k_cache);
-                        pages[layout.k_at(slot / store.page_size, head - store.heads, slot % store.page_size, first)] = from_float<bf16>(y1);
-                        pages[layout.k_at(slot / store.page_size, head - store.heads, slot % store.page_size, second)] = from_float<bf16>(y2);
-                    } else if (slot >= 0) {
-                        bf16* pages = static_cast<bf16*>(store.v_cache);
-                        const int kv_head = head - store.heads - store.kv_heads;
-                        pages[layout.v_at(slot / store.page_size, kv_head, slot % store.page_size, first)] = from_float<bf16>(y1);
-                        pages[layout.v_at(slot / store.page_size, kv_head, slot % store.page_size, second)] = from_float<bf16>(y2);
+                for (int half = 0; half < 2; ++half) {
+                    const float x1 = acc[nt][mt][2 * half] + bias_first[nt][half], x2 = acc[nt][mt][2 * half + 1] + bias_second[nt][half];
+                    const float c = cos_sin[nt][mt][half].x, sn = cos_sin[nt][mt][half].y;
+                    if (target_first[nt][mt][half] != nullptr) {
+                        *target_first[nt][mt][half] = from_float<bf16>(rotates[nt][half] ? rotate_first(x1, x2, c, sn) : x1);
+                        *target_second[nt][mt][half] = from_float<bf16>(rotates[nt][half] ? rotate_second(x1, x2, c, sn) : x2);
                     }
                 }
             }
         }
         if (EPILOGUE == 4) {
-            // The row's sum over the tile's 16 columns: the four lanes of a row, in a fixed order. One entry per
-            // tile of W, so that the sums do not depend on how many tiles a workgroup takes.
-            squares = sum_lanes_16_apart(squares);
-            if (quad == 0 && col < m) extras.residual.sumsq_out[static_cast<int64_t>(col) * extras.residual.sumsq_stride + n_tile] = squares;
+            // The row's sum over the tile's columns: the lanes of a row, in a fixed order. One entry per tile of W (or
+            // half of one), so that the sums do not depend on how many tiles a workgroup takes.
+#pragma unroll
+            for (int mt = 0; mt < MT; ++mt) {
+                const float over_tile = sum_lanes_16_apart(squares[mt]);
+                const int row = mt * TILE + token;
+                if (quad == 0 && mine && row < m) extras.residual.sumsq_out[static_cast<int64_t>(row) * extras.residual.sumsq_stride + n_tile] = over_tile;
+            }
         }
     }
+}
+
+// Weights of at most this many tiles of 16 rows are read in halves of tiles: a compute unit brings about 45 GB/s from
+// memory however much it asks for, so that 56 of them take 4.5 us for 7 MB and 112 take 3.5 (a kernel that only reads).
+// Product of 896 x 4864 at one row: 7.1 us with the whole tiles of before, 6.7 with whole tiles in this kernel, 5.2 in halves; 2048 x 8192:
+// 11.2, 9.5, 8.3. Above that line the activations, which every workgroup reads, cost more than the halves
+// give (224 tiles, 3584 x 18944 at 8 rows: 26 us, in halves 36).
+constexpr int kHalfTiles = 128;
+static bool in_halves(int n_tiles) { return n_tiles <= kHalfTiles; }
+
+// Waves a workgroup: 16 k steps a wave, so that a wave asks for all it needs at once without asking past the end, at most
+// 16 waves and about eight thousand over the whole launch. A function of (n, k) alone, like the split of k it implies.
+static int skinny_waves(int n_tiles, int k_steps) {
+    const int waves = min(min(16, 8192 / n_tiles), (k_steps + 15) / 16);
+    return max(1, waves);
+}
+
+template <int MT, int NT, int EPILOGUE, int GROUP, int HALF, bool SPLIT>
+static void launch_one(const bf16* a, const bf16* w, void* out, int m, int n, int k, int n_tiles,
+                       int k_steps, const MllSkinnyExtras& extras, hipStream_t stream) {
+    const int waves = skinny_waves(n_tiles, k_steps);
+    const int units = HALF ? (n + 7) / 8 : n_tiles;
+    const int groups = (units + NT - 1) / NT;
+    size_t lds = waves > 1 ? static_cast<size_t>(waves - 1) * NT * MT * kWave * sizeof(floatx4) : 0;
+    if (MT * (HALF ? 8 : 16) <= 16 && extras.scale.sumsq != nullptr) {
+        lds += (static_cast<size_t>(m) * extras.scale.stride * sizeof(float) + 1023) / 1024 * 1024;
+        gemm_skinny_kernel<MT, NT, EPILOGUE, (MT * (HALF ? 8 : 16) <= 16), GROUP, HALF, SPLIT><<<groups, waves * kWave, lds, stream>>>(
+            a, w, out, m, n, k, units, k_steps, extras);
+    } else {
+        gemm_skinny_kernel<MT, NT, EPILOGUE, false, GROUP, HALF, SPLIT><<<groups, waves * kWave, lds, stream>>>(
+            a, w, out, m, n, k, units, k_steps, extras);
+    }
+}
+
+// Up to 16 rows: halves of tiles (with few steps a wave both blocks in flight hold one run of steps, else two), or
+// whole tiles with as many steps an A load as the rows allow.
+template <int NT, int EPILOGUE>
+static void launch_few(const bf16* a, const bf16* w, void* out, int m, int n, int k, int n_tiles,
+                       int k_steps, const MllSkinnyExtras& extras, hipStream_t stream) {
+    if constexpr (NT == 1) {
+        if (in_halves(n_tiles)) {
+            const bool few_steps = k_steps <= 2 * kChunk * skinny_waves(n_tiles, k_steps);
+            if (m <= 8 && few_steps) launch_one<1, 1, EPILOGUE, 1, 1, false>(a, w, out, m, n, k, n_tiles, k_steps, extras, stream);
+            else if (m <= 8) launch_one<1, 1, EPILOGUE, 1, 2, false>(a, w, out, m, n, k, n_tiles, k_steps, extras, stream);
+            else launch_one<2, 1, EPILOGUE, 1, 1, false>(a, w, out, m, n, k, n_tiles, k_steps, extras, stream);
+            return;
+        }
+    }
+    if (m <= 4) launch_one<1, NT, EPILOGUE, 4, 0, false>(a, w, out, m, n, k, n_tiles, k_steps, extras, stream);
+    else if (m <= 8) launch_one<1, NT, EPILOGUE, 2, 0, false>(a, w, out, m, n, k, n_tiles, k_steps, extras, stream);
+    else launch_one<1, NT, EPILOGUE, 1, 0, false>(a, w, out, m, n, k, n_tiles, k_steps, extras, stream);
 }
 
 template <int MT, int NT, int EPILOGUE>
-static void launch_one(const bf16* a, const bf16* w, void* out, int m, int n, int k, int n_tiles,
-                       int k_steps, const MllSkinnyExtras& extras, hipStream_t stream) {
-    const int groups = (n_tiles + NT - 1) / NT;
-    // Waves per workgroup: enough that about sixteen thousand waves would stream W one tile each (timed inside the
-    // decode step of 7B sizes: 1 % faster than eight thousand at 8 and 16 rows, the same at one; thirty-two thousand
-    // lose at one row), at most 16, and no more than there are chunks of k for them. A function of (n, k) alone,
-    // like the split of k it implies.
-    int waves = 1;
-    while (waves < 16 && n_tiles * waves * 2 <= 16384 && waves * 2 * kChunk <= k_steps) waves *= 2;
-    size_t lds = waves > 1 ? static_cast<size_t>(waves - 1) * NT * MT * kWave * sizeof(floatx4) : 0;
-    const bool scaled = extras.scale.sumsq != nullptr;
-    // PAIRED pays from three rows on (measured on MI355X: 18944 x 3584 at 8 rows 27 -> 25.6 us, at 16 rows 34 -> 30.7;
-    // at one row 22.8 -> 24.4).
-#define MLL_SKINNY_LAUNCH(SCALED_, PAIRED_)                                                                            \
-    gemm_skinny_kernel<MT, NT, EPILOGUE, SCALED_, PAIRED_><<<groups, waves * kWave, lds, stream>>>(                    \
-        a, w, out, m, n, k, n_tiles, k_steps, extras)
-    if constexpr (MT == 1) {
-        const bool paired = m > 2;
-        if (scaled) {
-            lds += (static_cast<size_t>(m) * extras.scale.stride * sizeof(float) + 1023) / 1024 * 1024;
-            if (paired) MLL_SKINNY_LAUNCH(true, true); else MLL_SKINNY_LAUNCH(true, false);
-        } else {
-            if (paired) MLL_SKINNY_LAUNCH(false, true); else MLL_SKINNY_LAUNCH(false, false);
-        }
-    } else {
-        MLL_SKINNY_LAUNCH(false, false);
-    }
-#undef MLL_SKINNY_LAUNCH
+static void launch_many(const bf16* a, const bf16* w, void* out, int m, int n, int k, int n_tiles,
+                        int k_steps, const MllSkinnyExtras& extras, hipStream_t stream) {
+    if (in_halves(n_tiles)) launch_one<MT, NT, EPILOGUE, 1, 0, true>(a, w, out, m, n, k, n_tiles, k_steps, extras, stream);
+    else launch_one<MT, NT, EPILOGUE, 1, 0, false>(a, w, out, m, n, k, n_tiles, k_steps, extras, stream);
 }
 
-// Tiles of W a workgroup takes. Few tiles of W: one, so that the GPU is filled. Many tiles of W, or several rows of
-// A and at least 128 workgroups left: two, so that every piece of A is used twice (all measured on MI355X; four
-// tiles a workgroup were slower).
+// Tiles of W a workgroup takes: two where enough workgroups are left, so that every piece of A is used twice (MI355X, one
+// against two: 608 tiles of 896 at 8 rows 6.3 and 6.7 us, 1024 tiles of 2048 13.4 and 13.1, at one row 12.4 and 13.0; 2368 tiles
+// of 3584 at 8 rows 45.3 and 43.1, at one row 44.6 and 44.3; four tiles a workgroup were slower).
 static int tiles_per_group(int m, int n_tiles) {
-    if (m <= 16) return (n_tiles >= 2048 || (m > 4 && n_tiles >= 256)) ? 2 : 1;
+    if (m <= 16) return (n_tiles >= 2048 || (m > 4 && n_tiles >= 1024)) ? 2 : 1;
     if (m <= 32) return n_tiles >= 2048 ? 2 : 1;
     return 2;
 }
@@ -413,21 +553,21 @@ static int launch_skinny(const void* a, const void* w_packed, void* out, int m, 
     const bool two = tiles_per_group(m, n_tiles) == 2;
     if constexpr (EPILOGUE == 3 || EPILOGUE == 4 || EPILOGUE == 6 || EPILOGUE == 7) {
         if (m_tiles != 1) return fail("gemm_skinny: this epilogue takes at most 16 rows");
-        if (two) launch_one<1, 2, EPILOGUE>(a_, w_, out, m, n, k, n_tiles, k_steps, extras, stream);
-        else launch_one<1, 1, EPILOGUE>(a_, w_, out, m, n, k, n_tiles, k_steps, extras, stream);
+        if (two) launch_few<2, EPILOGUE>(a_, w_, out, m, n, k, n_tiles, k_steps, extras, stream);
+        else launch_few<1, EPILOGUE>(a_, w_, out, m, n, k, n_tiles, k_steps, extras, stream);
         return check_launch("gemm_skinny");
     }
     switch (m_tiles) {
         case 1:
-            if (two) launch_one<1, 2, EPILOGUE>(a_, w_, out, m, n, k, n_tiles, k_steps, extras, stream);
-            else launch_one<1, 1, EPILOGUE>(a_, w_, out, m, n, k, n_tiles, k_steps, extras, stream);
+            if (two) launch_few<2, EPILOGUE>(a_, w_, out, m, n, k, n_tiles, k_steps, extras, stream);
+            else launch_few<1, EPILOGUE>(a_, w_, out, m, n, k, n_tiles, k_steps, extras, stream);
             break;
         case 2:
-            if (two) launch_one<2, 2, EPILOGUE>(a_, w_, out, m, n, k, n_tiles, k_steps, extras, stream);
-            else launch_one<2, 1, EPILOGUE>(a_, w_, out, m, n, k, n_tiles, k_steps, extras, stream);
+            if (two) launch_many<2, 2, EPILOGUE>(a_, w_, out, m, n, k, n_tiles, k_steps, extras, stream);
+            else launch_many<2, 1, EPILOGUE>(a_, w_, out, m, n, k, n_tiles, k_steps, extras, stream);
             break;
-        case 3: launch_one<3, 2, EPILOGUE>(a_, w_, out, m, n, k, n_tiles, k_steps, extras, stream); break;
-        case 4: launch_one<4, 2, EPILOGUE>(a_, w_, out, m, n, k, n_tiles, k_steps, extras, stream); break;
+        case 3: launch_many<3, 2, EPILOGUE>(a_, w_, out, m, n, k, n_tiles, k_steps, extras, stream); break;
+        case 4: launch_many<4, 2, EPILOGUE>(a_, w_, out, m, n, k, n_tiles, k_steps, extras, stream); break;
         default: return fail("gemm_skinny: more than 64 rows");
     }
     return check_launch("gemm_skinny");
@@ -512,13 +652,16 @@ extern "C" int mll_gemm_skinny_qkv(const void* a, const void* w_packed, int m, i
     return launch_skinny<3>(a, w_packed, nullptr, m, n, k, extras, stream);
 }
 
+extern "C" int mll_skinny_sum_columns(int n) { return in_halves((n + 15) / 16) ? 8 : 16; }
+
 extern "C" int mll_gemm_skinny_residual(const void* a, const void* w_packed, int m, int n, int k,
                                         const MllResidualNorm* residual, const MllRowScale* scale, hipStream_t stream) {
     MLL_REQUIRE(residual != nullptr && residual->h && residual->norm_weight && residual->x_out && residual->sumsq_out,
                 "gemm_skinny_residual: the residual stream, the norm's weight and both outputs are needed");
     MLL_REQUIRE(m >= 0 && m <= 16, "gemm_skinny_residual: takes at most 16 rows");
     MLL_REQUIRE(n > 0 && k > 0 && k % 8 == 0, "gemm_skinny_residual: k must be a positive multiple of 8");
-    MLL_REQUIRE(residual->sumsq_stride >= (n + 15) / 16, "gemm_skinny_residual: the rows of sums are too short");
+    const int columns = mll_skinny_sum_columns(n);
+    MLL_REQUIRE(residual->sumsq_stride >= (n + columns - 1) / columns, "gemm_skinny_residual: the rows of sums are too short");
     if (check_scale(scale, m) != 0) return 1;
     if (m == 0) return 0;
     MllSkinnyExtras extras{};

@@ -180,14 +180,15 @@ int mll_gemm_skinny_qkv(const void* a, const void* w_packed, int m, int k, const
 
 // The product of at most 16 rows added to the residual stream, and the next RMS norm begun: h += A . W^T;
 // x_out = h * norm_weight (the norm's input without the rows' factors); sumsq_out[r][g] = the sum of h[r]^2 over
-// columns 16 g .. 16 g + 15, g < ceil(n / 16): what MllRowScale takes.
+// columns c g .. c g + c - 1, g < ceil(n / c), with c = mll_skinny_sum_columns(n): what MllRowScale takes.
 struct MllResidualNorm {
     float* h;                  // [m][n]
     const float* norm_weight;  // [n]
     void* x_out;               // bfloat16 [m][n]
-    float* sumsq_out;          // [m][sumsq_stride]; the first ceil(n / 16) of a row are written
+    float* sumsq_out;          // [m][sumsq_stride]; the first ceil(n / mll_skinny_sum_columns(n)) of a row are written
     int sumsq_stride;
 };
+int mll_skinny_sum_columns(int n);
 int mll_gemm_skinny_residual(const void* a, const void* w_packed, int m, int n, int k, const MllResidualNorm* residual,
                              const MllRowScale* scale, hipStream_t stream);
 

@@ -412,7 +412,7 @@ def gemm_skinny_residual(x: torch.Tensor, packed: torch.Tensor, h: torch.Tensor,
     _need(k % 8 == 0, "gemm_skinny_residual needs k to be a multiple of 8")
     _need(packed.dim() == 5 and tuple(packed.shape[2:]) == (4, 16, 8) and packed.shape[0] == -(-n // 16)
           and packed.shape[1] == -(-k // 32), "the packed weight does not fit n and k")
-    groups = -(-n // 16)
+    groups = -(-n // lib.mll_skinny_sum_columns(n))
     x_out = torch.empty((m, n), dtype=torch.bfloat16, device=x.device)
     sumsq = torch.empty((m, -(-groups // 4) * 4), dtype=torch.float32, device=x.device)
     residual = _ResidualNorm(_ptr(h), _ptr(norm_weight), _ptr(x_out), _ptr(sumsq), sumsq.shape[1])
