@@ -167,6 +167,12 @@ class BatchBuilder:
         self._staging: Optional[torch.Tensor] = None
         self._device_buffer: Optional[torch.Tensor] = None
         self._copied = None
+        # Tokens that are filled in later have staging of their own, two buffers in turn: the copy of the metadata that
+        # was built ahead waits on the device for the step before it, and the tokens must not wait on the host for that copy
+        # (the GPU stood still between two decode steps for as long as the host then took to launch the next).
+        self._token_staging: List[Optional[torch.Tensor]] = [None, None]
+        self._tokens_copied: list = [None, None]
+        self._token_turn = 0
 
     def _buffers(self, size: int):
         if self._staging is None or self._staging.numel() < size:
@@ -182,12 +188,16 @@ class BatchBuilder:
         """Put the tokens of a step of single tokens into the buffers that ``build`` filled for it ahead of time
         (with any tokens): they lie first in the packed buffer."""
         count = len(tokens)
-        if self._copied is not None:
-            self._copied.synchronize()
-        self._staging.numpy()[:count] = tokens
-        copy_to_device(self._device_buffer[:count], self._staging[:count], non_blocking=True)
-        self._copied = torch.cuda.Event()
-        self._copied.record()
+        turn = self._token_turn = 1 - self._token_turn
+        staging = self._token_staging[turn]
+        if staging is None or staging.numel() < count:
+            staging = self._token_staging[turn] = torch.empty(max(64, count), dtype=torch.int32, pin_memory=True)
+        elif self._tokens_copied[turn] is not None:
+            self._tokens_copied[turn].synchronize()     # the copy before last has left this buffer
+        staging.numpy()[:count] = tokens
+        copy_to_device(self._device_buffer[:count], staging[:count], non_blocking=True)
+        self._tokens_copied[turn] = torch.cuda.Event()
+        self._tokens_copied[turn].record()
 
     def build(self, requests: Sequence[RequestCache], token_lists: Sequence[Sequence[int]],
               wants: Sequence[Sequence[int]], fixed_width: Optional[int] = None) -> StepContext:

@@ -245,7 +245,8 @@ class Engine:
         every_row = [[0]] * n   # the graph computes the logits of every row; the wanted ones are picked after
         ahead, self._ahead = self._ahead, None
         if ahead is not None and state.graph is not None and ahead.holds_for(state, requests):
-            state.builder.fill_tokens([entry.tokens[0] for entry in entries])
+            if self._device_tokens is None or any(entry.token_from is None for entry in entries):
+                state.builder.fill_tokens([entry.tokens[0] for entry in entries])      # else they all come from the device
             ctx = ahead.ctx
             self.steps_built_ahead += 1
         else:
