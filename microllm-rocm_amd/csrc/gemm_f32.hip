@@ -1,6 +1,8 @@
-// The float32 matrix product of the true 32-bit path: C = A * W^T (+ bias), tiles staged through LDS.
-// Every output element is summed by one thread in ascending k, so a row's result is the same whatever
-// other rows the call holds and whichever of the kernels here computes it.
+// The float32 matrix product of the true 32-bit path: C = A * W^T (+ bias).
+// Every output element is one chain of fused multiply-adds in ascending k, so a row's result is the same whatever
+// other rows the call holds and whichever of the kernels here computes it. The chains run on the matrix units: the
+// float32 MFMAs of gfx950 give, element by element, the bits of fmaf(a[k], b[k], c) applied in ascending k (checked on
+// MI355X over normal, large, cancelling and denormal values), so they and the vector kernels may stand in for each other.
 #include "common.h"
 #include "microllm_hip.h"
 
@@ -18,20 +20,241 @@ namespace mll {
     c += static_cast<int64_t>(blockIdx.z) * m * n;                                   \
     if (blockIdx.z != 0) bias = nullptr;
 
-// Tiles for more than 16 rows. A workgroup of THREADS threads takes (THREADS / 16) * TR rows and 16 * TC columns of
-// C; a thread TR x TC elements (rows r + (THREADS / 16) * i, columns c + 16 * j), each summed by that thread alone in
-// ascending k with one fused multiply-add a term: the bits of the kernels for few rows below. Both operands come in
-// chunks of DEPTH of k with 16-byte loads of whole rows (the next chunk is on its way while this one is summed) and lie
-// in LDS as [row][k] with rows four banks apart, so that a thread's four consecutive k are one read and the rows a
-// wave reads at one k fall on different banks. Two shapes are used: 64 x 64 with 4 x 4 elements a thread (one read
-// from LDS for eight multiply-adds) wherever that gives the GPU enough workgroups (prompts; weights of many rows), and
-// 16 x 32 with 2 x 2 (one for four) where C is small: 64 rows of a weight of 3584 are 224 tiles of 64 x 64 but 896
-// of 16 x 32.
-template <int THREADS, int TR, int TC, int DEPTH, bool VECTOR>
-__global__ __launch_bounds__(THREADS) void gemm_f32_tile_kernel(const float* __restrict__ a, const float* __restrict__ w,
+typedef unsigned uintx4 __attribute__((ext_vector_type(4)));
+typedef float floatx4 __attribute__((ext_vector_type(4)));
+typedef float floatx16 __attribute__((ext_vector_type(16)));
+
+// Tiles for more than 16 rows: four waves of (32 TM) x (32 TN) elements on v_mfma_f32_32x32x2_f32, WAVES_M of them along
+// the rows. Both operands come in chunks of kTileDepth of k with 16-byte loads (the next chunk is on its way while this
+// one is multiplied) into one of two stages of LDS. An MFMA takes k from its lower 32 lanes and k + 1 from its upper 32, so a row
+// of a chunk lies as [k % 2][k / 2]: a lane's 16-byte read holds its operands of four products in a row. Rows lie four
+// banks apart, so that the eight rows of a 128-byte read fall on different banks. Bound by the matrix units (155 TFLOP/s of
+// nothing but these products; the vector units' single multiply-adds, which the tiles ran on before, give half of that) and
+// by filling the compute units: 2048 x 37888 x 3584 7190 -> 4500 us (124 TFLOP/s), 2048 x 3584 x 18944 3370 -> 2120, 1003 x 9728 x 896 257 ->
+// 165, 64 x 37888 x 3584 323 -> 202.
+constexpr int kTileDepth = 32;
+constexpr int kBufferFlags = 0x00027000;    // a raw buffer of 32-bit words
+constexpr int kNonTemporal = 2;
+constexpr int kPast = 0x40000000;           // past the end of every descriptor here, and with any row's offset added to it
+constexpr int kWidestVector = 1 << 20;      // k up to which the byte offsets of 128 rows stay below kPast
+
+// The byte offset of element `at` of a row, past the end from element `end` on. Opaque to the compiler, which would
+// otherwise branch around the loads that take it, and then wait for each of them.
+__device__ inline int offset_below(int at, int end) {
+    int offset = at < end ? at * 4 : kPast;
+    asm("" : "+v"(offset));
+    return offset;
+}
+
+template <int WAVES_M, int TM, int TN, bool VECTOR>
+__global__ __launch_bounds__(256) void gemm_f32_tile_kernel(const float* __restrict__ a, const float* __restrict__ w,
+                                                            const float* __restrict__ bias, float* __restrict__ c,
+                                                            int m, int n, int k, int k_split) {
+    MLL_F32_SPLIT_RANGE
+    constexpr int WAVES_N = 4 / WAVES_M;
+    constexpr int ROWS = WAVES_M * TM * 32, COLUMNS = WAVES_N * TN * 32;
+    constexpr int QUADS = kTileDepth / 4;                  // float4 in a row of a chunk
+    constexpr int LOADS_A = ROWS * QUADS / 256, LOADS_W = COLUMNS * QUADS / 256;
+    constexpr int STRIDE = kTileDepth + 4;
+    __shared__ __align__(16) float a_tile[2][ROWS][STRIDE];
+    __shared__ __align__(16) float w_tile[2][COLUMNS][STRIDE];
+    const int row0 = blockIdx.y * ROWS;
+    const int col0 = blockIdx.x * COLUMNS;
+    const int lane = threadIdx.x % kWave, wave = threadIdx.x / kWave;
+    const int half = lane / 32;
+    const int wave_row = wave / WAVES_N * TM * 32, wave_col = wave % WAVES_N * TN * 32;
+    // VECTOR (k a multiple of 4, 16-byte aligned rows): through buffer descriptors of the tile's rows, whose loads give
+    // zeros past the end, so that no branch (and with it a wait for every load before) stands between the loads.
+    const __amdgpu_buffer_rsrc_t a_rsrc = __builtin_amdgcn_make_buffer_rsrc(
+        const_cast<float*>(a) + static_cast<int64_t>(row0) * ld, 0, VECTOR ? min(ROWS, m - row0) * ld * 4 : 0, kBufferFlags);
+    const __amdgpu_buffer_rsrc_t w_rsrc = __builtin_amdgcn_make_buffer_rsrc(
+        const_cast<float*>(w) + static_cast<int64_t>(col0) * ld, 0, VECTOR ? min(COLUMNS, n - col0) * ld * 4 : 0, kBufferFlags);
+    auto load4 = [&](const float* matrix, const __amdgpu_buffer_rsrc_t& rsrc, int rows, int first_row, int index, int k0) {
+        const int r = index / QUADS, kk = k0 + (index % QUADS) * 4;
+        if constexpr (VECTOR) {
+            return __builtin_bit_cast(floatx4, __builtin_amdgcn_raw_buffer_load_b128(rsrc, r * ld * 4 + offset_below(kk, k), 0, 0));
+        } else {
+            const bool live = first_row + r < rows;
+            const float* source = matrix + static_cast<int64_t>(live ? first_row + r : 0) * ld + kk;
+            floatx4 v;
+#pragma unroll
+            for (int e = 0; e < 4; ++e) v[e] = (live && kk + e < k) ? source[e] : 0.0f;
+            return v;
+        }
+    };
+    floatx4 a_next[LOADS_A], w_next[LOADS_W];
+    auto fetch = [&](int k0) {
+#pragma unroll
+        for (int j = 0; j < LOADS_A; ++j) a_next[j] = load4(a, a_rsrc, m, row0, threadIdx.x + j * 256, k0);
+#pragma unroll
+        for (int j = 0; j < LOADS_W; ++j) w_next[j] = load4(w, w_rsrc, n, col0, threadIdx.x + j * 256, k0);
+    };
+    auto put = [&](float (*tile)[STRIDE], int index, const floatx4& v) {
+        float* row = &tile[index / QUADS][index % QUADS * 2];
+        *reinterpret_cast<float2*>(row) = make_float2(v[0], v[2]);
+        *reinterpret_cast<float2*>(row + kTileDepth / 2) = make_float2(v[1], v[3]);
+    };
+    floatx16 acc[TM][TN];
+#pragma unroll
+    for (int i = 0; i < TM; ++i)
+#pragma unroll
+        for (int j = 0; j < TN; ++j)
+#pragma unroll
+            for (int e = 0; e < 16; ++e) acc[i][j][e] = 0.0f;
+    fetch(k_lo);
+    int stage = 0;
+    for (int k0 = k_lo; k0 < k; k0 += kTileDepth, stage ^= 1) {
+#pragma unroll
+        for (int j = 0; j < LOADS_A; ++j) put(a_tile[stage], threadIdx.x + j * 256, a_next[j]);
+#pragma unroll
+        for (int j = 0; j < LOADS_W; ++j) put(w_tile[stage], threadIdx.x + j * 256, w_next[j]);
+        __syncthreads();        // the stage written two chunks ago was read before the last barrier
+        fetch(k0 + kTileDepth);     // zeros past the last chunk
+        __builtin_amdgcn_sched_barrier(0);      // else the loads sink behind the products and are waited for at once
+#pragma unroll
+        for (int kk = 0; kk < kTileDepth / 2; kk += 4) {
+            floatx4 av[TM], wv[TN];
+#pragma unroll
+            for (int i = 0; i < TM; ++i)
+                av[i] = *reinterpret_cast<const floatx4*>(&a_tile[stage][wave_row + 32 * i + lane % 32][half * (kTileDepth / 2) + kk]);
+#pragma unroll
+            for (int j = 0; j < TN; ++j)
+                wv[j] = *reinterpret_cast<const floatx4*>(&w_tile[stage][wave_col + 32 * j + lane % 32][half * (kTileDepth / 2) + kk]);
+#pragma unroll
+            for (int step = 0; step < 4; ++step)
+#pragma unroll
+                for (int i = 0; i < TM; ++i)
+#pragma unroll
+                    for (int j = 0; j < TN; ++j)
+                        acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x2f32(av[i][step], wv[j][step], acc[i][j], 0, 0, 0);
+        }
+    }
+#pragma unroll
+    for (int j = 0; j < TN; ++j) {
+        const int col = col0 + wave_col + 32 * j + lane % 32;
+        const float shift = (bias && col < n) ? bias[col] : 0.0f;
+#pragma unroll
+        for (int i = 0; i < TM; ++i)
+#pragma unroll
+            for (int e = 0; e < 16; ++e) {
+                const int r = row0 + wave_row + 32 * i + (e / 4) * 8 + half * 4 + e % 4;
+                if (r < m && col < n) c[static_cast<int64_t>(r) * n + col] = acc[i][j][e] + shift;
+            }
+    }
+}
+
+// At most 16 rows (decoding), k a multiple of 4: a wave takes NT tiles of 16 columns of C and its part of k, on
+// v_mfma_f32_16x16x4_f32 with 16 rows of W as its A operand. A wave's load brings 256 bytes of each of four rows, without a
+// branch between the loads, two blocks of 64 of k at a time; the wave then passes them through LDS of its own
+// (no other wave reads it), where a row of 64 lies as [k % 4][k / 4]: of every four consecutive k the product wants one in
+// each quarter of the wave, and a lane's 16-byte read holds its operands of four products in a row. GROUPS: how many
+// times four rows of A there are. Bound by reading W; against the vector kernels below at 8 rows: 37888 x 3584 109 -> 101 us
+// (5.4 TB/s), 3584 x 18944 63 -> 52, 3584 x 3584 18.4 -> 15.4, 152064 x 3584 420 -> 352 (with two tiles a wave at 9 to 16 rows 496
+// -> 367). Two blocks of 128 instead of 64 of k in flight are slower (more is asked for past the ends: 52 -> 57).
+constexpr int64_t kFewWaves = 384;      // waves from which this kernel is taken: 1152 x 896 in two parts, 144 waves, takes 5.6 us in the vector kernel and 7.7 here; 896 x 4864 in eight, 448 waves, 10.8 and 9.6
+constexpr int kFewRow = 64 + 16;        // floats from one row in LDS to the next: the four rows of a load on different banks
+
+template <int NT, int GROUPS>
+__global__ __launch_bounds__(256) void gemm_f32_few_kernel(const float* __restrict__ a, const float* __restrict__ w,
+                                                           const float* __restrict__ bias, float* __restrict__ c,
+                                                           int m, int n, int k, int k_split) {
+    MLL_F32_SPLIT_RANGE
+    __shared__ __align__(16) float shared[4][NT + 1][16][kFewRow];
+    const int lane = threadIdx.x % kWave;
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave);
+    const int col = lane % 16, quad = lane / 16;
+    const int first = (blockIdx.x * 4 + wave) * 16 * NT;        // the wave's first column of C, row of W
+    if (first >= n) return;
+    const __amdgpu_buffer_rsrc_t w_rsrc = __builtin_amdgcn_make_buffer_rsrc(const_cast<float*>(w) + static_cast<int64_t>(first) * ld, 0,
+                                                                            min(16 * NT, n - first) * ld * 4, kBufferFlags);
+    const __amdgpu_buffer_rsrc_t a_rsrc = __builtin_amdgcn_make_buffer_rsrc(const_cast<float*>(a), 0, m * ld * 4, kBufferFlags);
+    floatx4 acc[NT];
+#pragma unroll
+    for (int nt = 0; nt < NT; ++nt) acc[nt] = floatx4{0.0f, 0.0f, 0.0f, 0.0f};
+    struct Block {
+        floatx4 w[NT][4], a[GROUPS];
+    };
+    auto load = [&](int k0, Block& block) {
+        const int at = offset_below(k0 + col * 4, k);
+#pragma unroll
+        for (int nt = 0; nt < NT; ++nt)
+#pragma unroll
+            for (int g = 0; g < 4; ++g)
+                block.w[nt][g] = __builtin_bit_cast(floatx4, __builtin_amdgcn_raw_buffer_load_b128(w_rsrc, (16 * nt + 4 * g + quad) * ld * 4 + at, 0, kNonTemporal));
+#pragma unroll
+        for (int g = 0; g < GROUPS; ++g)
+            block.a[g] = __builtin_bit_cast(floatx4, __builtin_amdgcn_raw_buffer_load_b128(a_rsrc, (4 * g + quad) * ld * 4 + at, 0, 0));
+    };
+    auto put = [&](float (*rows)[kFewRow], int g, const floatx4& v) {
+#pragma unroll
+        for (int e = 0; e < 4; ++e) rows[4 * g + quad][16 * e + col] = v[e];
+    };
+    auto multiply = [&](Block& block) {
+        // LDS takes a wave's accesses in order; the fences keep the compiler to it.
+        __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+#pragma unroll
+        for (int g = 0; g < GROUPS; ++g) put(shared[wave][NT], g, block.a[g]);
+#pragma unroll
+        for (int nt = 0; nt < NT; ++nt)
+#pragma unroll
+            for (int g = 0; g < 4; ++g) put(shared[wave][nt], g, block.w[nt][g]);
+        __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+#pragma unroll
+        for (int part = 0; part < 4; ++part) {
+            const floatx4 av = *reinterpret_cast<const floatx4*>(&shared[wave][NT][col % (4 * GROUPS)][16 * quad + 4 * part]);
+            floatx4 wv[NT];
+#pragma unroll
+            for (int nt = 0; nt < NT; ++nt) wv[nt] = *reinterpret_cast<const floatx4*>(&shared[wave][nt][col][16 * quad + 4 * part]);
+#pragma unroll
+            for (int step = 0; step < 4; ++step)
+#pragma unroll
+                for (int nt = 0; nt < NT; ++nt) acc[nt] = __builtin_amdgcn_mfma_f32_16x16x4f32(wv[nt][step], av[step], acc[nt], 0, 0, 0);
+        }
+    };
+    Block even, odd;
+    constexpr int kBlock = 64;
+    load(k_lo, even);
+    load(k_lo + kBlock, odd);
+    for (int k0 = k_lo + 2 * kBlock; k0 < k; k0 += 2 * kBlock) {
+        multiply(even);
+        load(k0, even);
+        __builtin_amdgcn_sched_barrier(0);      // else the loads sink below the next products, behind their waits
+        multiply(odd);
+        load(k0 + kBlock, odd);
+        __builtin_amdgcn_sched_barrier(0);
+    }
+    multiply(even);
+    multiply(odd);
+    // acc[nt][i] = C[row col][column first + 16 nt + 4 quad + i]; columns of rows that are none hold other rows' sums
+#pragma unroll
+    for (int nt = 0; nt < NT; ++nt)
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+            const int column = first + 16 * nt + 4 * quad + i;
+            if (col < m && column < n) c[static_cast<int64_t>(col) * n + column] = acc[nt][i] + (bias ? bias[column] : 0.0f);
+        }
+}
+
+template <int NT>
+static void launch_few(const float* a, const float* w, const float* bias, float* c, int m, int n, int k, int k_split,
+                       unsigned parts, hipStream_t stream) {
+    const dim3 grid((n + 64 * NT - 1) / (64 * NT), 1, parts);
+    if (m <= 4) gemm_f32_few_kernel<NT, 1><<<grid, 256, 0, stream>>>(a, w, bias, c, m, n, k, k_split);
+    else if (m <= 8) gemm_f32_few_kernel<NT, 2><<<grid, 256, 0, stream>>>(a, w, bias, c, m, n, k, k_split);
+    else gemm_f32_few_kernel<NT, 4><<<grid, 256, 0, stream>>>(a, w, bias, c, m, n, k, k_split);
+}
+
+// Tiles of 16 x 32 for more than 16 rows of small weights, where tiles of the matrix units would be a handful of workgroups,
+// each waiting for one chunk of k after the other: a thread takes 2 x 2 elements (rows r and r + 8, columns c and c + 16), each summed by
+// that thread alone in ascending k. Chunks of 128 of k lie in LDS as [row][k] with rows four banks apart, so that a thread's
+// four consecutive k are one read and the rows a wave reads at one k fall on different banks.
+constexpr int64_t kGrainBelow = 64;     // workgroups of the matrix units' tiles (64 x 896 x 1152, 36 of them: 13.4 us there, 12.2 here; 24 x 896 x 9728, 76: 17.2 and 20.7)
+template <bool VECTOR>
+__global__ __launch_bounds__(128) void gemm_f32_grain_kernel(const float* __restrict__ a, const float* __restrict__ w,
                                                                 const float* __restrict__ bias, float* __restrict__ c,
                                                                 int m, int n, int k, int k_split) {
     MLL_F32_SPLIT_RANGE
+    constexpr int THREADS = 128, TR = 2, TC = 2, DEPTH = 128;
     constexpr int ROW_STEP = THREADS / 16;
     constexpr int ROWS = ROW_STEP * TR;
     constexpr int COLUMNS = 16 * TC;
@@ -335,7 +558,13 @@ extern "C" int mll_gemm_f32(const float* a, const float* w, const float* bias, f
     const int k_split = splits == 1 ? k : ((k + splits - 1) / splits + 3) / 4 * 4;
     MLL_REQUIRE(static_cast<int64_t>(k_split) * (splits - 1) < k, "gemm_f32: a part of the reduction would be empty");
     const unsigned parts = static_cast<unsigned>(splits);
-    const bool vector = k % 4 == 0 && reinterpret_cast<uintptr_t>(a) % 16 == 0 && reinterpret_cast<uintptr_t>(w) % 16 == 0;
+    const bool vector = k % 4 == 0 && k <= kWidestVector && reinterpret_cast<uintptr_t>(a) % 16 == 0 && reinterpret_cast<uintptr_t>(w) % 16 == 0;
+    const int64_t waves = static_cast<int64_t>((n + 15) / 16) * splits;
+    if (m <= 16 && vector && f32_small_variant == 0 && waves >= kFewWaves) {
+        if (n >= kWideFrom && m > 8) launch_few<2>(a, w, bias, c, m, n, k, k_split, parts, stream);
+        else launch_few<1>(a, w, bias, c, m, n, k, k_split, parts, stream);
+        return check_launch("gemm_f32");
+    }
     if (m <= 16) {
         // Up to 8 rows: one row and four columns a thread where that still gives the GPU its workgroups (weights of
         // many rows; the others with their parts); else two rows and two columns where that does, else the kernel of
@@ -364,28 +593,35 @@ extern "C" int mll_gemm_f32(const float* a, const float* w, const float* bias, f
         else gemm_f32_small_kernel<false><<<grid, 256, 0, stream>>>(a, w, bias, c, m, n, k, k_split);
         return check_launch("gemm_f32");
     }
-    // Tiles of 64 x 64 wherever they are enough workgroups for the GPU; for at most 32 rows of a weight with many rows
-    // tiles of 32 x 64 (the same 4 x 4 elements a thread: the head at 17 to 32 rows 940 -> 640 us); else tiles of 16 x 32.
-    const int64_t column_tiles = (n + 63) / 64;
-    if (m >= 512 && column_tiles * ((m + 127) / 128) * splits >= 512) {
-        const dim3 grid(column_tiles, (m + 127) / 128, parts);
-        MLL_REQUIRE(grid.y <= 65535, "gemm_f32: too many rows for one call");
-        if (vector) gemm_f32_tile_kernel<256, 8, 4, 32, true><<<grid, 256, 0, stream>>>(a, w, bias, c, m, n, k, k_split);
-        else gemm_f32_tile_kernel<256, 8, 4, 32, false><<<grid, 256, 0, stream>>>(a, w, bias, c, m, n, k, k_split);
-    } else if (m > 32 && column_tiles * ((m + 63) / 64) * splits >= 384) {
-        const dim3 grid(column_tiles, (m + 63) / 64, parts);
-        MLL_REQUIRE(grid.y <= 65535, "gemm_f32: too many rows for one call");
-        if (vector) gemm_f32_tile_kernel<256, 4, 4, 32, true><<<grid, 256, 0, stream>>>(a, w, bias, c, m, n, k, k_split);
-        else gemm_f32_tile_kernel<256, 4, 4, 32, false><<<grid, 256, 0, stream>>>(a, w, bias, c, m, n, k, k_split);
-    } else if (m <= 32 && n >= kWideFrom) {
-        const dim3 grid(column_tiles, (m + 31) / 32, parts);
-        if (vector) gemm_f32_tile_kernel<128, 4, 4, 32, true><<<grid, 128, 0, stream>>>(a, w, bias, c, m, n, k, k_split);
-        else gemm_f32_tile_kernel<128, 4, 4, 32, false><<<grid, 128, 0, stream>>>(a, w, bias, c, m, n, k, k_split);
-    } else {
-        const dim3 grid((n + 31) / 32, (m + 15) / 16, parts);
-        MLL_REQUIRE(grid.y <= 65535, "gemm_f32: too many rows for one call");
-        if (vector) gemm_f32_tile_kernel<128, 2, 2, 128, true><<<grid, 128, 0, stream>>>(a, w, bias, c, m, n, k, k_split);
-        else gemm_f32_tile_kernel<128, 2, 2, 128, false><<<grid, 128, 0, stream>>>(a, w, bias, c, m, n, k, k_split);
+    // The tile whose workgroups fill the compute units best: the matrix units' time is the rounds of 256 workgroups times
+    // a tile's size. Up to 32 rows there is one row of tiles.
+    struct Shape { int rows, columns; };
+    const Shape shapes[4] = {{128, 128}, {128, 64}, {64, 64}, {32, 128}};
+    int best = 3;
+    double least = 1e300;
+    for (int index = 0; index < 4; ++index) {
+        const Shape& shape = shapes[index];
+        const int64_t groups = static_cast<int64_t>((n + shape.columns - 1) / shape.columns) * ((m + shape.rows - 1) / shape.rows) * splits;
+        const double rounds = groups >= 4096 ? groups / 256.0 : static_cast<double>((groups + 255) / 256);
+        const double cost = rounds * shape.rows * shape.columns;
+        if (cost < least) least = cost, best = index;
     }
+    const Shape& shape = shapes[best];
+    if (static_cast<int64_t>((n + shape.columns - 1) / shape.columns) * ((m + shape.rows - 1) / shape.rows) * splits < kGrainBelow) {
+        const dim3 grid((n + 31) / 32, (m + 15) / 16, parts);
+        if (vector) gemm_f32_grain_kernel<true><<<grid, 128, 0, stream>>>(a, w, bias, c, m, n, k, k_split);
+        else gemm_f32_grain_kernel<false><<<grid, 128, 0, stream>>>(a, w, bias, c, m, n, k, k_split);
+        return check_launch("gemm_f32");
+    }
+    const dim3 grid((n + shape.columns - 1) / shape.columns, (m + shape.rows - 1) / shape.rows, parts);
+    MLL_REQUIRE(grid.y <= 65535, "gemm_f32: too many rows for one call");
+#define MLL_F32_TILE(WAVES_M, TM, TN)                                                                                  \
+    if (vector) gemm_f32_tile_kernel<WAVES_M, TM, TN, true><<<grid, 256, 0, stream>>>(a, w, bias, c, m, n, k, k_split); \
+    else gemm_f32_tile_kernel<WAVES_M, TM, TN, false><<<grid, 256, 0, stream>>>(a, w, bias, c, m, n, k, k_split)
+    if (best == 0) { MLL_F32_TILE(2, 2, 2); }
+    else if (best == 1) { MLL_F32_TILE(2, 2, 1); }
+    else if (best == 2) { MLL_F32_TILE(2, 1, 1); }
+    else { MLL_F32_TILE(1, 1, 1); }
+#undef MLL_F32_TILE
     return check_launch("gemm_f32");
 }
