@@ -9,6 +9,10 @@
 // (steps with many rows: portions of prompts), or one wave per chunk leaves its result in a workspace and a
 // second kernel merges them (steps with few rows, whose keys would otherwise be walked by a handful of waves).
 // Sums that decide bits are written with explicit fused multiply-adds, so that both kernels round alike.
+//
+// Runs of 16 tokens of one request in steps with many rows (prompts) take a third kernel in float32, which does the
+// same operations in the same order on the matrix units: a float32 MFMA of gfx950 gives, element by element, the bits of
+// fused multiply-adds in ascending order of its terms (gemm_f32.hip).
 #include <type_traits>
 
 #include "cache_layout.h"
@@ -133,6 +137,34 @@ __device__ inline float merged(float so_far, float keep, float chunk, float add)
     return __fmaf_rn(so_far, keep, __fmul_rn(chunk, add));
 }
 
+// ---- runs of 16 tokens on the matrix units -----------------------------------------------------------------------
+typedef float floatx4 __attribute__((ext_vector_type(4)));
+constexpr int kRunTokens = 16;
+
+// The tokens 16 * block .. + 15 of the step in stretches of places of one request in a row: bit i is set where token i begins
+// one. Tokens that only pad the step, or lie past its end, begin one each and belong to none (`none`).
+struct TokenRuns {
+    unsigned begins, none;
+    __device__ int end_of(int begin) const {      // where the stretch that begins there ends
+        const unsigned after = begins & ~((2u << begin) - 1);
+        return after ? __ffs(after) - 1 : kRunTokens;
+    }
+    // Few enough stretches for the kernel that takes them one after the other; else (single tokens of many requests) a wave a token.
+    __device__ bool taken() const { return __popc(begins & ~none) <= kMostRuns; }
+    static constexpr int kMostRuns = 3;
+};
+__device__ inline TokenRuns token_runs(const int32_t* seq_of_token, const int32_t* positions, int block, int n_tokens) {
+    const int at = static_cast<int>(threadIdx.x) % kRunTokens;
+    const int token = min(block * kRunTokens + at, n_tokens - 1), before = max(token - 1, 0);
+    const int seq = seq_of_token[token];
+    const bool none = block * kRunTokens + at >= n_tokens || seq < 0;
+    const bool begins = none || at == 0 || seq_of_token[before] != seq || positions[before] + 1 != positions[token];
+    TokenRuns runs;
+    runs.begins = static_cast<unsigned>(__ballot(begins)) & 0xffffu;
+    runs.none = static_cast<unsigned>(__ballot(none)) & 0xffffu;
+    return runs;
+}
+
 // DIMS: dims a lane holds (head_dim <= 64 * DIMS). MODE 0: one wave per (token, head) walks all chunks. MODE 1: one wave per (token, head, chunk) writes
 // part_o[row][slot][dim] and part_ml[row][slot] = (maximum, sum), slot counting from the row's first chunk.
 template <typename T, int MODE, int DIMS>
@@ -141,7 +173,7 @@ __global__ __launch_bounds__(kWave) void paged_attention_rowwise_kernel(
     const int32_t* __restrict__ block_table, int table_width, const int32_t* __restrict__ seq_of_token,
     const int32_t* __restrict__ positions, T* __restrict__ out, float* __restrict__ part_o,
     float* __restrict__ part_ml, int max_chunks, float scale, int window, int heads, int kv_heads, int head_dim,
-    int page_size) {
+    int page_size, int runs_apart) {
     __shared__ float q_shared[kRowwiseMaxHeadDim];
     __shared__ float p_shared[kWave];
     __shared__ int64_t v_shared[2][kWave];
@@ -152,6 +184,7 @@ __global__ __launch_bounds__(kWave) void paged_attention_rowwise_kernel(
     const int lane = threadIdx.x;
     const int seq = seq_of_token[token];
     if (seq < 0) return;      // a row that only pads the step to a fixed shape: its output stays as it is
+    if (MODE == 0 && runs_apart && token_runs(seq_of_token, positions, token / kRunTokens, gridDim.x).taken()) return;
     const int position = positions[token];
     const int low = window > 0 ? max(0, position - window + 1) : 0;
     const int first_chunk = low / kRowwiseChunk, last_chunk = position / kRowwiseChunk;
@@ -222,13 +255,14 @@ __global__ __launch_bounds__(kWave) void paged_attention_rowwise_kernel(
 // order of the keys; only what is independent of the head (addresses, loads) is done once. Writes what MODE 1 writes,
 // bit for bit. Head sizes up to 64 * DIMS <= 128.
 // MODE as in the kernel for one head a wave: 0 walks all chunks of the row and merges as it goes (out), 1 takes the chunk
-// blockIdx.z and leaves its result in the workspace (part_o, part_ml).
+// blockIdx.z and leaves its result in the workspace (part_o, part_ml). runs_apart (MODE 0, both kernels): tokens that
+// paged_attention_rowwise_runs_kernel takes are passed over.
 template <typename T, int MODE, int DIMS, int GW>
 __global__ __launch_bounds__(kWave) void paged_attention_rowwise_heads_kernel(
     const T* __restrict__ q, const T* __restrict__ k_cache, const T* __restrict__ v_cache,
     const int32_t* __restrict__ block_table, int table_width, const int32_t* __restrict__ seq_of_token,
     const int32_t* __restrict__ positions, T* __restrict__ out, float* __restrict__ part_o, float* __restrict__ part_ml,
-    int max_chunks, float scale, int window, int heads, int kv_heads, int head_dim, int page_size) {
+    int max_chunks, float scale, int window, int heads, int kv_heads, int head_dim, int page_size, int runs_apart) {
     __shared__ float q_shared[GW][64 * DIMS];
     __shared__ float p_shared[GW][kWave];
     __shared__ int64_t v_shared[2][kWave];
@@ -243,6 +277,7 @@ __global__ __launch_bounds__(kWave) void paged_attention_rowwise_heads_kernel(
     const int heads_here = min(GW, group - first_in_group);      // heads past them repeat the last one and write nothing
     const int seq = seq_of_token[token];
     if (seq < 0) return;
+    if (MODE == 0 && runs_apart && token_runs(seq_of_token, positions, token / kRunTokens, gridDim.x).taken()) return;
     const int position = positions[token];
     const int low = window > 0 ? max(0, position - window + 1) : 0;
     const int first_chunk = low / kRowwiseChunk, last_chunk = position / kRowwiseChunk;
@@ -390,6 +425,246 @@ __global__ __launch_bounds__(kWave) void paged_attention_rowwise_heads_kernel(
     }
 }
 
+// Register j of quarter q of the wave becomes register q of quarter j.
+__device__ inline floatx4 transpose_quarters(floatx4 v) {
+    auto swap32 = [](unsigned& low, unsigned& high) {
+        const auto both = __builtin_amdgcn_permlane32_swap(low, high, false, false);
+        low = both[0], high = both[1];
+    };
+    auto swap16 = [](unsigned& low, unsigned& high) {
+        const auto both = __builtin_amdgcn_permlane16_swap(low, high, false, false);
+        low = both[0], high = both[1];
+    };
+    const float e0 = v[0], e1 = v[1], e2 = v[2], e3 = v[3];
+    unsigned r0 = __builtin_bit_cast(unsigned, e0), r1 = __builtin_bit_cast(unsigned, e1);
+    unsigned r2 = __builtin_bit_cast(unsigned, e2), r3 = __builtin_bit_cast(unsigned, e3);
+    swap32(r0, r2);
+    swap32(r1, r3);
+    swap16(r0, r1);
+    swap16(r2, r3);
+    return floatx4{__builtin_bit_cast(float, r0), __builtin_bit_cast(float, r1), __builtin_bit_cast(float, r2), __builtin_bit_cast(float, r3)};
+}
+
+// The value of the lane 32, or 16, away (xor), without LDS.
+__device__ inline float from_32_away(float value) {
+    const unsigned bits = __builtin_bit_cast(unsigned, value);
+    const auto halves = __builtin_amdgcn_permlane32_swap(bits, bits, false, false);
+    const unsigned low = halves[0], high = halves[1];       // every lane: the lower half's value, the upper half's
+    return __builtin_bit_cast(float, threadIdx.x % kWave < 32 ? high : low);
+}
+__device__ inline float from_16_away(float value) {
+    const unsigned bits = __builtin_bit_cast(unsigned, value);
+    const auto rows = __builtin_amdgcn_permlane16_swap(bits, bits, false, false);
+    const unsigned even = rows[0], odd = rows[1];
+    return __builtin_bit_cast(float, threadIdx.x % 32 < 16 ? odd : even);
+}
+
+// A wave takes 16 tokens of the step and one head, the stretches of one request in them (token_runs) one after the other, and walks the chunks and tiles of 64 keys as the kernels above do for
+// one token, on v_mfma_f32_16x16x4_f32: S^T = K . Q^T leaves in lane (token, quarter) the scores of keys 16 t + 4 quarter +
+// i, whose sum over the tile meets in the order of wave_sum (32, 16 in the lane, 8 and 4 between lanes, 2, 1 in the
+// lane); O^T = V^T . P^T adds the keys in ascending order. All three operands come from memory with 16 bytes a lane, four consecutive
+// terms of the reduction, where the product wants one of every four consecutive ones a quarter: transpose_quarters. The four waves of
+// a workgroup are neighbouring heads, which mostly read the same keys. The last tile's keys, which not every token sees, are
+// multiplied with a weight of zero where a token does not see them, which changes nothing unless a value is not finite:
+// then that tile's values are added one by one as above.
+// Bound by the matrix units and, with one wave a SIMD (up to 477 registers), by the loads of a tile's keys and values, which
+// fly over one tile's arithmetic. Prompts of 1003 tokens of 14 heads of 64: 292 -> 80 us against a wave a token and four heads, 300 of
+// 28 heads of 128: 123 -> 55, 1500: 985 -> 330.
+template <int HD_TILES>
+__global__ __launch_bounds__(256) void paged_attention_rowwise_runs_kernel(
+    const float* __restrict__ q, const float* __restrict__ k_cache, const float* __restrict__ v_cache,
+    const int32_t* __restrict__ block_table, int table_width, const int32_t* __restrict__ seq_of_token,
+    const int32_t* __restrict__ positions, float* __restrict__ out, float scale, int n_tokens, int heads, int kv_heads, int page_size) {
+#pragma clang fp contract(off)      // a scaled score less the maximum is two roundings, as in the kernels above
+    constexpr int HD = HD_TILES * 16;
+    const int lane = threadIdx.x % kWave, wave = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave);
+    const int col = lane % 16, quad = lane / 16;
+    const int blocks = (n_tokens + kRunTokens - 1) / kRunTokens;
+    const int unit = blockIdx.x * 4 + wave;
+    if (unit >= blocks * heads) return;
+    const int block = blocks - 1 - unit / heads, head = unit % heads;       // the last tokens see the most keys: they go first
+    const TokenRuns runs = token_runs(seq_of_token, positions, block, n_tokens);
+    if (!runs.taken()) return;
+    const CacheLayout layout(kv_heads, page_size, HD);
+    const int kv_head = head / (heads / kv_heads);
+    for (int begin = 0, end; begin < kRunTokens; begin = end) {
+    end = __builtin_amdgcn_readfirstlane(runs.end_of(begin));
+    if ((runs.none >> begin) & 1) continue;
+    const int first_token = block * kRunTokens + begin, count = end - begin;
+    const int token = first_token + min(col, count - 1);         // lanes past the stretch repeat its last token and write nothing
+    const int first_position = __builtin_amdgcn_readfirstlane(positions[first_token]);
+    const int position = first_position + min(col, count - 1), last_position = first_position + count - 1;
+    const int32_t* table = block_table + static_cast<int64_t>(__builtin_amdgcn_readfirstlane(seq_of_token[first_token])) * table_width;
+
+    floatx4 q_piece[HD_TILES];      // the B operand: lane (token, quarter) holds dims 16 d + 4 j + quarter
+#pragma unroll
+    for (int d = 0; d < HD_TILES; ++d)
+        q_piece[d] = transpose_quarters(*reinterpret_cast<const floatx4*>(q + (static_cast<int64_t>(token) * heads + head) * HD + 16 * d + 4 * quad));
+
+    auto pages_of = [&](int tile, int64_t (&page)[4]) {
+#pragma unroll
+        for (int t = 0; t < 4; ++t) page[t] = max(table[min((tile + 16 * t) / page_size, table_width - 1)], 0);     // keys that nobody sees may have none
+    };
+    auto load_keys = [&](int tile, const int64_t (&page)[4], floatx4 (&k)[4][HD_TILES]) {
+#pragma unroll
+        for (int t = 0; t < 4; ++t) {
+            const float* from = k_cache + layout.k_tile(page[t], kv_head, (tile + 16 * t) % page_size / 16) + (quad / 2) * 128 + col * 8 + (quad % 2) * 4;
+#pragma unroll
+            for (int d = 0; d < HD_TILES; ++d) k[t][d] = *reinterpret_cast<const floatx4*>(from + d * 256);
+        }
+    };
+    auto load_values = [&](int tile, const int64_t (&page)[4], floatx4 (&v)[4][HD_TILES]) {
+#pragma unroll
+        for (int t = 0; t < 4; ++t) {
+            const float* from = v_cache + layout.v_tile(page[t], kv_head, (tile + 16 * t) % page_size / 16);
+#pragma unroll
+            for (int d = 0; d < HD_TILES; ++d) {
+                const int width = (HD_TILES % 2 == 1 && d == HD_TILES - 1) ? 16 : 32;      // dims of the block of 32 this tile of 16 lies in
+                v[t][d] = *reinterpret_cast<const floatx4*>(from + (d / 2) * 512 + ((quad / 2) * width + (d % 2) * 16 + col) * 8 + (quad % 2) * 4);
+            }
+        }
+    };
+
+    floatx4 acc[HD_TILES], total[HD_TILES];
+#pragma unroll
+    for (int d = 0; d < HD_TILES; ++d) acc[d] = total[d] = floatx4{0.0f, 0.0f, 0.0f, 0.0f};
+    float chunk_max = -INFINITY, chunk_sum = 0.0f, total_max = -INFINITY, total_sum = 0.0f;
+    floatx4 k[4][HD_TILES], v[4][HD_TILES];
+    int64_t page[4];
+    pages_of(0, page);
+    load_keys(0, page, k);
+    load_values(0, page, v);
+    for (int tile = 0; tile <= last_position; tile += kWave) {
+        float score[4][4];
+#pragma unroll
+        for (int t = 0; t < 4; ++t) {
+            floatx4 s = floatx4{0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll
+            for (int d = 0; d < HD_TILES; ++d) {
+                const floatx4 piece = transpose_quarters(k[t][d]);
+#pragma unroll
+                for (int step = 0; step < 4; ++step) s = __builtin_amdgcn_mfma_f32_16x16x4f32(piece[step], q_piece[d][step], s, 0, 0, 0);
+            }
+#pragma unroll
+            for (int i = 0; i < 4; ++i) score[t][i] = tile + 16 * t + 4 * quad + i <= position ? __fmul_rn(s[i], scale) : -INFINITY;
+        }
+        const int next = min(tile + kWave, last_position / kWave * kWave);      // after the last tile that one again, dropped
+        int64_t next_page[4];
+        pages_of(next, next_page);
+        load_keys(next, next_page, k);
+
+        float tile_max = score[0][0];
+#pragma unroll
+        for (int t = 0; t < 4; ++t)
+#pragma unroll
+            for (int i = 0; i < 4; ++i) tile_max = fmaxf(tile_max, score[t][i]);
+        tile_max = fmaxf(tile_max, from_32_away(tile_max));
+        tile_max = fmaxf(tile_max, from_16_away(tile_max));
+        // A token before the tile has nothing in it: its numbers stay what they are.
+        const bool here = tile <= position;
+        const float new_max = here ? fmaxf(chunk_max, tile_max) : chunk_max;
+        const float rescale = here ? expf(chunk_max - new_max) : 1.0f;
+        float p[4][4];
+#pragma unroll
+        for (int t = 0; t < 4; ++t)
+#pragma unroll
+            for (int i = 0; i < 4; ++i) p[t][i] = tile + 16 * t + 4 * quad + i <= position ? expf(score[t][i] - new_max) : 0.0f;
+        float part[4];
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+            part[i] = (p[0][i] + p[2][i]) + (p[1][i] + p[3][i]);
+            part[i] += from_32_away(part[i]);
+            part[i] += from_16_away(part[i]);
+        }
+        const float tile_sum = (part[0] + part[2]) + (part[1] + part[3]);
+        chunk_sum = here ? __fmaf_rn(chunk_sum, rescale, tile_sum) : chunk_sum;
+        chunk_max = new_max;
+
+        const bool whole = tile + kWave - 1 <= first_position;      // every token sees every key
+        bool finite = true;
+        if (!whole) {
+#pragma unroll
+            for (int t = 0; t < 4; ++t)
+#pragma unroll
+                for (int d = 0; d < HD_TILES; ++d)
+#pragma unroll
+                    for (int i = 0; i < 4; ++i) {
+                        if (tile + 16 * t + 4 * quad + i > last_position) v[t][d][i] = 0.0f;       // what lies there may be stale
+                        finite = finite && __builtin_isfinite(v[t][d][i]);
+                    }
+            finite = __all(finite);
+        }
+#pragma unroll
+        for (int d = 0; d < HD_TILES; ++d)
+#pragma unroll
+            for (int i = 0; i < 4; ++i) acc[d][i] = __fmul_rn(acc[d][i], rescale);
+        if (finite) {
+#pragma unroll
+            for (int t = 0; t < 4; ++t) {
+                const floatx4 weights = transpose_quarters(floatx4{p[t][0], p[t][1], p[t][2], p[t][3]});
+#pragma unroll
+                for (int d = 0; d < HD_TILES; ++d) {
+                    const floatx4 piece = transpose_quarters(v[t][d]);
+#pragma unroll
+                    for (int step = 0; step < 4; ++step) acc[d] = __builtin_amdgcn_mfma_f32_16x16x4f32(piece[step], weights[step], acc[d], 0, 0, 0);
+                }
+            }
+        } else {
+            for (int key = tile; key <= min(last_position, tile + kWave - 1); ++key) {
+                const int in_tile = key - tile;
+                float weight = 0.0f;
+#pragma unroll
+                for (int t = 0; t < 4; ++t)
+#pragma unroll
+                    for (int i = 0; i < 4; ++i) {
+                        const float there = __shfl(p[t][i], 16 * (in_tile % 16 / 4) + col, kWave);
+                        if (in_tile == 16 * t + in_tile % 16 / 4 * 4 + i) weight = there;
+                    }
+                const float* from = v_cache + layout.v_tile(page[0], kv_head, 0);
+#pragma unroll
+                for (int t = 0; t < 4; ++t)
+                    if (in_tile / 16 == t) from = v_cache + layout.v_tile(page[t], kv_head, (tile + 16 * t) % page_size / 16);
+#pragma unroll
+                for (int d = 0; d < HD_TILES; ++d)
+#pragma unroll
+                    for (int i = 0; i < 4; ++i) {
+                        const float value = from[layout.v_in_tile(key % 16, 16 * d + 4 * quad + i)];
+                        if (key <= position) acc[d][i] = __fmaf_rn(weight, value, acc[d][i]);
+                    }
+            }
+        }
+#pragma unroll
+        for (int t = 0; t < 4; ++t) page[t] = next_page[t];
+        load_values(next, page, v);
+
+        if (tile % kRowwiseChunk == kRowwiseChunk - kWave || tile + kWave > last_position) {       // the chunk's last tile
+            const bool some = tile / kRowwiseChunk * kRowwiseChunk <= position;
+            float merged_max, keep, add;
+            merge_scales(total_max, chunk_max, merged_max, keep, add);
+            total_sum = some ? merged(total_sum, keep, chunk_sum, add) : total_sum;
+            total_max = some ? merged_max : total_max;
+#pragma unroll
+            for (int d = 0; d < HD_TILES; ++d)
+#pragma unroll
+                for (int i = 0; i < 4; ++i) {
+                    total[d][i] = some ? merged(total[d][i], keep, acc[d][i], add) : total[d][i];
+                    acc[d][i] = 0.0f;
+                }
+            chunk_max = -INFINITY;
+            chunk_sum = 0.0f;
+        }
+    }
+    const float inverse = 1.0f / total_sum;
+#pragma unroll
+    for (int d = 0; d < HD_TILES; ++d) {
+        floatx4 result;
+#pragma unroll
+        for (int i = 0; i < 4; ++i) result[i] = __fmul_rn(total[d][i], inverse);
+        if (col < count) *reinterpret_cast<floatx4*>(out + (static_cast<int64_t>(token) * heads + head) * HD + 16 * d + 4 * quad) = result;
+    }
+    }
+}
+
 // How many query heads of a kv head one wave of the kernel above takes in a step of `rows` (token, kv head, chunk)
 // items: as many as leave the GPU its waves, of the counts that fill the group's waves evenly (7 heads: 7, or 4
 // and 3, or 2, 2, 2 and 1; not 5 and 2). One: the kernel for one head a wave.
@@ -472,7 +747,7 @@ static int launch_rowwise_dims(const void* q, const void* k_cache, const void* v
         paged_attention_rowwise_heads_kernel<T, MODE, DIMS, GW><<<heads_grid, kWave, 0, stream>>>(                      \
             static_cast<const T*>(q), static_cast<const T*>(k_cache), static_cast<const T*>(v_cache), block_table,    \
             table_width, seq_of_token, positions, static_cast<T*>(out), part_o, part_ml, max_chunks, scale, window,   \
-            heads, kv_heads, head_dim, page_size);                                                                     \
+            heads, kv_heads, head_dim, page_size, runs_apart);                                                         \
         break;
 #define MLL_ROWWISE_HEADS_ALL(MODE)                                                                                    \
     switch (gw) {                                                                                                      \
@@ -480,7 +755,29 @@ static int launch_rowwise_dims(const void* q, const void* k_cache, const void* v
         MLL_ROWWISE_HEADS(MODE, 6) MLL_ROWWISE_HEADS(MODE, 7) MLL_ROWWISE_HEADS(MODE, 8)                               \
         default: break;                                                                                                \
     }
+    int runs_apart = 0;
     if (max_chunks == 0) {
+        if constexpr (std::is_same<T, float>::value && DIMS <= 2) {
+            if (window == 0 && head_dim % 16 == 0) {
+                runs_apart = 1;
+                const int64_t units = static_cast<int64_t>((n_tokens + kRunTokens - 1) / kRunTokens) * heads;
+                MLL_REQUIRE(units < (static_cast<int64_t>(1) << 31) - 4, "paged_attention: too many rows for one call");
+                const dim3 run_grid((units + 3) / 4);
+#define MLL_ROWWISE_RUNS(TILES)                                                                                        \
+    case TILES:                                                                                                        \
+        paged_attention_rowwise_runs_kernel<TILES><<<run_grid, 256, 0, stream>>>(                                      \
+            static_cast<const T*>(q), static_cast<const T*>(k_cache), static_cast<const T*>(v_cache), block_table, table_width, seq_of_token, \
+            positions, static_cast<T*>(out), scale, n_tokens, heads, kv_heads, page_size);                            \
+        break;
+                switch (head_dim / 16) {
+                    MLL_ROWWISE_RUNS(1) MLL_ROWWISE_RUNS(2) MLL_ROWWISE_RUNS(3) MLL_ROWWISE_RUNS(4)
+                    MLL_ROWWISE_RUNS(5) MLL_ROWWISE_RUNS(6) MLL_ROWWISE_RUNS(7) MLL_ROWWISE_RUNS(8)
+                    default: break;
+                }
+#undef MLL_ROWWISE_RUNS
+                if (const int status = check_launch("paged_attention_rowwise")) return status;
+            }
+        }
         if constexpr (std::is_same<T, float>::value && DIMS <= 2) {
             if (several_heads) {
                 const dim3 heads_grid(n_tokens, group_waves);
@@ -491,7 +788,7 @@ static int launch_rowwise_dims(const void* q, const void* k_cache, const void* v
         paged_attention_rowwise_kernel<T, 0, DIMS><<<dim3(n_tokens, heads), kWave, 0, stream>>>(
             static_cast<const T*>(q), static_cast<const T*>(k_cache), static_cast<const T*>(v_cache), block_table,
             table_width, seq_of_token, positions, static_cast<T*>(out), nullptr, nullptr, 0, scale, window, heads,
-            kv_heads, head_dim, page_size);
+            kv_heads, head_dim, page_size, runs_apart);
         return check_launch("paged_attention_rowwise");
     }
     // Several query heads of a kv head in one wave where the step still has rows enough for the GPU that way
@@ -508,7 +805,7 @@ static int launch_rowwise_dims(const void* q, const void* k_cache, const void* v
         paged_attention_rowwise_kernel<T, 1, DIMS><<<dim3(n_tokens, heads, max_chunks), kWave, 0, stream>>>(
             static_cast<const T*>(q), static_cast<const T*>(k_cache), static_cast<const T*>(v_cache), block_table,
             table_width, seq_of_token, positions, static_cast<T*>(out), part_o, part_ml, max_chunks, scale, window, heads,
-            kv_heads, head_dim, page_size);
+            kv_heads, head_dim, page_size, 0);
     if (const int status = check_launch("paged_attention_rowwise")) return status;
     paged_attention_rowwise_merge_kernel<T, DIMS><<<dim3(n_tokens, heads), kWave, 0, stream>>>(
         part_o, part_ml, seq_of_token, positions, static_cast<T*>(out), max_chunks, window, heads, head_dim);
