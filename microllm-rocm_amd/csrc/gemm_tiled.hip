@@ -116,14 +116,15 @@ __device__ __attribute__((always_inline)) inline void operands_arrived(TiledOper
 
 // EPILOGUE: 0 = float32 [M, N]; 1 = bfloat16 [M, N]; 2 = bfloat16 [M, N / 2] = silu(even rows of W) * (odd rows);
 // 3 = queries, keys and values: bias, rotation, queries to `store.q_out`, keys and values into their pages (W's rows
-// in rotary pair order; see MllQkvStore).
+// in rotary pair order; see MllQkvStore); 5 = 2 with GELU; 7 = 2 with clamped gates, from the float32 sums (`limit`, `slope`).
 // WM: a workgroup's tile of C has 32 WM rows (a wave WM row tiles of 16), 4 to 8: fewer where 256 rows a tile would
 // leave many compute units without one.
 // With epilogue 0 the stages of k may be dealt to gridDim.y workgroups, each writing its own [M, N] of partial sums.
 template <int EPILOGUE, int WM>
 __global__ __launch_bounds__(kTiledThreads, 1) void gemm_tiled_kernel(const bf16* __restrict__ a, const bf16* __restrict__ w_packed,
                                                                       void* __restrict__ out, int m, int n, int k, int n_tiles,
-                                                                      int k_steps, int m_blocks, int n_blocks, MllQkvStore store) {
+                                                                      int k_steps, int m_blocks, int n_blocks, MllQkvStore store,
+                                                                      float limit, float slope) {
     static_assert(WM >= 4 && WM <= kMaxWaveTilesM, "a wave takes 4 to 8 row tiles");
     constexpr int TILE_M = 32 * WM;
     constexpr int A_LOADS = 4 * WM;                       // a stage of A: 2 WM pieces of 16 rows, two loads of 8 rows each
@@ -358,16 +359,19 @@ __global__ __launch_bounds__(kTiledThreads, 1) void gemm_tiled_kernel(const bf16
                         if (column + i < n) target[i] = from_float<bf16>(acc[nt][mt][i]);
                 }
             } else {
+                auto gated = [&](float gate, float up) {
+                    return EPILOGUE == 7 ? gated_value(gate, up, kActClampedGlu, limit, slope) : gate_fast<EPILOGUE == 5>(gate) * up;
+                };
                 bf16* target = static_cast<bf16*>(out) + static_cast<int64_t>(row) * (n / 2) + column / 2;
                 if (column + 3 < n && n % 4 == 0) {
                     bf16x2 two;
 #pragma unroll
-                    for (int i = 0; i < 2; ++i) two[i] = static_cast<__bf16>(gate_fast<EPILOGUE == 5>(acc[nt][mt][2 * i]) * acc[nt][mt][2 * i + 1]);
+                    for (int i = 0; i < 2; ++i) two[i] = static_cast<__bf16>(gated(acc[nt][mt][2 * i], acc[nt][mt][2 * i + 1]));
                     *reinterpret_cast<bf16x2*>(target) = two;
                 } else {
 #pragma unroll
                     for (int i = 0; i < 4; i += 2)
-                        if (column + i < n) target[i / 2] = from_float<bf16>(gate_fast<EPILOGUE == 5>(acc[nt][mt][i]) * acc[nt][mt][i + 1]);
+                        if (column + i < n) target[i / 2] = from_float<bf16>(gated(acc[nt][mt][i], acc[nt][mt][i + 1]));
                 }
             }
         }
@@ -376,12 +380,12 @@ __global__ __launch_bounds__(kTiledThreads, 1) void gemm_tiled_kernel(const bf16
 
 template <int EPILOGUE, int WM>
 static int launch_tiled_rows(const void* a, const void* w_packed, void* out, int m, int n, int k, int splits, hipStream_t stream,
-                             const MllQkvStore& store) {
+                             const MllQkvStore& store, float limit, float slope) {
     const int n_tiles = (n + 15) / 16, k_steps = k / 32;
     const int m_blocks = (m + 32 * WM - 1) / (32 * WM), n_blocks = (n + kTileN - 1) / kTileN;
     const dim3 grid(8 * ((m_blocks * n_blocks + 7) / 8), splits);
     gemm_tiled_kernel<EPILOGUE, WM><<<grid, kTiledThreads, 0, stream>>>(static_cast<const bf16*>(a), static_cast<const bf16*>(w_packed),
-                                                                        out, m, n, k, n_tiles, k_steps, m_blocks, n_blocks, store);
+                                                                        out, m, n, k, n_tiles, k_steps, m_blocks, n_blocks, store, limit, slope);
     return check_launch("gemm_tiled");
 }
 
@@ -403,13 +407,13 @@ static int choose_tile_rows(int m, int n, int splits) {
 
 template <int EPILOGUE>
 static int launch_tiled(const void* a, const void* w_packed, void* out, int m, int n, int k, int splits, int tile_rows,
-                        hipStream_t stream, const MllQkvStore& store = MllQkvStore{}) {
+                        hipStream_t stream, const MllQkvStore& store = MllQkvStore{}, float limit = 0.0f, float slope = 0.0f) {
     if (tile_rows == 0) tile_rows = choose_tile_rows(m, n, splits);
     switch (tile_rows) {
-        case 256: return launch_tiled_rows<EPILOGUE, 8>(a, w_packed, out, m, n, k, splits, stream, store);
-        case 192: return launch_tiled_rows<EPILOGUE, 6>(a, w_packed, out, m, n, k, splits, stream, store);
-        case 160: return launch_tiled_rows<EPILOGUE, 5>(a, w_packed, out, m, n, k, splits, stream, store);
-        case 128: return launch_tiled_rows<EPILOGUE, 4>(a, w_packed, out, m, n, k, splits, stream, store);
+        case 256: return launch_tiled_rows<EPILOGUE, 8>(a, w_packed, out, m, n, k, splits, stream, store, limit, slope);
+        case 192: return launch_tiled_rows<EPILOGUE, 6>(a, w_packed, out, m, n, k, splits, stream, store, limit, slope);
+        case 160: return launch_tiled_rows<EPILOGUE, 5>(a, w_packed, out, m, n, k, splits, stream, store, limit, slope);
+        case 128: return launch_tiled_rows<EPILOGUE, 4>(a, w_packed, out, m, n, k, splits, stream, store, limit, slope);
         default: return fail("gemm_tiled: a tile has 256, 192, 160 or 128 rows (0: chosen here)");
     }
 }
@@ -436,6 +440,16 @@ extern "C" int mll_gemm_tiled(const void* a, const void* w_packed, void* out, in
         case 5: return launch_tiled<5>(a, w_packed, out, m, n, k, splits, tile_rows, stream);
         default: return fail("gemm_tiled: unknown epilogue");
     }
+}
+
+extern "C" int mll_gemm_tiled_clamped(const void* a, const void* w_packed, void* out, int m, int n, int k, float limit, float slope,
+                                      int tile_rows, hipStream_t stream) {
+    MLL_REQUIRE(m >= 0 && n > 0 && n % 2 == 0 && k > 0 && k % 32 == 0, "gemm_tiled_clamped: an even number of weight rows, k a multiple of 32");
+    MLL_REQUIRE(static_cast<int64_t>(kTileN) * k < (int64_t{1} << 30), "gemm_tiled_clamped: k is too long");
+    MLL_REQUIRE(reinterpret_cast<uintptr_t>(a) % 16 == 0, "gemm_tiled_clamped: the activations must be 16-byte aligned");
+    MLL_REQUIRE(limit > 0.0f, "gemm_tiled_clamped: the limit must be positive");
+    if (m == 0) return 0;
+    return launch_tiled<7>(a, w_packed, out, m, n, k, 1, tile_rows, stream, MllQkvStore{}, limit, slope);
 }
 
 extern "C" int mll_gemm_tiled_qkv(const void* a, const void* w_packed, int m, int k, const MllQkvStore* store, int tile_rows,

@@ -237,6 +237,9 @@ int mll_gemm_medium(const void* a, const void* w_packed, void* out, int epilogue
 int mll_gemm_tiled(const void* a, const void* w_packed, void* out, int epilogue, int m, int n, int k,
                    int splits, int tile_rows, hipStream_t stream);
 int mll_tiled_tile_rows(int m, int n, int splits);
+// The gated product finished as mll_clamped_glu does (interleaved rows): bfloat16 out [m, n / 2].
+int mll_gemm_tiled_clamped(const void* a, const void* w_packed, void* out, int m, int n, int k, float limit, float slope,
+                           int tile_rows, hipStream_t stream);
 // Queries, keys and values of many rows: the tiled product finished as mll_gemm_skinny_qkv finishes its own (the
 // same MllQkvStore, the weight in rotary pair order). k a multiple of 32, store->n_freq even, no rows' factors; a
 // workgroup owns a whole tile of the result and the reduction is never taken in parts.

@@ -1177,13 +1177,32 @@ def tiled_fill(m: int, n: int, splits: int = 1) -> float:
     return blocks / (-(-blocks // COMPUTE_UNITS) * COMPUTE_UNITS)
 
 
+def tiled_gated_pays(rows: int, k: int, from_float: bool = False) -> bool:
+    """Whether a gated product (gate, up and activation) of this many rows is the tiled kernel's although the weight is also
+    kept as stored. Its epilogue saves the library's product a pass over twice the result, and its rate moves less with the
+    number of rows: against the untuned library and the activation's kernel (MI355X, time of those over this one's) 37888 x
+    3584 at 768, 1024, 1280, 1536, 2048, 3072 and 4096 rows 0.95, 1.18, 1.37, 0.99, 1.20, 1.11 and 0.96; 16384 x 2048 at 256,
+    512, 1024, 2048, 3072 and 4096 0.94, 1.14, 1.13, 1.02, 0.99 and 0.96; 9728 x 896 at 192, 256, 512, 2048 and 4096 0.90, 1.04, 1.26, 1.45 and 1.21.
+    Where the activation takes the float32 sums (``from_float``: clamped gates), the library's way writes and reads twice as
+    much and has no upper line: 37888 x 3584 at 768, 1024, 3072 and 8192 rows 1.07, 1.11, 1.27 and 1.23; 16384 x 2048 at 256, 512,
+    3584 and 8192 0.97, 1.10, 1.22 and 1.30; 9728 x 896 at 192, 256 and 8192 0.92, 1.08 and 1.56.
+    A tuned library is 3 to 8 % faster than the tiled kernel where it matters most and keeps the product. The lines lie where
+    no step's rows and the rows it is padded to (multiples of 64, above 1024 of 256) fall on different sides."""
+    if library_tuning() or k % 32 != 0:
+        return False
+    if k <= 1024:
+        return 192 < rows and (from_float or rows <= 4096)
+    return (448 if k <= 2048 else 960) < rows and (from_float or rows <= 3072)
+
+
 def gemm_tiled(x: torch.Tensor, packed: torch.Tensor, n: int, epilogue: str = "f32", splits: int = 1,
-               tile_rows: int = 0) -> torch.Tensor:
+               tile_rows: int = 0, limit: float = 0.0, slope: float = 0.0) -> torch.Tensor:
     """``x @ W.T`` for many bfloat16 rows and a packed weight, on this package's tiled MFMA kernel (0.9 to 1.1 of
     the library's untuned rate at 2048 rows and more, 1.1 to 1.4 PFLOP/s: for weights that are kept in the packed
-    order alone). ``k`` must be
+    order alone, and for gated products where ``tiled_gated_pays``). ``k`` must be
     a multiple of 32. With ``splits`` > 1 (float32 only) the result is ``[splits, m, n]`` sums over parts of the
-    reduction for the caller to add in order."""
+    reduction for the caller to add in order. ``epilogue`` ``clamped``: bfloat16 ``[m, n / 2]`` as ``clamped_glu`` makes it of
+    interleaved rows, with ``limit`` and ``slope``."""
     lib = library.load()
     _device_tensor(x, "gemm input", torch.bfloat16)
     _device_tensor(packed, "packed weight", torch.bfloat16)
@@ -1191,7 +1210,7 @@ def gemm_tiled(x: torch.Tensor, packed: torch.Tensor, n: int, epilogue: str = "f
     m, k = x.shape
     _need(k % 32 == 0, "gemm_tiled needs k to be a multiple of 32")
     _need(packed.shape[0] == -(-n // 16) and packed.shape[1] == k // 32, "the packed weight does not fit n and k")
-    _need(epilogue not in ("gated", "gated_gelu") or n % 2 == 0, "the gated epilogue needs an even number of weight rows")
+    _need(epilogue not in ("gated", "gated_gelu", "clamped") or n % 2 == 0, "the gated epilogue needs an even number of weight rows")
     _need(splits >= 1 and (splits == 1 or epilogue == "f32"), "only the float32 epilogue takes the reduction in parts")
     if epilogue == "f32":
         code, out = 0, torch.empty((m, n) if splits == 1 else (splits, m, n), dtype=torch.float32, device=x.device)
@@ -1201,6 +1220,11 @@ def gemm_tiled(x: torch.Tensor, packed: torch.Tensor, n: int, epilogue: str = "f
         code, out = 2, torch.empty((m, n // 2), dtype=torch.bfloat16, device=x.device)
     elif epilogue == "gated_gelu":
         code, out = 5, torch.empty((m, n // 2), dtype=torch.bfloat16, device=x.device)
+    elif epilogue == "clamped":
+        out = torch.empty((m, n // 2), dtype=torch.bfloat16, device=x.device)
+        _check(lib.mll_gemm_tiled_clamped(_ptr(x), _ptr(packed), _ptr(out), m, n, k, ctypes.c_float(limit), ctypes.c_float(slope), tile_rows,
+                                          _stream()), lib)
+        return out
     else:
         raise KernelLibraryError(f"unknown epilogue {epilogue!r}")
     _check(lib.mll_gemm_tiled(_ptr(x), _ptr(packed), _ptr(out), code, m, n, k, splits, tile_rows, _stream()), lib)

@@ -102,10 +102,13 @@ def takes_packed(weight: "Weight", rows: int, gated: bool = False) -> bool:
 
 def linear_clamped_glu(x: torch.Tensor, weight: "Weight", limit: float, slope: float) -> torch.Tensor:
     """``g * sigmoid(slope * g) * (u + 1)`` of half the width, in x's dtype, with ``g = min(gate, limit)`` and ``u = clamp(up,
-    -limit, limit)`` of a gated weight's product (rows ``[gate; up]``): in the product's epilogue for few rows, else from its
-    float32 sums, rounded once."""
+    -limit, limit)`` of a gated weight's product (rows ``[gate; up]``): in the product's epilogue for few rows and where
+    ``kernels.tiled_gated_pays``, else from its float32 sums, rounded once."""
     if x.dtype == torch.bfloat16 and weight.packed is not None and weight.gated and x.shape[0] <= SKINNY_ROWS:
         return kernels.gemm_skinny_clamped(x, weight.packed, weight.out_features, limit, slope)
+    if (x.dtype == torch.bfloat16 and weight.packed is not None and weight.gated and x.shape[0] > MEDIUM_ROWS
+            and kernels.tiled_gated_pays(x.shape[0], weight.in_features, from_float=True)):
+        return kernels.gemm_tiled(x, weight.packed, weight.out_features, "clamped", limit=limit, slope=slope)
     # the packed copy's rows, and so its products' columns, hold gate and up by turns
     by_turns = weight.gated and x.dtype == weight.dtype and takes_packed(weight, x.shape[0])
     return kernels.clamped_glu(linear(x, weight, out_dtype=torch.float32), limit, slope, x.dtype, interleaved=by_turns)
@@ -164,6 +167,8 @@ def linear(x: Union[torch.Tensor, UnscaledRows], weight, out_dtype: Optional[tor
             return kernels.gemm_medium(x, weight.packed, weight.out_features, "f32", plan=plan)
         return kernels.gemm_medium(x, weight.packed, weight.out_features, "bf16")
     if gated:
+        if weight.packed is not None and weight.gated and kernels.tiled_gated_pays(rows, weight.in_features):
+            return kernels.gemm_tiled(x, weight.packed, weight.out_features, gate)
         return kernels.gated_activation(kernels.gemm_bf16(x, w, torch.bfloat16), activation)
     if partials and out_dtype == torch.float32:
         parts = kernels.library_splits(rows, weight.out_features, weight.in_features)

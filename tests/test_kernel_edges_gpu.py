@@ -1,0 +1,86 @@
+"""The kernels at the sizes where their tiles, their remainders and the choice between them can go wrong."""
+import math
+
+import numpy as np
+import pytest
+import torch
+
+from test_kernels_gpu import DEVICE, build_paged_case, kernels, reference_attention, to_bf16_exact
+
+pytestmark = pytest.mark.gpu
+
+F32_STEP = 2.0 ** -24       # half a unit in the last place, relative
+
+
+def device(values, dtype=torch.float32):
+    return torch.as_tensor(np.asarray(values)).to(dtype).to(DEVICE)
+
+
+@pytest.mark.parametrize("n", [16, 2048, 2049, 2064, 16384, 16400, 32768])      # 128 | 129 tiles (half ones below), 1024, 2048
+@pytest.mark.parametrize("k", [8, 32, 480, 544, 4128])
+def test_streaming_product_tiles(n, k):
+    """Any float32 sum of exact bfloat16 products errs by at most k roundings of the sum of their sizes; a row's bits are the
+    same in every batch."""
+    rng = np.random.default_rng(n + k)
+    x_exact, x = to_bf16_exact(rng.normal(size=(16, k)))
+    w_exact, w = to_bf16_exact(rng.normal(size=(n, k)))
+    packed = kernels().pack_weight(w)
+    whole = kernels().gemm_skinny(x, packed, n, "f32")
+    bound = (k + 1) * F32_STEP * (np.abs(x_exact) @ np.abs(w_exact).T)
+    assert (np.abs(whole.double().cpu().numpy() - x_exact @ w_exact.T) <= bound).all()
+    for m in (1, 4, 5, 8, 9):
+        assert torch.equal(kernels().gemm_skinny(x[:m].contiguous(), packed, n, "f32"), whole[:m]), m
+
+
+@pytest.mark.parametrize("n,k", [(331, 120), (896, 901), (4096, 64), (1000, 1536)])
+def test_float32_product_has_one_order_of_sums_in_every_kernel(n, k):
+    """Few rows, tiles of four shapes and small tiles for few workgroups: each element is the chain of fused multiply-adds in
+    ascending k, so every batch gives a row the same bits."""
+    rng = np.random.default_rng(n)
+    a = device(rng.normal(size=(1003, k)))
+    w = device(rng.normal(size=(n, k)))
+    whole = kernels().gemm_f32(a, w)
+    bound = (k + 1) * F32_STEP * (a.abs().double() @ w.abs().double().T)
+    assert bool(((whole.double() - a.double() @ w.double().T).abs() <= bound).all())
+    for rows in (1, 2, 15, 16, 17, 31, 33, 64, 65, 127, 129, 320):
+        assert torch.equal(kernels().gemm_f32(a[1003 - rows:].contiguous(), w), whole[1003 - rows:]), rows
+
+
+@pytest.mark.parametrize("heads,kv_heads,hd,page_size", [(4, 2, 16, 16), (7, 1, 128, 16), (3, 3, 48, 48), (12, 2, 112, 32)])
+@pytest.mark.parametrize("broken", [None, float("inf"), float("nan")])
+def test_runs_of_a_requests_tokens_have_a_tokens_bits(heads, kv_heads, hd, page_size, broken):
+    """Portions that end before, on and after a stretch of 16, alone and several to a block of 16 tokens, against each of the
+    same tokens alone; and a value that is not finite changes the tokens after it alone."""
+    rng = np.random.default_rng(hd)
+    lengths, counts = [300, 16, 17, 140, 40, 5, 129, 33, 64], [290, 16, 17, 1, 2, 5, 31, 15, 48]
+    t, q_exact, ek, ev, seq, pos = build_paged_case(rng, torch.float32, lengths, counts, heads, kv_heads, hd, page_size)
+    scale = 1.0 / math.sqrt(hd)
+    if broken is not None:
+        at = 150        # of the first request: seen by its later tokens alone
+        block, offset = t["table"][0, at // page_size].item(), at % page_size
+        from microllm_rocm_amd.cache.layout import value_rows, write_value_rows
+        rows = value_rows(t["v"], hd).clone()
+        rows[block, :, offset, 1] = broken
+        write_value_rows(t["v"], rows)
+    run = lambda index: kernels().paged_attention_rowwise(t["q"][index].contiguous(), t["k"], t["v"], t["table"], t["seq"][index].contiguous(),
+                                                          t["pos"][index].contiguous(), scale, 0, heads, kv_heads, hd)
+    together = run(slice(None))
+    alone = torch.cat([run(slice(token, token + 1)) for token in range(len(pos))])
+    assert torch.equal(torch.nan_to_num(together, 7.0, 8.0, 9.0), torch.nan_to_num(alone, 7.0, 8.0, 9.0))
+    reference = reference_attention(q_exact, ek, ev, seq, pos, heads, kv_heads, hd, scale, 0)
+    sound = ~((seq == 0) & (pos >= 150)) if broken is not None else np.ones(len(pos), dtype=bool)
+    np.testing.assert_allclose(together.cpu().numpy()[sound], reference[sound], rtol=1e-5, atol=1e-5)
+
+
+@pytest.mark.parametrize("m,width,k,tile_rows", [(65, 24, 32, 0), (129, 200, 544, 0), (300, 129, 64, 0), (300, 512, 96, 128)])
+def test_tiled_product_with_clamped_gates(m, width, k, tile_rows):
+    """From the float32 sums, rounded once: half a unit of bfloat16 beside what the sums' own errors come to."""
+    rng = np.random.default_rng(m)
+    x_exact, x = to_bf16_exact(rng.normal(size=(m, k)))
+    w_exact, w = to_bf16_exact(rng.normal(size=(2 * width, k)) * 0.3)
+    got = kernels().gemm_tiled(x, kernels().pack_weight(w, interleave_halves=True), 2 * width, "clamped", tile_rows=tile_rows, limit=2.5, slope=1.7)
+    product = x_exact @ w_exact.T
+    gate, up = np.minimum(product[:, :width], 2.5), np.clip(product[:, width:], -2.5, 2.5)
+    want = gate / (1.0 + np.exp(-1.7 * gate)) * (up + 1.0)
+    assert (np.abs(got.double().cpu().numpy() - want) <= 2.0 ** -8 * np.abs(want) + 1e-4).all()
+    assert float(got.float().abs().max()) > 1.0
