@@ -22,20 +22,43 @@ namespace mll {
 constexpr int kWideHeadRows = 8;
 constexpr int kUsualRows = 4;
 
-// decay[t, c] = exp(log_sigmoid(z) / tau), z = bias[c] + sum_r a2[c, r] * low[t, r]
+// decay[t, c] = exp(log_sigmoid(z) / tau), z = bias[c] + sum_r a2[c, r] * low[t, r]; with `base_two` the exponent's
+// logarithm to base two instead. A thread keeps its channel's row of a2 for kDecayTokens tokens (a row apiece for every token
+// and channel were 2-byte loads a row apart: 3117 tokens of 512 channels 60 -> 18 us), 16 numbers of it at a time.
+constexpr int kDecayTokens = 8;
+constexpr int kDecayRank = 16;
 template <typename W>
-__global__ void gla_decay_kernel(const float* __restrict__ proj, int64_t proj_stride, int low_offset, int rank,
-                                 const W* __restrict__ a2, const float* __restrict__ bias, float inv_tau,
-                                 float* __restrict__ decay, int channels) {
-    const int token = blockIdx.y;
+__global__ void __launch_bounds__(128)
+gla_decay_kernel(const float* __restrict__ proj, int64_t proj_stride, int low_offset, int rank,
+                 const W* __restrict__ a2, const float* __restrict__ bias, float inv_tau,
+                 float* __restrict__ decay, int channels, int n_tokens, int base_two) {
+    const int first = blockIdx.y * kDecayTokens;
     const int c = blockIdx.x * blockDim.x + threadIdx.x;
     if (c >= channels) return;
-    const float* low = proj + static_cast<int64_t>(token) * proj_stride + low_offset;
-    float z = bias ? bias[c] : 0.0f;
-    for (int r = 0; r < rank; ++r) z = fmaf(to_float(a2[static_cast<int64_t>(c) * rank + r]), low[r], z);
-    // log(sigmoid(z)) = -(max(-z, 0) + log1p(exp(-|z|)))
-    const float log_sigmoid = -(fmaxf(-z, 0.0f) + log1pf(expf(-fabsf(z))));
-    decay[static_cast<int64_t>(token) * channels + c] = expf(log_sigmoid * inv_tau);
+    float z[kDecayTokens];
+#pragma unroll
+    for (int t = 0; t < kDecayTokens; ++t) z[t] = bias ? bias[c] : 0.0f;
+    for (int r0 = 0; r0 < rank; r0 += kDecayRank) {
+        float weight[kDecayRank];       // past the row: zero times its last number
+#pragma unroll
+        for (int r = 0; r < kDecayRank; ++r) {
+            const float value = to_float(a2[static_cast<int64_t>(c) * rank + min(r0 + r, rank - 1)]);
+            weight[r] = r0 + r < rank ? value : 0.0f;
+        }
+#pragma unroll
+        for (int t = 0; t < kDecayTokens; ++t) {
+            const float* low = proj + static_cast<int64_t>(min(first + t, n_tokens - 1)) * proj_stride + low_offset;
+#pragma unroll
+            for (int r = 0; r < kDecayRank; ++r) z[t] = fmaf(weight[r], low[min(r0 + r, rank - 1)], z[t]);
+        }
+    }
+#pragma unroll
+    for (int t = 0; t < kDecayTokens; ++t) {
+        if (first + t >= n_tokens) break;
+        // log(sigmoid(z)) = -(max(-z, 0) + log1p(exp(-|z|)))
+        const float log_sigmoid = -(fmaxf(-z[t], 0.0f) + log1pf(expf(-fabsf(z[t]))));
+        decay[static_cast<int64_t>(first + t) * channels + c] = base_two ? log_sigmoid * inv_tau * 1.44269504088896340736f : expf(log_sigmoid * inv_tau);
+    }
 }
 
 // One wave a (request, head, group of value channels). lane = column_in_group * lanes_a_column + r; lane r of a
@@ -316,18 +339,18 @@ using namespace mll;
 extern "C" {
 
 int mll_gla_decay(const float* proj, int64_t proj_stride, int low_offset, int rank, const void* a2, int a2_dtype,
-                  const float* bias, float tau, float* decay, int n_tokens, int channels, hipStream_t stream) {
+                  const float* bias, float tau, float* decay, int n_tokens, int channels, int base_two, hipStream_t stream) {
     MLL_REQUIRE(n_tokens >= 0 && channels > 0 && rank > 0 && tau > 0.0f, "gla_decay: sizes and tau must be positive");
     MLL_REQUIRE(low_offset >= 0 && low_offset + rank <= proj_stride, "gla_decay: the low-rank input lies outside its row");
     if (n_tokens == 0) return 0;
     MLL_REQUIRE(n_tokens <= 65535, "gla_decay: more than 65535 tokens in one call");
-    const dim3 grid((channels + 127) / 128, n_tokens);
+    const dim3 grid((channels + 127) / 128, (n_tokens + kDecayTokens - 1) / kDecayTokens);
     if (a2_dtype == kF32) {
         gla_decay_kernel<float><<<grid, 128, 0, stream>>>(proj, proj_stride, low_offset, rank, static_cast<const float*>(a2), bias,
-                                                         1.0f / tau, decay, channels);
+                                                         1.0f / tau, decay, channels, n_tokens, base_two);
     } else if (a2_dtype == kBF16) {
         gla_decay_kernel<bf16><<<grid, 128, 0, stream>>>(proj, proj_stride, low_offset, rank, static_cast<const bf16*>(a2), bias,
-                                                        1.0f / tau, decay, channels);
+                                                        1.0f / tau, decay, channels, n_tokens, base_two);
     } else {
         return fail("gla_decay: unknown weight dtype");
     }

@@ -11,6 +11,16 @@
 // its own), and the results (all chunks at once). All products are float32 on the matrix units
 // (v_mfma_f32_16x16x4_f32); state, powers of the decay and sums are float32. A chunk begins at every 64th token of a
 // request's portion, so where a portion was cut changes a result by rounding alone.
+//
+// The kernels gla_channel_* do the same for a decay a key channel and token, a_t[d] = 2^(l_t[d]). With B_t[d] the sum of
+// l over the chunk's tokens up to t,
+//
+//   o_t = (2^B_t q_t)^T S + sum_{j <= t} (sum_d q_t[d] k_j[d] 2^(B_t[d] - B_j[d])) v_j,
+//
+// and a chunk leaves 2^B_n S + sum_j (2^(B_n - B_j) k_j) v_j^T. No power has a positive exponent, so none overflows whatever
+// the decays: 16 tokens among themselves take 2^(B_t - B_j) pair by pair, with those before them the query takes
+// 2^(B_t - B_r) and the key 2^(B_r - B_j), r being the last token before the 16. The sums are kept within parts of 16
+// tokens, so that a difference of two of them loses little.
 #include "common.h"
 #include "microllm_hip.h"
 
@@ -200,6 +210,250 @@ gla_chunk_out_kernel(const float* __restrict__ proj, int64_t proj_stride, int q_
     }
 }
 
+// ---- a decay a key channel and token -------------------------------------------------------------------------------
+// Two requests of 2000 and 1117 tokens, 8 heads of 64 x 128: 287 us by the walk, 73 here (results 47, states 15, walk over the
+// chunks 11), bound by one workgroup's chain of LDS reads and products. Sums run in four chains, which both shortens the waits and
+// keeps the error against float64 below the walk's: 1.25e-7 (root mean square, of the results') against 1.65e-7 at 512 tokens.
+constexpr int kChannelKeys = 64;        // the widest key heads here: queries, keys and decays of a chunk lie in LDS together
+
+constexpr int kPart = 16;
+constexpr int kParts = kScanChunk / kPart;
+
+// A chunk's logarithms. Below 2^-149 a factor is zero in float32, and a sum of larger numbers would lose the others' digits.
+__device__ inline float usable_log(float value) { return value < -150.0f ? -150.0f : value; }
+
+// `sums[t][c]`: logarithms to their sums from their part's first token on, in place; whole[part][c]: the part's sum. Called by
+// every thread; the first and last things it does are barriers.
+__device__ inline void sum_parts(float (*sums)[kChannelKeys + 1], float (*whole)[kChannelKeys]) {
+    const int c = threadIdx.x % kChannelKeys, part = threadIdx.x / kChannelKeys;
+    static_assert(kScanThreads == kParts * kChannelKeys, "a thread a channel and part");
+    __syncthreads();
+    float total = 0.0f;
+#pragma unroll
+    for (int t = 0; t < kPart; ++t) {
+        total += sums[kPart * part + t][c];
+        sums[kPart * part + t][c] = total;
+    }
+    whole[part][c] = total;
+    __syncthreads();
+}
+
+// whole[first] + .. + whole[last - 1] of channel c.
+__device__ inline float sum_between(float (*whole)[kChannelKeys], int first, int last, int c) {
+    float total = 0.0f;
+    for (int part = first; part < last; ++part) total += whole[part][c];
+    return total;
+}
+
+__device__ inline float power_of_two(float exponent) { return __builtin_amdgcn_exp2f(exponent); }
+
+// added[number][head][d][c] = sum_t 2^(B_n - B_t)[d] k_t[d] v_t[c]; whole[number][head][d] = 2^B_n[d].
+__global__ void __launch_bounds__(kScanThreads)
+gla_channel_state_kernel(const float* __restrict__ proj, int64_t proj_stride, int k_offset, int v_offset, const float* __restrict__ log_decay,
+                         const int32_t* __restrict__ cu_tokens, float* __restrict__ added, float* __restrict__ whole, int n_seqs, int heads,
+                         int key_dim, int value_dim) {
+    __shared__ float keys[kScanChunk][kChannelKeys + 1];
+    __shared__ float sums[kScanChunk][kChannelKeys + 1];
+    __shared__ float values[kScanChunk][kScanValues + 1];
+    __shared__ float parts[kParts][kChannelKeys];
+    const int number = blockIdx.x, head = blockIdx.y;
+    int seq, first, count;
+    if (!find_chunk(cu_tokens, n_seqs, number, &seq, &first, &count)) return;
+    const int lane = threadIdx.x % kWave, wave = threadIdx.x / kWave;
+    const int col = lane % 16, quad = lane / 16;
+    const float* row = proj + first * proj_stride;
+    load_tile<kScanChunk, kChannelKeys>(log_decay + (static_cast<int64_t>(first) * heads + head) * key_dim, static_cast<int64_t>(heads) * key_dim, count,
+                                        key_dim, [&](int t, int c, float value) { sums[t][c] = usable_log(value); });
+    load_tile<kScanChunk, kChannelKeys>(row + k_offset + head * key_dim, proj_stride, count, key_dim,
+                                        [&](int t, int c, float value) { keys[t][c] = value; });
+    sum_parts(sums, parts);
+    for (int index = threadIdx.x; index < kScanChunk * kChannelKeys; index += kScanThreads) {
+        const int t = index / kChannelKeys, c = index % kChannelKeys, part = t / kPart;
+        keys[t][c] *= power_of_two(parts[part][c] - sums[t][c] + sum_between(parts, part + 1, kParts, c));
+    }
+    if (threadIdx.x < key_dim)
+        whole[(static_cast<int64_t>(number) * heads + head) * key_dim + threadIdx.x] = power_of_two(sum_between(parts, 0, kParts, threadIdx.x));
+    float* to = added + (static_cast<int64_t>(number) * heads + head) * key_dim * value_dim;
+    for (int v0 = 0; v0 < value_dim; v0 += kScanValues) {
+        __syncthreads();      // the tile before has been read (the first time: the keys are there)
+        load_tile<kScanChunk, kScanValues>(row + v_offset + head * value_dim + v0, proj_stride, count, value_dim - v0,
+                                           [&](int t, int c, float value) { values[t][c] = value; });
+        __syncthreads();
+        const int column = v0 + 16 * wave + col;
+        for (int tile = 0; tile < (key_dim + 15) / 16; ++tile) {
+            floatx4 sum[kParts] = {};
+#pragma unroll
+            for (int t = 0; t < kPart; t += 4)
+#pragma unroll
+                for (int part = 0; part < kParts; ++part)
+                    sum[part] = __builtin_amdgcn_mfma_f32_16x16x4f32(keys[kPart * part + t + quad][16 * tile + col],
+                                                                     values[kPart * part + t + quad][16 * wave + col], sum[part], 0, 0, 0);
+            const floatx4 acc = (sum[0] + sum[1]) + (sum[2] + sum[3]);
+#pragma unroll
+            for (int i = 0; i < 4; ++i) {
+                const int d = 16 * tile + 4 * quad + i;
+                if (d < key_dim && column < value_dim) to[static_cast<int64_t>(d) * value_dim + column] = acc[i];
+            }
+        }
+    }
+}
+
+// gla_chunk_carry_kernel with a factor a chunk and key channel.
+__global__ void __launch_bounds__(256)
+gla_channel_carry_kernel(float* __restrict__ added, const float* __restrict__ whole, float* __restrict__ state,
+                         const int32_t* __restrict__ cu_tokens, const int32_t* __restrict__ slots, int heads, int key_dim, int value_dim) {
+    const int seq = blockIdx.x, head = blockIdx.y;
+    const int elements = key_dim * value_dim;
+    const int element = blockIdx.z * blockDim.x + threadIdx.x;
+    const int begin = cu_tokens[seq], tokens = cu_tokens[seq + 1] - begin;
+    if (tokens <= 0 || element >= elements) return;
+    const int chunks = (tokens + kScanChunk - 1) / kScanChunk;
+    const int64_t step = static_cast<int64_t>(heads) * elements, factor_step = static_cast<int64_t>(heads) * key_dim;
+    const int64_t base_number = begin / kScanChunk + seq;
+    float* place = added + (base_number * heads + head) * elements + element;
+    const float* factors = whole + (base_number * heads + head) * key_dim + element / value_dim;
+    float* kept = state + (static_cast<int64_t>(slots[seq]) * heads + head) * elements + element;
+    float s = *kept;
+    constexpr int kAtATime = 8;      // chunks asked for at a time, then walked in order
+    for (int base = 0; base < chunks; base += kAtATime) {
+        float more[kAtATime], factor[kAtATime];
+#pragma unroll
+        for (int j = 0; j < kAtATime; ++j) {
+            more[j] = base + j < chunks ? place[(base + j) * step] : 0.0f;
+            factor[j] = base + j < chunks ? factors[(base + j) * factor_step] : 0.0f;
+        }
+#pragma unroll
+        for (int j = 0; j < kAtATime; ++j)
+            if (base + j < chunks) {
+                place[(base + j) * step] = s;
+                s = fmaf(factor[j], s, more[j]);
+            }
+    }
+    *kept = s;
+}
+
+// The results of a chunk's tokens; wave w takes tokens 16 w .. 16 w + 15 of it.
+__global__ void __launch_bounds__(kScanThreads)
+gla_channel_out_kernel(const float* __restrict__ proj, int64_t proj_stride, int q_offset, int k_offset, int v_offset,
+                       const float* __restrict__ log_decay, const int32_t* __restrict__ cu_tokens, const float* __restrict__ starts,
+                       float* __restrict__ out, int n_seqs, int heads, int key_dim, int value_dim, float q_scale) {
+    __shared__ float queries[kScanChunk][kChannelKeys + 1];
+    __shared__ float keys[kScanChunk][kChannelKeys + 1];
+    __shared__ float sums[kScanChunk][kChannelKeys + 1];
+    __shared__ float weights[kScanChunk][kScanChunk + 1];
+    __shared__ float parts[kParts][kChannelKeys];
+    const int number = blockIdx.x, head = blockIdx.y;
+    int seq, first, count;
+    if (!find_chunk(cu_tokens, n_seqs, number, &seq, &first, &count)) return;
+    const int lane = threadIdx.x % kWave, wave = threadIdx.x / kWave;
+    const int col = lane % 16, quad = lane / 16;
+    const float* row = proj + first * proj_stride;
+    load_tile<kScanChunk, kChannelKeys>(log_decay + (static_cast<int64_t>(first) * heads + head) * key_dim, static_cast<int64_t>(heads) * key_dim, count,
+                                        key_dim, [&](int t, int c, float value) { sums[t][c] = usable_log(value); });
+    load_tile<kScanChunk, kChannelKeys>(row + q_offset + head * key_dim, proj_stride, count, key_dim,
+                                        [&](int t, int c, float value) { queries[t][c] = value; });
+    load_tile<kScanChunk, kChannelKeys>(row + k_offset + head * key_dim, proj_stride, count, key_dim,
+                                        [&](int t, int c, float value) { keys[t][c] = value; });
+    sum_parts(sums, parts);
+    const int own = kPart * wave + col;     // the token whose query this lane holds as a row of the first operand
+    // weights[t][j] = sum_d q_t[d] k_j[d] 2^(B_t[d] - B_j[d]) for j <= t: the wave's tokens among themselves, four pairs a lane ...
+    {
+        float pair[4][4] = {};      // the sums over the channels, in four parts
+        for (int d0 = 0; d0 < key_dim; d0 += 4)
+#pragma unroll
+            for (int d = 0; d < 4; ++d) {       // channels past the head are zero
+                const float q = queries[own][d0 + d], b = sums[own][d0 + d];
+#pragma unroll
+                for (int i = 0; i < 4; ++i) {
+                    const int j = kPart * wave + 4 * quad + i;
+                    pair[d][i] = fmaf(q * keys[j][d0 + d], power_of_two(fminf(b - sums[j][d0 + d], 0.0f)), pair[d][i]);
+                }
+            }
+#pragma unroll
+        for (int i = 0; i < 4; ++i) weights[own][kPart * wave + 4 * quad + i] = 4 * quad + i <= col ? (pair[0][i] + pair[1][i]) + (pair[2][i] + pair[3][i]) : 0.0f;
+    }
+    // ... and with the parts before them
+    float reaching[kChannelKeys / 4];       // 2^(B_t - B_r) q_t
+#pragma unroll
+    for (int d = 0; d < kChannelKeys; d += 4) reaching[d / 4] = queries[own][d + quad] * power_of_two(sums[own][d + quad]);
+    for (int part = 0; part < wave; ++part) {
+        floatx4 sum[4] = {};
+#pragma unroll
+        for (int d = 0; d < kChannelKeys; d += 4) {
+            const int c = d + quad, j = kPart * part + col;
+            const float k = keys[j][c] * power_of_two(parts[part][c] - sums[j][c] + sum_between(parts, part + 1, wave, c));
+            sum[d / 4 % 4] = __builtin_amdgcn_mfma_f32_16x16x4f32(reaching[d / 4], k, sum[d / 4 % 4], 0, 0, 0);
+        }
+        const floatx4 acc = (sum[0] + sum[1]) + (sum[2] + sum[3]);
+#pragma unroll
+        for (int i = 0; i < 4; ++i) weights[kPart * wave + 4 * quad + i][kPart * part + col] = acc[i];
+    }
+    const float* from = starts + (static_cast<int64_t>(number) * heads + head) * key_dim * value_dim;
+    float decayed[kChannelKeys / 4];        // 2^B_t q_t: the operand that meets the state
+#pragma unroll
+    for (int d = 0; d < kChannelKeys; d += 4) decayed[d / 4] = queries[own][d + quad] * power_of_two(sums[own][d + quad] + sum_between(parts, 0, wave, d + quad));
+    float own_weight[kPart / 4];            // the weights of the wave's tokens among themselves
+#pragma unroll
+    for (int j = 0; j < kPart / 4; ++j) own_weight[j] = weights[own][kPart * wave + 4 * j + quad];
+    float weight[kScanChunk / 4 - kPart / 4];       // and with those of the parts before them: rows that the wave wrote itself
+#pragma unroll
+    for (int j = 0; j < kScanChunk - kPart; j += 4) weight[j / 4] = j < kPart * wave ? weights[own][j + quad] : 0.0f;
+    // Queries and keys are done with: the state and the values take their place.
+    float (*start)[kScanValues + 1] = queries;
+    float (*values)[kScanValues + 1] = keys;
+    static_assert(kScanValues == kChannelKeys, "one shape");
+    for (int v0 = 0; v0 < value_dim; v0 += kScanValues) {
+        __syncthreads();      // the tile before has been read (the first time: queries and keys have, and the weights are there)
+        load_tile<kScanChunk, kScanValues>(row + v_offset + head * value_dim + v0, proj_stride, count, value_dim - v0,
+                                           [&](int t, int c, float value) { values[t][c] = value; });
+        load_tile<kChannelKeys, kScanValues>(from + v0, value_dim, key_dim, value_dim - v0, [&](int d, int c, float value) { start[d][c] = value; });
+        __syncthreads();
+        for (int tile = 0; tile < kScanValues / 16; ++tile) {
+            const int column = v0 + 16 * tile + col;
+            if (v0 + 16 * tile >= value_dim) break;
+            floatx4 sum[4] = {};
+#pragma unroll
+            for (int d = 0; d < kChannelKeys; d += 4)
+                sum[d / 4 % 4] = __builtin_amdgcn_mfma_f32_16x16x4f32(decayed[d / 4], start[d + quad][16 * tile + col], sum[d / 4 % 4], 0, 0, 0);
+            floatx4 acc = (sum[0] + sum[1]) + (sum[2] + sum[3]);
+#pragma unroll
+            for (int part = 0; part < kParts - 1; ++part) {
+                if (part >= wave) break;
+                floatx4 more = {};
+#pragma unroll
+                for (int j = kPart * part; j < kPart * (part + 1); j += 4)
+                    more = __builtin_amdgcn_mfma_f32_16x16x4f32(weight[j / 4], values[j + quad][16 * tile + col], more, 0, 0, 0);
+                acc += more;
+            }
+            // A value that is not finite must not reach the tokens before its own, as zero times it would.
+            float own_values[kPart / 4];
+            bool finite = true;
+#pragma unroll
+            for (int j = 0; j < kPart / 4; ++j) {
+                own_values[j] = values[kPart * wave + 4 * j + quad][16 * tile + col];
+                finite = finite && isfinite(own_values[j]);
+            }
+            if (__all(finite)) {
+                floatx4 more = {};
+#pragma unroll
+                for (int j = 0; j < kPart / 4; ++j) more = __builtin_amdgcn_mfma_f32_16x16x4f32(own_weight[j], own_values[j], more, 0, 0, 0);
+                acc += more;
+            } else {
+#pragma unroll
+                for (int i = 0; i < 4; ++i)
+                    for (int j = kPart * wave; j <= kPart * wave + 4 * quad + i; ++j)
+                        acc[i] = fmaf(weights[kPart * wave + 4 * quad + i][j], values[j][16 * tile + col], acc[i]);
+            }
+#pragma unroll
+            for (int i = 0; i < 4; ++i) {
+                const int t = kPart * wave + 4 * quad + i;
+                if (t < count && column < value_dim)
+                    out[(static_cast<int64_t>(first + t) * heads + head) * value_dim + column] = acc[i] * q_scale;
+            }
+        }
+    }
+}
+
 }  // namespace mll
 
 using namespace mll;
@@ -237,6 +491,32 @@ int mll_gla_chunks(const float* proj, int64_t proj_stride, int q_offset, int k_o
     else MLL_CHUNKS(128, false);
 #undef MLL_CHUNKS
     return check_launch("gla_chunks");
+}
+
+int64_t mll_gla_channel_chunks_scratch(int n_tokens, int n_seqs, int heads, int key_dim, int value_dim) {
+    return (static_cast<int64_t>(n_tokens) / kScanChunk + n_seqs) * heads * key_dim * (static_cast<int64_t>(value_dim) + 1);
+}
+
+int mll_gla_channel_chunks(const float* proj, int64_t proj_stride, int q_offset, int k_offset, int v_offset, const float* log_decay, float* state,
+                           const int32_t* cu_tokens, const int32_t* slots, float* out, float* scratch, int n_tokens, int n_seqs, int heads,
+                           int key_dim, int value_dim, float q_scale, hipStream_t stream) {
+    MLL_REQUIRE(n_tokens >= 0 && n_seqs >= 0 && heads > 0 && key_dim > 0 && value_dim > 0, "gla_channel_chunks: sizes must be positive");
+    MLL_REQUIRE(key_dim <= kChannelKeys, "gla_channel_chunks: key heads wider than 64 are not supported");
+    MLL_REQUIRE(q_offset >= 0 && k_offset >= 0 && v_offset >= 0 && q_offset + heads * key_dim <= proj_stride &&
+                    k_offset + heads * key_dim <= proj_stride && v_offset + heads * value_dim <= proj_stride,
+                "gla_channel_chunks: a projection lies outside its row");
+    if (n_tokens == 0 || n_seqs == 0) return 0;
+    const int64_t elements = static_cast<int64_t>(key_dim) * value_dim;
+    MLL_REQUIRE(heads <= 65535 && elements <= 65535ll * 256, "gla_channel_chunks: too many heads or a state too large for one launch");
+    const dim3 chunks(n_tokens / kScanChunk + n_seqs, heads);
+    float* whole = scratch + static_cast<int64_t>(chunks.x) * heads * elements;
+    gla_channel_state_kernel<<<chunks, kScanThreads, 0, stream>>>(proj, proj_stride, k_offset, v_offset, log_decay, cu_tokens, scratch, whole, n_seqs,
+                                                                  heads, key_dim, value_dim);
+    gla_channel_carry_kernel<<<dim3(n_seqs, heads, static_cast<unsigned>((elements + 255) / 256)), 256, 0, stream>>>(
+        scratch, whole, state, cu_tokens, slots, heads, key_dim, value_dim);
+    gla_channel_out_kernel<<<chunks, kScanThreads, 0, stream>>>(proj, proj_stride, q_offset, k_offset, v_offset, log_decay, cu_tokens, scratch, out,
+                                                                n_seqs, heads, key_dim, value_dim, q_scale);
+    return check_launch("gla_channel_chunks");
 }
 
 }  // extern "C"

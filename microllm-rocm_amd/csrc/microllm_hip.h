@@ -404,7 +404,7 @@ int mll_bias_attention(const void* q, const void* k_pages, const void* v_pages, 
 
 // decay[t][c] = sigmoid(z)^(1 / tau), z = bias[c] + sum_r a2[c][r] * proj[t][low_offset + r]; float32 but a2.
 int mll_gla_decay(const float* proj, int64_t proj_stride, int low_offset, int rank, const void* a2, int a2_dtype,
-                  const float* bias, float tau, float* decay, int n_tokens, int channels, hipStream_t stream);
+                  const float* bias, float tau, float* decay, int n_tokens, int channels, int base_two, hipStream_t stream);
 
 // For every request i of the step, its tokens cu_tokens[i] .. cu_tokens[i + 1] - 1 in order, per head:
 //   S = diag(decay_t) S + k_t v_t^T;  out[t][head] = S^T (q_t * q_scale)
@@ -431,6 +431,13 @@ int64_t mll_gla_chunks_scratch(int n_tokens, int n_seqs, int heads, int key_dim,
 int mll_gla_chunks(const float* proj, int64_t proj_stride, int q_offset, int k_offset, int v_offset, const float* decay, float* state,
                    const int32_t* cu_tokens, const int32_t* slots, float* out, float* scratch, int n_tokens, int n_seqs, int heads,
                    int key_dim, int value_dim, float q_scale, int silu_inputs, hipStream_t stream);
+
+// The same for a decay a key channel and token, given as logarithms to base two ([tokens][heads * key_dim], none positive); key
+// heads of at most 64 channels. `scratch`: mll_gla_channel_chunks_scratch(...) floats.
+int64_t mll_gla_channel_chunks_scratch(int n_tokens, int n_seqs, int heads, int key_dim, int value_dim);
+int mll_gla_channel_chunks(const float* proj, int64_t proj_stride, int q_offset, int k_offset, int v_offset, const float* log_decay, float* state,
+                           const int32_t* cu_tokens, const int32_t* slots, float* out, float* scratch, int n_tokens, int n_seqs, int heads,
+                           int key_dim, int value_dim, float q_scale, hipStream_t stream);
 
 // Columns first .. first + count - 1 of every row of proj, in place: silu.
 int mll_gla_silu(float* proj, int64_t proj_stride, int first, int count, int n_tokens, hipStream_t stream);

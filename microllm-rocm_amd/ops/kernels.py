@@ -1591,8 +1591,10 @@ def bias_attention(q: torch.Tensor, k_pages: torch.Tensor, v_pages: torch.Tensor
 
 
 # ---- gated linear attention -----------------------------------------------------------------------------------
-def gla_decay(proj: torch.Tensor, low_offset: int, a2: torch.Tensor, bias: Optional[torch.Tensor], tau: float) -> torch.Tensor:
-    """``sigmoid(a2 @ low + bias)^(1 / tau)`` per token and key channel, ``low`` being columns of ``proj``'s rows."""
+def gla_decay(proj: torch.Tensor, low_offset: int, a2: torch.Tensor, bias: Optional[torch.Tensor], tau: float,
+              base_two: bool = False) -> torch.Tensor:
+    """``sigmoid(a2 @ low + bias)^(1 / tau)`` per token and key channel, ``low`` being columns of ``proj``'s rows; with
+    ``base_two`` its logarithm to base two."""
     lib = library.load()
     _device_tensor(proj, "projections", torch.float32)
     _device_tensor(a2, "decay weight")
@@ -1607,7 +1609,7 @@ def gla_decay(proj: torch.Tensor, low_offset: int, a2: torch.Tensor, bias: Optio
         count = min(65535, n_tokens - start)
         _check(lib.mll_gla_decay(ctypes.c_void_p(proj.data_ptr() + start * proj.shape[1] * 4), ctypes.c_int64(proj.shape[1]),
                                  low_offset, rank, _ptr(a2), _code(a2.dtype), _ptr(bias), ctypes.c_float(tau),
-                                 ctypes.c_void_p(decay.data_ptr() + start * channels * 4), count, channels, _stream()), lib)
+                                 ctypes.c_void_p(decay.data_ptr() + start * channels * 4), count, channels, int(base_two), _stream()), lib)
     return decay
 
 
@@ -1662,6 +1664,33 @@ def gla_chunks(proj: torch.Tensor, q_offset: int, k_offset: int, v_offset: int, 
     _check(lib.mll_gla_chunks(_ptr(proj), ctypes.c_int64(proj.shape[1]), q_offset, k_offset, v_offset, _ptr(decay), _ptr(state),
                               _ptr(cu_tokens), _ptr(slots), _ptr(out), _ptr(scratch), n_tokens, n_seqs, heads, key_dim, value_dim,
                               ctypes.c_float(q_scale), int(silu_inputs), _stream()), lib)
+    return out
+
+
+GLA_CHANNEL_CHUNK_KEYS = 64     # the same where every key channel has decays of its own
+
+
+def gla_channel_chunks(proj: torch.Tensor, q_offset: int, k_offset: int, v_offset: int, log_decay: torch.Tensor, state: torch.Tensor,
+                       cu_tokens: torch.Tensor, slots: torch.Tensor, n_seqs: int, heads: int, key_dim: int, value_dim: int,
+                       q_scale: float) -> torch.Tensor:
+    """``gla_scan`` for long portions with a decay a token and key channel, given as ``gla_decay``'s logarithms to base two
+    (``[tokens, heads * key_dim]``, none positive): chunks of 64 tokens side by side on the matrix units, the same result but for rounding."""
+    lib = library.load()
+    _device_tensor(proj, "projections", torch.float32)
+    _device_tensor(log_decay, "decays", torch.float32)
+    _device_tensor(state, "state", torch.float32)
+    _device_tensor(cu_tokens, "token offsets", torch.int32)
+    _device_tensor(slots, "state slots", torch.int32)
+    n_tokens = proj.shape[0]
+    _need(proj.dim() == 2 and tuple(log_decay.shape) == (n_tokens, heads * key_dim), "decays are [tokens, heads * key_dim]")
+    _need(state.dim() == 4 and tuple(state.shape[1:]) == (heads, key_dim, value_dim), "state is [slots, heads, key_dim, value_dim]")
+    _need(cu_tokens.shape[0] >= n_seqs + 1 and slots.shape[0] >= n_seqs, "offsets and slots for every request")
+    _need(key_dim <= GLA_CHANNEL_CHUNK_KEYS, "key heads of at most 64 channels")
+    out = torch.empty((n_tokens, heads * value_dim), dtype=torch.float32, device=proj.device)
+    scratch = torch.empty(lib.mll_gla_channel_chunks_scratch(n_tokens, n_seqs, heads, key_dim, value_dim), dtype=torch.float32, device=proj.device)
+    _check(lib.mll_gla_channel_chunks(_ptr(proj), ctypes.c_int64(proj.shape[1]), q_offset, k_offset, v_offset, _ptr(log_decay), _ptr(state),
+                                      _ptr(cu_tokens), _ptr(slots), _ptr(out), _ptr(scratch), n_tokens, n_seqs, heads, key_dim, value_dim,
+                                      ctypes.c_float(q_scale), _stream()), lib)
     return out
 
 

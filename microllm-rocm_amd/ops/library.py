@@ -181,6 +181,7 @@ def load() -> ctypes.CDLL:
     _library.mll_sample_workspace.restype = ctypes.c_int64
     _library.mll_rglru_scan_scratch.restype = ctypes.c_int64
     _library.mll_gla_chunks_scratch.restype = ctypes.c_int64
+    _library.mll_gla_channel_chunks_scratch.restype = ctypes.c_int64
     return _library
 
 

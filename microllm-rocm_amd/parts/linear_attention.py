@@ -13,7 +13,8 @@ multiplied by ``silu(Wg x)`` and projected by ``Wo``. With ``heads_together`` al
 mean square instead, the weight is ``[heads * value_dim]`` and the gate ``sigmoid(Wg x)``; with ``silu_inputs`` queries, keys
 and values pass SiLU before they enter the recurrence (lightning attention is both, with a fixed decay). With ``chunked``
 (and a fixed decay, key heads of at most 128 channels) long portions run in chunks of 64 tokens side by side on the matrix
-units instead of token after token: the same sums in another order. The state starts at zero, is float32, and lives in the
+units instead of token after token: the same sums in another order; a bfloat16 engine does the same for decays a channel and
+key heads of at most 64 channels. The state starts at zero, is float32, and lives in the
 request's state slot, so a request can be cut into steps anywhere. The five projections that read ``x`` are one
 stacked product with a float32 result; decays, the recurrence, the norm and the gate are float32.
 """
@@ -37,6 +38,9 @@ class GatedLinearAttention(Mixer):
     LONG_PORTION = 8        # from this many tokens of one request in a step on, the walk stages its operands through LDS
 
     CHUNKED_PORTION = 128   # and with ``chunked`` chunks of 64 tokens are taken side by side from this many on
+    # With decays a channel: 8 heads of 64 x 128, one request of 256, 512 and 8000 tokens 42, 75 and 1030 us by the walk and 49,
+    # 51 and 152 in chunks; 300 tokens beside seven single ones 192 and 55.
+    CHANNEL_CHUNKED_PORTION = 320
 
     def __init__(self, spec: PartSpec, runtime: Runtime):
         super().__init__(spec, runtime)
@@ -54,6 +58,10 @@ class GatedLinearAttention(Mixer):
         self.heads_together = bool(p.get("heads_together", False))
         self.silu_inputs = bool(p.get("silu_inputs", False))
         self.chunked = bool(p.get("chunked", False)) and self.fixed_decay is not None and self.key_dim <= kernels.GLA_CHUNK_KEYS
+        # The same for decays a channel and token, in a bfloat16 engine: a float32 engine gives a row the same bits however a
+        # request is cut, which chunks that begin where a portion does cannot.
+        self.channel_chunked = (runtime.dtype == torch.bfloat16 and self.fixed_decay is None and not self.silu_inputs
+                                and self.key_dim <= kernels.GLA_CHANNEL_CHUNK_KEYS)
         self.eps = float(p.get("eps", 1e-6))
         self.query_scale = float(p.get("query_scale", self.key_dim ** -0.5))
         keys, values = self.heads * self.key_dim, self.heads * self.value_dim
@@ -115,6 +123,12 @@ class GatedLinearAttention(Mixer):
 
     def forward_inner(self, x, ctx, cache, out: Optional[torch.Tensor] = None, out_scale: float = 1.0) -> torch.Tensor:
         proj = linear(x, self.in_weight, out_dtype=torch.float32)
+        if self.channel_chunked and ctx.max_count >= self.CHANNEL_CHUNKED_PORTION:
+            log_decay = kernels.gla_decay(proj, self.low_at, self.decay_weight, self.decay_bias, self.tau, base_two=True)
+            o = kernels.gla_channel_chunks(proj, self.q_at, self.k_at, self.v_at, log_decay, cache.state, ctx.cu_tokens, ctx.slots, ctx.n_seqs,
+                                           self.heads, self.key_dim, self.value_dim, self.query_scale)
+            return kernels.gla_gate(o, proj, self.g_at, self.norm_weight, self.eps, self.heads, self.value_dim, out_scale,
+                                    self.runtime.dtype, out=out, heads_together=self.heads_together)
         if self.fixed_decay is None:
             decay = kernels.gla_decay(proj, self.low_at, self.decay_weight, self.decay_bias, self.tau)
         else:

@@ -84,3 +84,40 @@ def test_tiled_product_with_clamped_gates(m, width, k, tile_rows):
     want = gate / (1.0 + np.exp(-1.7 * gate)) * (up + 1.0)
     assert (np.abs(got.double().cpu().numpy() - want) <= 2.0 ** -8 * np.abs(want) + 1e-4).all()
     assert float(got.float().abs().max()) > 1.0
+
+
+@pytest.mark.parametrize("heads,dim,vdim", [(2, 64, 128), (3, 20, 70), (1, 16, 8), (4, 33, 129)])
+@pytest.mark.parametrize("strength", [0.02, 1.0, 400.0])
+def test_chunks_with_a_decay_a_channel(heads, dim, vdim, strength):
+    """Requests without tokens, of one token and about a chunk's and a part's edges, each from a state of its own, against the walk
+    in float64; decays close to one, of ordinary size and that leave nothing. Sums of up to 64 logarithms err by 64 roundings of
+    up to 150, of which a power takes 0.7: far below the bound wherever the power is not below it itself."""
+    rng = np.random.default_rng(dim)
+    lengths, slots = [130, 1, 0, 64, 63, 65, 17, 200], [3, 0, 7, 5, 1, 2, 6, 8]
+    cu = np.concatenate([[0], np.cumsum(lengths)])
+    n, keys, values = cu[-1], heads * dim, heads * vdim
+    q, k, v = (rng.normal(size=(n, heads, size)).astype(np.float32) for size in (dim, dim, vdim))
+    logs = (-strength * rng.exponential(size=(n, heads, dim))).astype(np.float32)
+    before = rng.normal(size=(9, heads, dim, vdim)).astype(np.float32)
+    proj = device(np.concatenate([a.reshape(n, -1) for a in (q, k, v)], axis=1))
+    state = device(before)
+    run = lambda p, s: kernels().gla_channel_chunks(p, 0, keys, 2 * keys, device(logs.reshape(n, keys)), s, device(cu, torch.int32),
+                                                    device(slots, torch.int32), len(lengths), heads, dim, vdim, 0.5)
+    got = run(proj, state).cpu().numpy().reshape(n, heads, vdim)
+    for index, slot in enumerate(slots):
+        kept = before[slot].astype(np.float64)
+        want = np.zeros((lengths[index], heads, vdim))
+        for at, token in enumerate(range(cu[index], cu[index + 1])):
+            kept = kept * np.exp2(logs[token].astype(np.float64))[:, :, None] + k[token][:, :, None].astype(np.float64) * v[token][:, None, :]
+            want[at] = 0.5 * np.einsum("hd,hdv->hv", q[token].astype(np.float64), kept)
+        assert np.abs(state[slot].cpu().numpy() - kept).max() < 2e-5 * np.abs(kept).max(), index
+        if lengths[index]:
+            assert np.abs(got[cu[index]:cu[index + 1]] - want).max() < 2e-5 * np.abs(want).max(), index
+    assert torch.equal(state[4], device(before)[4]) and torch.equal(state[7], device(before)[7])
+    # a value that is not finite reaches its own token and those after it
+    for broken in (float("inf"), float("nan")):
+        proj[100, 2 * keys] = broken
+        after = run(proj, device(before)).cpu().numpy().reshape(n, heads, vdim)
+        assert np.isfinite(after[:100]).all() and not np.isfinite(after[100, 0, 0])
+        np.testing.assert_array_equal(after[130:], got[130:])
+        np.testing.assert_allclose(after[:100], got[:100], rtol=0, atol=2e-5 * np.abs(got).max())
