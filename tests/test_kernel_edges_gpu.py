@@ -121,3 +121,27 @@ def test_chunks_with_a_decay_a_channel(heads, dim, vdim, strength):
         assert np.isfinite(after[:100]).all() and not np.isfinite(after[100, 0, 0])
         np.testing.assert_array_equal(after[130:], got[130:])
         np.testing.assert_allclose(after[:100], got[:100], rtol=0, atol=2e-5 * np.abs(got).max())
+
+
+@pytest.mark.parametrize("streams", [1, 2, 3, 4, 5])
+@pytest.mark.parametrize("width", [4, 260, 1024, 2044, 2046, 6148])
+@pytest.mark.parametrize("parts,rms", [(1, 0), (2, 1), (5, 0), (6, 1)])
+def test_stream_norm_by_groups_of_four(streams, width, parts, rms):
+    rng = np.random.default_rng(width + streams)
+    x, y = rng.normal(size=(5, streams, width)).astype(np.float32), rng.normal(size=(parts, 5, width)).astype(np.float32)
+    mix, give, take = rng.normal(size=(streams, streams)).astype(np.float32), rng.normal(size=streams).astype(np.float32), rng.normal(size=streams).astype(np.float32)
+    weight = rng.normal(size=width).astype(np.float32)
+    fresh = np.einsum("st,nsw->ntw", mix.astype(np.float64), x) + give[None, :, None].astype(np.float64) * y.astype(np.float64).sum(0)[:, None, :]
+
+    def norm(rows):
+        u = np.einsum("t,ntw->nw", take.astype(np.float64), rows)
+        u = u if rms else u - u.mean(-1, keepdims=True)
+        return u / np.sqrt((u ** 2).mean(-1, keepdims=True) + 1e-5) * weight
+
+    x_device = device(x)
+    got = kernels().stream_norm(x_device, device(weight), 1e-5, torch.float32, rms=bool(rms), delta=device(y), mix=device(mix), give=device(give),
+                                take=device(take), write_x=True)
+    np.testing.assert_allclose(x_device.cpu().numpy(), fresh, rtol=2e-5, atol=2e-5 * np.abs(fresh).max())
+    np.testing.assert_allclose(got.cpu().numpy(), norm(fresh), rtol=2e-5, atol=2e-5 * np.abs(norm(fresh)).max())
+    some = kernels().stream_norm(x_device, device(weight), 1e-5, torch.bfloat16, rms=bool(rms), take=device(take), rows=device([4, 0], torch.int32))
+    np.testing.assert_allclose(some.float().cpu().numpy(), norm(fresh)[[4, 0]], rtol=2.0 ** -8, atol=2e-5 * np.abs(norm(fresh)).max())
