@@ -1,17 +1,26 @@
 // Matrix products with 17 to 64 rows (decoding many requests, short portions of prompts): C = A . W^T for
 // bfloat16 A [M, K] (row-major) and the packed weight the streaming kernel reads ([N/16][K/32][4][16][8]).
 // Still bound by reading W once from HBM, but with this many rows the activations a wave needs per piece of W
-// are several times the piece: here the 4 or 8 waves of a workgroup walk the same k steps, each over its own
-// tiles of W, and share the activations through LDS (8 k steps at a time, double buffered, brought in MFMA
-// operand order by all waves together). A wave keeps two batches of pieces of W in registers: one on its way
-// while the other is multiplied.
+// are several times the piece: here the 4 or 8 waves of a workgroup walk the same k steps, each over its own one
+// or two tiles of W, and share the activations through LDS (8 k steps at a time, double buffered, brought in MFMA
+// operand order by all waves together). A wave keeps two stages of its tiles in registers: one on its way while
+// the other is multiplied. All loads go through buffer descriptors, which return zeros past their end: a load
+// under a condition would make the compiler wait for all loads before it.
+//
+// A workgroup takes so many tiles that the workgroups fill the compute units evenly (see balanced_tiles): of
+// 37888 x 3584 10 a workgroup, 237 of them, where 16 would leave 108 of the 256 units without one. 64 rows of it
+// 66.1 -> 51.7 us (the reads alone take 40), of 152064 x 3584 214.6 -> 205.3 us (155), 32 rows of 9728 x 896 10.3 -> 7.4 us,
+// of 896 x 4864 7.2 -> 5.4 us, of 1152 x 896 5.0 -> 3.5 us. With 64 rows the products and the reads of LDS take about as
+// long as W's way, and the stages' barriers keep them from covering each other whole.
 //
 // Where W has too few tiles to fill the GPU this way, k is split over `splits` workgroups (grid y), each of
 // which writes its own float32 partial sum [split][M][N]; the consumer adds them in order. Which k steps a
 // sum holds, and in which order, depends on (n, k, splits) alone: a row's result does not depend on the
-// other rows.
+// other rows, nor on the tiles a workgroup takes.
 #include "common.h"
 #include "microllm_hip.h"
+
+#include <type_traits>
 
 namespace mll {
 
@@ -21,76 +30,76 @@ typedef unsigned int uintx4 __attribute__((ext_vector_type(4)));
 
 namespace medium {
 
-constexpr int kStepsPerStage = 8;    // k steps of activations in one LDS buffer
-constexpr int kBatch = 4;            // k steps of W a wave loads at a time; two batches make a stage
+constexpr int kStepsPerStage = 8;    // k steps of activations in one LDS buffer, and of W in one batch of loads
+constexpr int kMostTiles = 16;       // two a wave of 8
+constexpr unsigned kPast = 0x40000000;   // an offset past the end of every descriptor here
+constexpr int kMostSteps = static_cast<int>(kPast) / (kMostTiles * 1024);      // so that a workgroup's tiles end before it
+constexpr int kBufferFlags = 0x00027000;   // a raw buffer of 32-bit words
+constexpr int kNonTemporal = 2;      // W is read once a step: past the caches
 
 union Piece {
     bf16x8 v;
     uintx4 raw;
 };
 
-
-template <int NT>
-__device__ inline void load_batch(Piece (&pieces)[kBatch][NT], const bf16* const (&w_ptr)[NT], const bool (&w_live)[NT],
-                                  int first_step, int end_step) {
-#pragma unroll
-    for (int u = 0; u < kBatch; ++u) {
-        const int ks = first_step + u;
-#pragma unroll
-        for (int nt = 0; nt < NT; ++nt) {
-            pieces[u][nt].raw = uintx4{0u, 0u, 0u, 0u};
-            if (ks < end_step && w_live[nt]) {
-                const uintx4* source = reinterpret_cast<const uintx4*>(w_ptr[nt] + static_cast<int64_t>(ks) * 512);
-                pieces[u][nt].raw = __builtin_nontemporal_load(source);      // W is read once a step: past the caches
-            }
-        }
-    }
-}
-
 // EPILOGUE: 0 = float32 [splits][M, N]; 1 = bfloat16 [M, N]; 2 = bfloat16 [M, N / 2] = silu(even rows of W) * (odd
-// rows). 1 and 2 need splits == 1.
+// rows). 1 and 2 need splits == 1. A workgroup takes `tiles` tiles of W, a wave its wave-th and (NT = 2) that kWaves on.
 template <int MT, int NT, int kWaves, int EPILOGUE>
 __global__ __launch_bounds__(kWaves * kWave) void gemm_medium_kernel(
     const bf16* __restrict__ a, const bf16* __restrict__ w_packed, void* __restrict__ out,
-    int m, int n, int k, int n_tiles, int k_steps, int steps_per_split) {
+    int m, int n, int k, int n_tiles, int k_steps, int steps_per_split, int tiles) {
     constexpr int kStagePieces = MT * kStepsPerStage;             // pieces of A in a buffer, 1 KB each
     constexpr int kPiecesPerWave = kStagePieces / kWaves;
-    static_assert(kStagePieces % kWaves == 0, "the waves share the copying evenly");
     extern __shared__ uintx4 stage[];                             // [2][MT][kStepsPerStage][64 lanes]
 
     const int lane = threadIdx.x % kWave;
-    const int wave = threadIdx.x / kWave;
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave);
     const int col = lane % 16, quad = lane / 16;
-    const int tile0 = (blockIdx.x * kWaves + wave) * NT;
+    const int tile0 = blockIdx.x * tiles;
+    const int live_tiles = min(tiles, n_tiles - tile0);
     const int first_step = blockIdx.y * steps_per_split;
     const int end_step = min(k_steps, first_step + steps_per_split);
     const int n_stages = (end_step - first_step + kStepsPerStage - 1) / kStepsPerStage;
 
-    const bf16* w_ptr[NT];
-    bool w_live[NT];
+    const __amdgpu_buffer_rsrc_t w_rsrc = __builtin_amdgcn_make_buffer_rsrc(
+        const_cast<bf16*>(w_packed) + static_cast<int64_t>(tile0) * k_steps * 512, 0, live_tiles * k_steps * 1024, kBufferFlags);
+    const __amdgpu_buffer_rsrc_t a_rsrc = __builtin_amdgcn_make_buffer_rsrc(const_cast<bf16*>(a), 0, m * k * 2, kBufferFlags);
+    unsigned w_at[NT];
 #pragma unroll
     for (int nt = 0; nt < NT; ++nt) {
-        w_live[nt] = tile0 + nt < n_tiles;
-        w_ptr[nt] = w_packed + static_cast<int64_t>(w_live[nt] ? tile0 + nt : 0) * k_steps * 512 + lane * 8;
+        w_at[nt] = wave + kWaves * nt < live_tiles ? static_cast<unsigned>((wave + kWaves * nt) * k_steps * 1024 + lane * 16) : kPast;
+        asm("" : "+v"(w_at[nt]));       // else the choice becomes a branch around the loads
     }
+    // This wave's share of a buffer: every kWaves-th k step of a stage, of all rows.
+    static_assert(kStepsPerStage % kWaves == 0, "the waves share the copying evenly");
+    unsigned a_at[MT];
+#pragma unroll
+    for (int mt = 0; mt < MT; ++mt) {
+        a_at[mt] = 16 * mt + col < m ? static_cast<unsigned>((16 * mt + col) * k * 2 + quad * 16) : kPast;
+        asm("" : "+v"(a_at[mt]));
+    }
+    const int a_end = min(k, end_step * 32) - quad * 8;      // a lane's steps begin before this element
 
-    // This wave's share of a buffer: pieces wave, wave + kWaves, ...; piece p holds rows 16 * (p / 8) .. + 15 at k step p % 8.
-    auto load_share = [&](uintx4 (&share)[kPiecesPerWave], int stage_first_step) {
+    auto load_w = [&](Piece (&pieces)[kStepsPerStage][NT], int stage_number) {
+        const int step = first_step + stage_number * kStepsPerStage;
+#pragma unroll
+        for (int u = 0; u < kStepsPerStage; ++u) {
+            const unsigned at = step + u < end_step ? static_cast<unsigned>(step + u) * 1024 : kPast;
+#pragma unroll
+            for (int nt = 0; nt < NT; ++nt) pieces[u][nt].raw = __builtin_amdgcn_raw_buffer_load_b128(w_rsrc, w_at[nt] + at, 0, kNonTemporal);
+        }
+    };
+    auto load_share = [&](uintx4 (&share)[kPiecesPerWave], int stage_number) {
 #pragma unroll
         for (int j = 0; j < kPiecesPerWave; ++j) {
-            const int piece = wave + kWaves * j;
-            const int row = (piece / kStepsPerStage) * 16 + col;
-            const int ks = stage_first_step + piece % kStepsPerStage;
-            const int k_offset = ks * 32 + quad * 8;
-            share[j] = uintx4{0u, 0u, 0u, 0u};
-            if (row < m && ks < end_step && k_offset < k)
-                share[j] = *reinterpret_cast<const uintx4*>(a + static_cast<int64_t>(row) * k + k_offset);
+            const int step = first_step + stage_number * kStepsPerStage + wave + kWaves * (j / MT);
+            share[j] = __builtin_amdgcn_raw_buffer_load_b128(a_rsrc, a_at[j % MT] + (step * 32 < a_end ? static_cast<unsigned>(step) * 64 : kPast), 0, 0);
         }
     };
     auto store_share = [&](const uintx4 (&share)[kPiecesPerWave], int buffer) {
 #pragma unroll
         for (int j = 0; j < kPiecesPerWave; ++j)
-            stage[(buffer * kStagePieces + wave + kWaves * j) * kWave + lane] = share[j];
+            stage[(buffer * kStagePieces + j % MT * kStepsPerStage + wave + kWaves * (j / MT)) * kWave + lane] = share[j];
     };
 
     floatx4 acc[NT][MT];
@@ -99,13 +108,13 @@ __global__ __launch_bounds__(kWaves * kWave) void gemm_medium_kernel(
 #pragma unroll
         for (int mt = 0; mt < MT; ++mt) acc[nt][mt] = floatx4{0.0f, 0.0f, 0.0f, 0.0f};
 
-    auto multiply = [&](const Piece (&pieces)[kBatch][NT], int buffer, int step_in_stage) {
+    auto multiply = [&](const Piece (&pieces)[kStepsPerStage][NT], int buffer) {
 #pragma unroll
-        for (int u = 0; u < kBatch; ++u) {
+        for (int u = 0; u < kStepsPerStage; ++u) {
             Piece a_piece[MT];
 #pragma unroll
             for (int mt = 0; mt < MT; ++mt)
-                a_piece[mt].raw = stage[(buffer * kStagePieces + mt * kStepsPerStage + step_in_stage + u) * kWave + lane];
+                a_piece[mt].raw = stage[(buffer * kStagePieces + mt * kStepsPerStage + u) * kWave + lane];
 #pragma unroll
             for (int nt = 0; nt < NT; ++nt)
 #pragma unroll
@@ -114,30 +123,37 @@ __global__ __launch_bounds__(kWaves * kWave) void gemm_medium_kernel(
         }
     };
 
+    // The activations of a stage are asked for before its tiles: loads come back in order, and the copy into LDS must not wait
+    // for the tiles. A buffer was last read in the stage before the one that fills it, and every wave has passed that
+    // stage's barrier.
     uintx4 share[kPiecesPerWave];
-    Piece w_even[kBatch][NT], w_odd[kBatch][NT];
-    load_share(share, first_step);
-    load_batch<NT>(w_even, w_ptr, w_live, first_step, end_step);
+    Piece w_even[kStepsPerStage][NT], w_odd[kStepsPerStage][NT];
+    load_share(share, 0);
+    load_w(w_even, 0);
+    __builtin_amdgcn_sched_barrier(0);
     store_share(share, 0);
     __syncthreads();
-    for (int s = 0; s < n_stages; ++s) {
-        const int stage_step = first_step + s * kStepsPerStage;
-        const int buffer = s % 2;
-        if (s + 1 < n_stages) load_share(share, stage_step + kStepsPerStage);
-        load_batch<NT>(w_odd, w_ptr, w_live, stage_step + kBatch, end_step);
-        multiply(w_even, buffer, 0);
-        load_batch<NT>(w_even, w_ptr, w_live, stage_step + kStepsPerStage, end_step);
-        multiply(w_odd, buffer, kBatch);
-        // The other buffer was last read in the stage before this one, and every wave has passed that stage's barrier.
-        if (s + 1 < n_stages) store_share(share, 1 - buffer);
+    for (int s = 0; s < n_stages; s += 2) {
+        load_share(share, s + 1);
+        load_w(w_odd, s + 1);
+        __builtin_amdgcn_sched_barrier(0);      // else the loads sink below the products, behind their waits
+        multiply(w_even, 0);
+        store_share(share, 1);
+        __syncthreads();
+        if (s + 1 >= n_stages) break;
+        load_share(share, s + 2);
+        load_w(w_even, s + 2);
+        __builtin_amdgcn_sched_barrier(0);
+        multiply(w_odd, 1);
+        store_share(share, 0);
         __syncthreads();
     }
 
-    // acc[nt][mt][i] = C[row mt*16 + col][column (tile0 + nt)*16 + quad*4 + i]
+    // acc[nt][mt][i] = C[row mt*16 + col][column n_tile*16 + quad*4 + i]
 #pragma unroll
     for (int nt = 0; nt < NT; ++nt) {
-        const int n_tile = tile0 + nt;
-        if (n_tile >= n_tiles) continue;
+        if (wave + kWaves * nt >= live_tiles) continue;
+        const int n_tile = tile0 + wave + kWaves * nt;
 #pragma unroll
         for (int mt = 0; mt < MT; ++mt) {
             const int row = mt * 16 + col;
@@ -171,40 +187,56 @@ __global__ __launch_bounds__(kWaves * kWave) void gemm_medium_kernel(
     }
 }
 
-template <int MT, int NT, int kWaves, int EPILOGUE>
-static void launch_one(const bf16* a, const bf16* w, void* out, int m, int n, int k, int n_tiles, int k_steps,
-                       int splits, hipStream_t stream) {
-    const dim3 grid((n_tiles + kWaves * NT - 1) / (kWaves * NT), splits);
+// The tiles of W a workgroup takes, at most `most`: so that the compute units' rounds times what a round takes (its tiles, and the
+// activations' copy, which costs about two) come to the least. 64 rows of
+// 37888 x 3584 with 10 tiles 51.7 us, with 5 69.2 and with 4 74.5.
+static int balanced_tiles(int n_tiles, int splits, int most) {
+    constexpr int kUnits = 256, kCopy = 2;
+    int best = 1, least = 0x7fffffff;
+    for (int tiles = 1; tiles <= most; ++tiles) {
+        const int64_t groups = static_cast<int64_t>((n_tiles + tiles - 1) / tiles) * splits;
+        const int64_t cost = (groups + kUnits - 1) / kUnits * (tiles + kCopy);
+        if (cost < least) {
+            best = tiles;
+            least = static_cast<int>(cost);
+        }
+    }
+    return best;
+}
+
+template <int MT, int EPILOGUE>
+static void launch_rows(const bf16* a, const bf16* w, void* out, int m, int n, int k, int most_tiles, int splits, hipStream_t stream) {
+    const int n_tiles = (n + 15) / 16, k_steps = (k + 31) / 32;
+    const int tiles = balanced_tiles(n_tiles, splits, most_tiles);
+    const dim3 grid((n_tiles + tiles - 1) / tiles, splits);
     // Each split takes whole stages, so that the stages of a sum begin at the same k whatever the split.
     const int stages = (k_steps + kStepsPerStage - 1) / kStepsPerStage;
     const int steps_per_split = ((stages + splits - 1) / splits) * kStepsPerStage;
     const size_t lds = 2 * MT * kStepsPerStage * kWave * sizeof(uintx4);
-    gemm_medium_kernel<MT, NT, kWaves, EPILOGUE><<<grid, kWaves * kWave, lds, stream>>>(a, w, out, m, n, k, n_tiles, k_steps, steps_per_split);
+    const auto launch = [&](auto tiles_a_wave, auto waves) {
+        constexpr int kWaves = decltype(waves)::value;
+        gemm_medium_kernel<MT, decltype(tiles_a_wave)::value, kWaves, EPILOGUE><<<grid, kWaves * kWave, lds, stream>>>(
+            a, w, out, m, n, k, n_tiles, k_steps, steps_per_split, tiles);
+    };
+    using std::integral_constant;
+    // Four waves where there are no more tiles (64 rows of 9728 x 896, 3 tiles a workgroup: 11.7 -> 9.6 us). Four waves of up to four
+    // tiles each read LDS half as often, but hold too much: 64 rows of 37888 x 3584 51.7 -> 55.6 us.
+    if (tiles <= 4) launch(integral_constant<int, 1>{}, integral_constant<int, 4>{});
+    else if (tiles <= 8) launch(integral_constant<int, 1>{}, integral_constant<int, 8>{});
+    else launch(integral_constant<int, 2>{}, integral_constant<int, 8>{});
 }
 
 template <int EPILOGUE>
-static int launch_medium(const void* a, const void* w_packed, void* out, int m, int n, int k, int tiles_per_wave,
-                         int waves, int splits, hipStream_t stream) {
-    const int n_tiles = (n + 15) / 16;
-    const int k_steps = (k + 31) / 32;
+static int launch_medium(const void* a, const void* w_packed, void* out, int m, int n, int k, int most_tiles, int splits, hipStream_t stream) {
     const bf16* a_ = static_cast<const bf16*>(a);
     const bf16* w_ = static_cast<const bf16*>(w_packed);
-    const int m_tiles = (m + 15) / 16;
-#define MLL_MEDIUM_CASE(MT)                                                                                          \
-    case MT:                                                                                                         \
-        if (tiles_per_wave == 2 && waves == 8) launch_one<MT, 2, 8, EPILOGUE>(a_, w_, out, m, n, k, n_tiles, k_steps, splits, stream); \
-        else if (tiles_per_wave == 2) launch_one<MT, 2, 4, EPILOGUE>(a_, w_, out, m, n, k, n_tiles, k_steps, splits, stream);          \
-        else if (waves == 8) launch_one<MT, 1, 8, EPILOGUE>(a_, w_, out, m, n, k, n_tiles, k_steps, splits, stream);                  \
-        else launch_one<MT, 1, 4, EPILOGUE>(a_, w_, out, m, n, k, n_tiles, k_steps, splits, stream);                                   \
-        break;
-    switch (m_tiles) {
-        MLL_MEDIUM_CASE(1)
-        MLL_MEDIUM_CASE(2)
-        MLL_MEDIUM_CASE(3)
-        MLL_MEDIUM_CASE(4)
+    switch ((m + 15) / 16) {
+        case 1: launch_rows<1, EPILOGUE>(a_, w_, out, m, n, k, most_tiles, splits, stream); break;
+        case 2: launch_rows<2, EPILOGUE>(a_, w_, out, m, n, k, most_tiles, splits, stream); break;
+        case 3: launch_rows<3, EPILOGUE>(a_, w_, out, m, n, k, most_tiles, splits, stream); break;
+        case 4: launch_rows<4, EPILOGUE>(a_, w_, out, m, n, k, most_tiles, splits, stream); break;
         default: return fail("gemm_medium: more than 64 rows");
     }
-#undef MLL_MEDIUM_CASE
     return check_launch("gemm_medium");
 }
 
@@ -219,16 +251,17 @@ extern "C" int mll_gemm_medium(const void* a, const void* w_packed, void* out, i
     MLL_REQUIRE(n > 0 && k > 0 && k % 8 == 0, "gemm_medium: k must be a positive multiple of 8");
     MLL_REQUIRE(tiles_per_wave == 1 || tiles_per_wave == 2, "gemm_medium: a wave takes one or two tiles of the weight");
     MLL_REQUIRE(waves == 4 || waves == 8, "gemm_medium: workgroups of 4 or 8 waves");
+    MLL_REQUIRE((k + 31) / 32 <= medium::kMostSteps, "gemm_medium: the reduction is too long for 32-bit offsets");
     MLL_REQUIRE(splits >= 1 && splits <= 64, "gemm_medium: between 1 and 64 splits of k");
     MLL_REQUIRE(epilogue == 0 || splits == 1, "gemm_medium: only float32 partial sums can be split over k");
     MLL_REQUIRE((epilogue != 2 && epilogue != 5) || n % 2 == 0, "gemm_medium: the gated epilogue needs an even number of weight rows");
     MLL_REQUIRE(reinterpret_cast<uintptr_t>(a) % 16 == 0, "gemm_medium: the activations must be 16-byte aligned");
     if (m == 0) return 0;
     switch (epilogue) {
-        case 0: return medium::launch_medium<0>(a, w_packed, out, m, n, k, tiles_per_wave, waves, splits, stream);
-        case 1: return medium::launch_medium<1>(a, w_packed, out, m, n, k, tiles_per_wave, waves, splits, stream);
-        case 2: return medium::launch_medium<2>(a, w_packed, out, m, n, k, tiles_per_wave, waves, splits, stream);
-        case 5: return medium::launch_medium<5>(a, w_packed, out, m, n, k, tiles_per_wave, waves, splits, stream);
+        case 0: return medium::launch_medium<0>(a, w_packed, out, m, n, k, tiles_per_wave * waves, splits, stream);
+        case 1: return medium::launch_medium<1>(a, w_packed, out, m, n, k, tiles_per_wave * waves, splits, stream);
+        case 2: return medium::launch_medium<2>(a, w_packed, out, m, n, k, tiles_per_wave * waves, splits, stream);
+        case 5: return medium::launch_medium<5>(a, w_packed, out, m, n, k, tiles_per_wave * waves, splits, stream);
         default: return fail("gemm_medium: unknown epilogue");
     }
 }

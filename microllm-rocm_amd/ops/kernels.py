@@ -1089,27 +1089,28 @@ def gemm_skinny_clamped(x: torch.Tensor, packed: torch.Tensor, n: int, limit: fl
 
 
 MEDIUM_WORKGROUPS = 224     # workgroups of 8 waves that gemm_medium wants at least (MI355X has 256 compute units)
-MEDIUM_WHOLE_WORKGROUPS = 128     # where the reduction cannot be split, two tiles a wave from this many workgroups on
 
 
 def medium_plan(n: int, k: int, may_split: bool = True) -> Tuple[int, int, int]:
-    """(tiles of W a wave takes, waves a workgroup, splits of k) for ``gemm_medium``.
+    """(tiles of W a wave takes at most, waves a workgroup at most, splits of k) for ``gemm_medium``, which takes of the tiles
+    what fills the compute units evenly.
 
-    A function of the weight's shape alone, so that a row's sum does not depend on the other rows. Two tiles a
-    wave halve the reads of the activations; they are taken where splitting k (at most 16 times, a stage of 256
-    at least per split) still gives enough workgroups.
+    A function of the weight's shape alone, so that a row's sum does not depend on the other rows. k is split (at most 16
+    times, a stage of 256 at least per split) until workgroups of 16 tiles, or of 8 where those would still be too few, are
+    enough.
     """
     n_tiles = -(-n // 16)
     stages = -(-k // 256)
     most = 1
     while may_split and most * 2 <= min(16, stages):
         most *= 2
-    tiles_per_wave = 2 if -(-n_tiles // 16) * most >= (MEDIUM_WORKGROUPS if may_split else MEDIUM_WHOLE_WORKGROUPS) else 1
-    groups = -(-n_tiles // (8 * tiles_per_wave))
+    groups = -(-n_tiles // 16)
+    if groups * most < MEDIUM_WORKGROUPS:
+        groups = -(-n_tiles // 8)
     splits = 1
     while splits < most and groups * splits < MEDIUM_WORKGROUPS:
         splits *= 2
-    return tiles_per_wave, 8, splits
+    return 2, 8, splits
 
 
 def gemm_medium(x: torch.Tensor, packed: torch.Tensor, n: int, epilogue: str = "f32",

@@ -37,12 +37,12 @@ class Weight:
 
 MAX_FACTOR_WIDTH = 8192   # the widest norm whose rows' factors the streaming product applies (its sums sit in LDS)
 SKINNY_ROWS = 16        # up to this many rows gemm_skinny beats the library on MI355X for every weight
-MEDIUM_ROWS = 64        # and up to this many gemm_medium does, except for
-MEDIUM_WIDE_TILES = 2048   # weights with this many tiles of 16 rows or more (gate/up, the head), where the
-MEDIUM_WIDE_ROWS = 40      # library is as fast from about this many rows on
-MEDIUM_GATED_ROWS = 48     # a gated product (silu(gate) * up in the epilogue) is gemm_medium's up to this many rows: in the
-                           # decode step against the tuned library product and the SiLU kernel, 7B sizes +2.5 % at 17 to 32
-                           # rows, +1 % at 48, -0.6 % at 56 and 64; 0.5B sizes +9 % at 17, +7 % at 32, the same at 64
+MEDIUM_ROWS = 64        # and up to this many gemm_medium does: at 17, 32 and 64 rows (the library's time, with the activation's kernel
+                        # for gate and up, over this one's) 37888 x 3584 gated 1.27, 1.33 and 1.34, 9728 x 896 gated 2.06, 1.95 and
+                        # 1.53, 16384 x 2048 gated 1.42, 1.37 and 1.10, 3584 x 18944 4.2, 4.1 and 2.9; except for
+MEDIUM_WIDE_TILES = 2048   # weights with this many tiles of 16 rows or more that are not gated (the head), where the library is
+MEDIUM_WIDE_ROWS = 40      # nearly as fast beyond this many: 152064 x 3584 at 32, 48 and 64 rows 1.37, 1.05 and 1.06
+MEDIUM_GATED_ROWS = MEDIUM_ROWS
 
 
 @dataclass

@@ -145,3 +145,18 @@ def test_stream_norm_by_groups_of_four(streams, width, parts, rms):
     np.testing.assert_allclose(got.cpu().numpy(), norm(fresh), rtol=2e-5, atol=2e-5 * np.abs(norm(fresh)).max())
     some = kernels().stream_norm(x_device, device(weight), 1e-5, torch.bfloat16, rms=bool(rms), take=device(take), rows=device([4, 0], torch.int32))
     np.testing.assert_allclose(some.float().cpu().numpy(), norm(fresh)[[4, 0]], rtol=2.0 ** -8, atol=2e-5 * np.abs(norm(fresh)).max())
+
+
+@pytest.mark.parametrize("n", [1024, 16384, 16400, 20480, 36864, 36888])      # 1, 4, 5, 5, 9 and 10 tiles a workgroup, some the last one
+@pytest.mark.parametrize("k", [24, 256, 264, 776])
+def test_product_for_64_rows_by_tiles_a_workgroup(n, k):
+    rng = np.random.default_rng(n + k)
+    x_exact, x = to_bf16_exact(rng.normal(size=(64, k)))
+    w_exact, w = to_bf16_exact(rng.normal(size=(n, k)))
+    packed = kernels().pack_weight(w)
+    plan = kernels().medium_plan(n, k, may_split=False)
+    whole = kernels().gemm_medium(x, packed, n, "f32", plan=plan)
+    bound = (k + 1) * F32_STEP * (np.abs(x_exact) @ np.abs(w_exact).T)
+    assert (np.abs(whole.double().cpu().numpy() - x_exact @ w_exact.T) <= bound).all()
+    for m in (16, 17, 33, 48):
+        assert torch.equal(kernels().gemm_medium(x[:m].contiguous(), packed, n, "f32", plan=plan), whole[:m]), m
