@@ -140,6 +140,7 @@ __device__ inline float merged(float so_far, float keep, float chunk, float add)
 // ---- runs of 16 tokens on the matrix units -----------------------------------------------------------------------
 typedef float floatx4 __attribute__((ext_vector_type(4)));
 constexpr int kRunTokens = 16;
+constexpr int kRunsFrom = 4;             // tokens a request: with fewer, most blocks of 16 have more stretches than a wave takes
 
 // The tokens 16 * block .. + 15 of the step in stretches of places of one request in a row: bit i is set where token i begins
 // one. Tokens that only pad the step, or lie past its end, begin one each and belong to none (`none`).
@@ -733,7 +734,7 @@ __global__ __launch_bounds__(kWave) void paged_attention_rowwise_merge_kernel(
 }
 
 template <typename T, int DIMS>
-static int launch_rowwise_dims(const void* q, const void* k_cache, const void* v_cache, const int32_t* block_table,
+static int launch_rowwise_dims(const void* q, const void* k_cache, const void* v_cache, const int32_t* block_table, int requests,
                           int table_width, const int32_t* seq_of_token, const int32_t* positions, void* out,
                           float* part_o, float* part_ml, int max_chunks, int usual_chunks, float scale, int window, int n_tokens,
                           int heads, int kv_heads, int head_dim, int page_size, hipStream_t stream) {
@@ -758,7 +759,8 @@ static int launch_rowwise_dims(const void* q, const void* k_cache, const void* v
     int runs_apart = 0;
     if (max_chunks == 0) {
         if constexpr (std::is_same<T, float>::value && DIMS <= 2) {
-            if (window == 0 && head_dim % 16 == 0) {
+            // With few tokens a request there are no stretches for the launch to find: 32 requests of one token each lose 5 us.
+            if (window == 0 && head_dim % 16 == 0 && n_tokens >= kRunsFrom * static_cast<int64_t>(requests)) {
                 runs_apart = 1;
                 const int64_t units = static_cast<int64_t>((n_tokens + kRunTokens - 1) / kRunTokens) * heads;
                 MLL_REQUIRE(units < (static_cast<int64_t>(1) << 31) - 4, "paged_attention: too many rows for one call");
@@ -815,12 +817,12 @@ static int launch_rowwise_dims(const void* q, const void* k_cache, const void* v
 }
 
 template <typename T>
-static int launch_rowwise(const void* q, const void* k_cache, const void* v_cache, const int32_t* block_table,
+static int launch_rowwise(const void* q, const void* k_cache, const void* v_cache, const int32_t* block_table, int requests,
                           int table_width, const int32_t* seq_of_token, const int32_t* positions, void* out,
                           float* part_o, float* part_ml, int max_chunks, int usual_chunks, float scale, int window, int n_tokens,
                           int heads, int kv_heads, int head_dim, int page_size, hipStream_t stream) {
 #define MLL_ROWWISE_DIMS(D)                                                                                            \
-    return launch_rowwise_dims<T, D>(q, k_cache, v_cache, block_table, table_width, seq_of_token, positions, out, part_o, \
+    return launch_rowwise_dims<T, D>(q, k_cache, v_cache, block_table, requests, table_width, seq_of_token, positions, out, part_o, \
                                      part_ml, max_chunks, usual_chunks, scale, window, n_tokens, heads, kv_heads, head_dim, page_size, stream)
     if (head_dim <= kWave) MLL_ROWWISE_DIMS(1);
     if (head_dim <= 2 * kWave) MLL_ROWWISE_DIMS(2);
@@ -846,10 +848,11 @@ extern "C" int mll_rowwise_heads_a_wave(int count) {
 // max_chunks 0: one wave per (token, head). Otherwise one wave per chunk, for rows whose keys span at most
 // max_chunks chunks (the caller's promise: a row with more would lose its last ones), with part_o
 // [n_tokens * heads * max_chunks * head_dim] and part_ml [n_tokens * heads * max_chunks * 2] floats as workspace.
+// requests: rows of block_table, at least as many as the tokens' requests; only which kernel takes the tokens follows from it.
 // usual_chunks (0: max_chunks): how many chunks the step's rows have now, where max_chunks leaves room for later
 // steps of the same shape; only how many heads a wave takes follows from it.
 extern "C" int mll_paged_attention_rowwise(const void* q, int dtype, const void* k_cache, const void* v_cache,
-                                           const int32_t* block_table, int table_width,
+                                           const int32_t* block_table, int requests, int table_width,
                                            const int32_t* seq_of_token, const int32_t* positions, void* out,
                                            float* part_o, float* part_ml, int max_chunks, int usual_chunks, float scale,
                                            int window, int n_tokens, int heads, int kv_heads, int head_dim, int page_size,
@@ -863,10 +866,10 @@ extern "C" int mll_paged_attention_rowwise(const void* q, int dtype, const void*
     MLL_REQUIRE(max_chunks == 0 || (part_o && part_ml), "paged_attention: chunks need the partial buffers");
     if (n_tokens == 0) return 0;
     if (dtype == kF32)
-        return launch_rowwise<float>(q, k_cache, v_cache, block_table, table_width, seq_of_token, positions, out, part_o,
+        return launch_rowwise<float>(q, k_cache, v_cache, block_table, requests, table_width, seq_of_token, positions, out, part_o,
                                      part_ml, max_chunks, usual_chunks, scale, window, n_tokens, heads, kv_heads, head_dim, page_size, stream);
     if (dtype == kBF16)
-        return launch_rowwise<bf16>(q, k_cache, v_cache, block_table, table_width, seq_of_token, positions, out, part_o,
+        return launch_rowwise<bf16>(q, k_cache, v_cache, block_table, requests, table_width, seq_of_token, positions, out, part_o,
                                     part_ml, max_chunks, usual_chunks, scale, window, n_tokens, heads, kv_heads, head_dim, page_size, stream);
     return fail("paged_attention: unknown dtype");
 }

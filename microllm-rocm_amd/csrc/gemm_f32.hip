@@ -143,23 +143,23 @@ __global__ __launch_bounds__(256) void gemm_f32_tile_kernel(const float* __restr
     }
 }
 
-// At most 16 rows (decoding), k a multiple of 4: a wave takes NT tiles of 16 columns of C and its part of k, on
-// v_mfma_f32_16x16x4_f32 with 16 rows of W as its A operand. A wave's load brings 256 bytes of each of four rows, without a
+// At most 16 rows (decoding), or 32 (SIXTEENS = 2) and groups of them (blockIdx.y), k a multiple of 4: a wave takes NT tiles of 16
+// columns of C and its part of k, on v_mfma_f32_16x16x4_f32 with 16 rows of W as its A operand. A wave's load brings 256 bytes of each of four rows, without a
 // branch between the loads, two blocks of 64 of k at a time; the wave then passes them through LDS of its own
 // (no other wave reads it), where a row of 64 lies as [k % 4][k / 4]: of every four consecutive k the product wants one in
 // each quarter of the wave, and a lane's 16-byte read holds its operands of four products in a row. GROUPS: how many
 // times four rows of A there are. Bound by reading W; against the vector kernels below at 8 rows: 37888 x 3584 109 -> 101 us
 // (5.4 TB/s), 3584 x 18944 63 -> 52, 3584 x 3584 18.4 -> 15.4, 152064 x 3584 420 -> 352 (with two tiles a wave at 9 to 16 rows 496
-// -> 367). Two blocks of 128 instead of 64 of k in flight are slower (more is asked for past the ends: 52 -> 57).
+// -> 367); at 32 rows, against the matrix units' tiles, 168 -> 159, 84 -> 78, and 24 x 896 x 4864 19.0 -> 12.0. Two blocks of 128 instead of 64 of k in flight are slower (more is asked for past the ends: 52 -> 57).
 constexpr int64_t kFewWaves = 384;      // waves from which this kernel is taken: 1152 x 896 in two parts, 144 waves, takes 5.6 us in the vector kernel and 7.7 here; 896 x 4864 in eight, 448 waves, 10.8 and 9.6
 constexpr int kFewRow = 64 + 16;        // floats from one row in LDS to the next: the four rows of a load on different banks
 
-template <int NT, int GROUPS>
+template <int NT, int GROUPS, int SIXTEENS>
 __global__ __launch_bounds__(256) void gemm_f32_few_kernel(const float* __restrict__ a, const float* __restrict__ w,
                                                            const float* __restrict__ bias, float* __restrict__ c,
                                                            int m, int n, int k, int k_split) {
     MLL_F32_SPLIT_RANGE
-    __shared__ __align__(16) float shared[4][NT + 1][16][kFewRow];
+    __shared__ __align__(16) float shared[4][NT + SIXTEENS][16][kFewRow];
     const int lane = threadIdx.x % kWave;
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave);
     const int col = lane % 16, quad = lane / 16;
@@ -167,12 +167,15 @@ __global__ __launch_bounds__(256) void gemm_f32_few_kernel(const float* __restri
     if (first >= n) return;
     const __amdgpu_buffer_rsrc_t w_rsrc = __builtin_amdgcn_make_buffer_rsrc(const_cast<float*>(w) + static_cast<int64_t>(first) * ld, 0,
                                                                             min(16 * NT, n - first) * ld * 4, kBufferFlags);
-    const __amdgpu_buffer_rsrc_t a_rsrc = __builtin_amdgcn_make_buffer_rsrc(const_cast<float*>(a), 0, m * ld * 4, kBufferFlags);
-    floatx4 acc[NT];
+    const int row0 = blockIdx.y * 16 * SIXTEENS, rows = min(16 * SIXTEENS, m - row0);
+    const __amdgpu_buffer_rsrc_t a_rsrc = __builtin_amdgcn_make_buffer_rsrc(const_cast<float*>(a) + static_cast<int64_t>(row0) * ld, 0, rows * ld * 4, kBufferFlags);
+    floatx4 acc[NT][SIXTEENS];
 #pragma unroll
-    for (int nt = 0; nt < NT; ++nt) acc[nt] = floatx4{0.0f, 0.0f, 0.0f, 0.0f};
+    for (int nt = 0; nt < NT; ++nt)
+#pragma unroll
+        for (int s = 0; s < SIXTEENS; ++s) acc[nt][s] = floatx4{0.0f, 0.0f, 0.0f, 0.0f};
     struct Block {
-        floatx4 w[NT][4], a[GROUPS];
+        floatx4 w[NT][4], a[SIXTEENS * GROUPS];
     };
     auto load = [&](int k0, Block& block) {
         const int at = offset_below(k0 + col * 4, k);
@@ -182,7 +185,7 @@ __global__ __launch_bounds__(256) void gemm_f32_few_kernel(const float* __restri
             for (int g = 0; g < 4; ++g)
                 block.w[nt][g] = __builtin_bit_cast(floatx4, __builtin_amdgcn_raw_buffer_load_b128(w_rsrc, (16 * nt + 4 * g + quad) * ld * 4 + at, 0, kNonTemporal));
 #pragma unroll
-        for (int g = 0; g < GROUPS; ++g)
+        for (int g = 0; g < SIXTEENS * GROUPS; ++g)
             block.a[g] = __builtin_bit_cast(floatx4, __builtin_amdgcn_raw_buffer_load_b128(a_rsrc, (4 * g + quad) * ld * 4 + at, 0, 0));
     };
     auto put = [&](float (*rows)[kFewRow], int g, const floatx4& v) {
@@ -193,7 +196,7 @@ __global__ __launch_bounds__(256) void gemm_f32_few_kernel(const float* __restri
         // LDS takes a wave's accesses in order; the fences keep the compiler to it.
         __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
 #pragma unroll
-        for (int g = 0; g < GROUPS; ++g) put(shared[wave][NT], g, block.a[g]);
+        for (int g = 0; g < SIXTEENS * GROUPS; ++g) put(shared[wave][NT + g / GROUPS], g % GROUPS, block.a[g]);
 #pragma unroll
         for (int nt = 0; nt < NT; ++nt)
 #pragma unroll
@@ -201,14 +204,20 @@ __global__ __launch_bounds__(256) void gemm_f32_few_kernel(const float* __restri
         __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
 #pragma unroll
         for (int part = 0; part < 4; ++part) {
-            const floatx4 av = *reinterpret_cast<const floatx4*>(&shared[wave][NT][col % (4 * GROUPS)][16 * quad + 4 * part]);
+            floatx4 av[SIXTEENS];
+#pragma unroll
+            for (int s = 0; s < SIXTEENS; ++s)
+                av[s] = *reinterpret_cast<const floatx4*>(&shared[wave][NT + s][col % (4 * GROUPS)][16 * quad + 4 * part]);
             floatx4 wv[NT];
 #pragma unroll
             for (int nt = 0; nt < NT; ++nt) wv[nt] = *reinterpret_cast<const floatx4*>(&shared[wave][nt][col][16 * quad + 4 * part]);
 #pragma unroll
             for (int step = 0; step < 4; ++step)
 #pragma unroll
-                for (int nt = 0; nt < NT; ++nt) acc[nt] = __builtin_amdgcn_mfma_f32_16x16x4f32(wv[nt][step], av[step], acc[nt], 0, 0, 0);
+                for (int nt = 0; nt < NT; ++nt)
+#pragma unroll
+                    for (int s = 0; s < SIXTEENS; ++s)
+                        acc[nt][s] = __builtin_amdgcn_mfma_f32_16x16x4f32(wv[nt][step], av[s][step], acc[nt][s], 0, 0, 0);
         }
     };
     Block even, odd;
@@ -225,29 +234,33 @@ __global__ __launch_bounds__(256) void gemm_f32_few_kernel(const float* __restri
     }
     multiply(even);
     multiply(odd);
-    // acc[nt][i] = C[row col][column first + 16 nt + 4 quad + i]; columns of rows that are none hold other rows' sums
+    // acc[nt][s][i] = C[row row0 + 16 s + col][column first + 16 nt + 4 quad + i]; columns of rows that are none hold other rows' sums
 #pragma unroll
     for (int nt = 0; nt < NT; ++nt)
 #pragma unroll
-        for (int i = 0; i < 4; ++i) {
-            const int column = first + 16 * nt + 4 * quad + i;
-            if (col < m && column < n) c[static_cast<int64_t>(col) * n + column] = acc[nt][i] + (bias ? bias[column] : 0.0f);
-        }
+        for (int s = 0; s < SIXTEENS; ++s)
+#pragma unroll
+            for (int i = 0; i < 4; ++i) {
+                const int column = first + 16 * nt + 4 * quad + i, row = 16 * s + col;
+                if (row < rows && column < n) c[static_cast<int64_t>(row0 + row) * n + column] = acc[nt][s][i] + (bias ? bias[column] : 0.0f);
+            }
 }
 
 template <int NT>
 static void launch_few(const float* a, const float* w, const float* bias, float* c, int m, int n, int k, int k_split,
                        unsigned parts, hipStream_t stream) {
-    const dim3 grid((n + 64 * NT - 1) / (64 * NT), 1, parts);
-    if (m <= 4) gemm_f32_few_kernel<NT, 1><<<grid, 256, 0, stream>>>(a, w, bias, c, m, n, k, k_split);
-    else if (m <= 8) gemm_f32_few_kernel<NT, 2><<<grid, 256, 0, stream>>>(a, w, bias, c, m, n, k, k_split);
-    else gemm_f32_few_kernel<NT, 4><<<grid, 256, 0, stream>>>(a, w, bias, c, m, n, k, k_split);
+    const dim3 grid((n + 64 * NT - 1) / (64 * NT), m <= 16 ? 1 : (m + 31) / 32, parts);
+    if (m <= 4) gemm_f32_few_kernel<NT, 1, 1><<<grid, 256, 0, stream>>>(a, w, bias, c, m, n, k, k_split);
+    else if (m <= 8) gemm_f32_few_kernel<NT, 2, 1><<<grid, 256, 0, stream>>>(a, w, bias, c, m, n, k, k_split);
+    else if (m <= 16) gemm_f32_few_kernel<NT, 4, 1><<<grid, 256, 0, stream>>>(a, w, bias, c, m, n, k, k_split);
+    else gemm_f32_few_kernel<NT, 4, 2><<<grid, 256, 0, stream>>>(a, w, bias, c, m, n, k, k_split);
 }
 
 // Tiles of 16 x 32 for more than 16 rows of small weights, where tiles of the matrix units would be a handful of workgroups,
 // each waiting for one chunk of k after the other: a thread takes 2 x 2 elements (rows r and r + 8, columns c and c + 16), each summed by
 // that thread alone in ascending k. Chunks of 128 of k lie in LDS as [row][k] with rows four banks apart, so that a thread's
 // four consecutive k are one read and the rows a wave reads at one k fall on different banks.
+constexpr int64_t kFewBelow = 128;      // workgroups of the matrix units' tiles
 constexpr int64_t kGrainBelow = 64;     // workgroups of the matrix units' tiles (64 x 896 x 1152, 36 of them: 13.4 us there, 12.2 here; 24 x 896 x 9728, 76: 17.2 and 20.7)
 template <bool VECTOR>
 __global__ __launch_bounds__(128) void gemm_f32_grain_kernel(const float* __restrict__ a, const float* __restrict__ w,
@@ -560,7 +573,7 @@ extern "C" int mll_gemm_f32(const float* a, const float* w, const float* bias, f
     const unsigned parts = static_cast<unsigned>(splits);
     const bool vector = k % 4 == 0 && k <= kWidestVector && reinterpret_cast<uintptr_t>(a) % 16 == 0 && reinterpret_cast<uintptr_t>(w) % 16 == 0;
     const int64_t waves = static_cast<int64_t>((n + 15) / 16) * splits;
-    if (m <= 16 && vector && f32_small_variant == 0 && waves >= kFewWaves) {
+    if (m <= 32 && vector && waves >= kFewWaves && (m > 16 || f32_small_variant == 0)) {
         if (n >= kWideFrom && m > 8) launch_few<2>(a, w, bias, c, m, n, k, k_split, parts, stream);
         else launch_few<1>(a, w, bias, c, m, n, k, k_split, parts, stream);
         return check_launch("gemm_f32");
@@ -594,12 +607,12 @@ extern "C" int mll_gemm_f32(const float* a, const float* w, const float* bias, f
         return check_launch("gemm_f32");
     }
     // The tile whose workgroups fill the compute units best: the matrix units' time is the rounds of 256 workgroups times
-    // a tile's size. Up to 32 rows there is one row of tiles.
+    // a tile's size. Up to 32 rows take tiles of 32 rows (32 x 9728 x 896 in tiles of 64 x 64 26.6 us, of 32 x 128 17.7).
     struct Shape { int rows, columns; };
     const Shape shapes[4] = {{128, 128}, {128, 64}, {64, 64}, {32, 128}};
     int best = 3;
     double least = 1e300;
-    for (int index = 0; index < 4; ++index) {
+    for (int index = m <= 32 ? 3 : 0; index < 4; ++index) {
         const Shape& shape = shapes[index];
         const int64_t groups = static_cast<int64_t>((n + shape.columns - 1) / shape.columns) * ((m + shape.rows - 1) / shape.rows) * splits;
         const double rounds = groups >= 4096 ? groups / 256.0 : static_cast<double>((groups + 255) / 256);
@@ -607,7 +620,14 @@ extern "C" int mll_gemm_f32(const float* a, const float* w, const float* bias, f
         if (cost < least) least = cost, best = index;
     }
     const Shape& shape = shapes[best];
-    if (static_cast<int64_t>((n + shape.columns - 1) / shape.columns) * ((m + shape.rows - 1) / shape.rows) * splits < kGrainBelow) {
+    const int64_t tiles = static_cast<int64_t>((n + shape.columns - 1) / shape.columns) * ((m + shape.rows - 1) / shape.rows) * splits;
+    // Few tiles: 32 rows a wave and several groups of rows, each reading W from the caches: 64 x 896 x 4864 in eight parts, 112 tiles, 19.6 us
+    // in them, 13.5 so; 64 x 896 x 9728, 152 tiles, 22.8 and 25.4; 48 x 896 x 1152 in two 11.4 in the small tiles below, 10.5 so.
+    if (tiles < kFewBelow && m <= 128 && vector && waves * ((m + 31) / 32) >= kFewWaves / 2) {
+        launch_few<1>(a, w, bias, c, m, n, k, k_split, parts, stream);
+        return check_launch("gemm_f32");
+    }
+    if (tiles < kGrainBelow) {
         const dim3 grid((n + 31) / 32, (m + 15) / 16, parts);
         if (vector) gemm_f32_grain_kernel<true><<<grid, 128, 0, stream>>>(a, w, bias, c, m, n, k, k_split);
         else gemm_f32_grain_kernel<false><<<grid, 128, 0, stream>>>(a, w, bias, c, m, n, k, k_split);

@@ -497,7 +497,7 @@ def paged_attention_rowwise(q: torch.Tensor, k_cache: torch.Tensor, v_cache: tor
     else:
         chunks = 0      # one chunk a row: the wave per row is the wave per chunk
     _check(lib.mll_paged_attention_rowwise(_ptr(q), _code(q.dtype), _ptr(k_cache), _ptr(v_cache), _ptr(block_table),
-                                           block_table.shape[1], _ptr(seq_of_token), _ptr(positions), _ptr(out),
+                                           block_table.shape[0], block_table.shape[1], _ptr(seq_of_token), _ptr(positions), _ptr(out),
                                            _ptr(part_o), _ptr(part_ml), chunks, usual_chunks, ctypes.c_float(scale), int(window),
                                            n_tokens, heads, kv_heads, head_dim, page_size, _stream()), lib)
     return out
