@@ -545,6 +545,7 @@ static int tiles_per_group(int m, int n_tiles) {
 template <int EPILOGUE>
 static int launch_skinny(const void* a, const void* w_packed, void* out, int m, int n, int k,
                          const MllSkinnyExtras& extras, hipStream_t stream) {
+    MLL_REQUIRE(k <= 1 << 23, "gemm_skinny: the reduction is too long for 32-bit offsets");
     const int n_tiles = (n + 15) / 16;
     const int k_steps = (k + 31) / 32;
     const bf16* a_ = static_cast<const bf16*>(a);

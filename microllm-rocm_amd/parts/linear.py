@@ -5,8 +5,9 @@ The reference stores ``[in, out]`` and transposes every linear at load
 lets several weights that share an input be stacked along ``out``. A bfloat16
 weight is held twice on the GPU: as stored, for the library product that steps
 with many rows use, and packed in the order the MFMA consumes it, for the two
-kernels that stream it once when a step has few rows (decoding): one for up to
-16 rows, one that shares the activations between waves for up to 64.
+kernels that stream it once when a step has few rows (decoding), one for up to
+16 rows, one that shares the activations between waves for up to 64, and for the
+tiled product where a prompt's gated product is better there.
 """
 from __future__ import annotations
 
@@ -42,7 +43,9 @@ MEDIUM_ROWS = 64        # and up to this many gemm_medium does: at 17, 32 and 64
                         # 1.53, 16384 x 2048 gated 1.42, 1.37 and 1.10, 3584 x 18944 4.2, 4.1 and 2.9; except for
 MEDIUM_WIDE_TILES = 2048   # weights with this many tiles of 16 rows or more that are not gated (the head), where the library is
 MEDIUM_WIDE_ROWS = 40      # nearly as fast beyond this many: 152064 x 3584 at 32, 48 and 64 rows 1.37, 1.05 and 1.06
-MEDIUM_GATED_ROWS = MEDIUM_ROWS
+MEDIUM_GATED_ROWS = 48     # gated weights with fewer tiles than compute units stay with the library from here on. It is 2 to 3 us a
+MEDIUM_GATED_TILES = 256   # layer slower (64 rows: 1024 x 256 7.7 and 5.4, 4080 x 512 9.2 and 6.9), but rounds gate and up, and steps of
+                           # 49 to 64 rows of the smallest models keep the results that they have always had
 
 
 @dataclass
@@ -94,9 +97,10 @@ def takes_packed(weight: "Weight", rows: int, gated: bool = False) -> bool:
         return False
     if rows <= SKINNY_ROWS or weight.tensor is None:
         return True
+    tiles = -(-weight.out_features // 16)
     if gated:
-        return rows <= MEDIUM_GATED_ROWS
-    wide = -(-weight.out_features // 16) >= MEDIUM_WIDE_TILES
+        return rows <= (MEDIUM_ROWS if tiles >= MEDIUM_GATED_TILES else MEDIUM_GATED_ROWS)
+    wide = tiles >= MEDIUM_WIDE_TILES
     return rows <= (MEDIUM_WIDE_ROWS if wide else MEDIUM_ROWS)
 
 
