@@ -39,17 +39,24 @@ gla_decay_kernel(const float* __restrict__ proj, int64_t proj_stride, int low_of
 #pragma unroll
     for (int t = 0; t < kDecayTokens; ++t) z[t] = bias ? bias[c] : 0.0f;
     for (int r0 = 0; r0 < rank; r0 += kDecayRank) {
-        float weight[kDecayRank];       // past the row: zero times its last number
+        float weight[kDecayRank];       // past the row: its last number, left out below
 #pragma unroll
-        for (int r = 0; r < kDecayRank; ++r) {
-            const float value = to_float(a2[static_cast<int64_t>(c) * rank + min(r0 + r, rank - 1)]);
-            weight[r] = r0 + r < rank ? value : 0.0f;
-        }
+        for (int r = 0; r < kDecayRank; ++r) weight[r] = to_float(a2[static_cast<int64_t>(c) * rank + min(r0 + r, rank - 1)]);
+        const bool whole = r0 + kDecayRank <= rank;
 #pragma unroll
         for (int t = 0; t < kDecayTokens; ++t) {
             const float* low = proj + static_cast<int64_t>(min(first + t, n_tokens - 1)) * proj_stride + low_offset;
+            if (whole) {
 #pragma unroll
-            for (int r = 0; r < kDecayRank; ++r) z[t] = fmaf(weight[r], low[min(r0 + r, rank - 1)], z[t]);
+                for (int r = 0; r < kDecayRank; ++r) z[t] = fmaf(weight[r], low[r0 + r], z[t]);
+            } else {
+                // A weight of zero would not do: the row's last number may be infinite.
+#pragma unroll
+                for (int r = 0; r < kDecayRank; ++r) {
+                    const float more = fmaf(weight[r], low[min(r0 + r, rank - 1)], z[t]);
+                    z[t] = r0 + r < rank ? more : z[t];
+                }
+            }
         }
     }
 #pragma unroll

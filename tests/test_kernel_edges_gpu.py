@@ -160,3 +160,27 @@ def test_product_for_64_rows_by_tiles_a_workgroup(n, k):
     assert (np.abs(whole.double().cpu().numpy() - x_exact @ w_exact.T) <= bound).all()
     for m in (16, 17, 33, 48):
         assert torch.equal(kernels().gemm_medium(x[:m].contiguous(), packed, n, "f32", plan=plan), whole[:m]), m
+
+
+@pytest.mark.parametrize("rank", [1, 4, 15, 16, 17, 20, 32, 37])
+@pytest.mark.parametrize("n_tokens", [1, 7, 8, 9, 600])
+def test_decays_of_every_rank_and_of_infinite_inputs(rank, n_tokens):
+    """Whole and broken groups of 16 numbers of the low rank, whole and broken groups of tokens. An input that is infinite drives
+    a channel's decay to zero or one by its weight's sign; one that is no number leaves none."""
+    rng = np.random.default_rng(rank)
+    channels, tau, offset = 130, 16.0, 3
+    low, a2, bias = rng.normal(size=(n_tokens, rank)), rng.normal(size=(channels, rank)), rng.normal(size=channels)
+    low[n_tokens - 1, rank - 1] = np.inf
+    low[n_tokens // 2, 0] = -np.inf
+    proj = np.concatenate([rng.normal(size=(n_tokens, offset)), low], axis=1).astype(np.float32)
+    low, a2, bias = (value.astype(np.float32).astype(np.float64) for value in (low, a2, bias))
+    with np.errstate(over="ignore", invalid="ignore"):      # infinity less infinity, where one token and one number have both
+        z = low @ a2.T + bias
+        logs = -np.logaddexp(0.0, -z) / tau
+    for base_two, want in ((False, np.exp(logs)), (True, logs / math.log(2.0))):
+        got = kernels().gla_decay(device(proj), offset, device(a2), device(bias), tau, base_two=base_two).double().cpu().numpy()
+        # rank + 2 roundings of z's terms and a few of the logarithm's and the power's own
+        bound = (rank + 8) * 2 * F32_STEP * (np.abs(np.nan_to_num(low, posinf=0, neginf=0)) @ np.abs(a2).T + np.abs(bias) + 1.0)
+        finite = np.isfinite(want)
+        assert (np.abs(got[finite] - want[finite]) <= bound[finite]).all()
+        np.testing.assert_array_equal(np.where(finite, 0.0, got), np.where(finite, 0.0, want))
