@@ -23,44 +23,44 @@ constexpr int kWideHeadRows = 8;
 constexpr int kUsualRows = 4;
 
 // decay[t, c] = exp(log_sigmoid(z) / tau), z = bias[c] + sum_r a2[c, r] * low[t, r]; with `base_two` the exponent's
-// logarithm to base two instead. A thread keeps its channel's row of a2 for kDecayTokens tokens (a row apiece for every token
-// and channel were 2-byte loads a row apart: 3117 tokens of 512 channels 60 -> 18 us), 16 numbers of it at a time.
-constexpr int kDecayTokens = 8;
+// logarithm to base two instead. A thread takes a channel of TOKENS tokens and 16 numbers of its row of a2 at a time, all asked for
+// before the first is used. Few tokens are bound by the waits: one a thread (8 tokens of 512 channels, rank 16: 3.8 us, eight a
+// thread 6.0, one number at a time 4.7). Many by reading a2, which eight tokens then share: from kDecaySeveral multiplications on (2000
+// tokens of 512 channels, rank 16: one 8.1, eight 8.3; rank 32: 18.6 and 9.6; 3117 of 2048, rank 16: 31.3 and 27.2). The same bits.
+constexpr int64_t kDecaySeveral = 1 << 24;
 constexpr int kDecayRank = 16;
-template <typename W>
+template <typename W, int TOKENS>
 __global__ void __launch_bounds__(128)
 gla_decay_kernel(const float* __restrict__ proj, int64_t proj_stride, int low_offset, int rank,
                  const W* __restrict__ a2, const float* __restrict__ bias, float inv_tau,
                  float* __restrict__ decay, int channels, int n_tokens, int base_two) {
-    const int first = blockIdx.y * kDecayTokens;
+    const int first = blockIdx.y * TOKENS;
     const int c = blockIdx.x * blockDim.x + threadIdx.x;
     if (c >= channels) return;
-    float z[kDecayTokens];
+    float z[TOKENS];
 #pragma unroll
-    for (int t = 0; t < kDecayTokens; ++t) z[t] = bias ? bias[c] : 0.0f;
-    for (int r0 = 0; r0 < rank; r0 += kDecayRank) {
-        float weight[kDecayRank];       // past the row: its last number, left out below
+    for (int t = 0; t < TOKENS; ++t) z[t] = bias ? bias[c] : 0.0f;
+    const W* row = a2 + static_cast<int64_t>(c) * rank;
+    int r0 = 0;
+    for (; r0 + kDecayRank <= rank; r0 += kDecayRank) {
+        float weight[kDecayRank];
 #pragma unroll
-        for (int r = 0; r < kDecayRank; ++r) weight[r] = to_float(a2[static_cast<int64_t>(c) * rank + min(r0 + r, rank - 1)]);
-        const bool whole = r0 + kDecayRank <= rank;
+        for (int r = 0; r < kDecayRank; ++r) weight[r] = to_float(row[r0 + r]);
 #pragma unroll
-        for (int t = 0; t < kDecayTokens; ++t) {
-            const float* low = proj + static_cast<int64_t>(min(first + t, n_tokens - 1)) * proj_stride + low_offset;
-            if (whole) {
+        for (int t = 0; t < TOKENS; ++t) {
+            const float* low = proj + static_cast<int64_t>(min(first + t, n_tokens - 1)) * proj_stride + low_offset + r0;
 #pragma unroll
-                for (int r = 0; r < kDecayRank; ++r) z[t] = fmaf(weight[r], low[r0 + r], z[t]);
-            } else {
-                // A weight of zero would not do: the row's last number may be infinite.
-#pragma unroll
-                for (int r = 0; r < kDecayRank; ++r) {
-                    const float more = fmaf(weight[r], low[min(r0 + r, rank - 1)], z[t]);
-                    z[t] = r0 + r < rank ? more : z[t];
-                }
-            }
+            for (int r = 0; r < kDecayRank; ++r) z[t] = fmaf(weight[r], low[r], z[t]);
         }
     }
+    for (; r0 < rank; ++r0) {       // one by one: a weight of zero past the row would make an infinite input no number
+        const float weight = to_float(row[r0]);
 #pragma unroll
-    for (int t = 0; t < kDecayTokens; ++t) {
+        for (int t = 0; t < TOKENS; ++t)
+            z[t] = fmaf(weight, proj[static_cast<int64_t>(min(first + t, n_tokens - 1)) * proj_stride + low_offset + r0], z[t]);
+    }
+#pragma unroll
+    for (int t = 0; t < TOKENS; ++t) {
         if (first + t >= n_tokens) break;
         // log(sigmoid(z)) = -(max(-z, 0) + log1p(exp(-|z|)))
         const float log_sigmoid = -(fmaxf(-z[t], 0.0f) + log1pf(expf(-fabsf(z[t]))));
@@ -351,16 +351,20 @@ int mll_gla_decay(const float* proj, int64_t proj_stride, int low_offset, int ra
     MLL_REQUIRE(low_offset >= 0 && low_offset + rank <= proj_stride, "gla_decay: the low-rank input lies outside its row");
     if (n_tokens == 0) return 0;
     MLL_REQUIRE(n_tokens <= 65535, "gla_decay: more than 65535 tokens in one call");
-    const dim3 grid((channels + 127) / 128, (n_tokens + kDecayTokens - 1) / kDecayTokens);
-    if (a2_dtype == kF32) {
-        gla_decay_kernel<float><<<grid, 128, 0, stream>>>(proj, proj_stride, low_offset, rank, static_cast<const float*>(a2), bias,
-                                                         1.0f / tau, decay, channels, n_tokens, base_two);
-    } else if (a2_dtype == kBF16) {
-        gla_decay_kernel<bf16><<<grid, 128, 0, stream>>>(proj, proj_stride, low_offset, rank, static_cast<const bf16*>(a2), bias,
-                                                        1.0f / tau, decay, channels, n_tokens, base_two);
-    } else {
-        return fail("gla_decay: unknown weight dtype");
-    }
+    MLL_REQUIRE(a2_dtype == kF32 || a2_dtype == kBF16, "gla_decay: unknown weight dtype");
+    const auto launch = [&](auto element, auto tokens) {
+        using W = decltype(element);
+        constexpr int kTokens = decltype(tokens)::value;
+        const dim3 grid((channels + 127) / 128, (n_tokens + kTokens - 1) / kTokens);
+        gla_decay_kernel<W, kTokens><<<grid, 128, 0, stream>>>(proj, proj_stride, low_offset, rank, static_cast<const W*>(a2), bias, 1.0f / tau,
+                                                               decay, channels, n_tokens, base_two);
+    };
+    const auto launch_tokens = [&](auto element) {
+        if (static_cast<int64_t>(n_tokens) * channels * rank >= kDecaySeveral) launch(element, std::integral_constant<int, 8>{});
+        else launch(element, std::integral_constant<int, 1>{});
+    };
+    if (a2_dtype == kF32) launch_tokens(float{});
+    else launch_tokens(bf16{});
     return check_launch("gla_decay");
 }
 

@@ -163,7 +163,7 @@ def test_product_for_64_rows_by_tiles_a_workgroup(n, k):
 
 
 @pytest.mark.parametrize("rank", [1, 4, 15, 16, 17, 20, 32, 37])
-@pytest.mark.parametrize("n_tokens", [1, 7, 8, 9, 600])
+@pytest.mark.parametrize("n_tokens", [1, 7, 8, 9, 600, 33001])       # the last: several tokens a thread from rank 4 on
 def test_decays_of_every_rank_and_of_infinite_inputs(rank, n_tokens):
     """Whole and broken groups of 16 numbers of the low rank, whole and broken groups of tokens. An input that is infinite drives
     a channel's decay to zero or one by its weight's sign; one that is no number leaves none."""
