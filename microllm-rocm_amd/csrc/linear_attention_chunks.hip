@@ -388,6 +388,9 @@ gla_channel_out_kernel(const float* __restrict__ proj, int64_t proj_stride, int 
 #pragma unroll
         for (int i = 0; i < 4; ++i) weights[kPart * wave + 4 * quad + i][kPart * part + col] = acc[i];
     }
+    // What other lanes of the wave wrote to `weights` is read below: LDS takes a wave's accesses in order, the fence keeps the
+    // compiler to it (it could tell a thread's own stores from the loads and move these up).
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
     const float* from = starts + (static_cast<int64_t>(number) * heads + head) * key_dim * value_dim;
     float decayed[kChannelKeys / 4];        // 2^B_t q_t: the operand that meets the state
 #pragma unroll
