@@ -19,8 +19,9 @@
 //
 // and a chunk leaves 2^B_n S + sum_j (2^(B_n - B_j) k_j) v_j^T. No power has a positive exponent, so none overflows whatever
 // the decays: 16 tokens among themselves take 2^(B_t - B_j) pair by pair, with those before them the query takes
-// 2^(B_t - B_r) and the key 2^(B_r - B_j), r being the last token before the 16. The sums are kept within parts of 16
-// tokens, so that a difference of two of them loses little.
+// 2^(B_t - B_r) and the key 2^(B_r - B_j), r being the last token before the 16. Every exponent is the sum of the logarithms
+// between its two tokens, never a difference of two sums: after a token that leaves nothing (-150) a difference would keep
+// 1e-5 of the small logarithms that follow it.
 #include "common.h"
 #include "microllm_hip.h"
 
@@ -211,9 +212,10 @@ gla_chunk_out_kernel(const float* __restrict__ proj, int64_t proj_stride, int q_
 }
 
 // ---- a decay a key channel and token -------------------------------------------------------------------------------
-// Two requests of 2000 and 1117 tokens, 8 heads of 64 x 128: 287 us by the walk, 73 here (results 47, states 15, walk over the
-// chunks 11), bound by one workgroup's chain of LDS reads and products. Sums run in four chains, which both shortens the waits and
-// keeps the error against float64 below the walk's: 1.25e-7 (root mean square, of the results') against 1.65e-7 at 512 tokens.
+// Two requests of 2000 and 1117 tokens, 8 heads of 64 x 128: 285 us by the walk, 78 here, bound by one workgroup's chain of LDS
+// reads and products. Sums run in four chains, which both shortens the waits and keeps the error against float64 below the walk's
+// for ordinary decays: 1.2e-7 (root mean square, of the results') against 1.65e-7 at 512 tokens; where strong and slow decays
+// meet both err by a few 1e-7 (with exponents as differences of sums, 5 us faster, it was 1e-5 of the largest result).
 constexpr int kChannelKeys = 64;        // the widest key heads here: queries, keys and decays of a chunk lie in LDS together
 
 constexpr int kPart = 16;
@@ -222,20 +224,46 @@ constexpr int kParts = kScanChunk / kPart;
 // A chunk's logarithms. Below 2^-149 a factor is zero in float32, and a sum of larger numbers would lose the others' digits.
 __device__ inline float usable_log(float value) { return value < -150.0f ? -150.0f : value; }
 
-// `sums[t][c]`: logarithms to their sums from their part's first token on, in place; whole[part][c]: the part's sum. Called by
-// every thread; the first and last things it does are barriers.
-__device__ inline void sum_parts(float (*sums)[kChannelKeys + 1], float (*whole)[kChannelKeys]) {
+// whole[part][c]: the sum of a part's logarithms `logs[t][c]`; with AFTER, logs[t][c] becomes the sum of those after it in its
+// part. Called by every thread; the first and last things it does are barriers.
+template <bool AFTER>
+__device__ inline void sum_parts(float (*logs)[kChannelKeys + 1], float (*whole)[kChannelKeys]) {
     const int c = threadIdx.x % kChannelKeys, part = threadIdx.x / kChannelKeys;
     static_assert(kScanThreads == kParts * kChannelKeys, "a thread a channel and part");
     __syncthreads();
     float total = 0.0f;
 #pragma unroll
-    for (int t = 0; t < kPart; ++t) {
-        total += sums[kPart * part + t][c];
-        sums[kPart * part + t][c] = total;
+    for (int t = kPart - 1; t >= 0; --t) {
+        const float own = logs[kPart * part + t][c];
+        if (AFTER) logs[kPart * part + t][c] = total;
+        total += own;
     }
     whole[part][c] = total;
     __syncthreads();
+}
+
+// The value of the lane STEPS before, or after, within every 16 lanes; 0 where there is none.
+template <int STEPS>
+__device__ inline float lane_before(float value) {
+    return __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, value), 0x110 + STEPS, 0xf, 0xf, false));
+}
+template <int STEPS>
+__device__ inline float lane_after(float value) {
+    return __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, value), 0x100 + STEPS, 0xf, 0xf, false));
+}
+// The sum of the lanes up to this one, or of those after it, within every 16 lanes (all lanes of the wave come here).
+__device__ inline float sum_up_to(float value) {
+    value += lane_before<1>(value);
+    value += lane_before<2>(value);
+    value += lane_before<4>(value);
+    return value + lane_before<8>(value);
+}
+__device__ inline float sum_after(float value) {
+    value = lane_after<1>(value);
+    value += lane_after<1>(value);
+    value += lane_after<2>(value);
+    value += lane_after<4>(value);
+    return value + lane_after<8>(value);
 }
 
 // whole[first] + .. + whole[last - 1] of channel c.
@@ -266,10 +294,10 @@ gla_channel_state_kernel(const float* __restrict__ proj, int64_t proj_stride, in
                                         key_dim, [&](int t, int c, float value) { sums[t][c] = usable_log(value); });
     load_tile<kScanChunk, kChannelKeys>(row + k_offset + head * key_dim, proj_stride, count, key_dim,
                                         [&](int t, int c, float value) { keys[t][c] = value; });
-    sum_parts(sums, parts);
+    sum_parts<true>(sums, parts);
     for (int index = threadIdx.x; index < kScanChunk * kChannelKeys; index += kScanThreads) {
         const int t = index / kChannelKeys, c = index % kChannelKeys, part = t / kPart;
-        keys[t][c] *= power_of_two(parts[part][c] - sums[t][c] + sum_between(parts, part + 1, kParts, c));
+        keys[t][c] *= power_of_two(sums[t][c] + sum_between(parts, part + 1, kParts, c));
     }
     if (threadIdx.x < key_dim)
         whole[(static_cast<int64_t>(number) * heads + head) * key_dim + threadIdx.x] = power_of_two(sum_between(parts, 0, kParts, threadIdx.x));
@@ -339,7 +367,7 @@ gla_channel_out_kernel(const float* __restrict__ proj, int64_t proj_stride, int 
                        float* __restrict__ out, int n_seqs, int heads, int key_dim, int value_dim, float q_scale) {
     __shared__ float queries[kScanChunk][kChannelKeys + 1];
     __shared__ float keys[kScanChunk][kChannelKeys + 1];
-    __shared__ float sums[kScanChunk][kChannelKeys + 1];
+    __shared__ float logs[kScanChunk][kChannelKeys + 1];
     __shared__ float weights[kScanChunk][kScanChunk + 1];
     __shared__ float parts[kParts][kChannelKeys];
     const int number = blockIdx.x, head = blockIdx.y;
@@ -349,12 +377,12 @@ gla_channel_out_kernel(const float* __restrict__ proj, int64_t proj_stride, int 
     const int col = lane % 16, quad = lane / 16;
     const float* row = proj + first * proj_stride;
     load_tile<kScanChunk, kChannelKeys>(log_decay + (static_cast<int64_t>(first) * heads + head) * key_dim, static_cast<int64_t>(heads) * key_dim, count,
-                                        key_dim, [&](int t, int c, float value) { sums[t][c] = usable_log(value); });
+                                        key_dim, [&](int t, int c, float value) { logs[t][c] = usable_log(value); });
     load_tile<kScanChunk, kChannelKeys>(row + q_offset + head * key_dim, proj_stride, count, key_dim,
                                         [&](int t, int c, float value) { queries[t][c] = value; });
     load_tile<kScanChunk, kChannelKeys>(row + k_offset + head * key_dim, proj_stride, count, key_dim,
                                         [&](int t, int c, float value) { keys[t][c] = value; });
-    sum_parts(sums, parts);
+    sum_parts<false>(logs, parts);
     const int own = kPart * wave + col;     // the token whose query this lane holds as a row of the first operand
     // weights[t][j] = sum_d q_t[d] k_j[d] 2^(B_t[d] - B_j[d]) for j <= t: the wave's tokens among themselves, four pairs a lane ...
     {
@@ -362,26 +390,33 @@ gla_channel_out_kernel(const float* __restrict__ proj, int64_t proj_stride, int 
         for (int d0 = 0; d0 < key_dim; d0 += 4)
 #pragma unroll
             for (int d = 0; d < 4; ++d) {       // channels past the head are zero
-                const float q = queries[own][d0 + d], b = sums[own][d0 + d];
+                const float q = queries[own][d0 + d], log = logs[own][d0 + d];
+                // the logarithms after the lane's four keys up to its token, then with those between the keys as well
+                float exponent = sum_up_to(col > 4 * quad + 3 ? log : 0.0f);
 #pragma unroll
-                for (int i = 0; i < 4; ++i) {
+                for (int i = 3; i >= 0; --i) {
                     const int j = kPart * wave + 4 * quad + i;
-                    pair[d][i] = fmaf(q * keys[j][d0 + d], power_of_two(fminf(b - sums[j][d0 + d], 0.0f)), pair[d][i]);
+                    pair[d][i] = fmaf(q * keys[j][d0 + d], power_of_two(exponent), pair[d][i]);
+                    exponent += 4 * quad + i <= col ? logs[j][d0 + d] : 0.0f;
                 }
             }
 #pragma unroll
         for (int i = 0; i < 4; ++i) weights[own][kPart * wave + 4 * quad + i] = 4 * quad + i <= col ? (pair[0][i] + pair[1][i]) + (pair[2][i] + pair[3][i]) : 0.0f;
     }
     // ... and with the parts before them
+    float up_to[kChannelKeys / 4];          // B_t - B_r
     float reaching[kChannelKeys / 4];       // 2^(B_t - B_r) q_t
 #pragma unroll
-    for (int d = 0; d < kChannelKeys; d += 4) reaching[d / 4] = queries[own][d + quad] * power_of_two(sums[own][d + quad]);
+    for (int d = 0; d < kChannelKeys; d += 4) {
+        up_to[d / 4] = sum_up_to(logs[own][d + quad]);
+        reaching[d / 4] = queries[own][d + quad] * power_of_two(up_to[d / 4]);
+    }
     for (int part = 0; part < wave; ++part) {
         floatx4 sum[4] = {};
 #pragma unroll
         for (int d = 0; d < kChannelKeys; d += 4) {
             const int c = d + quad, j = kPart * part + col;
-            const float k = keys[j][c] * power_of_two(parts[part][c] - sums[j][c] + sum_between(parts, part + 1, wave, c));
+            const float k = keys[j][c] * power_of_two(sum_after(logs[j][c]) + sum_between(parts, part + 1, wave, c));
             sum[d / 4 % 4] = __builtin_amdgcn_mfma_f32_16x16x4f32(reaching[d / 4], k, sum[d / 4 % 4], 0, 0, 0);
         }
         const floatx4 acc = (sum[0] + sum[1]) + (sum[2] + sum[3]);
@@ -394,7 +429,7 @@ gla_channel_out_kernel(const float* __restrict__ proj, int64_t proj_stride, int 
     const float* from = starts + (static_cast<int64_t>(number) * heads + head) * key_dim * value_dim;
     float decayed[kChannelKeys / 4];        // 2^B_t q_t: the operand that meets the state
 #pragma unroll
-    for (int d = 0; d < kChannelKeys; d += 4) decayed[d / 4] = queries[own][d + quad] * power_of_two(sums[own][d + quad] + sum_between(parts, 0, wave, d + quad));
+    for (int d = 0; d < kChannelKeys; d += 4) decayed[d / 4] = queries[own][d + quad] * power_of_two(up_to[d / 4] + sum_between(parts, 0, wave, d + quad));
     float own_weight[kPart / 4];            // the weights of the wave's tokens among themselves
 #pragma unroll
     for (int j = 0; j < kPart / 4; ++j) own_weight[j] = weights[own][kPart * wave + 4 * j + quad];

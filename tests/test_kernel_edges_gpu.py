@@ -184,3 +184,33 @@ def test_decays_of_every_rank_and_of_infinite_inputs(rank, n_tokens):
         finite = np.isfinite(want)
         assert (np.abs(got[finite] - want[finite]) <= bound[finite]).all()
         np.testing.assert_array_equal(np.where(finite, 0.0, got), np.where(finite, 0.0, want))
+
+
+@pytest.mark.parametrize("strong_first", [1, 3, 4, 12, 15])
+@pytest.mark.parametrize("strong", [20.0, 150.0, 4000.0])
+def test_chunks_where_slow_decays_follow_strong_ones(strong_first, strong):
+    """Every 16 tokens begin with some that leave (next to) nothing, then decays close to one. A weight between two tokens errs by the
+    roundings of the logarithms between them alone, however strong those before: 2^-24 for each of up to 64 sums of an exponent x,
+    times x log 2 relative to the term; products, powers and the sums over channels and tokens add at most 48 roundings."""
+    rng = np.random.default_rng(strong_first)
+    heads, dim, vdim, n = 2, 4, 8, 64
+    keys, values = heads * dim, heads * vdim
+    q, k, v = (rng.normal(size=(n, heads, size)).astype(np.float32) for size in (dim, dim, vdim))
+    logs = (-0.01 * rng.exponential(size=(n, heads, dim))).astype(np.float32)
+    strong_ones = np.arange(n) % 16 < strong_first
+    logs[strong_ones] = -strong * rng.uniform(0.9, 1.0, size=(strong_ones.sum(), heads, dim))
+    proj = device(np.concatenate([a.reshape(n, -1) for a in (q, k, v)], axis=1))
+    state = torch.zeros((1, heads, dim, vdim), device=DEVICE)
+    got = kernels().gla_channel_chunks(proj, 0, keys, 2 * keys, device(logs.reshape(n, keys)), state, device([0, n], torch.int32), device([0], torch.int32), 1,
+                                       heads, dim, vdim, 1.0).double().cpu().numpy().reshape(n, heads, vdim)
+    q, k, v, logs = (a.astype(np.float64) for a in (q, k, v, logs))
+    before = np.concatenate([np.zeros((1, heads, dim)), np.cumsum(logs, axis=0)])
+    exponents = before[1:, None] - before[None, 1:]                       # [t, j, head, channel]: the logarithms of tokens j + 1 .. t
+    pairs = np.where(np.tri(n, dtype=bool)[:, :, None, None], np.exp2(np.minimum(exponents, 0.0)), 0.0)
+    roundings = 48 + 64 * math.log(2.0) * np.abs(exponents)
+    want = np.einsum("thd,jhd,tjhd,jhv->thv", q, k, pairs, v)
+    bound = np.einsum("thd,jhd,tjhd,jhv->thv", np.abs(q), np.abs(k), pairs * roundings, np.abs(v)) * F32_STEP
+    assert (np.abs(got - want) <= bound).all(), float((np.abs(got - want) / bound).max())
+    left = np.einsum("jhd,jhd,jhv->hdv", k, pairs[-1], v)
+    bound = np.einsum("jhd,jhd,jhv->hdv", np.abs(k), (pairs * roundings)[-1], np.abs(v)) * F32_STEP
+    assert (np.abs(state[0].double().cpu().numpy() - left) <= bound).all()
