@@ -84,15 +84,18 @@ class FixedShape:
     """The shape a step is padded to so that it can be replayed from a graph: rows of tokens, of requests and of
     wanted logits, the block tables' width and the rows of every planner's arrays. Padding rows hold token 0 at
     position 0 of request ``PADDING`` with slot ``PADDING`` (nothing is stored for them and attention passes them
-    over); padding requests hold no tokens; a planner pads its arrays with the values it names in ``padding``."""
+    over); padding requests hold no tokens; a planner pads its arrays with the values it names in ``padding``.
+    ``lines_passed``: how many of the model's ``portion_lines`` the longest portion reaches. Nothing is padded to it; it
+    is part of the shape because kernels are chosen by it."""
     tokens: int
     requests: int
     wanted: int
     width: int
     planned: Mapping[Tuple[Hashable, str], int]
+    lines_passed: int = 0
 
     def key(self) -> tuple:
-        return (self.tokens, self.requests, self.wanted, self.width, tuple(sorted(self.planned.items(), key=repr)))
+        return (self.tokens, self.requests, self.wanted, self.width, tuple(sorted(self.planned.items(), key=repr)), self.lines_passed)
 
 
 class StepPlanner:

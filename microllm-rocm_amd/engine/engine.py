@@ -277,7 +277,9 @@ class Engine:
         wanted = int(batch.want_rows.size)
         if step.n_tokens > MAX_GRAPH_TOKENS or step.n_seqs > MAX_GRAPH_REQUESTS or wanted > MAX_GRAPH_WANTED:
             return None
-        return FixedShape(tokens=_token_rows(step.n_tokens), requests=_power_of_two(step.n_seqs),
+        requests, longest = _power_of_two(step.n_seqs), max(step.counts)
+        return FixedShape(tokens=_token_rows(step.n_tokens), requests=requests,
+                          lines_passed=sum(longest >= line for line in self.model.portion_lines(requests)),
                           wanted=_wanted_rows(wanted), width=_power_of_two(batch.blocks_needed, MIN_GRAPH_WIDTH),
                           planned={name: _power_of_two(rows) if rows else 0 for name, rows in batch.planned_rows().items()})
 

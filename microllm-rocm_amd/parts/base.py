@@ -65,6 +65,13 @@ class Part:
         the step's other metadata; None otherwise. ``ctx.plan_of(planner)`` gives the plan in ``forward``."""
         return None
 
+    def portion_line(self, requests: int) -> Optional[int]:
+        """How many tokens of one request in a step of ``requests`` make this part's kernels sum in another order (a
+        recurrence in chunks instead of token by token); None if none do. The engine keeps the side of the line that a
+        step's longest portion is on in the shape that the step is replayed by, so that it gives the same bits
+        whether it is captured or not."""
+        return None
+
     def flops(self, tokens: int) -> float:
         """Floating-point operations of this part over one request's prompt of ``tokens`` ids (2 per multiply-add);
         by default those of its matrix products: its attributes that are a ``linear.Weight``."""

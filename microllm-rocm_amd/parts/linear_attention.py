@@ -108,6 +108,11 @@ class GatedLinearAttention(Mixer):
             self.decay_row = per_head.repeat_interleave(self.key_dim).contiguous()
         self.norm_weight = tensors[self.name("norm")] if self.has_norm_weight else None
 
+    def portion_line(self, requests: int) -> Optional[int]:
+        if self.chunked:
+            return self.CHUNKED_PORTION
+        return self.CHANNEL_CHUNKED_PORTION if self.channel_chunked else None
+
     def take_output_projection(self) -> Optional[torch.Tensor]:
         tensor, self.o_tensor = self.o_tensor, None
         return tensor
@@ -123,7 +128,9 @@ class GatedLinearAttention(Mixer):
 
     def forward_inner(self, x, ctx, cache, out: Optional[torch.Tensor] = None, out_scale: float = 1.0) -> torch.Tensor:
         proj = linear(x, self.in_weight, out_dtype=torch.float32)
-        if self.channel_chunked and ctx.max_count >= self.CHANNEL_CHUNKED_PORTION:
+        line = self.portion_line(ctx.n_seqs)
+        in_chunks = line is not None and ctx.max_count >= line
+        if self.channel_chunked and in_chunks:
             log_decay = kernels.gla_decay(proj, self.low_at, self.decay_weight, self.decay_bias, self.tau, base_two=True)
             o = kernels.gla_channel_chunks(proj, self.q_at, self.k_at, self.v_at, log_decay, cache.state, ctx.cu_tokens, ctx.slots, ctx.n_seqs,
                                            self.heads, self.key_dim, self.value_dim, self.query_scale)
@@ -133,7 +140,7 @@ class GatedLinearAttention(Mixer):
             decay = kernels.gla_decay(proj, self.low_at, self.decay_weight, self.decay_bias, self.tau)
         else:
             decay = self.decay_row
-        if self.chunked and ctx.max_count >= self.CHUNKED_PORTION:
+        if in_chunks:
             o = kernels.gla_chunks(proj, self.q_at, self.k_at, self.v_at, self.head_decay, cache.state, ctx.cu_tokens, ctx.slots, ctx.n_seqs,
                                    self.heads, self.key_dim, self.value_dim, self.query_scale, silu_inputs=self.silu_inputs)
             return kernels.gla_gate(o, proj, self.g_at, self.norm_weight, self.eps, self.heads, self.value_dim, out_scale,

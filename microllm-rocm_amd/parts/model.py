@@ -7,7 +7,7 @@ reads an earlier entry's. Logits are computed in float32 for the wanted rows onl
 """
 from __future__ import annotations
 
-from typing import Dict, List, Mapping, Optional
+from typing import Dict, List, Mapping, Optional, Tuple
 
 import torch
 
@@ -109,6 +109,7 @@ class Model:
         # Called as observer(run entry, h, pending) after every entry of a step when set (the replay tool's dump of
         # the stream layer by layer; the reference traces tensors by name, include/microllm/profiling/trace.h:63).
         self.observer = None
+        self._portion_lines: Dict[int, Tuple[int, ...]] = {}
 
     # ---- tensors -------------------------------------------------------------------------
     def tensors(self) -> Dict[str, TensorDecl]:
@@ -163,6 +164,14 @@ class Model:
             if planner is not None and all(planner.key != known.key for known in planners):
                 planners.append(planner)
         return planners
+
+    def portion_lines(self, requests: int) -> Tuple[int, ...]:
+        """The lines of all parts (``Part.portion_line``) for a step of ``requests``, ascending."""
+        lines = self._portion_lines.get(requests)
+        if lines is None:
+            lines = tuple(sorted({line for line in (part.portion_line(requests) for part in self.parts()) if line is not None}))
+            self._portion_lines[requests] = lines
+        return lines
 
     def cache_needs(self) -> List[Optional[CacheNeed]]:
         """The cache need of every run entry; None for an entry that owns none."""

@@ -80,6 +80,9 @@ class GatedLinearRecurrence(Mixer):
     def flops(self, tokens: int) -> float:
         return super().flops(tokens) + 2.0 * tokens * self.width * (2 * self.size + self.taps + 8)
 
+    def portion_line(self, requests: int) -> int:
+        return self.LONG_PORTION
+
     def takes_unscaled(self, rows: int) -> bool:
         return takes_unscaled(self.in_weight, rows)
 
