@@ -215,7 +215,7 @@ gla_chunk_out_kernel(const float* __restrict__ proj, int64_t proj_stride, int q_
 // Two requests of 2000 and 1117 tokens, 8 heads of 64 x 128: 285 us by the walk, 78 here, bound by one workgroup's chain of LDS
 // reads and products. Sums run in four chains, which both shortens the waits and keeps the error against float64 below the walk's
 // for ordinary decays: 1.2e-7 (root mean square, of the results') against 1.65e-7 at 512 tokens; where strong and slow decays
-// meet both err by a few 1e-7 (with exponents as differences of sums, 5 us faster, it was 1e-5 of the largest result).
+// meet both err by 1e-7 (with exponents as differences of sums, 5 us faster, it was 1e-5 of the largest result).
 constexpr int kChannelKeys = 64;        // the widest key heads here: queries, keys and decays of a chunk lie in LDS together
 
 constexpr int kPart = 16;

@@ -38,9 +38,13 @@ class GatedLinearAttention(Mixer):
     LONG_PORTION = 8        # from this many tokens of one request in a step on, the walk stages its operands through LDS
 
     CHUNKED_PORTION = 128   # and with ``chunked`` chunks of 64 tokens are taken side by side from this many on
-    # With decays a channel: 8 heads of 64 x 128, one request of 256, 512 and 8000 tokens 42, 75 and 1030 us by the walk and 49,
-    # 51 and 152 in chunks; 300 tokens beside seven single ones 192 and 55.
+    # With decays a channel the walk takes 0.145 us a token of the longest portion while a step's waves are few, twice as much from
+    # requests * heads * value_dim = CHANNEL_WALK_WIDTH on and more in proportion; chunks take longer the wider a head's values are.
+    # One request, the walk and chunks in us: values of 64 (16 heads) at 320 tokens 51 and 46; of 128 (8 heads) at 320 and 512 51
+    # and 55, 75 and 56; of 256 (4 heads) at 320, 480 and 512 51 and 73, 71 and 74, 76 and 75; of 512 (2 heads) at 512, 736 and 1024 77 and
+    # 110, 108 and 112, 142 and 114. Four requests, one of 320 tokens: 102 and 57 (8 heads of 128), 103 and 110 (2 of 512).
     CHANNEL_CHUNKED_PORTION = 320
+    CHANNEL_WALK_WIDTH = 4096
 
     def __init__(self, spec: PartSpec, runtime: Runtime):
         super().__init__(spec, runtime)
@@ -111,7 +115,11 @@ class GatedLinearAttention(Mixer):
     def portion_line(self, requests: int) -> Optional[int]:
         if self.chunked:
             return self.CHUNKED_PORTION
-        return self.CHANNEL_CHUNKED_PORTION if self.channel_chunked else None
+        if not self.channel_chunked:
+            return None
+        if requests * self.heads * self.value_dim >= self.CHANNEL_WALK_WIDTH:
+            return self.CHANNEL_CHUNKED_PORTION
+        return max(self.CHANNEL_CHUNKED_PORTION, self.value_dim + 224)
 
     def take_output_projection(self) -> Optional[torch.Tensor]:
         tensor, self.o_tensor = self.o_tensor, None

@@ -62,3 +62,16 @@ def test_a_captured_shape_is_not_replayed_across_a_line(tmp_path, configs, which
         assert engine.mixed_graph_replays >= 1
         for _ in range(3):
             assert same(step(engine, (below, above)[second]), eager[second])
+
+
+@pytest.mark.parametrize("heads,value_dim,requests,line", [(8, 64, 1, 320), (8, 128, 1, 352), (8, 128, 2, 352), (8, 128, 4, 320), (32, 128, 1, 320),
+                                                           (4, 256, 1, 480), (2, 512, 1, 736), (2, 512, 4, 320)])
+def test_where_a_decay_a_channel_runs_in_chunks(heads, value_dim, requests, line):
+    """Narrow values and steps of many waves from 320 tokens of one request on, wide values of a few requests later."""
+    from microllm_rocm_amd.parts.base import Runtime
+    from microllm_rocm_amd.parts.registry import build_part
+    from microllm_rocm_amd.parts.spec import PartSpec
+    sizes = {"hidden_size": 64, "heads": heads, "key_dim": 64, "value_dim": value_dim, "decay_rank": 4, "tau": 16.0}
+    part = lambda dtype: build_part("mixer", PartSpec("gated_linear_attention", sizes, {}), Runtime(dtype=dtype, device=torch.device("cpu")))
+    assert part(torch.bfloat16).portion_line(requests) == line
+    assert part(torch.float32).portion_line(requests) is None
