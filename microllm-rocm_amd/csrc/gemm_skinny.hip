@@ -11,6 +11,8 @@
 #include "common.h"
 #include "microllm_hip.h"
 
+#include <type_traits>
+
 namespace mll {
 
 typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
@@ -85,7 +87,9 @@ __global__ __launch_bounds__(1024) void gemm_skinny_kernel(
     // loads, so the compiler counts those in flight instead of waiting for all of them. A wave keeps two blocks of loads
     // on their way; with few steps a wave everything is asked for at once, before the epilogue's own loads.
     constexpr int kPast = 0x7ffffff0, kPastRow = 0x40000000;       // offsets past the end of every descriptor here
-    constexpr int DEPTH = HALF ? HALF * kChunk / 2 : (MT + NT <= 3) ? 4 : 2;       // loads of W a tile and block
+    constexpr bool kHolds = EPILOGUE == 3 || EPILOGUE == 4 || EPILOGUE == 6;     // the epilogue holds values of its own meanwhile
+    // loads of W a tile and block: what stays in 128 registers beside the sums and those values
+    constexpr int DEPTH = HALF ? HALF * kChunk / 2 : (MT + NT <= 3) ? (kHolds && NT == 2 && GROUP <= (EPILOGUE == 3 ? 2 : 1) ? 2 : 4) : MT <= 2 ? 2 : 1;
     __amdgpu_buffer_rsrc_t w_rsrc[NT];
 #pragma unroll
     for (int nt = 0; nt < NT; ++nt) {
@@ -149,7 +153,7 @@ __global__ __launch_bounds__(1024) void gemm_skinny_kernel(
             }
         }
     };
-    auto multiply = [&](Piece (&w_piece)[DEPTH][NT], Piece (&a_piece)[DEPTH][MT]) {
+    auto multiply = [&](Piece (&w_piece)[DEPTH][NT], Piece (&a_piece)[DEPTH][MT], auto block) {     // block: of the two, the even or the odd one
         if constexpr (GROUP > 1 && !HALF) {
 #pragma unroll
             for (int u = 0; u < DEPTH; ++u)
@@ -180,9 +184,13 @@ __global__ __launch_bounds__(1024) void gemm_skinny_kernel(
 #pragma unroll
             for (int nt = 0; nt < NT; ++nt)
 #pragma unroll
-                for (int mt = 0; mt < MT; ++mt)
-                    sums[u % SETS][nt][mt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(w_piece[u][nt].v, a_piece[u][mt].v, sums[u % SETS][nt][mt], 0, 0, 0);
+                for (int mt = 0; mt < MT; ++mt) {
+                    floatx4& sum = sums[(decltype(block)::value * DEPTH + u) % SETS][nt][mt];
+                    sum = __builtin_amdgcn_mfma_f32_16x16x32_bf16(w_piece[u][nt].v, a_piece[u][mt].v, sum, 0, 0, 0);
+                }
     };
+    constexpr std::integral_constant<int, 0> even{};
+    constexpr std::integral_constant<int, 1> odd{};
     Piece w_even[DEPTH][NT], w_odd[DEPTH][NT], a_even[DEPTH][MT], a_odd[DEPTH][MT];
     load(0, w_even, a_even);
     load(1, w_odd, a_odd);
@@ -313,15 +321,15 @@ __global__ __launch_bounds__(1024) void gemm_skinny_kernel(
     constexpr int kBlockSteps = HALF ? HALF * kChunk : DEPTH;
     const int blocks = (k_steps + waves * kChunk - 1) / (waves * kChunk) * kChunk;     // steps of the wave with the most, whole runs
     for (int done = 2 * kBlockSteps; done < blocks; done += 2 * kBlockSteps) {
-        multiply(w_even, a_even);
+        multiply(w_even, a_even, even);
         load(done / kBlockSteps, w_even, a_even);
         __builtin_amdgcn_sched_barrier(0);      // else the loads sink below the next products, behind their waits
-        multiply(w_odd, a_odd);
+        multiply(w_odd, a_odd, odd);
         load(done / kBlockSteps + 1, w_odd, a_odd);
         __builtin_amdgcn_sched_barrier(0);
     }
-    multiply(w_even, a_even);
-    multiply(w_odd, a_odd);
+    multiply(w_even, a_even, even);
+    multiply(w_odd, a_odd, odd);
 
     floatx4 (&acc)[NT][MT] = sums[0];
     if constexpr (HALF != 0 || SPLIT) {         // the even steps' sums and the odd ones'
@@ -357,7 +365,9 @@ __global__ __launch_bounds__(1024) void gemm_skinny_kernel(
         for (int mt = 0; mt < MT; ++mt) row_factor[mt] = HALF ? __shfl(factor, mt * 8 + token, kWave) : factor;
     }
 
-    // The waves' sums, added in wave order by wave 0; four slots are read at a time.
+    // The waves' sums, added in wave order by wave 0; several slots are read at a time, as many as stay in registers beside what
+    // the epilogue holds.
+    constexpr int kAtATime = NT * MT >= 6 ? 1 : NT * MT >= 3 || (kHolds && NT * MT == 2) ? 2 : 4;
     if (waves > 1) {
         floatx4* slots = reinterpret_cast<floatx4*>(reduce_shared);
         if (wave > 0) {
@@ -368,10 +378,10 @@ __global__ __launch_bounds__(1024) void gemm_skinny_kernel(
         }
         __syncthreads();
         if (wave > 0) return;
-        for (int first = 0; first < waves - 1; first += 4) {
-            floatx4 part[4][NT][MT];
+        for (int first = 0; first < waves - 1; first += kAtATime) {
+            floatx4 part[kAtATime][NT][MT];
 #pragma unroll
-            for (int i = 0; i < 4; ++i) {
+            for (int i = 0; i < kAtATime; ++i) {
                 const int other = min(first + i, waves - 2);
 #pragma unroll
                 for (int nt = 0; nt < NT; ++nt)
@@ -379,7 +389,7 @@ __global__ __launch_bounds__(1024) void gemm_skinny_kernel(
                     for (int mt = 0; mt < MT; ++mt) part[i][nt][mt] = slots[(other * NT * MT + nt * MT + mt) * kWave + lane];
             }
 #pragma unroll
-            for (int i = 0; i < 4; ++i)
+            for (int i = 0; i < kAtATime; ++i)
                 if (first + i < waves - 1) {
 #pragma unroll
                     for (int nt = 0; nt < NT; ++nt)
@@ -526,10 +536,13 @@ static void launch_few(const bf16* a, const bf16* w, void* out, int m, int n, in
     else launch_one<1, NT, EPILOGUE, 1, 0, false>(a, w, out, m, n, k, n_tiles, k_steps, extras, stream);
 }
 
+// 17 to 64 rows: what gemm_medium is for; kept for callers of the entry. 64 rows of 896 x 4864 22 us, 3584 x 18944 100, 37888 x
+// 3584 102 (with two steps a block and four slots read at a time, which spilled up to 670 registers, 81, 163 and 190).
 template <int MT, int NT, int EPILOGUE>
 static void launch_many(const bf16* a, const bf16* w, void* out, int m, int n, int k, int n_tiles,
                         int k_steps, const MllSkinnyExtras& extras, hipStream_t stream) {
-    if (in_halves(n_tiles)) launch_one<MT, NT, EPILOGUE, 1, 0, true>(a, w, out, m, n, k, n_tiles, k_steps, extras, stream);
+    // Narrow weights: one tile a workgroup, so that its two sets of sums stay in registers beside the loads.
+    if (in_halves(n_tiles)) launch_one<MT, 1, EPILOGUE, 1, 0, true>(a, w, out, m, n, k, n_tiles, k_steps, extras, stream);
     else launch_one<MT, NT, EPILOGUE, 1, 0, false>(a, w, out, m, n, k, n_tiles, k_steps, extras, stream);
 }
 
@@ -552,24 +565,20 @@ static int launch_skinny(const void* a, const void* w_packed, void* out, int m, 
     const bf16* w_ = static_cast<const bf16*>(w_packed);
     const int m_tiles = (m + 15) / 16;
     const bool two = tiles_per_group(m, n_tiles) == 2;
-    if constexpr (EPILOGUE == 3 || EPILOGUE == 4 || EPILOGUE == 6 || EPILOGUE == 7) {
-        if (m_tiles != 1) return fail("gemm_skinny: this epilogue takes at most 16 rows");
+    if (m_tiles == 1) {
         if (two) launch_few<2, EPILOGUE>(a_, w_, out, m, n, k, n_tiles, k_steps, extras, stream);
         else launch_few<1, EPILOGUE>(a_, w_, out, m, n, k, n_tiles, k_steps, extras, stream);
-        return check_launch("gemm_skinny");
-    }
-    switch (m_tiles) {
-        case 1:
-            if (two) launch_few<2, EPILOGUE>(a_, w_, out, m, n, k, n_tiles, k_steps, extras, stream);
-            else launch_few<1, EPILOGUE>(a_, w_, out, m, n, k, n_tiles, k_steps, extras, stream);
-            break;
-        case 2:
-            if (two) launch_many<2, 2, EPILOGUE>(a_, w_, out, m, n, k, n_tiles, k_steps, extras, stream);
-            else launch_many<2, 1, EPILOGUE>(a_, w_, out, m, n, k, n_tiles, k_steps, extras, stream);
-            break;
-        case 3: launch_many<3, 2, EPILOGUE>(a_, w_, out, m, n, k, n_tiles, k_steps, extras, stream); break;
-        case 4: launch_many<4, 2, EPILOGUE>(a_, w_, out, m, n, k, n_tiles, k_steps, extras, stream); break;
-        default: return fail("gemm_skinny: more than 64 rows");
+    } else if constexpr (EPILOGUE == 3 || EPILOGUE == 4 || EPILOGUE == 6 || EPILOGUE == 7) {
+        return fail("gemm_skinny: this epilogue takes at most 16 rows");
+    } else if (m_tiles == 2) {
+        if (two) launch_many<2, 2, EPILOGUE>(a_, w_, out, m, n, k, n_tiles, k_steps, extras, stream);
+        else launch_many<2, 1, EPILOGUE>(a_, w_, out, m, n, k, n_tiles, k_steps, extras, stream);
+    } else if (m_tiles == 3) {
+        launch_many<3, 2, EPILOGUE>(a_, w_, out, m, n, k, n_tiles, k_steps, extras, stream);
+    } else if (m_tiles == 4) {
+        launch_many<4, 2, EPILOGUE>(a_, w_, out, m, n, k, n_tiles, k_steps, extras, stream);
+    } else {
+        return fail("gemm_skinny: more than 64 rows");
     }
     return check_launch("gemm_skinny");
 }

@@ -16,19 +16,19 @@ def device(values, dtype=torch.float32):
     return torch.as_tensor(np.asarray(values)).to(dtype).to(DEVICE)
 
 
-@pytest.mark.parametrize("n", [16, 2048, 2049, 2064, 16384, 16400, 32768])      # 128 | 129 tiles (half ones below), 1024, 2048
-@pytest.mark.parametrize("k", [8, 32, 480, 544, 4128])
+@pytest.mark.parametrize("n", [16, 2048, 2049, 2064, 4608, 8192, 16384, 16400, 32768])      # 128 | 129 tiles (half ones below), 288, 512, 1024, 2048
+@pytest.mark.parametrize("k", [8, 32, 480, 544, 1536, 4128])
 def test_streaming_product_tiles(n, k):
     """Any float32 sum of exact bfloat16 products errs by at most k roundings of the sum of their sizes; a row's bits are the
     same in every batch."""
     rng = np.random.default_rng(n + k)
-    x_exact, x = to_bf16_exact(rng.normal(size=(16, k)))
+    x_exact, x = to_bf16_exact(rng.normal(size=(64, k)))
     w_exact, w = to_bf16_exact(rng.normal(size=(n, k)))
     packed = kernels().pack_weight(w)
     whole = kernels().gemm_skinny(x, packed, n, "f32")
     bound = (k + 1) * F32_STEP * (np.abs(x_exact) @ np.abs(w_exact).T)
     assert (np.abs(whole.double().cpu().numpy() - x_exact @ w_exact.T) <= bound).all()
-    for m in (1, 4, 5, 8, 9):
+    for m in (1, 4, 5, 8, 9, 16, 17, 33, 48):
         assert torch.equal(kernels().gemm_skinny(x[:m].contiguous(), packed, n, "f32"), whole[:m]), m
 
 
