@@ -547,12 +547,19 @@ static void launch_many(const bf16* a, const bf16* w, void* out, int m, int n, i
 }
 
 // Tiles of W a workgroup takes: two where enough workgroups are left, so that every piece of A is used twice (MI355X, one
-// against two: 608 tiles of 896 at 8 rows 6.3 and 6.7 us, 1024 tiles of 2048 13.4 and 13.1, at one row 12.4 and 13.0; 2368 tiles
-// of 3584 at 8 rows 45.3 and 43.1, at one row 44.6 and 44.3; four tiles a workgroup were slower).
-static int tiles_per_group(int m, int n_tiles) {
-    if (m <= 16) return (n_tiles >= 2048 || (m > 4 && n_tiles >= 1024)) ? 2 : 1;
-    if (m <= 32) return n_tiles >= 2048 ? 2 : 1;
-    return 2;
+// against two: 1024 tiles of 2048 at 8 rows 12.4 and 11.9, at one row 12.5 and 12.5; 2368 tiles of 3584 at 8 rows 43.1 and 41.9; four
+// tiles a workgroup were slower), and where one a workgroup would leave a second round of the 256 compute units half empty, of
+// 257 to 512 tiles: 288 tiles of 3584 at 1, 8 and 16 rows 9.1 and 8.9, 10.5 and 9.8, 13.3 and 11.1, of 8192 18.0 and 15.9,
+// 20.4 and 18.1, 26.0 and 20.5; 512 tiles of 3584 11.5 and 11.4, 11.5 and 11.0, 13.9 and 11.9, at 4 rows 10.9 and 11.2; 608 tiles of
+// 3584 13.4 and 15.7, 14.8 and 16.4, 18.6 and 19.0. With fewer than 48 steps it makes no difference. The q/k/v epilogue holds
+// so much that few rows lose: 288 tiles of 3584 at 1, 5, 8 and 16 rows 9.7 and 11.6, 10.1 and 10.7, 11.1 and 10.8, 12.7 and 11.1.
+template <int EPILOGUE>
+static int tiles_per_group(int m, int n_tiles, int k_steps) {
+    if (m > 32) return 2;
+    if (m > 16) return n_tiles >= 2048 ? 2 : 1;
+    if (n_tiles >= 2048 || (m > 4 && n_tiles >= 1024)) return 2;
+    const bool half_a_round = n_tiles > 256 && n_tiles <= (m > 4 ? 512 : 384) && k_steps >= 48;
+    return half_a_round && (EPILOGUE != 3 || m > 5) ? 2 : 1;
 }
 
 template <int EPILOGUE>
@@ -564,7 +571,7 @@ static int launch_skinny(const void* a, const void* w_packed, void* out, int m, 
     const bf16* a_ = static_cast<const bf16*>(a);
     const bf16* w_ = static_cast<const bf16*>(w_packed);
     const int m_tiles = (m + 15) / 16;
-    const bool two = tiles_per_group(m, n_tiles) == 2;
+    const bool two = tiles_per_group<EPILOGUE>(m, n_tiles, k_steps) == 2;
     if (m_tiles == 1) {
         if (two) launch_few<2, EPILOGUE>(a_, w_, out, m, n, k, n_tiles, k_steps, extras, stream);
         else launch_few<1, EPILOGUE>(a_, w_, out, m, n, k, n_tiles, k_steps, extras, stream);

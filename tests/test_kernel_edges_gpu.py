@@ -214,3 +214,36 @@ def test_chunks_where_slow_decays_follow_strong_ones(strong_first, strong):
     left = np.einsum("jhd,jhd,jhv->hdv", k, pairs[-1], v)
     bound = np.einsum("jhd,jhd,jhv->hdv", np.abs(k), (pairs * roundings)[-1], np.abs(v)) * F32_STEP
     assert (np.abs(state[0].double().cpu().numpy() - left) <= bound).all()
+
+
+@pytest.mark.parametrize("tiles", [127, 128, 129, 256, 257, 384, 385, 512, 513])       # half tiles up to 128, two a workgroup from 257 to 512
+@pytest.mark.parametrize("m", [1, 5, 6, 9, 16])
+def test_streaming_epilogues_by_tiles(tiles, m):
+    """The residual and the q/k/v epilogue on both sides of the lines where a workgroup takes half a tile, one and two, against
+    the plain product (the same sums to the bit) and the kernels that they replace."""
+    rng = np.random.default_rng(tiles + m)
+    ka, n, k = kernels(), 16 * tiles, 1536
+    _, x = to_bf16_exact(rng.normal(size=(m, k)))
+    _, w = to_bf16_exact(rng.normal(size=(n, k)) * 0.1)
+    packed = ka.pack_weight(w)
+    product = ka.gemm_skinny(x, packed, n, "f32")
+    stream, norm = rng.normal(size=(m, n)), device(rng.normal(size=n))
+    if n <= 8192:
+        h = device(stream)
+        values, scale = ka.gemm_skinny_residual(x, packed, h, norm, n, 1e-5)
+        assert torch.equal(h, device(stream) + product)
+        assert torch.equal(values, (h * norm).to(torch.bfloat16))
+        # the sums of squares, through a product that applies the rows' factors to the identity's columns
+        eye = ka.pack_weight(torch.eye(n, dtype=torch.bfloat16, device=DEVICE)[:16].contiguous())
+        factor = 1.0 / torch.sqrt(h.double().pow(2).mean(1, keepdim=True) + 1e-5)
+        got = ka.gemm_skinny(values, eye, 16, "f32", scale=scale).double()
+        assert torch.allclose(got, values[:, :16].double() * factor, rtol=(n / 8 + 8) * 2 * F32_STEP, atol=0.0)
+    heads, hd, rotary = tiles, 16, 16
+    order = ka.rotary_pair_order(heads, 0, hd, rotary // 2)
+    positions = device(rng.integers(0, 30000, size=m), torch.int32)
+    table = ka.rope_table(positions, device(1e4 ** -(np.arange(0, rotary, 2) / rotary), torch.float64))
+    bias = device(rng.normal(size=n))
+    one = ka.gemm_skinny_qkv(x, ka.pack_weight(w, row_order=order), bias, None, table, None, None, heads, 0, hd, 16)
+    two = ka.qkv_rope_store(product, bias, positions, None, device(1e4 ** -(np.arange(0, rotary, 2) / rotary), torch.float64), None, None, heads, 0, hd, 16,
+                            torch.bfloat16)
+    assert torch.equal(one, two)
