@@ -57,8 +57,9 @@ __device__ inline unsigned turn_lanes(unsigned value, int steps) {
 // units idle: a wave's A operand holds the 8 rows at one k step in its first 8 rows and at the next step in its last 8,
 // and the B operand 8 rows of the activations at the first step and again at the next, so that the product's upper left
 // 8 x 8 is the even step's and its lower right 8 x 8 the odd step's; the other two quarters are read by nobody. MT counts
-// 8 rows of the activations then. SPLIT (more than 16 rows): the same sums in the same order with whole tiles.
-template <int MT, int NT, int EPILOGUE, bool SCALED, int GROUP, int HALF, bool SPLIT>
+// 8 rows of the activations then. SPLIT (more than 16 rows): the same sums in the same order with whole tiles. FAR: 64-bit addresses
+// and loads under conditions, for reductions beyond what a descriptor's 32-bit offsets reach.
+template <int MT, int NT, int EPILOGUE, bool SCALED, int GROUP, int HALF, bool SPLIT, bool FAR>
 __global__ __launch_bounds__(1024) void gemm_skinny_kernel(
     const bf16* __restrict__ a, const bf16* __restrict__ w_packed, void* __restrict__ out,
     int m, int n, int k, int n_tiles, int k_steps, MllSkinnyExtras extras) {
@@ -111,25 +112,33 @@ __global__ __launch_bounds__(1024) void gemm_skinny_kernel(
     const bool upper = col >= 8;
     // Where a lane reads W and A at step 0; for a row that is none, past the end (and with every step's offset added to it).
     const int w_at = HALF ? (col / 8) * 1024 + quad * 256 + (tile0 % 2) * 128 + (col % 8) * 16 : lane * 16;
-    int a_at[MT == 1 ? 2 : MT];
-    if constexpr (HALF) {
+    const int a_lane = (HALF ? (col / 8) * 64 : GROUP > 1 ? (col / GROUP_ROWS) * 64 : PAIRED && upper ? 64 : 0) + quad * 16;
+    int a_row[MT == 1 ? 2 : MT], a_at[MT == 1 ? 2 : MT];
 #pragma unroll
-        for (int mt = 0; mt < MT; ++mt) a_at[mt] = mt * 8 + token < m ? (mt * 8 + token) * k * 2 + (col / 8) * 64 + quad * 16 : kPastRow;
-    } else if constexpr (GROUP > 1) {
-        const int row = col % GROUP_ROWS;
-        a_at[0] = row < m ? row * k * 2 + (col / GROUP_ROWS) * 64 + quad * 16 : kPastRow;
-    } else if constexpr (PAIRED) {
-#pragma unroll
-        for (int half = 0; half < 2; ++half) {
-            const int row = (col & 7) + 8 * half;
-            a_at[half] = row < m ? row * k * 2 + (upper ? 64 : 0) + quad * 16 : kPastRow;
-        }
-    } else {
-#pragma unroll
-        for (int mt = 0; mt < MT; ++mt) a_at[mt] = mt * 16 + col < m ? (mt * 16 + col) * k * 2 + quad * 16 : kPastRow;
+    for (int i = 0; i < (MT == 1 ? 2 : MT); ++i) {
+        a_row[i] = HALF ? i * 8 + token : GROUP > 1 ? col % GROUP_ROWS : PAIRED ? (col & 7) + 8 * i : i * 16 + col;
+        a_at[i] = a_row[i] < m ? a_row[i] * k * 2 + a_lane : kPastRow;
     }
     const int k_left = k - quad * 8 - (HALF || GROUP > 1 ? col / GROUP_ROWS : (PAIRED && upper)) * 32;     // a lane reads A at steps below this many elements
 
+    auto load_w = [&](int nt, int step) -> uintx4 {
+        if constexpr (FAR) {
+            const bool there = tile0 + nt < n_tiles && step + (HALF ? col / 8 : 0) < k_steps;
+            const int64_t at = (static_cast<int64_t>((tile0 + nt) / (HALF ? 2 : 1)) * k_steps + step) * 1024 + w_at;
+            return there ? *reinterpret_cast<const uintx4*>(reinterpret_cast<const char*>(w_packed) + at) : uintx4{0u, 0u, 0u, 0u};
+        } else {
+            return __builtin_amdgcn_raw_buffer_load_b128(w_rsrc[nt], w_at + step * 1024, 0, kNonTemporal);
+        }
+    };
+    auto load_a = [&](int i, int step) -> uintx4 {
+        if constexpr (FAR) {
+            const bool there = a_row[i] < m && static_cast<int64_t>(step) * 32 < k_left;
+            const int64_t at = static_cast<int64_t>(a_row[i]) * k * 2 + a_lane + static_cast<int64_t>(step) * 64;
+            return there ? *reinterpret_cast<const uintx4*>(reinterpret_cast<const char*>(a) + at) : uintx4{0u, 0u, 0u, 0u};
+        } else {
+            return __builtin_amdgcn_raw_buffer_load_b128(a_rsrc, step * 32 < k_left ? a_at[i] + step * 64 : kPast, 0, 0);
+        }
+    };
     auto load = [&](int block, Piece (&w_piece)[DEPTH][NT], Piece (&a_piece)[DEPTH][MT]) {
 #pragma unroll
         for (int u = 0; u < DEPTH; ++u) {
@@ -138,18 +147,18 @@ __global__ __launch_bounds__(1024) void gemm_skinny_kernel(
             const int step = (run * waves + wave) * kChunk + within;
 #pragma unroll
             for (int nt = 0; nt < NT; ++nt)
-                w_piece[u][nt].raw = __builtin_amdgcn_raw_buffer_load_b128(w_rsrc[nt], w_at + step * 1024, 0, kNonTemporal);
+                w_piece[u][nt].raw = load_w(nt, step);
             if constexpr (GROUP > 1 && !HALF) {
                 if (u % GROUP == 0)
-                    a_piece[u][0].raw = __builtin_amdgcn_raw_buffer_load_b128(a_rsrc, step * 32 < k_left ? a_at[0] + step * 64 : kPast, 0, 0);
+                    a_piece[u][0].raw = load_a(0, step);
             } else if constexpr (PAIRED) {
                 // a_piece[u] of an even u: rows 0..7 (both steps of the pair); of the odd u after it: rows 8..15
                 const int pair = step - (u & 1);
-                a_piece[u][0].raw = __builtin_amdgcn_raw_buffer_load_b128(a_rsrc, pair * 32 < k_left ? a_at[u & 1] + pair * 64 : kPast, 0, 0);
+                a_piece[u][0].raw = load_a(u & 1, pair);
             } else {
 #pragma unroll
                 for (int mt = 0; mt < MT; ++mt)
-                    a_piece[u][mt].raw = __builtin_amdgcn_raw_buffer_load_b128(a_rsrc, step * 32 < k_left ? a_at[mt] + step * 64 : kPast, 0, 0);
+                    a_piece[u][mt].raw = load_a(mt, step);
             }
         }
     };
@@ -500,7 +509,7 @@ static int skinny_waves(int n_tiles, int k_steps) {
     return max(1, waves);
 }
 
-template <int MT, int NT, int EPILOGUE, int GROUP, int HALF, bool SPLIT>
+template <int MT, int NT, int EPILOGUE, int GROUP, int HALF, bool SPLIT, bool FAR = false>
 static void launch_one(const bf16* a, const bf16* w, void* out, int m, int n, int k, int n_tiles,
                        int k_steps, const MllSkinnyExtras& extras, hipStream_t stream) {
     const int waves = skinny_waves(n_tiles, k_steps);
@@ -509,10 +518,10 @@ static void launch_one(const bf16* a, const bf16* w, void* out, int m, int n, in
     size_t lds = waves > 1 ? static_cast<size_t>(waves - 1) * NT * MT * kWave * sizeof(floatx4) : 0;
     if (MT * (HALF ? 8 : 16) <= 16 && extras.scale.sumsq != nullptr) {
         lds += (static_cast<size_t>(m) * extras.scale.stride * sizeof(float) + 1023) / 1024 * 1024;
-        gemm_skinny_kernel<MT, NT, EPILOGUE, (MT * (HALF ? 8 : 16) <= 16), GROUP, HALF, SPLIT><<<groups, waves * kWave, lds, stream>>>(
+        gemm_skinny_kernel<MT, NT, EPILOGUE, (MT * (HALF ? 8 : 16) <= 16), GROUP, HALF, SPLIT, FAR><<<groups, waves * kWave, lds, stream>>>(
             a, w, out, m, n, k, units, k_steps, extras);
     } else {
-        gemm_skinny_kernel<MT, NT, EPILOGUE, false, GROUP, HALF, SPLIT><<<groups, waves * kWave, lds, stream>>>(
+        gemm_skinny_kernel<MT, NT, EPILOGUE, false, GROUP, HALF, SPLIT, FAR><<<groups, waves * kWave, lds, stream>>>(
             a, w, out, m, n, k, units, k_steps, extras);
     }
 }
@@ -534,6 +543,22 @@ static void launch_few(const bf16* a, const bf16* w, void* out, int m, int n, in
     if (m <= 4) launch_one<1, NT, EPILOGUE, 4, 0, false>(a, w, out, m, n, k, n_tiles, k_steps, extras, stream);
     else if (m <= 8) launch_one<1, NT, EPILOGUE, 2, 0, false>(a, w, out, m, n, k, n_tiles, k_steps, extras, stream);
     else launch_one<1, NT, EPILOGUE, 1, 0, false>(a, w, out, m, n, k, n_tiles, k_steps, extras, stream);
+}
+
+// Reductions whose byte offsets (64 rows of the activations) pass what descriptors reach: 16 rows at a time, the same sums.
+constexpr int kWidestNear = 1 << 23;
+template <int EPILOGUE>
+static void launch_far(const bf16* a, const bf16* w, void* out, int m, int n, int k, int n_tiles, int k_steps, const MllSkinnyExtras& extras,
+                       hipStream_t stream) {
+    const int64_t row_bytes = EPILOGUE == 0 ? 4ll * n : EPILOGUE == 1 || EPILOGUE == 6 ? 2ll * n : n;
+    for (int first = 0; first < m; first += 16) {
+        const int rows = min(16, m - first);
+        const bf16* a_ = a + static_cast<int64_t>(first) * k;
+        void* out_ = static_cast<char*>(out) + first * row_bytes;
+        if (in_halves(n_tiles) && rows <= 8) launch_one<1, 1, EPILOGUE, 1, 1, false, true>(a_, w, out_, rows, n, k, n_tiles, k_steps, extras, stream);
+        else if (in_halves(n_tiles)) launch_one<2, 1, EPILOGUE, 1, 1, false, true>(a_, w, out_, rows, n, k, n_tiles, k_steps, extras, stream);
+        else launch_one<1, 1, EPILOGUE, 1, 0, false, true>(a_, w, out_, rows, n, k, n_tiles, k_steps, extras, stream);
+    }
 }
 
 // 17 to 64 rows: what gemm_medium is for; kept for callers of the entry. 64 rows of 896 x 4864 22 us, 3584 x 18944 100, 37888 x
@@ -565,14 +590,15 @@ static int tiles_per_group(int m, int n_tiles, int k_steps) {
 template <int EPILOGUE>
 static int launch_skinny(const void* a, const void* w_packed, void* out, int m, int n, int k,
                          const MllSkinnyExtras& extras, hipStream_t stream) {
-    MLL_REQUIRE(k <= 1 << 23, "gemm_skinny: the reduction is too long for 32-bit offsets");
     const int n_tiles = (n + 15) / 16;
     const int k_steps = (k + 31) / 32;
     const bf16* a_ = static_cast<const bf16*>(a);
     const bf16* w_ = static_cast<const bf16*>(w_packed);
     const int m_tiles = (m + 15) / 16;
     const bool two = tiles_per_group<EPILOGUE>(m, n_tiles, k_steps) == 2;
-    if (m_tiles == 1) {
+    if (k > kWidestNear) {
+        launch_far<EPILOGUE>(a_, w_, out, m, n, k, n_tiles, k_steps, extras, stream);
+    } else if (m_tiles == 1) {
         if (two) launch_few<2, EPILOGUE>(a_, w_, out, m, n, k, n_tiles, k_steps, extras, stream);
         else launch_few<1, EPILOGUE>(a_, w_, out, m, n, k, n_tiles, k_steps, extras, stream);
     } else if constexpr (EPILOGUE == 3 || EPILOGUE == 4 || EPILOGUE == 6 || EPILOGUE == 7) {

@@ -247,3 +247,25 @@ def test_streaming_epilogues_by_tiles(tiles, m):
     two = ka.qkv_rope_store(product, bias, positions, None, device(1e4 ** -(np.arange(0, rotary, 2) / rotary), torch.float64), None, None, heads, 0, hd, 16,
                             torch.bfloat16)
     assert torch.equal(one, two)
+
+
+def whole_numbers(generator, *shape):
+    """-1, 0 and 1 in bfloat16: products whose float32 sums are exact whatever their order."""
+    return torch.randint(-1, 2, shape, generator=generator, device=DEVICE).to(torch.bfloat16)
+
+
+@pytest.mark.parametrize("n", [40, 2064])        # half and whole tiles
+def test_streaming_product_of_the_longest_reductions(n):
+    """Byte offsets of 2^30 and more, where the kernel's 32-bit offsets end: the same sums with 64-bit addresses."""
+    generator = torch.Generator(device=DEVICE).manual_seed(n)
+    k = (1 << 23) + 40 if n == 40 else (1 << 23) + 8
+    x = whole_numbers(generator, 20, k)
+    w = torch.zeros((n, k), dtype=torch.bfloat16, device=DEVICE)
+    w[:40] = whole_numbers(generator, 40, k)
+    w[n - 1, k - 3:] = 1.0
+    packed = kernels().pack_weight(w)
+    want = torch.cat([x.float() @ part.float().T for part in w.split(64)], dim=1)
+    del w
+    for m in (1, 9, 20):
+        assert torch.equal(kernels().gemm_skinny(x[:m].contiguous(), packed, n, "f32"), want[:m])
+        assert torch.equal(kernels().gemm_skinny(x[:m].contiguous(), packed, n, "bf16"), want[:m].to(torch.bfloat16))
