@@ -43,8 +43,9 @@ union Piece {
 };
 
 // EPILOGUE: 0 = float32 [splits][M, N]; 1 = bfloat16 [M, N]; 2 = bfloat16 [M, N / 2] = silu(even rows of W) * (odd
-// rows). 1 and 2 need splits == 1. A workgroup takes `tiles` tiles of W, a wave its wave-th and (NT = 2) that kWaves on.
-template <int MT, int NT, int kWaves, int EPILOGUE>
+// rows). 1 and 2 need splits == 1. A workgroup takes `tiles` tiles of W, a wave its wave-th and (NT = 2) that kWaves on. FAR: 64-bit
+// addresses and loads under conditions, for reductions beyond what a descriptor's 32-bit offsets reach.
+template <int MT, int NT, int kWaves, int EPILOGUE, bool FAR>
 __global__ __launch_bounds__(kWaves * kWave) void gemm_medium_kernel(
     const bf16* __restrict__ a, const bf16* __restrict__ w_packed, void* __restrict__ out,
     int m, int n, int k, int n_tiles, int k_steps, int steps_per_split, int tiles) {
@@ -78,7 +79,7 @@ __global__ __launch_bounds__(kWaves * kWave) void gemm_medium_kernel(
         a_at[mt] = 16 * mt + col < m ? static_cast<unsigned>((16 * mt + col) * k * 2 + quad * 16) : kPast;
         asm("" : "+v"(a_at[mt]));
     }
-    const int a_end = min(k, end_step * 32) - quad * 8;      // a lane's steps begin before this element
+    const int a_end = (end_step < k_steps ? end_step * 32 : k) - quad * 8;      // a lane's steps begin before this element
 
     auto load_w = [&](Piece (&pieces)[kStepsPerStage][NT], int stage_number) {
         const int step = first_step + stage_number * kStepsPerStage;
@@ -86,14 +87,28 @@ __global__ __launch_bounds__(kWaves * kWave) void gemm_medium_kernel(
         for (int u = 0; u < kStepsPerStage; ++u) {
             const unsigned at = step + u < end_step ? static_cast<unsigned>(step + u) * 1024 : kPast;
 #pragma unroll
-            for (int nt = 0; nt < NT; ++nt) pieces[u][nt].raw = __builtin_amdgcn_raw_buffer_load_b128(w_rsrc, w_at[nt] + at, 0, kNonTemporal);
+            for (int nt = 0; nt < NT; ++nt) {
+                if constexpr (FAR) {
+                    const int tile = wave + kWaves * nt;
+                    const bf16* from = w_packed + (static_cast<int64_t>(tile0 + tile) * k_steps + step + u) * 512 + lane * 8;
+                    pieces[u][nt].raw = tile < live_tiles && step + u < end_step ? *reinterpret_cast<const uintx4*>(from) : uintx4{0u, 0u, 0u, 0u};
+                } else {
+                    pieces[u][nt].raw = __builtin_amdgcn_raw_buffer_load_b128(w_rsrc, w_at[nt] + at, 0, kNonTemporal);
+                }
+            }
         }
     };
     auto load_share = [&](uintx4 (&share)[kPiecesPerWave], int stage_number) {
 #pragma unroll
         for (int j = 0; j < kPiecesPerWave; ++j) {
             const int step = first_step + stage_number * kStepsPerStage + wave + kWaves * (j / MT);
-            share[j] = __builtin_amdgcn_raw_buffer_load_b128(a_rsrc, a_at[j % MT] + (step * 32 < a_end ? static_cast<unsigned>(step) * 64 : kPast), 0, 0);
+            if constexpr (FAR) {
+                const int row = 16 * (j % MT) + col;
+                const bf16* from = a + static_cast<int64_t>(row) * k + static_cast<int64_t>(step) * 32 + quad * 8;
+                share[j] = row < m && static_cast<int64_t>(step) * 32 < a_end ? *reinterpret_cast<const uintx4*>(from) : uintx4{0u, 0u, 0u, 0u};
+            } else {
+                share[j] = __builtin_amdgcn_raw_buffer_load_b128(a_rsrc, a_at[j % MT] + (step * 32 < a_end ? static_cast<unsigned>(step) * 64 : kPast), 0, 0);
+            }
         }
     };
     auto store_share = [&](const uintx4 (&share)[kPiecesPerWave], int buffer) {
@@ -207,7 +222,8 @@ static int balanced_tiles(int n_tiles, int splits, int most) {
 template <int MT, int EPILOGUE>
 static void launch_rows(const bf16* a, const bf16* w, void* out, int m, int n, int k, int most_tiles, int splits, hipStream_t stream) {
     const int n_tiles = (n + 15) / 16, k_steps = (k + 31) / 32;
-    const int tiles = balanced_tiles(n_tiles, splits, most_tiles);
+    const bool far = k_steps > kMostSteps;
+    const int tiles = far ? 4 : balanced_tiles(n_tiles, splits, most_tiles);
     const dim3 grid((n_tiles + tiles - 1) / tiles, splits);
     // Each split takes whole stages, so that the stages of a sum begin at the same k whatever the split.
     const int stages = (k_steps + kStepsPerStage - 1) / kStepsPerStage;
@@ -215,10 +231,14 @@ static void launch_rows(const bf16* a, const bf16* w, void* out, int m, int n, i
     const size_t lds = 2 * MT * kStepsPerStage * kWave * sizeof(uintx4);
     const auto launch = [&](auto tiles_a_wave, auto waves) {
         constexpr int kWaves = decltype(waves)::value;
-        gemm_medium_kernel<MT, decltype(tiles_a_wave)::value, kWaves, EPILOGUE><<<grid, kWaves * kWave, lds, stream>>>(
+        gemm_medium_kernel<MT, decltype(tiles_a_wave)::value, kWaves, EPILOGUE, false><<<grid, kWaves * kWave, lds, stream>>>(
             a, w, out, m, n, k, n_tiles, k_steps, steps_per_split, tiles);
     };
     using std::integral_constant;
+    if (far) {
+        gemm_medium_kernel<MT, 1, 4, EPILOGUE, true><<<grid, 4 * kWave, lds, stream>>>(a, w, out, m, n, k, n_tiles, k_steps, steps_per_split, tiles);
+        return;
+    }
     // Four waves where there are no more tiles (64 rows of 9728 x 896, 3 tiles a workgroup: 11.7 -> 9.6 us). Four waves of up to four
     // tiles each read LDS half as often, but hold too much: 64 rows of 37888 x 3584 51.7 -> 55.6 us.
     if (tiles <= 4) launch(integral_constant<int, 1>{}, integral_constant<int, 4>{});
@@ -251,7 +271,6 @@ extern "C" int mll_gemm_medium(const void* a, const void* w_packed, void* out, i
     MLL_REQUIRE(n > 0 && k > 0 && k % 8 == 0, "gemm_medium: k must be a positive multiple of 8");
     MLL_REQUIRE(tiles_per_wave == 1 || tiles_per_wave == 2, "gemm_medium: a wave takes one or two tiles of the weight");
     MLL_REQUIRE(waves == 4 || waves == 8, "gemm_medium: workgroups of 4 or 8 waves");
-    MLL_REQUIRE((k + 31) / 32 <= medium::kMostSteps, "gemm_medium: the reduction is too long for 32-bit offsets");
     MLL_REQUIRE(splits >= 1 && splits <= 64, "gemm_medium: between 1 and 64 splits of k");
     MLL_REQUIRE(epilogue == 0 || splits == 1, "gemm_medium: only float32 partial sums can be split over k");
     MLL_REQUIRE((epilogue != 2 && epilogue != 5) || n % 2 == 0, "gemm_medium: the gated epilogue needs an even number of weight rows");

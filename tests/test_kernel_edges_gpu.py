@@ -269,3 +269,18 @@ def test_streaming_product_of_the_longest_reductions(n):
     for m in (1, 9, 20):
         assert torch.equal(kernels().gemm_skinny(x[:m].contiguous(), packed, n, "f32"), want[:m])
         assert torch.equal(kernels().gemm_skinny(x[:m].contiguous(), packed, n, "bf16"), want[:m].to(torch.bfloat16))
+
+
+@pytest.mark.parametrize("n,splits", [(40, 1), (40, 16), (200, 2)])
+def test_product_for_64_rows_of_the_longest_reductions(n, splits):
+    """Where a workgroup's tiles pass what 32-bit offsets reach: the same sums with 64-bit addresses, whole and in parts."""
+    generator = torch.Generator(device=DEVICE).manual_seed(n)
+    k = (1 << 21) + 40
+    x, w = whole_numbers(generator, 64, k), whole_numbers(generator, n, k)
+    packed = kernels().pack_weight(w)
+    want = x.float() @ w.float().T
+    for m in (17, 64):
+        got = kernels().gemm_medium(x[:m].contiguous(), packed, n, "f32", plan=(2, 8, splits))
+        assert torch.equal(got.sum(0) if splits > 1 else got, want[:m])
+    if splits == 1:
+        assert torch.equal(kernels().gemm_medium(x, packed, n, "bf16"), want.to(torch.bfloat16))
