@@ -79,7 +79,7 @@ __global__ __launch_bounds__(kWaves * kWave) void gemm_medium_kernel(
         a_at[mt] = 16 * mt + col < m ? static_cast<unsigned>((16 * mt + col) * k * 2 + quad * 16) : kPast;
         asm("" : "+v"(a_at[mt]));
     }
-    const int a_end = (end_step < k_steps ? end_step * 32 : k) - quad * 8;      // a lane's steps begin before this element
+    const int a_end = (FAR && end_step == k_steps ? k : min(k, end_step * 32)) - quad * 8;      // a lane's steps begin before this element
 
     auto load_w = [&](Piece (&pieces)[kStepsPerStage][NT], int stage_number) {
         const int step = first_step + stage_number * kStepsPerStage;
@@ -203,31 +203,39 @@ __global__ __launch_bounds__(kWaves * kWave) void gemm_medium_kernel(
 }
 
 // The tiles of W a workgroup takes, at most `most`: so that the compute units' rounds times what a round takes (its tiles, and the
-// activations' copy, which costs about two) come to the least. 64 rows of
-// 37888 x 3584 with 10 tiles 51.7 us, with 5 69.2 and with 4 74.5.
-static int balanced_tiles(int n_tiles, int splits, int most) {
-    constexpr int kUnits = 256, kCopy = 2;
+// activations' copy, which costs about two) come to the least. 64 rows of 37888 x 3584 with 10 tiles 51.7 us, with 5 69.2 and
+// with 4 74.5. `parts`: the splits that hold stages; the others store zeros, which costs a little where they begin a round of their own
+// (4864 in 16 splits of whole stages fills ten: counted as 16, 4608 x 4864 at 17 and 64 rows took 14.2 and 21.9 us, now 11.7 and 17.8). Above
+// 8 tiles a workgroup's registers leave a compute unit room for no other. Where a workgroup has few stages (one or two, up to four where it
+// would take 16 tiles) and there is work for several rounds, its first loads then stand in the open; up to 32 rows 8 tiles and two workgroups a unit are
+// better: 32 rows of 20480 x 1536 with 8, 12 and 16 tiles 14.4, 18.8 and 16.6, of 11008 x 2048 13.3, 14.7 and 15.9, of 152064 x 64 14.9, 19.9 and
+// 17.1, 17 of 8192 x 8192 27.4, 28.5 and 30.1; but 64 rows of 20480 x 1536 21.0, 24.7 and 21.1, 17 of 11008 x 8192 in four
+// stages with 8 and 11 tiles 36.4 and 32.9, of 16384 x 8192 in eight with 8 and 16 47.7 and 43.7.
+static int balanced_tiles(int n_tiles, int splits, int parts, int stages, int row_tiles, int most) {
+    constexpr int kUnits = 256, kCopy = 2, kFewStages = 2, kSeveralRounds = 12 * kUnits;
     int best = 1, least = 0x7fffffff;
     for (int tiles = 1; tiles <= most; ++tiles) {
-        const int64_t groups = static_cast<int64_t>((n_tiles + tiles - 1) / tiles) * splits;
-        const int64_t cost = (groups + kUnits - 1) / kUnits * (tiles + kCopy);
+        const int64_t groups = static_cast<int64_t>((n_tiles + tiles - 1) / tiles), rounds = (groups * parts + kUnits - 1) / kUnits;
+        const int64_t cost = rounds * (tiles + kCopy) + (groups * splits > rounds * kUnits ? 2 * kCopy : 0);
         if (cost < least) {
             best = tiles;
             least = static_cast<int>(cost);
         }
     }
+    const bool few_stages = parts > 1 ? stages <= kFewStages || (best == 16 && stages <= 2 * kFewStages) : stages == 1;
+    if (row_tiles <= 2 && few_stages && static_cast<int64_t>(n_tiles) * parts >= kSeveralRounds) return min(8, most);
     return best;
 }
 
 template <int MT, int EPILOGUE>
 static void launch_rows(const bf16* a, const bf16* w, void* out, int m, int n, int k, int most_tiles, int splits, hipStream_t stream) {
     const int n_tiles = (n + 15) / 16, k_steps = (k + 31) / 32;
-    const bool far = k_steps > kMostSteps;
-    const int tiles = far ? 4 : balanced_tiles(n_tiles, splits, most_tiles);
-    const dim3 grid((n_tiles + tiles - 1) / tiles, splits);
     // Each split takes whole stages, so that the stages of a sum begin at the same k whatever the split.
     const int stages = (k_steps + kStepsPerStage - 1) / kStepsPerStage;
-    const int steps_per_split = ((stages + splits - 1) / splits) * kStepsPerStage;
+    const int stages_per_split = (stages + splits - 1) / splits, steps_per_split = stages_per_split * kStepsPerStage;
+    const bool far = k_steps > kMostSteps;
+    const int tiles = far ? 4 : balanced_tiles(n_tiles, splits, (stages + stages_per_split - 1) / stages_per_split, stages_per_split, MT, most_tiles);
+    const dim3 grid((n_tiles + tiles - 1) / tiles, splits);
     const size_t lds = 2 * MT * kStepsPerStage * kWave * sizeof(uintx4);
     const auto launch = [&](auto tiles_a_wave, auto waves) {
         constexpr int kWaves = decltype(waves)::value;
