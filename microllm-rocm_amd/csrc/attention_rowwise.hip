@@ -140,19 +140,25 @@ __device__ inline float merged(float so_far, float keep, float chunk, float add)
 // ---- runs of 16 tokens on the matrix units -----------------------------------------------------------------------
 typedef float floatx4 __attribute__((ext_vector_type(4)));
 constexpr int kRunTokens = 16;
-constexpr int kRunsFrom = 4;             // tokens a request: with fewer, most blocks of 16 have more stretches than a wave takes
+constexpr int kMostRuns = 3;             // stretches of a block
+constexpr int64_t kRunsWork = 50000000;  // tokens * heads * head size * keys: 100 tokens of one request, 28 heads of 128, 40 million, take 26 us a wave a token and 31 so
+// Tokens a request, on average, from which a step's stretches are worth a launch of their own beside the kernels for the rest, by
+// how many keys the step reaches (28 heads of 128, a wave a token and so): 32 requests of 33 and 48 new tokens 75 and 86 us, 103
+// and 62; 128 of 16 after 500 1383 and 391; 32 of 12 after 500 235 and 105, of 6 175 and 220.
+static int64_t runs_from(int64_t keys) { return keys < kWave ? 40 : keys < 4 * kWave ? 16 : 8; }
 
 // The tokens 16 * block .. + 15 of the step in stretches of places of one request in a row: bit i is set where token i begins
 // one. Tokens that only pad the step, or lie past its end, begin one each and belong to none (`none`).
 struct TokenRuns {
     unsigned begins, none;
+    int most;       // stretches with which the block is taken
     __device__ int end_of(int begin) const {      // where the stretch that begins there ends
         const unsigned after = begins & ~((2u << begin) - 1);
         return after ? __ffs(after) - 1 : kRunTokens;
     }
-    // Few enough stretches for the kernel that takes them one after the other; else (single tokens of many requests) a wave a token.
-    __device__ bool taken() const { return __popc(begins & ~none) <= kMostRuns; }
-    static constexpr int kMostRuns = 3;
+    // A wave on the matrix units takes as long for one token as for 16, 22 + 0.17 ns a key over the whole GPU (28 heads of 128), a wave a
+    // token 1.7 + 0.044: the more keys, the shorter a stretch may be.
+    __device__ bool taken() const { return __popc(begins & ~none) <= most; }
 };
 __device__ inline TokenRuns token_runs(const int32_t* seq_of_token, const int32_t* positions, int block, int n_tokens) {
     const int at = static_cast<int>(threadIdx.x) % kRunTokens;
@@ -163,6 +169,8 @@ __device__ inline TokenRuns token_runs(const int32_t* seq_of_token, const int32_
     TokenRuns runs;
     runs.begins = static_cast<unsigned>(__ballot(begins)) & 0xffffu;
     runs.none = static_cast<unsigned>(__ballot(none)) & 0xffffu;
+    const int position = none ? 0 : positions[token];
+    runs.most = __ballot(position >= 4 * kWave) != 0 ? kMostRuns : __ballot(position >= kWave) != 0 ? 2 : 1;
     return runs;
 }
 
@@ -460,8 +468,8 @@ __device__ inline float from_16_away(float value) {
     return __builtin_bit_cast(float, threadIdx.x % 32 < 16 ? odd : even);
 }
 
-// A wave takes 16 tokens of the step and one head, the stretches of one request in them (token_runs) one after the other, and walks the chunks and tiles of 64 keys as the kernels above do for
-// one token, on v_mfma_f32_16x16x4_f32: S^T = K . Q^T leaves in lane (token, quarter) the scores of keys 16 t + 4 quarter +
+// A wave takes a stretch of one request's tokens (token_runs: up to `sides` waves a block of 16 tokens, one stretch each) and one head, and walks the
+// chunks and tiles of 64 keys as the kernels above do for one token, on v_mfma_f32_16x16x4_f32: S^T = K . Q^T leaves in lane (token, quarter) the scores of keys 16 t + 4 quarter +
 // i, whose sum over the tile meets in the order of wave_sum (32, 16 in the lane, 8 and 4 between lanes, 2, 1 in the
 // lane); O^T = V^T . P^T adds the keys in ascending order. All three operands come from memory with 16 bytes a lane, four consecutive
 // terms of the reduction, where the product wants one of every four consecutive ones a quarter: transpose_quarters. The four waves of
@@ -470,27 +478,31 @@ __device__ inline float from_16_away(float value) {
 // then that tile's values are added one by one as above.
 // Bound by the matrix units and, with one wave a SIMD (up to 477 registers), by the loads of a tile's keys and values, which
 // fly over one tile's arithmetic. Prompts of 1003 tokens of 14 heads of 64: 292 -> 80 us against a wave a token and four heads, 300 of
-// 28 heads of 128: 123 -> 55, 1500: 985 -> 330.
+// 28 heads of 128: 123 -> 55, 1500: 985 -> 330. A block's stretches one after the other in one wave made 32 requests of 10 tokens after 500
+// slower than a wave a token (207 -> 236 us); side by side they take 115.
 template <int HD_TILES>
 __global__ __launch_bounds__(256) void paged_attention_rowwise_runs_kernel(
     const float* __restrict__ q, const float* __restrict__ k_cache, const float* __restrict__ v_cache,
     const int32_t* __restrict__ block_table, int table_width, const int32_t* __restrict__ seq_of_token,
-    const int32_t* __restrict__ positions, float* __restrict__ out, float scale, int n_tokens, int heads, int kv_heads, int page_size) {
+    const int32_t* __restrict__ positions, float* __restrict__ out, float scale, int n_tokens, int heads, int kv_heads, int page_size, int sides) {
 #pragma clang fp contract(off)      // a scaled score less the maximum is two roundings, as in the kernels above
     constexpr int HD = HD_TILES * 16;
     const int lane = threadIdx.x % kWave, wave = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave);
     const int col = lane % 16, quad = lane / 16;
     const int blocks = (n_tokens + kRunTokens - 1) / kRunTokens;
     const int unit = blockIdx.x * 4 + wave;
-    if (unit >= blocks * heads) return;
-    const int block = blocks - 1 - unit / heads, head = unit % heads;       // the last tokens see the most keys: they go first
+    if (unit >= blocks * sides * heads) return;
+    // The last tokens see the most keys: they go first, and every block's first stretch before any block's second, which is mostly none.
+    const int block = blocks - 1 - unit / heads % blocks, head = unit % heads;
     const TokenRuns runs = token_runs(seq_of_token, positions, block, n_tokens);
     if (!runs.taken()) return;
     const CacheLayout layout(kv_heads, page_size, HD);
     const int kv_head = head / (heads / kv_heads);
+    int number = unit / heads / blocks;        // of the block's stretches the wave's own, then every sides-th after it
     for (int begin = 0, end; begin < kRunTokens; begin = end) {
     end = __builtin_amdgcn_readfirstlane(runs.end_of(begin));
-    if ((runs.none >> begin) & 1) continue;
+    if (((runs.none >> begin) & 1) || number-- > 0) continue;
+    number = sides - 1;
     const int first_token = block * kRunTokens + begin, count = end - begin;
     const int token = first_token + min(col, count - 1);         // lanes past the stretch repeat its last token and write nothing
     const int first_position = __builtin_amdgcn_readfirstlane(positions[first_token]);
@@ -736,7 +748,7 @@ __global__ __launch_bounds__(kWave) void paged_attention_rowwise_merge_kernel(
 template <typename T, int DIMS>
 static int launch_rowwise_dims(const void* q, const void* k_cache, const void* v_cache, const int32_t* block_table, int requests,
                           int table_width, const int32_t* seq_of_token, const int32_t* positions, void* out,
-                          float* part_o, float* part_ml, int max_chunks, int usual_chunks, float scale, int window, int n_tokens,
+                          float* part_o, float* part_ml, int max_chunks, int usual_chunks, float scale, int window, int reach, int n_tokens,
                           int heads, int kv_heads, int head_dim, int page_size, hipStream_t stream) {
     const int group = heads / kv_heads;
     const int64_t rows = static_cast<int64_t>(n_tokens) * kv_heads * (max_chunks > 0 ? (usual_chunks > 0 ? usual_chunks : max_chunks) : 1);
@@ -759,17 +771,19 @@ static int launch_rowwise_dims(const void* q, const void* k_cache, const void* v
     int runs_apart = 0;
     if (max_chunks == 0) {
         if constexpr (std::is_same<T, float>::value && DIMS <= 2) {
-            // With few tokens a request there are no stretches for the launch to find: 32 requests of one token each lose 5 us.
-            if (window == 0 && head_dim % 16 == 0 && n_tokens >= kRunsFrom * static_cast<int64_t>(requests)) {
+            const int64_t keys = reach > 0 ? min(reach, table_width * page_size) : table_width * page_size;
+            const int64_t work = static_cast<int64_t>(n_tokens) * heads * head_dim * keys;
+            if (window == 0 && head_dim % 16 == 0 && n_tokens >= runs_from(keys) * requests && work >= kRunsWork) {
                 runs_apart = 1;
-                const int64_t units = static_cast<int64_t>((n_tokens + kRunTokens - 1) / kRunTokens) * heads;
+                const int sides = requests > 1 ? kMostRuns : 1;
+                const int64_t units = static_cast<int64_t>((n_tokens + kRunTokens - 1) / kRunTokens) * sides * heads;
                 MLL_REQUIRE(units < (static_cast<int64_t>(1) << 31) - 4, "paged_attention: too many rows for one call");
                 const dim3 run_grid((units + 3) / 4);
 #define MLL_ROWWISE_RUNS(TILES)                                                                                        \
     case TILES:                                                                                                        \
         paged_attention_rowwise_runs_kernel<TILES><<<run_grid, 256, 0, stream>>>(                                      \
             static_cast<const T*>(q), static_cast<const T*>(k_cache), static_cast<const T*>(v_cache), block_table, table_width, seq_of_token, \
-            positions, static_cast<T*>(out), scale, n_tokens, heads, kv_heads, page_size);                            \
+            positions, static_cast<T*>(out), scale, n_tokens, heads, kv_heads, page_size, sides);                     \
         break;
                 switch (head_dim / 16) {
                     MLL_ROWWISE_RUNS(1) MLL_ROWWISE_RUNS(2) MLL_ROWWISE_RUNS(3) MLL_ROWWISE_RUNS(4)
@@ -819,11 +833,11 @@ static int launch_rowwise_dims(const void* q, const void* k_cache, const void* v
 template <typename T>
 static int launch_rowwise(const void* q, const void* k_cache, const void* v_cache, const int32_t* block_table, int requests,
                           int table_width, const int32_t* seq_of_token, const int32_t* positions, void* out,
-                          float* part_o, float* part_ml, int max_chunks, int usual_chunks, float scale, int window, int n_tokens,
+                          float* part_o, float* part_ml, int max_chunks, int usual_chunks, float scale, int window, int reach, int n_tokens,
                           int heads, int kv_heads, int head_dim, int page_size, hipStream_t stream) {
 #define MLL_ROWWISE_DIMS(D)                                                                                            \
     return launch_rowwise_dims<T, D>(q, k_cache, v_cache, block_table, requests, table_width, seq_of_token, positions, out, part_o, \
-                                     part_ml, max_chunks, usual_chunks, scale, window, n_tokens, heads, kv_heads, head_dim, page_size, stream)
+                                     part_ml, max_chunks, usual_chunks, scale, window, reach, n_tokens, heads, kv_heads, head_dim, page_size, stream)
     if (head_dim <= kWave) MLL_ROWWISE_DIMS(1);
     if (head_dim <= 2 * kWave) MLL_ROWWISE_DIMS(2);
     if (head_dim <= 4 * kWave) MLL_ROWWISE_DIMS(4);
@@ -848,14 +862,15 @@ extern "C" int mll_rowwise_heads_a_wave(int count) {
 // max_chunks 0: one wave per (token, head). Otherwise one wave per chunk, for rows whose keys span at most
 // max_chunks chunks (the caller's promise: a row with more would lose its last ones), with part_o
 // [n_tokens * heads * max_chunks * head_dim] and part_ml [n_tokens * heads * max_chunks * 2] floats as workspace.
-// requests: rows of block_table, at least as many as the tokens' requests; only which kernel takes the tokens follows from it.
+// requests: rows of block_table, at least as many as the tokens' requests; reach: the step's longest request once it is done (0: what
+// the table can hold). Only which kernel takes the tokens follows from them.
 // usual_chunks (0: max_chunks): how many chunks the step's rows have now, where max_chunks leaves room for later
 // steps of the same shape; only how many heads a wave takes follows from it.
 extern "C" int mll_paged_attention_rowwise(const void* q, int dtype, const void* k_cache, const void* v_cache,
                                            const int32_t* block_table, int requests, int table_width,
                                            const int32_t* seq_of_token, const int32_t* positions, void* out,
                                            float* part_o, float* part_ml, int max_chunks, int usual_chunks, float scale,
-                                           int window, int n_tokens, int heads, int kv_heads, int head_dim, int page_size,
+                                           int window, int reach, int n_tokens, int heads, int kv_heads, int head_dim, int page_size,
                                            hipStream_t stream) {
     MLL_REQUIRE(heads > 0 && kv_heads > 0 && heads % kv_heads == 0, "paged_attention: heads must divide into kv_heads groups");
     MLL_REQUIRE(head_dim > 0 && head_dim <= kRowwiseMaxHeadDim, "paged_attention: head_dim must be in [1, 512]");
@@ -867,9 +882,9 @@ extern "C" int mll_paged_attention_rowwise(const void* q, int dtype, const void*
     if (n_tokens == 0) return 0;
     if (dtype == kF32)
         return launch_rowwise<float>(q, k_cache, v_cache, block_table, requests, table_width, seq_of_token, positions, out, part_o,
-                                     part_ml, max_chunks, usual_chunks, scale, window, n_tokens, heads, kv_heads, head_dim, page_size, stream);
+                                     part_ml, max_chunks, usual_chunks, scale, window, reach, n_tokens, heads, kv_heads, head_dim, page_size, stream);
     if (dtype == kBF16)
         return launch_rowwise<bf16>(q, k_cache, v_cache, block_table, requests, table_width, seq_of_token, positions, out, part_o,
-                                    part_ml, max_chunks, usual_chunks, scale, window, n_tokens, heads, kv_heads, head_dim, page_size, stream);
+                                    part_ml, max_chunks, usual_chunks, scale, window, reach, n_tokens, heads, kv_heads, head_dim, page_size, stream);
     return fail("paged_attention: unknown dtype");
 }

@@ -102,13 +102,13 @@ int mll_paged_attention_rowwise_chunk();
 // once) where the step still has waves enough for the GPU that way. This forces the count (1 to 8; 0: the launch
 // chooses again) and returns the value before. The same bits whatever the count.
 int mll_rowwise_heads_a_wave(int count);
-// requests: rows of block_table, at least as many as the tokens have requests; only which kernel takes the tokens follows
-// from it (the same bits).
+// requests: rows of block_table, at least as many as the tokens have requests; reach: the step's longest request once it is
+// done (0: what the table can hold). Only which kernel takes the tokens follows from them (the same bits).
 int mll_paged_attention_rowwise(const void* q, int dtype, const void* k_cache, const void* v_cache,
                                 const int32_t* block_table, int requests, int table_width,
                                 const int32_t* seq_of_token, const int32_t* positions, void* out,
                                 float* part_o, float* part_ml, int max_chunks, int usual_chunks, float scale, int window,
-                                int n_tokens, int heads, int kv_heads, int head_dim, int page_size,
+                                int reach, int n_tokens, int heads, int kv_heads, int head_dim, int page_size,
                                 hipStream_t stream);
 
 // The same attention for bfloat16 portions of prompts with MFMA: one workgroup per (two tiles of up to

@@ -472,7 +472,7 @@ def paged_attention_rowwise(q: torch.Tensor, k_cache: torch.Tensor, v_cache: tor
     (default: what the block table can hold). ``split``: a wave per chunk of keys and a merge, or a wave per row;
     by default by the number of rows. Both give the same bits. ``usual``: how far the step's rows reach now
     (default ``longest``, which may leave room for later steps of the same shape): how many query heads a wave
-    of the float32 kernel takes goes by it, nothing else."""
+    of the float32 kernel takes goes by it, and whether stretches of a request's tokens share a wave; nothing else."""
     lib = library.load()
     page_size = _check_paged(q, k_cache, v_cache, block_table, heads, kv_heads, head_dim)
     n_tokens = q.shape[0]
@@ -499,7 +499,7 @@ def paged_attention_rowwise(q: torch.Tensor, k_cache: torch.Tensor, v_cache: tor
     _check(lib.mll_paged_attention_rowwise(_ptr(q), _code(q.dtype), _ptr(k_cache), _ptr(v_cache), _ptr(block_table),
                                            block_table.shape[0], block_table.shape[1], _ptr(seq_of_token), _ptr(positions), _ptr(out),
                                            _ptr(part_o), _ptr(part_ml), chunks, usual_chunks, ctypes.c_float(scale), int(window),
-                                           n_tokens, heads, kv_heads, head_dim, page_size, _stream()), lib)
+                                           longest if usual is None else min(int(usual), longest), n_tokens, heads, kv_heads, head_dim, page_size, _stream()), lib)
     return out
 
 

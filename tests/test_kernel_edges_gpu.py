@@ -46,11 +46,14 @@ def test_float32_product_has_one_order_of_sums_in_every_kernel(n, k):
         assert torch.equal(kernels().gemm_f32(a[1003 - rows:].contiguous(), w), whole[1003 - rows:]), rows
 
 
-@pytest.mark.parametrize("heads,kv_heads,hd,page_size", [(4, 2, 16, 16), (7, 1, 128, 16), (3, 3, 48, 48), (12, 2, 112, 32)])
+@pytest.mark.parametrize("heads,kv_heads,hd,page_size", [(28, 4, 16, 16), (14, 2, 32, 32), (10, 2, 48, 48), (7, 1, 64, 16), (6, 3, 80, 48), (5, 1, 96, 16),
+                                                         (4, 2, 112, 32), (4, 4, 128, 48)])
 @pytest.mark.parametrize("broken", [None, float("inf"), float("nan")])
 def test_runs_of_a_requests_tokens_have_a_tokens_bits(heads, kv_heads, hd, page_size, broken):
-    """Portions that end before, on and after a stretch of 16, alone and several to a block of 16 tokens, against each of the
-    same tokens alone; and a value that is not finite changes the tokens after it alone."""
+    """Portions that end before, on and after a stretch of 16, alone and several to a block of 16 tokens, on the kernel of stretches
+    (a step that is not split, of 47 tokens a request and 58 million multiplications) and, where a block holds too many, on that of a wave a
+    row; against each of the same tokens alone by a wave a chunk. A value that is not finite changes the tokens after it
+    alone. Every head size of the kernel; pages of 48 positions, which tiles of 64 keys straddle."""
     rng = np.random.default_rng(hd)
     lengths, counts = [300, 16, 17, 140, 40, 5, 129, 33, 64], [290, 16, 17, 1, 2, 5, 31, 15, 48]
     t, q_exact, ek, ev, seq, pos = build_paged_case(rng, torch.float32, lengths, counts, heads, kv_heads, hd, page_size)
@@ -62,10 +65,10 @@ def test_runs_of_a_requests_tokens_have_a_tokens_bits(heads, kv_heads, hd, page_
         rows = value_rows(t["v"], hd).clone()
         rows[block, :, offset, 1] = broken
         write_value_rows(t["v"], rows)
-    run = lambda index: kernels().paged_attention_rowwise(t["q"][index].contiguous(), t["k"], t["v"], t["table"], t["seq"][index].contiguous(),
-                                                          t["pos"][index].contiguous(), scale, 0, heads, kv_heads, hd)
-    together = run(slice(None))
-    alone = torch.cat([run(slice(token, token + 1)) for token in range(len(pos))])
+    run = lambda index, split: kernels().paged_attention_rowwise(t["q"][index].contiguous(), t["k"], t["v"], t["table"], t["seq"][index].contiguous(),
+                                                                 t["pos"][index].contiguous(), scale, 0, heads, kv_heads, hd, split=split)
+    together = run(slice(None), False)
+    alone = torch.cat([run(slice(token, token + 1), True) for token in range(len(pos))])
     assert torch.equal(torch.nan_to_num(together, 7.0, 8.0, 9.0), torch.nan_to_num(alone, 7.0, 8.0, 9.0))
     reference = reference_attention(q_exact, ek, ev, seq, pos, heads, kv_heads, hd, scale, 0)
     sound = ~((seq == 0) & (pos >= 150)) if broken is not None else np.ones(len(pos), dtype=bool)
