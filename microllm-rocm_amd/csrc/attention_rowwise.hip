@@ -479,7 +479,7 @@ __device__ inline float from_16_away(float value) {
 // Bound by the matrix units and, with one wave a SIMD (up to 477 registers), by the loads of a tile's keys and values, which
 // fly over one tile's arithmetic. Prompts of 1003 tokens of 14 heads of 64: 292 -> 80 us against a wave a token and four heads, 300 of
 // 28 heads of 128: 123 -> 55, 1500: 985 -> 330. A block's stretches one after the other in one wave made 32 requests of 10 tokens after 500
-// slower than a wave a token (207 -> 236 us); side by side they take 115.
+// slower than a wave a token (206 -> 236 us); side by side they take 169.
 template <int HD_TILES>
 __global__ __launch_bounds__(256) void paged_attention_rowwise_runs_kernel(
     const float* __restrict__ q, const float* __restrict__ k_cache, const float* __restrict__ v_cache,

@@ -152,6 +152,13 @@ __global__ __launch_bounds__(256) void gemm_f32_tile_kernel(const float* __restr
 // (5.4 TB/s), 3584 x 18944 63 -> 52, 3584 x 3584 18.4 -> 15.4, 152064 x 3584 420 -> 352 (with two tiles a wave at 9 to 16 rows 496
 // -> 367); at 32 rows, against the matrix units' tiles, 168 -> 159, 84 -> 78, and 24 x 896 x 4864 19.0 -> 12.0. Two blocks of 128 instead of 64 of k in flight are slower (more is asked for past the ends: 52 -> 57).
 constexpr int64_t kFewWaves = 384;      // waves from which this kernel is taken: 1152 x 896 in two parts, 144 waves, takes 5.6 us in the vector kernel and 7.7 here; 896 x 4864 in eight, 448 waves, 10.8 and 9.6
+// 17 to 32 rows take it for parts of the reduction longer than this, or where the tiles would be a handful: 32 rows of 3584 x 3584 in parts
+// of 448 19.4 us here and 17.2 in the tiles, of 37888 x 512 26.8 and 27.2, x 64 12.8 and 9.0, of 3584 x 18944 in parts of 2368 73.0 and
+// 72.8 (17 rows 63.4 and 70.3), of 37888 x 2048 87 and 94.
+constexpr int kFewLong = 600;
+// Two tiles a wave, for 9 rows on, where one would read A too often: 16 rows of 152064 x 896 with one and two 100 and 93 us, 32 rows
+// 141 and 123; of 37888 x 2048 66 and 80, of 16384 x 2048 28.5 and 35.4.
+constexpr int kPairsFrom = 65536;
 constexpr int kFewRow = 64 + 16;        // floats from one row in LDS to the next: the four rows of a load on different banks
 
 template <int NT, int GROUPS, int SIXTEENS>
@@ -261,7 +268,9 @@ static void launch_few(const float* a, const float* w, const float* bias, float*
 // that thread alone in ascending k. Chunks of 128 of k lie in LDS as [row][k] with rows four banks apart, so that a thread's
 // four consecutive k are one read and the rows a wave reads at one k fall on different banks.
 constexpr int64_t kFewBelow = 128;      // workgroups of the matrix units' tiles
-constexpr int64_t kGrainBelow = 64;     // workgroups of the matrix units' tiles (64 x 896 x 1152, 36 of them: 13.4 us there, 12.2 here; 24 x 896 x 9728, 76: 17.2 and 20.7)
+// Small tiles up to this many: 200 x 1152 x 256, 468 of them, 11.2 us in the matrix units' tiles and 9.6 in these, 320 x 1152 x 256, 720, 11.2
+// and 10.3, 33 x 2048 x 2048, 768, 16.8 and 15.4; 512 x 896 x 256, 896, 11.4 and 11.4, 2048 x 256 x 512, 1024, 17.1 and 18.7.
+constexpr int64_t kGrainMost = 800;
 template <bool VECTOR>
 __global__ __launch_bounds__(128) void gemm_f32_grain_kernel(const float* __restrict__ a, const float* __restrict__ w,
                                                                 const float* __restrict__ bias, float* __restrict__ c,
@@ -573,8 +582,13 @@ extern "C" int mll_gemm_f32(const float* a, const float* w, const float* bias, f
     const unsigned parts = static_cast<unsigned>(splits);
     const bool vector = k % 4 == 0 && k <= kWidestVector && reinterpret_cast<uintptr_t>(a) % 16 == 0 && reinterpret_cast<uintptr_t>(w) % 16 == 0;
     const int64_t waves = static_cast<int64_t>((n + 15) / 16) * splits;
-    if (m <= 32 && vector && waves >= kFewWaves && (m > 16 || f32_small_variant == 0)) {
-        if (n >= kWideFrom && m > 8) launch_few<2>(a, w, bias, c, m, n, k, k_split, parts, stream);
+    const int64_t thirty_twos = static_cast<int64_t>((n + 127) / 128) * splits;     // the matrix units' tiles for 17 to 32 rows
+    // Rows of W a multiple of 32 KB apart fall on the same channels of the memory, of which a wave asks for 16 rows at a time; the vector
+    // kernels ask for fewer: 4608 x 8192 in parts at 1, 8 and 16 rows 39, 42 and 45 us here, 33, 34 and 39 there, 9728 x 8192 70, 75
+    // and 77, 65, 66 and 71, 3584 x 8192 29, 31 and 33, 29, 29 and 31; 2048 x 8192 16.8 and 25.1, whole 16384 x 8192 107 and 163.
+    const bool same_channels = k % 8192 == 0 && splits > 1 && n >= 3584;
+    if (vector && waves >= kFewWaves && (m <= 16 ? f32_small_variant == 0 && !same_channels : m <= 32 && (k_split > kFewLong || thirty_twos <= kFewBelow))) {
+        if (n >= kPairsFrom && m > 8) launch_few<2>(a, w, bias, c, m, n, k, k_split, parts, stream);
         else launch_few<1>(a, w, bias, c, m, n, k, k_split, parts, stream);
         return check_launch("gemm_f32");
     }
@@ -607,9 +621,13 @@ extern "C" int mll_gemm_f32(const float* a, const float* w, const float* bias, f
         return check_launch("gemm_f32");
     }
     // The tile whose workgroups fill the compute units best: the matrix units' time is the rounds of 256 workgroups times
-    // a tile's size. Up to 32 rows take tiles of 32 rows (32 x 9728 x 896 in tiles of 64 x 64 26.6 us, of 32 x 128 17.7).
+    // a tile's size. Of tiles that come to the same the smaller ones where parts of the reduction are short, since several share a
+    // unit and cover each other's ends: 512 x 3584 x 3584 in parts of 448 in tiles of 128 x 64 and 64 x 64 129 and 119 us, 1003 x 37888 x 64
+    // 92 and 72, 2048 x 9728 x 896 in tiles of 128 x 128 338 and 317; but 512 x 3584 x 2048 in parts of 512 73 and
+    // 79, 320 x 37888 x 256 68 and 74, 1003 x 16384 x 8192 2107 and 2471. Up to 32 rows take tiles of 32 rows (32 x 9728 x 896 in tiles of 64 x 64 26.6 us, of 32 x 128 17.7).
     struct Shape { int rows, columns; };
     const Shape shapes[4] = {{128, 128}, {128, 64}, {64, 64}, {32, 128}};
+    const bool smaller = k_split <= (splits > 1 ? 448 : 128);
     int best = 3;
     double least = 1e300;
     for (int index = m <= 32 ? 3 : 0; index < 4; ++index) {
@@ -617,7 +635,8 @@ extern "C" int mll_gemm_f32(const float* a, const float* w, const float* bias, f
         const int64_t groups = static_cast<int64_t>((n + shape.columns - 1) / shape.columns) * ((m + shape.rows - 1) / shape.rows) * splits;
         const double rounds = groups >= 4096 ? groups / 256.0 : static_cast<double>((groups + 255) / 256);
         const double cost = rounds * shape.rows * shape.columns;
-        if (cost < least) least = cost, best = index;
+        const bool fits = (m + shape.rows - 1) / shape.rows <= 65535;       // as the grid's second size
+        if (fits && (index < 3 && smaller ? cost <= least : cost < least)) least = cost, best = index;
     }
     const Shape& shape = shapes[best];
     const int64_t tiles = static_cast<int64_t>((n + shape.columns - 1) / shape.columns) * ((m + shape.rows - 1) / shape.rows) * splits;
@@ -627,7 +646,7 @@ extern "C" int mll_gemm_f32(const float* a, const float* w, const float* bias, f
         launch_few<1>(a, w, bias, c, m, n, k, k_split, parts, stream);
         return check_launch("gemm_f32");
     }
-    if (tiles < kGrainBelow) {
+    if (static_cast<int64_t>((n + 31) / 32) * ((m + 15) / 16) * splits <= kGrainMost) {
         const dim3 grid((n + 31) / 32, (m + 15) / 16, parts);
         if (vector) gemm_f32_grain_kernel<true><<<grid, 128, 0, stream>>>(a, w, bias, c, m, n, k, k_split);
         else gemm_f32_grain_kernel<false><<<grid, 128, 0, stream>>>(a, w, bias, c, m, n, k, k_split);

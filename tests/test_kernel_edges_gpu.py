@@ -32,17 +32,18 @@ def test_streaming_product_tiles(n, k):
         assert torch.equal(kernels().gemm_skinny(x[:m].contiguous(), packed, n, "f32"), whole[:m]), m
 
 
-@pytest.mark.parametrize("n,k", [(331, 120), (896, 901), (4096, 64), (1000, 1536)])
+@pytest.mark.parametrize("n,k", [(331, 120), (896, 901), (4096, 64), (1000, 1536), (6150, 700), (65560, 640), (37888, 64)])
 def test_float32_product_has_one_order_of_sums_in_every_kernel(n, k):
-    """Few rows, tiles of four shapes and small tiles for few workgroups: each element is the chain of fused multiply-adds in
-    ascending k, so every batch gives a row the same bits."""
+    """The vector kernels, that of few rows (one and two tiles a wave, up to 16 and 32 rows, several groups of them), tiles of four
+    shapes and small tiles for few workgroups: each element is the chain of fused multiply-adds in ascending k, so every batch gives
+    a row the same bits."""
     rng = np.random.default_rng(n)
     a = device(rng.normal(size=(1003, k)))
     w = device(rng.normal(size=(n, k)))
     whole = kernels().gemm_f32(a, w)
     bound = (k + 1) * F32_STEP * (a.abs().double() @ w.abs().double().T)
     assert bool(((whole.double() - a.double() @ w.double().T).abs() <= bound).all())
-    for rows in (1, 2, 15, 16, 17, 31, 33, 64, 65, 127, 129, 320):
+    for rows in (1, 2, 5, 9, 15, 16, 17, 24, 31, 32, 33, 64, 65, 100, 127, 129, 320):
         assert torch.equal(kernels().gemm_f32(a[1003 - rows:].contiguous(), w), whole[1003 - rows:]), rows
 
 

@@ -420,12 +420,12 @@ def test_gemm_f32_and_row_independence(m, n, k):
     assert torch.equal(alone[0], out[-1])
 
 
-@pytest.mark.parametrize("n,k,parts", [(3584, 3584, 8), (1152, 1792, 4), (896, 4864, 8), (37888, 512, 1), (640, 901, 2), (3000, 1026, 2), (200, 300, 1)])
+@pytest.mark.parametrize("n,k,parts", [(3584, 3584, 8), (1152, 1792, 4), (896, 4864, 8), (37888, 512, 1), (37900, 768, 1), (3600, 8192, 8), (640, 901, 2), (3000, 1026, 2), (200, 300, 1)])
 def test_gemm_f32_in_parts_gives_every_row_the_same_bits_in_every_batch(n, k, parts):
     """The 32-bit product cuts the reduction of a weight with few rows of its own into parts by the weight's shape
     alone; the parts, added in order, are the product, and a row's parts are the same bits whether it comes alone, with
-    15 others (one element a thread, or 2 x 2), with 40 (tiles of 16 x 32 or 32 x 64), 64 (64 x 64) or 600 (128 x 64):
-    every kernel sums an element in ascending k with one fused multiply-add a term. Reductions that are no multiple of 4
+    up to 31 others (the kernel of few rows, or one element a thread, or 2 x 2), with 32 to 63 or 599 (the matrix units' tiles,
+    small tiles where those would be few): every kernel sums an element in ascending k with one fused multiply-add a term. Reductions that are no multiple of 4
     (no 16-byte loads) and of 2 mod 4 are among the shapes."""
     ka = kernels()
     assert ka.f32_splits(n, k) == parts
@@ -443,7 +443,7 @@ def test_gemm_f32_in_parts_gives_every_row_the_same_bits_in_every_batch(n, k, pa
         part_length = -(-(-(-k // parts)) // 4) * 4
         second = a[:3, part_length:2 * part_length].astype(np.float64) @ w[:, part_length:2 * part_length].astype(np.float64).T
         np.testing.assert_allclose(whole[1, :3].double().cpu().numpy(), second, rtol=3e-5, atol=3e-5 * np.abs(second).max())
-    for rows in (1, 7, 8, 9, 16, 40, 64):
+    for rows in (1, 7, 8, 9, 16, 17, 24, 31, 32, 33, 40, 64):
         fewer = ka.gemm_f32(device_a[:rows].contiguous(), device_w, device_bias, partials=True)
         assert torch.equal(fewer, whole[..., :rows, :]), f"{rows} rows: other bits than the same rows among 600"
     # up to 16 rows any of three kernels may take the product: the same bits
