@@ -104,14 +104,20 @@ def takes_packed(weight: "Weight", rows: int, gated: bool = False) -> bool:
     return rows <= (MEDIUM_WIDE_ROWS if wide else MEDIUM_ROWS)
 
 
+def takes_tiled(x: torch.Tensor, weight: "Weight", from_float: bool = False) -> bool:
+    """Whether a gated product of these rows is the tiled kernel's, although the weight is also kept as stored: where
+    ``kernels.tiled_gated_pays`` and the rows lie at a 16-byte boundary, as its loads need (the library takes any)."""
+    return (x.dtype == torch.bfloat16 and weight.packed is not None and weight.gated and x.data_ptr() % 16 == 0
+            and kernels.tiled_gated_pays(x.shape[0], weight.in_features, from_float))
+
+
 def linear_clamped_glu(x: torch.Tensor, weight: "Weight", limit: float, slope: float) -> torch.Tensor:
     """``g * sigmoid(slope * g) * (u + 1)`` of half the width, in x's dtype, with ``g = min(gate, limit)`` and ``u = clamp(up,
     -limit, limit)`` of a gated weight's product (rows ``[gate; up]``): in the product's epilogue for few rows and where
-    ``kernels.tiled_gated_pays``, else from its float32 sums, rounded once."""
+    ``takes_tiled``, else from its float32 sums, rounded once."""
     if x.dtype == torch.bfloat16 and weight.packed is not None and weight.gated and x.shape[0] <= SKINNY_ROWS:
         return kernels.gemm_skinny_clamped(x, weight.packed, weight.out_features, limit, slope)
-    if (x.dtype == torch.bfloat16 and weight.packed is not None and weight.gated and x.shape[0] > MEDIUM_ROWS
-            and kernels.tiled_gated_pays(x.shape[0], weight.in_features, from_float=True)):
+    if x.shape[0] > MEDIUM_ROWS and takes_tiled(x, weight, from_float=True):
         return kernels.gemm_tiled(x, weight.packed, weight.out_features, "clamped", limit=limit, slope=slope)
     # the packed copy's rows, and so its products' columns, hold gate and up by turns
     by_turns = weight.gated and x.dtype == weight.dtype and takes_packed(weight, x.shape[0])
@@ -171,7 +177,7 @@ def linear(x: Union[torch.Tensor, UnscaledRows], weight, out_dtype: Optional[tor
             return kernels.gemm_medium(x, weight.packed, weight.out_features, "f32", plan=plan)
         return kernels.gemm_medium(x, weight.packed, weight.out_features, "bf16")
     if gated:
-        if weight.packed is not None and weight.gated and kernels.tiled_gated_pays(rows, weight.in_features):
+        if takes_tiled(x, weight):
             return kernels.gemm_tiled(x, weight.packed, weight.out_features, gate)
         return kernels.gated_activation(kernels.gemm_bf16(x, w, torch.bfloat16), activation)
     if partials and out_dtype == torch.float32:

@@ -288,3 +288,20 @@ def test_product_for_64_rows_of_the_longest_reductions(n, splits):
         assert torch.equal(got.sum(0) if splits > 1 else got, want[:m])
     if splits == 1:
         assert torch.equal(kernels().gemm_medium(x, packed, n, "bf16"), want.to(torch.bfloat16))
+
+
+@pytest.mark.parametrize("rows,n,k", [(512, 19456, 896), (1024, 8192, 2048)])
+def test_gated_products_of_rows_at_any_address(rows, n, k):
+    """Rows that begin at no 16-byte boundary go to the library, whose product rounds gate and up first: a unit of bfloat16 each, and
+    the sums' own errors, beside the tiled kernel's result for the same rows at a boundary."""
+    from microllm_rocm_amd.parts.linear import Weight, linear, linear_clamped_glu, takes_tiled
+    rng = np.random.default_rng(rows)
+    _, x = to_bf16_exact(rng.normal(size=(rows, k)))
+    _, w = to_bf16_exact(rng.normal(size=(n, k)) * k ** -0.5)
+    weight = Weight(w, gated=True)
+    apart = torch.empty(rows * k + 1, dtype=torch.bfloat16, device=DEVICE)[1:].view(rows, k)
+    apart.copy_(x)
+    assert takes_tiled(x, weight) and takes_tiled(x, weight, from_float=True) and apart.data_ptr() % 16 != 0
+    for product in (lambda rows_: linear(rows_, weight, gated=True), lambda rows_: linear_clamped_glu(rows_, weight, 7.0, 1.7)):
+        got, want = product(apart).float(), product(x).float()
+        assert bool(((got - want).abs() <= 2.0 ** -6 * want.abs() + 2.0 ** -6 * 0.1).all())
