@@ -7,6 +7,7 @@ a kernel never sees operands that do not fit what its grid assumes.
 from __future__ import annotations
 
 import ctypes
+import functools
 import os
 from typing import List, NamedTuple, Optional, Sequence, Tuple
 
@@ -1178,22 +1179,48 @@ def tiled_fill(m: int, n: int, splits: int = 1) -> float:
     return blocks / (-(-blocks // COMPUTE_UNITS) * COMPUTE_UNITS)
 
 
-def tiled_gated_pays(rows: int, k: int, from_float: bool = False) -> bool:
-    """Whether a gated product (gate, up and activation) of this many rows is the tiled kernel's although the weight is also
-    kept as stored. Its epilogue saves the library's product a pass over twice the result, and its rate moves less with the
-    number of rows: against the untuned library and the activation's kernel (MI355X, time of those over this one's) 37888 x
-    3584 at 768, 1024, 1280, 1536, 2048, 3072 and 4096 rows 0.95, 1.18, 1.37, 0.99, 1.20, 1.11 and 0.96; 16384 x 2048 at 256,
-    512, 1024, 2048, 3072 and 4096 0.94, 1.14, 1.13, 1.02, 0.99 and 0.96; 9728 x 896 at 192, 256, 512, 2048 and 4096 0.90, 1.04, 1.26, 1.45 and 1.21.
-    Where the activation takes the float32 sums (``from_float``: clamped gates), the library's way writes and reads twice as
-    much and has no upper line: 37888 x 3584 at 768, 1024, 3072 and 8192 rows 1.07, 1.11, 1.27 and 1.23; 16384 x 2048 at 256, 512,
-    3584 and 8192 0.97, 1.10, 1.22 and 1.30; 9728 x 896 at 192, 256 and 8192 0.92, 1.08 and 1.56.
-    A tuned library is 3 to 8 % faster than the tiled kernel where it matters most and keeps the product. The lines lie where
-    no step's rows and the rows it is padded to (multiples of 64, above 1024 of 256) fall on different sides."""
+@functools.lru_cache(maxsize=4096)
+def _tiled_fill_of(m: int, n: int) -> float:
+    return tiled_fill(m, n)
+
+
+TILED_WIDE = 32768      # rows of a weight that gives the tiled kernel work for every compute unit
+
+
+def tiled_gated_pays(rows: int, k: int, from_float: bool = False, n: int = TILED_WIDE) -> bool:
+    """Whether a gated product (gate, up and activation) of this many rows and a weight of ``n`` rows is the tiled kernel's although the
+    weight is also kept as stored. Its epilogue saves the library's product a pass over twice the result; a workgroup's tile of
+    256 columns takes its time however few of them there are. Against the untuned library and the activation's kernel (MI355X, time of
+    those over this one's), from 256 rows on:
+
+    k up to 1024 from ``rows * n`` of 3700 k on: 512 x 512 at 1024, 3072 and 4096 rows 0.78, 0.99 and 1.07; 2816 x 1024 at 512, 1024, 1536 and 4096
+    0.76, 0.91, 1.06 and 1.51; 9728 x 896 at 192, 512, 2048 and 4096 0.91, 1.24, 1.39 and 1.21. Up to 2048 from 3000 k on: 1408 x 2048 at 1024
+    and 3072 0.61 and 0.91; 4096 x 2048 at 1024, 1536 and 2048 0.86, 1.02 and 1.13; 16384 x 2048 at 256, 512, 1024, 2048, 3072 and 4096 0.95,
+    1.10, 1.12, 1.01, 0.96 and 0.96. Longer reductions: the library's rate jumps with the shape, this one's only where the last round of
+    workgroups leaves units idle; from 3584 to 6144 where they are nine tenths filled: 37888 x 3584 at 1280, 1536 (0.87 filled), 2048 and 3072
+    1.32, 0.92, 1.15 and 1.10; 22016 x 4096 at 1024 (0.67), 1536, 2048 and 2560 (0.84) 0.85, 1.35, 1.48 and 0.94; but 17920 x 2560 at 1536, 2560, 3072
+    and 3584 0.92, 1.39, 0.85 and 0.92, 59136 x 8192 at 1024 to 4096 0.88 to 0.99, 8192 x 8192 0.85 to 0.99.
+
+    Where the activation takes the float32 sums (``from_float``: clamped gates), the library's way writes and reads twice as much and has no
+    upper line: 16384 x 2048 at 256, 512, 3584 and 8192 rows 0.97, 1.15, 1.22 and 1.30; 4096 x 2048 at 1024, 1536 and 8192 0.90, 1.05 and 1.18; 37888 x 3584
+    at 768, 1024, 3072 and 8192 1.07, 1.12, 1.24 and 1.22; 4096 x 4096 at 1024, 1536 and 2048 0.77, 0.96 and 1.10; 59136 x 8192 at 1024 to 6144 0.97 to 1.07.
+
+    A tuned library is 3 to 8 % faster than the tiled kernel where it matters most and keeps the product. Steps are padded to
+    multiples of 64 rows, above 1024 of 256: the line is drawn at the padded number, so that both are on one side of it."""
     if library_tuning() or k % 32 != 0:
         return False
+    multiple = 64 if rows <= 1024 else 256
+    rows = -(-rows // multiple) * multiple
+    if rows < 256:
+        return False
+    work = rows * n
+    if from_float:
+        return work >= 3500 * k if k <= 1024 else work >= 2800 * k if k <= 2048 else rows > 960 and work >= 1650 * k
     if k <= 1024:
-        return 192 < rows and (from_float or rows <= 4096)
-    return (448 if k <= 2048 else 960) < rows and (from_float or rows <= 3072)
+        return rows <= 4096 and work >= 3700 * k
+    if k <= 2048:
+        return rows <= 3072 and work >= 3000 * k
+    return 3584 <= k <= 6144 and 960 < rows <= 3072 and _tiled_fill_of(rows, n) >= 0.9
 
 
 def gemm_tiled(x: torch.Tensor, packed: torch.Tensor, n: int, epilogue: str = "f32", splits: int = 1,

@@ -13,3 +13,21 @@ def test_a_padded_step_takes_the_kernel_of_its_own_rows(k, from_float):
         padded = -(-rows // multiple) * multiple
         assert kernels.tiled_gated_pays(rows, k, from_float) == kernels.tiled_gated_pays(padded, k, from_float), rows
     assert not kernels.tiled_gated_pays(2048, k + 8, from_float)       # the tiled kernel's steps of 32
+
+
+@pytest.mark.parametrize("from_float", [False, True])
+@pytest.mark.parametrize("n", [64, 1408, 4096, 9728, 37888, 59136])
+@pytest.mark.parametrize("k", [512, 1024, 2048, 2560, 3584, 8192])
+def test_a_padded_step_takes_the_kernel_of_its_own_rows_for_every_weight(n, k, from_float):
+    for rows in range(1, 8193, 7):
+        multiple = 64 if rows <= 1024 else 256
+        assert kernels.tiled_gated_pays(rows, k, from_float, n) == kernels.tiled_gated_pays(-(-rows // multiple) * multiple, k, from_float, n), rows
+
+
+@pytest.mark.parametrize("rows,n,k,pays,clamped", [(2048, 1408, 2048, False, False), (4096, 512, 512, True, True), (512, 512, 512, False, False),
+                                                   (2048, 37888, 3584, True, True), (1536, 37888, 3584, False, True), (2048, 59136, 8192, False, True),
+                                                   (512, 9728, 896, True, True), (1024, 16384, 2048, True, True), (2048, 17920, 2560, False, True)])
+def test_where_the_tiled_kernel_takes_gated_products(rows, n, k, pays, clamped):
+    """Weights of few rows and of long reductions stay with the library where that is faster."""
+    assert kernels.tiled_gated_pays(rows, k, False, n) == pays
+    assert kernels.tiled_gated_pays(rows, k, True, n) == clamped
