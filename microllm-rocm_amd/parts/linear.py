@@ -91,15 +91,16 @@ def linear_into_stream(x: torch.Tensor, weight: "Weight", residual: Residual) ->
     return UnscaledRows(values, scale)
 
 
-def takes_packed(weight: "Weight", rows: int, gated: bool = False) -> bool:
-    """Whether ``linear`` multiplies this many rows with the packed copy (whose rows may be in ``row_order``)."""
+def takes_packed(weight: "Weight", rows: int, gated: bool = False, address: int = 0) -> bool:
+    """Whether ``linear`` multiplies this many rows, that begin at ``address``, with the packed copy (whose rows may be in
+    ``row_order``). From 49 gated rows on the library takes those that begin at no 16-byte boundary, which gemm_medium's loads need."""
     if weight.packed is None:
         return False
     if rows <= SKINNY_ROWS or weight.tensor is None:
         return True
     tiles = -(-weight.out_features // 16)
     if gated:
-        return rows <= (MEDIUM_ROWS if tiles >= MEDIUM_GATED_TILES else MEDIUM_GATED_ROWS)
+        return rows <= (MEDIUM_ROWS if tiles >= MEDIUM_GATED_TILES and address % 16 == 0 else MEDIUM_GATED_ROWS)
     wide = tiles >= MEDIUM_WIDE_TILES
     return rows <= (MEDIUM_WIDE_ROWS if wide else MEDIUM_ROWS)
 
@@ -170,7 +171,7 @@ def linear(x: Union[torch.Tensor, UnscaledRows], weight, out_dtype: Optional[tor
         pieces = [kernels.gemm_medium(x[first:first + MEDIUM_ROWS], weight.packed, weight.out_features, epilogue, plan=plan)
                   for first in range(0, rows, MEDIUM_ROWS)]
         return torch.cat(pieces)
-    if w is None or takes_packed(weight, rows, gated):
+    if w is None or takes_packed(weight, rows, gated, x.data_ptr()):
         if gated:
             return kernels.gemm_medium(x, weight.packed, weight.out_features, gate)
         if out_dtype == torch.float32:

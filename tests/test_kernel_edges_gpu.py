@@ -305,3 +305,20 @@ def test_gated_products_of_rows_at_any_address(rows, n, k):
     for product in (lambda rows_: linear(rows_, weight, gated=True), lambda rows_: linear_clamped_glu(rows_, weight, 7.0, 1.7)):
         got, want = product(apart).float(), product(x).float()
         assert bool(((got - want).abs() <= 2.0 ** -6 * want.abs() + 2.0 ** -6 * 0.1).all())
+
+
+@pytest.mark.parametrize("rows", [49, 64])
+@pytest.mark.parametrize("n,k", [(4096, 128), (8192, 1000)])      # 256 tiles, from which the packed copy takes 49 rows and more
+def test_gated_products_of_49_to_64_rows_at_any_address(rows, n, k):
+    """Rows that begin at no 16-byte boundary go to the library, which rounds gate g and up first: two roundings of 2^-9 beside the
+    results' own two, of which |g silu'(g)| <= 1.3 |silu(g)| + 0.3 makes less than the bound for every |up| below 5."""
+    from microllm_rocm_amd.parts.linear import Weight, linear, takes_packed
+    rng = np.random.default_rng(rows)
+    _, x = to_bf16_exact(rng.normal(size=(rows, k)))
+    _, w = to_bf16_exact(rng.normal(size=(n, k)) * k ** -0.5)
+    weight = Weight(w, gated=True)
+    apart = torch.empty(rows * k + 1, dtype=torch.bfloat16, device=DEVICE)[1:].view(rows, k)
+    apart.copy_(x)
+    assert takes_packed(weight, rows, True, x.data_ptr()) and not takes_packed(weight, rows, True, apart.data_ptr())
+    got, want = linear(apart, weight, gated=True).float(), linear(x, weight, gated=True).float()
+    assert bool(((got - want).abs() <= 2.0 ** -6 * want.abs() + 2.0 ** -6 * 0.1).all())
