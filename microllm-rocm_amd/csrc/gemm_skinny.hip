@@ -576,13 +576,19 @@ static void launch_many(const bf16* a, const bf16* w, void* out, int m, int n, i
 // tiles a workgroup were slower), and where one a workgroup would leave a second round of the 256 compute units half empty, of
 // 257 to 512 tiles: 288 tiles of 3584 at 1, 8 and 16 rows 9.1 and 8.9, 10.5 and 9.8, 13.3 and 11.1, of 8192 18.0 and 15.9,
 // 20.4 and 18.1, 26.0 and 20.5; 512 tiles of 3584 11.5 and 11.4, 11.5 and 11.0, 13.9 and 11.9, at 4 rows 10.9 and 11.2; 608 tiles of
-// 3584 13.4 and 15.7, 14.8 and 16.4, 18.6 and 19.0. With fewer than 48 steps it makes no difference. The q/k/v epilogue holds
+// 3584 13.4 and 15.7, 14.8 and 16.4, 18.6 and 19.0. With fewer than 48 steps it makes no difference. Above three rounds, 768 tiles, two are better
+// again from few rows on: 769 to 1023 tiles at 8, 12 and 16 rows, 864 of 2560 14.2 and 13.2, 18.4 and 14.8, 19.7 and 15.3, of 5120 29.8 and
+// 25.8, 37.0 and 29.1, 40.9 and 30.5, 1008 of 3584 19.7 and 19.2, 21.9 and 19.7, 24.3 and 20.5 (864 of 5120 at 5 rows 27.8 and 25.1, at 4
+// 26.8 and 24.7, but 960 24.9 and 24.5 and 864 of 896 7.0 and 7.1); 768 of 3584 15.9 and 17.3, 17.5 and 18.3, 19.1 and 19.3, of 2560 at
+// 16 rows 17.3 and 15.1. So are they from 13 rows on where a workgroup has 9 waves or more, which leave a compute unit room for no other: 640
+// tiles of 5120 at 12 and 16 rows 25.6 and 25.2, 28.8 and 26.6, of 8192 37.3 and 38.6, 41.1 and 40.2. The q/k/v epilogue holds
 // so much that few rows lose: 288 tiles of 3584 at 1, 5, 8 and 16 rows 9.7 and 11.6, 10.1 and 10.7, 11.1 and 10.8, 12.7 and 11.1.
 template <int EPILOGUE>
 static int tiles_per_group(int m, int n_tiles, int k_steps) {
     if (m > 32) return 2;
     if (m > 16) return n_tiles >= 2048 ? 2 : 1;
-    if (n_tiles >= 2048 || (m > 4 && n_tiles >= 1024)) return 2;
+    if (n_tiles >= 2048 || (m > 4 && n_tiles > (m > 12 ? 767 : 768))) return 2;
+    if (m > 12 && n_tiles > 512 && skinny_waves(n_tiles, k_steps) > 8) return 2;
     const bool half_a_round = n_tiles > 256 && n_tiles <= (m > 4 ? 512 : 384) && k_steps >= 48;
     return half_a_round && (EPILOGUE != 3 || m > 5) ? 2 : 1;
 }

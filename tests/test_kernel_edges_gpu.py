@@ -16,7 +16,8 @@ def device(values, dtype=torch.float32):
     return torch.as_tensor(np.asarray(values)).to(dtype).to(DEVICE)
 
 
-@pytest.mark.parametrize("n", [16, 2048, 2049, 2064, 4608, 8192, 16384, 16400, 32768])      # 128 | 129 tiles (half ones below), 288, 512, 1024, 2048
+# 128 | 129 tiles (half ones below), 288, 512, 521, 768 | 769 (two a workgroup above, at 16 rows from 521 or 768 on), 1024, 2048
+@pytest.mark.parametrize("n", [16, 2048, 2049, 2064, 4608, 8192, 8336, 12288, 12304, 16384, 16400, 32768])
 @pytest.mark.parametrize("k", [8, 32, 480, 544, 1536, 4128])
 def test_streaming_product_tiles(n, k):
     """Any float32 sum of exact bfloat16 products errs by at most k roundings of the sum of their sizes; a row's bits are the
@@ -220,7 +221,7 @@ def test_chunks_where_slow_decays_follow_strong_ones(strong_first, strong):
     assert (np.abs(state[0].double().cpu().numpy() - left) <= bound).all()
 
 
-@pytest.mark.parametrize("tiles", [127, 128, 129, 256, 257, 384, 385, 512, 513])       # half tiles up to 128, two a workgroup from 257 to 512
+@pytest.mark.parametrize("tiles", [127, 128, 129, 256, 257, 384, 385, 512, 513, 768, 769])       # half tiles up to 128, two a workgroup from 257 to 512 and from 769
 @pytest.mark.parametrize("m", [1, 5, 6, 9, 16])
 def test_streaming_epilogues_by_tiles(tiles, m):
     """The residual and the q/k/v epilogue on both sides of the lines where a workgroup takes half a tile, one and two, against
