@@ -504,9 +504,18 @@ static bool in_halves(int n_tiles) { return n_tiles <= kHalfTiles; }
 
 // Waves a workgroup: 16 k steps a wave, so that a wave asks for all it needs at once without asking past the end, at most
 // 16 waves and about eight thousand over the whole launch. A function of (n, k) alone, like the split of k it implies.
+// From 9 waves on a compute unit holds one workgroup whatever their number: more are taken where the waves' runs, of which the main
+// loop takes two rounds at a time, then fill their rounds better by an eighth. 520 tiles of 8192 with 15 and 16 waves at 1, 8, 12
+// and 16 rows 27.2 and 25.8 us, 30.8 and 28.8, 36.4 and 32.0, 41.8 and 36.7; 576 of 11008 with 14 and 16 at 12 rows 49.2 and 46.1; but
+// 640 of 11008, as well filled with 12 as with 16, 39.7 and 42.6 at 8.
 static int skinny_waves(int n_tiles, int k_steps) {
-    const int waves = min(min(16, 8192 / n_tiles), (k_steps + 15) / 16);
-    return max(1, waves);
+    const int waves = max(1, min(min(16, 8192 / n_tiles), (k_steps + 15) / 16));
+    if (waves <= 8) return waves;
+    const auto slots = [k_steps](int count) { return ((k_steps + count * kChunk - 1) / (count * kChunk) + 1) / 2 * count; };
+    int best = waves;
+    for (int more = waves + 1; more <= 16; ++more)
+        if (slots(more) < slots(best)) best = more;
+    return 9 * slots(best) <= 8 * slots(waves) ? best : waves;
 }
 
 template <int MT, int NT, int EPILOGUE, int GROUP, int HALF, bool SPLIT, bool FAR = false>
