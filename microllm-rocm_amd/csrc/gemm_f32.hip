@@ -437,8 +437,10 @@ __global__ __launch_bounds__(256) void gemm_f32_small_kernel(const float* __rest
     if (row < m && col < n) c[static_cast<int64_t>(row) * n + col] = acc + (bias ? bias[col] : 0.0f);
 }
 
-// The same for weights with many rows (gate/up, the head), where the kernel above is bound by its reads from LDS (two a
-// multiply-add): a workgroup of 128 threads takes 32 columns of C and a thread 2 rows x 2 columns (rows r and r + 8,
+// The same for weights with many rows, where the kernel above is bound by its reads from LDS (two a multiply-add). Of those,
+// gemm_f32_few_kernel has what it can read 16 bytes at a time; this kernel has the others (reductions that are no multiple of 4,
+// operands at no 16-byte boundary) and the weights whose rows lie a multiple of 32 KB apart (mll_gemm_f32). The figures here were
+// measured before that kernel took gate/up and the head. A workgroup of 128 threads takes 32 columns of C and a thread 2 rows x 2 columns (rows r and r + 8,
 // columns c and c + 16): half the reads a multiply-add, and four chains of additions a thread. Every element is still
 // summed by one thread in ascending k: the same bits. Measured on MI355X at 7B sizes, 8 rows: gate/up 179 -> 140 us
 // (3.9 TB/s), the head 602 -> 450 (4.8 TB/s); with few columns it has too few waves (q/k/v 37 -> 65 us, down 136 -> 330).
@@ -448,7 +450,7 @@ __global__ __launch_bounds__(256) void gemm_f32_small_kernel(const float* __rest
 constexpr int kWideThreads = 128;
 constexpr int kWideDepth = 128;                      // of k in a chunk
 constexpr int kWideQuads = kWideDepth / 4;           // float4 in a row of a chunk
-constexpr int kWideFrom = 16384;                     // columns of C from which this kernel is taken whatever the parts
+constexpr int kWideFrom = 16384;                     // columns of C from which the reduction is not cut, and this kernel taken before the one above
 
 // TR x TC elements a thread: rows r (+ 8), columns c, c + 16, ... of the workgroup's 8 TR rows and 16 TC columns. Per
 // four k a thread reads TR + TC times from LDS for 4 TR TC multiply-adds, and every element of W is read by 8 threads:
@@ -552,9 +554,6 @@ static void launch_small_wide(const float* a, const float* w, const float* bias,
 
 using namespace mll;
 
-// Into how many parts the reduction over k is cut for a weight [n, k]: a function of the weight's shape alone. A
-// weight with few rows of its own (q/k/v, o, down) gives the GPU too few tiles of C; its parts go to workgroups of
-// their own. Parts are at least 448 terms long and at most 8.
 // Which kernel takes a product of at most 16 rows: 0 the choice below; for measurements and tests 1 (an element a
 // thread), 2 (2 x 2) or 4 (1 x 4, at most 8 rows). The same bits whichever.
 static int f32_small_variant = 0;
@@ -564,6 +563,9 @@ extern "C" int mll_gemm_f32_small_variant(int variant) {
     return before;
 }
 
+// Into how many parts the reduction over k is cut for a weight [n, k]: a function of the weight's shape alone. A
+// weight with few rows of its own (q/k/v, o, down) gives the GPU too few tiles of C; its parts go to workgroups of
+// their own. Parts are at least 448 terms long and at most 8.
 extern "C" int mll_gemm_f32_splits(int n, int k) {
     if (n >= kWideFrom) return 1;
     int splits = 1;
@@ -593,7 +595,7 @@ extern "C" int mll_gemm_f32(const float* a, const float* w, const float* bias, f
         return check_launch("gemm_f32");
     }
     if (m <= 16) {
-        // Up to 8 rows: one row and four columns a thread where that still gives the GPU its workgroups (weights of
+        // What the kernel of few rows does not take. Up to 8 rows: one row and four columns a thread where that still gives the GPU its workgroups (weights of
         // many rows; the others with their parts); else two rows and two columns where that does, else the kernel of
         // one element a thread. (Two rows and four columns for 9 to 16 rows are slower than two and two: gate/up at
         // 7B sizes 131 -> 156 us. A column a thread with all rows, which reads an element of W from LDS once, is

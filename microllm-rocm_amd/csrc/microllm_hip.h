@@ -223,7 +223,8 @@ struct MllSkinnyExtras {
 };
 
 // The same product for up to 64 rows with the activations shared through LDS by the waves of a workgroup
-// (faster than mll_gemm_skinny from 17 rows on). A wave takes tiles_per_wave (1 or 2) tiles of W. With
+// (faster than mll_gemm_skinny from 17 rows on). tiles_per_wave (1 or 2) times waves (4 or 8) is the most tiles of W
+// that a workgroup takes; of as many as that it takes those that fill the compute units evenly. With
 // splits > 1 (epilogue 0 only) k is cut into that many ranges and out is [splits][m][n]: partial sums that the
 // caller adds in order. The order of additions is fixed by (n, k, splits).
 int mll_gemm_medium(const void* a, const void* w_packed, void* out, int epilogue, int m, int n, int k,

@@ -41,11 +41,12 @@ SKINNY_ROWS = 16        # up to this many rows gemm_skinny beats the library on 
 MEDIUM_ROWS = 64        # and up to this many gemm_medium does: at 17, 32 and 64 rows (the library's time, with the activation's kernel
                         # for gate and up, over this one's) 37888 x 3584 gated 1.27, 1.33 and 1.34, 9728 x 896 gated 2.06, 1.95 and
                         # 1.53, 16384 x 2048 gated 1.42, 1.37 and 1.10, 3584 x 18944 4.2, 4.1 and 2.9; except for
-MEDIUM_WIDE_TILES = 2048   # weights with this many tiles of 16 rows or more that are not gated (the head), where the library is
-MEDIUM_WIDE_ROWS = 40      # nearly as fast beyond this many: 152064 x 3584 at 32, 48 and 64 rows 1.37, 1.05 and 1.06
-MEDIUM_GATED_ROWS = 48     # gated weights with fewer tiles than compute units stay with the library from here on. It is 2 to 3 us a
-MEDIUM_GATED_TILES = 256   # layer slower (64 rows: 1024 x 256 7.7 and 5.4, 4080 x 512 9.2 and 6.9), but rounds gate and up, and steps of
-                           # 49 to 64 rows of the smallest models keep the results that they have always had
+MEDIUM_WIDE_TILES = 2048   # weights with this many tiles of 16 rows or more that are not gated (the head), which the library has
+MEDIUM_WIDE_ROWS = 40      # beyond this many. It lost less there when the line was drawn than it does now: 152064 x 3584 at 32, 48 and 64
+                           # rows 1.35, 1.07 and 1.06, 151936 x 2048 1.39, 1.33 and 1.35, 151936 x 896 1.15, 1.19 and 1.09
+MEDIUM_GATED_ROWS = 48     # gated weights with fewer tiles than compute units are the library's beyond this many. Nothing but their results
+MEDIUM_GATED_TILES = 256   # speaks for it (it rounds gate and up, and those steps of the smallest models keep what they gave): it is 2 to
+                           # 3 us a layer slower (64 rows: 1024 x 256 7.7 and 5.4, 4080 x 512 9.2 and 6.9)
 
 
 @dataclass

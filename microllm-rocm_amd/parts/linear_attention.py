@@ -42,7 +42,8 @@ class GatedLinearAttention(Mixer):
     # requests * heads * value_dim = CHANNEL_WALK_WIDTH on and more in proportion; chunks take longer the wider a head's values are.
     # One request, the walk and chunks in us: values of 64 (16 heads) at 320 tokens 51 and 46; of 128 (8 heads) at 320 and 512 51
     # and 55, 75 and 56; of 256 (4 heads) at 320, 480 and 512 51 and 73, 71 and 74, 76 and 75; of 512 (2 heads) at 512, 736 and 1024 77 and
-    # 110, 108 and 112, 142 and 114. Four requests, one of 320 tokens: 102 and 57 (8 heads of 128), 103 and 110 (2 of 512).
+    # 110, 108 and 112, 142 and 114. Four requests, one of 320 tokens: 102 and 57 (8 heads of 128), 103 and 110 (2 of 512). With many waves the walk already loses
+    # below the line: 8 requests of 128 tokens 98 and 57, 128 beside 31 others 359 and 82 (8 heads of 128).
     CHANNEL_CHUNKED_PORTION = 320
     CHANNEL_WALK_WIDTH = 4096
 
