@@ -11,11 +11,16 @@
 #include "common.h"
 #include "microllm_hip.h"
 
+#include <type_traits>
+
 namespace mll {
 
 typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
 typedef __bf16 bf16x4 __attribute__((ext_vector_type(4)));
 typedef float floatx4 __attribute__((ext_vector_type(4)));
+
+// Extras of a launch: none, without a bias by distance, with one.
+constexpr int kPlain = 0, kExtras = 1, kBiased = 2;
 
 constexpr int kDecodeWaves = 4;
 constexpr int kDecodeThreads = kDecodeWaves * kWave;
@@ -23,8 +28,9 @@ constexpr int kDecodeThreads = kDecodeWaves * kWave;
 typedef unsigned uintx4 __attribute__((ext_vector_type(4)));
 
 // 16 bytes of keys or values. STREAM: read past the caches (nothing is read twice): with a workgroup or more per
-// compute unit the pages then come in at 6.4 instead of 5.6 TB/s (64 requests of 4096 positions, 8 of 32000); with
-// fewer workgroups it is slower (128 workgroups: 41 -> 64 us), so the launch decides.
+// compute unit the pages then come in at 6.3 instead of 5.6 TB/s (64 requests of 3000 positions 70.4 and 62.6 us), with half as many
+// 8 requests of 4096 positions in 4 splits take 19.6 instead of 21.0 us, 16 of 2048 with heads of 64 10.3 instead of 11.1; heads wider
+// than 128 lose (8 of 4096 in 16 splits 20.8 and 20.0), and so do fewer workgroups where the pages of all layers stay in the last cache.
 template <bool STREAM>
 __device__ inline uint4 load_piece(const bf16* from) {
     if (STREAM) {
@@ -38,6 +44,7 @@ union Frag8 {
     bf16x8 v;
     bf16x4 h[2];
     uint4 raw;
+    int words[4];
 };
 
 // The factor of the gate on channel `dim` of a head's result: sigmoid of the head's number or of the channel's own
@@ -59,13 +66,17 @@ __device__ inline void store_result(const MllAttentionExtras& extras, bf16* out,
 // exp(extras.sink[head]) (counted once, where the waves' or the splits' results meet), the result is multiplied by
 // extras.out_scale and by its gate and its rows lie extras.out_stride elements apart; with extras.chunk the keys
 // seen begin at the query's chunk of positions; with extras.softcap the scaled scores pass a tanh. Without EXTRA the kernel is what it was.
-template <int HD_TILES, bool STREAM, bool EXTRA>
-__global__ __launch_bounds__(kDecodeThreads) void paged_attention_decode_kernel(
+// Bound by what a compute unit brings from memory (about 50 GB/s, one or two workgroups on it) and by the chain of a workgroup: place,
+// page, keys, join. Two workgroups a unit, so registers for two waves a SIMD (64 ragged requests in splits 40 -> 35 us). A workgroup's
+// neighbours are the other heads of its token, so that ragged requests spread over the dies (64 x <3000 in 8 splits 50.7 -> 44.5 us).
+template <int HD_TILES, bool STREAM, int FORM>
+__global__ __launch_bounds__(kDecodeThreads, HD_TILES <= 8 ? 2 : 1) void paged_attention_decode_kernel(
     const bf16* __restrict__ q, const bf16* __restrict__ k_cache, const bf16* __restrict__ v_cache,
     const int32_t* __restrict__ block_table, int table_width, const int32_t* __restrict__ seq_of_token,
     const int32_t* __restrict__ positions, const int32_t* __restrict__ token_ids, bf16* __restrict__ out,
     float* __restrict__ part_o, float* __restrict__ part_ml, float scale, int window, int heads, int kv_heads,
     int page_size, int n_splits, MllAttentionExtras extras) {
+    constexpr bool EXTRA = FORM != kPlain, BIAS = FORM == kBiased;
     constexpr int HD = HD_TILES * 16;
     constexpr int K_STEPS = (HD + 31) / 32;
     constexpr int K_CHUNKS = HD / 8;
@@ -76,13 +87,14 @@ __global__ __launch_bounds__(kDecodeThreads) void paged_attention_decode_kernel(
     __shared__ float m_shared[kSlots][16];
     __shared__ float l_shared[kSlots][16];
 
-    const int token = token_ids ? token_ids[blockIdx.x] : blockIdx.x;   // a step may give the kernel some of its tokens only
-    if (token < 0) return;      // an entry that only pads the list to a fixed length
     const int group = heads / kv_heads;
     const int chunks = (group + 15) / 16;
-    const int kv_head = blockIdx.y / chunks;
-    const int chunk = blockIdx.y % chunks;
-    const int split = blockIdx.z;
+    const int entry = blockIdx.x / (kv_heads * chunks), within = blockIdx.x % (kv_heads * chunks);
+    const int token = token_ids ? token_ids[entry] : entry;   // a step may give the kernel some of its tokens only
+    if (token < 0) return;      // an entry that only pads the list to a fixed length
+    const int kv_head = within / chunks;
+    const int chunk = within % chunks;
+    const int split = blockIdx.y;
     const int head0 = kv_head * group + chunk * 16;
     const int heads_here = min(16, group - chunk * 16);
     const CacheLayout layout(kv_heads, page_size, HD);
@@ -121,12 +133,7 @@ __global__ __launch_bounds__(kDecodeThreads) void paged_attention_decode_kernel(
     for (int d = 0; d < HD_TILES; ++d) o_acc[d] = floatx4{0.0f, 0.0f, 0.0f, 0.0f};
     float running_max = -INFINITY, running_sum = 0.0f;
     // The bias of this lane's head: one column of the table; every distance from `longest` on has the last row's.
-    const float* bias_column = nullptr;
-    float far_bias = 0.0f;
-    if (EXTRA && extras.bias != nullptr) {
-        bias_column = extras.bias + head0 + min(col, heads_here - 1);
-        far_bias = bias_column[static_cast<int64_t>(extras.longest) * heads];
-    }
+    const float* bias_column = BIAS ? extras.bias + head0 + min(col, heads_here - 1) : nullptr;
 
     // A pair's keys and values, from the pages into registers. A lane's 8 k-slots of the second product are the
     // 8 positions 8 * (quad % 2) .. + 7 of tile quad / 2 of the pair: one load of 16 bytes per 16 dims from the
@@ -136,23 +143,37 @@ __global__ __launch_bounds__(kDecodeThreads) void paged_attention_decode_kernel(
     // Every load is issued, none behind a branch (a tile that no query sees is read from page 0 and masked like a
     // stale one): only of straight-line code does the compiler know how many loads are still on their way, and
     // waits for one pair alone while the next flies.
-    auto load_pair = [&](int pair_index, const int (&page)[2], Frag8 (&k_frag)[2][K_STEPS], Frag8 (&v_frag)[HD_TILES]) {
+    // Eight neighbouring lanes read 8 positions of a tile, a whole line of 128 bytes, and then the other 8. A lane's own rows are 4 of
+    // either; were it to read those, a load would take half of every line, and the other half would be brought again (past the caches; 64
+    // ragged requests 46.3 -> 37.3 us). Lanes c < 4 of eight read position c and the partner's 11 - c, lanes c >= 4 the partner's
+    // 11 - c and 8 + c, and partners (c, 7 - c) exchange in attend_pair.
+    const int lane_of_8 = col % 8;
+    const int k_place[2] = {(lane_of_8 < 4 ? lane_of_8 : 11 - lane_of_8) * 8, (lane_of_8 < 4 ? 11 - lane_of_8 : 8 + lane_of_8) * 8};
+    auto load_pair = [&](int pair_index, const int (&page)[2], Frag8 (&k_frag)[2][K_STEPS], Frag8 (&v_frag)[HD_TILES], float (&bias)[8]) {
+        // With the keys, not where they are used: a load there would wait for the next pair's, which are on their way (2 requests of 1600
+        // positions, 16 heads of 128 in 4 splits 17.9 -> 12.2 us).
+        if constexpr (BIAS) {
+#pragma unroll
+            for (int j = 0; j < 8; ++j) {
+                const int distance = position - (pair_index * 32 + 8 * quad + j);
+                bias[j] = bias_column[static_cast<int64_t>(distance < 0 ? extras.longest : min(distance, extras.longest)) * heads];
+            }
+        }
         const int k_side = col / 8, v_side = quad / 2;      // which tile of the pair the lane's row / its k-slots lie in
         const int k_offset = (pair_index * 32 + 16 * k_side) % page_size;
         const int v_offset = (pair_index * 32 + 16 * v_side) % page_size;
-        const bf16* k_tile = k_cache + layout.k_tile(max(k_side ? page[1] : page[0], 0), kv_head, k_offset / 16) +
-                             (8 * ((col / 4) % 2) + col % 4) * 8;
+        const bf16* k_tile = k_cache + layout.k_tile(max(k_side ? page[1] : page[0], 0), kv_head, k_offset / 16);
         const bf16* v_tile = v_cache + layout.v_tile(max(v_side ? page[1] : page[0], 0), kv_head, v_offset / 16);
 #pragma unroll
-        for (int t = 0; t < 2; ++t) {
+        for (int ks = 0; ks < K_STEPS; ++ks) {
 #pragma unroll
-            for (int ks = 0; ks < K_STEPS; ++ks) {
+            for (int t = 0; t < 2; ++t) {
                 const int piece = ks * 4 + quad;
                 if (HD % 32 == 0) {
-                    k_frag[t][ks].raw = load_piece<STREAM>(k_tile + piece * 128 + t * 32);
+                    k_frag[t][ks].raw = load_piece<STREAM>(k_tile + piece * 128 + k_place[t]);
                 } else {      // the last 32 dims are not all there: nothing may be read past the tile
                     k_frag[t][ks].raw = make_uint4(0, 0, 0, 0);
-                    if (piece < K_CHUNKS) k_frag[t][ks].raw = load_piece<STREAM>(k_tile + piece * 128 + t * 32);
+                    if (piece < K_CHUNKS) k_frag[t][ks].raw = load_piece<STREAM>(k_tile + piece * 128 + k_place[t]);
                 }
             }
         }
@@ -163,8 +184,17 @@ __global__ __launch_bounds__(kDecodeThreads) void paged_attention_decode_kernel(
             v_frag[d].raw = load_piece<STREAM>(v_tile + (d / 2) * 512 + ((quad % 2) * width + (d % 2) * 16 + col) * 8);
         }
     };
-    auto attend_pair = [&](int pair_index, const Frag8 (&k_frag)[2][K_STEPS], Frag8 (&v_frag)[HD_TILES]) {
+    auto attend_pair = [&](int pair_index, const Frag8 (&k_frag)[2][K_STEPS], Frag8 (&v_frag)[HD_TILES], const float (&bias)[8]) {
         const int key0 = pair_index * 32;
+        Frag8 k_row[2][K_STEPS];
+#pragma unroll
+        for (int ks = 0; ks < K_STEPS; ++ks)
+#pragma unroll
+            for (int i = 0; i < 4; ++i) {
+                const int low8 = k_frag[0][ks].words[i], high8 = k_frag[1][ks].words[i];
+                k_row[0][ks].words[i] = __builtin_amdgcn_update_dpp(low8, high8, 0x141, 0xf, 0xa, false);   // lanes 4..7 of eight: the partner's
+                k_row[1][ks].words[i] = __builtin_amdgcn_update_dpp(high8, low8, 0x141, 0xf, 0x5, false);   // lanes 0..3
+            }
         // S^T = K . Q^T: lane holds head `col`, keys 8 * quad + 4 * t + i of the pair from product t.
         float score[8];
 #pragma unroll
@@ -172,16 +202,13 @@ __global__ __launch_bounds__(kDecodeThreads) void paged_attention_decode_kernel(
             floatx4 s = floatx4{0.0f, 0.0f, 0.0f, 0.0f};
 #pragma unroll
             for (int ks = 0; ks < K_STEPS; ++ks)
-                s = __builtin_amdgcn_mfma_f32_16x16x32_bf16(k_frag[t][ks].v, q_frag[ks].v, s, 0, 0, 0);
+                s = __builtin_amdgcn_mfma_f32_16x16x32_bf16(k_row[t][ks].v, q_frag[ks].v, s, 0, 0, 0);
 #pragma unroll
             for (int i = 0; i < 4; ++i) {
                 const int key = key0 + 8 * quad + 4 * t + i;
                 float value = s[i] * scale;
                 if (EXTRA && extras.softcap > 0.0f) value = softcap_fast(value, extras.softcap, 1.0f / extras.softcap);
-                if (EXTRA && bias_column != nullptr) {
-                    const int distance = position - key;
-                    value += (distance >= extras.longest || distance < 0) ? far_bias : bias_column[static_cast<int64_t>(distance) * heads];
-                }
+                if (BIAS) value += bias[4 * t + i];
                 score[4 * t + i] = (key >= low && key <= position) ? value : -INFINITY;
             }
         }
@@ -233,18 +260,19 @@ __global__ __launch_bounds__(kDecodeThreads) void paged_attention_decode_kernel(
         const int last = pair + (pair_end - 1 - pair) / kDecodeWaves * kDecodeWaves;      // this wave's last pair
         Frag8 k_first[2][K_STEPS], k_second[2][K_STEPS];
         Frag8 v_first[HD_TILES], v_second[HD_TILES];
+        float bias_first[8], bias_second[8];
         // Loads arrive in the order they were issued: a look-up is issued before the keys and values of the same
         // round, so that waiting for it a round later does not wait for them.
         int page[2] = {page_of(pair * 32), page_of(pair * 32 + 16)};
         int following = min(pair + kDecodeWaves, last);
         int next_page[2] = {page_of(following * 32), page_of(following * 32 + 16)};
-        load_pair(pair, page, k_first, v_first);
+        load_pair(pair, page, k_first, v_first, bias_first);
         while (true) {
             int after = min(following + kDecodeWaves, last);
             page[0] = page_of(after * 32);
             page[1] = page_of(after * 32 + 16);
-            load_pair(following, next_page, k_second, v_second);
-            attend_pair(pair, k_first, v_first);
+            load_pair(following, next_page, k_second, v_second, bias_second);
+            attend_pair(pair, k_first, v_first, bias_first);
             if (pair == last) break;
             pair = following;
             following = after;
@@ -252,8 +280,8 @@ __global__ __launch_bounds__(kDecodeThreads) void paged_attention_decode_kernel(
             after = min(following + kDecodeWaves, last);
             next_page[0] = page_of(after * 32);
             next_page[1] = page_of(after * 32 + 16);
-            load_pair(following, page, k_first, v_first);
-            attend_pair(pair, k_second, v_second);
+            load_pair(following, page, k_first, v_first, bias_first);
+            attend_pair(pair, k_second, v_second, bias_second);
             if (pair == last) break;
             pair = following;
             following = after;
@@ -314,7 +342,7 @@ __global__ __launch_bounds__(kDecodeThreads) void paged_attention_decode_kernel(
         }
         if (sink_here) sum += __expf(extras.sink[head0 + h] - top);
         const int64_t row = static_cast<int64_t>(token) * heads + head0 + h;
-        const int64_t part_row = static_cast<int64_t>(blockIdx.x) * heads + head0 + h;   // partial results are kept densely
+        const int64_t part_row = static_cast<int64_t>(entry) * heads + head0 + h;   // partial results are kept densely
         if (whole) {
             if (EXTRA) store_result(extras, out, token, (head0 + h) * HD + dim, total / sum * extras.out_scale * result_gate(extras, token, head0 + h, HD, dim));
             else out[row * HD + dim] = from_float<bf16>(total / sum);
@@ -435,19 +463,21 @@ static int launch_decode(const void* q, const void* k_cache, const void* v_cache
                          hipStream_t stream) {
     const int group = heads / kv_heads;
     const MllAttentionExtras given = extras ? *extras : MllAttentionExtras{nullptr, 0, nullptr, 1.0f, 0};
-    const dim3 grid(n_tokens, kv_heads * ((group + 15) / 16), n_splits);
-    const bool stream_pages = static_cast<int64_t>(grid.x) * grid.y * grid.z >= 256;      // a workgroup per compute unit or more
-#define MLL_DECODE_LAUNCH(STREAM, EXTRA)                                                                              \
-    paged_attention_decode_kernel<HD_TILES, STREAM, EXTRA><<<grid, kDecodeThreads, 0, stream>>>(                      \
-        static_cast<const bf16*>(q), static_cast<const bf16*>(k_cache), static_cast<const bf16*>(v_cache), block_table, \
-        table_width, seq_of_token, positions, token_ids, static_cast<bf16*>(out), part_o, part_ml, scale, window, heads, \
-        kv_heads, page_size, n_splits, given)
-    if (extras) {
-        if (stream_pages) MLL_DECODE_LAUNCH(true, true); else MLL_DECODE_LAUNCH(false, true);
-    } else {
-        if (stream_pages) MLL_DECODE_LAUNCH(true, false); else MLL_DECODE_LAUNCH(false, false);
-    }
-#undef MLL_DECODE_LAUNCH
+    const dim3 grid(n_tokens * (kv_heads * ((group + 15) / 16)), n_splits);
+    const bool stream_pages = static_cast<int64_t>(grid.x) * grid.y >= (HD_TILES <= 8 ? 128 : 256);      // see load_piece
+    const auto launch = [&](auto streamed, auto form) {
+        paged_attention_decode_kernel<HD_TILES, decltype(streamed)::value, decltype(form)::value><<<grid, kDecodeThreads, 0, stream>>>(
+            static_cast<const bf16*>(q), static_cast<const bf16*>(k_cache), static_cast<const bf16*>(v_cache), block_table,
+            table_width, seq_of_token, positions, token_ids, static_cast<bf16*>(out), part_o, part_ml, scale, window, heads,
+            kv_heads, page_size, n_splits, given);
+    };
+    const auto launch_form = [&](auto form) {
+        if (stream_pages) launch(std::true_type{}, form); else launch(std::false_type{}, form);
+    };
+    using std::integral_constant;
+    if (!extras) launch_form(integral_constant<int, kPlain>{});
+    else if (!extras->bias) launch_form(integral_constant<int, kExtras>{});
+    else launch_form(integral_constant<int, kBiased>{});
     return check_launch("paged_attention_decode");
 }
 
@@ -508,13 +538,12 @@ extern "C" int mll_paged_attention_decode_extra(const void* q, const void* k_cac
     }
     if (n_splits > 1) {
         const int threads = head_dim <= 64 ? 64 : (head_dim <= 128 ? 128 : 256);
-        if (extras) {
-            paged_attention_join_kernel<true><<<n_tokens * heads, threads, 0, stream>>>(part_o, part_ml, token_ids, static_cast<bf16*>(out),
-                                                                                       heads, head_dim, n_splits, *extras);
-        } else {
-            paged_attention_join_kernel<false><<<n_tokens * heads, threads, 0, stream>>>(part_o, part_ml, token_ids, static_cast<bf16*>(out),
-                                                                                        heads, head_dim, n_splits, MllAttentionExtras{nullptr, 0, nullptr, 1.0f, 0});
-        }
+        if (extras)
+            paged_attention_join_kernel<true><<<n_tokens * heads, threads, 0, stream>>>(
+                part_o, part_ml, token_ids, static_cast<bf16*>(out), heads, head_dim, n_splits, *extras);
+        else
+            paged_attention_join_kernel<false><<<n_tokens * heads, threads, 0, stream>>>(
+                part_o, part_ml, token_ids, static_cast<bf16*>(out), heads, head_dim, n_splits, MllAttentionExtras{nullptr, 0, nullptr, 1.0f, 0});
         return check_launch("paged_attention_join");
     }
     return 0;

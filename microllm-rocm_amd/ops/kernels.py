@@ -840,6 +840,25 @@ def decode_splits(n_tokens: int, kv_heads: int, longest: int) -> int:
     return splits
 
 
+FEW_ROWS_SPLITS = 8         # splits of the keys from 1024 on where a step has few (token, kv head) rows, and up to twice as many,
+FEW_ROWS_KEYS = 256         # of this many keys each
+
+
+def decode_parts(n_tokens: int, kv_heads: int, longest: int, head_dim: int) -> int:
+    """The splits a step's decode attention takes: ``decode_splits`` where the rows alone give a quarter of the compute units
+    their workgroups or the keys are few, else more and shorter ones, since a workgroup brings no more than about 50 GB/s and eight parts
+    are joined in one round of loads (MI355X, attention and join, 28 heads of 128 over 4: one request of 1024 positions with 2 and 8 splits
+    11.1 and 8.7 us, of 2048 with 4 and 8 11.0 and 9.5, of 4096 with 8, 16 and 32 11.1, 10.7 and 12.4; 8 of 4096 with 4 and 8 21.0 and 18.4; 16 of
+    1024 with 2 and 4 15.0 and 14.0; but 32 of 1024 with 1 and 2 18.1 and 18.8, one of 512 with 1 and 2 7.9 and 8.8. 14 heads of 64 over 2:
+    one of 1024 with 2 and 8 8.8 and 6.6, 32 of 1024 with 2 and 4 11.2 and 9.8). Heads wider than 128 have half the waves' loads in flight
+    and take splits of 128 keys from 512 on (one of 512 with 1 and 4 15.1 and 13.0, of 2048 with 4 and 16 18.4 and 14.7, of 4096 with 16 and 32 16.5 and 17.0)."""
+    usual, room = decode_splits(n_tokens, kv_heads, longest), 256 // max(1, n_tokens * kv_heads)
+    wide = 2 if head_dim > 128 else 1
+    if room < 4 or longest < 4 * FEW_ROWS_KEYS // wide:
+        return usual
+    return min(room, max(usual, min(2 * FEW_ROWS_SPLITS, max(FEW_ROWS_SPLITS // wide, longest * wide // FEW_ROWS_KEYS))))
+
+
 def paged_attention_decode(q: torch.Tensor, k_cache: torch.Tensor, v_cache: torch.Tensor, block_table: torch.Tensor,
                            seq_of_token: torch.Tensor, positions: torch.Tensor, scale: float, window: int,
                            heads: int, kv_heads: int, head_dim: int, n_splits: int,
@@ -957,7 +976,7 @@ def paged_attention(q: torch.Tensor, k_cache: torch.Tensor, v_cache: torch.Tenso
         longest = max(ctx.planned_total, ctx.max_total)
         reach = window if window > 0 else (extras.chunk if extras is not None else 0)      # the most keys a query sees, 0: all
         visible = min(longest, reach) if reach > 0 else longest
-        splits = decode_splits(ctx.n_tokens, kv_heads, visible)
+        splits = decode_parts(ctx.n_tokens, kv_heads, visible, head_dim)
         if out is None and two is not None:
             out = torch.empty((q.shape[0], heads // 2 * two.value_dim), dtype=q.dtype, device=q.device)
         return paged_attention_decode(q, k_cache, v_cache, view.block_table, ctx.seq_of_token, ctx.positions,
@@ -982,7 +1001,7 @@ def paged_attention(q: torch.Tensor, k_cache: torch.Tensor, v_cache: torch.Tenso
             longest = max(plan.max_single_total, ctx.planned_total) if ctx.fixed else plan.max_single_total
             reach = window if window > 0 else (extras.chunk if extras is not None else 0)
             visible = min(longest, reach) if reach > 0 else longest
-            splits = decode_splits(plan.single_tokens.shape[0], kv_heads, visible)
+            splits = decode_parts(plan.single_tokens.shape[0], kv_heads, visible, head_dim)
             paged_attention_decode(q, k_cache, v_cache, view.block_table, ctx.seq_of_token, ctx.positions,
                                    scale, window, heads, kv_heads, head_dim, splits, out=out, token_ids=plan.single_tokens,
                                    extras=extras)

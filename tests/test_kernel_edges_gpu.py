@@ -5,7 +5,7 @@ import numpy as np
 import pytest
 import torch
 
-from test_kernels_gpu import DEVICE, build_paged_case, kernels, reference_attention, to_bf16_exact
+from test_kernels_gpu import DEVICE, build_paged_case, kernels, reference_attention, to_bf16_exact, tolerance
 
 pytestmark = pytest.mark.gpu
 
@@ -323,3 +323,26 @@ def test_gated_products_of_49_to_64_rows_at_any_address(rows, n, k):
     assert takes_packed(weight, rows, True, x.data_ptr()) and not takes_packed(weight, rows, True, apart.data_ptr())
     got, want = linear(apart, weight, gated=True).float(), linear(x, weight, gated=True).float()
     assert bool(((got - want).abs() <= 2.0 ** -6 * want.abs() + 2.0 ** -6 * 0.1).all())
+
+# ---- decode attention: both sides of the line past which pages are read past the caches, with and without a bias ----
+@pytest.mark.parametrize("heads,kv_heads,hd,page_size,splits,biased", [
+    (4, 4, 64, 16, 8, False), (4, 4, 64, 16, 3, True), (8, 4, 128, 32, 5, True), (8, 4, 128, 16, 4, False), (2, 2, 192, 48, 19, True),
+    (3, 3, 48, 16, 11, True), (5, 1, 256, 16, 16, False), (18, 1, 80, 16, 9, True)])
+def test_decode_attention_reads_every_line_of_its_pages(heads, kv_heads, hd, page_size, splits, biased):
+    rng = np.random.default_rng(heads + hd + splits)
+    lengths = [417, 1, 33, 260, 16, 31, 129, 8]
+    t, q_exact, ek, ev, seq, pos = build_paged_case(rng, torch.bfloat16, lengths, [1] * len(lengths), heads, kv_heads, hd, page_size)
+    scale, longest = 1.0 / math.sqrt(hd), 90
+    table = rng.normal(size=(longest + 1, heads)).astype(np.float32) if biased else np.zeros((longest + 1, heads), np.float32)
+    want = np.zeros((len(lengths), heads, hd))
+    for token, length in enumerate(lengths):
+        distance = np.minimum(length - 1 - np.arange(length), longest)
+        for head in range(heads):
+            scores = ek[token][:, head // (heads // kv_heads)] @ q_exact[token].reshape(heads, hd)[head] * scale + table[distance, head]
+            weights = np.exp(scores - scores.max())
+            want[token, head] = weights / weights.sum() @ ev[token][:, head // (heads // kv_heads)]
+    k = kernels()
+    extras = k.AttentionExtras(bias=torch.tensor(table, device=DEVICE)) if biased else None
+    out = torch.zeros_like(t["q"])
+    k.paged_attention_decode(t["q"], t["k"], t["v"], t["table"], t["seq"], t["pos"], scale, 0, heads, kv_heads, hd, splits, out=out, extras=extras)
+    np.testing.assert_allclose(out.float().cpu().numpy(), want.reshape(len(lengths), -1), **tolerance(torch.bfloat16))
