@@ -460,7 +460,7 @@ __global__ __launch_bounds__(1024) void gemm_skinny_kernel(
                 for (int i = 0; i < 4; i += 2) {
                     const int column = n_tile * (TILE / 2) + quad * 2 + i / 2;
                     if (column < n / 2)
-                        target[column] = from_float<bf16>(gated_value(acc[nt][mt][i], acc[nt][mt][i + 1], kActClampedGlu, extras.glu_limit, extras.glu_slope));
+                        target[column] = from_float<bf16>(gated_value_fast(acc[nt][mt][i], acc[nt][mt][i + 1], kActClampedGlu, extras.glu_limit, extras.glu_slope));
                 }
             } else if (EPILOGUE == 2 || EPILOGUE == 5) {
                 bf16* target = static_cast<bf16*>(out) + static_cast<int64_t>(row) * (n / 2);

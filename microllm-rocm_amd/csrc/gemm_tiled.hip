@@ -20,99 +20,23 @@
 // Workgroups are numbered so that the 32 that run together on one of the 8 XCDs (each with a second-level cache of
 // its own) own about 4 x 8 neighbouring tiles of C, and so share their rows of A and of W there, and so that every
 // XCD gets the same number of tiles.
-#include <utility>
-
 #include "cache_layout.h"
 #include "common.h"
 #include "microllm_hip.h"
+#include "tiled_operands.h"
 
 namespace mll {
 
-typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
 typedef __bf16 bf16x4 __attribute__((ext_vector_type(4)));
 typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
-typedef float floatx4 __attribute__((ext_vector_type(4)));
-typedef unsigned uintx4 __attribute__((ext_vector_type(4)));
-typedef __attribute__((address_space(3))) bf16 lds_bf16;
 
 constexpr int kTileN = 256;
-constexpr int kMaxWaveTilesM = 8;                         // a wave's part of C is at most 128 x 64
-constexpr int kTiledWaves = 8;
-constexpr int kTiledThreads = kTiledWaves * kWave;
 constexpr int kPieceElements = 512;                       // of W: 16 rows x 32 k in MFMA operand order, 1 KB
-constexpr int kWaveTilesN = 4;                            // a wave's 64 columns of C
-constexpr int kSlotBytes = 65536;                         // a stage of 64 of k: up to 32 KB of A, then 32 KB of W
-constexpr int kSlotElements = kSlotBytes / 2;
-constexpr int kWBytes = 32768;                            // where W begins in a slot
+constexpr int kPackedStep = 1024;                         // from a tile's first k step to its second in a slot
 constexpr int kSuperM = 4, kSuperN = 8;                   // tiles of C that run together on an XCD
 
 __device__ __align__(16) const unsigned zero_piece[256] = {};      // a piece of W past the end of k
 
-
-__device__ inline unsigned lds_address(bf16* place) { return static_cast<unsigned>(reinterpret_cast<uintptr_t>((lds_bf16*)place)); }
-
-template <int WM>
-struct TiledOperands {       // of one k step: the wave's WM pieces of A and 4 of W, 16 bytes a lane each
-    uintx4 a[WM];
-    uintx4 w[kWaveTilesN];
-};
-
-#define MLL_DS_READ(TARGET, ADDRESS, BYTES) asm volatile("ds_read_b128 %0, %1 offset:%2" : "=v"(TARGET) : "v"(ADDRESS), "n"(BYTES))
-#define MLL_MFMA(ACC, W, A) asm volatile("v_mfma_f32_16x16x32_bf16 %0, %1, %2, %0" : "+v"(ACC) : "v"(W), "v"(A))
-
-// The INDEX-th of the 4 + WM reads of k step STEP (0, 1) of a stage: pieces of A are 2 KB apart in a slot, tiles of W
-// too, with the tile's second step 1 KB after its first. An INDEX beyond the reads is nothing.
-template <int WM, int INDEX, int STEP>
-__device__ __attribute__((always_inline)) inline void read_operand(TiledOperands<WM>& f, unsigned a_address, unsigned w_address) {
-    constexpr int W = kWBytes + STEP * 1024;
-    if constexpr (INDEX == 0) MLL_DS_READ(f.w[0], w_address, W);
-    if constexpr (INDEX == 1) MLL_DS_READ(f.w[1], w_address, W + 2048);
-    if constexpr (INDEX == 2) MLL_DS_READ(f.a[0], a_address, 0);
-    if constexpr (INDEX == 3) MLL_DS_READ(f.a[1], a_address, 2048);
-    if constexpr (INDEX == 4) MLL_DS_READ(f.w[2], w_address, W + 4096);
-    if constexpr (INDEX == 5) MLL_DS_READ(f.w[3], w_address, W + 6144);
-    if constexpr (INDEX >= 6 && INDEX < 4 + WM) MLL_DS_READ(f.a[INDEX - 4], a_address, (INDEX - 4) * 2048);
-}
-template <int WM, int STEP, int... INDEX>
-__device__ __attribute__((always_inline)) inline void read_operands(TiledOperands<WM>& f, unsigned a_address, unsigned w_address,
-                                                                    std::integer_sequence<int, INDEX...>) {
-    (read_operand<WM, INDEX, STEP>(f, a_address, w_address), ...);
-}
-
-// The four products of row tile MT of a k step, and after every second of them a read of the next step's operands
-// (the first 4 + WM of the 2 WM places take one).
-template <int WM, int NEXT_STEP, int MT>
-__device__ __attribute__((always_inline)) inline void products_of_row_tile(floatx4 (&acc)[kWaveTilesN][WM], const TiledOperands<WM>& now,
-                                                                           TiledOperands<WM>& next, unsigned a_address, unsigned w_address) {
-    MLL_MFMA(acc[0][MT], now.w[0], now.a[MT]);
-    MLL_MFMA(acc[1][MT], now.w[1], now.a[MT]);
-    read_operand<WM, 2 * MT, NEXT_STEP>(next, a_address, w_address);
-    MLL_MFMA(acc[2][MT], now.w[2], now.a[MT]);
-    MLL_MFMA(acc[3][MT], now.w[3], now.a[MT]);
-    read_operand<WM, 2 * MT + 1, NEXT_STEP>(next, a_address, w_address);
-}
-template <int WM, int NEXT_STEP, int... MT>
-__device__ __attribute__((always_inline)) inline void products(floatx4 (&acc)[kWaveTilesN][WM], const TiledOperands<WM>& now,
-                                                               TiledOperands<WM>& next, unsigned a_address, unsigned w_address,
-                                                               std::integer_sequence<int, MT...>) {
-    (products_of_row_tile<WM, NEXT_STEP, MT>(acc, now, next, a_address, w_address), ...);
-}
-
-// The reads into `f` have arrived (and, LOADS, the wave's loads into LDS have landed). `f` passes through the
-// statements, so that nothing that uses it is placed before.
-template <bool LOADS, int WM>
-__device__ __attribute__((always_inline)) inline void operands_arrived(TiledOperands<WM>& f) {
-    if constexpr (LOADS)
-        asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)"
-                     : "+v"(f.a[0]), "+v"(f.a[1]), "+v"(f.a[2]), "+v"(f.a[3]), "+v"(f.w[0]), "+v"(f.w[1]), "+v"(f.w[2]), "+v"(f.w[3])
-                     :: "memory");
-    else
-        asm volatile("s_waitcnt lgkmcnt(0)"
-                     : "+v"(f.a[0]), "+v"(f.a[1]), "+v"(f.a[2]), "+v"(f.a[3]), "+v"(f.w[0]), "+v"(f.w[1]), "+v"(f.w[2]), "+v"(f.w[3])
-                     :: "memory");
-#pragma unroll
-    for (int i = 4; i < WM; ++i) asm volatile("" : "+v"(f.a[i]));
-}
 
 // EPILOGUE: 0 = float32 [M, N]; 1 = bfloat16 [M, N]; 2 = bfloat16 [M, N / 2] = silu(even rows of W) * (odd rows);
 // 3 = queries, keys and values: bias, rotation, queries to `store.q_out`, keys and values into their pages (W's rows
@@ -232,18 +156,18 @@ __global__ __launch_bounds__(kTiledThreads, 1) void gemm_tiled_kernel(const bf16
         if (a_loads == A_TURNS) asm volatile("s_waitcnt vmcnt(%0)" :: "n"(A_TURNS + 4) : "memory");
         else asm volatile("s_waitcnt vmcnt(%0)" :: "n"(A_TURNS + 3) : "memory");
         __builtin_amdgcn_s_barrier();
-        read_operands<WM, 0>(even, a_step0, w_lane, std::make_integer_sequence<int, 4 + WM>{});
+        read_operands<kPackedStep, WM, 0>(even, a_step0, w_lane, std::make_integer_sequence<int, 4 + WM>{});
         // A stage that lies in slot SLOT. Its first step is multiplied while its second is read. Then the wave's
         // loads of the next stage have landed; after the barrier everyone's have, and everyone has read this stage,
         // whose slot the stage after next may take. The second step is multiplied while the next stage's first is read.
 #define MLL_TILED_STAGE(SLOT)                                                                              \
     {                                                                                                      \
         operands_arrived<false>(even);                                                                     \
-        products<WM, 1>(acc, even, odd, a_step1 + SLOT * kSlotBytes, w_lane + SLOT * kSlotBytes, std::make_integer_sequence<int, WM>{}); \
+        products<kPackedStep, WM, 1>(acc, even, odd, a_step1 + SLOT * kSlotBytes, w_lane + SLOT * kSlotBytes, std::make_integer_sequence<int, WM>{}); \
         operands_arrived<true>(odd);                                                                       \
         __builtin_amdgcn_s_barrier();                                                                      \
         copy_stage(stage + 2, SLOT);                                                                       \
-        products<WM, 0>(acc, odd, even, a_step0 + (1 - SLOT) * kSlotBytes, w_lane + (1 - SLOT) * kSlotBytes, std::make_integer_sequence<int, WM>{}); \
+        products<kPackedStep, WM, 0>(acc, odd, even, a_step0 + (1 - SLOT) * kSlotBytes, w_lane + (1 - SLOT) * kSlotBytes, std::make_integer_sequence<int, WM>{}); \
         ++stage;                                                                                           \
     }
         // Two stages a round; a stage past the end multiplies by zeros.
@@ -360,7 +284,7 @@ __global__ __launch_bounds__(kTiledThreads, 1) void gemm_tiled_kernel(const bf16
                 }
             } else {
                 auto gated = [&](float gate, float up) {
-                    return EPILOGUE == 7 ? gated_value(gate, up, kActClampedGlu, limit, slope) : gate_fast<EPILOGUE == 5>(gate) * up;
+                    return EPILOGUE == 7 ? gated_value_fast(gate, up, kActClampedGlu, limit, slope) : gate_fast<EPILOGUE == 5>(gate) * up;
                 };
                 bf16* target = static_cast<bf16*>(out) + static_cast<int64_t>(row) * (n / 2) + column / 2;
                 if (column + 3 < n && n % 4 == 0) {

@@ -13,6 +13,10 @@
 // four pairs and a pair's sums never depend on the other pairs. These serve every dtype and number of tokens.
 #include "common.h"
 #include "microllm_hip.h"
+#include "moe_tiled.h"
+
+#include <algorithm>
+#include <type_traits>
 
 namespace mll {
 
@@ -691,7 +695,7 @@ moe_stream_kernel(const bf16* __restrict__ x, const bf16* __restrict__ in, const
 #pragma unroll
                 for (int i = 0; i < 4; i += 2) {
                     const int column = first + quad * 2 + i / 2;
-                    if (column < n_out) to[column] = from_float<bf16>(gated_value(acc[i], acc[i + 1], form.activation, form.limit, form.slope));
+                    if (column < n_out) to[column] = from_float<bf16>(gated_value_fast(acc[i], acc[i + 1], form.activation, form.limit, form.slope));
                 }
             } else if (FORM == 2) {
                 bf16* to = static_cast<bf16*>(out) + static_cast<int64_t>(mine) * n_out;
@@ -945,7 +949,7 @@ moe_grouped_kernel(const bf16* __restrict__ a, const bf16* __restrict__ w, const
                 for (int i = 0; i < 4; ++i) {
                     const int column = col0 + wn * (kGroupCols / 4) + nt * 16 + quad * 4 + i;
                     const float g = acc[mt][nt][i], u = acc[mt][nt + kTiles / 2][i];
-                    if (column < n_out) to[column] = from_float<bf16>(gated_value(g, u, activation, form.limit, form.slope));
+                    if (column < n_out) to[column] = from_float<bf16>(gated_value_fast(g, u, activation, form.limit, form.slope));
                 }
         } else if (FORM == 2) {
             bf16* to = static_cast<bf16*>(out) + static_cast<int64_t>(first_row + row) * n_out;
@@ -1133,15 +1137,27 @@ int mll_moe_grouped(const void* x, const int32_t* ids, const float* weights, int
     }
     const int tiles = (n_pairs + kGroupRows - 1) / kGroupRows + experts + 1;
     MLL_REQUIRE(tiles < 65536, "moe_grouped: too many tiles of rows for one launch");
-#define MLL_MOE_GROUPED(FORM, columns, from, weight, to, n_out, k, from_tokens)                                                   \
-    moe_grouped_kernel<FORM><<<dim3(((columns) + kGroupCols - 1) / kGroupCols, tiles), 256, 0, stream>>>(                         \
-        from, static_cast<const bf16*>(weight), offsets, order, weights, n_out, k, to, top, n_tokens, weight_on_input, from_tokens, \
-        static_cast<const bf16*>(x), *form)
-    if (form->gated) MLL_MOE_GROUPED(1, 2 * ff, inputs, gate_up, act, ff, width, !weight_on_input);
-    else MLL_MOE_GROUPED(2, ff, inputs, gate_up, act, ff, width, !weight_on_input);
-    MLL_MOE_GROUPED(0, width, static_cast<const bf16*>(act), down, out, width, ff, 0);
-#undef MLL_MOE_GROUPED
-    return check_launch("moe_grouped");
+    const auto product = [&](auto form_number, int columns, const bf16* from, const void* weight, void* to, int n_out, int k, int from_tokens) {
+        constexpr int FORM = decltype(form_number)::value;
+        const bf16* w = static_cast<const bf16*>(weight);
+        const bool aligned = (reinterpret_cast<uintptr_t>(from) | reinterpret_cast<uintptr_t>(w) | reinterpret_cast<uintptr_t>(x)) % 16 == 0;
+        const int64_t row_bytes = 2 * static_cast<int64_t>(k), a_rows = from_tokens ? n_tokens : n_pairs, w_rows = FORM == 1 ? 2 * n_out : n_out;
+        // Large tiles where the experts have pairs for them, or are many enough that their weights' tiles make two rounds of the compute units
+        // (gate, up and down; 16 experts of 2048 x 2048, 4 of 20 choices: 400 tokens 129 and 139 us, 800 184 and 146, 3117 426 and 343, 6000 739 and
+        // 559; 64 of 1024 x 2048, 6 choices: 400 tokens 243 and 214, 3117 524 and 398; 8 of 4096 x 2048, 2 choices: 400 tokens 138 and 141, 800 157 and 143).
+        const bool fills = n_pairs >= 128 * static_cast<int64_t>(experts) || experts * ((w_rows + 255) / 256) >= 512;
+        if (k % 128 == 0 && aligned && std::max(a_rows, w_rows) * row_bytes < (int64_t{1} << 32) && fills)
+            return launch_moe_tiled(FORM, from, w, offsets, order, weights, n_out, k, to, top, n_tokens, weight_on_input, from_tokens,
+                                    static_cast<const bf16*>(x), *form, stream);
+        moe_grouped_kernel<FORM><<<dim3((columns + kGroupCols - 1) / kGroupCols, tiles), 256, 0, stream>>>(
+            from, w, offsets, order, weights, n_out, k, to, top, n_tokens, weight_on_input, from_tokens, static_cast<const bf16*>(x), *form);
+        return check_launch("moe_grouped");
+    };
+    using std::integral_constant;
+    const int inner = form->gated ? product(integral_constant<int, 1>{}, 2 * ff, inputs, gate_up, act, ff, width, !weight_on_input)
+                                  : product(integral_constant<int, 2>{}, ff, inputs, gate_up, act, ff, width, !weight_on_input);
+    if (inner != 0) return inner;
+    return product(integral_constant<int, 0>{}, width, static_cast<const bf16*>(act), down, out, width, ff, 0);
 }
 
 int mll_moe_choose(const void* x, int dtype, const float* w, int n_tokens, int n_out, int width, int experts, int top, int softmax_scores,

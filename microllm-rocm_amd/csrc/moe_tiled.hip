@@ -1,0 +1,275 @@
+// The chosen experts' products for many (token, choice) pairs, in large tiles: the pairs lie in the order of their experts
+// (moe_sort_kernel in moe.hip), and a workgroup of 8 waves takes up to 256 pairs of one expert and 256 rows of its weight, with the main loop of
+// gemm_tiled.hip: stages of 64 of the reduction by direct loads into one of two LDS slots, the operands of a k step read from
+// LDS between the products of the step before. Here both sides are rows of memory, 8 rows of 128 bytes a load, and A's rows are taken from
+// wherever their tokens lie. Bound by the loads of a stage (64 KB, which a compute unit brings in 1.5 us) and by a tile's beginning and end, which
+// nothing overlaps: as many workgroups as compute units go from tile to tile, and the height of the tiles is chosen so that their rounds are done
+// first (an expert's last pairs take a tile of 192 or 128 rows where that is enough). 3117 tokens with 4 of 16 experts of 2048 x 2048 and 4
+// ids that return their input: 426 -> 343 us with gate, up, down and the sort (tiles of 256 by a workgroup each 401), 0.73 PFLOP/s.
+// The tiles of all experts stand in a row, an expert after another, its columns one after another and down the rows first; every XCD takes
+// an equal stretch, so that the workgroups that run together there share an expert's rows and neighbouring rows of its weight.
+// A result's additions are those of moe_grouped_kernel in the same order, so a pair's bits do not depend on which of the two it meets.
+#include "common.h"
+#include "microllm_hip.h"
+#include "moe_tiled.h"
+#include "tiled_operands.h"
+
+namespace mll {
+
+namespace {
+
+typedef __bf16 bf16x4 __attribute__((ext_vector_type(4)));
+
+constexpr int kTileCols = 256;              // rows of the weight in a tile
+constexpr int kComputeUnits = 256;
+constexpr int kHeights[3] = {256, 192, 128};    // pairs of a tile, at most
+
+struct Tiling {
+    int height, tiles;       // tiles of pairs over all experts
+};
+struct TileOfExpert {
+    int expert, first_row, rows, column;
+};
+
+// The height of which all tiles are done first, if every round of the compute units takes as long as a stage's loads (rows + columns). A
+// lane an expert, 64 at a time.
+__device__ inline Tiling choose_tiling(const int32_t* __restrict__ offsets, int experts, int n_blocks, int lane) {
+    int tiles[3] = {0, 0, 0};
+    for (int base = 0; base < experts; base += kWave) {
+        const int e = base + lane;
+        const int count = e < experts ? offsets[e + 1] - offsets[e] : 0;
+#pragma unroll
+        for (int i = 0; i < 3; ++i) tiles[i] += (count + kHeights[i] - 1) / kHeights[i];
+    }
+    Tiling best = {0, 0};
+    int64_t least = 0;
+#pragma unroll
+    for (int i = 0; i < 3; ++i) {
+        for (int offset = kWave / 2; offset > 0; offset >>= 1) tiles[i] += __shfl_xor(tiles[i], offset, kWave);
+        const int64_t cost = (static_cast<int64_t>(tiles[i]) * n_blocks + kComputeUnits - 1) / kComputeUnits * (kHeights[i] + kTileCols);
+        if (i == 0 || cost < least) {
+            best = Tiling{kHeights[i], tiles[i]};
+            least = cost;
+        }
+    }
+    return Tiling{__builtin_amdgcn_readfirstlane(best.height), __builtin_amdgcn_readfirstlane(best.tiles)};
+}
+
+// The tile at a place of the row of all tiles (which has one there).
+__device__ inline TileOfExpert tile_at(int place, const int32_t* __restrict__ offsets, int experts, int n_blocks, int height, int lane) {
+    TileOfExpert found = {0, 0, 0, 0};
+    int before = 0;         // tiles of the experts so far
+    for (int base = 0; base < experts; base += kWave) {
+        const int e = base + lane;
+        const int begin = e < experts ? offsets[e] : 0, count = e < experts ? offsets[e + 1] - begin : 0;
+        const int tiles = (count + height - 1) / height;
+        int up_to_me = tiles;
+        for (int offset = 1; offset < kWave; offset <<= 1) {
+            const int theirs = __shfl_up(up_to_me, offset, kWave);
+            if (lane >= offset) up_to_me += theirs;
+        }
+        const int last = (before + up_to_me) * n_blocks, first = last - tiles * n_blocks;
+        const unsigned long long here = __ballot(place >= first && place < last);
+        if (here != 0) {
+            const int owner = __ffsll(here) - 1;
+            const int within = place - __shfl(first, owner, kWave), high = __shfl(tiles, owner, kWave);
+            const int row = within % high * height;
+            found.expert = __builtin_amdgcn_readfirstlane(base + owner);
+            found.first_row = __builtin_amdgcn_readfirstlane(__shfl(begin, owner, kWave) + row);
+            found.rows = __builtin_amdgcn_readfirstlane(min(height, __shfl(count, owner, kWave) - row));
+            found.column = __builtin_amdgcn_readfirstlane(within / high);
+            break;
+        }
+        before += __shfl(up_to_me, kWave - 1, kWave);
+    }
+    return found;
+}
+
+// FORM as in moe_grouped_kernel: 1 gated, 2 one inner weight, 0 down. The products of a tile of up to 32 WM pairs.
+template <int FORM, int WM>
+__device__ __attribute__((always_inline)) inline void tile_products(bf16* slots, const TileOfExpert& tile, const bf16* __restrict__ a,
+                                                                    const bf16* __restrict__ w, const int32_t* __restrict__ order,
+                                                                    const float* __restrict__ weights, int n_out, int k, void* __restrict__ out,
+                                                                    int top, int n_tokens, int weight_on_input, int from_tokens,
+                                                                    const MllExpertForm& form) {
+    constexpr bool GATED = FORM == 1;
+    constexpr int A_TURNS = WM / 2;        // loads of 8 rows a wave and stage
+    constexpr int W_TURNS = 4;
+    const int lane = threadIdx.x % kWave;
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave);
+    const int col = lane % 16, quad = lane / 16;
+    const int wave_m = wave / 4, wave_n = wave % 4;
+    // A gated tile holds 128 gate rows and the 128 up rows that belong to them: of a wave's four tiles of 16 two are gate's and two up's.
+    const int column0 = tile.column * (GATED ? kTileCols / 2 : kTileCols);
+    const bf16* w_expert = w + static_cast<int64_t>(tile.expert) * (GATED ? 2 * n_out : n_out) * k;
+
+    // Load i of a stage brings rows 8 i .. 8 i + 7 of the tile, lane L chunk (L % 8) ^ (row / 2) of row L / 8 of them; a wave takes
+    // the loads wave, wave + 8, ... Rows past the end repeat the last one.
+    const int row_in_piece = 8 * (wave % 2) + lane / 8;
+    const int chunk = ((lane % 8) ^ (row_in_piece / 2)) * 8;
+    unsigned a_from[A_TURNS], w_from[W_TURNS];         // bytes from `a` and from the expert's weight: 32 bits, which the caller has checked
+#pragma unroll
+    for (int t = 0; t < A_TURNS; ++t) {
+        const int row = tile.first_row + min((wave + t * kTiledWaves) * 8 + lane / 8, tile.rows - 1);
+        a_from[t] = (static_cast<unsigned>(from_tokens ? order[row] / top : row) * static_cast<unsigned>(k) + chunk) * 2;
+    }
+#pragma unroll
+    for (int t = 0; t < W_TURNS; ++t) {
+        const int row = (wave + t * kTiledWaves) * 8 + lane / 8;       // 64 of a wave's columns of C, 16 a tile
+        int w_row;
+        if (GATED) {
+            const int column = min(column0 + row / 64 * 32 + row % 32, n_out - 1);
+            w_row = row % 64 < 32 ? column : n_out + column;
+        } else {
+            w_row = min(column0 + row, n_out - 1);
+        }
+        w_from[t] = (static_cast<unsigned>(w_row) * static_cast<unsigned>(k) + chunk) * 2;
+    }
+    const char* a_bytes = reinterpret_cast<const char*>(a);
+    const char* w_bytes = reinterpret_cast<const char*>(w_expert);
+    auto copy_stage = [&](int stage, int slot) __attribute__((always_inline)) {
+        bf16* a_place = slots + slot * kSlotElements;
+        bf16* w_place = a_place + kWBytes / 2;
+#pragma unroll
+        for (int t = 0; t < A_TURNS; ++t)
+            __builtin_amdgcn_global_load_lds(a_bytes + stage * 128 + a_from[t], a_place + wave * 512 + t * (kTiledWaves * 512), 16, 0, 0);
+#pragma unroll
+        for (int t = 0; t < W_TURNS; ++t)
+            __builtin_amdgcn_global_load_lds(w_bytes + stage * 128 + w_from[t], w_place + wave * 512 + t * (kTiledWaves * 512), 16, 0, 0);
+    };
+    const unsigned base = lds_address(slots);
+    const unsigned step0 = col * 128 + ((quad ^ (col / 2)) * 16), step1 = col * 128 + (((4 + quad) ^ (col / 2)) * 16);
+    const unsigned a_at = base + wave_m * WM * 2048, w_at = base + wave_n * kWaveTilesN * 2048;
+
+    floatx4 acc[kWaveTilesN][WM];     // acc[nt][mt][i] = C[pair mt*16 + col][weight row nt*16 + quad*4 + i] of the wave's part
+#pragma unroll
+    for (int nt = 0; nt < kWaveTilesN; ++nt)
+#pragma unroll
+        for (int mt = 0; mt < WM; ++mt) acc[nt][mt] = floatx4{0.0f, 0.0f, 0.0f, 0.0f};
+
+    const int stages = k / 64;        // an even number: a way out between the two of a round would make the compiler keep the accumulators twice
+    TiledOperands<WM> even, odd;      // of a stage's first and second k step
+    copy_stage(0, 0);
+    copy_stage(1, 1);
+    asm volatile("s_waitcnt vmcnt(%0)" :: "n"(A_TURNS + W_TURNS) : "memory");      // this wave's loads of the first stage have landed
+    __builtin_amdgcn_s_barrier();
+    read_operands<0, WM, 0>(even, a_at + step0, w_at + step0, std::make_integer_sequence<int, 4 + WM>{});
+    // A stage in slot SLOT: its first step is multiplied while its second is read; then the next stage has landed (the wave's loads before
+    // the barrier, everyone's after it) and this one has been read by all, so that its slot may take the stage after next. After
+    // the last stage nothing is copied, and what is read then is multiplied by nobody.
+#define MLL_MOE_STAGE(STAGE, SLOT)                                                                                                                     \
+    operands_arrived<false>(even);                                                                                                                     \
+    products<0, WM, 1>(acc, even, odd, a_at + step1 + SLOT * kSlotBytes, w_at + step1 + SLOT * kSlotBytes, std::make_integer_sequence<int, WM>{});      \
+    operands_arrived<true>(odd);                                                                                                                       \
+    __builtin_amdgcn_s_barrier();                                                                                                                      \
+    if (STAGE + 2 < stages) copy_stage(STAGE + 2, SLOT);                                                                                               \
+    products<0, WM, 0>(acc, odd, even, a_at + step0 + (1 - SLOT) * kSlotBytes, w_at + step0 + (1 - SLOT) * kSlotBytes, std::make_integer_sequence<int, WM>{});
+    for (int stage = 0; stage < stages; stage += 2) {
+        MLL_MOE_STAGE(stage, 0)
+        MLL_MOE_STAGE(stage + 1, 1)
+    }
+#undef MLL_MOE_STAGE
+    // No read may be on its way into registers that something else takes, and the last products must have written their results before these are
+    // read (the compiler does not know that the asm statements are products).
+    operands_arrived<true>(even);
+    asm volatile("s_nop 15\n\ts_nop 15" ::: "memory");
+
+#pragma unroll
+    for (int mt = 0; mt < WM; ++mt) {
+        const int row = wave_m * (WM * 16) + mt * 16 + col;
+        if (row >= tile.rows) continue;
+        const int sorted = tile.first_row + row;
+        if constexpr (FORM == 0) {
+            const int pair = order[sorted];
+            const float factor = weight_on_input ? 1.0f : weights[pair];
+            float* to = static_cast<float*>(out) + (static_cast<int64_t>(pair % top) * n_tokens + pair / top) * n_out;
+#pragma unroll
+            for (int nt = 0; nt < kWaveTilesN; ++nt) {
+                const int column = column0 + wave_n * 64 + nt * 16 + quad * 4;      // four columns or none: n_out is a multiple of 8
+                if (column < n_out) *reinterpret_cast<floatx4*>(to + column) = acc[nt][mt] * factor;
+            }
+        } else {
+            bf16* to = static_cast<bf16*>(out) + static_cast<int64_t>(sorted) * n_out;
+#pragma unroll
+            for (int nt = 0; nt < (GATED ? kWaveTilesN / 2 : kWaveTilesN); ++nt) {
+                const int column = column0 + wave_n * (GATED ? 32 : 64) + nt * 16 + quad * 4;
+                bf16x4 four;
+#pragma unroll
+                for (int i = 0; i < 4; ++i)
+                    four[i] = static_cast<__bf16>(GATED ? gated_value_fast(acc[nt][mt][i], acc[GATED ? nt + 2 : nt][mt][i], form.activation, form.limit, form.slope)
+                                                        : activate(acc[nt][mt][i], form.activation));
+                if (column < n_out) *reinterpret_cast<bf16x4*>(to + column) = four;
+            }
+        }
+    }
+}
+
+}  // namespace
+
+template <int FORM>
+__global__ __launch_bounds__(kTiledThreads, 1) void moe_tiled_kernel(const bf16* __restrict__ a, const bf16* __restrict__ w,
+                                                                     const int32_t* __restrict__ offsets, const int32_t* __restrict__ order,
+                                                                     const float* __restrict__ weights, int n_out, int k, void* __restrict__ out,
+                                                                     int top, int n_tokens, int weight_on_input, int from_tokens,
+                                                                     const bf16* __restrict__ x, MllExpertForm form) {
+    __shared__ __align__(16) bf16 slots[2 * kSlotElements];
+    constexpr int kOutputsATile = FORM == 1 ? kTileCols / 2 : kTileCols;
+    const int lane = threadIdx.x % kWave;
+    const int n_blocks = (n_out + kOutputsATile - 1) / kOutputsATile;
+    const Tiling tiling = choose_tiling(offsets, form.experts, n_blocks, lane);
+    // Workgroups 8 apart in number run on one XCD: an equal stretch of the tiles each, whose workgroups go along it together.
+    const int all = tiling.tiles * n_blocks, per_xcd = (all + 7) / 8;
+    for (int index = blockIdx.x / 8; index < per_xcd; index += gridDim.x / 8) {
+        const int place = blockIdx.x % 8 * per_xcd + index;
+        if (place >= all) break;        // the same for every thread of the workgroup
+        const TileOfExpert tile = tile_at(place, offsets, form.experts, n_blocks, tiling.height, lane);
+        __builtin_amdgcn_s_barrier();       // every wave has read the last tile's stages
+        if (tile.rows > 192) tile_products<FORM, 8>(slots, tile, a, w, order, weights, n_out, k, out, top, n_tokens, weight_on_input, from_tokens, form);
+        else if (tile.rows > 128) tile_products<FORM, 6>(slots, tile, a, w, order, weights, n_out, k, out, top, n_tokens, weight_on_input, from_tokens, form);
+        else if (tile.rows > 0) tile_products<FORM, 4>(slots, tile, a, w, order, weights, n_out, k, out, top, n_tokens, weight_on_input, from_tokens, form);
+    }
+    if (FORM != 0 || form.identity == 0) return;
+    // The pairs of ids that return their input stand behind the experts': their inputs times their weights, eight columns a thread.
+    const int first = offsets[form.experts], last = offsets[form.experts + form.identity];
+    const int pieces = n_out / 8;       // n_out is a multiple of 8
+    const int64_t count = static_cast<int64_t>(last - first) * pieces;
+    for (int64_t index = static_cast<int64_t>(blockIdx.x) * kTiledThreads + threadIdx.x; index < count; index += static_cast<int64_t>(gridDim.x) * kTiledThreads) {
+        const int pair = order[first + static_cast<int>(index / pieces)], column = static_cast<int>(index % pieces) * 8;
+        const float weight = weights[pair];
+        const uintx4 given = *reinterpret_cast<const uintx4*>(x + static_cast<int64_t>(pair / top) * n_out + column);
+        floatx4* to = reinterpret_cast<floatx4*>(static_cast<float*>(out) + (static_cast<int64_t>(pair % top) * n_tokens + pair / top) * n_out + column);
+        floatx4 values[2];
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+            values[i / 2][2 * i % 4] = __builtin_bit_cast(float, given[i] << 16) * weight;
+            values[i / 2][(2 * i + 1) % 4] = __builtin_bit_cast(float, given[i] & 0xffff0000u) * weight;
+        }
+        to[0] = values[0];
+        to[1] = values[1];
+    }
+}
+
+template <int FORM>
+static int launch_form(const bf16* a, const bf16* w, const int32_t* offsets, const int32_t* order, const float* weights, int n_out, int k, void* out,
+                       int top, int n_tokens, int weight_on_input, int from_tokens, const bf16* x, const MllExpertForm& form, hipStream_t stream) {
+    const int columns = FORM == 1 ? kTileCols / 2 : kTileCols;
+    // as many workgroups as run at once, fewer where there cannot be as many tiles (every expert's last one may hold one pair)
+    const int64_t most = (static_cast<int64_t>(n_tokens) * top / kHeights[2] + form.experts) * ((n_out + columns - 1) / columns);
+    MLL_REQUIRE(most < (1ll << 31), "moe_tiled: too many tiles");
+    const int groups = static_cast<int>(most < kComputeUnits ? (most + 7) / 8 * 8 : kComputeUnits);
+    moe_tiled_kernel<FORM><<<groups, kTiledThreads, 0, stream>>>(
+        a, w, offsets, order, weights, n_out, k, out, top, n_tokens, weight_on_input, from_tokens, x, form);
+    return check_launch("moe_tiled");
+}
+
+int launch_moe_tiled(int form_number, const bf16* a, const bf16* w, const int32_t* offsets, const int32_t* order, const float* weights, int n_out,
+                     int k, void* out, int top, int n_tokens, int weight_on_input, int from_tokens, const bf16* x, const MllExpertForm& form,
+                     hipStream_t stream) {
+    switch (form_number) {
+        case 1: return launch_form<1>(a, w, offsets, order, weights, n_out, k, out, top, n_tokens, weight_on_input, from_tokens, x, form, stream);
+        case 2: return launch_form<2>(a, w, offsets, order, weights, n_out, k, out, top, n_tokens, weight_on_input, from_tokens, x, form, stream);
+        default: return launch_form<0>(a, w, offsets, order, weights, n_out, k, out, top, n_tokens, weight_on_input, from_tokens, x, form, stream);
+    }
+}
+
+}  // namespace mll

@@ -346,3 +346,30 @@ def test_decode_attention_reads_every_line_of_its_pages(heads, kv_heads, hd, pag
     out = torch.zeros_like(t["q"])
     k.paged_attention_decode(t["q"], t["k"], t["v"], t["table"], t["seq"], t["pos"], scale, 0, heads, kv_heads, hd, splits, out=out, extras=extras)
     np.testing.assert_allclose(out.float().cpu().numpy(), want.reshape(len(lengths), -1), **tolerance(torch.bfloat16))
+
+
+# ---- experts in large tiles: heights of 128, 192 and 256 rows, remainders of each, experts without a pair, more experts than a wave has lanes ----
+@pytest.mark.parametrize("n,width,ff,experts,top,identity,gated", [
+    (700, 128, 384, 3, 2, 0, True), (520, 256, 128, 2, 1, 1, True), (1300, 128, 264, 5, 2, 2, False), (400, 128, 128, 70, 3, 0, True),
+    (129, 384, 128, 1, 1, 0, True), (3000, 128, 256, 4, 2, 1, True)])
+def test_experts_in_large_tiles(n, width, ff, experts, top, identity, gated):
+    """Against the kernels that take a pair at a time, whose sums have another order; and the bits of the same pairs in steps too small for
+    the large tiles, which the smaller ones take."""
+    k, rng = kernels(), np.random.default_rng(n + ff)
+    x = device(rng.normal(size=(n, width)), torch.bfloat16)
+    gate_up = device(rng.normal(size=(experts, (2 if gated else 1) * ff, width)) * 0.2, torch.bfloat16)
+    down = device(rng.normal(size=(experts, width, ff)) * 0.2, torch.bfloat16)
+    ids = np.argsort(rng.random((n, experts + identity)) + np.linspace(0, 0.9, experts + identity), axis=1)[:, :top]      # the last ones are rarely chosen
+    ids = device(np.where((ids == experts - 1) & (experts > 3), 0, ids), torch.int32)       # and one never
+    weights = device(rng.uniform(0.2, 1.5, size=(n, top)))
+    for on_input in (False, True):
+        options = dict(gated=gated, activation="silu", identity=identity)
+        if on_input and identity:
+            continue
+        tiled = k.moe_experts(x, ids, weights, gate_up, down, on_input, grouped=True, **options)
+        one_by_one = k.moe_experts(x, ids, weights, gate_up, down, on_input, grouped=False, **options)
+        assert float((tiled - one_by_one).abs().max()) < 0.02 * float(one_by_one.abs().max())      # the inner values are rounded from sums in another order
+        few = 100 * experts // top       # below 128 pairs an expert
+        if experts * (-(-ff // 128)) < 512:
+            small = k.moe_experts(x[:few], ids[:few].contiguous(), weights[:few].contiguous(), gate_up, down, on_input, grouped=True, **options)
+            assert torch.equal(small, tiled[:, :few])
