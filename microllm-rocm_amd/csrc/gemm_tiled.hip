@@ -4,19 +4,18 @@
 // A workgroup of 8 waves (two on every SIMD) owns a 256 x 256 tile of C, a wave 128 x 64 of it (8 x 4 MFMA tiles,
 // 128 accumulator registers); or a tile of 192, 160 or 128 rows (a wave 6, 5 or 4 row tiles), where tiles of 256
 // rows would leave many compute units without one. k is walked in stages of 64. A stage's 256 rows of A and of W (64 KB) are brought
-// into one of two LDS slots by direct global-to-LDS loads, 1 KB a wave-wide instruction: of A 8 rows of 128 bytes
+// into LDS slots (two of A, three of W) by direct global-to-LDS loads, 1 KB a wave-wide instruction: of A 8 rows of 128 bytes
 // (whole cache lines: with half lines, 64 bytes of 16 rows, the loads alone take a quarter longer), of W a piece as
 // it lies in memory. A row's eight 16-byte chunks are stored at places exchanged by (row / 2), so that the 64 lanes
 // of an operand read (row = lane % 16, chunk = 4 step + lane / 16) fall on all banks.
 // A wave holds the operands of two k steps of 32 in registers: while it multiplies one step's (32 products), the
-// next step's 12 reads from LDS are issued between the products, one after every second, and have arrived when the
-// products are done. The workgroup meets once a stage, when the next stage has landed and the slot of the stage
-// before is free for the stage after next. The reads and the products are volatile asm, which pins their order;
+// next step's 12 reads from LDS are issued between the products, one after every second, and a stage's eight loads likewise
+// (tiled_operands.h): a compute unit takes a load in 16 cycles, and asked for in one go, as before, 64 of them held the
+// products up for a third of a stage. The reads and the products are volatile asm, which pins their order;
 // the compiler neither sees the reads (and so orders nothing against the loads in flight) nor moves the products.
-// Timed on MI355X against reads and a barrier before each stage's products, with half lines of A:
-// 8192 x 37888 x 3584 2200 -> 1800 us (1.24 PFLOP/s), 2048 x 37888 x 3584 580 -> 480 us.
-// Taken apart at 8192 x 37888 x 3584: products and barriers alone 1230 us, the loads alone (one stage in flight)
-// 1550, everything 1790.
+// Bound by the loads: a compute unit brings a stage's 64 KB in 1.3 to 1.5 us. Gated, before and with the loads between the products, results stored
+// as whole rows, and as many workgroups as compute units going from tile to tile: 8192 x 37888 x 3584 1747 -> 1622 us (1.37 PFLOP/s),
+// 16301 rows 3599 -> 3215, 2048 rows 455 -> 411, 8192 x 16384 x 2048 440 -> 397, 2048 x 9728 x 896 45.7 -> 37.0.
 // Workgroups are numbered so that the 32 that run together on one of the 8 XCDs (each with a second-level cache of
 // its own) own about 4 x 8 neighbouring tiles of C, and so share their rows of A and of W there, and so that every
 // XCD gets the same number of tiles.
@@ -47,8 +46,8 @@ __device__ __align__(16) const unsigned zero_piece[256] = {};      // a piece of
 template <int EPILOGUE, int WM>
 __global__ __launch_bounds__(kTiledThreads, 1) void gemm_tiled_kernel(const bf16* __restrict__ a, const bf16* __restrict__ w_packed,
                                                                       void* __restrict__ out, int m, int n, int k, int n_tiles,
-                                                                      int k_steps, int m_blocks, int n_blocks, MllQkvStore store,
-                                                                      float limit, float slope) {
+                                                                      int k_steps, int m_blocks, int n_blocks, int whole_rows,
+                                                                      MllQkvStore store, float limit, float slope) {
     static_assert(WM >= 4 && WM <= kMaxWaveTilesM, "a wave takes 4 to 8 row tiles");
     constexpr int TILE_M = 32 * WM;
     constexpr int A_LOADS = 4 * WM;                       // a stage of A: 2 WM pieces of 16 rows, two loads of 8 rows each
@@ -56,7 +55,7 @@ __global__ __launch_bounds__(kTiledThreads, 1) void gemm_tiled_kernel(const bf16
     // Two slots. In a slot: A as [2 WM pieces of 16 rows][row][8 places of 16 bytes], the row's chunk c of 8 elements
     // at place c ^ (row / 2); then W as [16 tiles][2 k steps][1 KB in MFMA operand order]. Only the direct loads write
     // this memory and only the asm reads read it.
-    __shared__ __align__(16) bf16 slots[2 * kSlotElements];
+    __shared__ __align__(16) bf16 slots[kStageElements];
 
     // Workgroups 8 apart in number run on one XCD, 32 of them at a time. The tiles of C are put in a row, blocks of
     // 4 x 8 neighbouring tiles after one another (down the rows of C first, narrower at the edges), and every XCD
@@ -64,238 +63,218 @@ __global__ __launch_bounds__(kTiledThreads, 1) void gemm_tiled_kernel(const bf16
     // has more than one tile more than another.
     const int tiles = m_blocks * n_blocks;
     const int per_xcd = (tiles + 7) / 8;
-    const int place = (blockIdx.x % 8) * per_xcd + blockIdx.x / 8;
-    if (blockIdx.x / 8 >= per_xcd || place >= tiles) return;
-    const int column = place / (m_blocks * kSuperN);                       // of blocks, kSuperN tiles wide
-    const int width = min(kSuperN, n_blocks - column * kSuperN);
-    const int in_column = place - column * m_blocks * kSuperN;
-    const int block = in_column / (kSuperM * width);                       // in the column, kSuperM tiles high
-    const int height = min(kSuperM, m_blocks - block * kSuperM);
-    const int in_block = in_column - block * kSuperM * width;
-    const int m_block = block * kSuperM + in_block % height;
-    const int n_block = column * kSuperN + in_block / height;
+    for (int index = blockIdx.x / 8; index < per_xcd; index += gridDim.x / 8) {
+        const int place = (blockIdx.x % 8) * per_xcd + index;
+        if (place >= tiles) return;
+        const int column = place / (m_blocks * kSuperN);                       // of blocks, kSuperN tiles wide
+        const int width = min(kSuperN, n_blocks - column * kSuperN);
+        const int in_column = place - column * m_blocks * kSuperN;
+        const int block = in_column / (kSuperM * width);                       // in the column, kSuperM tiles high
+        const int height = min(kSuperM, m_blocks - block * kSuperM);
+        const int in_block = in_column - block * kSuperM * width;
+        const int m_block = block * kSuperM + in_block % height;
+        const int n_block = column * kSuperN + in_block / height;
 
-    const int lane = threadIdx.x % kWave;
-    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave);
-    const int col = lane % 16, quad = lane / 16;
-    const int wave_m = wave / 4, wave_n = wave % 4;        // which (16 WM) x 64 of the tile
-    const int m0 = m_block * TILE_M, n_tile0 = n_block * (kTileN / 16);
+        const int lane = threadIdx.x % kWave;
+        const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave);
+        const int col = lane % 16, quad = lane / 16;
+        const int wave_m = wave / 4, wave_n = wave % 4;        // which (16 WM) x 64 of the tile
+        const int m0 = m_block * TILE_M, n_tile0 = n_block * (kTileN / 16);
 
-    // What this wave copies per stage. Of A the loads wave, wave + 8, ... of the stage's 4 WM: load i brings 8 rows
-    // (half h = i % 2 of piece i / 2; lane L: row L / 8 of the 8, place L % 8 of the row). Of W tiles 2 * wave and
-    // 2 * wave + 1, a k step an instruction.
-    const bf16* a_block = a + static_cast<int64_t>(m0) * k;
-    int a_offset[A_TURNS];    // of the lane's 16 bytes from a_block, at stage 0
-    const int a_loads = (A_LOADS - wave + kTiledWaves - 1) / kTiledWaves;      // of this wave
-#pragma unroll
-    for (int t = 0; t < A_TURNS; ++t) {
-        const int load = min(wave + t * kTiledWaves, A_LOADS - 1);
-        const int row_in_piece = 8 * (load % 2) + lane / 8;
-        const int row = min((load / 2) * 16 + row_in_piece, m - 1 - m0);           // rows past the end repeat the last one
-        a_offset[t] = row * k + (((lane % 8) ^ (row_in_piece / 2)) * 8);
-    }
-    const bf16* w_tile[2];    // the lane's 16 bytes of the tile's piece at k step 0
-#pragma unroll
-    for (int p = 0; p < 2; ++p) {
-        const int tile = min(n_tile0 + wave * 2 + p, n_tiles - 1);
-        w_tile[p] = w_packed + static_cast<int64_t>(tile) * k_steps * kPieceElements + lane * 8;
-    }
-    const int all_stages = (k_steps + 1) / 2;
-    const int stages_per_split = (all_stages + gridDim.y - 1) / gridDim.y;
-    const int first_stage = blockIdx.y * stages_per_split;
-    const int stages = min(all_stages, first_stage + stages_per_split);
-    const int last = stages - 1;
-    // A k step past the end (k an odd multiple of 32; the stage after the last, which the loop's second half may
-    // take) gets zeros for W and, for A, values that lie in the row: the chunks of the stage's second half step
-    // back by 64 bytes there, the stage after the last is the last again.
-    auto copy_stage = [&](int stage, int slot) __attribute__((always_inline)) {
-        bf16* a_place = slots + slot * kSlotElements;
-        bf16* w_place = a_place + kWBytes / 2;
-        const int a_stage = min(stage, last);
-        const bool half_stage = 2 * a_stage + 1 >= k_steps;
+        // What this wave copies per stage. Of A the loads wave, wave + 8, ... of the stage's 4 WM: load i brings 8 rows
+        // (half h = i % 2 of piece i / 2; lane L: row L / 8 of the 8, place L % 8 of the row). Of W tiles 2 * wave and
+        // 2 * wave + 1, a k step an instruction.
+        const bf16* a_block = a + static_cast<int64_t>(m0) * k;
+        unsigned a_offset[A_TURNS];    // of the lane's 16 bytes from a_block, at stage 0, in bytes
+        const int a_loads = A_LOADS % kTiledWaves == 0 ? A_TURNS : (A_LOADS - wave + kTiledWaves - 1) / kTiledWaves;      // of this wave
 #pragma unroll
         for (int t = 0; t < A_TURNS; ++t) {
-            if (t < a_loads) {
-                const int piece = (wave + t * kTiledWaves) / 2, h = wave % 2;      // the wave's loads are all of one half
-                const bool upper = (((lane >> 2) & 1) ^ h) != 0;      // the lane's chunk is one of the row's second four
-                const bf16* a_source = a_block + a_stage * 64 + a_offset[t] - ((half_stage && upper) ? 32 : 0);
-                // (the place is computed here: with a subscript of a captured array in this call the host pass
-                // drops the kernel's stub without a word)
-                __builtin_amdgcn_global_load_lds(a_source, a_place + piece * 1024 + h * 512, 16, 0, 0);
-            }
+            const int load = min(wave + t * kTiledWaves, A_LOADS - 1);
+            const int row_in_piece = 8 * (load % 2) + lane / 8;
+            const int row = min((load / 2) * 16 + row_in_piece, m - 1 - m0);           // rows past the end repeat the last one
+            a_offset[t] = (static_cast<unsigned>(row) * static_cast<unsigned>(k) + (((lane % 8) ^ (row_in_piece / 2)) * 8)) * 2;
         }
+        const char* w_tile[2];    // the tile's piece at k step 0
 #pragma unroll
         for (int p = 0; p < 2; ++p) {
-#pragma unroll
-            for (int h = 0; h < 2; ++h) {
-                const bool real = stage <= last && 2 * stage + h < k_steps;
-                const bf16* w_source = real ? w_tile[p] + static_cast<int64_t>(2 * stage + h) * kPieceElements
-                                            : reinterpret_cast<const bf16*>(zero_piece) + lane * 8;
-                __builtin_amdgcn_global_load_lds(w_source, w_place + (wave * 2 + p) * 1024 + h * 512, 16, 0, 0);
-            }
+            const int tile = min(n_tile0 + wave * 2 + p, n_tiles - 1);
+            w_tile[p] = reinterpret_cast<const char*>(w_packed + static_cast<int64_t>(tile) * k_steps * kPieceElements);
         }
-    };
-    // Where the lane reads its operands: row `col` of a piece, chunk 4 step + quad at its place.
-    const unsigned base = lds_address(slots);
-    const unsigned a_row = base + wave_m * WM * 2048 + col * 128;
-    const unsigned a_step0 = a_row + ((quad ^ (col / 2)) * 16), a_step1 = a_row + (((4 + quad) ^ (col / 2)) * 16);
-    const unsigned w_lane = base + wave_n * kWaveTilesN * 2048 + lane * 16;
+        const unsigned w_offset = lane * 16;
+        const int all_stages = (k_steps + 1) / 2;
+        const int stages_per_split = (all_stages + gridDim.y - 1) / gridDim.y;
+        const int first_stage = blockIdx.y * stages_per_split;
+        const int stages = min(all_stages, first_stage + stages_per_split);
+        // A k step past the end (k an odd multiple of 32) gets zeros for W and, for A, values that lie in the row: the chunks of the stage's second
+        // half step back by 64 bytes there.
+        auto copy_a = [&](int turn, int stage, unsigned slot) __attribute__((always_inline)) {
+            bf16* a_place = slots + slot * kSlotElements;
+            const int piece = (wave + turn * kTiledWaves) / 2, h = wave % 2;      // the wave's loads are all of one half
+            const bool upper = (((lane >> 2) & 1) ^ h) != 0;      // the lane's chunk is one of the row's second four
+            const char* a_source = reinterpret_cast<const char*>(a_block) + stage * 128 + (a_offset[turn] - ((2 * stage + 1 >= k_steps && upper) ? 64u : 0u));
+            // (the place is computed here: with a subscript of a captured array in this call the host pass
+            // drops the kernel's stub without a word)
+            __builtin_amdgcn_global_load_lds(a_source, a_place + piece * 1024 + h * 512, 16, 0, 0);
+        };
+        auto copy_w = [&](int turn, int stage, unsigned slot) __attribute__((always_inline)) {      // turn: which of the wave's two tiles and k steps
+            bf16* w_place = slots + (kASlots + slot) * kSlotElements;
+            const int p = turn / 2, h = turn % 2;
+            const char* w_source = 2 * stage + h < k_steps ? w_tile[p] + static_cast<int64_t>(2 * stage + h) * (kPieceElements * 2)
+                                                           : reinterpret_cast<const char*>(zero_piece);
+            __builtin_amdgcn_global_load_lds(w_source + w_offset, w_place + (wave * 2 + p) * 1024 + h * 512, 16, 0, 0);
+        };
+        // Where the lane reads its operands: row `col` of a piece, chunk 4 step + quad at its place.
+        const unsigned base = lds_address(slots);
+        const unsigned a_row = base + wave_m * WM * 2048 + col * 128;
+        const unsigned a_step0 = a_row + ((quad ^ (col / 2)) * 16), a_step1 = a_row + (((4 + quad) ^ (col / 2)) * 16);
+        const unsigned w_lane = base + kASlots * kSlotBytes + wave_n * kWaveTilesN * 2048 + lane * 16;
 
-    floatx4 acc[kWaveTilesN][WM];     // acc[nt][mt][i] = C[m = mt*16 + col][n = nt*16 + quad*4 + i] of the wave's part
+        floatx4 acc[kWaveTilesN][WM];     // acc[nt][mt][i] = C[m = mt*16 + col][n = nt*16 + quad*4 + i] of the wave's part
 #pragma unroll
-    for (int nt = 0; nt < kWaveTilesN; ++nt)
+        for (int nt = 0; nt < kWaveTilesN; ++nt)
 #pragma unroll
-        for (int mt = 0; mt < WM; ++mt) acc[nt][mt] = floatx4{0.0f, 0.0f, 0.0f, 0.0f};
+            for (int mt = 0; mt < WM; ++mt) acc[nt][mt] = floatx4{0.0f, 0.0f, 0.0f, 0.0f};
 
-    if (first_stage < stages) {
-        int stage = first_stage;
-        copy_stage(stage, 0);
-        copy_stage(stage + 1, 1);
-        TiledOperands<WM> even, odd;      // of a stage's first and second k step
-        // The first stage's loads of this wave have landed when only the second stage's are on their way.
-        if (a_loads == A_TURNS) asm volatile("s_waitcnt vmcnt(%0)" :: "n"(A_TURNS + 4) : "memory");
-        else asm volatile("s_waitcnt vmcnt(%0)" :: "n"(A_TURNS + 3) : "memory");
-        __builtin_amdgcn_s_barrier();
-        read_operands<kPackedStep, WM, 0>(even, a_step0, w_lane, std::make_integer_sequence<int, 4 + WM>{});
-        // A stage that lies in slot SLOT. Its first step is multiplied while its second is read. Then the wave's
-        // loads of the next stage have landed; after the barrier everyone's have, and everyone has read this stage,
-        // whose slot the stage after next may take. The second step is multiplied while the next stage's first is read.
-#define MLL_TILED_STAGE(SLOT)                                                                              \
-    {                                                                                                      \
-        operands_arrived<false>(even);                                                                     \
-        products<kPackedStep, WM, 1>(acc, even, odd, a_step1 + SLOT * kSlotBytes, w_lane + SLOT * kSlotBytes, std::make_integer_sequence<int, WM>{}); \
-        operands_arrived<true>(odd);                                                                       \
-        __builtin_amdgcn_s_barrier();                                                                      \
-        copy_stage(stage + 2, SLOT);                                                                       \
-        products<kPackedStep, WM, 0>(acc, odd, even, a_step0 + (1 - SLOT) * kSlotBytes, w_lane + (1 - SLOT) * kSlotBytes, std::make_integer_sequence<int, WM>{}); \
-        ++stage;                                                                                           \
-    }
-        // Two stages a round; a stage past the end multiplies by zeros.
-        while (stage < stages) {
-            MLL_TILED_STAGE(0)
-            MLL_TILED_STAGE(1)
+        if (first_stage < stages) {
+            if (index != static_cast<int>(blockIdx.x) / 8) workgroup_meets();        // every wave is done with the slots of the tile before
+            multiply_stages<kPackedStep, WM, A_TURNS>(acc, first_stage, stages, a_loads, a_step0, a_step1, w_lane, w_lane, copy_a, copy_w);
         }
-#undef MLL_TILED_STAGE
-        // No load may be on its way into LDS when the workgroup ends, and the last products must have written
-        // their results before these are read (the compiler does not know that the asm statements are products).
-        asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)\n\ts_nop 15\n\ts_nop 15" ::: "memory");
-    }
 
-    if constexpr (EPILOGUE == 3) {
-        // The lane's 4 columns of a tile lie in one head (head_dim is a multiple of 16). In a query or key head
-        // columns 2p and 2p + 1 hold dims p and p + n_freq, the two that rotate together, so the lane's columns are
-        // dims p, p + n_freq, p + 1, p + 1 + n_freq with p even: two neighbours in each half, stored as one word
-        // each. Dims beyond the rotated ones, and values, are in place.
-        const CacheLayout layout(store.kv_heads, store.page_size, store.head_dim);
+        if constexpr (EPILOGUE == 3) {
+            // The lane's 4 columns of a tile lie in one head (head_dim is a multiple of 16). In a query or key head
+            // columns 2p and 2p + 1 hold dims p and p + n_freq, the two that rotate together, so the lane's columns are
+            // dims p, p + n_freq, p + 1, p + 1 + n_freq with p even: two neighbours in each half, stored as one word
+            // each. Dims beyond the rotated ones, and values, are in place.
+            const CacheLayout layout(store.kv_heads, store.page_size, store.head_dim);
 #pragma unroll
-        for (int nt = 0; nt < kWaveTilesN; ++nt) {
-            const int column = (n_tile0 + wave_n * kWaveTilesN + nt) * 16 + quad * 4;
-            if (column >= n) continue;
-            const int head = column / store.head_dim, within = column % store.head_dim;
-            const bool is_query = head < store.heads;
-            const bool is_value = head >= store.heads + store.kv_heads;
-            const bool rotate = !is_value && within + 3 < 2 * store.n_freq;        // both pairs or, n_freq being even here, none
-            const int pair = within / 2;
-            // dims of the lane's four results, in the order of the accumulator
-            int dim[4];
+            for (int nt = 0; nt < kWaveTilesN; ++nt) {
+                const int column = (n_tile0 + wave_n * kWaveTilesN + nt) * 16 + quad * 4;
+                if (column >= n) continue;
+                const int head = column / store.head_dim, within = column % store.head_dim;
+                const bool is_query = head < store.heads;
+                const bool is_value = head >= store.heads + store.kv_heads;
+                const bool rotate = !is_value && within + 3 < 2 * store.n_freq;        // both pairs or, n_freq being even here, none
+                const int pair = within / 2;
+                // dims of the lane's four results, in the order of the accumulator
+                int dim[4];
 #pragma unroll
-            for (int i = 0; i < 4; ++i) dim[i] = rotate ? pair + i / 2 + (i % 2) * store.n_freq : within + i;
-            float bias[4] = {0.0f, 0.0f, 0.0f, 0.0f};
-            if (store.bias) {
+                for (int i = 0; i < 4; ++i) dim[i] = rotate ? pair + i / 2 + (i % 2) * store.n_freq : within + i;
+                float bias[4] = {0.0f, 0.0f, 0.0f, 0.0f};
+                if (store.bias) {
 #pragma unroll
-                for (int i = 0; i < 4; ++i) bias[i] = store.bias[head * store.head_dim + dim[i]];
-            }
-#pragma unroll
-            for (int mt = 0; mt < WM; ++mt) {
-                const int row = m0 + wave_m * (WM * 16) + mt * 16 + col;
-                if (row >= m) continue;
-                float y[4];
-#pragma unroll
-                for (int i = 0; i < 4; ++i) y[i] = acc[nt][mt][i] + bias[i];
-                if (rotate) {
-                    const floatx4 cs = *reinterpret_cast<const floatx4*>(store.cos_sin + (static_cast<int64_t>(row) * store.n_freq + pair) * 2);
-                    const float x0 = y[0], x1 = y[1], x2 = y[2], x3 = y[3];
-                    y[0] = rotate_first(x0, x1, cs[0], cs[1]);
-                    y[1] = rotate_second(x0, x1, cs[0], cs[1]);
-                    y[2] = rotate_first(x2, x3, cs[2], cs[3]);
-                    y[3] = rotate_second(x2, x3, cs[2], cs[3]);
+                    for (int i = 0; i < 4; ++i) bias[i] = store.bias[head * store.head_dim + dim[i]];
                 }
-                // y[0], y[2] are neighbours in dim (dim[0], dim[0] + 1) when rotated, and so are y[1], y[3]
-                bf16x2 low, high;
-                if (rotate) {
-                    low[0] = static_cast<__bf16>(y[0]); low[1] = static_cast<__bf16>(y[2]);
-                    high[0] = static_cast<__bf16>(y[1]); high[1] = static_cast<__bf16>(y[3]);
-                } else {
-                    low[0] = static_cast<__bf16>(y[0]); low[1] = static_cast<__bf16>(y[1]);
-                    high[0] = static_cast<__bf16>(y[2]); high[1] = static_cast<__bf16>(y[3]);
-                }
-                const int low_dim = dim[0], high_dim = rotate ? dim[1] : dim[2];
-                if (is_query) {
-                    bf16* q_row = static_cast<bf16*>(store.q_out) + (static_cast<int64_t>(row) * store.heads + head) * store.head_dim;
-                    *reinterpret_cast<bf16x2*>(q_row + low_dim) = low;
-                    *reinterpret_cast<bf16x2*>(q_row + high_dim) = high;
-                    continue;
-                }
-                if (!store.slot_mapping) continue;
-                const int slot = store.slot_mapping[row];
-                if (slot < 0) continue;
-                const int page = slot / store.page_size, offset = slot % store.page_size;
-                if (!is_value) {
-                    bf16* pages = static_cast<bf16*>(store.k_cache);        // two neighbouring dims are neighbours in a page of keys
-                    *reinterpret_cast<bf16x2*>(pages + layout.k_at(page, head - store.heads, offset, low_dim)) = low;
-                    *reinterpret_cast<bf16x2*>(pages + layout.k_at(page, head - store.heads, offset, high_dim)) = high;
-                } else {
-                    bf16* pages = static_cast<bf16*>(store.v_cache);        // and 8 elements apart in a page of values
-                    const int kv_head = head - store.heads - store.kv_heads;
 #pragma unroll
-                    for (int i = 0; i < 4; ++i) pages[layout.v_at(page, kv_head, offset, within + i)] = from_float<bf16>(y[i]);
+                for (int mt = 0; mt < WM; ++mt) {
+                    const int row = m0 + wave_m * (WM * 16) + mt * 16 + col;
+                    if (row >= m) continue;
+                    float y[4];
+#pragma unroll
+                    for (int i = 0; i < 4; ++i) y[i] = acc[nt][mt][i] + bias[i];
+                    if (rotate) {
+                        const floatx4 cs = *reinterpret_cast<const floatx4*>(store.cos_sin + (static_cast<int64_t>(row) * store.n_freq + pair) * 2);
+                        const float x0 = y[0], x1 = y[1], x2 = y[2], x3 = y[3];
+                        y[0] = rotate_first(x0, x1, cs[0], cs[1]);
+                        y[1] = rotate_second(x0, x1, cs[0], cs[1]);
+                        y[2] = rotate_first(x2, x3, cs[2], cs[3]);
+                        y[3] = rotate_second(x2, x3, cs[2], cs[3]);
+                    }
+                    // y[0], y[2] are neighbours in dim (dim[0], dim[0] + 1) when rotated, and so are y[1], y[3]
+                    bf16x2 low, high;
+                    if (rotate) {
+                        low[0] = static_cast<__bf16>(y[0]); low[1] = static_cast<__bf16>(y[2]);
+                        high[0] = static_cast<__bf16>(y[1]); high[1] = static_cast<__bf16>(y[3]);
+                    } else {
+                        low[0] = static_cast<__bf16>(y[0]); low[1] = static_cast<__bf16>(y[1]);
+                        high[0] = static_cast<__bf16>(y[2]); high[1] = static_cast<__bf16>(y[3]);
+                    }
+                    const int low_dim = dim[0], high_dim = rotate ? dim[1] : dim[2];
+                    if (is_query) {
+                        bf16* q_row = static_cast<bf16*>(store.q_out) + (static_cast<int64_t>(row) * store.heads + head) * store.head_dim;
+                        *reinterpret_cast<bf16x2*>(q_row + low_dim) = low;
+                        *reinterpret_cast<bf16x2*>(q_row + high_dim) = high;
+                        continue;
+                    }
+                    if (!store.slot_mapping) continue;
+                    const int slot = store.slot_mapping[row];
+                    if (slot < 0) continue;
+                    const int page = slot / store.page_size, offset = slot % store.page_size;
+                    if (!is_value) {
+                        bf16* pages = static_cast<bf16*>(store.k_cache);        // two neighbouring dims are neighbours in a page of keys
+                        *reinterpret_cast<bf16x2*>(pages + layout.k_at(page, head - store.heads, offset, low_dim)) = low;
+                        *reinterpret_cast<bf16x2*>(pages + layout.k_at(page, head - store.heads, offset, high_dim)) = high;
+                    } else {
+                        bf16* pages = static_cast<bf16*>(store.v_cache);        // and 8 elements apart in a page of values
+                        const int kv_head = head - store.heads - store.kv_heads;
+#pragma unroll
+                        for (int i = 0; i < 4; ++i) pages[layout.v_at(page, kv_head, offset, within + i)] = from_float<bf16>(y[i]);
+                    }
                 }
             }
+            continue;
         }
-        return;
-    }
+        auto gated = [&](float gate, float up) {
+            return EPILOGUE == 7 ? gated_value_fast(gate, up, kActClampedGlu, limit, slope) : gate_fast<EPILOGUE == 5>(gate) * up;
+        };
+        if constexpr (EPILOGUE == 2 || EPILOGUE == 5 || EPILOGUE == 7) {
+            if (whole_rows) {
+                workgroup_meets();
 #pragma unroll
-    for (int mt = 0; mt < WM; ++mt) {
-        const int row = m0 + wave_m * (WM * 16) + mt * 16 + col;
-        if (row >= m) continue;
+                for (int mt = 0; mt < WM; ++mt)
 #pragma unroll
-        for (int nt = 0; nt < kWaveTilesN; ++nt) {
-            const int column = (n_tile0 + wave_n * kWaveTilesN + nt) * 16 + quad * 4;
-            if (EPILOGUE == 0) {
-                float* target = static_cast<float*>(out) + (static_cast<int64_t>(blockIdx.y) * m + row) * n + column;
-                if (column + 3 < n && n % 4 == 0) {
-                    *reinterpret_cast<floatx4*>(target) = acc[nt][mt];
+                    for (int nt = 0; nt < kWaveTilesN; ++nt) {
+                        bf16x2 two;
+#pragma unroll
+                        for (int i = 0; i < 2; ++i) two[i] = static_cast<__bf16>(gated(acc[nt][mt][2 * i], acc[nt][mt][2 * i + 1]));
+                        *reinterpret_cast<bf16x2*>(reinterpret_cast<char*>(slots) + (wave_m * (WM * 16) + mt * 16 + col) * kResultStride +
+                                                   wave_n * 64 + nt * 16 + quad * 4) = two;
+                    }
+                workgroup_meets();
+                store_result_rows(slots, static_cast<bf16*>(out) + static_cast<int64_t>(m0) * (n / 2) + n_block * kResultColumns, min(TILE_M, m - m0), n / 2,
+                                  n / 2 - n_block * kResultColumns);
+                continue;
+            }
+        }
+#pragma unroll
+        for (int mt = 0; mt < WM; ++mt) {
+            const int row = m0 + wave_m * (WM * 16) + mt * 16 + col;
+            if (row >= m) continue;
+#pragma unroll
+            for (int nt = 0; nt < kWaveTilesN; ++nt) {
+                const int column = (n_tile0 + wave_n * kWaveTilesN + nt) * 16 + quad * 4;
+                if (EPILOGUE == 0) {
+                    float* target = static_cast<float*>(out) + (static_cast<int64_t>(blockIdx.y) * m + row) * n + column;
+                    if (column + 3 < n && n % 4 == 0) {
+                        *reinterpret_cast<floatx4*>(target) = acc[nt][mt];
+                    } else {
+#pragma unroll
+                        for (int i = 0; i < 4; ++i)
+                            if (column + i < n) target[i] = acc[nt][mt][i];
+                    }
+                } else if (EPILOGUE == 1) {
+                    bf16* target = static_cast<bf16*>(out) + static_cast<int64_t>(row) * n + column;
+                    if (column + 3 < n && n % 4 == 0) {
+                        bf16x4 four;
+#pragma unroll
+                        for (int i = 0; i < 4; ++i) four[i] = static_cast<__bf16>(acc[nt][mt][i]);
+                        *reinterpret_cast<bf16x4*>(target) = four;
+                    } else {
+#pragma unroll
+                        for (int i = 0; i < 4; ++i)
+                            if (column + i < n) target[i] = from_float<bf16>(acc[nt][mt][i]);
+                    }
                 } else {
+                    bf16* target = static_cast<bf16*>(out) + static_cast<int64_t>(row) * (n / 2) + column / 2;
+                    if (column + 3 < n && n % 4 == 0) {
+                        bf16x2 two;
 #pragma unroll
-                    for (int i = 0; i < 4; ++i)
-                        if (column + i < n) target[i] = acc[nt][mt][i];
-                }
-            } else if (EPILOGUE == 1) {
-                bf16* target = static_cast<bf16*>(out) + static_cast<int64_t>(row) * n + column;
-                if (column + 3 < n && n % 4 == 0) {
-                    bf16x4 four;
+                        for (int i = 0; i < 2; ++i) two[i] = static_cast<__bf16>(gated(acc[nt][mt][2 * i], acc[nt][mt][2 * i + 1]));
+                        *reinterpret_cast<bf16x2*>(target) = two;
+                    } else {
 #pragma unroll
-                    for (int i = 0; i < 4; ++i) four[i] = static_cast<__bf16>(acc[nt][mt][i]);
-                    *reinterpret_cast<bf16x4*>(target) = four;
-                } else {
-#pragma unroll
-                    for (int i = 0; i < 4; ++i)
-                        if (column + i < n) target[i] = from_float<bf16>(acc[nt][mt][i]);
-                }
-            } else {
-                auto gated = [&](float gate, float up) {
-                    return EPILOGUE == 7 ? gated_value_fast(gate, up, kActClampedGlu, limit, slope) : gate_fast<EPILOGUE == 5>(gate) * up;
-                };
-                bf16* target = static_cast<bf16*>(out) + static_cast<int64_t>(row) * (n / 2) + column / 2;
-                if (column + 3 < n && n % 4 == 0) {
-                    bf16x2 two;
-#pragma unroll
-                    for (int i = 0; i < 2; ++i) two[i] = static_cast<__bf16>(gated(acc[nt][mt][2 * i], acc[nt][mt][2 * i + 1]));
-                    *reinterpret_cast<bf16x2*>(target) = two;
-                } else {
-#pragma unroll
-                    for (int i = 0; i < 4; i += 2)
-                        if (column + i < n) target[i / 2] = from_float<bf16>(gated(acc[nt][mt][i], acc[nt][mt][i + 1]));
+                        for (int i = 0; i < 4; i += 2)
+                            if (column + i < n) target[i / 2] = from_float<bf16>(gated(acc[nt][mt][i], acc[nt][mt][i + 1]));
+                    }
                 }
             }
         }
@@ -307,9 +286,12 @@ static int launch_tiled_rows(const void* a, const void* w_packed, void* out, int
                              const MllQkvStore& store, float limit, float slope) {
     const int n_tiles = (n + 15) / 16, k_steps = k / 32;
     const int m_blocks = (m + 32 * WM - 1) / (32 * WM), n_blocks = (n + kTileN - 1) / kTileN;
-    const dim3 grid(8 * ((m_blocks * n_blocks + 7) / 8), splits);
+    // As many workgroups as run at once go from tile to tile; parts of the reduction are workgroups of their own.
+    const int all = 8 * ((m_blocks * n_blocks + 7) / 8);
+    const dim3 grid(splits > 1 ? all : min(all, 256), splits);
+    const int whole_rows = n % 16 == 0 && reinterpret_cast<uintptr_t>(out) % 16 == 0;      // of a gated result: pieces of 16 bytes
     gemm_tiled_kernel<EPILOGUE, WM><<<grid, kTiledThreads, 0, stream>>>(static_cast<const bf16*>(a), static_cast<const bf16*>(w_packed),
-                                                                        out, m, n, k, n_tiles, k_steps, m_blocks, n_blocks, store, limit, slope);
+                                                                        out, m, n, k, n_tiles, k_steps, m_blocks, n_blocks, whole_rows, store, limit, slope);
     return check_launch("gemm_tiled");
 }
 

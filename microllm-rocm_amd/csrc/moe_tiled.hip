@@ -127,19 +127,17 @@ __device__ __attribute__((always_inline)) inline void tile_products(bf16* slots,
     }
     const char* a_bytes = reinterpret_cast<const char*>(a);
     const char* w_bytes = reinterpret_cast<const char*>(w_expert);
-    auto copy_stage = [&](int stage, int slot) __attribute__((always_inline)) {
-        bf16* a_place = slots + slot * kSlotElements;
-        bf16* w_place = a_place + kWBytes / 2;
-#pragma unroll
-        for (int t = 0; t < A_TURNS; ++t)
-            __builtin_amdgcn_global_load_lds(a_bytes + stage * 128 + a_from[t], a_place + wave * 512 + t * (kTiledWaves * 512), 16, 0, 0);
-#pragma unroll
-        for (int t = 0; t < W_TURNS; ++t)
-            __builtin_amdgcn_global_load_lds(w_bytes + stage * 128 + w_from[t], w_place + wave * 512 + t * (kTiledWaves * 512), 16, 0, 0);
+    auto copy_a = [&](int turn, int stage, unsigned slot) __attribute__((always_inline)) {
+        bf16* place = slots + slot * kSlotElements + wave * 512;
+        __builtin_amdgcn_global_load_lds(a_bytes + stage * 128 + a_from[turn], place + turn * (kTiledWaves * 512), 16, 0, 0);
+    };
+    auto copy_w = [&](int turn, int stage, unsigned slot) __attribute__((always_inline)) {
+        bf16* place = slots + (kASlots + slot) * kSlotElements + wave * 512;
+        __builtin_amdgcn_global_load_lds(w_bytes + stage * 128 + w_from[turn], place + turn * (kTiledWaves * 512), 16, 0, 0);
     };
     const unsigned base = lds_address(slots);
     const unsigned step0 = col * 128 + ((quad ^ (col / 2)) * 16), step1 = col * 128 + (((4 + quad) ^ (col / 2)) * 16);
-    const unsigned a_at = base + wave_m * WM * 2048, w_at = base + wave_n * kWaveTilesN * 2048;
+    const unsigned a_at = base + wave_m * WM * 2048, w_at = base + kASlots * kSlotBytes + wave_n * kWaveTilesN * 2048;
 
     floatx4 acc[kWaveTilesN][WM];     // acc[nt][mt][i] = C[pair mt*16 + col][weight row nt*16 + quad*4 + i] of the wave's part
 #pragma unroll
@@ -147,33 +145,25 @@ __device__ __attribute__((always_inline)) inline void tile_products(bf16* slots,
 #pragma unroll
         for (int mt = 0; mt < WM; ++mt) acc[nt][mt] = floatx4{0.0f, 0.0f, 0.0f, 0.0f};
 
-    const int stages = k / 64;        // an even number: a way out between the two of a round would make the compiler keep the accumulators twice
-    TiledOperands<WM> even, odd;      // of a stage's first and second k step
-    copy_stage(0, 0);
-    copy_stage(1, 1);
-    asm volatile("s_waitcnt vmcnt(%0)" :: "n"(A_TURNS + W_TURNS) : "memory");      // this wave's loads of the first stage have landed
-    __builtin_amdgcn_s_barrier();
-    read_operands<0, WM, 0>(even, a_at + step0, w_at + step0, std::make_integer_sequence<int, 4 + WM>{});
-    // A stage in slot SLOT: its first step is multiplied while its second is read; then the next stage has landed (the wave's loads before
-    // the barrier, everyone's after it) and this one has been read by all, so that its slot may take the stage after next. After
-    // the last stage nothing is copied, and what is read then is multiplied by nobody.
-#define MLL_MOE_STAGE(STAGE, SLOT)                                                                                                                     \
-    operands_arrived<false>(even);                                                                                                                     \
-    products<0, WM, 1>(acc, even, odd, a_at + step1 + SLOT * kSlotBytes, w_at + step1 + SLOT * kSlotBytes, std::make_integer_sequence<int, WM>{});      \
-    operands_arrived<true>(odd);                                                                                                                       \
-    __builtin_amdgcn_s_barrier();                                                                                                                      \
-    if (STAGE + 2 < stages) copy_stage(STAGE + 2, SLOT);                                                                                               \
-    products<0, WM, 0>(acc, odd, even, a_at + step0 + (1 - SLOT) * kSlotBytes, w_at + step0 + (1 - SLOT) * kSlotBytes, std::make_integer_sequence<int, WM>{});
-    for (int stage = 0; stage < stages; stage += 2) {
-        MLL_MOE_STAGE(stage, 0)
-        MLL_MOE_STAGE(stage + 1, 1)
-    }
-#undef MLL_MOE_STAGE
-    // No read may be on its way into registers that something else takes, and the last products must have written their results before these are
-    // read (the compiler does not know that the asm statements are products).
-    operands_arrived<true>(even);
-    asm volatile("s_nop 15\n\ts_nop 15" ::: "memory");
+    multiply_stages<0, WM, A_TURNS>(acc, 0, k / 64, A_TURNS, a_at + step0, a_at + step1, w_at + step0, w_at + step1, copy_a, copy_w);
 
+    if constexpr (GATED) {
+        workgroup_meets();
+#pragma unroll
+        for (int mt = 0; mt < WM; ++mt)
+#pragma unroll
+            for (int nt = 0; nt < kWaveTilesN / 2; ++nt) {
+                bf16x4 four;
+#pragma unroll
+                for (int i = 0; i < 4; ++i)
+                    four[i] = static_cast<__bf16>(gated_value_fast(acc[nt][mt][i], acc[nt + 2][mt][i], form.activation, form.limit, form.slope));
+                *reinterpret_cast<bf16x4*>(reinterpret_cast<char*>(slots) + (wave_m * (WM * 16) + mt * 16 + col) * kResultStride + wave_n * 64 +
+                                           nt * 32 + quad * 8) = four;
+            }
+        workgroup_meets();
+        store_result_rows(slots, static_cast<bf16*>(out) + static_cast<int64_t>(tile.first_row) * n_out + column0, tile.rows, n_out, n_out - column0);
+        return;
+    }
 #pragma unroll
     for (int mt = 0; mt < WM; ++mt) {
         const int row = wave_m * (WM * 16) + mt * 16 + col;
@@ -191,13 +181,12 @@ __device__ __attribute__((always_inline)) inline void tile_products(bf16* slots,
         } else {
             bf16* to = static_cast<bf16*>(out) + static_cast<int64_t>(sorted) * n_out;
 #pragma unroll
-            for (int nt = 0; nt < (GATED ? kWaveTilesN / 2 : kWaveTilesN); ++nt) {
-                const int column = column0 + wave_n * (GATED ? 32 : 64) + nt * 16 + quad * 4;
+            for (int nt = 0; nt < kWaveTilesN; ++nt) {
+                const int column = column0 + wave_n * 64 + nt * 16 + quad * 4;
                 bf16x4 four;
 #pragma unroll
                 for (int i = 0; i < 4; ++i)
-                    four[i] = static_cast<__bf16>(GATED ? gated_value_fast(acc[nt][mt][i], acc[GATED ? nt + 2 : nt][mt][i], form.activation, form.limit, form.slope)
-                                                        : activate(acc[nt][mt][i], form.activation));
+                    four[i] = static_cast<__bf16>(activate(acc[nt][mt][i], form.activation));
                 if (column < n_out) *reinterpret_cast<bf16x4*>(to + column) = four;
             }
         }
@@ -212,7 +201,7 @@ __global__ __launch_bounds__(kTiledThreads, 1) void moe_tiled_kernel(const bf16*
                                                                      const float* __restrict__ weights, int n_out, int k, void* __restrict__ out,
                                                                      int top, int n_tokens, int weight_on_input, int from_tokens,
                                                                      const bf16* __restrict__ x, MllExpertForm form) {
-    __shared__ __align__(16) bf16 slots[2 * kSlotElements];
+    __shared__ __align__(16) bf16 slots[kStageElements];
     constexpr int kOutputsATile = FORM == 1 ? kTileCols / 2 : kTileCols;
     const int lane = threadIdx.x % kWave;
     const int n_blocks = (n_out + kOutputsATile - 1) / kOutputsATile;
@@ -223,7 +212,7 @@ __global__ __launch_bounds__(kTiledThreads, 1) void moe_tiled_kernel(const bf16*
         const int place = blockIdx.x % 8 * per_xcd + index;
         if (place >= all) break;        // the same for every thread of the workgroup
         const TileOfExpert tile = tile_at(place, offsets, form.experts, n_blocks, tiling.height, lane);
-        __builtin_amdgcn_s_barrier();       // every wave has read the last tile's stages
+        workgroup_meets();      // every wave is done with the slots of the tile before
         if (tile.rows > 192) tile_products<FORM, 8>(slots, tile, a, w, order, weights, n_out, k, out, top, n_tokens, weight_on_input, from_tokens, form);
         else if (tile.rows > 128) tile_products<FORM, 6>(slots, tile, a, w, order, weights, n_out, k, out, top, n_tokens, weight_on_input, from_tokens, form);
         else if (tile.rows > 0) tile_products<FORM, 4>(slots, tile, a, w, order, weights, n_out, k, out, top, n_tokens, weight_on_input, from_tokens, form);

@@ -1,8 +1,9 @@
 // What the products of large tiles (gemm_tiled.hip, moe_tiled.hip) share: the operands of a k step in registers, read from a stage in
-// LDS between the products of the step before. A stage of 64 of k lies in a slot: up to 256 rows of A in pieces of 16 rows (2 KB), then 256
+// LDS between the products of the step before. A stage of 64 of k lies in slots: up to 256 rows of A in pieces of 16 rows (2 KB), 256
 // rows of W in tiles of 16 (2 KB). Rows of 128 bytes have their eight 16-byte chunks at places exchanged by (row / 2).
 #pragma once
 
+#include <type_traits>
 #include <utility>
 
 #include "common.h"
@@ -18,9 +19,12 @@ constexpr int kMaxWaveTilesM = 8;                         // a wave's part of C 
 constexpr int kTiledWaves = 8;
 constexpr int kTiledThreads = kTiledWaves * kWave;
 constexpr int kWaveTilesN = 4;                            // a wave's 64 columns of C
-constexpr int kSlotBytes = 65536;                         // a stage of 64 of k: up to 32 KB of A, then 32 KB of W
+// A stage of 64 of k: two slots for up to 256 rows of A, then three for 256 rows of W, 32 KB each. W has one more, so that its loads may be on
+// their way while the workgroup has not met since the slot before them was read.
+constexpr int kSlotBytes = 32768;
 constexpr int kSlotElements = kSlotBytes / 2;
-constexpr int kWBytes = 32768;                            // where W begins in a slot
+constexpr int kASlots = 2, kWSlots = 3;
+constexpr int kStageElements = (kASlots + kWSlots) * kSlotElements;
 
 __device__ inline unsigned lds_address(bf16* place) { return static_cast<unsigned>(reinterpret_cast<uintptr_t>((lds_bf16*)place)); }
 
@@ -37,7 +41,7 @@ struct TiledOperands {       // of one k step: the wave's WM pieces of A and 4 o
 // too, with the tile's second step W_STEP bytes after its first (0: the caller's address says which step). An INDEX beyond the reads is nothing.
 template <int W_STEP, int WM, int INDEX, int STEP>
 __device__ __attribute__((always_inline)) inline void read_operand(TiledOperands<WM>& f, unsigned a_address, unsigned w_address) {
-    constexpr int W = kWBytes + STEP * W_STEP;
+    constexpr int W = STEP * W_STEP;
     if constexpr (INDEX == 0) MLL_DS_READ(f.w[0], w_address, W);
     if constexpr (INDEX == 1) MLL_DS_READ(f.w[1], w_address, W + 2048);
     if constexpr (INDEX == 2) MLL_DS_READ(f.a[0], a_address, 0);
@@ -52,39 +56,125 @@ __device__ __attribute__((always_inline)) inline void read_operands(TiledOperand
     (read_operand<W_STEP, WM, INDEX, STEP>(f, a_address, w_address), ...);
 }
 
-// The four products of row tile MT of a k step, and after every second of them a read of the next step's operands
-// (the first 4 + WM of the 2 WM places take one).
-template <int W_STEP, int WM, int NEXT_STEP, int MT>
+// The four products of row tile MT of a k step, and after every second of them a read of the next step's operands (the first 4 + WM of the
+// 2 WM places take one) and what `between` does at that place: one load of a later stage here and there, so that the loads, which a compute
+// unit takes one in 16 cycles, are not asked for in one go while no product is formed.
+template <int W_STEP, int WM, int NEXT_STEP, int MT, typename Between>
 __device__ __attribute__((always_inline)) inline void products_of_row_tile(floatx4 (&acc)[kWaveTilesN][WM], const TiledOperands<WM>& now,
-                                                                           TiledOperands<WM>& next, unsigned a_address, unsigned w_address) {
+                                                                           TiledOperands<WM>& next, unsigned a_address, unsigned w_address,
+                                                                           const Between& between) {
     MLL_MFMA(acc[0][MT], now.w[0], now.a[MT]);
     MLL_MFMA(acc[1][MT], now.w[1], now.a[MT]);
     read_operand<W_STEP, WM, 2 * MT, NEXT_STEP>(next, a_address, w_address);
+    between(std::integral_constant<int, 2 * MT>{});
     MLL_MFMA(acc[2][MT], now.w[2], now.a[MT]);
     MLL_MFMA(acc[3][MT], now.w[3], now.a[MT]);
     read_operand<W_STEP, WM, 2 * MT + 1, NEXT_STEP>(next, a_address, w_address);
+    between(std::integral_constant<int, 2 * MT + 1>{});
 }
-template <int W_STEP, int WM, int NEXT_STEP, int... MT>
+template <int W_STEP, int WM, int NEXT_STEP, typename Between, int... MT>
 __device__ __attribute__((always_inline)) inline void products(floatx4 (&acc)[kWaveTilesN][WM], const TiledOperands<WM>& now,
                                                                TiledOperands<WM>& next, unsigned a_address, unsigned w_address,
-                                                               std::integer_sequence<int, MT...>) {
-    (products_of_row_tile<W_STEP, WM, NEXT_STEP, MT>(acc, now, next, a_address, w_address), ...);
+                                                               const Between& between, std::integer_sequence<int, MT...>) {
+    (products_of_row_tile<W_STEP, WM, NEXT_STEP, MT>(acc, now, next, a_address, w_address, between), ...);
 }
 
-// The reads into `f` have arrived (and, LOADS, the wave's loads into LDS have landed). `f` passes through the
+// The reads into `f` have arrived (and, LOADS >= 0, of the wave's loads into LDS all but the last LOADS have landed). `f` passes through the
 // statements, so that nothing that uses it is placed before.
-template <bool LOADS, int WM>
+template <int LOADS, int WM>
 __device__ __attribute__((always_inline)) inline void operands_arrived(TiledOperands<WM>& f) {
-    if constexpr (LOADS)
-        asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)"
+    if constexpr (LOADS >= 0)
+        asm volatile("s_waitcnt vmcnt(%8) lgkmcnt(0)"
                      : "+v"(f.a[0]), "+v"(f.a[1]), "+v"(f.a[2]), "+v"(f.a[3]), "+v"(f.w[0]), "+v"(f.w[1]), "+v"(f.w[2]), "+v"(f.w[3])
-                     :: "memory");
+                     : "n"(LOADS) : "memory");
     else
         asm volatile("s_waitcnt lgkmcnt(0)"
                      : "+v"(f.a[0]), "+v"(f.a[1]), "+v"(f.a[2]), "+v"(f.a[3]), "+v"(f.w[0]), "+v"(f.w[1]), "+v"(f.w[2]), "+v"(f.w[3])
                      :: "memory");
 #pragma unroll
     for (int i = 4; i < WM; ++i) asm volatile("" : "+v"(f.a[i]));
+}
+
+// The stages of a tile, from `first` to before `stages`, one at least. copy_a(turn, stage, slot) and copy_w(turn, stage, slot) issue one of a wave's
+// A_TURNS (a_loads of this wave: all or all but one) and four loads of a stage. While a stage's first step is multiplied its second is read, and W's loads of the stage after next go out, into the slot
+// that was read a stage ago; then the next stage has landed (the wave's loads before the barrier, everyone's after it) and this one has been read
+// by all: A's loads of the stage after next go out while the second step is multiplied and the next stage's first is read. After the last
+// stage nothing is copied, and what is read then is multiplied by nobody.
+template <int W_STEP, int WM, int A_TURNS, typename CopyA, typename CopyW>
+__device__ __attribute__((always_inline)) inline void multiply_stages(floatx4 (&acc)[kWaveTilesN][WM], int first, int stages, int a_loads, unsigned a_step0,
+                                                                      unsigned a_step1, unsigned w_step0, unsigned w_step1, const CopyA& copy_a,
+                                                                      const CopyW& copy_w) {
+    constexpr std::make_integer_sequence<int, WM> row_tiles{};
+    TiledOperands<WM> even, odd;      // of a stage's first and second k step
+    const bool second = first + 1 < stages;
+#pragma unroll
+    for (int t = 0; t < A_TURNS; ++t)
+        if (t < a_loads) copy_a(t, first, 0);
+#pragma unroll
+    for (int t = 0; t < 4; ++t) copy_w(t, first, 0);
+    if (second) {
+#pragma unroll
+        for (int t = 0; t < A_TURNS; ++t)
+            if (t < a_loads) copy_a(t, first + 1, 1);
+#pragma unroll
+        for (int t = 0; t < 4; ++t) copy_w(t, first + 1, 1);
+        // the first stage's loads of this wave have landed when only the second stage's are on their way
+        if (a_loads == A_TURNS) asm volatile("s_waitcnt vmcnt(%0)" :: "n"(A_TURNS + 4) : "memory");
+        else asm volatile("s_waitcnt vmcnt(%0)" :: "n"(A_TURNS + 3) : "memory");
+    } else {
+        asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+    }
+    __builtin_amdgcn_s_barrier();
+    read_operands<W_STEP, WM, 0>(even, a_step0, w_step0, std::make_integer_sequence<int, 4 + WM>{});
+    operands_arrived<-1>(even);
+    unsigned a_now = 0, w_now = 0, w_next = 1, w_after = 2;        // slots
+    // MORE: there is a stage after next. Operands on their way never pass from one block to another (the compiler may copy a value there, and does
+    // not know that it has not arrived): no branch stands in a stage, and a stage ends when the next one's first operands have arrived.
+    auto multiply_stage = [&](int stage, auto more) __attribute__((always_inline)) {
+        constexpr bool MORE = decltype(more)::value;
+        products<W_STEP, WM, 1>(acc, even, odd, a_step1 + a_now * kSlotBytes, w_step1 + w_now * kSlotBytes, [&](auto place) __attribute__((always_inline)) {
+            constexpr int kPlace = decltype(place)::value, kApart = 2 * WM / 4;
+            if constexpr (MORE && kPlace % kApart == 0 && kPlace / kApart < 4) copy_w(kPlace / kApart, stage + 2, w_after);
+        }, row_tiles);
+        operands_arrived<MORE ? 4 : 0>(odd);
+        __builtin_amdgcn_s_barrier();
+        products<W_STEP, WM, 0>(acc, odd, even, a_step0 + (1 - a_now) * kSlotBytes, w_step0 + w_next * kSlotBytes, [&](auto place) __attribute__((always_inline)) {
+            constexpr int kPlace = decltype(place)::value;
+            if constexpr (MORE && kPlace % 2 == 0 && kPlace / 2 < A_TURNS) {
+                if (kPlace / 2 < a_loads) copy_a(kPlace / 2, stage + 2, a_now);
+            }
+        }, row_tiles);
+        operands_arrived<-1>(even);
+        a_now = 1 - a_now;
+        const unsigned w = w_now;
+        w_now = w_next, w_next = w_after, w_after = w;
+    };
+    int stage = first;
+    for (; stage + 2 < stages; ++stage) multiply_stage(stage, std::true_type{});
+    for (; stage < stages; ++stage) multiply_stage(stage, std::false_type{});
+    // No load is on its way into LDS now and no read into registers; the last products must have written their results before these are read (the
+    // compiler does not know that the asm statements are products).
+    asm volatile("s_nop 15\n\ts_nop 15" ::: "memory");
+}
+
+// Every wave's reads and writes of the slots before this are done: the slots may hold something else after it.
+__device__ __attribute__((always_inline)) inline void workgroup_meets() {
+    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+    __builtin_amdgcn_s_barrier();
+    asm volatile("" ::: "memory");
+}
+
+// A tile's results of 128 columns in bfloat16 go through the slots, so that they leave as whole rows of 256 bytes: a lane has 4 or 8 bytes of a
+// row, which would touch every line of memory 8 to 32 times (9728 columns of 1280 rows, reduction 896: 34 -> 30 us). Rows in LDS are 272 bytes apart, so that 16
+// rows' words meet no bank twice.
+constexpr int kResultStride = 272, kResultColumns = 128;
+__device__ __attribute__((always_inline)) inline void store_result_rows(const bf16* slots, bf16* __restrict__ out, int rows, int row_elements, int columns) {
+    for (int piece = threadIdx.x; piece < rows * (kResultColumns / 8); piece += kTiledThreads) {
+        const int row = piece / (kResultColumns / 8), column = piece % (kResultColumns / 8) * 8;
+        if (column < columns)
+            *reinterpret_cast<uintx4*>(out + static_cast<int64_t>(row) * row_elements + column) =
+                *reinterpret_cast<const uintx4*>(reinterpret_cast<const char*>(slots) + row * kResultStride + column * 2);
+    }
 }
 
 }  // namespace mll

@@ -1215,10 +1215,12 @@ def tiled_gated_pays(rows: int, k: int, from_float: bool = False, n: int = TILED
     k up to 1024 from ``rows * n`` of 3700 k on: 512 x 512 at 1024, 3072 and 4096 rows 0.78, 0.99 and 1.07; 2816 x 1024 at 512, 1024, 1536 and 4096
     0.76, 0.91, 1.06 and 1.51; 9728 x 896 at 192, 512, 2048 and 4096 0.91, 1.24, 1.39 and 1.21. Up to 2048 from 3000 k on: 1408 x 2048 at 1024
     and 3072 0.61 and 0.91; 4096 x 2048 at 1024, 1536 and 2048 0.86, 1.02 and 1.13; 16384 x 2048 at 256, 512, 1024, 2048, 3072 and 4096 0.95,
-    1.10, 1.12, 1.01, 0.96 and 0.96. Longer reductions: the library's rate jumps with the shape, this one's only where the last round of
+    1.10, 1.12, 1.01, 0.96 and 0.96 (at 3072, 4096, 8192 and 16384 with the loads between the products 1.10, 1.13, 1.11 and 1.11). Longer reductions: the library's rate jumps with the shape, this one's only where the last round of
     workgroups leaves units idle; from 3584 to 6144 where they are nine tenths filled: 37888 x 3584 at 1280, 1536 (0.87 filled), 2048 and 3072
     1.32, 0.92, 1.15 and 1.10; 22016 x 4096 at 1024 (0.67), 1536, 2048 and 2560 (0.84) 0.85, 1.35, 1.48 and 0.94; but 17920 x 2560 at 1536, 2560, 3072
-    and 3584 0.92, 1.39, 0.85 and 0.92, 59136 x 8192 at 1024 to 4096 0.88 to 0.99, 8192 x 8192 0.85 to 0.99.
+    and 3584 0.92, 1.39, 0.85 and 0.92, 59136 x 8192 at 1024 to 4096 0.88 to 0.99, 8192 x 8192 0.85 to 0.99. Above 3072 rows timed alone the
+    tiled kernel is faster there by now (37888 x 3584 at 4096, 8192 and 16384 1.07, 1.12 and 1.05), but a pass of 16301 tokens runs at the power cap
+    and takes 75.4 ms with it and 74.0 with the library. 9728 x 896 at 4096, 8192 and 16384 1.47, 1.48 and 1.44.
 
     Where the activation takes the float32 sums (``from_float``: clamped gates), the library's way writes and reads twice as much and has no
     upper line: 16384 x 2048 at 256, 512, 3584 and 8192 rows 0.97, 1.15, 1.22 and 1.30; 4096 x 2048 at 1024, 1536 and 8192 0.90, 1.05 and 1.18; 37888 x 3584
@@ -1236,15 +1238,15 @@ def tiled_gated_pays(rows: int, k: int, from_float: bool = False, n: int = TILED
     if from_float:
         return work >= 3500 * k if k <= 1024 else work >= 2800 * k if k <= 2048 else rows > 960 and work >= 1650 * k
     if k <= 1024:
-        return rows <= 4096 and work >= 3700 * k
+        return work >= 3700 * k
     if k <= 2048:
-        return rows <= 3072 and work >= 3000 * k
+        return work >= 3000 * k
     return 3584 <= k <= 6144 and 960 < rows <= 3072 and _tiled_fill_of(rows, n) >= 0.9
 
 
 def gemm_tiled(x: torch.Tensor, packed: torch.Tensor, n: int, epilogue: str = "f32", splits: int = 1,
                tile_rows: int = 0, limit: float = 0.0, slope: float = 0.0) -> torch.Tensor:
-    """``x @ W.T`` for many bfloat16 rows and a packed weight, on this package's tiled MFMA kernel (0.9 to 1.1 of
+    """``x @ W.T`` for many bfloat16 rows and a packed weight, on this package's tiled MFMA kernel (0.85 to 1.1 of
     the library's untuned rate at 2048 rows and more, 1.1 to 1.4 PFLOP/s: for weights that are kept in the packed
     order alone, and for gated products where ``tiled_gated_pays``). ``k`` must be
     a multiple of 32. With ``splits`` > 1 (float32 only) the result is ``[splits, m, n]`` sums over parts of the

@@ -31,3 +31,9 @@ def test_where_the_tiled_kernel_takes_gated_products(rows, n, k, pays, clamped):
     """Weights of few rows and of long reductions stay with the library where that is faster."""
     assert kernels.tiled_gated_pays(rows, k, False, n) == pays
     assert kernels.tiled_gated_pays(rows, k, True, n) == clamped
+
+
+@pytest.mark.parametrize("rows,n,k,pays", [(4096, 9728, 896, True), (16384, 9728, 896, True), (4096, 16384, 2048, True), (3200, 37888, 3584, False),
+                                           (16301, 37888, 3584, False), (4096, 17920, 2560, False), (4096, 1408, 4096, False), (8192, 59136, 8192, False)])
+def test_many_rows_of_gated_products(rows, n, k, pays):
+    assert kernels.tiled_gated_pays(rows, k, False, n) == pays
