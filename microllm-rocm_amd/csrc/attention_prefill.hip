@@ -152,7 +152,7 @@ __global__ __launch_bounds__(kPrefillThreads, 1) void paged_attention_prefill_ke
     const int count = entry[2 + 2 * side];
     const int first_token = entry[1 + 2 * side];
     const int tile_position = tile_positions[side];
-    const int block_first = 32 * (wave % 4);                              // in the tile
+    const int block_first = 32 * (side == 0 ? wave % 4 : 3 - wave % 4);   // in the tile; tiles of 64 tokens then have a wave on every SIMD
     const int block_valid = min(32, max(0, count - block_first));
     const int block_position = tile_position + block_first;
     const int block_last = block_position + block_valid - 1;

@@ -144,7 +144,7 @@ class BucketBiasAttention(Mixer):
                       and self.stored_dim <= 256 and 0 < table_rows <= kernels.MFMA_BIAS_ROWS)
         # the width of a head's result as the kernels leave it
         self.result_dim = self.stored_dim if self.tiled else self.value_dim
-        self.planner = QueryTilePlanner(bool(self.window or self.chunk)) if self.tiled else None
+        self.planner = QueryTilePlanner(bool(self.window or self.chunk), self.heads) if self.tiled else None
         self.slopes = self.o_bias = self.qkv_bias = self.conv = None
         self.qkv_weight: Optional[Weight] = None
         self.o_tensor: Optional[torch.Tensor] = None

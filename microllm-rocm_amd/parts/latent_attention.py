@@ -65,7 +65,7 @@ class LatentAttention(Mixer):
             raise ValueError("the rotated part turns whole, by the split-half rule")
         self.row = self.kv_rank + self.rot_dim
         self.tiled = bool(p.get("mfma", True)) and runtime.dtype == torch.bfloat16 and self.row % 16 == 0 and self.row <= 256
-        self.planner = QueryTilePlanner(bool(self.window)) if self.tiled else None
+        self.planner = QueryTilePlanner(bool(self.window), self.heads) if self.tiled else None
         self.q_width = self.heads * (self.dim + self.rot_dim)
         self.gate_width = (self.heads if self.gate_a_head else self.heads * self.vdim) if self.output_gate else 0
         self.q_at = 0

@@ -192,3 +192,13 @@ def test_kept_graphs_stay_bounded_and_mixed_shapes_never_push_decode_graphs_out(
 def test_decode_parts(tokens, kv_heads, longest, head_dim, splits):
     assert kernels.decode_parts(tokens, kv_heads, longest, head_dim) == splits
     assert splits >= kernels.decode_splits(tokens, kv_heads, longest)
+
+
+def test_tiles_of_half_the_queries_where_whole_ones_leave_compute_units_idle():
+    from microllm_rocm_amd.parts.attention import QueryTilePlanner
+    assert QueryTilePlanner(False).tile_rows([512]) == 128
+    planner = QueryTilePlanner(False, 14)
+    assert planner.tile_rows([]) == 128
+    assert [planner.tile_rows([count]) for count in (2, 128, 2048, 2304, 2305)] == [64, 64, 64, 64, 128]      # 9 pairs of tiles of 14 heads: 126
+    assert planner.tile_rows([512, 512, 600]) == 64 and planner.tile_rows([300] * 5) == 128
+    assert planner.key != QueryTilePlanner(False, 28).key

@@ -373,3 +373,20 @@ def test_experts_in_large_tiles(n, width, ff, experts, top, identity, gated):
         if experts * (-(-ff // 128)) < 512:
             small = k.moe_experts(x[:few], ids[:few].contiguous(), weights[:few].contiguous(), gate_up, down, on_input, grouped=True, **options)
             assert torch.equal(small, tiled[:, :few])
+
+
+@pytest.mark.parametrize("heads,kv_heads,hd,window", [(14, 2, 64, 0), (4, 2, 48, 100), (4, 1, 128, 0), (2, 1, 256, 33)])
+def test_prompts_in_tiles_of_half_the_queries_have_the_same_bits(heads, kv_heads, hd, window):
+    """Tiles of 64 queries, whose second one in a workgroup goes to the waves from the last on, against tiles of 128."""
+    rng, k = np.random.default_rng(hd + window), kernels()
+    lengths, counts = [517, 300, 97, 64, 131, 33], [130, 300, 65, 64, 128, 1]
+    t, *_ = build_paged_case(rng, torch.bfloat16, lengths, counts, heads, kv_heads, hd, 16)
+    results = []
+    for rows in (128, 64):
+        tiles, start = [], 0
+        for index, (length, count) in enumerate(zip(lengths, counts)):
+            tiles += [(index, start + offset, min(rows, count - offset), length - count + offset) for offset in range(0, count, rows)]
+            start += count
+        pairs = torch.tensor(k.pair_query_tiles(tiles, adjacent=window > 0), dtype=torch.int32, device=DEVICE)
+        results.append(k.paged_attention_prefill(t["q"], t["k"], t["v"], t["table"], pairs, t["pos"], hd ** -0.5, window, heads, kv_heads, hd))
+    assert torch.equal(*results)
