@@ -464,6 +464,23 @@ def rowwise_chunks(longest: int, window: int) -> int:
     return max(1, -(-longest // chunk))
 
 
+ROWWISE_WORKSPACE = 256 << 20   # bytes that chunks' results may take in steps of more rows than that
+
+
+def rowwise_splits(n_tokens: int, heads: int, kv_heads: int, head_dim: int, chunks: int, dtype: torch.dtype) -> bool:
+    """Whether a step's rows go by chunks of keys. The kernel that takes all heads of a kv head in float32 makes that the faster way for
+    more rows, the more heads it has (MI355X, a wave a row or stretches, and by chunks: 28 heads of 128 over 4, 100 tokens after 1000 170 and
+    77 us, 146 from 0 38 and 22, 290 56 and 47, 400 73 and 73, 200 requests of 300 positions 139 and 67; 32 over 8, 100 tokens after 1000 167
+    and 134, 16 tokens of 8 requests after 500 93 and 99, 200 from 0 47 and 49)."""
+    rows = n_tokens * heads
+    if rows < ROWWISE_SPLIT_BELOW:
+        return True
+    group = heads // kv_heads
+    below = ROWWISE_SPLIT_BELOW * (4 if group >= 7 else 2 if group >= 4 else 1)
+    return (dtype == torch.float32 and head_dim % 16 == 0 and head_dim <= 128 and rows < below
+            and rows * chunks * (head_dim + 2) * 4 <= ROWWISE_WORKSPACE)
+
+
 def paged_attention_rowwise(q: torch.Tensor, k_cache: torch.Tensor, v_cache: torch.Tensor,
                             block_table: torch.Tensor, seq_of_token: torch.Tensor, positions: torch.Tensor,
                             scale: float, window: int, heads: int, kv_heads: int, head_dim: int,
@@ -488,7 +505,7 @@ def paged_attention_rowwise(q: torch.Tensor, k_cache: torch.Tensor, v_cache: tor
     capacity = block_table.shape[1] * page_size
     longest = capacity if longest is None else min(int(longest), capacity)
     if split is None:
-        split = n_tokens * heads < ROWWISE_SPLIT_BELOW
+        split = rowwise_splits(n_tokens, heads, kv_heads, head_dim, rowwise_chunks(max(longest, 1), window), q.dtype)
     chunks = rowwise_chunks(max(longest, 1), window) if split else 0
     usual_chunks = rowwise_chunks(max(min(int(usual), longest), 1), window) if split and usual is not None else 0
     part_o = part_ml = None

@@ -202,3 +202,12 @@ def test_tiles_of_half_the_queries_where_whole_ones_leave_compute_units_idle():
     assert [planner.tile_rows([count]) for count in (2, 128, 2048, 2304, 2305)] == [64, 64, 64, 64, 128]      # 9 pairs of tiles of 14 heads: 126
     assert planner.tile_rows([512, 512, 600]) == 64 and planner.tile_rows([300] * 5) == 128
     assert planner.key != QueryTilePlanner(False, 28).key
+
+
+@pytest.mark.parametrize("tokens,heads,kv_heads,head_dim,chunks,dtype,splits", [
+    (73, 28, 4, 128, 200, torch.float32, True), (74, 28, 4, 128, 8, torch.float32, True), (292, 28, 4, 128, 8, torch.float32, True),
+    (293, 28, 4, 128, 8, torch.float32, False), (292, 28, 4, 128, 64, torch.float32, False), (292, 28, 4, 120, 8, torch.float32, False),
+    (127, 32, 8, 128, 8, torch.float32, True), (128, 32, 8, 128, 8, torch.float32, False), (256, 8, 8, 128, 8, torch.float32, False),
+    (74, 28, 4, 128, 8, torch.bfloat16, False), (74, 28, 4, 144, 8, torch.float32, False)])
+def test_rowwise_splits(tokens, heads, kv_heads, head_dim, chunks, dtype, splits):
+    assert kernels.rowwise_splits(tokens, heads, kv_heads, head_dim, chunks, dtype) == splits

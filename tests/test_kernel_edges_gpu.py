@@ -390,3 +390,20 @@ def test_prompts_in_tiles_of_half_the_queries_have_the_same_bits(heads, kv_heads
         pairs = torch.tensor(k.pair_query_tiles(tiles, adjacent=window > 0), dtype=torch.int32, device=DEVICE)
         results.append(k.paged_attention_prefill(t["q"], t["k"], t["v"], t["table"], pairs, t["pos"], hd ** -0.5, window, heads, kv_heads, hd))
     assert torch.equal(*results)
+
+
+# ---- float32 attention by chunks, all heads of a kv head together: every head size, one head a kv head to more than 16, windows that begin in
+# either tile of a chunk, and values that are not finite where a token sees them and where it does not ----
+@pytest.mark.parametrize("heads,kv_heads,hd,page_size", [(28, 4, 16, 16), (14, 2, 32, 32), (9, 9, 48, 48), (7, 1, 64, 16), (40, 2, 80, 48), (5, 1, 96, 16),
+                                                         (34, 2, 112, 32), (4, 1, 128, 16)])
+@pytest.mark.parametrize("window", [0, 70, 190])
+def test_chunks_for_all_heads_have_the_bits_of_a_wave_a_row(heads, kv_heads, hd, page_size, window):
+    k, rng = kernels(), np.random.default_rng(hd + window)
+    lengths, counts = [300, 1, 64, 65, 128, 129, 700, 193], [1, 1, 3, 1, 1, 2, 4, 1]
+    t, *_ = build_paged_case(rng, torch.float32, lengths, counts, heads, kv_heads, hd, page_size)
+    for broken in (None, float("nan"), float("inf")):
+        if broken is not None:
+            t["v"].view(-1)[::997] = broken
+        run = lambda **way: k.paged_attention_rowwise(t["q"], t["k"], t["v"], t["table"], t["seq"], t["pos"], hd ** -0.5, window, heads, kv_heads, hd, **way)
+        by_chunks, by_rows = run(split=True), run(split=False)
+        assert torch.equal(torch.nan_to_num(by_chunks, 7.0, 8.0, 9.0), torch.nan_to_num(by_rows, 7.0, 8.0, 9.0)), broken
