@@ -96,15 +96,18 @@ __device__ inline float gated_value(float g, float u, int act, float limit, floa
     return g / (1.0f + expf(-slope * g)) * (u + 1.0f);
 }
 
-// n / (1 + exp(-t)) to about an ulp, in a third of the instructions of expf and a division: exp by the hardware's exp2 with what the product with
-// log2(e) loses put back, and a reciprocal refined once. t beyond 87 in size, where the quotient is n or nothing that a bfloat16 sum notices, counts as 87.
+// n / (1 + exp(-t)) to about an ulp, in fewer instructions than expf and a division: exp by the hardware's exp2 with what the product with
+// log2(e) loses put back, and a reciprocal refined once, for t up to 87 in size, where neither leaves the numbers. Beyond 87 the quotient is n; below -87,
+// where it is n exp(t), it goes on to nothing by a factor of its own, which is one otherwise: n has no bound, so a quotient that stayed at
+// exp(-87) would leave 5.6 of the lowest bfloat16. (The factor is free in rows that wait for memory; tiled gated products 397 -> 404 us and 38.4 -> 39.9.)
 __device__ inline float over_one_plus_exp(float n, float t) {
     constexpr float kLog2e = 1.44269502162933349609f, kLog2eRest = 1.92596299112661746887e-8f, kLn2 = 0.69314718055994530942f;
-    t = __builtin_amdgcn_fmed3f(t, -87.0f, 87.0f);
-    const float high = -t * kLog2e, low = fmaf(-t, kLog2eRest, fmaf(-t, kLog2e, -high));
+    constexpr float k87Log2e = 125.514473f;     // not less than 87 kLog2e
+    const float within = __builtin_amdgcn_fmed3f(t, -87.0f, 87.0f);
+    const float high = -within * kLog2e, low = fmaf(-within, kLog2eRest, fmaf(-within, kLog2e, -high));
     const float power = __builtin_amdgcn_exp2f(high), d = 1.0f + fmaf(power, low * kLn2, power);
     const float r = __builtin_amdgcn_rcpf(d);
-    return n * fmaf(fmaf(-d, r, 1.0f), r, r);
+    return n * fmaf(fmaf(-d, r, 1.0f), r, r) * __builtin_amdgcn_exp2f(fminf(fmaf(t, kLog2e, k87Log2e), 0.0f));
 }
 
 // The gate of a gated product's epilogue: silu(z), or the tanh form of gelu, which is z sigmoid(2 sqrt(2 / pi) (z + 0.044715 z^3)).

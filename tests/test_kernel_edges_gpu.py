@@ -407,3 +407,63 @@ def test_chunks_for_all_heads_have_the_bits_of_a_wave_a_row(heads, kv_heads, hd,
         run = lambda **way: k.paged_attention_rowwise(t["q"], t["k"], t["v"], t["table"], t["seq"], t["pos"], hd ** -0.5, window, heads, kv_heads, hd, **way)
         by_chunks, by_rows = run(split=True), run(split=False)
         assert torch.equal(torch.nan_to_num(by_chunks, 7.0, 8.0, 9.0), torch.nan_to_num(by_rows, 7.0, 8.0, 9.0)), broken
+
+
+# ---- gates of every size: where exp(-gate) leaves the numbers the quotient is the gate or nothing, in every kernel that forms one ----
+GATES = [-1.0, -20.0, -86.5, -87.5, -90.0, -100.0, -1e3, -1e13, -1e30, -3.3895313892515355e38, 1.0, 87.5, 1e3, 1e13, 1e30, 3.3895313892515355e38]
+CLAMP, SLOPE = 7.0, 1.702
+
+
+def gated_in_64_bits(gate, up, kind):
+    """``gate * sigmoid(t) * up`` without a step that leaves the numbers; at -inf it is no number, as -inf * 0 is."""
+    gate, up = np.asarray(gate, np.float64), np.asarray(up, np.float64)
+    if kind == "clamped":
+        gate, up = np.minimum(gate, CLAMP), np.clip(up, -CLAMP, CLAMP) + 1.0
+    t = {"silu": gate, "gelu_tanh": math.sqrt(8.0 / math.pi) * (gate + 0.044715 * gate ** 3), "clamped": SLOPE * gate}[kind]
+    small = np.exp(-np.abs(t))
+    with np.errstate(invalid="ignore"):
+        return gate * (np.where(t < 0, small, 1.0) / (1.0 + small)) * up
+
+
+def assert_gated(got, gate, up, kind):
+    """A rounding to bfloat16 and a little, or below its smallest normal number."""
+    gate, up = (torch.tensor(values).to(torch.bfloat16).double().numpy() for values in (gate, up))
+    want = np.broadcast_to(gated_in_64_bits(gate, up, kind), got.shape)
+    np.testing.assert_allclose(got.double().cpu().numpy(), want, rtol=2.0 ** -8, atol=2.0 ** -126)
+
+
+@pytest.mark.parametrize("kind", ["silu", "gelu_tanh"])
+@pytest.mark.parametrize("shift", [0, 1])       # rows that begin at a 16-byte boundary or not
+def test_activations_of_gates_of_every_size(kind, shift):
+    gates = GATES + [float("-inf"), float("inf"), float("nan")] + [-0.0] * 5
+    ups = [0.5, -0.25] * (len(gates) // 2)
+    rows = torch.empty(3 * 2 * len(gates) + shift, dtype=torch.bfloat16, device=DEVICE)[shift:].view(3, 2 * len(gates))
+    rows.copy_(torch.tensor(gates + ups))
+    assert_gated(kernels().gated_activation(rows, kind), gates, ups, kind)
+
+
+@pytest.mark.parametrize("product,rows,kind", [(product, rows, kind) for product, rows in (("skinny", 5), ("skinny", 16), ("medium", 40), ("tiled", 130))
+                                                for kind in ("silu", "gelu_tanh", "clamped") if (product, kind) != ("medium", "clamped")])
+@pytest.mark.parametrize("width", [16, 13])     # whole pieces of 16 bytes of results, and not
+def test_products_with_gates_of_every_size(product, rows, kind, width):
+    k, gates, ups = kernels(), GATES[:width], ([0.5, -0.25] * 8)[:width]
+    x, weight = torch.zeros((rows, 64), dtype=torch.bfloat16, device=DEVICE), torch.zeros((2 * width, 64), dtype=torch.bfloat16, device=DEVICE)
+    x[:, 40], weight[:, 40] = 1.0, torch.tensor(gates + ups, device=DEVICE)      # so that the sums are the gates themselves
+    packed = k.pack_weight(weight, interleave_halves=True)
+    if kind == "clamped":
+        got = k.gemm_skinny_clamped(x, packed, 2 * width, CLAMP, SLOPE) if product == "skinny" else k.gemm_tiled(x, packed, 2 * width, "clamped", limit=CLAMP, slope=SLOPE)
+    else:
+        got = {"skinny": k.gemm_skinny, "medium": k.gemm_medium, "tiled": k.gemm_tiled}[product](x, packed, 2 * width, "gated" if kind == "silu" else "gated_gelu")
+    assert_gated(got, gates, ups, kind)
+
+
+@pytest.mark.parametrize("tokens,grouped", [(4, False), (60, True), (700, True)])       # few pairs on the matrix units, tiles of pairs, large tiles
+@pytest.mark.parametrize("kind", ["silu", "clamped"])
+def test_experts_with_gates_of_every_size(tokens, grouped, kind):
+    k, size, gates, ups = kernels(), 512, GATES * 32, [0.5, -0.25] * 256
+    x, gate_up = torch.zeros((tokens, size), dtype=torch.bfloat16, device=DEVICE), torch.zeros((2, 2 * size, size), dtype=torch.bfloat16, device=DEVICE)
+    x[:, 40], gate_up[:, :, 40] = 1.0, torch.tensor(gates + ups, device=DEVICE)
+    down = torch.eye(size, device=DEVICE).to(torch.bfloat16).repeat(2, 1, 1)       # the result is the inner values
+    ids, weights = (torch.arange(tokens, device=DEVICE, dtype=torch.int32) % 2)[:, None].contiguous(), torch.ones((tokens, 1), device=DEVICE)
+    options = dict(activation="clamped_glu", limit=CLAMP, slope=SLOPE) if kind == "clamped" else {}
+    assert_gated(k.moe_experts(x, ids, weights, gate_up, down, False, grouped=grouped, **options)[0], gates, ups, kind)
