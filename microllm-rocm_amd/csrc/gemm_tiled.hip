@@ -86,10 +86,15 @@ __global__ __launch_bounds__(kTiledThreads, 1) void gemm_tiled_kernel(const bf16
         // 2 * wave + 1, a k step an instruction.
         const bf16* a_block = a + static_cast<int64_t>(m0) * k;
         unsigned a_offset[A_TURNS];    // of the lane's 16 bytes from a_block, at stage 0, in bytes
-        const int a_loads = A_LOADS % kTiledWaves == 0 ? A_TURNS : (A_LOADS - wave + kTiledWaves - 1) / kTiledWaves;      // of this wave
+        // Tiles of 160 rows have loads for half the waves' third turn: the others repeat their second, the same bytes to the same place, since no wave
+        // may pass a load over (tiled_operands.h).
+        auto a_load = [&](int turn) __attribute__((always_inline)) {
+            const int load = wave + turn * kTiledWaves;
+            return A_LOADS % kTiledWaves == 0 || load < A_LOADS ? load : load - kTiledWaves;
+        };
 #pragma unroll
         for (int t = 0; t < A_TURNS; ++t) {
-            const int load = min(wave + t * kTiledWaves, A_LOADS - 1);
+            const int load = a_load(t);
             const int row_in_piece = 8 * (load % 2) + lane / 8;
             const int row = min((load / 2) * 16 + row_in_piece, m - 1 - m0);           // rows past the end repeat the last one
             a_offset[t] = (static_cast<unsigned>(row) * static_cast<unsigned>(k) + (((lane % 8) ^ (row_in_piece / 2)) * 8)) * 2;
@@ -109,7 +114,7 @@ __global__ __launch_bounds__(kTiledThreads, 1) void gemm_tiled_kernel(const bf16
         // half step back by 64 bytes there.
         auto copy_a = [&](int turn, int stage, unsigned slot) __attribute__((always_inline)) {
             bf16* a_place = slots + slot * kSlotElements;
-            const int piece = (wave + turn * kTiledWaves) / 2, h = wave % 2;      // the wave's loads are all of one half
+            const int piece = a_load(turn) / 2, h = wave % 2;      // the wave's loads are all of one half
             const bool upper = (((lane >> 2) & 1) ^ h) != 0;      // the lane's chunk is one of the row's second four
             const char* a_source = reinterpret_cast<const char*>(a_block) + stage * 128 + (a_offset[turn] - ((2 * stage + 1 >= k_steps && upper) ? 64u : 0u));
             // (the place is computed here: with a subscript of a captured array in this call the host pass
@@ -137,7 +142,7 @@ __global__ __launch_bounds__(kTiledThreads, 1) void gemm_tiled_kernel(const bf16
 
         if (first_stage < stages) {
             if (index != static_cast<int>(blockIdx.x) / 8) workgroup_meets();        // every wave is done with the slots of the tile before
-            multiply_stages<kPackedStep, WM, A_TURNS>(acc, first_stage, stages, a_loads, a_step0, a_step1, w_lane, w_lane, copy_a, copy_w);
+            multiply_stages<kPackedStep, WM, A_TURNS>(acc, first_stage, stages, a_step0, a_step1, w_lane, w_lane, copy_a, copy_w);
         }
 
         if constexpr (EPILOGUE == 3) {

@@ -145,7 +145,7 @@ __device__ __attribute__((always_inline)) inline void tile_products(bf16* slots,
 #pragma unroll
         for (int mt = 0; mt < WM; ++mt) acc[nt][mt] = floatx4{0.0f, 0.0f, 0.0f, 0.0f};
 
-    multiply_stages<0, WM, A_TURNS>(acc, 0, k / 64, A_TURNS, a_at + step0, a_at + step1, w_at + step0, w_at + step1, copy_a, copy_w);
+    multiply_stages<0, WM, A_TURNS>(acc, 0, k / 64, a_at + step0, a_at + step1, w_at + step0, w_at + step1, copy_a, copy_w);
 
     if constexpr (GATED) {
         workgroup_meets();

@@ -96,31 +96,28 @@ __device__ __attribute__((always_inline)) inline void operands_arrived(TiledOper
 }
 
 // The stages of a tile, from `first` to before `stages`, one at least. copy_a(turn, stage, slot) and copy_w(turn, stage, slot) issue one of a wave's
-// A_TURNS (a_loads of this wave: all or all but one) and four loads of a stage. While a stage's first step is multiplied its second is read, and W's loads of the stage after next go out, into the slot
-// that was read a stage ago; then the next stage has landed (the wave's loads before the barrier, everyone's after it) and this one has been read
-// by all: A's loads of the stage after next go out while the second step is multiplied and the next stage's first is read. After the last
+// A_TURNS and four loads of a stage, every wave all of them. While a stage's first step is multiplied its second is read, and W's loads of the stage after
+// next go out, into the slot that was read a stage ago; then the next stage has landed (the wave's loads before the barrier, everyone's after it) and this
+// one has been read by all: A's loads of the stage after next go out while the second step is multiplied and the next stage's first is read. After the last
 // stage nothing is copied, and what is read then is multiplied by nobody.
 template <int W_STEP, int WM, int A_TURNS, typename CopyA, typename CopyW>
-__device__ __attribute__((always_inline)) inline void multiply_stages(floatx4 (&acc)[kWaveTilesN][WM], int first, int stages, int a_loads, unsigned a_step0,
+__device__ __attribute__((always_inline)) inline void multiply_stages(floatx4 (&acc)[kWaveTilesN][WM], int first, int stages, unsigned a_step0,
                                                                       unsigned a_step1, unsigned w_step0, unsigned w_step1, const CopyA& copy_a,
                                                                       const CopyW& copy_w) {
     constexpr std::make_integer_sequence<int, WM> row_tiles{};
     TiledOperands<WM> even, odd;      // of a stage's first and second k step
     const bool second = first + 1 < stages;
 #pragma unroll
-    for (int t = 0; t < A_TURNS; ++t)
-        if (t < a_loads) copy_a(t, first, 0);
+    for (int t = 0; t < A_TURNS; ++t) copy_a(t, first, 0);
 #pragma unroll
     for (int t = 0; t < 4; ++t) copy_w(t, first, 0);
     if (second) {
 #pragma unroll
-        for (int t = 0; t < A_TURNS; ++t)
-            if (t < a_loads) copy_a(t, first + 1, 1);
+        for (int t = 0; t < A_TURNS; ++t) copy_a(t, first + 1, 1);
 #pragma unroll
         for (int t = 0; t < 4; ++t) copy_w(t, first + 1, 1);
         // the first stage's loads of this wave have landed when only the second stage's are on their way
-        if (a_loads == A_TURNS) asm volatile("s_waitcnt vmcnt(%0)" :: "n"(A_TURNS + 4) : "memory");
-        else asm volatile("s_waitcnt vmcnt(%0)" :: "n"(A_TURNS + 3) : "memory");
+        asm volatile("s_waitcnt vmcnt(%0)" :: "n"(A_TURNS + 4) : "memory");
     } else {
         asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
     }
@@ -140,9 +137,7 @@ __device__ __attribute__((always_inline)) inline void multiply_stages(floatx4 (&
         __builtin_amdgcn_s_barrier();
         products<W_STEP, WM, 0>(acc, odd, even, a_step0 + (1 - a_now) * kSlotBytes, w_step0 + w_next * kSlotBytes, [&](auto place) __attribute__((always_inline)) {
             constexpr int kPlace = decltype(place)::value;
-            if constexpr (MORE && kPlace % 2 == 0 && kPlace / 2 < A_TURNS) {
-                if (kPlace / 2 < a_loads) copy_a(kPlace / 2, stage + 2, a_now);
-            }
+            if constexpr (MORE && kPlace % 2 == 0 && kPlace / 2 < A_TURNS) copy_a(kPlace / 2, stage + 2, a_now);
         }, row_tiles);
         operands_arrived<-1>(even);
         a_now = 1 - a_now;
