@@ -857,23 +857,36 @@ def decode_splits(n_tokens: int, kv_heads: int, longest: int) -> int:
     return splits
 
 
-FEW_ROWS_SPLITS = 8         # splits of the keys from 1024 on where a step has few (token, kv head) rows, and up to twice as many,
-FEW_ROWS_KEYS = 256         # of this many keys each
+FEW_ROWS_SPLITS = 8         # splits of the keys from 1024 positions on where a step has few (token, kv head) rows, and twice as many
+FEW_ROWS_LONG = 8192        # from this many on
+FEW_ROWS_WIDE_KEYS = 128    # keys of a split of heads wider than 128, of which 4 to 16 are made
 
 
 def decode_parts(n_tokens: int, kv_heads: int, longest: int, head_dim: int) -> int:
     """The splits a step's decode attention takes: ``decode_splits`` where the rows alone give a quarter of the compute units
     their workgroups or the keys are few, else more and shorter ones, since a workgroup brings no more than about 50 GB/s and eight parts
     are joined in one round of loads (MI355X, attention and join, 28 heads of 128 over 4: one request of 1024 positions with 2 and 8 splits
-    11.1 and 8.7 us, of 2048 with 4 and 8 11.0 and 9.5, of 4096 with 8, 16 and 32 11.1, 10.7 and 12.4; 8 of 4096 with 4 and 8 21.0 and 18.4; 16 of
-    1024 with 2 and 4 15.0 and 14.0; but 32 of 1024 with 1 and 2 18.1 and 18.8, one of 512 with 1 and 2 7.9 and 8.8. 14 heads of 64 over 2:
-    one of 1024 with 2 and 8 8.8 and 6.6, 32 of 1024 with 2 and 4 11.2 and 9.8). Heads wider than 128 have half the waves' loads in flight
-    and take splits of 128 keys from 512 on (one of 512 with 1 and 4 15.1 and 13.0, of 2048 with 4 and 16 18.4 and 14.7, of 4096 with 16 and 32 16.5 and 17.0)."""
+    11.1 and 8.6 us, of 2048 with 4 and 8 11.2 and 9.5; 8 of 4096 with 4 and 8 19.4 and 18.2; 16 of 1024 with 2 and 4 14.0 and 13.6; but 32 of 1024
+    with 1 and 2 18.1 and 18.8, one of 512 with 1 and 2 7.9 and 8.8. 14 heads of 64 over 2: one of 1024 with 2 and 8 8.5 and 6.7, 32 of 1024 with 2 and 4
+    10.4 and 9.8).
+
+    ``longest`` is what the step is planned for, a power of two that its requests pass half of, or one of them does; so each line lies where that and
+    full length are the faster for it. 8 for 2: one request of 513 of 1024 positions 9.5 and 8.0 us, 8 of 513 10.6 and 9.5, 768 beside seven of 70
+    10.5 and 8.7, heads of 64 7.6 and 6.5. 16 for 8 gain only from 8192 on: 4 requests of 8192, 4097, or 6144 beside three of 70
+    19.5 and 19.3, 14.5 and 14.8, 15.0 and 13.1 (4 splits a kv head before 21.1, 15.4, 14.8); of 4096 13.9 and 14.6, two of 2049 10.6 and 11.2, heads of 64, 4
+    of 2049 8.8 and 9.4, 3072 beside three of 70 8.6 and 9.2.
+
+    Heads wider than 128 have half the waves' loads in flight and take splits of 128 keys from 512 on (16 heads of 256 over one: one of 512 with 1 and 4
+    15.1 and 13.0, of 257 13.7 and 12.6, of 2048 with 4 and 16 18.5 and 14.8), from 1024 where 33 to 64 rows leave room for 4 (64 of 257, of 512, and
+    384 beside 63 of 70 with 1 and 4 16.8 and 17.9, 19.9 and 21.2, 13.8 and 15.3; of 513 and 1024 with 2 and 4 21.5 and 21.2, 26.0 and 26.6)."""
     usual, room = decode_splits(n_tokens, kv_heads, longest), 256 // max(1, n_tokens * kv_heads)
-    wide = 2 if head_dim > 128 else 1
-    if room < 4 or longest < 4 * FEW_ROWS_KEYS // wide:
+    if head_dim <= 128:
+        if room < 4 or longest < 1024:
+            return usual
+        return min(room, max(usual, FEW_ROWS_SPLITS * (2 if longest >= FEW_ROWS_LONG else 1)))
+    if room < 4 or longest < (512 if room >= 8 else 1024):
         return usual
-    return min(room, max(usual, min(2 * FEW_ROWS_SPLITS, max(FEW_ROWS_SPLITS // wide, longest * wide // FEW_ROWS_KEYS))))
+    return min(room, max(usual, min(16, max(4, longest // FEW_ROWS_WIDE_KEYS))))
 
 
 def paged_attention_decode(q: torch.Tensor, k_cache: torch.Tensor, v_cache: torch.Tensor, block_table: torch.Tensor,
