@@ -24,13 +24,15 @@ constexpr int kPlain = 0, kExtras = 1, kBiased = 2;
 
 constexpr int kDecodeWaves = 4;
 constexpr int kDecodeThreads = kDecodeWaves * kWave;
+constexpr int kStreamedFrom = 256;      // workgroups from which the pages are read past the caches: see load_piece
 
 typedef unsigned uintx4 __attribute__((ext_vector_type(4)));
 
 // 16 bytes of keys or values. STREAM: read past the caches (nothing is read twice): with a workgroup or more per
-// compute unit the pages then come in at 6.3 instead of 5.6 TB/s (64 requests of 3000 positions 70.4 and 62.6 us), with half as many
-// 8 requests of 4096 positions in 4 splits take 19.6 instead of 21.0 us, 16 of 2048 with heads of 64 10.3 instead of 11.1; heads wider
-// than 128 lose (8 of 4096 in 16 splits 20.8 and 20.0), and so do fewer workgroups where the pages of all layers stay in the last cache.
+// compute unit the pages then come in at 6.3 instead of 5.6 TB/s (64 requests of 3000 positions 70.4 and 62.6 us). With fewer it is the faster way only where
+// all of them have as much to read (12 requests of 4096 positions in 5 splits, 28 heads of 128 over 4, 26.2 and 24.3 us) and costs as much in ragged
+// steps, whose pages the last cache holds between two passes (4 requests from 3072 down to 230 positions in 8 splits 10.8 and 11.9, 32 of 384 down to
+// 20 7.8 and 8.8, 768 beside 31 of 70 10.0 and 11.7).
 template <bool STREAM>
 __device__ inline uint4 load_piece(const bf16* from) {
     if (STREAM) {
@@ -464,7 +466,7 @@ static int launch_decode(const void* q, const void* k_cache, const void* v_cache
     const int group = heads / kv_heads;
     const MllAttentionExtras given = extras ? *extras : MllAttentionExtras{nullptr, 0, nullptr, 1.0f, 0};
     const dim3 grid(n_tokens * (kv_heads * ((group + 15) / 16)), n_splits);
-    const bool stream_pages = static_cast<int64_t>(grid.x) * grid.y >= (HD_TILES <= 8 ? 128 : 256);      // see load_piece
+    const bool stream_pages = static_cast<int64_t>(grid.x) * grid.y >= kStreamedFrom;
     const auto launch = [&](auto streamed, auto form) {
         paged_attention_decode_kernel<HD_TILES, decltype(streamed)::value, decltype(form)::value><<<grid, kDecodeThreads, 0, stream>>>(
             static_cast<const bf16*>(q), static_cast<const bf16*>(k_cache), static_cast<const bf16*>(v_cache), block_table,

@@ -866,15 +866,15 @@ def decode_parts(n_tokens: int, kv_heads: int, longest: int, head_dim: int) -> i
     """The splits a step's decode attention takes: ``decode_splits`` where the rows alone give a quarter of the compute units
     their workgroups or the keys are few, else more and shorter ones, since a workgroup brings no more than about 50 GB/s and eight parts
     are joined in one round of loads (MI355X, attention and join, 28 heads of 128 over 4: one request of 1024 positions with 2 and 8 splits
-    11.1 and 8.6 us, of 2048 with 4 and 8 11.2 and 9.5; 8 of 4096 with 4 and 8 19.4 and 18.2; 16 of 1024 with 2 and 4 14.0 and 13.6; but 32 of 1024
-    with 1 and 2 18.1 and 18.8, one of 512 with 1 and 2 7.9 and 8.8. 14 heads of 64 over 2: one of 1024 with 2 and 8 8.5 and 6.7, 32 of 1024 with 2 and 4
-    10.4 and 9.8).
+    11.0 and 8.6 us, of 2048 with 4 and 8 11.2 and 9.5; 8 of 4096 with 4 and 8 20.8 and 18.3; 16 of 1024 with 2 and 4 14.9 and 14.0; but 32 of 1024
+    with 1 and 2 18.1 and 18.8, one of 512 with 1 and 2 7.9 and 8.8. 14 heads of 64 over 2: one of 1024 with 2 and 8 8.5 and 6.8, 32 of 1024 with 2 and 4
+    11.0 and 9.9).
 
     ``longest`` is what the step is planned for, a power of two that its requests pass half of, or one of them does; so each line lies where that and
-    full length are the faster for it. 8 for 2: one request of 513 of 1024 positions 9.5 and 8.0 us, 8 of 513 10.6 and 9.5, 768 beside seven of 70
-    10.5 and 8.7, heads of 64 7.6 and 6.5. 16 for 8 gain only from 8192 on: 4 requests of 8192, 4097, or 6144 beside three of 70
-    19.5 and 19.3, 14.5 and 14.8, 15.0 and 13.1 (4 splits a kv head before 21.1, 15.4, 14.8); of 4096 13.9 and 14.6, two of 2049 10.6 and 11.2, heads of 64, 4
-    of 2049 8.8 and 9.4, 3072 beside three of 70 8.6 and 9.2.
+    full length are the faster for it. 8 for 2: one request of 513 of 1024 positions 9.5 and 8.0 us, 8 of 513 10.3 and 9.6, 768 beside seven of 70
+    10.2 and 8.8, heads of 64 7.7 and 6.4. 16 for 8 only from 8192 on: 4 requests of 8192, 4097, and 6144 beside three of 70 20.9 and 19.4, 15.3 and 14.9,
+    15.1 and 13.2; of 4096, 2049, and 3072 beside three of 70 14.6 and 14.7, 12.1 and 12.2, 10.5 and 11.2, two of 2049 10.3 and 10.8, heads of 64, 4 of 2049
+    8.8 and 9.4, 3072 beside three of 70 8.5 and 9.1.
 
     Heads wider than 128 have half the waves' loads in flight and take splits of 128 keys from 512 on (16 heads of 256 over one: one of 512 with 1 and 4
     15.1 and 13.0, of 257 13.7 and 12.6, of 2048 with 4 and 16 18.5 and 14.8), from 1024 where 33 to 64 rows leave room for 4 (64 of 257, of 512, and

@@ -326,7 +326,7 @@ def test_gated_products_of_49_to_64_rows_at_any_address(rows, n, k):
 
 # ---- decode attention: both sides of the line past which pages are read past the caches, with and without a bias ----
 @pytest.mark.parametrize("heads,kv_heads,hd,page_size,splits,biased", [
-    (4, 4, 64, 16, 8, False), (4, 4, 64, 16, 3, True), (8, 4, 128, 32, 5, True), (8, 4, 128, 16, 4, False), (2, 2, 192, 48, 19, True),
+    (4, 4, 64, 16, 8, False), (4, 4, 64, 16, 3, True), (8, 4, 128, 32, 5, True), (8, 4, 128, 16, 4, False), (8, 4, 128, 16, 8, True), (8, 4, 128, 32, 9, False), (2, 2, 192, 48, 19, True),
     (3, 3, 48, 16, 11, True), (5, 1, 256, 16, 16, False), (18, 1, 80, 16, 9, True)])
 def test_decode_attention_reads_every_line_of_its_pages(heads, kv_heads, hd, page_size, splits, biased):
     rng = np.random.default_rng(heads + hd + splits)
