@@ -34,9 +34,10 @@ class QueryTilePlanner:
     without a window, the longest workgroups first, were measured too: a 16384-token prompt takes 3.0 instead of
     2.6 ms a layer that way.)
 
-    Where the tiles of 128 would give fewer workgroups (of the ``heads`` query heads) than half the compute units, tiles have 64 queries: twice
-    the workgroups, with one wave a SIMD instead of two, which share its exponentials (a pass of
-    portions of 512 beside single tokens at 0.5B sizes 25.5 -> 25.0 ms). A token's bits do not depend on its tile.
+    Where the tiles of 128 would give fewer workgroups (of the ``heads`` query heads) than half the compute units, requests of more than one such
+    tile have tiles of 64 queries: twice the workgroups, with one wave a SIMD instead of two, which share its exponentials (a pass of
+    portions of 512 beside single tokens at 0.5B sizes 25.5 -> 25.0 ms). The tiles of a portion of up to 128 would share a workgroup either
+    way, and take 5 % longer as two. A token's bits do not depend on its tile.
 
     Plan: ``tiles`` int32 [workgroups, 5]; ``single_tokens`` int32 [rows]; ``max_single_total``, the longest of
     the requests listed there."""
@@ -47,19 +48,21 @@ class QueryTilePlanner:
         self.heads = heads      # 0: whole tiles always
         self.key = ("paged_attention_query_tiles", windowed, heads)
 
-    def tile_rows(self, counts) -> int:
+    def tile_rows(self, counts):
+        """The queries a tile has of every request, by how many each brings."""
         pairs = sum((-(-count // kernels.QUERY_TILE) + 1) // 2 for count in counts)
-        return kernels.QUERY_TILE // 2 if 0 < 2 * pairs * self.heads <= kernels.COMPUTE_UNITS else kernels.QUERY_TILE
+        half = 0 < 2 * pairs * self.heads <= kernels.COMPUTE_UNITS
+        return [kernels.QUERY_TILE // 2 if half and count > kernels.QUERY_TILE else kernels.QUERY_TILE for count in counts]
 
     def plan(self, host):
         counts, cu = host.counts, host.cu
         if host.single_tokens_only:
             return {"tiles": np.zeros((0, 5), np.int32), "single_tokens": np.zeros(0, np.int32)}, {"max_single_total": 0}
         mixed = any(count == 1 for count in counts)
-        rows = self.tile_rows([count for count in counts if not (mixed and count == 1)])
-        tile_list = [(index, int(cu[index]) + offset, min(rows, count - offset), host.starts[index] + offset)
-                     for index, count in enumerate(counts) if not (mixed and count == 1)
-                     for offset in range(0, count, rows)]
+        portions = [index for index, count in enumerate(counts) if not (mixed and count == 1)]
+        tile_list = [(index, int(cu[index]) + offset, min(rows, counts[index] - offset), host.starts[index] + offset)
+                     for index, rows in zip(portions, self.tile_rows([counts[index] for index in portions]))
+                     for offset in range(0, counts[index], rows)]
         tiles = np.asarray(kernels.pair_query_tiles(tile_list, adjacent=self.windowed), dtype=np.int32).reshape(-1, 5)
         single = np.asarray([cu[index] for index, count in enumerate(counts) if mixed and count == 1], dtype=np.int32)
         longest = max((host.totals[index] for index, count in enumerate(counts) if mixed and count == 1), default=0)

@@ -198,11 +198,12 @@ def test_decode_parts(tokens, kv_heads, longest, head_dim, splits):
 
 def test_tiles_of_half_the_queries_where_whole_ones_leave_compute_units_idle():
     from microllm_rocm_amd.parts.attention import QueryTilePlanner
-    assert QueryTilePlanner(False).tile_rows([512]) == 128
+    assert QueryTilePlanner(False).tile_rows([512]) == [128]
     planner = QueryTilePlanner(False, 14)
-    assert planner.tile_rows([]) == 128
-    assert [planner.tile_rows([count]) for count in (2, 128, 2048, 2304, 2305)] == [64, 64, 64, 64, 128]      # 9 pairs of tiles of 14 heads: 126
-    assert planner.tile_rows([512, 512, 600]) == 64 and planner.tile_rows([300] * 5) == 128
+    assert planner.tile_rows([]) == []
+    # 9 pairs of tiles of 14 heads: 126; a portion of one tile has one workgroup either way
+    assert [planner.tile_rows([count])[0] for count in (2, 128, 129, 2048, 2304, 2305)] == [128, 128, 64, 64, 64, 128]
+    assert planner.tile_rows([512, 128, 600]) == [64, 128, 64] and planner.tile_rows([300] * 5) == [128] * 5
     assert planner.key != QueryTilePlanner(False, 28).key
 
 
