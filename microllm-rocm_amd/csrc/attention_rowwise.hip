@@ -859,6 +859,30 @@ static int rowwise_heads_a_wave(int group, int64_t rows) {
     return 1;
 }
 
+// Whether chunks go to the kernel for all heads of a kv head, by `work`, its workgroups. It takes about as long for a chunk of few keys as for a whole one,
+// and 18 to 29 us for 1000 of heads of 128 where the chip is full; a wave a chunk and head takes 6.3 for 1000 of tokens that read the same keys
+// (`portions`: more tokens than requests), so that with one or two heads a kv head many tokens of a portion are faster that way, but waits for memory 16
+// (64 keys) to 40 us (128 and more) first. us on MI355X, waves and together, workgroups in brackets:
+// few keys: 3 tokens 9.4 and 10.7, 160 single ones of 17, 28 heads of 128 over 4 (640), 17.0 and 21.5, 14 of 64 over 2 (320) 8.1 and 11.8, but 100 (200) 10.0 and 9.8;
+// a head a kv head, single tokens: 8 heads of 128, 64 and 100 of 40 (512, 800) 20.3 and 16.1, 21.1 and 23.7; 16 of 64, 64 and 100 of 70 (1024, 1600) 23 and 19,
+//   22.2 and 25.5; 12 of 48, 64 and 100 of 129 (1536, 2400) 24.2 and 21.9, 25.9 and 30.0; 8 of 128, 64 and 100 of 500 (2048, 3200) 72 and 63, 93 and 100;
+// portions: 8 of 128, 60, 100, 128 from 0 (480, 800, 1024) 16.9 and 14.5, 32 and 24, 36 and 26, 100 after 60 and 200 from 0 (1600, 3200) 38 and 29, 39 and 47; 12 of 48, 80
+//   from 0 (960) 13.9 and 15.3; 8 of 128, 32, 48 and 60 after 500 (1280, 1920, 2400) 40 and 29, 41 and 42, 41 and 49;
+// two, portions: 16 heads of 128 over 8, two of 40 (640) 15.0 and 19.0, 64 after 200 (1536) 41 and 31, 64 after 500 (2560) 46 and 52, 100 after 3000 (20000) 219
+//   and 339; single tokens: 64 of 1500 (6144) 166 and 158, one of 2000 beside 63 of 50 (8192, most of them empty) 57 and 84;
+// three, 12 of 96 over 4: two of 40 14.5 and 17.0 (640), 64 and 150 after 3000 (6400, 15000) 123 and 100, 192 and 223.
+static bool heads_together(int group, bool portions, int keys, int head_dim, int64_t work) {
+    if (keys <= 24) return !portions && work < 320;
+    if (group >= 4) return true;
+    if (portions) {
+        if (keys <= 64) return work < 320;
+        if (group == 1) return work <= (keys <= 128 ? 8 * head_dim : keys <= 256 ? 16 * head_dim : 1536);
+        return group == 3 || work < 2048;
+    }
+    if (group == 1) return work <= (keys <= 64 ? 640 : keys <= 128 ? 1280 : keys <= 256 ? 2048 : 2816);
+    return group == 3 || work < 8192;
+}
+
 // Merges what MODE 1 left, in the order and with the arithmetic of MODE 0. One wave per (token, head).
 template <typename T, int DIMS>
 __global__ __launch_bounds__(kWave) void paged_attention_rowwise_merge_kernel(
@@ -980,9 +1004,8 @@ static int launch_rowwise_dims(const void* q, const void* k_cache, const void* v
     if constexpr (std::is_same<T, float>::value && DIMS <= 2) {
         const bool aligned = (reinterpret_cast<uintptr_t>(q) | reinterpret_cast<uintptr_t>(k_cache) | reinterpret_cast<uintptr_t>(v_cache) |
                               reinterpret_cast<uintptr_t>(part_o)) % 16 == 0;
-        // A head a kv head shares nothing, and with 16 chunks a compute unit the matrix units then wait for memory as the wave a chunk does, which
-        // has less of it to wait for: 8 heads of 128, 8 requests of 4096 positions 75 and 63 us, 32 of 2000 101 and 108.
-        if (head_dim % 16 == 0 && aligned && forced_heads_a_wave == 0 && (group > 1 || rows < 4096)) {
+        const int keys = reach > 0 ? min(reach, table_width * page_size) : table_width * page_size;
+        if (head_dim % 16 == 0 && aligned && forced_heads_a_wave == 0 && heads_together(group, n_tokens > requests, keys, head_dim, rows)) {
             grouped = true;
             const dim3 group_grid(n_tokens, kv_heads * ((group + 15) / 16), max_chunks);
 #define MLL_ROWWISE_GROUP(TILES)                                                                                       \

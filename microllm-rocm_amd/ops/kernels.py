@@ -467,15 +467,20 @@ def rowwise_chunks(longest: int, window: int) -> int:
 ROWWISE_WORKSPACE = 256 << 20   # bytes that chunks' results may take in steps of more rows than that
 
 
-def rowwise_splits(n_tokens: int, heads: int, kv_heads: int, head_dim: int, chunks: int, dtype: torch.dtype) -> bool:
+def rowwise_splits(n_tokens: int, heads: int, kv_heads: int, head_dim: int, chunks: int, dtype: torch.dtype, requests: int = 0, keys: int = 0) -> bool:
     """Whether a step's rows go by chunks of keys. The kernel that takes all heads of a kv head in float32 makes that the faster way for
     more rows, the more heads it has (MI355X, a wave a row or stretches, and by chunks: 28 heads of 128 over 4, 100 tokens after 1000 170 and
     77 us, 146 from 0 38 and 22, 290 56 and 47, 400 73 and 73, 200 requests of 300 positions 139 and 67; 32 over 8, 100 tokens after 1000 167
-    and 134, 16 tokens of 8 requests after 500 93 and 99, 200 from 0 47 and 49)."""
+    and 134, 16 tokens of 8 requests after 500 93 and 99, 200 from 0 47 and 49). It takes whole chunks, so not where no request has more than a few ``keys``:
+    portions (more tokens than ``requests``) of up to 64, with 7 heads a kv head 48 (28 of 128 over 4, two prompts of 40 12.6 and 14.5, eight of 25 17.1 and 24.2,
+    but two of 64 18.9 and 15.7; 16 of 64 over 4, three of 64 11.0 and 13.2), single tokens, which pass that soon and whose captured steps go on to 256, up to 24 (160
+    of 17 17.0 and 21.5, of 40 20.8 and 22.1, of 70 33.9 and 25.7)."""
     rows = n_tokens * heads
     if rows < ROWWISE_SPLIT_BELOW:
         return True
     group = heads // kv_heads
+    if 0 < keys <= (24 if n_tokens <= requests else 48 if group >= 7 else 64):
+        return False
     below = ROWWISE_SPLIT_BELOW * (4 if group >= 7 else 2 if group >= 4 else 1)
     return (dtype == torch.float32 and head_dim % 16 == 0 and head_dim <= 128 and rows < below
             and rows * chunks * (head_dim + 2) * 4 <= ROWWISE_WORKSPACE)
@@ -505,7 +510,8 @@ def paged_attention_rowwise(q: torch.Tensor, k_cache: torch.Tensor, v_cache: tor
     capacity = block_table.shape[1] * page_size
     longest = capacity if longest is None else min(int(longest), capacity)
     if split is None:
-        split = rowwise_splits(n_tokens, heads, kv_heads, head_dim, rowwise_chunks(max(longest, 1), window), q.dtype)
+        split = rowwise_splits(n_tokens, heads, kv_heads, head_dim, rowwise_chunks(max(longest, 1), window), q.dtype, block_table.shape[0],
+                               longest if usual is None else min(int(usual), longest))
     chunks = rowwise_chunks(max(longest, 1), window) if split else 0
     usual_chunks = rowwise_chunks(max(min(int(usual), longest), 1), window) if split and usual is not None else 0
     part_o = part_ml = None

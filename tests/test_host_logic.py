@@ -214,3 +214,11 @@ def test_tiles_of_half_the_queries_where_whole_ones_leave_compute_units_idle():
     (74, 28, 4, 128, 8, torch.bfloat16, False), (74, 28, 4, 144, 8, torch.float32, False)])
 def test_rowwise_splits(tokens, heads, kv_heads, head_dim, chunks, dtype, splits):
     assert kernels.rowwise_splits(tokens, heads, kv_heads, head_dim, chunks, dtype) == splits
+
+
+@pytest.mark.parametrize("tokens,heads,kv_heads,requests,keys,splits", [
+    (80, 28, 4, 2, 48, False), (80, 28, 4, 2, 49, True), (80, 32, 8, 2, 64, False), (80, 32, 8, 2, 65, True), (80, 28, 4, 80, 24, False),
+    (80, 28, 4, 80, 25, True), (73, 28, 4, 2, 10, True), (80, 28, 4, 0, 0, True)])
+def test_rowwise_splits_of_few_keys(tokens, heads, kv_heads, requests, keys, splits):
+    """Rows of few keys stay with a wave a row, from as many rows on as may have one."""
+    assert kernels.rowwise_splits(tokens, heads, kv_heads, 128, 2, torch.float32, requests, keys) == splits

@@ -409,6 +409,22 @@ def test_chunks_for_all_heads_have_the_bits_of_a_wave_a_row(heads, kv_heads, hd,
         assert torch.equal(torch.nan_to_num(by_chunks, 7.0, 8.0, 9.0), torch.nan_to_num(by_rows, 7.0, 8.0, 9.0)), broken
 
 
+
+# Both sides of each line between the kernel for all heads and a wave a head (24, 64, 128 and 256 keys; 320 to 8192 workgroups), single tokens and portions
+@pytest.mark.parametrize("heads,kv_heads,hd", [(8, 8, 128), (12, 12, 48), (4, 2, 64), (9, 3, 16), (28, 4, 32)])
+@pytest.mark.parametrize("requests,portion,lengths", [(41, 1, (24, 25)), (81, 1, (40, 64, 65)), (100, 1, (128, 129)), (60, 1, (256, 600)), (2, 5, (24, 25)), (4, 20, (64, 65)),
+                                                       (1, 70, (128, 129)), (1, 48, (300, 600)), (3, 30, (1100,))])
+def test_chunks_have_the_same_bits_whichever_kernel_takes_them(heads, kv_heads, hd, requests, portion, lengths):
+    k = kernels()
+    for length in lengths:
+        rng = np.random.default_rng(length + hd)
+        t, *_ = build_paged_case(rng, torch.float32, [length] * requests, [min(portion, length)] * requests, heads, kv_heads, hd, 16)
+        run = lambda **way: k.paged_attention_rowwise(t["q"], t["k"], t["v"], t["table"], t["seq"], t["pos"], hd ** -0.5, 0, heads, kv_heads, hd, longest=2048,
+                                                      usual=length, **way)
+        by_rows = run(split=False)
+        assert torch.equal(run(split=True), by_rows) and torch.equal(run(), by_rows), length
+
+
 # ---- gates of every size: where exp(-gate) leaves the numbers the quotient is the gate or nothing, in every kernel that forms one ----
 GATES = [-1.0, -20.0, -86.5, -87.5, -90.0, -100.0, -1e3, -1e13, -1e30, -3.3895313892515355e38, 1.0, 87.5, 1e3, 1e13, 1e30, 3.3895313892515355e38]
 CLAMP, SLOPE = 7.0, 1.702
