@@ -5,7 +5,7 @@ import numpy as np
 import pytest
 import torch
 
-from test_kernels_gpu import DEVICE, build_paged_case, kernels, reference_attention, to_bf16_exact, tolerance
+from test_kernels_gpu import DEVICE, build_paged_case, kernels, key_page_shape, reference_attention, to_bf16_exact, tolerance, value_page_shape
 
 pytestmark = pytest.mark.gpu
 
@@ -348,9 +348,9 @@ def test_decode_attention_reads_every_line_of_its_pages(heads, kv_heads, hd, pag
     np.testing.assert_allclose(out.float().cpu().numpy(), want.reshape(len(lengths), -1), **tolerance(torch.bfloat16))
 
 
-# ---- experts in large tiles: heights of 128, 192 and 256 rows, remainders of each, experts without a pair, more experts than a wave has lanes ----
+# ---- experts in large tiles, of 128 rows and one a workgroup: remainders, experts without a pair, ids that return their input ----
 @pytest.mark.parametrize("n,width,ff,experts,top,identity,gated", [
-    (700, 128, 384, 3, 2, 0, True), (520, 256, 128, 2, 1, 1, True), (1300, 128, 264, 5, 2, 2, False), (400, 128, 128, 70, 3, 0, True),
+    (700, 128, 384, 3, 2, 0, True), (520, 256, 128, 2, 1, 1, True), (1300, 128, 264, 5, 2, 2, False),
     (129, 384, 128, 1, 1, 0, True), (3000, 128, 256, 4, 2, 1, True)])
 def test_experts_in_large_tiles(n, width, ff, experts, top, identity, gated):
     """Against the kernels that take a pair at a time, whose sums have another order; and the bits of the same pairs in steps too small for
@@ -370,9 +370,78 @@ def test_experts_in_large_tiles(n, width, ff, experts, top, identity, gated):
         one_by_one = k.moe_experts(x, ids, weights, gate_up, down, on_input, grouped=False, **options)
         assert float((tiled - one_by_one).abs().max()) < 0.02 * float(one_by_one.abs().max())      # the inner values are rounded from sums in another order
         few = 100 * experts // top       # below 128 pairs an expert
-        if experts * (-(-ff // 128)) < 512:
-            small = k.moe_experts(x[:few], ids[:few].contiguous(), weights[:few].contiguous(), gate_up, down, on_input, grouped=True, **options)
-            assert torch.equal(small, tiled[:, :few])
+        small = k.moe_experts(x[:few], ids[:few].contiguous(), weights[:few].contiguous(), gate_up, down, on_input, grouped=True, **options)
+        assert few < n and torch.equal(small, tiled[:, :few])
+
+
+def tiling(counts, n_out, columns):
+    """The height that the kernel chooses for experts of ``counts`` pairs, and how many tiles that makes: the first of those whose rounds of 256
+    workgroups cost least, a round as much as a stage of its rows and of 256 of the weight."""
+    blocks, best = -(-n_out // columns), None
+    for height in (256, 192, 128):
+        tiles = sum(-(-count // height) for count in counts) * blocks
+        cost = -(-tiles // 256) * (height + 256)
+        if best is None or cost < best[0]:
+            best = (cost, height, tiles)
+    return best[1:]
+
+
+ENDS_OF_256 = [600, 577, 640, 641, 700, 704, 705, 768, 0, 767, 1, 650, 740, 600, 768, 690]      # last tiles of up to 128, 192 and 256 rows, and of one
+ENDS_OF_192 = [192, 129, 191, 0, 190, 128, 192, 1, 180, 192] * 3
+ENDS_OF_128 = [128] * 29 + [129]
+MANY_EXPERTS = [(140 * e) % 331 if e % 9 else 0 for e in range(70)]          # experts on both sides of a wave's lanes, some without a pair
+
+
+# which product has more tiles than there are workgroups, and their height: gate and up (or up alone), or down
+@pytest.mark.parametrize("counts,width,ff,gated,identity,walks,height", [
+    (ENDS_OF_256, 128, 2048, True, 0, "inner", 256), (ENDS_OF_256, 4096, 128, True, 37, "down", 256), (ENDS_OF_256, 128, 4096, False, 0, "inner", 256),
+    (ENDS_OF_192, 128, 2048, True, 0, "inner", 192), (ENDS_OF_192, 4096, 128, True, 0, "down", 192),
+    (ENDS_OF_128, 128, 2048, True, 0, "inner", 128), (ENDS_OF_128, 4096, 128, False, 5, "down", 128), (MANY_EXPERTS, 128, 896, True, 40, "inner", 192)])
+def test_experts_in_more_large_tiles_than_workgroups(counts, width, ff, gated, identity, walks, height):
+    """A workgroup goes from tile to tile, whose rows and results take the LDS of the tile before: against the kernels that take a pair at a time, and the
+    bits of fewer pairs, which smaller tiles take."""
+    k, experts = kernels(), len(counts)
+    inner, outer = tiling(counts, ff, 128 if gated else 256), tiling(counts, width, 256)
+    chosen, tiles = inner if walks == "inner" else outer
+    assert chosen == height and tiles > 256 and sum(counts) + identity >= 128 * experts
+    generator = torch.Generator(device=DEVICE).manual_seed(width + ff + experts)
+    normal = lambda *shape: torch.randn(shape, generator=generator, device=DEVICE)
+    ids = torch.cat([torch.full((count,), e, dtype=torch.int32) for e, count in enumerate([*counts, identity])]).to(DEVICE)
+    ids = ids[torch.randperm(len(ids), generator=generator, device=DEVICE)][:, None].contiguous()
+    n = ids.shape[0]
+    x, weights = normal(n, width).to(torch.bfloat16), normal(n, 1).abs() + 0.2
+    gate_up, down = ((normal(experts, rows, terms) * terms ** -0.5).to(torch.bfloat16) for rows, terms in (((2 if gated else 1) * ff, width), (width, ff)))
+    for on_input in (False, True) if identity == 0 else (False,):
+        run = lambda rows, grouped: k.moe_experts(x[:rows], ids[:rows], weights[:rows], gate_up, down, on_input, grouped=grouped, gated=gated, activation="silu",
+                                                  identity=1 if identity else 0)
+        tiled, one_by_one = run(n, True), run(n, False)
+        assert float((tiled - one_by_one).abs().max()) < 0.02 * float(one_by_one.abs().max())      # the inner values are rounded from sums in another order
+        few = 128 * experts - 1
+        assert few < n and experts * -(-max((2 if gated else 1) * ff, width) // 256) < 512        # the smaller tiles take so few
+        assert torch.equal(run(few, True), tiled[:, :few])
+
+
+def test_queries_keys_and_values_of_more_tiles_than_workgroups():
+    """The tiled product's epilogue with rotation and pages where a workgroup takes a second tile (17 x 18 of 128 rows), against tiles of 256 (9 x 18), which fit one
+    round, and against the two kernels it replaces."""
+    k, generator = kernels(), torch.Generator(device=DEVICE).manual_seed(5)
+    heads, kv_heads, hd, hidden, m, page = 28, 4, 128, 64, 2100, 16
+    total = (heads + 2 * kv_heads) * hd
+    normal = lambda *shape: torch.randn(shape, generator=generator, device=DEVICE)
+    x, bias = normal(m, hidden).to(torch.bfloat16), normal(total)
+    packed = k.pack_weight((normal(total, hidden) * 0.2).to(torch.bfloat16), row_order=k.rotary_pair_order(heads, kv_heads, hd, hd // 2))
+    table = k.rope_table(torch.arange(m, dtype=torch.int32, device=DEVICE), 1e4 ** -(torch.arange(0, hd, 2, device=DEVICE, dtype=torch.float64) / hd))
+    slots = torch.randperm(m, generator=generator, device=DEVICE).to(torch.int32)
+    pages = lambda: [torch.full(shape(-(-m // page), kv_heads, page, hd), 7.0, dtype=torch.bfloat16, device=DEVICE) for shape in (key_page_shape, value_page_shape)]
+    results = []
+    for rows in (128, 256):
+        kept = pages()
+        results.append([k.gemm_tiled_qkv(x, packed, bias, slots, table, *kept, heads, kv_heads, hd, page, tile_rows=rows), *kept])
+    kept = pages()
+    results.append([k.qkv_rope_store(k.gemm_tiled(x, packed, total, "f32"), bias, torch.arange(m, dtype=torch.int32, device=DEVICE), slots, None, *kept, heads, kv_heads,
+                                     hd, page, torch.bfloat16, pair_order=True, cos_sin=table), *kept])
+    for other in results[1:]:
+        assert all(torch.equal(a, b) for a, b in zip(results[0], other))
 
 
 @pytest.mark.parametrize("heads,kv_heads,hd,window", [(14, 2, 64, 0), (4, 2, 48, 100), (4, 1, 128, 0), (2, 1, 256, 33)])

@@ -267,7 +267,7 @@ def attention_through_mfma(q, k, v, scale, table, longest, sink, portions_of, pa
         requests = device(np.zeros(count), torch.int32)
         if count == 1:
             kernels.paged_attention_decode(queries, k_pages, v_pages, block_table, requests, positions, scale, 0, heads, kv_heads, dim,
-                                           splits or kernels.decode_splits(1, kv_heads, position + 1), out=out, extras=extras)
+                                           splits or kernels.decode_parts(1, kv_heads, position + 1, dim), out=out, extras=extras)
         else:
             tiles = [(0, offset, min(kernels.QUERY_TILE, count - offset), position + offset) for offset in range(0, count, kernels.QUERY_TILE)]
             plan = device(np.asarray(kernels.pair_query_tiles(tiles)).reshape(-1, 5), torch.int32)

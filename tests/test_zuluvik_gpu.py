@@ -279,12 +279,16 @@ def test_differential_attention(heads, kv_heads, dim, vdim, n_taps, n, mfma):
             assert np.array_equal(again, got), portions_of      # a row does not depend on how the request was cut
 
 
-@pytest.mark.parametrize("heads,kv_heads,dim,vdim,n", [(2, 1, 16, 32, 1100), (3, 1, 24, 20, 5200)])
-def test_difference_where_the_splits_meet(heads, kv_heads, dim, vdim, n):
-    """Decoding over so many keys that they go to several workgroups, whose results meet in the kernel that combines the maps
-    (two splits, and more than eight of them)."""
+@pytest.mark.parametrize("heads,kv_heads,dim,vdim,n,splits", [(2, 1, 16, 32, 1100, 8), (3, 1, 24, 20, 5200, 10), (2, 1, 16, 32, 1100, 2), (3, 1, 24, 20, 1100, 3),
+                                                             (1, 1, 24, 20, 1100, 17)])
+def test_difference_where_the_splits_meet(heads, kv_heads, dim, vdim, n, splits, monkeypatch):
+    """Decoding over so many keys that they go to several workgroups, whose results meet eight at a time in the kernel that combines the maps: eight and ten as the
+    step chooses them, and, asked for, fewer than eight and a last round of one."""
     from microllm_rocm_amd.ops import kernels
-    assert kernels.decode_splits(1, kv_heads, n) == (2 if n == 1100 else 10)
+    if splits in (8, 10):
+        assert kernels.decode_parts(1, kv_heads, n, round_up(max(2 * dim, vdim), 16)) == splits
+    asked = []
+    monkeypatch.setattr(kernels, "decode_parts", lambda *sizes: asked.append(sizes) or splits)
     rng = np.random.default_rng(n)
     q, k, v = (as_bf16(rng.normal(size=shape)) for shape in ((n, heads, 2, dim), (n, kv_heads, 2, dim), (n, kv_heads, vdim)))
     q[n - 3:] *= 4.0        # the last queries single out a few keys
@@ -297,6 +301,7 @@ def test_difference_where_the_splits_meet(heads, kv_heads, dim, vdim, n):
             maps.append(torch.einsum("hj,jhd->hd", torch.softmax(s, -1), t64(v[:query + 1]).repeat_interleave(heads // kv_heads, 1)))
         want = (plain.rms(maps[0] - 0.4 * maps[1], 1e-5) * 0.4).numpy()
         assert np.abs(got[back] - want).max() < 0.03 * np.abs(want).max(), query
+    assert len(asked) == 3
 
 
 def test_differential_attention_on_plain_pages_in_bfloat16():
