@@ -509,6 +509,7 @@ def paged_attention_rowwise(q: torch.Tensor, k_cache: torch.Tensor, v_cache: tor
     _need(out.shape == q.shape, "attention output must have the queries' shape")
     capacity = block_table.shape[1] * page_size
     longest = capacity if longest is None else min(int(longest), capacity)
+    may_go_without = split is None and n_tokens * heads >= ROWWISE_SPLIT_BELOW     # such a step needs no workspace where there is no room for one
     if split is None:
         split = rowwise_splits(n_tokens, heads, kv_heads, head_dim, rowwise_chunks(max(longest, 1), window), q.dtype, block_table.shape[0],
                                longest if usual is None else min(int(usual), longest))
@@ -516,8 +517,13 @@ def paged_attention_rowwise(q: torch.Tensor, k_cache: torch.Tensor, v_cache: tor
     usual_chunks = rowwise_chunks(max(min(int(usual), longest), 1), window) if split and usual is not None else 0
     part_o = part_ml = None
     if chunks > 1:
-        part_o = torch.empty((n_tokens, heads, chunks, head_dim), dtype=torch.float32, device=q.device)
-        part_ml = torch.empty((n_tokens, heads, chunks, 2), dtype=torch.float32, device=q.device)
+        try:
+            part_o = torch.empty((n_tokens, heads, chunks, head_dim), dtype=torch.float32, device=q.device)
+            part_ml = torch.empty((n_tokens, heads, chunks, 2), dtype=torch.float32, device=q.device)
+        except torch.OutOfMemoryError:
+            if not may_go_without:
+                raise
+            chunks, part_o, part_ml = 0, None, None
     else:
         chunks = 0      # one chunk a row: the wave per row is the wave per chunk
     _check(lib.mll_paged_attention_rowwise(_ptr(q), _code(q.dtype), _ptr(k_cache), _ptr(v_cache), _ptr(block_table),

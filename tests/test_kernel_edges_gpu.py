@@ -494,6 +494,30 @@ def test_chunks_have_the_same_bits_whichever_kernel_takes_them(heads, kv_heads, 
         assert torch.equal(run(split=True), by_rows) and torch.equal(run(), by_rows), length
 
 
+
+def test_a_step_that_can_go_without_a_workspace_does_where_there_is_no_room(monkeypatch):
+    k, rng = kernels(), np.random.default_rng(3)
+    heads, kv_heads, hd = 28, 4, 32
+    allocate = torch.empty
+
+    def full(*sizes, **options):
+        if sizes and isinstance(sizes[0], tuple) and len(sizes[0]) == 4:      # the chunks' results
+            raise torch.OutOfMemoryError("no room")
+        return allocate(*sizes, **options)
+
+    for requests in (80, 20):       # 2240 rows, and 560, which always had a workspace
+        t, *_ = build_paged_case(rng, torch.float32, [300] * requests, [1] * requests, heads, kv_heads, hd, 16)
+        run = lambda: k.paged_attention_rowwise(t["q"], t["k"], t["v"], t["table"], t["seq"], t["pos"], hd ** -0.5, 0, heads, kv_heads, hd)
+        want = run()
+        with monkeypatch.context() as patch:
+            patch.setattr(torch, "empty", full)
+            if requests == 80:
+                assert torch.equal(run(), want)
+            else:
+                with pytest.raises(torch.OutOfMemoryError):
+                    run()
+
+
 # ---- gates of every size: where exp(-gate) leaves the numbers the quotient is the gate or nothing, in every kernel that forms one ----
 GATES = [-1.0, -20.0, -86.5, -87.5, -90.0, -100.0, -1e3, -1e13, -1e30, -3.3895313892515355e38, 1.0, 87.5, 1e3, 1e13, 1e30, 3.3895313892515355e38]
 CLAMP, SLOPE = 7.0, 1.702
