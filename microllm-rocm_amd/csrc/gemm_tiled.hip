@@ -52,9 +52,10 @@ __global__ __launch_bounds__(kTiledThreads, 1) void gemm_tiled_kernel(const bf16
     constexpr int TILE_M = 32 * WM;
     constexpr int A_LOADS = 4 * WM;                       // a stage of A: 2 WM pieces of 16 rows, two loads of 8 rows each
     constexpr int A_TURNS = (A_LOADS + kTiledWaves - 1) / kTiledWaves;
-    // Two slots. In a slot: A as [2 WM pieces of 16 rows][row][8 places of 16 bytes], the row's chunk c of 8 elements
-    // at place c ^ (row / 2); then W as [16 tiles][2 k steps][1 KB in MFMA operand order]. Only the direct loads write
-    // this memory and only the asm reads read it.
+    // Two slots of A, each [2 WM pieces of 16 rows][row][8 places of 16 bytes], the row's chunk c of 8 elements at place c ^ (row / 2); then three of W, each
+    // [16 tiles][2 k steps][1 KB in MFMA operand order]. While stages are multiplied the direct loads alone write this memory and the asm reads alone read
+    // it. Gated results pass through it as rows: the workgroup meets before they are written (its reads of the last stage have arrived), before they
+    // are read, and, where it has another tile, before that one's loads go out.
     __shared__ __align__(16) bf16 slots[kStageElements];
 
     // Workgroups 8 apart in number run on one XCD, 32 of them at a time. The tiles of C are put in a row, blocks of

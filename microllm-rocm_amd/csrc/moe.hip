@@ -1145,6 +1145,7 @@ int mll_moe_grouped(const void* x, const int32_t* ids, const float* weights, int
         // Large tiles where the experts have pairs for them, or are many enough that their weights' tiles make two rounds of the compute units
         // (gate, up and down; 16 experts of 2048 x 2048, 4 of 20 choices: 400 tokens 129 and 139 us, 800 184 and 146, 3117 426 and 343, 6000 739 and
         // 559; 64 of 1024 x 2048, 6 choices: 400 tokens 243 and 214, 3117 524 and 398; 8 of 4096 x 2048, 2 choices: 400 tokens 138 and 141, 800 157 and 143).
+        // k is asked to be a multiple of 128 although the stages are of 64: reductions of an odd number of them have not been measured here.
         const bool fills = n_pairs >= 128 * static_cast<int64_t>(experts) || experts * ((w_rows + 255) / 256) >= 512;
         if (k % 128 == 0 && aligned && std::max(a_rows, w_rows) * row_bytes < (int64_t{1} << 32) && fills)
             return launch_moe_tiled(FORM, from, w, offsets, order, weights, n_out, k, to, top, n_tokens, weight_on_input, from_tokens,

@@ -1,6 +1,6 @@
 // The chosen experts' products for many (token, choice) pairs, in large tiles: the pairs lie in the order of their experts
 // (moe_sort_kernel in moe.hip), and a workgroup of 8 waves takes up to 256 pairs of one expert and 256 rows of its weight, with the main loop of
-// gemm_tiled.hip: stages of 64 of the reduction by direct loads into one of two LDS slots, the operands of a k step read from
+// gemm_tiled.hip: stages of 64 of the reduction by direct loads into LDS slots (two of A, three of W), the operands of a k step read from
 // LDS between the products of the step before. Here both sides are rows of memory, 8 rows of 128 bytes a load, and A's rows are taken from
 // wherever their tokens lie. Bound by the loads of a stage (64 KB, which a compute unit brings in 1.5 us) and by a tile's beginning and end, which
 // nothing overlaps: as many workgroups as compute units go from tile to tile, and the height of the tiles is chosen so that their rounds are done
