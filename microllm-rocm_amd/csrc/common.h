@@ -99,7 +99,8 @@ __device__ inline float gated_value(float g, float u, int act, float limit, floa
 // n / (1 + exp(-t)) to about an ulp, in fewer instructions than expf and a division: exp by the hardware's exp2 with what the product with
 // log2(e) loses put back, and a reciprocal refined once, for t up to 87 in size, where neither leaves the numbers. Beyond 87 the quotient is n; below -87,
 // where it is n exp(t), it goes on to nothing by a factor of its own, which is one otherwise: n has no bound, so a quotient that stayed at
-// exp(-87) would leave 5.6 of the lowest bfloat16. (The factor is free in rows that wait for memory; tiled gated products 397 -> 404 us and 38.4 -> 39.9.)
+// exp(-87) would leave 5.6 of the lowest bfloat16. (The factor is free in rows that wait for memory; it holds up tiles of
+// gated products, 413 -> 419 us and 38.4 -> 39.9, of which a look at a wave's gates that leaves it out gave back a half, and made experts' tiles slower.)
 __device__ inline float over_one_plus_exp(float n, float t) {
     constexpr float kLog2e = 1.44269502162933349609f, kLog2eRest = 1.92596299112661746887e-8f, kLn2 = 0.69314718055994530942f;
     constexpr float k87Log2e = 125.514473f;     // not less than 87 kLog2e

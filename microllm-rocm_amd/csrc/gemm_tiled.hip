@@ -14,8 +14,8 @@
 // products up for a third of a stage. The reads and the products are volatile asm, which pins their order;
 // the compiler neither sees the reads (and so orders nothing against the loads in flight) nor moves the products.
 // Bound by the loads: a compute unit brings a stage's 64 KB in 1.3 to 1.5 us. Gated, before and with the loads between the products, results stored
-// as whole rows, and as many workgroups as compute units going from tile to tile: 8192 x 37888 x 3584 1747 -> 1622 us (1.37 PFLOP/s),
-// 16301 rows 3599 -> 3215, 2048 rows 455 -> 411, 8192 x 16384 x 2048 440 -> 397, 2048 x 9728 x 896 45.7 -> 37.0.
+// as whole rows, and as many workgroups as compute units going from tile to tile: 8192 x 37888 x 3584 1771 -> 1660 us (1.34 PFLOP/s),
+// 16301 rows 3621 -> 3284, 2048 rows 468 -> 433, 8192 x 16384 x 2048 456 -> 430, 2048 x 9728 x 896 45.8 -> 41.4.
 // Workgroups are numbered so that the 32 that run together on one of the 8 XCDs (each with a second-level cache of
 // its own) own about 4 x 8 neighbouring tiles of C, and so share their rows of A and of W there, and so that every
 // XCD gets the same number of tiles.
