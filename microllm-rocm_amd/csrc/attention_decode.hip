@@ -24,7 +24,12 @@ constexpr int kPlain = 0, kExtras = 1, kBiased = 2;
 
 constexpr int kDecodeWaves = 4;
 constexpr int kDecodeThreads = kDecodeWaves * kWave;
-constexpr int kStreamedFrom = 256;      // workgroups from which the pages are read past the caches: see load_piece
+
+// Workgroups from which the pages are read past the caches, by the head size and how many positions the step is planned for: see load_piece.
+static int streamed_from(int head_dim, int positions) {
+    if (head_dim > 128 || positions < 8192) return 256;
+    return head_dim == 128 ? 128 : 192;
+}
 
 typedef unsigned uintx4 __attribute__((ext_vector_type(4)));
 
@@ -32,7 +37,9 @@ typedef unsigned uintx4 __attribute__((ext_vector_type(4)));
 // compute unit the pages then come in at 6.3 instead of 5.6 TB/s (64 requests of 3000 positions 70.4 and 62.6 us). With fewer it is the faster way only where
 // all of them have as much to read (12 requests of 4096 positions in 5 splits, 28 heads of 128 over 4, 26.2 and 24.3 us) and costs as much in ragged
 // steps, whose pages the last cache holds between two passes (4 requests from 3072 down to 230 positions in 8 splits 10.8 and 11.9, 32 of 384 down to
-// 20 7.8 and 8.8, 768 beside 31 of 70 10.0 and 11.7).
+// 20 7.8 and 8.8, 768 beside 31 of 70 10.0 and 11.7), until the keys are many: planned for 8192, 12 of 8192, from 6144 down to 310, and three of 6144 beside nine of 70
+// 43.2 and 39.8, 23.1 and 22.5, 22.0 and 21.2, with two (128 workgroups) 15.7 and 14.9, 13.6 and 13.5, 13.0 and 13.0; with heads of 64, 12 in 10 splits (240) 17.8 and
+// 16.3, 12.3 and 12.1, 11.1 and 11.6, but 4 in 16 splits (128) 12.5 and 11.8, 9.9 and 10.3, 9.7 and 10.1.
 template <bool STREAM>
 __device__ inline uint4 load_piece(const bf16* from) {
     if (STREAM) {
@@ -466,7 +473,8 @@ static int launch_decode(const void* q, const void* k_cache, const void* v_cache
     const int group = heads / kv_heads;
     const MllAttentionExtras given = extras ? *extras : MllAttentionExtras{nullptr, 0, nullptr, 1.0f, 0};
     const dim3 grid(n_tokens * (kv_heads * ((group + 15) / 16)), n_splits);
-    const bool stream_pages = static_cast<int64_t>(grid.x) * grid.y >= kStreamedFrom;
+    const int reach = window > 0 ? window : given.chunk > 0 ? given.chunk : table_width * page_size;
+    const bool stream_pages = static_cast<int64_t>(grid.x) * grid.y >= streamed_from(HD_TILES * 16, min(reach, table_width * page_size));
     const auto launch = [&](auto streamed, auto form) {
         paged_attention_decode_kernel<HD_TILES, decltype(streamed)::value, decltype(form)::value><<<grid, kDecodeThreads, 0, stream>>>(
             static_cast<const bf16*>(q), static_cast<const bf16*>(k_cache), static_cast<const bf16*>(v_cache), block_table,

@@ -348,6 +348,18 @@ def test_decode_attention_reads_every_line_of_its_pages(heads, kv_heads, hd, pag
     np.testing.assert_allclose(out.float().cpu().numpy(), want.reshape(len(lengths), -1), **tolerance(torch.bfloat16))
 
 
+
+@pytest.mark.parametrize("heads,kv_heads,hd,tokens,splits", [(28, 4, 128, 4, 8), (14, 2, 64, 12, 8)])
+def test_decode_attention_of_long_steps_has_the_bits_of_fewer_tokens(heads, kv_heads, hd, tokens, splits):
+    """128 and 192 workgroups of a step planned for 8192 positions, from which pages are read past the caches, and one token less."""
+    rng, k = np.random.default_rng(hd), kernels()
+    t, *_ = build_paged_case(rng, torch.bfloat16, [8100] + [70] * (tokens - 1), [1] * tokens, heads, kv_heads, hd, 16)
+    table = torch.full((tokens, 512), -1, dtype=torch.int32, device=DEVICE)
+    table[:, :t["table"].shape[1]] = t["table"]
+    run = lambda n: k.paged_attention_decode(t["q"][:n], t["k"], t["v"], table, t["seq"][:n], t["pos"][:n], hd ** -0.5, 0, heads, kv_heads, hd, splits)
+    assert torch.equal(run(tokens)[:tokens - 1], run(tokens - 1))
+
+
 # ---- experts in large tiles, of 128 rows and one a workgroup: remainders, experts without a pair, ids that return their input ----
 @pytest.mark.parametrize("n,width,ff,experts,top,identity,gated", [
     (700, 128, 384, 3, 2, 0, True), (520, 256, 128, 2, 1, 1, True), (1300, 128, 264, 5, 2, 2, False),
