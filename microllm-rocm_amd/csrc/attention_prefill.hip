@@ -37,6 +37,7 @@ typedef float floatx16 __attribute__((ext_vector_type(16)));
 
 constexpr int kPrefillWaves = 8;
 constexpr int kPrefillThreads = kPrefillWaves * kWave;
+constexpr int kBufferFlags = 0x00027000;    // a raw buffer of 32-bit words
 constexpr int kPrefillTile = 128;     // tokens of one tile: four blocks of 32, a wave each
 
 union PFrag8 {
@@ -219,54 +220,62 @@ __global__ __launch_bounds__(kPrefillThreads, 1) void paged_attention_prefill_ke
         const int tile_key = block * BLOCK_KEYS + 16 * tile_of(pass);
         return (FULL_PASSES || tile_of(pass) < BLOCK_TILES) && tile_key <= group_last && (inside(block) || tile_seen(tile_key));
     };
-    // Pages mostly hold a power of two of tiles (often one): then the page of a tile is a shift, else a division.
-    // The choice is made once per block, not per tile.
-    auto page_index = [&](auto shift_tag, int tile_index) {
-        return decltype(shift_tag)::value ? tile_index >> page_shift : tile_index / tiles_per_page;
-    };
-    auto tile_in_its_page = [&](auto shift_tag, int tile_index) {
-        return decltype(shift_tag)::value ? tile_index & (tiles_per_page - 1) : tile_index % tiles_per_page;
-    };
     // The pages of a block's tiles are looked up one block ahead of the tiles themselves, so that no load waits
-    // for another. The look-up is a load of the vector unit also where the whole wave asks for one entry: those
-    // are counted with the loads into LDS and have arrived when these have, whereas a load of the scalar unit
-    // would be waited for by the first read from LDS that follows it.
-    int pages[PASSES];
-    int no_lane = 0;
-    asm volatile("v_mov_b32 %0, 0" : "=v"(no_lane));      // zero, but the compiler cannot tell: keeps the address per lane
-    auto look_up_with = [&](auto shift_tag, int block) __attribute__((always_inline)) {
-        const bool whole = FULL_PASSES && inside(block);      // the usual case: every tile of the block, no questions
+    // for another; where a wave's lanes stay within one tile, one load looks up the pages of all its passes, a lane
+    // each. The look-up is a load of the vector unit: those are counted with the loads into LDS and have arrived when
+    // these have, whereas a load of the scalar unit would be waited for by the first read from LDS that follows it.
+    constexpr int LOOKUPS = UNIFORM ? 1 : PASSES;
+    int pages[LOOKUPS];      // -1: the tile is not brought in
+    const int lane_pass = lane % PASSES;
+    auto look_up = [&](int block) __attribute__((always_inline)) {
 #pragma unroll
-        for (int pass = 0; pass < PASSES; ++pass) {
-            const int tile_index = block * BLOCK_TILES + tile_of(pass);
-            pages[pass] = -1;
-            if (whole || wanted(block, pass)) pages[pass] = table[page_index(shift_tag, tile_index) + no_lane];
+        for (int i = 0; i < LOOKUPS; ++i) {
+            const int pass = UNIFORM ? lane_pass : i;
+            const int tile_index = block * BLOCK_TILES + (UNIFORM ? (pass * kPrefillThreads + wave_chunk) / TILE_CHUNKS : tile_of(i));
+            const int tile_key = 16 * tile_index;
+            const bool want = (FULL_PASSES || tile_index - block * BLOCK_TILES < BLOCK_TILES) && tile_key <= group_last && tile_seen(tile_key);
+            pages[i] = -1;
+            if (want) pages[i] = table[page_shift >= 0 ? tile_index >> page_shift : tile_index / tiles_per_page];
         }
     };
-    auto look_up = [&](int block) __attribute__((always_inline)) {
-        if (page_shift >= 0) look_up_with(std::true_type{}, block);
-        else look_up_with(std::false_type{}, block);
-    };
-    auto fetch_with = [&](auto shift_tag, int block, bf16* stage) __attribute__((always_inline)) {      // after look_up(block)
+    // The loads are buffer loads: a global load into LDS is encoded as a flat one, and while such a load is under way the compiler waits for all reads
+    // from LDS and all loads, not for the ones it needs (16301 tokens, 28 heads of 128 over 4: 2.34 -> 2.25 ms).
+    auto fetch = [&](int block, bf16* stage) __attribute__((always_inline)) {      // after look_up(block)
+        if constexpr (UNIFORM) {
+            const int tile_index = block * BLOCK_TILES + (lane_pass * kPrefillThreads + wave_chunk) / TILE_CHUNKS;
+            const int tile_in_page = page_shift >= 0 ? tile_index & (tiles_per_page - 1) : tile_index % tiles_per_page;
+            const int64_t from = 2 * (pages[0] * page_elements + head_elements + tile_in_page * TILE_ELEMENTS);      // in bytes
+            const unsigned from_low = static_cast<unsigned>(from), from_high = static_cast<unsigned>(from >> 32);
 #pragma unroll
-        for (int pass = 0; pass < PASSES; ++pass) {
-            const int tile_index = block * BLOCK_TILES + tile_of(pass);
-            const int tile_in_page = tile_in_its_page(shift_tag, tile_index);
-            const int page = UNIFORM ? __builtin_amdgcn_readfirstlane(pages[pass]) : pages[pass];
-            if (page >= 0) {
-                const int64_t tile_start = page * page_elements + head_elements + tile_in_page * TILE_ELEMENTS;
+            for (int pass = 0; pass < PASSES; ++pass) {
+                if (__builtin_amdgcn_readlane(pages[0], pass) < 0) continue;
+                const uint64_t start = (static_cast<uint64_t>(static_cast<unsigned>(__builtin_amdgcn_readlane(from_high, pass))) << 32) +
+                                       static_cast<unsigned>(__builtin_amdgcn_readlane(from_low, pass)) +
+                                       static_cast<unsigned>(16 * ((pass * kPrefillThreads + wave_chunk) % TILE_CHUNKS));
+                char* key_piece = reinterpret_cast<char*>(const_cast<bf16*>(k_cache)) + start;
+                char* value_piece = reinterpret_cast<char*>(const_cast<bf16*>(v_cache)) + start;
+                const auto key_rsrc = __builtin_amdgcn_make_buffer_rsrc(key_piece, 0, kWave * 16, kBufferFlags);
+                const auto value_rsrc = __builtin_amdgcn_make_buffer_rsrc(value_piece, 0, kWave * 16, kBufferFlags);
+                bf16* key_place = stage + (pass * kPrefillThreads + wave_chunk) * 8;
+                bf16* value_place = key_place + HALF_CHUNKS * 8;
+                __builtin_amdgcn_raw_ptr_buffer_load_lds(key_rsrc, key_place, 16, lane * 16, 0, 0, 0);
+                __builtin_amdgcn_raw_ptr_buffer_load_lds(value_rsrc, value_place, 16, lane * 16, 0, 0, 0);
+            }
+        } else {
+#pragma unroll
+            for (int pass = 0; pass < PASSES; ++pass) {
+                if (pages[pass] < 0) continue;
+                const int tile_index = block * BLOCK_TILES + tile_of(pass);
+                const int tile_in_page = page_shift >= 0 ? tile_index & (tiles_per_page - 1) : tile_index % tiles_per_page;
+                const int64_t tile_start = pages[pass] * page_elements + head_elements + tile_in_page * TILE_ELEMENTS;
+                bf16* key_place = stage + (pass * kPrefillThreads + wave_chunk) * 8;
                 const bf16* key_piece = k_cache + tile_start + piece_of(pass) * 8;
                 const bf16* value_piece = v_cache + tile_start + piece_of(pass) * 8;
-                bf16* key_place = stage + (pass * kPrefillThreads + wave_chunk) * 8;      // the lane's 16 bytes follow by themselves
                 bf16* value_place = key_place + HALF_CHUNKS * 8;
                 __builtin_amdgcn_global_load_lds(key_piece, key_place, 16, 0, 0);
                 __builtin_amdgcn_global_load_lds(value_piece, value_place, 16, 0, 0);
             }
         }
-    };
-    auto fetch = [&](int block, bf16* stage) __attribute__((always_inline)) {
-        if (page_shift >= 0) fetch_with(std::true_type{}, block, stage);
-        else fetch_with(std::false_type{}, block, stage);
     };
     // A block at an end of what the tile's tokens see, once it lies in LDS: values at positions that no token
     // sees may be stale memory, and the places of tiles that were not brought in hold what was there before.
@@ -442,6 +451,124 @@ __global__ __launch_bounds__(kPrefillThreads, 1) void paged_attention_prefill_ke
             }
     };
 
+    // A block that the wave's tokens see whole, as two runs of 64 keys whose work overlaps within the wave: its matrix instructions are issued in one
+    // order (run 0's scores, run 1's scores, run 0's values, run 1's values), every operand read from LDS kAhead products before its use, and between
+    // run 1's scores and between run 0's values stand the weights (exponentials, sums, roundings) of run 0 and run 1. The numbers are process_keys' own,
+    // run by run. The order is the source's: the empty asm statements and the scheduling barriers keep the compiler from gathering the
+    // exponentials in front of the products, where nothing overlaps them. 16301 tokens, 28 heads of 128 over 4: 2.25 -> 2.12 ms; 2048 tokens 59 -> 56 us.
+    constexpr bool WHOLE_BLOCKS = !EXTRA && STEPS == 4;      // (with biases and caps the registers do not suffice: 71 -> 79 us)
+    auto process_block = [&](const bf16* stage) __attribute__((always_inline)) {
+        constexpr int SCORES = 2 * K_STEPS, VALUES = 4 * D_BLOCKS, PRODUCTS = 2 * (SCORES + VALUES);
+        constexpr int kAhead = 4, RING = kAhead + 1;
+        constexpr int PAIRS = 16;           // of a run's weights, a lane
+        floatx16 s[2][2];
+        PFrag8 p_frag[2][4];
+        PFrag8 ring[RING];
+        float rescale = 1.0f, step_sum = 0.0f, pending[2] = {0.0f, 0.0f};
+        const bf16* k_rows = stage + (column / 16) * TILE_ELEMENTS + (half * 16 + key_of_row % 16) * 8;
+        const bf16* v_rows = stage + HALF_CHUNKS * 8 + column * 8 + half * 256;
+        auto read = [&](int j) __attribute__((always_inline)) {      // product j's operand
+            PFrag8& place = ring[j % RING];
+            if (j < 2 * SCORES) {
+                const int run = j / SCORES, at = j % SCORES;        // the run's two 32s by turns
+                place.raw = *reinterpret_cast<const uint4*>(k_rows + (4 * run + 2 * (at % 2)) * TILE_ELEMENTS + (at / 2) * 256);
+            } else if (j < PRODUCTS) {
+                const int t = (j - 2 * SCORES) / D_BLOCKS, d = (j - 2 * SCORES) % D_BLOCKS;
+                if (HD % 32 == 0 || d < D_BLOCKS - 1) {
+                    place.raw = *reinterpret_cast<const uint4*>(v_rows + t * TILE_ELEMENTS + d * 512);
+                } else {
+                    place.raw = make_uint4(0, 0, 0, 0);
+                    if (column < 16)
+                        place.raw = *reinterpret_cast<const uint4*>((stage + (half * 16 + column) * 8) + (HALF_CHUNKS * 8 + t * TILE_ELEMENTS + d * 512));
+                }
+            }
+        };
+        auto multiply = [&](int j) __attribute__((always_inline)) {
+            read(j + kAhead);
+            if (j < 2 * SCORES) {
+                const int at = j % SCORES;
+                floatx16& sum = s[j / SCORES][at % 2];
+                if (at < 2) {
+#pragma unroll
+                    for (int i = 0; i < 16; ++i) sum[i] = 0.0f;
+                }
+                sum = __builtin_amdgcn_mfma_f32_32x32x16_bf16(ring[j % RING].v, q_frag[at / 2].v, sum, 0, 0, 0);
+                asm volatile("" : "+v"(sum));
+            } else {
+                const int t = (j - 2 * SCORES) / D_BLOCKS;
+                floatx16& sum = o_acc[(j - 2 * SCORES) % D_BLOCKS];
+                sum = __builtin_amdgcn_mfma_f32_32x32x16_bf16(ring[j % RING].v, p_frag[t / 4][t % 4].v, sum, 0, 0, 0);
+                asm volatile("" : "+v"(sum));
+            }
+        };
+        auto settle = [&](int run) __attribute__((always_inline)) {      // the running maximum over the run's scores
+            float tile_max = fmaxf(fmaxf(s[run][0][0], s[run][0][1]), s[run][0][2]);
+#pragma unroll
+            for (int i = 3; i < 15; i += 2) tile_max = fmaxf(fmaxf(tile_max, s[run][0][i]), s[run][0][i + 1]);
+            tile_max = fmaxf(tile_max, s[run][0][15]);
+#pragma unroll
+            for (int i = 0; i < 16; i += 2) tile_max = fmaxf(fmaxf(tile_max, s[run][1][i]), s[run][1][i + 1]);
+            rescale = 1.0f;
+            if (__any(tile_max > running_max)) {
+                tile_max = reduce_lanes_32_apart(tile_max, [](float x, float y) { return fmaxf(x, y); });
+                const float new_max = fmaxf(running_max, tile_max);
+                running_offset = -new_max * scale_log2;
+                rescale = new_max == running_max ? 1.0f : __builtin_amdgcn_exp2f(fmaf(running_max, scale_log2, running_offset));
+                running_max = new_max;
+            }
+            step_sum = 0.0f;
+        };
+        auto weigh = [&](int run, int pair) __attribute__((always_inline)) {      // a pair of weights is begun, the pair before it finished
+            if (pair > 0) {
+                const int i = 2 * (pair - 1);
+                step_sum += pending[0];
+                step_sum += pending[1];
+                PFrag8& place = p_frag[run][i / 8];
+                place.v[i % 8] = static_cast<__bf16>(pending[0]);
+                place.v[i % 8 + 1] = static_cast<__bf16>(pending[1]);
+            }
+            if (pair < PAIRS) {
+                asm volatile("" : "+v"(running_offset));
+#pragma unroll
+                for (int e = 0; e < 2; ++e)
+                    pending[e] = __builtin_amdgcn_exp2f(fmaf(s[run][pair / 8][2 * (pair % 8) + e], scale_log2, running_offset));
+                asm volatile("" : "+v"(pending[0]), "+v"(pending[1]));
+            }
+        };
+#pragma unroll
+        for (int j = 0; j < kAhead; ++j) read(j);
+        __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+        for (int j = 0; j < SCORES; ++j) {
+            multiply(j);
+            __builtin_amdgcn_sched_barrier(0);
+        }
+#pragma unroll
+        for (int run = 0; run < 2; ++run) {
+            const int first = run == 0 ? SCORES : 2 * SCORES, rest = (run == 0 ? SCORES : VALUES) - 1;
+            multiply(first);      // runs while the maximum is looked for
+            __builtin_amdgcn_sched_barrier(0);
+            settle(run);
+#pragma unroll
+            for (int j = 0; j < rest; ++j) {
+                multiply(first + 1 + j);
+#pragma unroll
+                for (int pair = j * (PAIRS + 1) / rest; pair < (j + 1) * (PAIRS + 1) / rest; ++pair) weigh(run, pair);
+                __builtin_amdgcn_sched_barrier(0);
+            }
+            running_sum = running_sum * rescale + step_sum;
+            if (__any(rescale != 1.0f)) {
+#pragma unroll
+                for (int d = 0; d < D_BLOCKS; ++d) o_acc[d] *= rescale;
+            }
+        }
+#pragma unroll
+        for (int j = 2 * SCORES + VALUES; j < PRODUCTS; ++j) {
+            multiply(j);
+            __builtin_amdgcn_sched_barrier(0);
+        }
+    };
+
     auto next_seen = [&](int block) {      // the next block after this one of which something is seen
         ++block;
         while (block * BLOCK_KEYS <= group_last && !block_seen(block)) ++block;
@@ -460,23 +587,29 @@ __global__ __launch_bounds__(kPrefillThreads, 1) void paged_attention_prefill_ke
         }
         // Unrolled: every read from LDS then has an address of the stage plus a constant (an address that a loop
         // carries along would make every read wait for the loads on their way into the other stage).
+        const bool whole = WHOLE_BLOCKS && block_valid > 0 && (block + 1) * BLOCK_KEYS - 1 <= block_position && block * BLOCK_KEYS >= block_last_low;
+        if constexpr (WHOLE_BLOCKS) {
+            if (whole) process_block(stage);
+        }
+        if (!whole) {
 #pragma unroll
-        for (int pair = 0; pair < STEPS / 2; ++pair) {
-            const int key0 = block * BLOCK_KEYS + 64 * pair;
-            bool see[2], hidden[2];
-#pragma unroll
-            for (int r = 0; r < 2; ++r) {
-                see[r] = block_valid > 0 && key0 + 32 * r <= block_last && key0 + 32 * r + 31 >= block_low;
-                hidden[r] = key0 + 32 * r + 31 > block_position || key0 + 32 * r < block_last_low;
-            }
-            if (see[0] && see[1] && !hidden[0] && !hidden[1]) {
-                process_keys(std::false_type{}, std::integral_constant<int, 2>{}, stage, 2 * pair, key0);
-            } else {
+            for (int pair = 0; pair < STEPS / 2; ++pair) {
+                const int key0 = block * BLOCK_KEYS + 64 * pair;
+                bool see[2], hidden[2];
 #pragma unroll
                 for (int r = 0; r < 2; ++r) {
-                    if (!see[r]) continue;      // nothing of this run is visible to the wave
-                    if (hidden[r]) process_keys(std::true_type{}, std::integral_constant<int, 1>{}, stage, 2 * pair + r, key0 + 32 * r);
-                    else process_keys(std::false_type{}, std::integral_constant<int, 1>{}, stage, 2 * pair + r, key0 + 32 * r);
+                    see[r] = block_valid > 0 && key0 + 32 * r <= block_last && key0 + 32 * r + 31 >= block_low;
+                    hidden[r] = key0 + 32 * r + 31 > block_position || key0 + 32 * r < block_last_low;
+                }
+                if (see[0] && see[1] && !hidden[0] && !hidden[1]) {
+                    process_keys(std::false_type{}, std::integral_constant<int, 2>{}, stage, 2 * pair, key0);
+                } else {
+#pragma unroll
+                    for (int r = 0; r < 2; ++r) {
+                        if (!see[r]) continue;      // nothing of this run is visible to the wave
+                        if (hidden[r]) process_keys(std::true_type{}, std::integral_constant<int, 1>{}, stage, 2 * pair + r, key0 + 32 * r);
+                        else process_keys(std::false_type{}, std::integral_constant<int, 1>{}, stage, 2 * pair + r, key0 + 32 * r);
+                    }
                 }
             }
         }

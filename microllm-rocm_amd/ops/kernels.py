@@ -952,8 +952,7 @@ def pair_query_tiles(tiles: Sequence[Tuple[int, int, int, int]], adjacent: bool 
 
     A tile's work grows with its position (it sees every earlier key), so of one request's tiles the last goes
     with the first, the last but one with the second and so on: every workgroup of a request then walks about as
-    many keys. With ``adjacent`` neighbours go together instead: under a window every tile sees about as many keys,
-    and neighbours see nearly the same ones. A request's odd tile goes alone."""
+    many keys. With ``adjacent`` neighbours go together instead, which see nearly the same keys. A request's odd tile goes alone."""
     by_request: dict = {}
     for tile in tiles:
         by_request.setdefault(tile[0], []).append(tile)

@@ -30,9 +30,11 @@ class QueryTilePlanner:
     decode kernel. In a step of single tokens only there is nothing to plan: the decode kernel takes every row.
 
     Which two tiles share a workgroup: a late tile of a prompt with an early one, so that all workgroups walk about
-    as many keys; under a window neighbours, which then read nearly the same keys. (Neighbours for long prompts
-    without a window, the longest workgroups first, were measured too: a 16384-token prompt takes 3.0 instead of
-    2.6 ms a layer that way.)
+    as many keys; under a window neighbours, which then read nearly the same keys; and neighbours too where the step has more
+    workgroups (of the ``heads`` query heads) than compute units. Two neighbours walk their keys together, a late and an early tile
+    for the early one's keys only, so neighbours' workgroups bring in two thirds of the blocks of keys, and started longest first
+    they end together once there is more than a round of them (28 heads of 128: 3000 tokens, 336 workgroups, 131 -> 104 us, 16301 2.13 ->
+    1.87 ms; in one round the last of a prompt's workgroups is the step's time: 2048 tokens, 224 workgroups, 56 -> 70 us).
 
     Where the tiles of 128 would give fewer workgroups (of the ``heads`` query heads) than half the compute units, requests of more than one such
     tile have tiles of 64 queries: twice the workgroups, with one wave a SIMD instead of two, which share its exponentials (a pass of
@@ -54,6 +56,10 @@ class QueryTilePlanner:
         half = 0 < 2 * pairs * self.heads <= kernels.COMPUTE_UNITS
         return [kernels.QUERY_TILE // 2 if half and count > kernels.QUERY_TILE else kernels.QUERY_TILE for count in counts]
 
+    def neighbours(self, counts):
+        """Whether neighbouring tiles share a workgroup, by how many tokens each request brings."""
+        return self.windowed or self.heads * sum((-(-count // kernels.QUERY_TILE) + 1) // 2 for count in counts) > kernels.COMPUTE_UNITS
+
     def plan(self, host):
         counts, cu = host.counts, host.cu
         if host.single_tokens_only:
@@ -63,7 +69,8 @@ class QueryTilePlanner:
         tile_list = [(index, int(cu[index]) + offset, min(rows, counts[index] - offset), host.starts[index] + offset)
                      for index, rows in zip(portions, self.tile_rows([counts[index] for index in portions]))
                      for offset in range(0, counts[index], rows)]
-        tiles = np.asarray(kernels.pair_query_tiles(tile_list, adjacent=self.windowed), dtype=np.int32).reshape(-1, 5)
+        tiles = np.asarray(kernels.pair_query_tiles(tile_list, adjacent=self.neighbours([counts[index] for index in portions])),
+                           dtype=np.int32).reshape(-1, 5)
         single = np.asarray([cu[index] for index, count in enumerate(counts) if mixed and count == 1], dtype=np.int32)
         longest = max((host.totals[index] for index, count in enumerate(counts) if mixed and count == 1), default=0)
         return {"tiles": tiles, "single_tokens": single}, {"max_single_total": longest}

@@ -1,5 +1,7 @@
 """Host-side rules that need no GPU: how the products split their work, the row order of a rotary weight, and how
 parts take their tensors from the loader."""
+from types import SimpleNamespace
+
 import numpy as np
 import pytest
 import torch
@@ -205,6 +207,17 @@ def test_tiles_of_half_the_queries_where_whole_ones_leave_compute_units_idle():
     assert [planner.tile_rows([count])[0] for count in (2, 128, 129, 2048, 2304, 2305)] == [128, 128, 64, 64, 64, 128]
     assert planner.tile_rows([512, 128, 600]) == [64, 128, 64] and planner.tile_rows([300] * 5) == [128] * 5
     assert planner.key != QueryTilePlanner(False, 28).key
+
+
+def test_neighbouring_tiles_share_a_workgroup_where_a_step_has_more_than_a_round_of_them():
+    from microllm_rocm_amd.parts.attention import QueryTilePlanner
+    planner = QueryTilePlanner(False, 28)       # 9 workgroups a head: 252, 10: 280
+    assert [planner.neighbours(counts) for counts in ([2304], [2305], [1, 2303], [128] * 9, [128] * 10, [])] == [False, True, True, False, True, False]
+    assert not QueryTilePlanner(False).neighbours([100000]) and QueryTilePlanner(True).neighbours([2])
+    host = SimpleNamespace(counts=[2305], cu=[0, 2305], starts=[0], totals=[2305], single_tokens_only=False)
+    tiles = planner.plan(host)[0]["tiles"]
+    assert tiles[0].tolist() == [0, 2048, 128, 2176, 128] and tiles[1].tolist() == [0, 1792, 128, 1920, 128]
+    assert sorted(tiles[:, 2] + tiles[:, 4]) == [1] + [256] * 9
 
 
 @pytest.mark.parametrize("tokens,heads,kv_heads,head_dim,chunks,dtype,splits", [

@@ -5,7 +5,7 @@ import numpy as np
 import pytest
 import torch
 
-from test_kernels_gpu import DEVICE, build_paged_case, kernels, key_page_shape, reference_attention, to_bf16_exact, tolerance, value_page_shape
+from test_kernels_gpu import DEVICE, build_paged_case, kernels, key_page_shape, query_tile_list, reference_attention, to_bf16_exact, tolerance, value_page_shape
 
 pytestmark = pytest.mark.gpu
 
@@ -471,6 +471,22 @@ def test_prompts_in_tiles_of_half_the_queries_have_the_same_bits(heads, kv_heads
         pairs = torch.tensor(k.pair_query_tiles(tiles, adjacent=window > 0), dtype=torch.int32, device=DEVICE)
         results.append(k.paged_attention_prefill(t["q"], t["k"], t["v"], t["table"], pairs, t["pos"], hd ** -0.5, window, heads, kv_heads, hd))
     assert torch.equal(*results)
+
+
+@pytest.mark.parametrize("heads,kv_heads,hd,page_size", [(4, 2, 16, 16), (3, 1, 48, 48), (14, 2, 64, 32), (6, 3, 96, 16), (7, 7, 112, 64), (28, 4, 128, 16)])
+@pytest.mark.parametrize("window", [0, 333])
+def test_blocks_seen_whole_have_the_bits_of_their_runs(heads, kv_heads, hd, page_size, window):
+    """Blocks of 128 keys that a wave sees whole are worked on as one, overlapped; with extras (here a bias of nothing) every run of keys by itself. Portions begin
+    and end within blocks; the larger scores move their maxima by more."""
+    k = kernels()
+    lengths, counts = [700, 517, 131, 129, 258], [700, 130, 2, 129, 97]
+    for larger in (1.0, 16.0):
+        t, *_ = build_paged_case(np.random.default_rng(hd + window), torch.bfloat16, lengths, counts, heads, kv_heads, hd, page_size)
+        t["q"].mul_(larger)
+        tiles = torch.tensor(k.pair_query_tiles(query_tile_list(lengths, counts), adjacent=window > 0), dtype=torch.int32, device=DEVICE)
+        run = lambda **more: k.paged_attention_prefill(t["q"], t["k"], t["v"], t["table"], tiles, t["pos"], hd ** -0.5, window, heads, kv_heads, hd, **more)
+        nothing = k.AttentionExtras(bias=torch.zeros(2, heads, device=DEVICE))
+        assert torch.equal(run(), run(extras=nothing, out=torch.empty_like(t["q"]))), larger
 
 
 # ---- float32 attention by chunks, all heads of a kv head together: every head size, one head a kv head to more than 16, windows that begin in
