@@ -206,14 +206,16 @@ __global__ __launch_bounds__(1024) void gemm_skinny_kernel(
 
     // What the epilogue reads beside the product is on its way while the weight streams. The sums of squares for the
     // rows' factors (SCALED) go straight from memory into LDS, behind the waves' slots: [m][stride] as it lies in
-    // memory, 1 KB per wave-wide load.
+    // memory, 1 KB per wave-wide load: buffer loads, since a global load into LDS is encoded as a flat one, and while one may be
+    // under way the compiler waits for all loads of the weight instead of the block it multiplies.
     float* factor_shared = reduce_shared + static_cast<size_t>(waves - 1) * NT * MT * kWave * 4;
     if (SCALED && wave == 0) {
         const int count = m * extras.scale.stride;                  // floats; stride is a multiple of 4
+        const auto sums_rsrc = __builtin_amdgcn_make_buffer_rsrc(const_cast<float*>(extras.scale.sumsq), 0, count * 4, kBufferFlags);
         for (int first = 0; first < count; first += 256) {
             const int index = first + lane * 4;
             if (index < count)
-                __builtin_amdgcn_global_load_lds(extras.scale.sumsq + index, factor_shared + first, 16, 0, 0);
+                __builtin_amdgcn_raw_ptr_buffer_load_lds(sums_rsrc, factor_shared + first, 16, index * 4, 0, 0, 0);
         }
     }
     // Epilogue 3: the lane's 4 columns lie in one head (head_dim is a multiple of 16). In a query or key head the weight's
