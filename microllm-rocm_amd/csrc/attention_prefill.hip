@@ -37,7 +37,6 @@ typedef float floatx16 __attribute__((ext_vector_type(16)));
 
 constexpr int kPrefillWaves = 8;
 constexpr int kPrefillThreads = kPrefillWaves * kWave;
-constexpr int kBufferFlags = 0x00027000;    // a raw buffer of 32-bit words
 constexpr int kPrefillTile = 128;     // tokens of one tile: four blocks of 32, a wave each
 
 union PFrag8 {

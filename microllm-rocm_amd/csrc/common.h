@@ -59,6 +59,15 @@ __device__ inline float sum_lanes_16_apart(float value) {
     return reduce_lanes_16_apart(value, [](float a, float b) { return a + b; });
 }
 
+// BYTES (4 or 16) a lane from `base` (the same for the whole wave) and the lane's `offset` in bytes, straight into LDS at `place` and what follows it.
+// Buffer loads: a global load into LDS is encoded as a flat one, and while one is under way the compiler waits for every load and for every read
+// from LDS, not for those it needs. Nothing is checked: the caller's offsets lie within what `base` holds. (A macro: as a function's arguments
+// the places lose their address space.)
+constexpr int kBufferFlags = 0x00027000;    // a raw buffer of 32-bit words
+#define MLL_LOAD_INTO_LDS(BYTES, base, offset, place)                                                                    \
+    __builtin_amdgcn_raw_ptr_buffer_load_lds(                                                                            \
+        __builtin_amdgcn_make_buffer_rsrc(const_cast<float*>(base), 0, 0x7fffffff, kBufferFlags), place, BYTES, offset, 0, 0, 0)
+
 template <typename T> __host__ __device__ inline T from_float(float value);
 template <> __host__ __device__ inline float from_float<float>(float value) { return value; }
 template <> __host__ __device__ inline bf16 from_float<bf16>(float value) {

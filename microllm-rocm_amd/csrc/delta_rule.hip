@@ -255,31 +255,31 @@ delta_scan_tiled_kernel(const float* __restrict__ u, const float* __restrict__ g
     constexpr int kValueCalls = (kTileTokens * kDeltaColumnsAWave + kWave - 1) / kWave;
     constexpr int kGateCalls = (kTileTokens * 2 + kWave - 1) / kWave;
     auto fetch = [&](int tile_first, float* buffer) __attribute__((always_inline)) {
+        const float* rows = u + static_cast<int64_t>(tile_first) * channels;
+        const float* gate_rows = gates + static_cast<int64_t>(tile_first) * 2 * heads;
+        const int left = last - 1 - tile_first;
 #pragma unroll
         for (int j = 0; j < kCalls; ++j) {
-            const int64_t token = min(tile_first + token_of[j], last - 1);
-            const float* row = u + token * channels + channel_of[j];
+            const int at = (min(token_of[j], left) * channels + channel_of[j]) * 4;
             float* place = buffer + j * kWave * kPiece;
             if constexpr (WIDE) {
-                __builtin_amdgcn_global_load_lds(row + k_at, place, 16, 0, 0);
-                __builtin_amdgcn_global_load_lds(row + q_at, place + kDeltaTileFloats, 16, 0, 0);
+                MLL_LOAD_INTO_LDS(16, rows + k_at, at, place);
+                MLL_LOAD_INTO_LDS(16, rows + q_at, at, place + kDeltaTileFloats);
             } else {
-                __builtin_amdgcn_global_load_lds(row + k_at, place, 4, 0, 0);
-                __builtin_amdgcn_global_load_lds(row + q_at, place + kDeltaTileFloats, 4, 0, 0);
+                MLL_LOAD_INTO_LDS(4, rows + k_at, at, place);
+                MLL_LOAD_INTO_LDS(4, rows + q_at, at, place + kDeltaTileFloats);
             }
         }
 #pragma unroll
         for (int j = 0; j < kValueCalls; ++j) {
             const int element = j * kWave + lane;
-            const int64_t token = min(tile_first + element / kDeltaColumnsAWave, last - 1);
             const int wanted = min(static_cast<int>(blockIdx.z) * kDeltaColumnsAWave + element % kDeltaColumnsAWave, value_dim - 1);
-            __builtin_amdgcn_global_load_lds(u + token * channels + v_at + wanted, buffer + kValuesAt + j * kWave, 4, 0, 0);
+            MLL_LOAD_INTO_LDS(4, rows + v_at, (min(element / kDeltaColumnsAWave, left) * channels + wanted) * 4, buffer + kValuesAt + j * kWave);
         }
 #pragma unroll
         for (int j = 0; j < kGateCalls; ++j) {
             const int element = j * kWave + lane;
-            const int64_t token = min(tile_first + element / 2, last - 1);
-            __builtin_amdgcn_global_load_lds(gates + token * 2 * heads + 2 * head + element % 2, buffer + kGatesAt + j * kWave, 4, 0, 0);
+            MLL_LOAD_INTO_LDS(4, gate_rows + 2 * head, (min(element / 2, left) * 2 * heads + element % 2) * 4, buffer + kGatesAt + j * kWave);
         }
     };
     auto walk_tokens = [&](auto every_channel, int tile_first, int count, const float* buffer) __attribute__((always_inline)) {
@@ -413,8 +413,8 @@ int mll_delta_scan(const float* u, const float* gates, float* state, const int32
     MLL_REQUIRE(heads < 65536 && groups < 65536, "delta_scan: too many heads or value channels for one launch");
     const dim3 grid(n_seqs, heads, groups);
     const int rows = (key_dim + kDeltaLanesAColumn - 1) / kDeltaLanesAColumn;
-    if (long_portions) {
-        const int channels = 2 * key_heads * key_dim + heads * value_dim;
+    const int64_t channels = 2ll * key_heads * key_dim + static_cast<int64_t>(heads) * value_dim;
+    if (long_portions && channels < (1 << 22)) {      // a tile of at most 64 rows within 32-bit offsets
         const bool wide = key_dim % 4 == 0 && channels % 4 == 0 && reinterpret_cast<uintptr_t>(u) % 16 == 0;
 #define MLL_DELTA_TILED(WIDE, ROWS) \
     delta_scan_tiled_kernel<WIDE, ROWS><<<grid, kWave, 0, stream>>>(u, gates, state, cu_tokens, slots, out, key_heads, heads, key_dim, value_dim)

@@ -33,7 +33,6 @@ typedef float floatx16 __attribute__((ext_vector_type(16)));
 // by filling the compute units: 2048 x 37888 x 3584 7190 -> 4500 us (124 TFLOP/s), 2048 x 3584 x 18944 3370 -> 2120, 1003 x 9728 x 896 257 ->
 // 165, 64 x 37888 x 3584 323 -> 202.
 constexpr int kTileDepth = 32;
-constexpr int kBufferFlags = 0x00027000;    // a raw buffer of 32-bit words
 constexpr int kNonTemporal = 2;
 constexpr int kPast = 0x40000000;           // past the end of every descriptor here, and with any row's offset added to it
 constexpr int kWidestVector = 1 << 20;      // k up to which the byte offsets of 128 rows stay below kPast

@@ -34,7 +34,6 @@ constexpr int kStepsPerStage = 8;    // k steps of activations in one LDS buffer
 constexpr int kMostTiles = 16;       // two a wave of 8
 constexpr unsigned kPast = 0x40000000;   // an offset past the end of every descriptor here
 constexpr int kMostSteps = static_cast<int>(kPast) / (kMostTiles * 1024);      // so that a workgroup's tiles end before it
-constexpr int kBufferFlags = 0x00027000;   // a raw buffer of 32-bit words
 constexpr int kNonTemporal = 2;      // W is read once a step: past the caches
 
 union Piece {

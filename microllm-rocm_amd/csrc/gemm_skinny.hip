@@ -20,7 +20,6 @@ typedef float floatx4 __attribute__((ext_vector_type(4)));
 typedef unsigned int uintx4 __attribute__((ext_vector_type(4)));
 
 
-constexpr int kBufferFlags = 0x00027000;   // a raw buffer of 32-bit words
 constexpr int kNonTemporal = 2;
 constexpr int kChunk = 4;     // k steps a wave takes in a row, then skips what the other waves take
 
