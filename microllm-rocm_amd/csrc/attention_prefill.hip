@@ -586,8 +586,10 @@ __global__ __launch_bounds__(kPrefillThreads, 1) void paged_attention_prefill_ke
         }
         // Unrolled: every read from LDS then has an address of the stage plus a constant (an address that a loop
         // carries along would make every read wait for the loads on their way into the other stage).
-        const bool whole = WHOLE_BLOCKS && block_valid > 0 && (block + 1) * BLOCK_KEYS - 1 <= block_position && block * BLOCK_KEYS >= block_last_low;
+        const int block_key = block * BLOCK_KEYS;
+        bool whole = false;
         if constexpr (WHOLE_BLOCKS) {
+            whole = block_valid > 0 && block_key + BLOCK_KEYS - 1 <= block_position && block_key >= block_last_low;
             if (whole) process_block(stage);
         }
         if (!whole) {
