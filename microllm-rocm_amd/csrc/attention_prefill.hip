@@ -243,7 +243,9 @@ __global__ __launch_bounds__(kPrefillThreads, 1) void paged_attention_prefill_ke
         if constexpr (UNIFORM) {
             const int tile_index = block * BLOCK_TILES + (lane_pass * kPrefillThreads + wave_chunk) / TILE_CHUNKS;
             const int tile_in_page = page_shift >= 0 ? tile_index & (tiles_per_page - 1) : tile_index % tiles_per_page;
-            const int64_t from = 2 * (pages[0] * page_elements + head_elements + tile_in_page * TILE_ELEMENTS);      // in bytes
+// in bytes; a page has less than 4 GB (in 64 bits throughout, tiles with a bias take 78 instead of 66 us, 2000 and 1117 tokens, 16 heads)
+            const uint64_t from = static_cast<uint64_t>(static_cast<unsigned>(pages[0])) * static_cast<unsigned>(page_elements * 2) +
+                                  static_cast<unsigned>(2 * (head_elements + tile_in_page * TILE_ELEMENTS));
             const unsigned from_low = static_cast<unsigned>(from), from_high = static_cast<unsigned>(from >> 32);
 #pragma unroll
             for (int pass = 0; pass < PASSES; ++pass) {
@@ -715,6 +717,7 @@ extern "C" int mll_paged_attention_prefill_extra(const void* q, const void* k_ca
     MLL_REQUIRE(head_dim % 16 == 0 && head_dim >= 16 && head_dim <= 256,
                 "paged_attention_prefill: head_dim must be a multiple of 16 in [16, 256]");
     MLL_REQUIRE(page_size > 0 && page_size % 16 == 0, "paged_attention_prefill: page_size must be a multiple of 16");
+    MLL_REQUIRE(static_cast<int64_t>(kv_heads) * page_size * head_dim < (1ll << 31), "paged_attention_prefill: a page of keys has 4 GB or more");
     MLL_REQUIRE(heads <= 65535, "paged_attention_prefill: more than 65535 heads");
     if (n_tiles == 0) return 0;
 #define MLL_PREFILL_CASE(TILES)                                                                                      \
