@@ -141,16 +141,46 @@ __device__ inline float softcap_fast(float value, float cap, float inverse_cap) 
     return fmaf(-2.0f * cap, __builtin_amdgcn_rcpf(1.0f + __expf(2.0f * value * inverse_cap)), cap);
 }
 
+// `value` of lane l ^ DISTANCE, for every lane (of a whole wave), without a way through LDS: two halves or rows exchanged (v_permlane32_swap,
+// v_permlane16_swap), or DPP within a row of 16.
+template <int CONTROL>
+__device__ inline int dpp(int value) { return __builtin_amdgcn_update_dpp(0, value, CONTROL, 0xf, 0xf, false); }
+template <int DISTANCE>
+__device__ inline float lane_across(float value) {
+    const int bits = __builtin_bit_cast(int, value);
+    static_assert(DISTANCE == 1 || DISTANCE == 2 || DISTANCE == 4 || DISTANCE == 8, "within a row of 16 lanes");
+    constexpr int kEveryFourMirrored = 0x1B, kEveryEightMirrored = 0x141;
+    const int there = DISTANCE == 1   ? dpp<0xB1>(bits)      // lanes 1, 0, 3, 2 of every four
+                      : DISTANCE == 2 ? dpp<0x4E>(bits)      // lanes 2, 3, 0, 1 of every four
+                      : DISTANCE == 4 ? dpp<kEveryFourMirrored>(dpp<kEveryEightMirrored>(bits))
+                                      : dpp<0x128>(bits);    // a row turned by eight
+    return __builtin_bit_cast(float, there);
+}
+
+// op over a wave, every lane of which gets the result: pairs of lanes 32 apart, then 16, 8, 4, 2, 1. Six exchanges in registers: through LDS
+// (__shfl_xor) each of them is a trip of its own for the wave, which kernels of few waves wait for.
+template <typename Op>
+__device__ inline float reduce_wave(float value, Op op) {
+    const unsigned bits = __builtin_bit_cast(unsigned, value);
+    const auto halves = __builtin_amdgcn_permlane32_swap(bits, bits, false, false);
+    const unsigned low = halves[0], high = halves[1];
+    value = op(__builtin_bit_cast(float, low), __builtin_bit_cast(float, high));
+    const unsigned joined = __builtin_bit_cast(unsigned, value);
+    const auto rows = __builtin_amdgcn_permlane16_swap(joined, joined, false, false);
+    const unsigned even = rows[0], odd = rows[1];
+    value = op(__builtin_bit_cast(float, even), __builtin_bit_cast(float, odd));
+    value = op(value, lane_across<8>(value));
+    value = op(value, lane_across<4>(value));
+    value = op(value, lane_across<2>(value));
+    return op(value, lane_across<1>(value));
+}
+
 __device__ inline float wave_sum(float value) {
-#pragma unroll
-    for (int offset = kWave / 2; offset > 0; offset >>= 1) value += __shfl_xor(value, offset, kWave);
-    return value;
+    return reduce_wave(value, [](float a, float b) { return a + b; });
 }
 
 __device__ inline float wave_max(float value) {
-#pragma unroll
-    for (int offset = kWave / 2; offset > 0; offset >>= 1) value = fmaxf(value, __shfl_xor(value, offset, kWave));
-    return value;
+    return reduce_wave(value, [](float a, float b) { return fmaxf(a, b); });
 }
 
 // Sum over a block of up to 1024 threads; every thread gets the total. `scratch` holds 16 floats.
@@ -164,7 +194,15 @@ __device__ inline float block_sum(float value, float* scratch) {
     if (lane == 0) scratch[wave] = value;
     __syncthreads();
     float total = 0.0f;
-    for (int index = 0; index < waves; ++index) total += scratch[index];
+    if (waves <= 4) {
+        for (int index = 0; index < waves; ++index) total += scratch[index];
+        return total;
+    }
+    float sums[16];     // all read at once: in a loop of unknown length every addition waits for its own read
+#pragma unroll
+    for (int index = 0; index < 16; ++index) sums[index] = scratch[index];
+#pragma unroll
+    for (int index = 0; index < 16; ++index) total = index < waves ? total + sums[index] : total;
     return total;
 }
 
