@@ -200,12 +200,13 @@ qk_norm_store_kernel(const float* __restrict__ qkv, int n_parts, int64_t part_st
     for (int c = lane; c < dim; c += kWave) {
         const float value = raw(c);
         own[c] = value;
-        float length = 1.0f;
         if (norm_turned && c < rot_dims) {      // a turned pair is as long as before, but for the factor within cos and sin
             const int pair = c < half ? c : c - half;
-            length = angles[2 * pair] * angles[2 * pair] + angles[2 * pair + 1] * angles[2 * pair + 1];
+            const float length = fmaf(angles[2 * pair], angles[2 * pair], angles[2 * pair + 1] * angles[2 * pair + 1]);
+            squares = fmaf(value * value, length, squares);
+        } else {
+            squares = fmaf(value, value, squares);
         }
-        squares += value * value * length;
     }
     const float* weight = is_q ? q_weight : (is_k ? k_weight : nullptr);
     const bool norm = (is_q || is_k) ? normed : values_normed;
@@ -243,7 +244,7 @@ qk_norm_store_kernel(const float* __restrict__ qkv, int n_parts, int64_t part_st
                 const int pair = c < half ? c : c - half;
                 const float other = prepared(c < half ? c + half : c - half);
                 const float cosine = angles[2 * pair], sine = angles[2 * pair + 1];
-                value = c < half ? value * cosine - other * sine : value * cosine + other * sine;
+                value = fmaf(value, cosine, c < half ? -(other * sine) : other * sine);
             }
             if (norm_turned) value = normed_value(value, c);
         }
@@ -254,6 +255,155 @@ qk_norm_store_kernel(const float* __restrict__ qkv, int n_parts, int64_t part_st
         } else {
             to[at] = rounded;
         }
+    }
+}
+
+// The same for steps of many rows that go into tiled bfloat16 pages: a wave takes one head of eight tokens, so that a tile is written in pieces of 16 bytes.
+// Written two bytes at a time, a line of a tile takes its 32 numbers from the waves of eight or sixteen tokens, and those writes bound the kernel above
+// from a few thousand rows on (fewer instructions, eight heads a wave, left it at 53 us; tokens of a tile on one die, whose cache then takes every write of a line:
+// 69): 3117 tokens of 24 heads of 128 46 -> 23 us, 16000 189 -> 79 us (98 MB to write and 197 to read).
+// Keys and values go by runs of tokens whose places follow one another within eight; a run begins where a place is a multiple of eight or does not follow
+// the place before. A wave takes the runs that begin among its eight tokens. The arithmetic of a vector is the kernel's above: the same bits.
+constexpr int kStoreTokens = 8;
+
+template <bool MORE, int WIDEST>
+__global__ void __launch_bounds__(kNormStoreWaves * kWave)
+qk_norm_store_tiles_kernel(const float* __restrict__ qkv, const float* __restrict__ q_weight, const float* __restrict__ k_weight, float eps,
+                           const int32_t* __restrict__ positions, const int32_t* __restrict__ slot_mapping, float temp_coef, int temp_every,
+                           bf16* __restrict__ q_out, bf16* __restrict__ k_pages, bf16* __restrict__ v_pages, int heads, int kv_heads, int dim,
+                           int page_size, const float* __restrict__ bias, int normed, int queries_only, int64_t row_stride,
+                           const float* __restrict__ cos_sin, int rot_dims, int values_normed, int n_tokens, int total, int turned_first) {
+    __shared__ float before[kNormStoreWaves][kStoreTokens * WIDEST];      // the vectors as they are before norm and turn
+    __shared__ __attribute__((aligned(16))) bf16 after[kNormStoreWaves][kStoreTokens * WIDEST];
+    const int lane = threadIdx.x % kWave, wave = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave);
+    const int vectors = queries_only ? heads : heads + 2 * kv_heads;
+    const int item = blockIdx.x * kNormStoreWaves + wave;
+    if (item >= total) return;
+    const int first_token = item / vectors * kStoreTokens, which = item % vectors;
+    const bool is_q = which < heads, is_k = !is_q && which < heads + kv_heads;
+    const int head = is_q ? which : (is_k ? which - heads : which - heads - kv_heads);
+    const int offset = which * dim;
+    float* own = before[wave];
+    bf16* results = after[wave];
+    const bool turns = cos_sin != nullptr && (is_q || is_k), norm_turned = MORE && turned_first && turns;
+    const bool norm = (is_q || is_k) ? normed : values_normed;
+    const float* weight = is_q ? q_weight : (is_k ? k_weight : nullptr);
+    const int half = rot_dims / 2;
+    auto meet = [&] {      // the wave's lanes read what its other lanes wrote
+        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+        __builtin_amdgcn_wave_barrier();
+        __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+    };
+    // Lane i has the place of token first_token + i (and the one before the first in lane 63); bit i of `starts`: a run begins there.
+    int slot = -1;
+    unsigned long long starts = 1ull;
+    if (!is_q) {
+        const int token = lane == kWave - 1 ? first_token - 1 : first_token + lane;
+        if (token >= 0 && token < n_tokens && (lane < 2 * kStoreTokens || lane == kWave - 1)) slot = slot_mapping[token];
+        const int previous = __shfl(slot, (lane + kWave - 1) % kWave, kWave);
+        starts = __ballot(slot < 0 || slot % kStoreTokens == 0 || slot != previous + 1);
+    }
+    auto run = [&](int first, int count, int first_slot) {
+        const int64_t row0 = first;
+        float factors[kStoreTokens], squares[kStoreTokens];
+#pragma unroll
+        for (int i = 0; i < kStoreTokens; ++i) squares[i] = 0.0f;
+        for (int c = lane; c < dim; c += kWave) {
+            float values[kStoreTokens];
+#pragma unroll
+            for (int i = 0; i < kStoreTokens; ++i) values[i] = qkv[(row0 + min(i, count - 1)) * row_stride + offset + c];
+            const float shift = bias ? bias[offset + c] : 0.0f;
+#pragma unroll
+            for (int i = 0; i < kStoreTokens; ++i) {
+                const float value = bias ? values[i] + shift : values[i];
+                own[i * dim + c] = value;
+                if (norm_turned && c < rot_dims) {      // a turned pair is as long as before, but for the factor within cos and sin
+                    const float* angle = cos_sin + (row0 + min(i, count - 1)) * rot_dims + 2 * (c < half ? c : c - half);
+                    const float length = fmaf(angle[0], angle[0], angle[1] * angle[1]);
+                    squares[i] = fmaf(value * value, length, squares[i]);
+                } else {
+                    squares[i] = fmaf(value, value, squares[i]);
+                }
+            }
+        }
+        float temperature = 1.0f;      // lane i: of the run's token i
+        if (is_q && temp_coef != 0.0f) {
+            const int steps = (positions[row0 + min(lane, count - 1)] + 1) / temp_every;
+            temperature = 1.0f + temp_coef * static_cast<float>(log(static_cast<double>(steps) + 1.0));
+        }
+#pragma unroll
+        for (int i = 0; i < kStoreTokens; ++i) {
+            factors[i] = norm ? 1.0f / sqrtf(wave_sum(squares[i]) / static_cast<float>(dim) + eps) : 1.0f;
+            if (is_q && temp_coef != 0.0f) factors[i] *= __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, temperature), i));
+        }
+        meet();
+        for (int c = lane; c < dim; c += kWave) {
+            const int across = c < half ? c + half : c - half;
+            const float own_weight = weight ? weight[c] : 1.0f, other_weight = weight && turns && c < rot_dims ? weight[across] : 1.0f;
+#pragma unroll
+            for (int i = 0; i < kStoreTokens; ++i) {
+                auto normed_value = [&](float value, float by) { return norm ? (weight ? value * factors[i] * by : value * factors[i]) : value; };
+                float value = norm_turned ? own[i * dim + c] : normed_value(own[i * dim + c], own_weight);
+                if (turns && c < rot_dims) {
+                    const float* angle = cos_sin + (row0 + min(i, count - 1)) * rot_dims + 2 * (c < half ? c : c - half);
+                    const float other = norm_turned ? own[i * dim + across] : normed_value(own[i * dim + across], other_weight);
+                    value = fmaf(value, angle[0], c < half ? -(other * angle[1]) : other * angle[1]);
+                }
+                if (norm_turned) value = normed_value(value, own_weight);
+                results[i * dim + c] = from_float<bf16>(value);
+            }
+        }
+        meet();
+        const int chunks = dim / 8;
+        if (is_q) {
+            for (int at = lane; at < count * chunks; at += kWave) {
+                const int i = at / chunks, chunk = at % chunks;
+                *reinterpret_cast<uint4*>(q_out + ((row0 + i) * heads + head) * dim + chunk * 8) = *reinterpret_cast<const uint4*>(results + i * dim + chunk * 8);
+            }
+        } else {
+            const CacheLayout layout(kv_heads, page_size, dim);
+            const int64_t page = first_slot / page_size;
+            const int in_page = first_slot % page_size;
+            if (is_k) {
+                for (int at = lane; at < kStoreTokens * chunks; at += kWave) {
+                    const int chunk = at / kStoreTokens, i = at % kStoreTokens;
+                    if (i < count)
+                        *reinterpret_cast<uint4*>(k_pages + layout.k_at(page, head, in_page + i, chunk * 8)) =
+                            *reinterpret_cast<const uint4*>(results + i * dim + chunk * 8);
+                }
+            } else {
+                for (int c = lane; c < dim; c += kWave) {
+                    bf16* to = v_pages + layout.v_at(page, head, in_page, c);
+                    union {
+                        bf16 eight[kStoreTokens];
+                        uint4 raw;
+                    } column;
+#pragma unroll
+                    for (int i = 0; i < kStoreTokens; ++i) column.eight[i] = results[i * dim + c];
+                    if (count == kStoreTokens) {
+                        *reinterpret_cast<uint4*>(to) = column.raw;
+                    } else {
+#pragma unroll
+                        for (int i = 0; i < kStoreTokens; ++i)
+                            if (i < count) to[i] = column.eight[i];
+                    }
+                }
+            }
+        }
+        meet();      // before the next run's vectors are written
+    };
+    if (is_q) {
+        run(first_token, min(kStoreTokens, n_tokens - first_token), 0);
+        return;
+    }
+    unsigned long long left = starts & ((1ull << kStoreTokens) - 1);
+    while (left != 0ull) {
+        const int at = __ffsll(left) - 1;
+        left &= left - 1ull;
+        const int first_slot = __builtin_amdgcn_readlane(slot, at);
+        if (first_slot < 0) continue;      // a row of no request, or past the step's end
+        const unsigned long long further = starts & ~((2ull << at) - 1ull);      // bit 2 kStoreTokens is set: no place is read there
+        run(first_token + at, __ffsll(further) - 1 - at, first_slot);
     }
 }
 
@@ -301,6 +451,27 @@ int mll_qk_norm_store(const float* qkv, int n_parts, int64_t part_stride, const 
         qkv, n_parts, part_stride, q_weight, k_weight, eps, positions, slot_mapping, temp_coef, temp_every, static_cast<T*>(q_out), \
         static_cast<T*>(k_pages), static_cast<T*>(v_pages), heads, kv_heads, key_dim, value_dim, tiled_page_size, bias, normed,     \
         queries_only, row_stride, cos_sin, rot_dims, values_normed, static_cast<int>(total), given)
+    // Eight tokens a wave where that leaves four waves a SIMD.
+    constexpr int64_t kManyWaves = 4 * 4 * 256;
+    const int vectors = queries_only ? heads : heads + 2 * kv_heads;
+    const int64_t waves = (static_cast<int64_t>(n_tokens) + kStoreTokens - 1) / kStoreTokens * vectors;
+    if (dtype == kBF16 && waves >= kManyWaves && n_parts == 1 && key_dim == value_dim && key_dim % 8 == 0 && key_dim <= 256 &&
+        (queries_only || (tiled_page_size > 0 && key_dim % 16 == 0)) && given.taps == nullptr && maps == 1 && (given.stored_dim == 0 || given.stored_dim == key_dim) &&
+        (reinterpret_cast<uintptr_t>(q_out) | reinterpret_cast<uintptr_t>(k_pages) | reinterpret_cast<uintptr_t>(v_pages)) % 16 == 0) {
+        const unsigned workgroups = static_cast<unsigned>((waves + kNormStoreWaves - 1) / kNormStoreWaves);
+#define MLL_NORM_STORE_TILES(MORE, WIDEST)                                                                                              \
+    qk_norm_store_tiles_kernel<MORE, WIDEST><<<workgroups, kNormStoreWaves * kWave, 0, stream>>>(                                           \
+        qkv, q_weight, k_weight, eps, positions, slot_mapping, temp_coef, temp_every, static_cast<bf16*>(q_out),                     \
+        static_cast<bf16*>(k_pages), static_cast<bf16*>(v_pages), heads, kv_heads, key_dim, tiled_page_size, bias, normed,           \
+        queries_only, row_stride, cos_sin, rot_dims, values_normed, n_tokens, static_cast<int>(waves), given.norm_turned)
+        if (given.norm_turned) {
+            if (key_dim <= 128) MLL_NORM_STORE_TILES(true, 128); else MLL_NORM_STORE_TILES(true, 256);
+        } else {
+            if (key_dim <= 128) MLL_NORM_STORE_TILES(false, 128); else MLL_NORM_STORE_TILES(false, 256);
+        }
+#undef MLL_NORM_STORE_TILES
+        return check_launch("qk_norm_store");
+    }
     if (dtype == kF32) {
         if (more) MLL_NORM_STORE(float, true); else MLL_NORM_STORE(float, false);
     } else if (dtype == kBF16) {

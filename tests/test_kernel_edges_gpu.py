@@ -489,6 +489,37 @@ def test_blocks_seen_whole_have_the_bits_of_their_runs(heads, kv_heads, hd, page
         assert torch.equal(run(), run(extras=nothing, out=torch.empty_like(t["q"]))), larger
 
 
+@pytest.mark.parametrize("heads,kv_heads,dim,page,options", [
+    (16, 4, 128, 16, dict(weights=True, temperature=True)), (9, 3, 96, 48, dict(bias=True, rot=64)), (5, 1, 16, 32, dict(values_normed=True, rot=16)),
+    (7, 7, 256, 16, dict(norm_turned=True, rot=128)), (13, 2, 72, 16, dict(queries_only=True)), (8, 2, 112, 64, dict(norm_turned=True, rot=112, weights=True))])
+def test_heads_of_eight_tokens_a_wave_have_the_bits_of_a_wave_each(heads, kv_heads, dim, page, options):
+    """A step of many rows, of whose heads a wave takes eight tokens, against the same rows by few, whose heads have a wave each: requests that begin and end within
+    eight places, pages in any order, rows without a place, places that are not one after the other."""
+    k, generator = kernels(), torch.Generator(device=DEVICE).manual_seed(dim + heads)
+    alone, rot = options.get("queries_only", False), options.get("rot", 0)
+    n, vectors = 9000 if heads < 8 and kv_heads == 1 else 4200, heads + (0 if alone else 2 * kv_heads)
+    assert -(-n // 8) * vectors >= 4096 > -(-125 // 8) * vectors        # both sides of the line
+    normal = lambda *shape: torch.randn(shape, generator=generator, device=DEVICE)
+    pages = -(-n // page) + 8
+    rows, positions = normal(n, vectors * dim), torch.arange(n, dtype=torch.int32, device=DEVICE) * 3
+    order = torch.randperm(pages, generator=generator, device=DEVICE)
+    slots = (order[:, None] * page + torch.arange(page, device=DEVICE)).view(-1).to(torch.int32)
+    slots = torch.cat([slots[5:1003], slots[1008:1017], slots[1030:]])[:n].contiguous()
+    slots[700:705], slots[2000:2100] = -1, slots[2000:2100].flip(0)
+    bias = normal(vectors * dim) if options.get("bias") else None
+    weights = [normal(dim) if options.get("weights") else None for _ in "qk"]
+    angles = normal(n, rot // 2, 2) if rot else None
+    def run(step):
+        kept = [torch.full(shape(pages, kv_heads, page, -(-dim // 16) * 16), 7.0, dtype=torch.bfloat16, device=DEVICE) for shape in (key_page_shape, value_page_shape)]
+        queries = [k.qk_norm_store(rows[i:i + step], *weights, 1e-6, positions[i:i + step], slots[i:i + step], 0.5 if options.get("temperature") else 0.0, 64, *kept, heads,
+                                   kv_heads, dim, dim, torch.bfloat16, tiled_page_size=page if not alone else 0, bias=bias, normed=True, queries_only=alone,
+                                   cos_sin=angles[i:i + step] if rot else None, values_normed=options.get("values_normed", False),
+                                   norm_turned=options.get("norm_turned", False)) for i in range(0, n, step)]
+        return [torch.cat(queries), *kept]
+    for whole, parts in zip(run(n), run(125)):
+        assert torch.equal(whole, parts)
+
+
 # ---- float32 attention by chunks, all heads of a kv head together: every head size, one head a kv head to more than 16, windows that begin in
 # either tile of a chunk, and values that are not finite where a token sees them and where it does not ----
 @pytest.mark.parametrize("heads,kv_heads,hd,page_size", [(28, 4, 16, 16), (14, 2, 32, 32), (9, 9, 48, 48), (7, 1, 64, 16), (40, 2, 80, 48), (5, 1, 96, 16),
