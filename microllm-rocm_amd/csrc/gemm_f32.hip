@@ -621,23 +621,24 @@ extern "C" int mll_gemm_f32(const float* a, const float* w, const float* bias, f
         else gemm_f32_small_kernel<false><<<grid, 256, 0, stream>>>(a, w, bias, c, m, n, k, k_split);
         return check_launch("gemm_f32");
     }
-    // The tile whose workgroups fill the compute units best: the matrix units' time is the rounds of 256 workgroups times
-    // a tile's size. Of tiles that come to the same the smaller ones where parts of the reduction are short, since several share a
-    // unit and cover each other's ends: 512 x 3584 x 3584 in parts of 448 in tiles of 128 x 64 and 64 x 64 129 and 119 us, 1003 x 37888 x 64
-    // 92 and 72, 2048 x 9728 x 896 in tiles of 128 x 128 338 and 317; but 512 x 3584 x 2048 in parts of 512 73 and
-    // 79, 320 x 37888 x 256 68 and 74, 1003 x 16384 x 8192 2107 and 2471. Up to 32 rows take tiles of 32 rows (32 x 9728 x 896 in tiles of 64 x 64 26.6 us, of 32 x 128 17.7).
-    struct Shape { int rows, columns; };
-    const Shape shapes[4] = {{128, 128}, {128, 64}, {64, 64}, {32, 128}};
-    const bool smaller = k_split <= (splits > 1 ? 448 : 128);
+    // The tile that is done first: a tile's size, times what its elements take, times the rounds of 256 workgroups, of which the last counts by
+    // four fifths of a whole one beside its share (workgroups that share a unit cover each other's ends). Where parts of the reduction are long the larger
+    // tiles read LDS less for every product; where they are short the smaller ones' beginnings and ends overlap. Fitted to the four shapes' times at
+    // 119 sizes (65 to 1500 rows of seven weights): 0.4 % above the fastest on the mean and 6 % at most, where rounds alone, whole below 4096 workgroups and
+    // not above, were 2.8 and 44 % above it (1500 x 37888 x 3584 in tiles of 32 x 128 4746 us, of 128 x 128 3290; 512 rows of it 1308 and 1176; 600 1866 and
+    // 1408; 512 x 896 x 4864 in eight parts 55 and, in tiles of 64 x 64, 49). Up to 32 rows take tiles of 32 rows (32 x 9728 x 896 in tiles of 64 x 64 26.6 us, of 32 x 128 17.7).
+    struct Shape { int rows, columns; double in_long, in_short; };
+    const Shape shapes[4] = {{128, 128, 1.0, 1.0}, {128, 64, 1.06, 0.98}, {64, 64, 1.10, 0.92}, {32, 128, 1.30, 0.975}};
+    constexpr int kLongParts = 1000;
     int best = 3;
     double least = 1e300;
     for (int index = m <= 32 ? 3 : 0; index < 4; ++index) {
         const Shape& shape = shapes[index];
         const int64_t groups = static_cast<int64_t>((n + shape.columns - 1) / shape.columns) * ((m + shape.rows - 1) / shape.rows) * splits;
-        const double rounds = groups >= 4096 ? groups / 256.0 : static_cast<double>((groups + 255) / 256);
-        const double cost = rounds * shape.rows * shape.columns;
+        const double rounds = 0.8 * static_cast<double>((groups + 255) / 256) + 0.2 * groups / 256.0;
+        const double cost = rounds * shape.rows * shape.columns * (k_split > kLongParts ? shape.in_long : shape.in_short);
         const bool fits = (m + shape.rows - 1) / shape.rows <= 65535;       // as the grid's second size
-        if (fits && (index < 3 && smaller ? cost <= least : cost < least)) least = cost, best = index;
+        if (fits && cost < least) least = cost, best = index;
     }
     const Shape& shape = shapes[best];
     const int64_t tiles = static_cast<int64_t>((n + shape.columns - 1) / shape.columns) * ((m + shape.rows - 1) / shape.rows) * splits;
