@@ -109,7 +109,7 @@ __global__ __launch_bounds__(kDecodeThreads, HD_TILES <= 8 ? 2 : 1) void paged_a
     const CacheLayout layout(kv_heads, page_size, HD);
 
     const int lane = threadIdx.x % kWave;
-    const int wave = threadIdx.x / kWave;
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave);      // the same for all lanes, which the compiler cannot tell
     const int col = lane % 16;   // head (B operands, results) or key/dim row (A operands)
     const int quad = lane / 16;  // which 8 of the 32 k-slots this lane supplies
 
@@ -275,14 +275,20 @@ __global__ __launch_bounds__(kDecodeThreads, HD_TILES <= 8 ? 2 : 1) void paged_a
         int page[2] = {page_of(pair * 32), page_of(pair * 32 + 16)};
         int following = min(pair + kDecodeWaves, last);
         int next_page[2] = {page_of(following * 32), page_of(following * 32 + 16)};
+
         load_pair(pair, page, k_first, v_first, bias_first);
-        while (true) {
+        // Two pairs a round, and what is left of an odd number after the rounds: were the loop left between the two, the compiler would think that
+        // it comes round with the second pair's loads on their way, and wait for all of them at the start of every round (64 ragged requests of at
+        // most 3000 positions, 28 heads of 128 over 4, in 4 splits 35.3 -> 32.1 us; one of 60, 14 heads of 64 over 2, 3.87 -> 3.54; one of 100, 16
+        // heads of 256 over 4, 8.9 -> 7.7; heads of 256 of 40 requests of 500 unsplit 21.9 -> 22.6, the one size found slower by more than 2 %).
+        const int pairs = (last - pair) / kDecodeWaves + 1;
+        for (int round = 0; round < pairs / 2; ++round) {
             int after = min(following + kDecodeWaves, last);
             page[0] = page_of(after * 32);
             page[1] = page_of(after * 32 + 16);
             load_pair(following, next_page, k_second, v_second, bias_second);
+
             attend_pair(pair, k_first, v_first, bias_first);
-            if (pair == last) break;
             pair = following;
             following = after;
 
@@ -290,11 +296,14 @@ __global__ __launch_bounds__(kDecodeThreads, HD_TILES <= 8 ? 2 : 1) void paged_a
             next_page[0] = page_of(after * 32);
             next_page[1] = page_of(after * 32 + 16);
             load_pair(following, page, k_first, v_first, bias_first);
+
             attend_pair(pair, k_second, v_second, bias_second);
-            if (pair == last) break;
             pair = following;
             following = after;
         }
+        // Asked for here also, or the compiler looks the pages up just before the rounds, behind the first pair's loads, and waits for both.
+        asm volatile("" ::"v"(next_page[0]), "v"(next_page[1]));
+        if (pairs % 2 != 0) attend_pair(pair, k_first, v_first, bias_first);
     }
 
     // Join the 4 waves in LDS: o_shared[slot][head][dim]; lane holds head `col`, dims d*16 + quad*4 + i.

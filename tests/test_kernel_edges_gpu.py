@@ -349,6 +349,19 @@ def test_decode_attention_reads_every_line_of_its_pages(heads, kv_heads, hd, pag
 
 
 
+@pytest.mark.parametrize("heads,kv_heads,hd,page_size,window,splits", [
+    (28, 4, 128, 16, 0, 1), (14, 2, 64, 16, 0, 1), (14, 2, 64, 48, 0, 2), (8, 4, 128, 32, 260, 1), (16, 4, 256, 16, 0, 1), (5, 5, 48, 16, 0, 1)])
+def test_decode_attention_of_waves_with_any_number_of_pairs(heads, kv_heads, hd, page_size, window, splits):
+    """A workgroup's four waves take pairs of tiles of 16 keys in turn, two a round and what is left of an odd number: none to five a wave, alike and one
+    more for some of the waves, the last pair's keys one or all."""
+    rng = np.random.default_rng(heads + hd + window)
+    lengths = [1, 32, 33, 128, 129, 160, 256, 257, 289, 384, 385, 512, 513, 609]
+    t, q_exact, ek, ev, seq, pos = build_paged_case(rng, torch.bfloat16, lengths, [1] * len(lengths), heads, kv_heads, hd, page_size)
+    out = kernels().paged_attention_decode(t["q"], t["k"], t["v"], t["table"], t["seq"], t["pos"], hd ** -0.5, window, heads, kv_heads, hd, splits)
+    want = reference_attention(q_exact, ek, ev, seq, pos, heads, kv_heads, hd, hd ** -0.5, window)
+    np.testing.assert_allclose(out.float().cpu().numpy(), want, **tolerance(torch.bfloat16))
+
+
 @pytest.mark.parametrize("heads,kv_heads,hd,tokens,splits", [(28, 4, 128, 4, 8), (14, 2, 64, 12, 8)])
 def test_decode_attention_of_long_steps_has_the_bits_of_fewer_tokens(heads, kv_heads, hd, tokens, splits):
     """128 and 192 workgroups of a step planned for 8192 positions, from which pages are read past the caches, and one token less."""
