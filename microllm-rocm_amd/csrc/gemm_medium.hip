@@ -9,8 +9,8 @@
 //
 // A workgroup takes so many tiles that the workgroups fill the compute units evenly (see balanced_tiles): of
 // 37888 x 3584 10 a workgroup, 237 of them, where 16 would leave 108 of the 256 units without one. 64 rows of it
-// 66.1 -> 51.7 us (the reads alone take 40), of 152064 x 3584 214.6 -> 205.3 us (155), 32 rows of 9728 x 896 10.3 -> 7.4 us,
-// of 896 x 4864 7.2 -> 5.4 us, of 1152 x 896 5.0 -> 3.5 us. With 64 rows the products and the reads of LDS take about as
+// 66.1 -> 51.7 us (the reads alone take 40), of 152064 x 3584 214.6 -> 205.3 us (155), 32 rows of 9728 x 896 10.3 -> 7.4 us (now 6.4),
+// of 896 x 4864 7.2 -> 5.4 us (4.9), of 1152 x 896 5.0 -> 3.5 us (2.9). With 64 rows the products and the reads of LDS take about as
 // long as W's way, and the stages' barriers keep them from covering each other whole.
 //
 // Where W has too few tiles to fill the GPU this way, k is split over `splits` workgroups (grid y), each of
@@ -147,21 +147,29 @@ __global__ __launch_bounds__(kWaves * kWave) void gemm_medium_kernel(
     __builtin_amdgcn_sched_barrier(0);
     store_share(share, 0);
     __syncthreads();
-    for (int s = 0; s < n_stages; s += 2) {
+    // Two stages a round, and what is left of an odd number after the rounds: were the loop left between the two, the compiler would think that it
+    // comes round with the odd tiles' loads on their way, and wait for all loads at the start of every round (17 rows of 9728 x 896
+    // 6.84 -> 5.87 us, of 3584 x 18944 23.8 -> 22.7, 64 rows of 1152 x 896 4.37 -> 3.64, of 896 x 4864 7.05 -> 6.67, of 37888 x 3584 50.6 -> 50.3).
+    // Of four waves, which bring more pieces of the activations each, the compiler would also mix these loads with the tiles' (48 rows of 9728 x 896
+    // 8.3 -> 7.7 us); eight waves of 64 rows lose by the same line (3584 x 3584 9.7 -> 10.1).
+    int s = 0;
+    for (; s + 1 < n_stages; s += 2) {
         load_share(share, s + 1);
+        if constexpr (kWaves == 4) __builtin_amdgcn_sched_barrier(0);
         load_w(w_odd, s + 1);
         __builtin_amdgcn_sched_barrier(0);      // else the loads sink below the products, behind their waits
         multiply(w_even, 0);
         store_share(share, 1);
         __syncthreads();
-        if (s + 1 >= n_stages) break;
         load_share(share, s + 2);
+        if constexpr (kWaves == 4) __builtin_amdgcn_sched_barrier(0);
         load_w(w_even, s + 2);
         __builtin_amdgcn_sched_barrier(0);
         multiply(w_odd, 1);
         store_share(share, 0);
         __syncthreads();
     }
+    if (s < n_stages) multiply(w_even, 0);
 
     // acc[nt][mt][i] = C[row mt*16 + col][column n_tile*16 + quad*4 + i]
 #pragma unroll
@@ -246,7 +254,7 @@ static void launch_rows(const bf16* a, const bf16* w, void* out, int m, int n, i
         gemm_medium_kernel<MT, 1, 4, EPILOGUE, true><<<grid, 4 * kWave, lds, stream>>>(a, w, out, m, n, k, n_tiles, k_steps, steps_per_split, tiles);
         return;
     }
-    // Four waves where there are no more tiles (64 rows of 9728 x 896, 3 tiles a workgroup: 11.7 -> 9.6 us). Four waves of up to four
+    // Four waves where there are no more tiles (64 rows of 9728 x 896, 3 tiles a workgroup: 11.7 -> 9.6 us, now 8.9). Four waves of up to four
     // tiles each read LDS half as often, but hold too much: 64 rows of 37888 x 3584 51.7 -> 55.6 us.
     if (tiles <= 4) launch(integral_constant<int, 1>{}, integral_constant<int, 4>{});
     else if (tiles <= 8) launch(integral_constant<int, 1>{}, integral_constant<int, 8>{});

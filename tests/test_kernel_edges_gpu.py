@@ -276,6 +276,19 @@ def test_streaming_product_of_the_longest_reductions(n):
         assert torch.equal(kernels().gemm_skinny(x[:m].contiguous(), packed, n, "bf16"), want[:m].to(torch.bfloat16))
 
 
+@pytest.mark.parametrize("n", [40, 16 * 300, 16 * 700 - 8, 16 * 2100])      # workgroups of four waves, of eight, of eight with two tiles each
+@pytest.mark.parametrize("k", [8, 256, 264, 512, 520, 768, 1000, 1280])       # one to five stages of 256, whole and begun
+def test_product_for_64_rows_of_any_number_of_stages(n, k):
+    """Two stages a round and what is left of an odd number; sums of whole numbers, which have no rounding to differ in."""
+    generator = torch.Generator(device=DEVICE).manual_seed(n + k)
+    x, w = whole_numbers(generator, 64, k), whole_numbers(generator, n, k)
+    packed, want = kernels().pack_weight(w), x.float() @ w.float().T
+    for m in (17, 32, 33, 64):
+        for splits in (1, 2, 3):
+            got = kernels().gemm_medium(x[:m].contiguous(), packed, n, "f32", plan=(2, 8, splits))
+            assert torch.equal(got.sum(0) if splits > 1 else got, want[:m])
+
+
 @pytest.mark.parametrize("n,splits", [(40, 1), (40, 16), (200, 2)])
 def test_product_for_64_rows_of_the_longest_reductions(n, splits):
     """Where a workgroup's tiles pass what 32-bit offsets reach: the same sums with 64-bit addresses, whole and in parts."""
