@@ -324,13 +324,8 @@ __global__ __launch_bounds__(kPrefillThreads, 1) void paged_attention_prefill_ke
     // column / 16), 8 dims (chunk 2 ks + half) per lane. Second: row = dim `column` of a block of 32 dims; the
     // lane's 8 k-slots are the keys its scores came for, positions 8 half .. + 7 of the tile, one read of 16 bytes;
     // the 64 lanes read 1024 consecutive bytes, which LDS gives without bank conflicts.
-    // The addresses are formed step by step (stage, then tile, then lane). The compiler follows an address back
-    // to its LDS variable over a few additions only, and of a read that it cannot place it assumes that the loads
-    // on their way into the other stage may write it: the first reads of every run of keys therefore wait for
-    // those loads. Formed as one sum (stage plus a per-lane term plus a constant) the reads do not wait, and the
-    // kernel is 5 % slower (836 against 791 us for 8192 tokens, 2680 against 2545 for 16384; waiting for the
-    // loads in other places does not give the same, nor does holding one tile's waves back for a while at the
-    // start of a block). Measured, not understood.
+    // The reads need no wait for the loads into the other stage. While those were flat loads, whose end the compiler cannot tell from that of
+    // reads of LDS, it waited for all of them here, or, with the addresses formed as one sum, elsewhere; buffer loads are counted apart.
     const int key_of_row = (column & ~12) | ((column & 4) << 1) | ((column & 8) >> 1);
     auto process_keys = [&](auto masked_tag, auto halves_tag, const bf16* stage, int first_run, int key0) __attribute__((always_inline)) {
         constexpr bool MASKED = decltype(masked_tag)::value;
