@@ -122,18 +122,30 @@ __global__ __launch_bounds__(kWaves * kWave) void gemm_medium_kernel(
 #pragma unroll
         for (int mt = 0; mt < MT; ++mt) acc[nt][mt] = floatx4{0.0f, 0.0f, 0.0f, 0.0f};
 
+    // With one tile a wave a step's activations are read from LDS while the step before is multiplied: left alone, the compiler reads them one or two
+    // ahead of their products (48 rows of 1152 x 896 3.46 -> 3.25 us, 64 rows of 9728 x 896 8.9 -> 8.5, of 3584 x 3584 9.67 -> 9.35). With two there
+    // are twice as many products to cover a read, and the order it chooses is the better one (32 rows of 37888 x 3584 44.3, 44.9 this way).
     auto multiply = [&](const Piece (&pieces)[kStepsPerStage][NT], int buffer) {
+        Piece a_piece[2][MT];
+        auto read = [&](int u) {
+#pragma unroll
+            for (int mt = 0; mt < MT; ++mt) a_piece[u % 2][mt].raw = stage[(buffer * kStagePieces + mt * kStepsPerStage + u) * kWave + lane];
+        };
+        if constexpr (NT == 1) read(0);
 #pragma unroll
         for (int u = 0; u < kStepsPerStage; ++u) {
-            Piece a_piece[MT];
-#pragma unroll
-            for (int mt = 0; mt < MT; ++mt)
-                a_piece[mt].raw = stage[(buffer * kStagePieces + mt * kStepsPerStage + u) * kWave + lane];
+            if constexpr (NT == 1) {
+                if (u + 1 < kStepsPerStage) read(u + 1);
+                __builtin_amdgcn_sched_barrier(0);
+            } else {
+                read(u);
+            }
 #pragma unroll
             for (int nt = 0; nt < NT; ++nt)
 #pragma unroll
                 for (int mt = 0; mt < MT; ++mt)
-                    acc[nt][mt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(pieces[u][nt].v, a_piece[mt].v, acc[nt][mt], 0, 0, 0);
+                    acc[nt][mt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(pieces[u][nt].v, a_piece[u % 2][mt].v, acc[nt][mt], 0, 0, 0);
+            if constexpr (NT == 1) __builtin_amdgcn_sched_barrier(0);
         }
     };
 
@@ -254,7 +266,7 @@ static void launch_rows(const bf16* a, const bf16* w, void* out, int m, int n, i
         gemm_medium_kernel<MT, 1, 4, EPILOGUE, true><<<grid, 4 * kWave, lds, stream>>>(a, w, out, m, n, k, n_tiles, k_steps, steps_per_split, tiles);
         return;
     }
-    // Four waves where there are no more tiles (64 rows of 9728 x 896, 3 tiles a workgroup: 11.7 -> 9.6 us, now 8.9). Four waves of up to four
+    // Four waves where there are no more tiles (64 rows of 9728 x 896, 3 tiles a workgroup: 11.7 -> 9.6 us, now 8.5). Four waves of up to four
     // tiles each read LDS half as often, but hold too much: 64 rows of 37888 x 3584 51.7 -> 55.6 us.
     if (tiles <= 4) launch(integral_constant<int, 1>{}, integral_constant<int, 4>{});
     else if (tiles <= 8) launch(integral_constant<int, 1>{}, integral_constant<int, 8>{});
