@@ -134,6 +134,16 @@ bias_attention_kernel(const T* __restrict__ q, const T* __restrict__ k_pages, co
 
 constexpr int kNormStoreWaves = 4;
 
+// The sum of a head's squares with one more channel of it, which counts by `length`. MORE: the square is rounded before it is multiplied and added, as
+// it has to be where the length is not 1; without, it is added by one multiply-add. Both kernels below take this one, so that a vector has the same bits in either.
+template <bool MORE>
+__device__ inline float with_square(float squares, float value, float length) {
+#pragma clang fp contract(off)
+    if (!MORE) return fmaf(value, value, squares);
+    const float square = value * value;
+    return fmaf(square, length, squares);
+}
+
 // One wave a (token, head of q, k or v), four to a workgroup: the norm of queries and keys over their head, the queries' factor by
 // position, and the write of keys and values into their pages. MORE: with what MllStoreExtras says (a convolution over time
 // before everything else, the norm after the turn, heads stored wider than they are, several keys a key head).
@@ -200,13 +210,12 @@ qk_norm_store_kernel(const float* __restrict__ qkv, int n_parts, int64_t part_st
     for (int c = lane; c < dim; c += kWave) {
         const float value = raw(c);
         own[c] = value;
+        float length = 1.0f;
         if (norm_turned && c < rot_dims) {      // a turned pair is as long as before, but for the factor within cos and sin
             const int pair = c < half ? c : c - half;
-            const float length = fmaf(angles[2 * pair], angles[2 * pair], angles[2 * pair + 1] * angles[2 * pair + 1]);
-            squares = fmaf(value * value, length, squares);
-        } else {
-            squares = fmaf(value, value, squares);
+            length = fmaf(angles[2 * pair], angles[2 * pair], angles[2 * pair + 1] * angles[2 * pair + 1]);
         }
+        squares = with_square<MORE>(squares, value, length);
     }
     const float* weight = is_q ? q_weight : (is_k ? k_weight : nullptr);
     const bool norm = (is_q || is_k) ? normed : values_normed;
@@ -317,13 +326,12 @@ qk_norm_store_tiles_kernel(const float* __restrict__ qkv, const float* __restric
             for (int i = 0; i < kStoreTokens; ++i) {
                 const float value = bias ? values[i] + shift : values[i];
                 own[i * dim + c] = value;
+                float length = 1.0f;
                 if (norm_turned && c < rot_dims) {      // a turned pair is as long as before, but for the factor within cos and sin
                     const float* angle = cos_sin + (row0 + min(i, count - 1)) * rot_dims + 2 * (c < half ? c : c - half);
-                    const float length = fmaf(angle[0], angle[0], angle[1] * angle[1]);
-                    squares[i] = fmaf(value * value, length, squares[i]);
-                } else {
-                    squares[i] = fmaf(value, value, squares[i]);
+                    length = fmaf(angle[0], angle[0], angle[1] * angle[1]);
                 }
+                squares[i] = with_square<MORE>(squares[i], value, length);
             }
         }
         float temperature = 1.0f;      // lane i: of the run's token i
@@ -464,7 +472,7 @@ int mll_qk_norm_store(const float* qkv, int n_parts, int64_t part_stride, const 
         qkv, q_weight, k_weight, eps, positions, slot_mapping, temp_coef, temp_every, static_cast<bf16*>(q_out),                     \
         static_cast<bf16*>(k_pages), static_cast<bf16*>(v_pages), heads, kv_heads, key_dim, tiled_page_size, bias, normed,           \
         queries_only, row_stride, cos_sin, rot_dims, values_normed, n_tokens, static_cast<int>(waves), given.norm_turned)
-        if (given.norm_turned) {
+        if (more) {
             if (key_dim <= 128) MLL_NORM_STORE_TILES(true, 128); else MLL_NORM_STORE_TILES(true, 256);
         } else {
             if (key_dim <= 128) MLL_NORM_STORE_TILES(false, 128); else MLL_NORM_STORE_TILES(false, 256);

@@ -546,6 +546,37 @@ def test_heads_of_eight_tokens_a_wave_have_the_bits_of_a_wave_each(heads, kv_hea
         assert torch.equal(whole, parts)
 
 
+@pytest.mark.parametrize("n,dtype", [(50, torch.float32), (50, torch.bfloat16), (9000, torch.bfloat16)])      # a wave a head, and eight tokens a wave
+@pytest.mark.parametrize("norm_turned", [False, True])
+def test_heads_norms_are_summed_in_one_order_with_the_same_roundings(n, dtype, norm_turned):
+    """The bits of a head's norm, spelled out: a lane takes every 64th channel in order, by one multiply-add each, where the norm is that of turned vectors by
+    a rounded square and an addition, in turned channels as in the others (of turned ones the square is multiplied by their length, here 1); lanes 32 apart
+    meet first, neighbours last. No tolerance: every step is one rounding."""
+    heads, kv_heads, dim, rot, eps = 3, 1, 192, 64, 1e-6
+    vectors = heads + 2 * kv_heads
+    assert (-(-n // 8) * vectors >= 4096) == (n == 9000)
+    generator = torch.Generator(device=DEVICE).manual_seed(n + norm_turned)
+    rows = torch.randn(n, vectors * dim, generator=generator, device=DEVICE)
+    angles = torch.tensor([1.0, 0.0], device=DEVICE).repeat(n, rot // 2, 1).contiguous()       # no turn, so that the length is 1 and the turn changes no bit
+    pages = -(-n // 16)
+    slots = torch.arange(n, dtype=torch.int32, device=DEVICE)
+    tiled = 16 if dtype == torch.bfloat16 else 0
+    kept = ([torch.zeros(shape(pages, kv_heads, 16, dim), dtype=dtype, device=DEVICE) for shape in (key_page_shape, value_page_shape)] if tiled else
+            [torch.zeros(pages, 16, kv_heads, dim, dtype=dtype, device=DEVICE) for _ in "kv"])
+    q = kernels().qk_norm_store(rows, None, None, eps, slots, slots, 0.0, 1, *kept, heads, kv_heads, dim, dim, dtype, tiled_page_size=tiled, normed=True,
+                                cos_sin=angles, norm_turned=norm_turned)
+    x = rows.cpu().numpy().reshape(n, vectors, dim // 64, 64)[:, :heads]
+    sums = np.zeros((n, heads, 64), np.float32)
+    for j in range(dim // 64):
+        square = x[:, :, j].astype(np.float64) ** 2                 # exact
+        sums = (sums + square.astype(np.float32) if norm_turned else (sums + square)).astype(np.float32)
+    for distance in (32, 16, 8, 4, 2, 1):
+        sums = sums + sums[:, :, np.arange(64) ^ distance]
+    factor = np.float32(1.0) / np.sqrt(sums[:, :, :1] / np.float32(dim) + np.float32(eps))
+    want = torch.from_numpy(x.reshape(n, heads, dim) * factor).to(dtype).view(n, heads * dim)
+    assert torch.equal(q.view(n, heads * dim).cpu(), want)
+
+
 # ---- float32 attention by chunks, all heads of a kv head together: every head size, one head a kv head to more than 16, windows that begin in
 # either tile of a chunk, and values that are not finite where a token sees them and where it does not ----
 @pytest.mark.parametrize("heads,kv_heads,hd,page_size", [(28, 4, 16, 16), (14, 2, 32, 32), (9, 9, 48, 48), (7, 1, 64, 16), (40, 2, 80, 48), (5, 1, 96, 16),
