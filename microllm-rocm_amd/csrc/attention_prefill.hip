@@ -209,8 +209,16 @@ __global__ __launch_bounds__(kPrefillThreads, 1) void paged_attention_prefill_ke
     // The page of a tile: pages hold tiles_per_page tiles of 16 positions (often one, mostly a power of two).
     const int tiles_per_page = page_size / 16;
     const int page_shift = (tiles_per_page & (tiles_per_page - 1)) == 0 ? __ffs(tiles_per_page) - 1 : -1;
-    const int64_t page_elements = static_cast<int64_t>(kv_heads) * tiles_per_page * TILE_ELEMENTS;
-    const int head_elements = kv_head * tiles_per_page * TILE_ELEMENTS;
+    // Places in the pools are counted in pieces of 256 elements (512 bytes), of which a tile has HD_TILES: a page's number of pieces fits 32 bits
+    // whatever fits the memory, so a tile's place is one 32 by 32 bit product (in 64 bits throughout, tiles with a bias take 78 instead
+    // of 66 us, 2000 and 1117 tokens, 16 heads).
+    constexpr int PIECE = 256;
+    static_assert(TILE_ELEMENTS == HD_TILES * PIECE, "a tile is whole pieces");
+    const unsigned page_pieces = static_cast<unsigned>(kv_heads) * tiles_per_page * HD_TILES;
+    const unsigned head_tiles = static_cast<unsigned>(kv_head) * tiles_per_page;
+    auto piece_at = [&](int page, int tile_in_page) {      // the tile's first
+        return static_cast<uint64_t>(static_cast<unsigned>(page)) * page_pieces + (head_tiles + tile_in_page) * HD_TILES;
+    };
     const int wave_chunk = __builtin_amdgcn_readfirstlane(wave) * kWave;      // the wave's first piece of pass 0
     auto tile_of = [&](int pass) { return (pass * kPrefillThreads + wave_chunk + (UNIFORM ? 0 : lane)) / TILE_CHUNKS; };   // in the block
     auto piece_of = [&](int pass) { return (pass * kPrefillThreads + wave_chunk + (UNIFORM ? 0 : lane)) % TILE_CHUNKS + (UNIFORM ? lane : 0); };
@@ -243,9 +251,7 @@ __global__ __launch_bounds__(kPrefillThreads, 1) void paged_attention_prefill_ke
         if constexpr (UNIFORM) {
             const int tile_index = block * BLOCK_TILES + (lane_pass * kPrefillThreads + wave_chunk) / TILE_CHUNKS;
             const int tile_in_page = page_shift >= 0 ? tile_index & (tiles_per_page - 1) : tile_index % tiles_per_page;
-// in bytes; a page has less than 4 GB (in 64 bits throughout, tiles with a bias take 78 instead of 66 us, 2000 and 1117 tokens, 16 heads)
-            const uint64_t from = static_cast<uint64_t>(static_cast<unsigned>(pages[0])) * static_cast<unsigned>(page_elements * 2) +
-                                  static_cast<unsigned>(2 * (head_elements + tile_in_page * TILE_ELEMENTS));
+            const uint64_t from = piece_at(pages[0], tile_in_page) * (PIECE * sizeof(bf16));
             const unsigned from_low = static_cast<unsigned>(from), from_high = static_cast<unsigned>(from >> 32);
 #pragma unroll
             for (int pass = 0; pass < PASSES; ++pass) {
@@ -268,7 +274,7 @@ __global__ __launch_bounds__(kPrefillThreads, 1) void paged_attention_prefill_ke
                 if (pages[pass] < 0) continue;
                 const int tile_index = block * BLOCK_TILES + tile_of(pass);
                 const int tile_in_page = page_shift >= 0 ? tile_index & (tiles_per_page - 1) : tile_index % tiles_per_page;
-                const int64_t tile_start = pages[pass] * page_elements + head_elements + tile_in_page * TILE_ELEMENTS;
+                const int64_t tile_start = static_cast<int64_t>(piece_at(pages[pass], tile_in_page)) * PIECE;
                 bf16* key_place = stage + (pass * kPrefillThreads + wave_chunk) * 8;
                 const bf16* key_piece = k_cache + tile_start + piece_of(pass) * 8;
                 const bf16* value_piece = v_cache + tile_start + piece_of(pass) * 8;
@@ -712,7 +718,6 @@ extern "C" int mll_paged_attention_prefill_extra(const void* q, const void* k_ca
     MLL_REQUIRE(head_dim % 16 == 0 && head_dim >= 16 && head_dim <= 256,
                 "paged_attention_prefill: head_dim must be a multiple of 16 in [16, 256]");
     MLL_REQUIRE(page_size > 0 && page_size % 16 == 0, "paged_attention_prefill: page_size must be a multiple of 16");
-    MLL_REQUIRE(static_cast<int64_t>(kv_heads) * page_size * head_dim < (1ll << 31), "paged_attention_prefill: a page of keys has 4 GB or more");
     MLL_REQUIRE(heads <= 65535, "paged_attention_prefill: more than 65535 heads");
     if (n_tiles == 0) return 0;
 #define MLL_PREFILL_CASE(TILES)                                                                                      \

@@ -515,6 +515,28 @@ def test_blocks_seen_whole_have_the_bits_of_their_runs(heads, kv_heads, hd, page
         assert torch.equal(run(), run(extras=nothing, out=torch.empty_like(t["q"]))), larger
 
 
+@pytest.mark.parametrize("heads,hd,bias", [(64, 128, False), (64, 128, True), (65, 144, False), (80, 112, False)])
+def test_prompts_in_pages_beyond_32_bits(heads, hd, bias):
+    """Pages of more than 2^31 elements, so that a page and its last heads begin beyond what 32 bits count in elements, and in bytes: the bits of pages of 16."""
+    k, length, large = kernels(), 300, 1 << 18
+    assert heads * large * hd >= 1 << 31
+    t, *_ = build_paged_case(np.random.default_rng(hd), torch.bfloat16, [length], [length], heads, heads, hd, 16, spare_pages=0)
+    tiles = torch.tensor(k.pair_query_tiles(query_tile_list([length], [length])), dtype=torch.int32, device=DEVICE)
+    extras = k.AttentionExtras(bias=torch.linspace(-1, 1, 50 * heads, device=DEVICE).view(50, heads)) if bias else None
+    run = lambda key, value, table: k.paged_attention_prefill(t["q"], key, value, table, tiles, t["pos"], hd ** -0.5, 0, heads, heads, hd, extras=extras,
+                                                              out=torch.empty_like(t["q"]))
+    want, order, last = run(t["k"], t["v"], t["table"]), t["table"][0, :-(-length // 16)].long(), 1
+    pools = []
+    for shape, small in ((key_page_shape, t["k"]), (value_page_shape, t["v"])):
+        pools.append(torch.empty(shape(last + 1, heads, large, hd), dtype=torch.bfloat16, device=DEVICE))
+        pools[-1][last, :, :len(order)] = small[order, :, 0].transpose(0, 1)
+    try:
+        assert torch.equal(run(*pools, torch.tensor([[last]], dtype=torch.int32, device=DEVICE)), want)
+    finally:
+        del pools
+        torch.cuda.empty_cache()
+
+
 @pytest.mark.parametrize("heads,kv_heads,dim,page,options", [
     (16, 4, 128, 16, dict(weights=True, temperature=True)), (9, 3, 96, 48, dict(bias=True, rot=64)), (5, 1, 16, 32, dict(values_normed=True, rot=16)),
     (7, 7, 256, 16, dict(norm_turned=True, rot=128)), (13, 2, 72, 16, dict(queries_only=True)), (8, 2, 112, 64, dict(norm_turned=True, rot=112, weights=True))])
