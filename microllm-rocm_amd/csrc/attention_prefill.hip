@@ -55,6 +55,33 @@ __device__ inline float reduce_lanes_32_apart(float value, Op op) {
 }
 
 
+// Which entry and head a workgroup takes, by its number. Workgroups go to the GPU's 8 dies (each with a second-level cache
+// of its own) by turns, in the order of their number. A class of 1, 2, 4 or 8 dies takes a class of heads, all heads of as many kv heads, and of those
+// the entries in the list's order (longest first), every head of an entry before the next one: a long prompt's keys then mostly come from
+// the die's own cache (numbered entry-first, where every die reads every kv head's keys: 8192 tokens at 7B sizes 680 -> 800 us,
+// 16384 2340 -> 2650), and the longest start first whatever the head. Where the kv heads do not divide, all heads are one class.
+struct PrefillOrder {
+    static constexpr int kDies = 8;
+    int entries, die_shift;      // a class of heads has 1 << die_shift dies
+    PrefillOrder(int entries_, int kv_heads) : entries(entries_), die_shift(0) {
+        const int classes = kv_heads % kDies == 0 ? kDies : (kDies % kv_heads == 0 ? kv_heads : 1);
+        while (classes << die_shift < kDies) ++die_shift;
+    }
+    // As many entries as give every die of a class as many workgroups; the last ones are none. (With one class the numbers are the items.)
+    int64_t rounded(int heads) const {
+        int64_t count = entries;
+        if (1 << die_shift < kDies)
+            while (count * (heads << die_shift) / kDies % (1 << die_shift) != 0) ++count;
+        return count;
+    }
+    __host__ __device__ void place(unsigned number, int heads, int& entry, int& head) const {
+        const unsigned class_heads = static_cast<unsigned>(heads << die_shift) / kDies, die = number % kDies;
+        const unsigned item = (number / kDies << die_shift) + (die & ((1u << die_shift) - 1));      // among the class's entries x heads
+        entry = item / class_heads;
+        head = (die >> die_shift) * class_heads + (item - entry * class_heads);
+    }
+};
+
 constexpr int kPrefillBiasRows = 4096;      // the longest bias table (one column of it is kept in LDS, 16 KB)
 
 // EXTRA: a bias by distance on the scores, a sink in the softmax, a factor on the result and a stride between its
@@ -65,7 +92,7 @@ constexpr int kPrefillBiasRows = 4096;      // the longest bias table (one colum
 template <int HD_TILES, bool EXTRA>
 __global__ __launch_bounds__(kPrefillThreads, 1) void paged_attention_prefill_kernel(
     const bf16* __restrict__ q, const bf16* __restrict__ k_cache, const bf16* __restrict__ v_cache,
-    const int32_t* __restrict__ block_table, int table_width, const int32_t* __restrict__ tiles,
+    const int32_t* __restrict__ block_table, int table_width, const int32_t* __restrict__ tiles, PrefillOrder order,
     const int32_t* __restrict__ positions, bf16* __restrict__ out, float scale, int window, int heads,
     int kv_heads, int page_size, MllAttentionExtras extras) {
     constexpr int HD = HD_TILES * 16;
@@ -83,25 +110,9 @@ __global__ __launch_bounds__(kPrefillThreads, 1) void paged_attention_prefill_ke
     __shared__ __align__(16) bf16 stage_odd[STAGE_ELEMENTS];
     __shared__ float bias_column[EXTRA ? kPrefillBiasRows : 1];
 
-    // Which entry and head this workgroup takes. Workgroups go to the GPU's 8 dies (each with a second-level cache
-    // of its own) by turns, in the order of their number; numbered entry-first, every die would read every kv
-    // head's keys and values. Instead a die takes the query heads of one kv head (of 8 / kv_heads dies each), the
-    // entries still in the list's order (longest first): a long prompt's keys then mostly come from the die's own
-    // cache (8192 tokens at 7B sizes: 800 -> 680 us; 16384: 2650 -> 2340). Where the numbers do not divide, the
-    // workgroups keep their plain numbering.
-    int entry_index = blockIdx.x, head = blockIdx.y;
-    {
-        constexpr int kDies = 8;
-        const int group = heads / kv_heads;
-        const int dies_per_kv_head = kv_heads <= kDies && kDies % kv_heads == 0 ? kDies / kv_heads : 0;
-        if (dies_per_kv_head > 0 && (gridDim.x * group) % dies_per_kv_head == 0) {
-            const int number = blockIdx.x + gridDim.x * blockIdx.y;
-            const int die = number % kDies, turn = number / kDies;
-            const int item = turn * dies_per_kv_head + die % dies_per_kv_head;      // among the kv head's entries x heads
-            entry_index = item / group;
-            head = (die / dies_per_kv_head) * group + item % group;
-        }
-    }
+    int entry_index, head;
+    order.place(blockIdx.x + gridDim.x * blockIdx.y, heads, entry_index, head);
+    if (entry_index >= order.entries) return;
     const int32_t* entry = tiles + 5 * entry_index;
     if (entry[2] <= 0 && entry[4] <= 0) return;      // an entry that only pads the list to a fixed length
     const int lane = threadIdx.x % kWave;
@@ -670,15 +681,16 @@ static int launch_prefill(const void* q, const void* k_cache, const void* v_cach
                           int table_width, const int32_t* tiles, int n_tiles, const int32_t* positions, void* out,
                           float scale, int window, int heads, int kv_heads, int page_size, const MllAttentionExtras* extras,
                           hipStream_t stream) {
-    const dim3 grid(n_tiles, heads);   // n_tiles: workgroups, of two tiles each
+    const PrefillOrder order(n_tiles, kv_heads);   // n_tiles: entries, of two tiles each
+    const dim3 grid(static_cast<unsigned>(order.rounded(heads)), heads);
     if (extras) {
         paged_attention_prefill_kernel<HD_TILES, true><<<grid, kPrefillThreads, 0, stream>>>(
             static_cast<const bf16*>(q), static_cast<const bf16*>(k_cache), static_cast<const bf16*>(v_cache), block_table,
-            table_width, tiles, positions, static_cast<bf16*>(out), scale, window, heads, kv_heads, page_size, *extras);
+            table_width, tiles, order, positions, static_cast<bf16*>(out), scale, window, heads, kv_heads, page_size, *extras);
     } else {
         paged_attention_prefill_kernel<HD_TILES, false><<<grid, kPrefillThreads, 0, stream>>>(
             static_cast<const bf16*>(q), static_cast<const bf16*>(k_cache), static_cast<const bf16*>(v_cache), block_table,
-            table_width, tiles, positions, static_cast<bf16*>(out), scale, window, heads, kv_heads, page_size,
+            table_width, tiles, order, positions, static_cast<bf16*>(out), scale, window, heads, kv_heads, page_size,
             MllAttentionExtras{nullptr, 0, nullptr, 1.0f, 0});
     }
     return check_launch("paged_attention_prefill");
@@ -690,7 +702,14 @@ using namespace mll;
 
 extern "C" int mll_paged_attention_prefill_tile() { return kPrefillTile; }
 
-
+extern "C" int64_t mll_paged_attention_prefill_order(int entries, int heads, int kv_heads, int64_t number) {
+    const PrefillOrder order(entries, kv_heads);
+    const int64_t workgroups = order.rounded(heads) * heads;
+    if (number < 0 || number >= workgroups) return -1;
+    int entry, head;
+    order.place(static_cast<unsigned>(number), heads, entry, head);
+    return entry < entries ? static_cast<int64_t>(entry) * heads + head : workgroups;
+}
 
 extern "C" int mll_paged_attention_prefill_bias_rows() { return kPrefillBiasRows; }
 

@@ -122,6 +122,8 @@ int mll_paged_attention_prefill(const void* q, const void* k_cache, const void* 
                                 int n_tiles, const int32_t* positions, void* out, float scale, int window,
                                 int heads, int kv_heads, int head_dim, int page_size, hipStream_t stream);
 int mll_paged_attention_prefill_tile();
+// For tests: entry * heads + query head that workgroup `number` of a launch takes; the number of workgroups for one that takes none, -1 beyond them.
+int64_t mll_paged_attention_prefill_order(int entries, int heads, int kv_heads, int64_t number);
 
 // out[t, c] = act(gate[t, c]) * up[t, c]; gate and up rows are `in_stride` elements apart. act: 0 SiLU, 2 the tanh gelu.
 int mll_gated_activation(const void* gate, const void* up, int64_t in_stride, void* out, int dtype,

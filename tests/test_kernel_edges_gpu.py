@@ -1,4 +1,5 @@
 """The kernels at the sizes where their tiles, their remainders and the choice between them can go wrong."""
+import ctypes
 import math
 
 import numpy as np
@@ -6,6 +7,8 @@ import pytest
 import torch
 
 from test_kernels_gpu import DEVICE, build_paged_case, kernels, key_page_shape, query_tile_list, reference_attention, to_bf16_exact, tolerance, value_page_shape
+
+from microllm_rocm_amd.ops import library
 
 pytestmark = pytest.mark.gpu
 
@@ -497,6 +500,24 @@ def test_prompts_in_tiles_of_half_the_queries_have_the_same_bits(heads, kv_heads
         pairs = torch.tensor(k.pair_query_tiles(tiles, adjacent=window > 0), dtype=torch.int32, device=DEVICE)
         results.append(k.paged_attention_prefill(t["q"], t["k"], t["v"], t["table"], pairs, t["pos"], hd ** -0.5, window, heads, kv_heads, hd))
     assert torch.equal(*results)
+
+
+@pytest.mark.parametrize("heads,kv_heads", [(28, 4), (14, 2), (16, 4), (64, 8), (9, 1), (16, 16), (48, 24), (12, 6), (15, 5), (7, 7)])
+def test_prefill_workgroups_take_the_longest_entries_of_all_heads_first(heads, kv_heads):
+    """Every entry and head once, whatever their numbers; of a round over the eight dies none takes an earlier entry than the round before; and where the kv
+    heads divide among the dies, a die keeps to its own."""
+    order = library.load().mll_paged_attention_prefill_order
+    for entries in (1, 2, 3, 7, 17, 33, 34):
+        taken, number = [], 0
+        while (item := order(entries, heads, kv_heads, ctypes.c_int64(number))) >= 0:
+            taken.append(item)
+            number += 1
+        assert sorted(taken) == list(range(entries * heads)) + [len(taken)] * (len(taken) - entries * heads)
+        rounds = [[item // heads for item in taken[i:i + 8] if item < entries * heads] for i in range(0, len(taken), 8)]
+        assert all(max(now) <= min(after) for now, after in zip(rounds, rounds[1:]) if now and after)
+        if 8 % kv_heads == 0 or kv_heads % 8 == 0:
+            own = [{item % heads // (heads // kv_heads) for item in taken[die::8] if item < entries * heads} for die in range(8)]
+            assert all(len(kv) <= max(1, kv_heads // 8) for kv in own)
 
 
 @pytest.mark.parametrize("heads,kv_heads,hd,page_size", [(4, 2, 16, 16), (3, 1, 48, 48), (14, 2, 64, 32), (6, 3, 96, 16), (7, 7, 112, 64), (28, 4, 128, 16)])
