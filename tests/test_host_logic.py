@@ -67,6 +67,8 @@ def test_query_tiles_go_in_twos_that_walk_about_as_many_keys():
     assert keys == sorted(keys, reverse=True), "the longest first"
     # under a window neighbours go together
     adjacent = kernels.pair_query_tiles(list(tiles), adjacent=True)
+    walked = [max(position[a] + ca, position[b] + cb if cb else 0) for _, a, ca, b, cb in adjacent]
+    assert walked == sorted(walked, reverse=True), "the longest first: of neighbours the later one's keys"
     assert sorted(pair[1:] for pair in adjacent if pair[0] == 0) == [(offset, 128, offset + 128, 128) for offset in range(0, 2048, 256)]
     assert sorted(pair[1:] for pair in adjacent if pair[0] == 1) == [(2048, 128, 2048 + 128, 128), (2048 + 256, 44, 0, 0)]
 
@@ -216,8 +218,9 @@ def test_neighbouring_tiles_share_a_workgroup_where_a_step_has_more_than_a_round
     assert not QueryTilePlanner(False).neighbours([100000]) and QueryTilePlanner(True).neighbours([2])
     host = SimpleNamespace(counts=[2305], cu=[0, 2305], starts=[0], totals=[2305], single_tokens_only=False)
     tiles = planner.plan(host)[0]["tiles"]
-    assert tiles[0].tolist() == [0, 2048, 128, 2176, 128] and tiles[1].tolist() == [0, 1792, 128, 1920, 128]
+    assert tiles[0].tolist() == [0, 2304, 1, 0, 0] and tiles[1].tolist() == [0, 2048, 128, 2176, 128]
     assert sorted(tiles[:, 2] + tiles[:, 4]) == [1] + [256] * 9
+    assert [max(a + ca, b + cb) for _, a, ca, b, cb in tiles.tolist()] == [2305] + list(range(2304, 0, -256)), "by the keys they walk"
 
 
 @pytest.mark.parametrize("tokens,heads,kv_heads,head_dim,chunks,dtype,splits", [
