@@ -89,7 +89,7 @@ constexpr int kPrefillBiasRows = 4096;      // the longest bias table (one colum
 // by scale); a run of keys all of which lie `longest` or further behind all of the wave's tokens takes the last
 // row's value for every score, any other run looks every score's distance up. The sink is where the running
 // maximum and sum start. Without EXTRA the kernel is what it was.
-template <int HD_TILES, bool EXTRA>
+template <int HD_TILES, bool EXTRA, bool WHOLE>
 __global__ __launch_bounds__(kPrefillThreads, 1) void paged_attention_prefill_kernel(
     const bf16* __restrict__ q, const bf16* __restrict__ k_cache, const bf16* __restrict__ v_cache,
     const int32_t* __restrict__ block_table, int table_width, const int32_t* __restrict__ tiles, PrefillOrder order,
@@ -469,7 +469,7 @@ __global__ __launch_bounds__(kPrefillThreads, 1) void paged_attention_prefill_ke
     // run 1's scores and between run 0's values stand the weights (exponentials, sums, roundings) of run 0 and run 1. The numbers are process_keys' own,
     // run by run. The order is the source's: the empty asm statements and the scheduling barriers keep the compiler from gathering the
     // exponentials in front of the products, where nothing overlaps them. 16301 tokens, 28 heads of 128 over 4: 2.25 -> 2.12 ms; 2048 tokens 59 -> 56 us.
-    constexpr bool WHOLE_BLOCKS = !EXTRA && STEPS == 4;      // (with biases and caps the registers do not suffice: 71 -> 79 us)
+    constexpr bool WHOLE_BLOCKS = WHOLE && !EXTRA && STEPS == 4;      // (with biases and caps the registers do not suffice: 71 -> 79 us)
     auto process_block = [&](const bf16* stage) __attribute__((always_inline)) {
         constexpr int SCORES = 2 * K_STEPS, VALUES = 4 * D_BLOCKS, PRODUCTS = 2 * (SCORES + VALUES);
         constexpr int kAhead = 4, RING = kAhead + 1;
@@ -676,6 +676,11 @@ __global__ __launch_bounds__(kPrefillThreads, 1) void paged_attention_prefill_ke
     }
 }
 
+// Heads of up to 32 take 104 registers without whole blocks and 154 with them, so that two workgroups share a compute unit without, one with them: whole blocks
+// only in steps that give no unit a second workgroup (28 heads of 16 over 4, 2000 tokens, 224 workgroups, 30.7 us without and 28.5 with; 2305, 280, 34.8 and 43.0;
+// of 32 30.2 and 27.6, 35.5 and 42.4).
+constexpr int kTwoAUnitTiles = 2, kPrefillUnits = 256;
+
 template <int HD_TILES>
 static int launch_prefill(const void* q, const void* k_cache, const void* v_cache, const int32_t* block_table,
                           int table_width, const int32_t* tiles, int n_tiles, const int32_t* positions, void* out,
@@ -683,16 +688,19 @@ static int launch_prefill(const void* q, const void* k_cache, const void* v_cach
                           hipStream_t stream) {
     const PrefillOrder order(n_tiles, kv_heads);   // n_tiles: entries, of two tiles each
     const dim3 grid(static_cast<unsigned>(order.rounded(heads)), heads);
+#define MLL_PREFILL_LAUNCH(EXTRA, WHOLE, EXTRAS)                                                                              \
+    paged_attention_prefill_kernel<HD_TILES, EXTRA, WHOLE><<<grid, kPrefillThreads, 0, stream>>>(                               \
+        static_cast<const bf16*>(q), static_cast<const bf16*>(k_cache), static_cast<const bf16*>(v_cache), block_table,          \
+        table_width, tiles, order, positions, static_cast<bf16*>(out), scale, window, heads, kv_heads, page_size, EXTRAS)
+    const MllAttentionExtras none{nullptr, 0, nullptr, 1.0f, 0};
     if (extras) {
-        paged_attention_prefill_kernel<HD_TILES, true><<<grid, kPrefillThreads, 0, stream>>>(
-            static_cast<const bf16*>(q), static_cast<const bf16*>(k_cache), static_cast<const bf16*>(v_cache), block_table,
-            table_width, tiles, order, positions, static_cast<bf16*>(out), scale, window, heads, kv_heads, page_size, *extras);
+        MLL_PREFILL_LAUNCH(true, false, *extras);
+    } else if (HD_TILES <= kTwoAUnitTiles && static_cast<int64_t>(n_tiles) * heads > kPrefillUnits) {
+        MLL_PREFILL_LAUNCH(false, (HD_TILES > kTwoAUnitTiles), none);
     } else {
-        paged_attention_prefill_kernel<HD_TILES, false><<<grid, kPrefillThreads, 0, stream>>>(
-            static_cast<const bf16*>(q), static_cast<const bf16*>(k_cache), static_cast<const bf16*>(v_cache), block_table,
-            table_width, tiles, order, positions, static_cast<bf16*>(out), scale, window, heads, kv_heads, page_size,
-            MllAttentionExtras{nullptr, 0, nullptr, 1.0f, 0});
+        MLL_PREFILL_LAUNCH(false, true, none);
     }
+#undef MLL_PREFILL_LAUNCH
     return check_launch("paged_attention_prefill");
 }
 

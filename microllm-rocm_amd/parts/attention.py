@@ -34,7 +34,9 @@ class QueryTilePlanner:
     workgroups (of the ``heads`` query heads) than compute units. Two neighbours walk their keys together, a late and an early tile
     for the early one's keys only, so neighbours' workgroups bring in two thirds of the blocks of keys, and started longest first
     they end together once there is more than a round of them (28 heads of 128: 3000 tokens, 336 workgroups, 131 -> 104 us, 16301 2.13 ->
-    1.87 ms; in one round the last of a prompt's workgroups is the step's time: 2048 tokens, 224 workgroups, 56 -> 70 us).
+    1.87 ms; in one round the last of a prompt's workgroups is the step's time: 2048 tokens, 224 workgroups, 56 -> 70 us). Of heads of up to 32
+    a unit takes two (``head_dim``: of kernels without extras), so that a round has twice as many (28 heads of 16: 2305 tokens, 280 workgroups, 34.8 -> 42.3 us
+    with neighbours, 6000, 672, 167 -> 132).
 
     Where the tiles of 128 would give fewer workgroups (of the ``heads`` query heads) than half the compute units, requests of more than one such
     tile have tiles of 64 queries: twice the workgroups, with one wave a SIMD instead of two, which share its exponentials (a pass of
@@ -45,10 +47,11 @@ class QueryTilePlanner:
     the requests listed there."""
     padding = {"tiles": 0, "single_tokens": -1}      # an entry of two empty tiles; a row that is none: both passed over
 
-    def __init__(self, windowed: bool, heads: int = 0):
+    def __init__(self, windowed: bool, heads: int = 0, head_dim: int = 0):
         self.windowed = windowed
         self.heads = heads      # 0: whole tiles always
-        self.key = ("paged_attention_query_tiles", windowed, heads)
+        self.at_once = kernels.COMPUTE_UNITS * (2 if 0 < head_dim <= kernels.PREFILL_TWO_A_UNIT else 1)
+        self.key = ("paged_attention_query_tiles", windowed, heads, self.at_once)
 
     def tile_rows(self, counts):
         """The queries a tile has of every request, by how many each brings."""
@@ -58,7 +61,7 @@ class QueryTilePlanner:
 
     def neighbours(self, counts):
         """Whether neighbouring tiles share a workgroup, by how many tokens each request brings."""
-        return self.windowed or self.heads * sum((-(-count // kernels.QUERY_TILE) + 1) // 2 for count in counts) > kernels.COMPUTE_UNITS
+        return self.windowed or self.heads * sum((-(-count // kernels.QUERY_TILE) + 1) // 2 for count in counts) > self.at_once
 
     def plan(self, host):
         counts, cu = host.counts, host.cu
@@ -94,7 +97,7 @@ class PagedAttention(Mixer):
             raise ValueError("num_heads must divide into num_kv_heads groups")
         position = p.get("position")
         self.position = build_part("position", position, runtime) if position is not None else None
-        self.planner = QueryTilePlanner(bool(self.window), self.heads)
+        self.planner = QueryTilePlanner(bool(self.window), self.heads, self.head_dim)
         self.qkv_weight: Optional[torch.Tensor] = None
         self.qkv_bias_vector: Optional[torch.Tensor] = None
         self.o_weight: Optional[torch.Tensor] = None

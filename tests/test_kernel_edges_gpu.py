@@ -502,6 +502,21 @@ def test_prompts_in_tiles_of_half_the_queries_have_the_same_bits(heads, kv_heads
     assert torch.equal(*results)
 
 
+@pytest.mark.parametrize("heads,kv_heads,hd", [(28, 4, 16), (33, 3, 32), (28, 4, 48)])
+def test_prompts_have_the_same_bits_in_steps_of_few_and_of_many_workgroups(heads, kv_heads, hd):
+    """Heads of up to 32 are worked on without whole blocks from 257 workgroups on: all of a step's entries in one launch, and by few."""
+    k, lengths = kernels(), [1300, 517, 129, 1100]
+    t, *_ = build_paged_case(np.random.default_rng(hd), torch.bfloat16, lengths, lengths, heads, kv_heads, hd, 16)
+    tiles = torch.tensor(k.pair_query_tiles(query_tile_list(lengths, lengths)), dtype=torch.int32, device=DEVICE)
+    few = 256 // heads
+    assert len(tiles) * heads > 256
+    run = lambda some, out: k.paged_attention_prefill(t["q"], t["k"], t["v"], t["table"], some, t["pos"], hd ** -0.5, 0, heads, kv_heads, hd, out=out)
+    parts = torch.empty_like(t["q"])
+    for first in range(0, len(tiles), few):
+        run(tiles[first:first + few].contiguous(), parts)
+    assert torch.equal(run(tiles, torch.empty_like(t["q"])), parts)
+
+
 @pytest.mark.parametrize("heads,kv_heads", [(28, 4), (14, 2), (16, 4), (64, 8), (9, 1), (16, 16), (48, 24), (12, 6), (15, 5), (7, 7)])
 def test_prefill_workgroups_take_the_longest_entries_of_all_heads_first(heads, kv_heads):
     """Every entry and head once, whatever their numbers; of a round over the eight dies none takes an earlier entry than the round before; and where the kv
