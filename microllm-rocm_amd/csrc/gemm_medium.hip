@@ -246,14 +246,23 @@ static int balanced_tiles(int n_tiles, int splits, int parts, int stages, int ro
     return best;
 }
 
+// Each split takes whole stages, so that the stages of a sum begin at the same k whatever the split.
+static int stages_of_a_split(int k, int splits) {
+    const int stages = ((k + 31) / 32 + kStepsPerStage - 1) / kStepsPerStage;
+    return (stages + splits - 1) / splits;
+}
+
+static int tiles_of(int m, int n, int k, int splits, int most) {
+    const int each = stages_of_a_split(k, splits), parts = (stages_of_a_split(k, 1) + each - 1) / each;
+    return (k + 31) / 32 > kMostSteps ? 4 : balanced_tiles((n + 15) / 16, splits, parts, each, (m + 15) / 16, most);
+}
+
 template <int MT, int EPILOGUE>
 static void launch_rows(const bf16* a, const bf16* w, void* out, int m, int n, int k, int most_tiles, int splits, hipStream_t stream) {
     const int n_tiles = (n + 15) / 16, k_steps = (k + 31) / 32;
-    // Each split takes whole stages, so that the stages of a sum begin at the same k whatever the split.
-    const int stages = (k_steps + kStepsPerStage - 1) / kStepsPerStage;
-    const int stages_per_split = (stages + splits - 1) / splits, steps_per_split = stages_per_split * kStepsPerStage;
+    const int steps_per_split = stages_of_a_split(k, splits) * kStepsPerStage;
     const bool far = k_steps > kMostSteps;
-    const int tiles = far ? 4 : balanced_tiles(n_tiles, splits, (stages + stages_per_split - 1) / stages_per_split, stages_per_split, MT, most_tiles);
+    const int tiles = tiles_of(m, n, k, splits, most_tiles);
     const dim3 grid((n_tiles + tiles - 1) / tiles, splits);
     const size_t lds = 2 * MT * kStepsPerStage * kWave * sizeof(uintx4);
     const auto launch = [&](auto tiles_a_wave, auto waves) {
@@ -291,6 +300,10 @@ static int launch_medium(const void* a, const void* w_packed, void* out, int m, 
 }  // namespace mll
 
 using namespace mll;
+
+extern "C" int mll_gemm_medium_tiles(int m, int n, int k, int tiles_per_wave, int waves, int splits) {
+    return medium::tiles_of(m, n, k, splits, tiles_per_wave * waves);
+}
 
 extern "C" int mll_gemm_medium(const void* a, const void* w_packed, void* out, int epilogue, int m, int n, int k,
                                int tiles_per_wave, int waves, int splits, hipStream_t stream) {

@@ -231,6 +231,8 @@ struct MllSkinnyExtras {
 // caller adds in order. The order of additions is fixed by (n, k, splits).
 int mll_gemm_medium(const void* a, const void* w_packed, void* out, int epilogue, int m, int n, int k,
                     int tiles_per_wave, int waves, int splits, hipStream_t stream);
+// For tests: the tiles of 16 weight rows that a workgroup of that call takes (up to 4: four waves of one, up to 8: eight of one, else eight of two).
+int mll_gemm_medium_tiles(int m, int n, int k, int tiles_per_wave, int waves, int splits);
 
 // The same product for many rows: 256 x 256 tiles of C per workgroup, pieces of A and W brought into LDS by
 // direct global-to-LDS loads. A is row-major [m, k] with k a multiple of 32; epilogues 0, 1, 2 and 5 of

@@ -279,10 +279,13 @@ def test_streaming_product_of_the_longest_reductions(n):
         assert torch.equal(kernels().gemm_skinny(x[:m].contiguous(), packed, n, "bf16"), want[:m].to(torch.bfloat16))
 
 
-@pytest.mark.parametrize("n", [40, 16 * 300, 16 * 700 - 8, 16 * 2100])      # workgroups of four waves, of eight, of eight with two tiles each
+# Tiles of a workgroup, unsplit and in three parts: up to four, workgroups of four waves; up to eight, of eight; more, of eight with two tiles each.
+@pytest.mark.parametrize("n,tiles,of_parts", [(40, 1, 1), (16 * 300, 2, 4), (16 * 700 - 8, 3, 9), (16 * 1500 - 8, 6, 12), (16 * 2100, 9, 9)])
 @pytest.mark.parametrize("k", [8, 256, 264, 512, 520, 768, 1000, 1280])       # one to five stages of 256, whole and begun
-def test_product_for_64_rows_of_any_number_of_stages(n, k):
+def test_product_for_64_rows_of_any_number_of_stages(n, tiles, of_parts, k):
     """Two stages a round and what is left of an odd number; sums of whole numbers, which have no rounding to differ in."""
+    chosen = library.load().mll_gemm_medium_tiles
+    assert all(chosen(m, n, k, 2, 8, 1) == tiles for m in (17, 32, 33, 64)) and chosen(64, n, 1000, 2, 8, 3) == of_parts
     generator = torch.Generator(device=DEVICE).manual_seed(n + k)
     x, w = whole_numbers(generator, 64, k), whole_numbers(generator, n, k)
     packed, want = kernels().pack_weight(w), x.float() @ w.float().T
