@@ -275,19 +275,19 @@ __global__ __launch_bounds__(kDecodeThreads, HD_TILES <= 8 ? 2 : 1) void paged_a
         int page[2] = {page_of(pair * 32), page_of(pair * 32 + 16)};
         int following = min(pair + kDecodeWaves, last);
         int next_page[2] = {page_of(following * 32), page_of(following * 32 + 16)};
-
         load_pair(pair, page, k_first, v_first, bias_first);
         // Two pairs a round, and what is left of an odd number after the rounds: were the loop left between the two, the compiler would think that
         // it comes round with the second pair's loads on their way, and wait for all of them at the start of every round (64 ragged requests of at
         // most 3000 positions, 28 heads of 128 over 4, in 4 splits 35.3 -> 32.1 us; one of 60, 14 heads of 64 over 2, 3.87 -> 3.54; one of 100, 16
-        // heads of 256 over 4, 8.9 -> 7.7; heads of 256 of 40 requests of 500 unsplit 21.9 -> 22.6, the one size found slower by more than 2 %).
+        // heads of 256 over 4, 8.9 -> 7.7). Heads of 256 gain and lose, by the splits that steps take from 0.86 to 1.04 of the time and 0.98 on the mean
+        // of 39 steps (16 over 4: 8 requests of 3000 25.0 -> 22.5, 64 of 600 31.8 -> 29.4, 10 of 1500 19.9 -> 20.5, 40 of 500 19.4 -> 20.2); long ones
+        // unsplit, which no step takes, lose up to 7 %.
         const int pairs = (last - pair) / kDecodeWaves + 1;
         for (int round = 0; round < pairs / 2; ++round) {
             int after = min(following + kDecodeWaves, last);
             page[0] = page_of(after * 32);
             page[1] = page_of(after * 32 + 16);
             load_pair(following, next_page, k_second, v_second, bias_second);
-
             attend_pair(pair, k_first, v_first, bias_first);
             pair = following;
             following = after;
@@ -296,7 +296,6 @@ __global__ __launch_bounds__(kDecodeThreads, HD_TILES <= 8 ? 2 : 1) void paged_a
             next_page[0] = page_of(after * 32);
             next_page[1] = page_of(after * 32 + 16);
             load_pair(following, page, k_first, v_first, bias_first);
-
             attend_pair(pair, k_second, v_second, bias_second);
             pair = following;
             following = after;

@@ -5,8 +5,9 @@
 // are the 32 columns of v_mfma_f32_32x32x16_bf16. Every SIMD thus has a wave of either tile, whose matrix and
 // vector work overlap. The host pairs a tile that sees many keys with one that sees few, so that every workgroup
 // walks about as many keys and the compute units finish together (under a causal mask the last tile of a prompt
-// has as many times the work of the first as there are tiles), and neighbouring tiles under a window, which read
-// nearly the same keys. Both tiles read the same keys from LDS. The second tile may be empty.
+// has as many times the work of the first as there are tiles), and neighbouring tiles, which read nearly the same
+// keys, under a window and in steps of more workgroups than run at once, where those with the most keys start
+// first. Both tiles read the same keys from LDS. The second tile may be empty.
 // The workgroup walks the keys its tokens can see in blocks of 128 (64 for head sizes above 128): the block's key
 // and value tiles are copied from the pages straight into LDS as they lie there (the pages are in MFMA order,
 // cache_layout.h), the next block's being on its way while this one is used. The two stages are two LDS
@@ -45,16 +46,6 @@ union PFrag8 {
     uint4 raw;
 };
 
-// op over the two lanes {l, l ^ 32} of a wave, both of which get the result (v_permlane32_swap of gfx950).
-template <typename Op>
-__device__ inline float reduce_lanes_32_apart(float value, Op op) {
-    const unsigned bits = __builtin_bit_cast(unsigned, value);
-    const auto halves = __builtin_amdgcn_permlane32_swap(bits, bits, false, false);
-    const unsigned low = halves[0], high = halves[1];
-    return op(__builtin_bit_cast(float, low), __builtin_bit_cast(float, high));
-}
-
-
 // Which entry and head a workgroup takes, by its number. Workgroups go to the GPU's 8 dies (each with a second-level cache
 // of its own) by turns, in the order of their number. A class of 1, 2, 4 or 8 dies takes a class of heads, all heads of as many kv heads, and of those
 // the entries in the list's order (longest first), every head of an entry before the next one: a long prompt's keys then mostly come from
@@ -88,7 +79,7 @@ constexpr int kPrefillBiasRows = 4096;      // the longest bias table (one colum
 // rows (MllAttentionExtras). The bias column of the workgroup's head lies in LDS in the scores' own units (divided
 // by scale); a run of keys all of which lie `longest` or further behind all of the wave's tokens takes the last
 // row's value for every score, any other run looks every score's distance up. The sink is where the running
-// maximum and sum start. Without EXTRA the kernel is what it was.
+// maximum and sum start. WHOLE: blocks that a wave sees whole are worked on as one (process_block).
 template <int HD_TILES, bool EXTRA, bool WHOLE>
 __global__ __launch_bounds__(kPrefillThreads, 1) void paged_attention_prefill_kernel(
     const bf16* __restrict__ q, const bf16* __restrict__ k_cache, const bf16* __restrict__ v_cache,
@@ -147,7 +138,7 @@ __global__ __launch_bounds__(kPrefillThreads, 1) void paged_attention_prefill_ke
     auto tile_seen = [&](int tile_key) {      // some of its 16 keys
         return (tile_key + 15 >= range_low[0] && tile_key <= range_last[0]) || (tile_key + 15 >= range_low[1] && tile_key <= range_last[1]);
     };
-    // A block all of whose keys one tile's tokens can see (most blocks) needs no checks per key tile.
+    // A block all of whose keys one tile's tokens can see (most blocks): nothing in it is to be cleared.
     auto inside = [&](int block) {
         const int first = block * BLOCK_KEYS, last = first + BLOCK_KEYS - 1;
         return (first >= range_low[0] && last <= range_last[0]) || (first >= range_low[1] && last <= range_last[1]);
@@ -236,7 +227,7 @@ __global__ __launch_bounds__(kPrefillThreads, 1) void paged_attention_prefill_ke
     constexpr bool FULL_PASSES = HALF_CHUNKS % kPrefillThreads == 0;      // every pass of every wave lies within the block
     auto wanted = [&](int block, int pass) {      // whether the tile is brought in: some token sees some of it
         const int tile_key = block * BLOCK_KEYS + 16 * tile_of(pass);
-        return (FULL_PASSES || tile_of(pass) < BLOCK_TILES) && tile_key <= group_last && (inside(block) || tile_seen(tile_key));
+        return (FULL_PASSES || tile_of(pass) < BLOCK_TILES) && tile_key <= group_last && tile_seen(tile_key);
     };
     // The pages of a block's tiles are looked up one block ahead of the tiles themselves, so that no load waits
     // for another; where a wave's lanes stay within one tile, one load looks up the pages of all its passes, a lane
@@ -256,8 +247,9 @@ __global__ __launch_bounds__(kPrefillThreads, 1) void paged_attention_prefill_ke
             if (want) pages[i] = table[page_shift >= 0 ? tile_index >> page_shift : tile_index / tiles_per_page];
         }
     };
-    // The loads are buffer loads: a global load into LDS is encoded as a flat one, and while such a load is under way the compiler waits for all reads
-    // from LDS and all loads, not for the ones it needs (16301 tokens, 28 heads of 128 over 4: 2.34 -> 2.25 ms).
+    // Where a wave's lanes stay within one tile the loads are buffer loads: a global load into LDS is encoded as a flat one, and while such a load is
+    // under way the compiler waits for all reads from LDS and all loads, not for the ones it needs (16301 tokens, 28 heads of 128 over 4: 2.34 -> 2.25 ms).
+    // Other head sizes (odd multiples of 16) have a page and an address a lane, which one descriptor does not cover, and keep the flat loads.
     auto fetch = [&](int block, bf16* stage) __attribute__((always_inline)) {      // after look_up(block)
         if constexpr (UNIFORM) {
             const int tile_index = block * BLOCK_TILES + (lane_pass * kPrefillThreads + wave_chunk) / TILE_CHUNKS;
@@ -341,8 +333,8 @@ __global__ __launch_bounds__(kPrefillThreads, 1) void paged_attention_prefill_ke
     // column / 16), 8 dims (chunk 2 ks + half) per lane. Second: row = dim `column` of a block of 32 dims; the
     // lane's 8 k-slots are the keys its scores came for, positions 8 half .. + 7 of the tile, one read of 16 bytes;
     // the 64 lanes read 1024 consecutive bytes, which LDS gives without bank conflicts.
-    // The reads need no wait for the loads into the other stage. While those were flat loads, whose end the compiler cannot tell from that of
-    // reads of LDS, it waited for all of them here, or, with the addresses formed as one sum, elsewhere; buffer loads are counted apart.
+    // The reads need no wait for the loads into the other stage. Of flat loads the compiler cannot tell the end from that of reads of LDS, and waits
+    // for all of them here, or, with the addresses formed as one sum, elsewhere; buffer loads are counted apart.
     const int key_of_row = (column & ~12) | ((column & 4) << 1) | ((column & 8) >> 1);
     auto process_keys = [&](auto masked_tag, auto halves_tag, const bf16* stage, int first_run, int key0) __attribute__((always_inline)) {
         constexpr bool MASKED = decltype(masked_tag)::value;
@@ -469,6 +461,7 @@ __global__ __launch_bounds__(kPrefillThreads, 1) void paged_attention_prefill_ke
     // run 1's scores and between run 0's values stand the weights (exponentials, sums, roundings) of run 0 and run 1. The numbers are process_keys' own,
     // run by run. The order is the source's: the empty asm statements and the scheduling barriers keep the compiler from gathering the
     // exponentials in front of the products, where nothing overlaps them. 16301 tokens, 28 heads of 128 over 4: 2.25 -> 2.12 ms; 2048 tokens 59 -> 56 us.
+    // (Head sizes that keep flat loads gain as much: 2000 tokens of 16 heads of 48, 80 and 112 over 4 38.4 -> 36.0, 48.3 -> 45.2 and 56.7 -> 54.2 us.)
     constexpr bool WHOLE_BLOCKS = WHOLE && !EXTRA && STEPS == 4;      // (with biases and caps the registers do not suffice: 71 -> 79 us)
     auto process_block = [&](const bf16* stage) __attribute__((always_inline)) {
         constexpr int SCORES = 2 * K_STEPS, VALUES = 4 * D_BLOCKS, PRODUCTS = 2 * (SCORES + VALUES);

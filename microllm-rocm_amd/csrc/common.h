@@ -37,21 +37,27 @@ __device__ inline float rotate_second(float x1, float x2, float c, float s) { re
 // then a barrier, if another wave's loads are read).
 __device__ inline void wait_for_loads() { asm volatile("s_waitcnt vmcnt(0)" ::: "memory"); }
 
-// op over the four lanes {l, l ^ 16, l ^ 32, l ^ 48} of a wave, every one of which gets the result: two
-// exchanges on the vector unit (v_permlane16_swap, v_permlane32_swap of gfx950) instead of four trips through
-// LDS. op must be commutative. (The elements of the builtins' result are copied to scalars before they are
-// reinterpreted: a reinterpretation of the element expression itself reads element 0 twice with this compiler.)
+// op over the two lanes {l, l ^ 32}, or {l, l ^ 16}, of a wave, both of which get the result: an exchange on the vector unit
+// (v_permlane32_swap, v_permlane16_swap of gfx950). op must be commutative. (The elements of the builtins' result are copied to scalars before they
+// are reinterpreted: a reinterpretation of the element expression itself reads element 0 twice with this compiler.)
 template <typename Op>
-__device__ inline float reduce_lanes_16_apart(float value, Op op) {
+__device__ inline float reduce_lanes_32_apart(float value, Op op) {
     const unsigned bits = __builtin_bit_cast(unsigned, value);
-    const auto rows = __builtin_amdgcn_permlane16_swap(bits, bits, false, false);
-    const unsigned even = rows[0], odd = rows[1];
-    value = op(__builtin_bit_cast(float, even), __builtin_bit_cast(float, odd));
-    const unsigned joined = __builtin_bit_cast(unsigned, value);
-    const auto halves = __builtin_amdgcn_permlane32_swap(joined, joined, false, false);
+    const auto halves = __builtin_amdgcn_permlane32_swap(bits, bits, false, false);
     const unsigned low = halves[0], high = halves[1];
     return op(__builtin_bit_cast(float, low), __builtin_bit_cast(float, high));
 }
+template <typename Op>
+__device__ inline float reduce_rows_apart(float value, Op op) {
+    const unsigned bits = __builtin_bit_cast(unsigned, value);
+    const auto rows = __builtin_amdgcn_permlane16_swap(bits, bits, false, false);
+    const unsigned even = rows[0], odd = rows[1];
+    return op(__builtin_bit_cast(float, even), __builtin_bit_cast(float, odd));
+}
+
+// op over the four lanes {l, l ^ 16, l ^ 32, l ^ 48} of a wave, every one of which gets the result, instead of four trips through LDS.
+template <typename Op>
+__device__ inline float reduce_lanes_16_apart(float value, Op op) { return reduce_lanes_32_apart(reduce_rows_apart(value, op), op); }
 __device__ inline float max_lanes_16_apart(float value) {
     return reduce_lanes_16_apart(value, [](float a, float b) { return fmaxf(a, b); });
 }
@@ -141,8 +147,7 @@ __device__ inline float softcap_fast(float value, float cap, float inverse_cap) 
     return fmaf(-2.0f * cap, __builtin_amdgcn_rcpf(1.0f + __expf(2.0f * value * inverse_cap)), cap);
 }
 
-// `value` of lane l ^ DISTANCE, for every lane (of a whole wave), without a way through LDS: two halves or rows exchanged (v_permlane32_swap,
-// v_permlane16_swap), or DPP within a row of 16.
+// `value` of lane l ^ DISTANCE, for every lane (of a whole wave), DISTANCE within a row of 16: by DPP, without a way through LDS.
 template <int CONTROL>
 __device__ inline int dpp(int value) { return __builtin_amdgcn_update_dpp(0, value, CONTROL, 0xf, 0xf, false); }
 template <int DISTANCE>
@@ -161,14 +166,7 @@ __device__ inline float lane_across(float value) {
 // (__shfl_xor) each of them is a trip of its own for the wave, which kernels of few waves wait for.
 template <typename Op>
 __device__ inline float reduce_wave(float value, Op op) {
-    const unsigned bits = __builtin_bit_cast(unsigned, value);
-    const auto halves = __builtin_amdgcn_permlane32_swap(bits, bits, false, false);
-    const unsigned low = halves[0], high = halves[1];
-    value = op(__builtin_bit_cast(float, low), __builtin_bit_cast(float, high));
-    const unsigned joined = __builtin_bit_cast(unsigned, value);
-    const auto rows = __builtin_amdgcn_permlane16_swap(joined, joined, false, false);
-    const unsigned even = rows[0], odd = rows[1];
-    value = op(__builtin_bit_cast(float, even), __builtin_bit_cast(float, odd));
+    value = reduce_rows_apart(reduce_lanes_32_apart(value, op), op);
     value = op(value, lane_across<8>(value));
     value = op(value, lane_across<4>(value));
     value = op(value, lane_across<2>(value));

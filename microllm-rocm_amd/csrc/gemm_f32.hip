@@ -626,7 +626,9 @@ extern "C" int mll_gemm_f32(const float* a, const float* w, const float* bias, f
     // tiles read LDS less for every product; where they are short the smaller ones' beginnings and ends overlap. Fitted to the four shapes' times at
     // 119 sizes (65 to 1500 rows of seven weights): 0.4 % above the fastest on the mean and 6 % at most, where rounds alone, whole below 4096 workgroups and
     // not above, were 2.8 and 44 % above it (1500 x 37888 x 3584 in tiles of 32 x 128 4746 us, of 128 x 128 3290; 512 rows of it 1308 and 1176; 600 1866 and
-    // 1408; 512 x 896 x 4864 in eight parts 55 and, in tiles of 64 x 64, 49). Up to 32 rows take tiles of 32 rows (32 x 9728 x 896 in tiles of 64 x 64 26.6 us, of 32 x 128 17.7).
+    // 1408; 512 x 896 x 4864 in eight parts 55 and, in tiles of 64 x 64, 49). The factors and the line at 1000 terms are that fit, no mechanism. At 221 sizes outside it
+    // (17 to 4096 rows of weights of 300 to 152064 rows, reductions of 64 to 16000) 0.99 of the time of rounds alone, 0.77 at least; slower by more than
+    // 2 %: 955 x 2048 x 8192 in eight parts 268 -> 283 us, 1468 x 16384 x 2048 798 -> 815. Up to 32 rows take tiles of 32 rows (32 x 9728 x 896 in tiles of 64 x 64 26.6 us, of 32 x 128 17.7).
     struct Shape { int rows, columns; double in_long, in_short; };
     const Shape shapes[4] = {{128, 128, 1.0, 1.0}, {128, 64, 1.06, 0.98}, {64, 64, 1.10, 0.92}, {32, 128, 1.30, 0.975}};
     constexpr int kLongParts = 1000;
