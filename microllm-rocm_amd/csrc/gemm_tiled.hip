@@ -13,9 +13,13 @@
 // (tiled_operands.h): a compute unit takes a load in 16 cycles, and asked for in one go, as before, 64 of them held the
 // products up for a third of a stage. The reads and the products are volatile asm, which pins their order;
 // the compiler neither sees the reads (and so orders nothing against the loads in flight) nor moves the products.
-// Bound by the loads: a compute unit brings a stage's 64 KB in 1.3 to 1.5 us. Gated, before and with the loads between the products, results stored
-// as whole rows, and as many workgroups as compute units going from tile to tile: 8192 x 37888 x 3584 1771 -> 1660 us (1.34 PFLOP/s),
-// 16301 rows 3621 -> 3284, 2048 rows 468 -> 433, 8192 x 16384 x 2048 456 -> 430, 2048 x 9728 x 896 45.8 -> 41.4.
+// Bound by the matrix units at the clock the power cap leaves (65 % busy, 1.94 GHz; products alone 2.0 PFLOP/s), the instructions beside them and a tile's
+// start and end: loads alone take 0.7 us a stage of 1.5, and no wait for them or for the workgroup shows. So loads go through buffer descriptors
+// (one instruction and a place in LDS instead of a 64-bit address each), and the first two stages of a workgroup's next tile are on their way
+// while a tile's results are made and stored. Gated, before and after, 1.03 to 1.05 times as fast: 8192 x 37888 x 3584 1633 -> 1575 us (1.41 PFLOP/s), 16301 rows
+// 3230 -> 3109, 2048 rows 439 -> 418, 8192 x 16384 x 2048 425 -> 404, 3584 rows 199 -> 189, 2048 x 9728 x 896 37.0 -> 35.2; float32, 2048 x 3584 x 18944 in two
+// parts 225 -> 210. Four waves of 128 x 128, accumulators in the other half of the registers: the stages 5 % faster still, a tile's start and
+// end, with nothing beside a wave that waits, 2 us longer (2048 x 9728 x 896 39.0).
 // Workgroups are numbered so that the 32 that run together on one of the 8 XCDs (each with a second-level cache of
 // its own) own about 4 x 8 neighbouring tiles of C, and so share their rows of A and of W there, and so that every
 // XCD gets the same number of tiles.
@@ -34,9 +38,6 @@ constexpr int kPieceElements = 512;                       // of W: 16 rows x 32 
 constexpr int kPackedStep = 1024;                         // from a tile's first k step to its second in a slot
 constexpr int kSuperM = 4, kSuperN = 8;                   // tiles of C that run together on an XCD
 
-__device__ __align__(16) const unsigned zero_piece[256] = {};      // a piece of W past the end of k
-
-
 // EPILOGUE: 0 = float32 [M, N]; 1 = bfloat16 [M, N]; 2 = bfloat16 [M, N / 2] = silu(even rows of W) * (odd rows);
 // 3 = queries, keys and values: bias, rotation, queries to `store.q_out`, keys and values into their pages (W's rows
 // in rotary pair order; see MllQkvStore); 5 = 2 with GELU; 7 = 2 with clamped gates, from the float32 sums (`limit`, `slope`).
@@ -54,9 +55,13 @@ __global__ __launch_bounds__(kTiledThreads, 1) void gemm_tiled_kernel(const bf16
     constexpr int A_TURNS = (A_LOADS + kTiledWaves - 1) / kTiledWaves;
     // Two slots of A, each [2 WM pieces of 16 rows][row][8 places of 16 bytes], the row's chunk c of 8 elements at place c ^ (row / 2); then three of W, each
     // [16 tiles][2 k steps][1 KB in MFMA operand order]. While stages are multiplied the direct loads alone write this memory and the asm reads alone read
-    // it. Gated results pass through it as rows: the workgroup meets before they are written (its reads of the last stage have arrived), before they
-    // are read, and, where it has another tile, before that one's loads go out.
+    // it. Gated results pass through the last slot as rows, while the next tile's first two stages are on their way into the others.
     __shared__ __align__(16) bf16 slots[kStageElements];
+
+    const int lane = threadIdx.x % kWave;
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave);
+    const int col = lane % 16, quad = lane / 16;
+    const int wave_m = wave / 4, wave_n = wave % 4;        // which (16 WM) x 64 of the tile
 
     // Workgroups 8 apart in number run on one XCD, 32 of them at a time. The tiles of C are put in a row, blocks of
     // 4 x 8 neighbouring tiles after one another (down the rows of C first, narrower at the edges), and every XCD
@@ -64,87 +69,107 @@ __global__ __launch_bounds__(kTiledThreads, 1) void gemm_tiled_kernel(const bf16
     // has more than one tile more than another.
     const int tiles = m_blocks * n_blocks;
     const int per_xcd = (tiles + 7) / 8;
-    for (int index = blockIdx.x / 8; index < per_xcd; index += gridDim.x / 8) {
+    struct Place {
+        int m_block, n_block;       // m_block < 0: none
+    };
+    auto place_of = [&](int index) __attribute__((always_inline)) {
         const int place = (blockIdx.x % 8) * per_xcd + index;
-        if (place >= tiles) return;
+        if (index >= per_xcd || place >= tiles) return Place{-1, 0};
         const int column = place / (m_blocks * kSuperN);                       // of blocks, kSuperN tiles wide
         const int width = min(kSuperN, n_blocks - column * kSuperN);
         const int in_column = place - column * m_blocks * kSuperN;
         const int block = in_column / (kSuperM * width);                       // in the column, kSuperM tiles high
         const int height = min(kSuperM, m_blocks - block * kSuperM);
         const int in_block = in_column - block * kSuperM * width;
-        const int m_block = block * kSuperM + in_block % height;
-        const int n_block = column * kSuperN + in_block / height;
+        return Place{block * kSuperM + in_block % height, column * kSuperN + in_block / height};
+    };
 
-        const int lane = threadIdx.x % kWave;
-        const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave);
-        const int col = lane % 16, quad = lane / 16;
-        const int wave_m = wave / 4, wave_n = wave % 4;        // which (16 WM) x 64 of the tile
-        const int m0 = m_block * TILE_M, n_tile0 = n_block * (kTileN / 16);
-
-        // What this wave copies per stage. Of A the loads wave, wave + 8, ... of the stage's 4 WM: load i brings 8 rows
-        // (half h = i % 2 of piece i / 2; lane L: row L / 8 of the 8, place L % 8 of the row). Of W tiles 2 * wave and
-        // 2 * wave + 1, a k step an instruction.
-        const bf16* a_block = a + static_cast<int64_t>(m0) * k;
-        unsigned a_offset[A_TURNS];    // of the lane's 16 bytes from a_block, at stage 0, in bytes
-        // Tiles of 160 rows have loads for half the waves' third turn: the others repeat their second, the same bytes to the same place, since no wave
-        // may pass a load over (tiled_operands.h).
-        auto a_load = [&](int turn) __attribute__((always_inline)) {
-            const int load = wave + turn * kTiledWaves;
-            return A_LOADS % kTiledWaves == 0 || load < A_LOADS ? load : load - kTiledWaves;
-        };
+    // What this wave copies per stage, through buffer descriptors: a load is then one instruction beside its place in LDS, where a global one
+    // works out a 64-bit address (135 -> 60 vector and scalar instructions a stage of 64 products). Of A the loads wave, wave + 8, ... of the stage's
+    // 4 WM: load i brings 8 rows (half h = i % 2 of piece i / 2; lane L: row L / 8 of the 8, place L % 8 of the row). Tiles of 160 rows have loads for
+    // half the waves' third turn: the others repeat their second, the same bytes to the same place, since no wave may pass a load over
+    // (tiled_operands.h). Of W tiles 2 * wave and 2 * wave + 1, a k step an instruction.
+    auto a_load = [&](int turn) __attribute__((always_inline)) {
+        const int load = wave + turn * kTiledWaves;
+        return A_LOADS % kTiledWaves == 0 || load < A_LOADS ? load : load - kTiledWaves;
+    };
+    constexpr int kNowhere = 0x7fffffff;        // past what the descriptors hold
+    __amdgpu_buffer_rsrc_t a_rsrc, w_rsrc;
+    int a_offset[A_TURNS], w_offset[kWTurns / 2];    // of the lane's 16 bytes from the block's first row or tile, at stage 0, in bytes
+    const bool single = k_steps == 1;
+    auto describe = [&](Place at) __attribute__((always_inline)) {
+        const int m0 = at.m_block * TILE_M, n_tile0 = at.n_block * (kTileN / 16);
+        a_rsrc = __builtin_amdgcn_make_buffer_rsrc(const_cast<bf16*>(a) + static_cast<int64_t>(m0) * k, 0, kNowhere, kBufferFlags);
 #pragma unroll
         for (int t = 0; t < A_TURNS; ++t) {
             const int load = a_load(t);
             const int row_in_piece = 8 * (load % 2) + lane / 8;
             const int row = min((load / 2) * 16 + row_in_piece, m - 1 - m0);           // rows past the end repeat the last one
-            a_offset[t] = (static_cast<unsigned>(row) * static_cast<unsigned>(k) + (((lane % 8) ^ (row_in_piece / 2)) * 8)) * 2;
+            const int chunk = (lane % 8) ^ (row_in_piece / 2);
+            a_offset[t] = (row * k + (single ? chunk % 4 : chunk) * 8) * 2;
         }
-        const char* w_tile[2];    // the tile's piece at k step 0
+        w_rsrc = __builtin_amdgcn_make_buffer_rsrc(const_cast<bf16*>(w_packed) + static_cast<int64_t>(n_tile0) * k_steps * kPieceElements, 0, kNowhere,
+                                                   kBufferFlags);
 #pragma unroll
-        for (int p = 0; p < 2; ++p) {
-            const int tile = min(n_tile0 + wave * 2 + p, n_tiles - 1);
-            w_tile[p] = reinterpret_cast<const char*>(w_packed + static_cast<int64_t>(tile) * k_steps * kPieceElements);
-        }
-        const unsigned w_offset = lane * 16;
-        const int all_stages = (k_steps + 1) / 2;
-        const int stages_per_split = (all_stages + gridDim.y - 1) / gridDim.y;
-        const int first_stage = blockIdx.y * stages_per_split;
-        const int stages = min(all_stages, first_stage + stages_per_split);
-        // A k step past the end (k an odd multiple of 32) gets zeros for W and, for A, values that lie in the row: the chunks of the stage's second
-        // half step back by 64 bytes there.
-        auto copy_a = [&](int turn, int stage, unsigned slot) __attribute__((always_inline)) {
-            bf16* a_place = slots + slot * kSlotElements;
-            const int piece = a_load(turn) / 2, h = wave % 2;      // the wave's loads are all of one half
-            const bool upper = (((lane >> 2) & 1) ^ h) != 0;      // the lane's chunk is one of the row's second four
-            const char* a_source = reinterpret_cast<const char*>(a_block) + stage * 128 + (a_offset[turn] - ((2 * stage + 1 >= k_steps && upper) ? 64u : 0u));
-            // (the place is computed here: with a subscript of a captured array in this call the host pass
-            // drops the kernel's stub without a word)
-            __builtin_amdgcn_global_load_lds(a_source, a_place + piece * 1024 + h * 512, 16, 0, 0);
-        };
-        auto copy_w = [&](int turn, int stage, unsigned slot) __attribute__((always_inline)) {      // turn: which of the wave's two tiles and k steps
-            bf16* w_place = slots + (kASlots + slot) * kSlotElements;
-            const int p = turn / 2, h = turn % 2;
-            const char* w_source = 2 * stage + h < k_steps ? w_tile[p] + static_cast<int64_t>(2 * stage + h) * (kPieceElements * 2)
-                                                           : reinterpret_cast<const char*>(zero_piece);
-            __builtin_amdgcn_global_load_lds(w_source + w_offset, w_place + (wave * 2 + p) * 1024 + h * 512, 16, 0, 0);
-        };
-        // Where the lane reads its operands: row `col` of a piece, chunk 4 step + quad at its place.
-        const unsigned base = lds_address(slots);
-        const unsigned a_row = base + wave_m * WM * 2048 + col * 128;
-        const unsigned a_step0 = a_row + ((quad ^ (col / 2)) * 16), a_step1 = a_row + (((4 + quad) ^ (col / 2)) * 16);
-        const unsigned w_lane = base + kASlots * kSlotBytes + wave_n * kWaveTilesN * 2048 + lane * 16;
+        for (int p = 0; p < kWTurns / 2; ++p)
+            w_offset[p] = min(wave * (kWTurns / 2) + p, n_tiles - 1 - n_tile0) * k_steps * (kPieceElements * 2) + lane * 16;
+    };
+    const int all_stages = (k_steps + 1) / 2;
+    const int stages_per_split = (all_stages + gridDim.y - 1) / gridDim.y;
+    const int first_stage = blockIdx.y * stages_per_split;
+    const int stages = min(all_stages, first_stage + stages_per_split);
+    // The last stage of an odd number of k steps is the last 64 of k, its first step with zeros for W (that step has been multiplied by the stage
+    // before; of a single step the second has zeros).
+    auto copy_a = [&](int turn, int stage, unsigned slot) __attribute__((always_inline)) {
+        // (arguments are worked out before the call: with a captured array's subscript in it the host pass drops the kernel's stub without a word)
+        bf16* place = slots + slot * kSlotElements + a_load(turn) * 512;
+        const int at = a_offset[turn], from = max(0, min(stage * 128, (k_steps - 2) * 64));
+        __builtin_amdgcn_raw_ptr_buffer_load_lds(a_rsrc, place, 16, at, from, 0, 0);
+    };
+    auto copy_w = [&](int turn, int stage, unsigned slot) __attribute__((always_inline)) {      // turn: which of the wave's two tiles and k steps
+        const int p = turn / 2, h = turn % 2;
+        bf16* place = slots + (kASlots + slot) * kSlotElements + (wave * (kWTurns / 2) + p) * 1024 + h * 512;
+        const bool last_alone = 2 * stage + 1 == k_steps;      // the stage has one step of its own
+        const int step = last_alone && !single ? k_steps - 1 : 2 * stage + h;
+        const int at = w_offset[p], from = last_alone && (h == 0) != single ? kNowhere : step * (kPieceElements * 2);
+        __builtin_amdgcn_raw_ptr_buffer_load_lds(w_rsrc, place, 16, at, from, 0, 0);
+    };
+    // Where the lane reads its operands: row `col` of a piece, chunk 4 step + quad at its place.
+    const unsigned base = lds_address(slots);
+    const unsigned a_row = base + wave_m * WM * 2048 + col * 128;
+    const unsigned a_step0 = a_row + ((quad ^ (col / 2)) * 16), a_step1 = a_row + (((4 + quad) ^ (col / 2)) * 16);
+    const unsigned w_lane = base + kASlots * kSlotBytes + wave_n * kWaveTilesN * 2048 + lane * 16;
 
+    constexpr bool GATED = EPILOGUE == 2 || EPILOGUE == 5 || EPILOGUE == 7;
+    constexpr int STORES = GATED ? WM : 0;         // of a wave that stores a whole gated tile
+    int index = blockIdx.x / 8;
+    Place at = place_of(index), next;
+    if (at.m_block < 0) return;
+    const bool any = EPILOGUE != 0 || first_stage < stages;      // a part of the reduction may be empty
+    if (any) {
+        describe(at);
+        begin_stages<A_TURNS>(first_stage, stages, copy_a, copy_w);
+    }
+    bool stored = false;      // whether the wave issued STORES stores after the tile's first loads
+    for (;; at = next) {
+        index += gridDim.x / 8;
+        next = place_of(index);
+        const int m0 = at.m_block * TILE_M, n_tile0 = at.n_block * (kTileN / 16), n_block = at.n_block;
         floatx4 acc[kWaveTilesN][WM];     // acc[nt][mt][i] = C[m = mt*16 + col][n = nt*16 + quad*4 + i] of the wave's part
+        if (any) {
+            multiply_stages<kPackedStep, WM, A_TURNS, STORES>(acc, first_stage, stages, stored, a_step0, a_step1, w_lane, w_lane, copy_a, copy_w);
+            if (GATED || next.m_block >= 0) workgroup_meets();        // every wave is done with the slots
+            if (next.m_block >= 0) {
+                describe(next);
+                begin_stages<A_TURNS>(first_stage, stages, copy_a, copy_w);
+            }
+        } else {
 #pragma unroll
-        for (int nt = 0; nt < kWaveTilesN; ++nt)
+            for (int nt = 0; nt < kWaveTilesN; ++nt)
 #pragma unroll
-            for (int mt = 0; mt < WM; ++mt) acc[nt][mt] = floatx4{0.0f, 0.0f, 0.0f, 0.0f};
-
-        if (first_stage < stages) {
-            if (index != static_cast<int>(blockIdx.x) / 8) workgroup_meets();        // every wave is done with the slots of the tile before
-            multiply_stages<kPackedStep, WM, A_TURNS>(acc, first_stage, stages, a_step0, a_step1, w_lane, w_lane, copy_a, copy_w);
+                for (int mt = 0; mt < WM; ++mt) acc[nt][mt] = floatx4{0.0f, 0.0f, 0.0f, 0.0f};
         }
+        stored = false;
 
         if constexpr (EPILOGUE == 3) {
             // The lane's 4 columns of a tile lie in one head (head_dim is a multiple of 16). In a query or key head
@@ -217,27 +242,50 @@ __global__ __launch_bounds__(kTiledThreads, 1) void gemm_tiled_kernel(const bf16
                     }
                 }
             }
+            if (next.m_block < 0) return;
             continue;
         }
         auto gated = [&](float gate, float up) {
             return EPILOGUE == 7 ? gated_value_fast(gate, up, kActClampedGlu, limit, slope) : gate_fast<EPILOGUE == 5>(gate) * up;
         };
-        if constexpr (EPILOGUE == 2 || EPILOGUE == 5 || EPILOGUE == 7) {
+        if constexpr (GATED) {
             if (whole_rows) {
-                workgroup_meets();
-#pragma unroll
-                for (int mt = 0; mt < WM; ++mt)
+                const int row0 = m0 + wave_m * (WM * 16), column = n_block * kResultColumns + wave_n * 32 + (lane % 4) * 8;
+                stored = m0 + TILE_M <= m && (n_block + 1) * kResultColumns <= n / 2;
+                const unsigned place = base + (kASlots + 2) * kSlotBytes + wave * (kResultRows * kResultBytes);
+                const unsigned word_at = place + col * kResultBytes + (col / 4) * 16 + quad * 4;      // of tile 0; tile nt's chunk is exchanged with it
+                bf16* to = static_cast<bf16*>(out) + static_cast<int64_t>(row0 + lane / 4) * (n / 2) + column;
+                auto put_tiles = [&](auto mt) __attribute__((always_inline)) {
+                    constexpr int MT = decltype(mt)::value;
 #pragma unroll
                     for (int nt = 0; nt < kWaveTilesN; ++nt) {
                         bf16x2 two;
 #pragma unroll
-                        for (int i = 0; i < 2; ++i) two[i] = static_cast<__bf16>(gated(acc[nt][mt][2 * i], acc[nt][mt][2 * i + 1]));
-                        *reinterpret_cast<bf16x2*>(reinterpret_cast<char*>(slots) + (wave_m * (WM * 16) + mt * 16 + col) * kResultStride +
-                                                   wave_n * 64 + nt * 16 + quad * 4) = two;
+                        for (int i = 0; i < 2; ++i) two[i] = static_cast<__bf16>(gated(acc[nt][MT][2 * i], acc[nt][MT][2 * i + 1]));
+                        put_result<MT % 4 * 16 * kResultBytes>(word_at ^ (nt * 16), __builtin_bit_cast(unsigned, two));
                     }
-                workgroup_meets();
-                store_result_rows(slots, static_cast<bf16*>(out) + static_cast<int64_t>(m0) * (n / 2) + n_block * kResultColumns, min(TILE_M, m - m0), n / 2,
-                                  n / 2 - n_block * kResultColumns);
+                };
+                auto half = [&](auto first_tile) __attribute__((always_inline)) {
+                    constexpr int FIRST = decltype(first_tile)::value, COUNT = WM - FIRST < 4 ? WM - FIRST : 4;
+                    put_tiles(std::integral_constant<int, FIRST>{});
+                    if constexpr (COUNT > 1) put_tiles(std::integral_constant<int, FIRST + (COUNT > 1)>{});
+                    if constexpr (COUNT > 2) put_tiles(std::integral_constant<int, FIRST + 2 * (COUNT > 2)>{});
+                    if constexpr (COUNT > 3) put_tiles(std::integral_constant<int, FIRST + 3 * (COUNT > 3)>{});
+                    uintx4 piece[4];
+                    get_results(piece, place, lane);      // 16 rows each; those past COUNT are stored by nobody
+                    if (stored) {
+#pragma unroll
+                        for (int i = 0; i < COUNT; ++i) *reinterpret_cast<uintx4*>(to + static_cast<int64_t>((FIRST + i) * 16) * (n / 2)) = piece[i];
+                    } else {
+#pragma unroll
+                        for (int i = 0; i < COUNT; ++i)
+                            if (row0 + (FIRST + i) * 16 + lane / 4 < m && column < n / 2)
+                                *reinterpret_cast<uintx4*>(to + static_cast<int64_t>((FIRST + i) * 16) * (n / 2)) = piece[i];
+                    }
+                };
+                half(std::integral_constant<int, 0>{});
+                if constexpr (WM > 4) half(std::integral_constant<int, 4>{});
+                if (next.m_block < 0) return;
                 continue;
             }
         }
@@ -284,6 +332,7 @@ __global__ __launch_bounds__(kTiledThreads, 1) void gemm_tiled_kernel(const bf16
                 }
             }
         }
+        if (next.m_block < 0) return;
     }
 }
 

@@ -2,10 +2,11 @@
 // (moe_sort_kernel in moe.hip), and a workgroup of 8 waves takes up to 256 pairs of one expert and 256 rows of its weight, with the main loop of
 // gemm_tiled.hip: stages of 64 of the reduction by direct loads into LDS slots (two of A, three of W), the operands of a k step read from
 // LDS between the products of the step before. Here both sides are rows of memory, 8 rows of 128 bytes a load, and A's rows are taken from
-// wherever their tokens lie. Bound by the loads of a stage (64 KB, which a compute unit brings in 1.5 us) and by a tile's beginning and end, which
+// wherever their tokens lie. Bound by the products of a stage with what stands between them (1.5 us; gemm_tiled.hip) and by a tile's beginning and end, which
 // nothing overlaps: as many workgroups as compute units go from tile to tile, and the height of the tiles is chosen so that their rounds are done
 // first (an expert's last pairs take a tile of 192 or 128 rows where that is enough). 3117 tokens with 4 of 16 experts of 2048 x 2048 and 4
-// ids that return their input: 426 -> 343 us with gate, up, down and the sort (tiles of 256 by a workgroup each 401), 0.73 PFLOP/s.
+// ids that return their input: 426 -> 343 us with gate, up, down and the sort (tiles of 256 by a workgroup each 401), 0.73 PFLOP/s; loads
+// through buffer descriptors, 16 experts without those ids, 352 -> 348 to 360 -> 352.
 // The tiles of all experts stand in a row, an expert after another, its columns one after another and down the rows first; every XCD takes
 // an equal stretch, so that the workgroups that run together there share an expert's rows and neighbouring rows of its weight.
 // A result's additions are those of moe_grouped_kernel in the same order, so a pair's bits do not depend on which of the two it meets.
@@ -125,43 +126,58 @@ __device__ __attribute__((always_inline)) inline void tile_products(bf16* slots,
         }
         w_from[t] = (static_cast<unsigned>(w_row) * static_cast<unsigned>(k) + chunk) * 2;
     }
-    const char* a_bytes = reinterpret_cast<const char*>(a);
-    const char* w_bytes = reinterpret_cast<const char*>(w_expert);
+    const __amdgpu_buffer_rsrc_t a_rsrc = __builtin_amdgcn_make_buffer_rsrc(const_cast<bf16*>(a), 0, 0xffffffff, kBufferFlags);
+    const __amdgpu_buffer_rsrc_t w_rsrc = __builtin_amdgcn_make_buffer_rsrc(const_cast<bf16*>(w_expert), 0, 0xffffffff, kBufferFlags);
     auto copy_a = [&](int turn, int stage, unsigned slot) __attribute__((always_inline)) {
         bf16* place = slots + slot * kSlotElements + wave * 512;
-        __builtin_amdgcn_global_load_lds(a_bytes + stage * 128 + a_from[turn], place + turn * (kTiledWaves * 512), 16, 0, 0);
+        const unsigned at = a_from[turn];
+        __builtin_amdgcn_raw_ptr_buffer_load_lds(a_rsrc, place + turn * (kTiledWaves * 512), 16, at, stage * 128, 0, 0);
     };
     auto copy_w = [&](int turn, int stage, unsigned slot) __attribute__((always_inline)) {
         bf16* place = slots + (kASlots + slot) * kSlotElements + wave * 512;
-        __builtin_amdgcn_global_load_lds(w_bytes + stage * 128 + w_from[turn], place + turn * (kTiledWaves * 512), 16, 0, 0);
+        const unsigned at = w_from[turn];
+        __builtin_amdgcn_raw_ptr_buffer_load_lds(w_rsrc, place + turn * (kTiledWaves * 512), 16, at, stage * 128, 0, 0);
     };
     const unsigned base = lds_address(slots);
     const unsigned step0 = col * 128 + ((quad ^ (col / 2)) * 16), step1 = col * 128 + (((4 + quad) ^ (col / 2)) * 16);
     const unsigned a_at = base + wave_m * WM * 2048, w_at = base + kASlots * kSlotBytes + wave_n * kWaveTilesN * 2048;
 
     floatx4 acc[kWaveTilesN][WM];     // acc[nt][mt][i] = C[pair mt*16 + col][weight row nt*16 + quad*4 + i] of the wave's part
-#pragma unroll
-    for (int nt = 0; nt < kWaveTilesN; ++nt)
-#pragma unroll
-        for (int mt = 0; mt < WM; ++mt) acc[nt][mt] = floatx4{0.0f, 0.0f, 0.0f, 0.0f};
-
-    multiply_stages<0, WM, A_TURNS>(acc, 0, k / 64, a_at + step0, a_at + step1, w_at + step0, w_at + step1, copy_a, copy_w);
+    begin_stages<A_TURNS>(0, k / 64, copy_a, copy_w);
+    multiply_stages<0, WM, A_TURNS, 0>(acc, 0, k / 64, false, a_at + step0, a_at + step1, w_at + step0, w_at + step1, copy_a, copy_w);
 
     if constexpr (GATED) {
         workgroup_meets();
-#pragma unroll
-        for (int mt = 0; mt < WM; ++mt)
+        const int row0 = wave_m * (WM * 16), column = column0 + wave_n * 32 + (lane % 4) * 8;
+        const unsigned place = base + (kASlots + 2) * kSlotBytes + wave * (kResultRows * kResultBytes);
+        const unsigned words_at = place + col * kResultBytes + (((quad / 2) ^ (col / 4)) * 16) + (quad % 2) * 8;
+        bf16* to = static_cast<bf16*>(out) + static_cast<int64_t>(tile.first_row + row0 + lane / 4) * n_out + column;
+        auto put_tiles = [&](auto mt) __attribute__((always_inline)) {
+            constexpr int MT = decltype(mt)::value;
 #pragma unroll
             for (int nt = 0; nt < kWaveTilesN / 2; ++nt) {
                 bf16x4 four;
 #pragma unroll
                 for (int i = 0; i < 4; ++i)
-                    four[i] = static_cast<__bf16>(gated_value_fast(acc[nt][mt][i], acc[nt + 2][mt][i], form.activation, form.limit, form.slope));
-                *reinterpret_cast<bf16x4*>(reinterpret_cast<char*>(slots) + (wave_m * (WM * 16) + mt * 16 + col) * kResultStride + wave_n * 64 +
-                                           nt * 32 + quad * 8) = four;
+                    four[i] = static_cast<__bf16>(gated_value_fast(acc[nt][MT][i], acc[nt + 2][MT][i], form.activation, form.limit, form.slope));
+                put_result<MT % 4 * 16 * kResultBytes>(words_at ^ (nt * 32), __builtin_bit_cast(uint64_t, four));
             }
-        workgroup_meets();
-        store_result_rows(slots, static_cast<bf16*>(out) + static_cast<int64_t>(tile.first_row) * n_out + column0, tile.rows, n_out, n_out - column0);
+        };
+        auto half = [&](auto first_tile) __attribute__((always_inline)) {
+            constexpr int FIRST = decltype(first_tile)::value, COUNT = WM - FIRST < 4 ? WM - FIRST : 4;
+            put_tiles(std::integral_constant<int, FIRST>{});
+            put_tiles(std::integral_constant<int, FIRST + 1>{});
+            if constexpr (COUNT > 2) put_tiles(std::integral_constant<int, FIRST + 2 * (COUNT > 2)>{});
+            if constexpr (COUNT > 3) put_tiles(std::integral_constant<int, FIRST + 3 * (COUNT > 3)>{});
+            uintx4 piece[4];
+            get_results(piece, place, lane);
+#pragma unroll
+            for (int i = 0; i < COUNT; ++i)
+                if (row0 + (FIRST + i) * 16 + lane / 4 < tile.rows && column < n_out)
+                    *reinterpret_cast<uintx4*>(to + static_cast<int64_t>((FIRST + i) * 16) * n_out) = piece[i];
+        };
+        half(std::integral_constant<int, 0>{});
+        if constexpr (WM > 4) half(std::integral_constant<int, 4>{});
         return;
     }
 #pragma unroll

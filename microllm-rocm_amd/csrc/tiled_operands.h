@@ -24,6 +24,7 @@ constexpr int kWaveTilesN = 4;                            // a wave's 64 columns
 constexpr int kSlotBytes = 32768;
 constexpr int kSlotElements = kSlotBytes / 2;
 constexpr int kASlots = 2, kWSlots = 3;
+constexpr int kWTurns = 32 / kTiledWaves;                 // loads of W a wave and stage, 1 KB each
 constexpr int kStageElements = (kASlots + kWSlots) * kSlotElements;
 
 __device__ inline unsigned lds_address(bf16* place) { return static_cast<unsigned>(reinterpret_cast<uintptr_t>((lds_bf16*)place)); }
@@ -42,13 +43,8 @@ struct TiledOperands {       // of one k step: the wave's WM pieces of A and 4 o
 template <int W_STEP, int WM, int INDEX, int STEP>
 __device__ __attribute__((always_inline)) inline void read_operand(TiledOperands<WM>& f, unsigned a_address, unsigned w_address) {
     constexpr int W = STEP * W_STEP;
-    if constexpr (INDEX == 0) MLL_DS_READ(f.w[0], w_address, W);
-    if constexpr (INDEX == 1) MLL_DS_READ(f.w[1], w_address, W + 2048);
-    if constexpr (INDEX == 2) MLL_DS_READ(f.a[0], a_address, 0);
-    if constexpr (INDEX == 3) MLL_DS_READ(f.a[1], a_address, 2048);
-    if constexpr (INDEX == 4) MLL_DS_READ(f.w[2], w_address, W + 4096);
-    if constexpr (INDEX == 5) MLL_DS_READ(f.w[3], w_address, W + 6144);
-    if constexpr (INDEX >= 6 && INDEX < 4 + WM) MLL_DS_READ(f.a[INDEX - 4], a_address, (INDEX - 4) * 2048);
+    if constexpr (INDEX < kWaveTilesN) MLL_DS_READ(f.w[INDEX], w_address, W + INDEX * 2048);
+    else if constexpr (INDEX < kWaveTilesN + WM) MLL_DS_READ(f.a[INDEX - kWaveTilesN], a_address, (INDEX - kWaveTilesN) * 2048);
 }
 template <int W_STEP, int WM, int STEP, int... INDEX>
 __device__ __attribute__((always_inline)) inline void read_operands(TiledOperands<WM>& f, unsigned a_address, unsigned w_address,
@@ -95,45 +91,62 @@ __device__ __attribute__((always_inline)) inline void operands_arrived(TiledOper
     for (int i = 4; i < WM; ++i) asm volatile("" : "+v"(f.a[i]));
 }
 
-// The stages of a tile, from `first` to before `stages`, one at least. copy_a(turn, stage, slot) and copy_w(turn, stage, slot) issue one of a wave's
-// A_TURNS and four loads of a stage, every wave all of them. While a stage's first step is multiplied its second is read, and W's loads of the stage after
-// next go out, into the slot that was read a stage ago; then the next stage has landed (the wave's loads before the barrier, everyone's after it) and this
-// one has been read by all: A's loads of the stage after next go out while the second step is multiplied and the next stage's first is read. After the last
-// stage nothing is copied, and what is read then is multiplied by nobody.
-template <int W_STEP, int WM, int A_TURNS, typename CopyA, typename CopyW>
-__device__ __attribute__((always_inline)) inline void multiply_stages(floatx4 (&acc)[kWaveTilesN][WM], int first, int stages, unsigned a_step0,
-                                                                      unsigned a_step1, unsigned w_step0, unsigned w_step1, const CopyA& copy_a,
-                                                                      const CopyW& copy_w) {
-    constexpr std::make_integer_sequence<int, WM> row_tiles{};
-    TiledOperands<WM> even, odd;      // of a stage's first and second k step
-    const bool second = first + 1 < stages;
+// The loads of a tile's first two stages, from `first` to before `stages`, go out: copy_a(turn, stage, slot) and copy_w(turn, stage, slot) issue one of a
+// wave's A_TURNS and kWTurns loads of a stage, every wave all of them. The slots are free: the workgroup has met since they were read.
+template <int A_TURNS, typename CopyA, typename CopyW>
+__device__ __attribute__((always_inline)) inline void begin_stages(int first, int stages, const CopyA& copy_a, const CopyW& copy_w) {
 #pragma unroll
     for (int t = 0; t < A_TURNS; ++t) copy_a(t, first, 0);
 #pragma unroll
-    for (int t = 0; t < 4; ++t) copy_w(t, first, 0);
-    if (second) {
+    for (int t = 0; t < kWTurns; ++t) copy_w(t, first, 0);
+    if (first + 1 < stages) {
 #pragma unroll
         for (int t = 0; t < A_TURNS; ++t) copy_a(t, first + 1, 1);
 #pragma unroll
-        for (int t = 0; t < 4; ++t) copy_w(t, first + 1, 1);
-        // the first stage's loads of this wave have landed when only the second stage's are on their way
-        asm volatile("s_waitcnt vmcnt(%0)" :: "n"(A_TURNS + 4) : "memory");
-    } else {
-        asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+        for (int t = 0; t < kWTurns; ++t) copy_w(t, first + 1, 1);
     }
+}
+
+// The stages of a tile, from `first` to before `stages`, one at least, whose first two are on their way (begin_stages); acc is written, not added to.
+// While a stage's first step is multiplied its second is read, and W's loads of the stage
+// after next go out, into the slot that was read a stage ago; then the next stage has landed (the wave's loads before the barrier, everyone's after it) and this
+// one has been read by all: A's loads of the stage after next go out while the second step is multiplied and the next stage's first is read. After the last
+// stage nothing is copied, and what is read then is multiplied by nobody.
+// STORES: how many stores to memory the wave has issued since begin_stages, at least, if `stored`: loads and stores are counted together as they
+// were issued, and a wait that names the stores lets them go on while the first stages are multiplied.
+template <int W_STEP, int WM, int A_TURNS, int STORES, typename CopyA, typename CopyW>
+__device__ __attribute__((always_inline)) inline void multiply_stages(floatx4 (&acc)[kWaveTilesN][WM], int first, int stages, bool stored, unsigned a_step0,
+                                                                      unsigned a_step1, unsigned w_step0, unsigned w_step1, const CopyA& copy_a,
+                                                                      const CopyW& copy_w) {
+    constexpr std::make_integer_sequence<int, WM> row_tiles{};
+    constexpr int kStage = A_TURNS + kWTurns, kMostCounted = 63;
+    constexpr int kStageAndStores = kStage + STORES < kMostCounted ? kStage + STORES : kMostCounted;
+    constexpr int kTurnsAndStores = kWTurns + STORES < kMostCounted ? kWTurns + STORES : kMostCounted;
+    TiledOperands<WM> even, odd;      // of a stage's first and second k step
+#pragma unroll
+    for (int nt = 0; nt < kWaveTilesN; ++nt)
+#pragma unroll
+        for (int mt = 0; mt < WM; ++mt) {
+            acc[nt][mt] = floatx4{0.0f, 0.0f, 0.0f, 0.0f};
+            asm volatile("" : "+v"(acc[nt][mt]));      // once and here, while the loads are on their way: left to itself the compiler does it on every way to the loops
+        }
+    // The first stage's loads of this wave have landed when only what was issued after them is on its way.
+    if (first + 1 == stages) asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+    else if (stored) asm volatile("s_waitcnt vmcnt(%0)" :: "n"(kStageAndStores) : "memory");
+    else asm volatile("s_waitcnt vmcnt(%0)" :: "n"(kStage) : "memory");
     __builtin_amdgcn_s_barrier();
-    read_operands<W_STEP, WM, 0>(even, a_step0, w_step0, std::make_integer_sequence<int, 4 + WM>{});
+    read_operands<W_STEP, WM, 0>(even, a_step0, w_step0, std::make_integer_sequence<int, kWaveTilesN + WM>{});
     operands_arrived<-1>(even);
     unsigned a_now = 0, w_now = 0, w_next = 1, w_after = 2;        // slots
-    // MORE: there is a stage after next. Operands on their way never pass from one block to another (the compiler may copy a value there, and does
+    // MORE: there is a stage after next. `wait`: how much of what was issued last may be on its way when the next stage has landed. Operands on their way never pass from one block to another (the compiler may copy a value there, and does
     // not know that it has not arrived): no branch stands in a stage, and a stage ends when the next one's first operands have arrived.
-    auto multiply_stage = [&](int stage, auto more) __attribute__((always_inline)) {
+    auto multiply_stage = [&](int stage, auto more, auto wait) __attribute__((always_inline)) {
         constexpr bool MORE = decltype(more)::value;
         products<W_STEP, WM, 1>(acc, even, odd, a_step1 + a_now * kSlotBytes, w_step1 + w_now * kSlotBytes, [&](auto place) __attribute__((always_inline)) {
-            constexpr int kPlace = decltype(place)::value, kApart = 2 * WM / 4;
-            if constexpr (MORE && kPlace % kApart == 0 && kPlace / kApart < 4) copy_w(kPlace / kApart, stage + 2, w_after);
+            constexpr int kPlace = decltype(place)::value, kApart = 2 * WM / kWTurns;
+            if constexpr (MORE && kPlace % kApart == 0 && kPlace / kApart < kWTurns) copy_w(kPlace / kApart, stage + 2, w_after);
         }, row_tiles);
-        operands_arrived<MORE ? 4 : 0>(odd);
+        operands_arrived<decltype(wait)::value>(odd);
         __builtin_amdgcn_s_barrier();
         products<W_STEP, WM, 0>(acc, odd, even, a_step0 + (1 - a_now) * kSlotBytes, w_step0 + w_next * kSlotBytes, [&](auto place) __attribute__((always_inline)) {
             constexpr int kPlace = decltype(place)::value;
@@ -145,8 +158,11 @@ __device__ __attribute__((always_inline)) inline void multiply_stages(floatx4 (&
         w_now = w_next, w_next = w_after, w_after = w;
     };
     int stage = first;
-    for (; stage + 2 < stages; ++stage) multiply_stage(stage, std::true_type{});
-    for (; stage < stages; ++stage) multiply_stage(stage, std::false_type{});
+    if (STORES > 0 && stored && stage + 2 < stages) multiply_stage(stage++, std::true_type{}, std::integral_constant<int, kTurnsAndStores>{});
+#pragma clang loop unroll(disable)
+    for (; stage + 2 < stages; ++stage) multiply_stage(stage, std::true_type{}, std::integral_constant<int, kWTurns>{});
+#pragma clang loop unroll(disable)
+    for (; stage < stages; ++stage) multiply_stage(stage, std::false_type{}, std::integral_constant<int, 0>{});
     // No load is on its way into LDS now and no read into registers; the last products must have written their results before these are read (the
     // compiler does not know that the asm statements are products).
     asm volatile("s_nop 15\n\ts_nop 15" ::: "memory");
@@ -159,17 +175,26 @@ __device__ __attribute__((always_inline)) inline void workgroup_meets() {
     asm volatile("" ::: "memory");
 }
 
-// A tile's results of 128 columns in bfloat16 go through the slots, so that they leave as whole rows of 256 bytes: a lane has 4 or 8 bytes of a
-// row, which would touch every line of memory 8 to 32 times (9728 columns of 1280 rows, reduction 896: 34 -> 30 us). Rows in LDS are 272 bytes apart, so that 16
-// rows' words meet no bank twice.
-constexpr int kResultStride = 272, kResultColumns = 128;
-__device__ __attribute__((always_inline)) inline void store_result_rows(const bf16* slots, bf16* __restrict__ out, int rows, int row_elements, int columns) {
-    for (int piece = threadIdx.x; piece < rows * (kResultColumns / 8); piece += kTiledThreads) {
-        const int row = piece / (kResultColumns / 8), column = piece % (kResultColumns / 8) * 8;
-        if (column < columns)
-            *reinterpret_cast<uintx4*>(out + static_cast<int64_t>(row) * row_elements + column) =
-                *reinterpret_cast<const uintx4*>(reinterpret_cast<const char*>(slots) + row * kResultStride + column * 2);
-    }
+// A tile's results of 128 columns in bfloat16, 32 of them a wave's, go through the last slot of W, so that they leave as rows of 64 bytes (a lane has 4
+// or 8 bytes of a row, which would touch every line of memory 8 to 32 times: 9728 columns of 1280 rows, reduction 896: 34 -> 30 us). A wave has 64 rows
+// of 64 bytes there, for itself: nobody waits for another wave, and the next tile's loads into the other slots are on their way meanwhile. By asm: the
+// compiler, which does not know which slots those fill, would wait for them. A row's 16-byte chunks lie at places exchanged by (row / 4): 16 rows' words meet
+// no bank twice.
+constexpr int kResultColumns = 128;      // of a tile
+constexpr int kResultRows = 64;          // of a wave at a time, 16 a store
+constexpr int kResultBytes = 64;         // of a wave's row
+template <int OFFSET> __device__ __attribute__((always_inline)) inline void put_result(unsigned address, unsigned word) {
+    asm volatile("ds_write_b32 %0, %1 offset:%2" ::"v"(address), "v"(word), "n"(OFFSET) : "memory");
+}
+template <int OFFSET> __device__ __attribute__((always_inline)) inline void put_result(unsigned address, uint64_t words) {
+    asm volatile("ds_write_b64 %0, %1 offset:%2" ::"v"(address), "v"(words), "n"(OFFSET) : "memory");
+}
+// The wave's rows 16 i + lane / 4, chunk lane % 4.
+__device__ __attribute__((always_inline)) inline void get_results(uintx4 (&piece)[4], unsigned place, int lane) {
+    const unsigned at = place + (lane / 4) * kResultBytes + (((lane % 4) ^ (lane / 16)) * 16);
+    asm volatile("ds_read_b128 %0, %4\n\tds_read_b128 %1, %4 offset:1024\n\tds_read_b128 %2, %4 offset:2048\n\tds_read_b128 %3, %4 offset:3072\n\t"
+                 "s_waitcnt lgkmcnt(0)"
+                 : "=&v"(piece[0]), "=&v"(piece[1]), "=&v"(piece[2]), "=&v"(piece[3]) : "v"(at) : "memory");
 }
 
 }  // namespace mll

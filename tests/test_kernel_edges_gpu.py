@@ -488,6 +488,24 @@ def test_queries_keys_and_values_of_more_tiles_than_workgroups():
         assert all(torch.equal(a, b) for a, b in zip(results[0], other))
 
 
+@pytest.mark.parametrize("k", [32, 64, 96, 128, 160, 192, 256, 352])
+@pytest.mark.parametrize("m,n", [(2200, 8192), (2048, 8448), (2100, 8210)])
+def test_tiles_whose_loads_go_out_before_the_tile_before_is_stored(m, n, k):
+    """One to six stages, odd numbers of k steps, whole tiles and ragged ones, of which workgroups take a second or third: the bits of the same rows and columns
+    by fewer tiles than workgroups, which each take one."""
+    ka, generator = kernels(), torch.Generator(device=DEVICE).manual_seed(m + n + k)
+    x, w = ((torch.randn(shape, generator=generator, device=DEVICE) * scale).to(torch.bfloat16) for shape, scale in (((m, k), 1.0), ((n, k), k ** -0.5)))
+    packed, band = ka.pack_weight(w), 512
+    for epilogue, tile_rows in (("gated", 256), ("gated", 128), ("bf16", 256), ("f32", 160)):
+        whole = ka.gemm_tiled(x, packed, n, epilogue, tile_rows=tile_rows)
+        width = band // 2 if epilogue == "gated" else band
+        for rows in (slice(0, 300), slice(m - 300, m)):
+            for at in (0, n // 2 // band * band, (n - 1) // band * band):
+                part = ka.gemm_tiled(x[rows].contiguous(), packed[at // 16:(at + band) // 16].contiguous(), min(band, n - at), epilogue, tile_rows=tile_rows)
+                assert torch.equal(part, whole[rows, at * width // band:at * width // band + part.shape[1]]), (epilogue, rows, at)
+    assert float((ka.gemm_tiled(x, packed, n, "f32") - x.float() @ w.float().T).abs().max()) < 1e-5 * k ** 0.5 + 1e-4      # sums of at most 352 products of size 1 / sqrt(k)
+
+
 @pytest.mark.parametrize("heads,kv_heads,hd,window", [(14, 2, 64, 0), (4, 2, 48, 100), (4, 1, 128, 0), (2, 1, 256, 33)])
 def test_prompts_in_tiles_of_half_the_queries_have_the_same_bits(heads, kv_heads, hd, window):
     """Tiles of 64 queries, whose second one in a workgroup goes to the waves from the last on, against tiles of 128."""
