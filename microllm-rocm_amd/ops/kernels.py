@@ -1289,6 +1289,22 @@ def tiled_gated_pays(rows: int, k: int, from_float: bool = False, n: int = TILED
     return 3584 <= k <= 6144 and 960 < rows <= 3072 and _tiled_fill_of(rows, n) >= 0.9
 
 
+def tiled_gated_pays_in_long_reductions(rows: int, k: int, n: int) -> bool:
+    """The same for reductions of more than 2048 and up to 6144 since the tiled kernel's loads go through descriptors and a workgroup's next tile is
+    on its way while one is stored: it is the faster one wherever its tiles fill three quarters of their rounds, and up to 768 rows, where the
+    library's tiles fill no more, always (14 weights from 13824 x 2304 to 32768 x 6144 at 19 numbers of rows from 256 to 8192, library and activation over
+    this kernel: 1.12 on the mean, 0.96 at the least; 37888 x 3584 at 384, 768, 1024, 2048, 4096, 8192 and 16384 rows 1.16, 1.04, 1.30, 1.34, 1.06, 1.11
+    and 1.06; 27648 x 5120 at 512 to 8192 1.10 to 1.29). Left out: 14336 x 4096 at 2560 rows (0.73 filled) 0.97, 13824 x 5120 at 320 and 1792 (0.63, 0.74) 0.96 and
+    0.95, 37888 x 3584 at 256 (0.58) 0.88; beyond, 28672 x 7168 0.93 to 1.12, 59136 x 8192 0.94 to 1.09. A tuned library keeps the product."""
+    if library_tuning() or k % 32 != 0 or not 2048 < k <= 6144:
+        return False
+    multiple = 64 if rows <= 1024 else 256
+    rows = -(-rows // multiple) * multiple
+    if rows < 256 or n < 8192:      # fewer columns were not measured
+        return False
+    return 384 <= rows <= 768 or _tiled_fill_of(rows, n) >= (0.8 if rows < 384 else 0.76)
+
+
 def gemm_tiled(x: torch.Tensor, packed: torch.Tensor, n: int, epilogue: str = "f32", splits: int = 1,
                tile_rows: int = 0, limit: float = 0.0, slope: float = 0.0) -> torch.Tensor:
     """``x @ W.T`` for many bfloat16 rows and a packed weight, on this package's tiled MFMA kernel (0.85 to 1.1 of

@@ -37,3 +37,16 @@ def test_where_the_tiled_kernel_takes_gated_products(rows, n, k, pays, clamped):
                                            (16301, 37888, 3584, False), (4096, 17920, 2560, False), (4096, 1408, 4096, False), (8192, 59136, 8192, False)])
 def test_many_rows_of_gated_products(rows, n, k, pays):
     assert kernels.tiled_gated_pays(rows, k, False, n) == pays
+
+
+@pytest.mark.parametrize("rows,n,k,pays", [(16301, 37888, 3584, True), (3200, 37888, 3584, True), (500, 37888, 3584, True), (256, 37888, 3584, False), (255, 27648, 5120, True),
+                                           (192, 27648, 5120, False), (2560, 14336, 4096, False), (1024, 22016, 4096, False), (2048, 1408, 4096, False),
+                                           (4096, 37888, 2048, False), (4096, 28672, 7168, False)])
+def test_where_the_tiled_kernel_takes_long_reductions(rows, n, k, pays):
+    """By how full its rounds are; a padded step takes the kernel of its own rows."""
+    assert kernels.tiled_gated_pays_in_long_reductions(rows, k, n) == pays
+    assert not kernels.tiled_gated_pays_in_long_reductions(rows, k + 8, n)
+    for count in range(1, 8193, 13):
+        multiple = 64 if count <= 1024 else 256
+        padded = -(-count // multiple) * multiple
+        assert kernels.tiled_gated_pays_in_long_reductions(count, k, n) == kernels.tiled_gated_pays_in_long_reductions(padded, k, n), count
