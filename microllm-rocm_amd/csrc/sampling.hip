@@ -27,10 +27,20 @@ __device__ inline Best better(Best a, Best b) {
 __device__ inline Best block_argmax(const float* row, int vocab, bool* bad, Best* best_scratch, int* bad_scratch) {
     Best best{-INFINITY, 0x7fffffff};
     int non_finite = 0;
-    for (int index = threadIdx.x; index < vocab; index += blockDim.x) {
-        const float value = row[index];
-        if (!isfinite(value)) non_finite = 1;
-        if (value > best.value) best = Best{value, index};  // ascending index: keeps the first maximum
+    constexpr int kAtOnce = 10;
+    for (int first = threadIdx.x; first < vocab; first += kAtOnce * blockDim.x) {
+        float value[kAtOnce];
+#pragma unroll
+        for (int j = 0; j < kAtOnce; ++j) {
+            const int index = first + j * static_cast<int>(blockDim.x);
+            value[j] = row[min(index, vocab - 1)];
+        }
+#pragma unroll
+        for (int j = 0; j < kAtOnce; ++j) {
+            const int index = first + j * static_cast<int>(blockDim.x);
+            if (index < vocab && !isfinite(value[j])) non_finite = 1;
+            if (index < vocab && value[j] > best.value) best = Best{value[j], index};  // ascending index: keeps the first maximum
+        }
     }
 #pragma unroll
     for (int offset = kWave / 2; offset > 0; offset >>= 1) {
@@ -138,7 +148,9 @@ __device__ inline V wave_inclusive_scan(V value) {
 // ---- sampling ------------------------------------------------------------------------------------------------
 // A row of a large vocabulary is too much for one workgroup (one compute unit waits for one load after the
 // other): the row is cut into slices, a workgroup of 4 waves per slice, each wave taking a quarter (a "piece"),
-// and the work into stages, one kernel each:
+// and the work into stages, one kernel each. A kernel is bound by the reads that wait for one another, so a thread asks for all of its
+// logits (about ten) and all that the earlier stages left before it uses any. 32 rows of 151936, a quarter of them with top-k,
+// 80 -> 49 us; without top-k 39 -> 19; one row 27 -> 13, with top-k 49 -> 30:
 //   1. every slice's maximum, first maximum's index and whether it holds a non-finite value;
 //   2. with top_k: the k-th largest key of the row by radix select, 11, 11 and 10 bits at a time: three kernels
 //      that each add their slice's histogram of the next digit to the row's (integer adds: the order does not
@@ -219,46 +231,60 @@ __global__ __launch_bounds__(kSliceThreads) void sample_slices_kernel(const floa
         mine[layout.histograms + index] = 0;
 }
 
-// The row's maximum (first index) and whether any slice saw a non-finite value; every thread gets the same.
-__device__ inline Best row_best(const int32_t* mine, const SampleLayout& layout, bool* bad) {
-    const ArgmaxPart* parts = reinterpret_cast<const ArgmaxPart*>(mine + layout.parts);
-    Best best{-INFINITY, 0x7fffffff};
-    int any_bad = 0;
-    for (int index = 0; index < layout.slices; ++index) {
-        const ArgmaxPart part = parts[index];
-        best = better(best, Best{part.value, part.index});
-        any_bad |= part.bad;
-    }
-    *bad = any_bad != 0;
+// The row's maximum (first index) and whether any slice saw a non-finite value; every thread gets the same. A lane a slice: there are at most
+// 64, and the first maximum does not depend on the order in which they are compared.
+static_assert(kWave == 64, "a lane a slice");
+struct SlicePart {      // the lane's, asked for early
+    ArgmaxPart part;
+};
+__device__ inline SlicePart ask_for_part(const int32_t* mine, const SampleLayout& layout, int lane) {
+    const int4 words = reinterpret_cast<const int4*>(mine + layout.parts)[min(lane, layout.slices - 1)];
+    return SlicePart{ArgmaxPart{__int_as_float(words.x), words.y, words.z, words.w}};
+}
+__device__ inline Best row_best(const SlicePart& of_lane, bool* bad) {
+    Best best{of_lane.part.value, of_lane.part.index};
+#pragma unroll
+    for (int offset = kWave / 2; offset > 0; offset >>= 1)
+        best = better(best, Best{__shfl_xor(best.value, offset, kWave), __shfl_xor(best.index, offset, kWave)});
+    *bad = __ballot(of_lane.part.bad != 0) != 0ull;
     return best;
 }
 
 __device__ inline int radix_shift(int pass) { return pass == 0 ? 21 : (pass == 1 ? 10 : 0); }
 __device__ inline int radix_bins(int pass) { return pass == 2 ? 1024 : kRadixBins; }
 
+// A thread's counters of a pass's histogram: thread t holds the counters bins - 1 - per * t downwards, per = 8 or 4.
+struct Counters {
+    int count[8];
+};
+__device__ inline Counters ask_for_counters(const int32_t* histogram, int pass) {
+    const int per = radix_bins(pass) / kSliceThreads;
+    const int4* words = reinterpret_cast<const int4*>(histogram + radix_bins(pass) - per * (static_cast<int>(threadIdx.x) + 1));
+    const int4 upper = words[per / 4 - 1];
+    int4 lower = make_int4(0, 0, 0, 0);
+    if (per == 8) lower = words[0];
+    return Counters{{upper.w, upper.z, upper.y, upper.x, lower.w, lower.z, lower.y, lower.x}};
+}
+
 // The digit of pass `pass` of the remaining-th largest key among those that share the earlier digits: walks the
-// row's histogram from the top. Thread t holds the counters bins - 1 - per * t downwards. All threads of the
+// row's histogram from the top. All threads of the
 // workgroup call it; the answer comes back in *prefix and *remaining.
-__device__ inline void pick_digit(const int32_t* histogram, int pass, uint32_t* prefix, int* remaining, int* scan_scratch,
+__device__ inline void pick_digit(const Counters& counters, int pass, uint32_t* prefix, int* remaining, int* scan_scratch,
                                   uint32_t* shared_prefix, int* shared_remaining) {
     const int bins = radix_bins(pass);
     const int per = bins / kSliceThreads;      // 8 or 4
     const int top = bins - 1 - per * static_cast<int>(threadIdx.x);
-    int count[8];
     int mine = 0;
 #pragma unroll
-    for (int j = 0; j < 8; ++j) {
-        count[j] = j < per ? histogram[top - j] : 0;
-        mine += count[j];
-    }
+    for (int j = 0; j < 8; ++j) mine += counters.count[j];
     const int above = block_exclusive_scan<int>(mine, scan_scratch);
     if (above < *remaining && *remaining <= above + mine) {
         int left = *remaining - above;
         int digit = top;
 #pragma unroll
         for (int j = 0; j < 8; ++j) {
-            if (j < per && left > count[j]) {
-                left -= count[j];
+            if (j < per && left > counters.count[j]) {
+                left -= counters.count[j];
                 digit = top - j - 1;
             } else {
                 break;
@@ -272,6 +298,8 @@ __device__ inline void pick_digit(const int32_t* histogram, int pass, uint32_t* 
     *remaining = *shared_remaining;
     __syncthreads();
 }
+
+constexpr int kLogitsAtOnce = 10;      // of a slice by a thread: all of a vocabulary of up to 163840
 
 __global__ __launch_bounds__(kSliceThreads) void sample_histogram_kernel(
     const float* __restrict__ logits, const float* __restrict__ temperature, const int32_t* __restrict__ top_k,
@@ -287,20 +315,31 @@ __global__ __launch_bounds__(kSliceThreads) void sample_histogram_kernel(
     const float* row = logits + static_cast<int64_t>(blockIdx.x) * vocab;
     const int lane = threadIdx.x % kWave;
 
-    uint32_t prefix = 0, mask = 0;
-    int remaining = rule.k;
-    for (int earlier = 0; earlier < pass; ++earlier) {
-        pick_digit(mine + layout.histograms + earlier * kRadixBins, earlier, &prefix, &remaining, scan_scratch, &shared_prefix, &shared_remaining);
-        mask |= static_cast<uint32_t>(radix_bins(earlier) - 1) << radix_shift(earlier);
-    }
-    for (int index = threadIdx.x; index < kRadixBins; index += kSliceThreads) histogram[index] = 0;
-    __syncthreads();
     const int shift = radix_shift(pass), bins = radix_bins(pass);
     const int begin = min(static_cast<int>(blockIdx.y) * layout.slice, vocab);
     const int end = min(begin + layout.slice, vocab);
-    for (int base = begin; base < end; base += kSliceThreads) {
-        const int index = base + threadIdx.x;
-        const uint32_t key = index < end ? order_key(row[index]) : 0u;
+    float value[kLogitsAtOnce];
+    auto ask = [&](int base) {
+#pragma unroll
+        for (int j = 0; j < kLogitsAtOnce; ++j) value[j] = row[min(base + j * kSliceThreads + static_cast<int>(threadIdx.x), vocab - 1)];
+    };
+    ask(begin);
+    Counters counters[kRadixPasses - 1];
+#pragma unroll
+    for (int earlier = 0; earlier < kRadixPasses - 1; ++earlier)
+        if (earlier < pass) counters[earlier] = ask_for_counters(mine + layout.histograms + earlier * kRadixBins, earlier);
+    for (int index = threadIdx.x; index < kRadixBins; index += kSliceThreads) histogram[index] = 0;
+    uint32_t prefix = 0, mask = 0;
+    int remaining = rule.k;
+#pragma unroll
+    for (int earlier = 0; earlier < kRadixPasses - 1; ++earlier) {
+        if (earlier >= pass) break;
+        pick_digit(counters[earlier], earlier, &prefix, &remaining, scan_scratch, &shared_prefix, &shared_remaining);
+        mask |= static_cast<uint32_t>(radix_bins(earlier) - 1) << radix_shift(earlier);
+    }
+    __syncthreads();
+    auto count_in = [&](int index, float logit) {
+        const uint32_t key = index < end ? order_key(logit) : 0u;
         const bool counts = index < end && (key & mask) == prefix;
         const int bin = static_cast<int>((key >> shift) & static_cast<uint32_t>(bins - 1));
         // Logits of one row share their top bits: most lanes of a wave want the same few counters, and LDS adds
@@ -315,10 +354,28 @@ __global__ __launch_bounds__(kSliceThreads) void sample_histogram_kernel(
             todo &= ~same;
         }
         if ((todo >> lane) & 1ull) atomicAdd(&histogram[bin], 1);
+    };
+    for (int base = begin; base < end; base += kLogitsAtOnce * kSliceThreads) {
+        if (base > begin) ask(base);
+#pragma unroll
+        for (int j = 0; j < kLogitsAtOnce; ++j)
+            if (base + j * kSliceThreads < end) count_in(base + j * kSliceThreads + static_cast<int>(threadIdx.x), value[j]);
     }
     __syncthreads();
     for (int index = threadIdx.x; index < bins; index += kSliceThreads)
         if (histogram[index] != 0) atomicAdd(&mine[layout.histograms + pass * kRadixBins + index], histogram[index]);
+}
+
+// A lane's four logits of a block of a piece.
+struct BlockLogits {
+    float value[4];
+};
+constexpr int kBlocksAtOnce = 3;      // all of a piece of a vocabulary of up to 196608
+__device__ inline BlockLogits ask_for_block(const float* row, int base, int lane, int vocab) {
+    BlockLogits block;
+#pragma unroll
+    for (int j = 0; j < 4; ++j) block.value[j] = row[min(base + j * kWave + lane, vocab - 1)];
+    return block;
 }
 
 __global__ __launch_bounds__(kSliceThreads) void sample_sums_kernel(
@@ -333,33 +390,43 @@ __global__ __launch_bounds__(kSliceThreads) void sample_sums_kernel(
     int32_t* mine = workspace + static_cast<int64_t>(blockIdx.x) * layout.per_row;
     const float* row = logits + static_cast<int64_t>(blockIdx.x) * vocab;
     const int lane = threadIdx.x % kWave, wave = threadIdx.x / kWave;
+    int begin, end;
+    piece_bounds(layout, vocab, blockIdx.y, wave, &begin, &end);
+    const SlicePart part = ask_for_part(mine, layout, lane);
+    Counters counters[kRadixPasses];
+    if (rule.k < vocab) {
+#pragma unroll
+        for (int pass = 0; pass < kRadixPasses; ++pass) counters[pass] = ask_for_counters(mine + layout.histograms + pass * kRadixBins, pass);
+    }
+    BlockLogits block[kBlocksAtOnce];
+#pragma unroll
+    for (int i = 0; i < kBlocksAtOnce; ++i) block[i] = ask_for_block(row, begin + i * kBlockTokens, lane, vocab);
     bool bad;
-    const Best best = row_best(mine, layout, &bad);
+    const Best best = row_best(part, &bad);
     if (bad) return;
 
     uint32_t threshold_key = 0;   // the k-th largest key; keys above it are in, of its equals the first take_equal
     int take_equal = 0;
     if (rule.k < vocab) {
         int remaining = rule.k;
+#pragma unroll
         for (int pass = 0; pass < kRadixPasses; ++pass)
-            pick_digit(mine + layout.histograms + pass * kRadixBins, pass, &threshold_key, &remaining, scan_scratch, &shared_prefix, &shared_remaining);
+            pick_digit(counters[pass], pass, &threshold_key, &remaining, scan_scratch, &shared_prefix, &shared_remaining);
         take_equal = remaining;
         if (blockIdx.y == 0 && threadIdx.x == 0) {
             mine[layout.select] = static_cast<int32_t>(threshold_key);
             mine[layout.select + 1] = take_equal;
         }
     }
-    int begin, end;
-    piece_bounds(layout, vocab, blockIdx.y, wave, &begin, &end);
     const float scaled_max = best.value / rule.tau;
     float lane_total = 0.0f;
     int lane_equal = 0;
-    for (int base = begin; base < end; base += kBlockTokens) {
+    auto weigh = [&](int base, const BlockLogits& logits) {
         float weight[4];
 #pragma unroll
         for (int j = 0; j < 4; ++j) {
             const int index = base + j * kWave + lane;
-            const float value = index < end ? row[index] : 0.0f;
+            const float value = logits.value[j];
             bool in = index < end;
             if (rule.k < vocab) {
                 const uint32_t key = order_key(value);
@@ -369,7 +436,11 @@ __global__ __launch_bounds__(kSliceThreads) void sample_sums_kernel(
             weight[j] = in ? expf(value / rule.tau - scaled_max) : 0.0f;
         }
         lane_total += (weight[0] + weight[1]) + (weight[2] + weight[3]);
-    }
+    };
+#pragma unroll
+    for (int i = 0; i < kBlocksAtOnce; ++i)
+        if (begin + i * kBlockTokens < end) weigh(begin + i * kBlockTokens, block[i]);
+    for (int base = begin + kBlocksAtOnce * kBlockTokens; base < end; base += kBlockTokens) weigh(base, ask_for_block(row, base, lane, vocab));
     const float total = wave_sum(lane_total);
     const int equal = wave_count(lane_equal);
     if (lane == 0) {
@@ -387,8 +458,16 @@ __global__ __launch_bounds__(kWave) void sample_draw_kernel(
     const float* row = logits + static_cast<int64_t>(row_index) * vocab;
     const int lane = threadIdx.x;
     const RowRule rule = row_rule(temperature, top_k, row_index, vocab);
+    const SlicePart part = ask_for_part(mine, layout, lane);
+    // The pieces' sums in order: lane l holds pieces 4l .. 4l + 3. (What a row that is not drawn from left there is not used.)
+    const int pieces = layout.slices * kSliceWaves;       // at most 256
+    const int last_words = layout.slices - 1;             // four pieces to a slice
+    const int4 sum_words = reinterpret_cast<const int4*>(mine + layout.sums)[min(lane, last_words)];
+    const int4 equal_words = reinterpret_cast<const int4*>(mine + layout.equals)[min(lane, last_words)];
+    const int select_key = mine[layout.select], select_equal = mine[layout.select + 1];
+    const float row_uniform = uniform[row_index];
     bool bad;
-    const Best best = row_best(mine, layout, &bad);
+    const Best best = row_best(part, &bad);
     if (bad || !rule.weighted) {
         if (lane == 0) out[row_index] = bad ? -1 : best.index;
         return;
@@ -400,21 +479,20 @@ __global__ __launch_bounds__(kWave) void sample_draw_kernel(
     int take_equal = 0;
     float equal_weight = 0.0f;      // every token equal to the k-th value weighs the same
     if (k < vocab) {
-        threshold_key = static_cast<uint32_t>(mine[layout.select]);
-        take_equal = mine[layout.select + 1];
+        threshold_key = static_cast<uint32_t>(select_key);
+        take_equal = select_equal;
         equal_weight = expf(value_of_key(threshold_key) / tau - scaled_max);
     }
 
-    // The pieces' sums in order: lane l holds pieces 4l .. 4l + 3.
-    const int pieces = layout.slices * kSliceWaves;       // at most 256
+    const int sum_word[4] = {sum_words.x, sum_words.y, sum_words.z, sum_words.w}, equal_word[4] = {equal_words.x, equal_words.y, equal_words.z, equal_words.w};
     float piece_sum[4];
     int piece_equal[4];
     int lane_equal = 0;
 #pragma unroll
     for (int j = 0; j < 4; ++j) {
         const int piece = 4 * lane + j;
-        piece_sum[j] = piece < pieces ? reinterpret_cast<const float*>(mine + layout.sums)[piece] : 0.0f;
-        piece_equal[j] = (piece < pieces && k < vocab) ? mine[layout.equals + piece] : 0;
+        piece_sum[j] = piece < pieces ? __int_as_float(sum_word[j]) : 0.0f;
+        piece_equal[j] = (piece < pieces && k < vocab) ? equal_word[j] : 0;
         lane_equal += piece_equal[j];
     }
     int equal_before[4];
@@ -432,7 +510,7 @@ __global__ __launch_bounds__(kWave) void sample_draw_kernel(
     const float inclusive = wave_inclusive_scan<float>(lane_sum);
     const float total = __shfl(inclusive, kWave - 1, kWave);
     const float exclusive_up = __shfl_up(inclusive, 1, kWave);
-    const float target = uniform[row_index] * total;
+    const float target = row_uniform * total;
     // The draw falls into the last piece that holds a selected token and begins at or below the target.
     float piece_before[4];
     int candidate = -1;
@@ -471,12 +549,19 @@ __global__ __launch_bounds__(kWave) void sample_draw_kernel(
     const unsigned long long lanes_below = (1ull << lane) - 1ull;
     float running = before;
     int chosen = -1, last_selected = -1;
+    BlockLogits ahead[kBlocksAtOnce];
+#pragma unroll
+    for (int i = 0; i < kBlocksAtOnce; ++i) ahead[i] = ask_for_block(row, begin + i * kBlockTokens, lane, vocab);
     for (int base = begin; base < end && chosen < 0; base += kBlockTokens) {
+        const BlockLogits logits = ahead[0];
+#pragma unroll
+        for (int i = 0; i + 1 < kBlocksAtOnce; ++i) ahead[i] = ahead[i + 1];
+        ahead[kBlocksAtOnce - 1] = ask_for_block(row, base + kBlocksAtOnce * kBlockTokens, lane, vocab);
         float weight[4];
 #pragma unroll
         for (int j = 0; j < 4; ++j) {
             const int index = base + j * kWave + lane;
-            const float value = index < end ? row[index] : 0.0f;
+            const float value = index < end ? logits.value[j] : 0.0f;
             bool in = index < end;
             if (k < vocab) {
                 const uint32_t key = order_key(value);

@@ -771,3 +771,22 @@ def test_experts_with_gates_of_every_size(tokens, grouped, kind):
     ids, weights = (torch.arange(tokens, device=DEVICE, dtype=torch.int32) % 2)[:, None].contiguous(), torch.ones((tokens, 1), device=DEVICE)
     options = dict(activation="clamped_glu", limit=CLAMP, slope=SLOPE) if kind == "clamped" else {}
     assert_gated(k.moe_experts(x, ids, weights, gate_up, down, False, grouped=grouped, **options)[0], gates, ups, kind)
+
+
+@pytest.mark.parametrize("vocab", [1, 63, 2048, 131072, 163840, 163841, 196608, 196609, 330000])
+def test_tokens_of_vocabularies_up_to_and_beyond_what_a_thread_asks_for_at_once(vocab):
+    """Ten logits of a slice a thread and twelve of a piece: one more, and the loops go round again. Top-k against torch's, ends of the range of draws."""
+    k, generator = kernels(), torch.Generator(device=DEVICE).manual_seed(vocab)
+    logits = torch.randn((6, vocab), generator=generator, device=DEVICE)
+    logits[1, vocab - 1] = 9.0                      # the last token of all is the first maximum
+    logits[2] = logits[2].round()                   # ties at the k-th value
+    top = min(vocab, 30)
+    values = torch.tensor([[0.8, 0.0, 0.7, 1.0, 0.9, 1.1], [0.0, 0.5, 0.999999, 0.5, 0.999999, 0.0]], device=DEVICE)
+    chosen = k.sample(logits, values[0], torch.tensor([top, 0, top, 1, 0, 0], dtype=torch.int32, device=DEVICE), values[1]).tolist()
+    assert chosen[1] == vocab - 1 and chosen[3] == int(logits[3].argmax()) and chosen[5] == 0 and chosen[4] > vocab - 1 - max(2, vocab // 100)
+    for row, first in ((0, True), (2, False)):      # the lowest ids among those that equal the k-th value
+        kept = sorted(torch.sort(logits[row], descending=True, stable=True).indices[:top].tolist())
+        assert chosen[row] in (kept[:2] if first else kept[-2:])
+    assert k.argmax(logits).tolist() == logits.argmax(1).tolist()
+    logits[4, vocab // 2] = float("inf")
+    assert k.argmax(logits)[4] == -1 and k.sample(logits, values[0], None, values[1])[4] == -1
