@@ -20,7 +20,7 @@ from ..cache.needs import flat_needs
 from ..cache.pages import OutOfPages
 from ..config.registry import architecture_named, load_config
 from ..ops import kernels, library
-from ..ops.transfers import device_copy, on_device
+from ..ops.transfers import device_copy, on_device_later
 from ..parts import Model, ModelSpec, Runtime
 from ..weights import load_folder, place_all, random_tensors
 from .batch import BatchBuilder, FixedShape, HostBatch, StepContext, StepEntry
@@ -263,7 +263,7 @@ class Engine:
             return None
         if len(wanted) == n:
             return state.logits if self._borrow else device_copy(state.logits)
-        return state.logits[on_device(wanted, self.device, dtype=torch.int64)]
+        return state.logits[on_device_later(np.asarray(wanted, dtype=np.int64), self.device)]
 
     # ---- mixed steps from graphs -----------------------------------------------------------
     def _fixed_shape(self, batch: HostBatch) -> Optional[FixedShape]:
@@ -304,7 +304,7 @@ class Engine:
         if [place for place, _ in taking] == list(range(count)) and [row for _, row in taking] == list(range(count)):
             tokens[:count].copy_(source[:count])      # the same requests in the same order as the step before
             return
-        both = on_device(np.asarray(taking, dtype=np.int64).T.copy(), self.device)
+        both = on_device_later(np.asarray(taking, dtype=np.int64).T.copy(), self.device)
         tokens.index_copy_(0, both[0], source.index_select(0, both[1]))
 
     def _mixed_graph_step(self, shape: FixedShape, batch: HostBatch) -> Optional[torch.Tensor]:

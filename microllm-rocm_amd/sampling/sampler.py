@@ -20,7 +20,7 @@ import numpy as np
 import torch
 
 from ..ops import kernels
-from ..ops.transfers import count_copy_to_host, on_device, on_host
+from ..ops.transfers import count_copy_to_host, on_device_later, on_host
 
 _MASK = (1 << 64) - 1
 
@@ -97,7 +97,7 @@ class Sampler:
         packed[0] = [0.0 if p.greedy else p.temperature for p in params]
         packed[1].view(np.int32)[:] = [p.top_k for p in params]
         packed[2] = [uniform_for(p.seed, d) for p, d in zip(params, draws)]
-        values = on_device(packed, logits.device)
+        values = on_device_later(packed, logits.device)
         temperature, top_k, uniform = values[0], values[1].view(torch.int32), values[2]
         if all(p.top_k == 0 for p in params):
             top_k = None      # no row is restricted: the kernel leaves its search for the k-th value out
