@@ -2,8 +2,8 @@
 // bfloat16 A [M, K] (row-major) and the packed weight the streaming kernel reads ([N/16][K/32][4][16][8]).
 // Still bound by reading W once from HBM, but with this many rows the activations a wave needs per piece of W
 // are several times the piece: here the 4 or 8 waves of a workgroup walk the same k steps, each over its own one
-// or two tiles of W, and share the activations through LDS (8 k steps at a time, double buffered, brought in MFMA
-// operand order by all waves together). A wave keeps two stages of its tiles in registers: one on its way while
+// or two tiles of W, and share the activations through LDS (8 k steps at a time, double buffered, loaded straight
+// into it by all waves together). A wave keeps two stages of its tiles in registers: one on its way while
 // the other is multiplied. All loads go through buffer descriptors, which return zeros past their end: a load
 // under a condition would make the compiler wait for all loads before it.
 //
@@ -50,7 +50,9 @@ __global__ __launch_bounds__(kWaves * kWave) void gemm_medium_kernel(
     int m, int n, int k, int n_tiles, int k_steps, int steps_per_split, int tiles) {
     constexpr int kStagePieces = MT * kStepsPerStage;             // pieces of A in a buffer, 1 KB each
     constexpr int kPiecesPerWave = kStagePieces / kWaves;
-    extern __shared__ uintx4 stage[];                             // [2][MT][kStepsPerStage][64 lanes]
+    // Two buffers, [pair of k steps][MT * 16 rows][8 places of 16 bytes]: 128 bytes of a row, whose chunk c is at place c ^ (row / 2). Two variables,
+    // so that the compiler knows which of them a load into LDS fills.
+    __shared__ uintx4 buffer_even[kStagePieces * kWave], buffer_odd[kStagePieces * kWave];
 
     const int lane = threadIdx.x % kWave;
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave);
@@ -70,15 +72,18 @@ __global__ __launch_bounds__(kWaves * kWave) void gemm_medium_kernel(
         w_at[nt] = wave + kWaves * nt < live_tiles ? static_cast<unsigned>((wave + kWaves * nt) * k_steps * 1024 + lane * 16) : kPast;
         asm("" : "+v"(w_at[nt]));       // else the choice becomes a branch around the loads
     }
-    // This wave's share of a buffer: every kWaves-th k step of a stage, of all rows.
-    static_assert(kStepsPerStage % kWaves == 0, "the waves share the copying evenly");
-    unsigned a_at[MT];
+    // This wave's share of a buffer: pieces wave, wave + kWaves, ... of 8 rows of 128 bytes (a pair of k steps). A piece is a load straight into LDS, of
+    // whole lines (in MFMA operand order, 64 bytes of 16 rows a load by way of registers, every line was asked for twice: 64 rows of
+    // 37888 x 3584 gated 54.9 -> 51.3 us, 3584 x 18944 31.1 -> 30.2, 9728 x 896 gated 9.0 -> 7.8, 896 x 4864 6.9 -> 5.9, 32 rows 47.2 -> 46.7, 25.4 -> 25.3, 6.5 -> 6.2
+    // and 5.1 -> 4.7; 16 weights at 17 to 64 rows 1.05 times as fast on the mean, none slower. Without the activations' loads 49.8 and 28.4 us.)
+    constexpr int kOctets = 2 * MT;      // groups of 8 rows
+    int a_at[kPiecesPerWave], a_left[kPiecesPerWave];      // where the lane reads at step 0, and below how many elements from there its steps begin
 #pragma unroll
-    for (int mt = 0; mt < MT; ++mt) {
-        a_at[mt] = 16 * mt + col < m ? static_cast<unsigned>((16 * mt + col) * k * 2 + quad * 16) : kPast;
-        asm("" : "+v"(a_at[mt]));
+    for (int j = 0; j < kPiecesPerWave; ++j) {
+        const int piece = wave + kWaves * j, row = piece % kOctets * 8 + lane / 8, chunk = (lane % 8) ^ (row % 16 / 2), element = piece / kOctets * 64 + chunk * 8;
+        a_at[j] = (row * k + element) * 2;
+        a_left[j] = row < m ? (FAR && end_step == k_steps ? k : min(k, end_step * 32)) - element : 0;
     }
-    const int a_end = (FAR && end_step == k_steps ? k : min(k, end_step * 32)) - quad * 8;      // a lane's steps begin before this element
 
     auto load_w = [&](Piece (&pieces)[kStepsPerStage][NT], int stage_number) {
         const int step = first_step + stage_number * kStepsPerStage;
@@ -97,23 +102,31 @@ __global__ __launch_bounds__(kWaves * kWave) void gemm_medium_kernel(
             }
         }
     };
-    auto load_share = [&](uintx4 (&share)[kPiecesPerWave], int stage_number) {
+    auto load_share = [&](uintx4* buffer, int stage_number) __attribute__((always_inline)) {
 #pragma unroll
         for (int j = 0; j < kPiecesPerWave; ++j) {
-            const int step = first_step + stage_number * kStepsPerStage + wave + kWaves * (j / MT);
+            const int step = first_step + stage_number * kStepsPerStage;
+            uintx4* place = buffer + (wave + kWaves * j) * kWave;
+            const bool there = static_cast<int64_t>(step) * 32 < a_left[j];
             if constexpr (FAR) {
-                const int row = 16 * (j % MT) + col;
-                const bf16* from = a + static_cast<int64_t>(row) * k + static_cast<int64_t>(step) * 32 + quad * 8;
-                share[j] = row < m && static_cast<int64_t>(step) * 32 < a_end ? *reinterpret_cast<const uintx4*>(from) : uintx4{0u, 0u, 0u, 0u};
+                const int piece = wave + kWaves * j, row = piece % kOctets * 8 + lane / 8, chunk = (lane % 8) ^ (row % 16 / 2);
+                const bf16* from = a + static_cast<int64_t>(row) * k + static_cast<int64_t>(step) * 32 + piece / kOctets * 64 + chunk * 8;
+                place[lane] = there ? *reinterpret_cast<const uintx4*>(from) : uintx4{0u, 0u, 0u, 0u};
             } else {
-                share[j] = __builtin_amdgcn_raw_buffer_load_b128(a_rsrc, a_at[j % MT] + (step * 32 < a_end ? static_cast<unsigned>(step) * 64 : kPast), 0, 0);
+                const int at = there ? a_at[j] + step * 64 : static_cast<int>(kPast);
+                __builtin_amdgcn_raw_ptr_buffer_load_lds(a_rsrc, place, 16, at, 0, 0, 0);
             }
         }
     };
-    auto store_share = [&](const uintx4 (&share)[kPiecesPerWave], int buffer) {
-#pragma unroll
-        for (int j = 0; j < kPiecesPerWave; ++j)
-            stage[(buffer * kStagePieces + j % MT * kStepsPerStage + wave + kWaves * (j / MT)) * kWave + lane] = share[j];
+    // The share that was asked for before the last `LATER` loads has landed, the wave's reads of the other buffer have arrived, and the workgroup meets.
+    auto share_landed = [&]() __attribute__((always_inline)) {
+        if constexpr (FAR) {
+            __syncthreads();
+        } else {
+            asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)" ::"n"(NT * kStepsPerStage) : "memory");
+            __builtin_amdgcn_s_barrier();
+            asm volatile("" ::: "memory");
+        }
     };
 
     floatx4 acc[NT][MT];
@@ -125,11 +138,12 @@ __global__ __launch_bounds__(kWaves * kWave) void gemm_medium_kernel(
     // With one tile a wave a step's activations are read from LDS while the step before is multiplied: left alone, the compiler reads them one or two
     // ahead of their products (48 rows of 1152 x 896 3.46 -> 3.25 us, 64 rows of 9728 x 896 8.9 -> 8.5, of 3584 x 3584 9.67 -> 9.35). With two there
     // are twice as many products to cover a read, and the order it chooses is the better one (32 rows of 37888 x 3584 44.3, 44.9 this way).
-    auto multiply = [&](const Piece (&pieces)[kStepsPerStage][NT], int buffer) {
+    const int a_place[2] = {col * 8 + (quad ^ (col / 2)), col * 8 + ((4 + quad) ^ (col / 2))};      // of a pair's first step and its second
+    auto multiply = [&](const Piece (&pieces)[kStepsPerStage][NT], const uintx4* buffer) __attribute__((always_inline)) {
         Piece a_piece[2][MT];
         auto read = [&](int u) {
 #pragma unroll
-            for (int mt = 0; mt < MT; ++mt) a_piece[u % 2][mt].raw = stage[(buffer * kStagePieces + mt * kStepsPerStage + u) * kWave + lane];
+            for (int mt = 0; mt < MT; ++mt) a_piece[u % 2][mt].raw = buffer[(u / 2 * MT + mt) * (2 * kWave) + a_place[u % 2]];
         };
         if constexpr (NT == 1) read(0);
 #pragma unroll
@@ -149,39 +163,30 @@ __global__ __launch_bounds__(kWaves * kWave) void gemm_medium_kernel(
         }
     };
 
-    // The activations of a stage are asked for before its tiles: loads come back in order, and the copy into LDS must not wait
-    // for the tiles. A buffer was last read in the stage before the one that fills it, and every wave has passed that
-    // stage's barrier.
-    uintx4 share[kPiecesPerWave];
+    // The activations of a stage are asked for before its tiles: loads come back in order, and the buffer must not wait
+    // for the tiles. A buffer was last read in the stage before the one that fills it, and the workgroup has met since.
     Piece w_even[kStepsPerStage][NT], w_odd[kStepsPerStage][NT];
-    load_share(share, 0);
+    load_share(buffer_even, 0);
     load_w(w_even, 0);
     __builtin_amdgcn_sched_barrier(0);
-    store_share(share, 0);
-    __syncthreads();
+    share_landed();
     // Two stages a round, and what is left of an odd number after the rounds: were the loop left between the two, the compiler would think that it
     // comes round with the odd tiles' loads on their way, and wait for all loads at the start of every round (17 rows of 9728 x 896
     // 6.84 -> 5.87 us, of 3584 x 18944 23.8 -> 22.7, 64 rows of 1152 x 896 4.37 -> 3.64, of 896 x 4864 7.05 -> 6.67, of 37888 x 3584 50.6 -> 50.3).
-    // Of four waves, which bring more pieces of the activations each, the compiler would also mix these loads with the tiles' (48 rows of 9728 x 896
-    // 8.3 -> 7.7 us); eight waves of 64 rows lose by the same line (3584 x 3584 9.7 -> 10.1).
     int s = 0;
     for (; s + 1 < n_stages; s += 2) {
-        load_share(share, s + 1);
-        if constexpr (kWaves == 4) __builtin_amdgcn_sched_barrier(0);
+        load_share(buffer_odd, s + 1);
         load_w(w_odd, s + 1);
         __builtin_amdgcn_sched_barrier(0);      // else the loads sink below the products, behind their waits
-        multiply(w_even, 0);
-        store_share(share, 1);
-        __syncthreads();
-        load_share(share, s + 2);
-        if constexpr (kWaves == 4) __builtin_amdgcn_sched_barrier(0);
+        multiply(w_even, buffer_even);
+        share_landed();
+        load_share(buffer_even, s + 2);
         load_w(w_even, s + 2);
         __builtin_amdgcn_sched_barrier(0);
-        multiply(w_odd, 1);
-        store_share(share, 0);
-        __syncthreads();
+        multiply(w_odd, buffer_odd);
+        share_landed();
     }
-    if (s < n_stages) multiply(w_even, 0);
+    if (s < n_stages) multiply(w_even, buffer_even);
 
     // acc[nt][mt][i] = C[row mt*16 + col][column n_tile*16 + quad*4 + i]
 #pragma unroll
@@ -264,15 +269,14 @@ static void launch_rows(const bf16* a, const bf16* w, void* out, int m, int n, i
     const bool far = k_steps > kMostSteps;
     const int tiles = tiles_of(m, n, k, splits, most_tiles);
     const dim3 grid((n_tiles + tiles - 1) / tiles, splits);
-    const size_t lds = 2 * MT * kStepsPerStage * kWave * sizeof(uintx4);
     const auto launch = [&](auto tiles_a_wave, auto waves) {
         constexpr int kWaves = decltype(waves)::value;
-        gemm_medium_kernel<MT, decltype(tiles_a_wave)::value, kWaves, EPILOGUE, false><<<grid, kWaves * kWave, lds, stream>>>(
+        gemm_medium_kernel<MT, decltype(tiles_a_wave)::value, kWaves, EPILOGUE, false><<<grid, kWaves * kWave, 0, stream>>>(
             a, w, out, m, n, k, n_tiles, k_steps, steps_per_split, tiles);
     };
     using std::integral_constant;
     if (far) {
-        gemm_medium_kernel<MT, 1, 4, EPILOGUE, true><<<grid, 4 * kWave, lds, stream>>>(a, w, out, m, n, k, n_tiles, k_steps, steps_per_split, tiles);
+        gemm_medium_kernel<MT, 1, 4, EPILOGUE, true><<<grid, 4 * kWave, 0, stream>>>(a, w, out, m, n, k, n_tiles, k_steps, steps_per_split, tiles);
         return;
     }
     // Four waves where there are no more tiles (64 rows of 9728 x 896, 3 tiles a workgroup: 11.7 -> 9.6 us, now 8.5). Four waves of up to four

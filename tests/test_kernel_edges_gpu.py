@@ -790,3 +790,22 @@ def test_tokens_of_vocabularies_up_to_and_beyond_what_a_thread_asks_for_at_once(
     assert k.argmax(logits).tolist() == logits.argmax(1).tolist()
     logits[4, vocab // 2] = float("inf")
     assert k.argmax(logits)[4] == -1 and k.sample(logits, values[0], None, values[1])[4] == -1
+
+
+@pytest.mark.parametrize("m", [17, 32, 33, 48, 49, 64])
+@pytest.mark.parametrize("n,k,splits", [(40, 8, 1), (300, 40, 1), (260, 264, 2), (1000, 1032, 3), (4112, 520, 1), (200, 2312, 4)])
+def test_activations_that_are_not_finite_stay_in_their_row(m, n, k, splits):
+    """Reductions that end within a k step, within a pair of them and within a stage: what lies behind a row's end is the next row, all of it NaN here."""
+    ka, generator = kernels(), torch.Generator(device=DEVICE).manual_seed(m + n + k)
+    x, w = ((torch.randn(shape, generator=generator, device=DEVICE) * scale).to(torch.bfloat16) for shape, scale in (((m, k), 1.0), ((n, k), k ** -0.5)))
+    packed, spoilt = ka.pack_weight(w), x.clone()
+    spoilt[1::2] = float("nan")
+    spoilt[m - 1] = float("inf") if m % 2 == 1 else float("nan")
+    for plan in ((2, 8, splits), (1, 4, splits)):
+        whole = ka.gemm_medium(x, packed, n, "f32", plan=plan)
+        got = ka.gemm_medium(spoilt, packed, n, "f32", plan=plan)
+        kept = [row for row in range(0, m - 1, 2)]
+        assert torch.equal(got[..., kept, :], whole[..., kept, :])
+        total = whole.sum(0) if splits > 1 else whole
+        assert float((total - x.float() @ w.float().T).abs().max()) < 2e-6 * k ** 0.5 + 1e-5      # k products of size 1 / sqrt(k)
+        assert not got[..., 1, :].isfinite().any() if splits == 1 else not got.sum(0)[1].isfinite().any()
