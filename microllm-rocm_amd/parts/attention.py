@@ -187,7 +187,7 @@ class PagedAttention(Mixer):
         fused = self.position is None or self.position.fused_split_half
         cos_sin = self.position.table(ctx) if self.position is not None and fused else None
         rotary_packed = weight.row_order is not None and weight.packed is not None and x.dtype == weight.dtype
-        pair_order = rotary_packed and takes_packed(weight, x.shape[0])
+        pair_order = rotary_packed and takes_packed(weight, x.shape[0], address=x.data_ptr())
         if pair_order and x.shape[0] <= SKINNY_ROWS:
             q = kernels.gemm_skinny_qkv(x, weight.packed, bias, slot_mapping, cos_sin, k_pages, v_pages,
                                         self.heads, stored_heads, self.head_dim, view.page_size, scale=scale)

@@ -41,9 +41,11 @@ SKINNY_ROWS = 16        # up to this many rows gemm_skinny beats the library on 
 MEDIUM_ROWS = 64        # and up to this many gemm_medium does: at 17, 32 and 64 rows (the library's time, with the activation's kernel
                         # for gate and up, over this one's) 37888 x 3584 gated 1.27, 1.33 and 1.34, 9728 x 896 gated 2.06, 1.95 and
                         # 1.53, 16384 x 2048 gated 1.42, 1.37 and 1.10, 3584 x 18944 4.2, 4.1 and 2.9; except for
-MEDIUM_WIDE_TILES = 2048   # weights with this many tiles of 16 rows or more that are not gated (the head), which the library has
-MEDIUM_WIDE_ROWS = 40      # beyond this many. It lost less there when the line was drawn than it does now: 152064 x 3584 at 32, 48 and 64
-                           # rows 1.35, 1.07 and 1.06, 151936 x 2048 1.39, 1.33 and 1.35, 151936 x 896 1.15, 1.19 and 1.09
+MEDIUM_WIDE_TILES = 2048   # weights with this many tiles of 16 rows or more that are not gated (the head) where the reduction is short
+MEDIUM_WIDE_ROWS = 40      # beyond this many, or the library tuned. From reductions of
+MEDIUM_WIDE_REDUCTION = 512    # this many on the library's time over this one's at 41, 49 and 64 rows is 1.08, 1.09 and 1.10 for 152064 x 3584, 1.21, 1.16
+                           # and 1.13 for 151936 x 896, 1.42, 1.41 and 1.38 for 151936 x 2048, 1.38, 1.35 and 1.28 for 32768 x 512, 1.20, 1.19 and
+                           # 1.20 for 152064 x 8192 (11 weights, 1.08 at the least); shorter ones were not measured
 MEDIUM_GATED_ROWS = 48     # gated weights with fewer tiles than compute units are the library's beyond this many. Nothing but their results
 MEDIUM_GATED_TILES = 256   # speaks for it (it rounds gate and up, and those steps of the smallest models keep what they gave): it is 2 to
                            # 3 us a layer slower (64 rows: 1024 x 256 7.7 and 5.4, 4080 x 512 9.2 and 6.9)
@@ -94,7 +96,8 @@ def linear_into_stream(x: torch.Tensor, weight: "Weight", residual: Residual) ->
 
 def takes_packed(weight: "Weight", rows: int, gated: bool = False, address: int = 0) -> bool:
     """Whether ``linear`` multiplies this many rows, that begin at ``address``, with the packed copy (whose rows may be in
-    ``row_order``). From 49 gated rows on the library takes those that begin at no 16-byte boundary, which gemm_medium's loads need."""
+    ``row_order``). From 49 gated rows on, and from 41 of wide weights, the library takes those that begin at no 16-byte boundary, which
+    gemm_medium's loads need."""
     if weight.packed is None:
         return False
     if rows <= SKINNY_ROWS or weight.tensor is None:
@@ -102,8 +105,9 @@ def takes_packed(weight: "Weight", rows: int, gated: bool = False, address: int 
     tiles = -(-weight.out_features // 16)
     if gated:
         return rows <= (MEDIUM_ROWS if tiles >= MEDIUM_GATED_TILES and address % 16 == 0 else MEDIUM_GATED_ROWS)
-    wide = tiles >= MEDIUM_WIDE_TILES
-    return rows <= (MEDIUM_WIDE_ROWS if wide else MEDIUM_ROWS)
+    if tiles >= MEDIUM_WIDE_TILES and rows > MEDIUM_WIDE_ROWS:
+        return rows <= MEDIUM_ROWS and weight.in_features >= MEDIUM_WIDE_REDUCTION and address % 16 == 0 and not kernels.library_tuning()
+    return rows <= MEDIUM_ROWS
 
 
 def takes_tiled(x: torch.Tensor, weight: "Weight", from_float: bool = False) -> bool:
@@ -124,7 +128,7 @@ def linear_clamped_glu(x: torch.Tensor, weight: "Weight", limit: float, slope: f
     if x.shape[0] > MEDIUM_ROWS and takes_tiled(x, weight, from_float=True):
         return kernels.gemm_tiled(x, weight.packed, weight.out_features, "clamped", limit=limit, slope=slope)
     # the packed copy's rows, and so its products' columns, hold gate and up by turns
-    by_turns = weight.gated and x.dtype == weight.dtype and takes_packed(weight, x.shape[0])
+    by_turns = weight.gated and x.dtype == weight.dtype and takes_packed(weight, x.shape[0], address=x.data_ptr())
     return kernels.clamped_glu(linear(x, weight, out_dtype=torch.float32), limit, slope, x.dtype, interleaved=by_turns)
 
 

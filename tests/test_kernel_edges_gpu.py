@@ -809,3 +809,19 @@ def test_activations_that_are_not_finite_stay_in_their_row(m, n, k, splits):
         total = whole.sum(0) if splits > 1 else whole
         assert float((total - x.float() @ w.float().T).abs().max()) < 2e-6 * k ** 0.5 + 1e-5      # k products of size 1 / sqrt(k)
         assert not got[..., 1, :].isfinite().any() if splits == 1 else not got.sum(0)[1].isfinite().any()
+
+
+@pytest.mark.parametrize("rows", [41, 64])
+def test_wide_products_of_41_to_64_rows_at_any_address(rows):
+    """A head's weight by the packed copy, and by the library where the rows begin at no 16-byte boundary: float32 sums of 512 products of size
+    1 / sqrt(512) in two orders."""
+    from microllm_rocm_amd.parts.linear import Weight, linear, takes_packed
+    generator = torch.Generator(device=DEVICE).manual_seed(rows)
+    n, k = 32768, 512
+    x, w = ((torch.randn(shape, generator=generator, device=DEVICE) * scale).to(torch.bfloat16) for shape, scale in (((rows, k), 1.0), ((n, k), k ** -0.5)))
+    weight = Weight(w)
+    apart = torch.empty(rows * k + 1, dtype=torch.bfloat16, device=DEVICE)[1:].view(rows, k)
+    apart.copy_(x)
+    assert takes_packed(weight, rows, address=x.data_ptr()) and not takes_packed(weight, rows, address=apart.data_ptr())
+    got, want = (linear(rows_, weight, out_dtype=torch.float32) for rows_ in (apart, x))
+    assert float((got - want).abs().max()) < 2e-5
