@@ -825,3 +825,26 @@ def test_wide_products_of_41_to_64_rows_at_any_address(rows):
     assert takes_packed(weight, rows, address=x.data_ptr()) and not takes_packed(weight, rows, address=apart.data_ptr())
     got, want = (linear(rows_, weight, out_dtype=torch.float32) for rows_ in (apart, x))
     assert float((got - want).abs().max()) < 2e-5
+
+
+@pytest.mark.parametrize("width", [4, 252, 896, 1028, 4096])
+@pytest.mark.parametrize("parts", [1, 2, 4, 8, 16])
+def test_norms_of_few_rows_have_the_bits_of_any_number_of_parts(width, parts):
+    """The kernel that asks for all parts at once against the one for any number, which parts of zeros lead to: the same additions."""
+    k, generator = kernels(), torch.Generator(device=DEVICE).manual_seed(width + parts)
+    draw = lambda *shape: torch.randn(shape, generator=generator, device=DEVICE)
+    h, weight, delta = draw(5, width), draw(width), draw(parts, 5, width)
+    more = torch.cat([delta, torch.zeros((1 if parts > 1 else 2, 5, width), device=DEVICE)])      # 3, 3, 5, 9 and 17
+    rows = torch.tensor([4, 0, 2], dtype=torch.int32, device=DEVICE)
+    for dtype in (torch.bfloat16, torch.float32):
+        for options in (dict(write_h=True), dict(rows=rows)):
+            streams, results = (h.clone(), h.clone()), []
+            for stream, given in zip(streams, (delta if parts > 1 else delta[0], more)):
+                results.append(k.rms_norm(stream, weight, 1e-6, dtype, delta=given, **options))
+            assert torch.equal(*results) and torch.equal(*streams)
+        alone = k.rms_norm(h, weight, 1e-6, dtype)
+        assert torch.equal(alone, k.rms_norm(h, weight, 1e-6, dtype, delta=torch.zeros((3, 5, width), device=DEVICE)))
+    v = h.double() + delta.double().sum(0)
+    want = v / torch.sqrt((v * v).mean(1, keepdim=True) + 1e-6) * weight.double()
+    got = k.rms_norm(h, weight, 1e-6, torch.float32, delta=delta if parts > 1 else delta[0])
+    assert float((got - want).norm() / want.norm()) < 4e-7 * parts ** 0.5      # parts + 1 additions of numbers rounded to 2^-24
