@@ -848,3 +848,24 @@ def test_norms_of_few_rows_have_the_bits_of_any_number_of_parts(width, parts):
     want = v / torch.sqrt((v * v).mean(1, keepdim=True) + 1e-6) * weight.double()
     got = k.rms_norm(h, weight, 1e-6, torch.float32, delta=delta if parts > 1 else delta[0])
     assert float((got - want).norm() / want.norm()) < 4e-7 * parts ** 0.5      # parts + 1 additions of numbers rounded to 2^-24
+
+
+@pytest.mark.parametrize("heads,kv_heads,hd,page_size", [(14, 2, 64, 16), (3, 1, 16, 32), (5, 5, 48, 16), (28, 4, 128, 16), (2, 0, 256, 16)])
+@pytest.mark.parametrize("parts,biased", [(1, True), (2, False), (4, True), (8, True), (16, True)])
+def test_queries_keys_and_values_in_pairs_have_the_bits_of_any_number_of_parts(heads, kv_heads, hd, page_size, parts, biased):
+    """Two pairs or four dims a thread against the kernel for any number of parts, which parts of zeros lead to; tokens without a place in a page among them."""
+    k, generator = kernels(), torch.Generator(device=DEVICE).manual_seed(heads + hd + parts)
+    tokens, total = 19, (heads + 2 * kv_heads) * hd
+    draw = lambda *shape: torch.randn(shape, generator=generator, device=DEVICE)
+    qkv, bias = draw(parts, tokens, total), draw(total) if biased else None
+    angle = draw(tokens, hd // 2)
+    cos_sin = torch.stack([angle.cos(), angle.sin()], dim=2).contiguous()
+    slots = (torch.randperm(3 * page_size, generator=generator, device=DEVICE)[:tokens]).to(torch.int32)
+    slots[[2, 11]] = -1
+    pos, results = torch.arange(tokens, device=DEVICE, dtype=torch.int32), []
+    for given in (qkv if parts > 1 else qkv[0], torch.cat([qkv, torch.zeros((1 if parts > 1 else 2, tokens, total), device=DEVICE)])):
+        pages = [torch.full(shape(3, max(kv_heads, 1), page_size, hd), 5.0, dtype=torch.bfloat16, device=DEVICE) for shape in (key_page_shape, value_page_shape)]
+        stored = (slots, None, *pages) if kv_heads else (None, None, None, None)
+        q = k.qkv_rope_store(given, bias, pos, *stored, heads, kv_heads, hd, page_size, torch.bfloat16, pair_order=True, cos_sin=cos_sin)
+        results.append([q, *pages])
+    assert all(torch.equal(a, b) for a, b in zip(*results))
