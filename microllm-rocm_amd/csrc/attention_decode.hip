@@ -374,45 +374,65 @@ __global__ __launch_bounds__(kDecodeThreads, HD_TILES <= 8 ? 2 : 1) void paged_a
 }
 
 // Joins the splits of one (token, head): out = sum_s w_s O_s / sum_s w_s l_s with w_s = exp(m_s - max m).
+constexpr int kJoinAtATime = 8;
+
 template <bool EXTRA>
 __global__ void paged_attention_join_kernel(const float* __restrict__ part_o, const float* __restrict__ part_ml,
                                             const int32_t* __restrict__ token_ids, bf16* __restrict__ out, int heads,
                                             int head_dim, int n_splits, MllAttentionExtras extras) {
     const int token = token_ids ? token_ids[blockIdx.x / heads] : blockIdx.x / heads;
-    if (token < 0) return;      // an entry that only pads the list to a fixed length
-    const int64_t row = static_cast<int64_t>(token) * heads + blockIdx.x % heads;
     const int64_t part_row = blockIdx.x;
-    // Eight splits at a time: their loads are asked for together, then used in the order of the splits.
+    // Eight splits at a time: their loads are asked for together, then used in the order of the splits. The first eight's results are asked for with
+    // their maxima and before the token's place is known (an entry that only pads the list has partial results of its own, unwritten ones), since
+    // the kernel's time is its waits for memory one after the other (attention and join, 28 heads of 128 over 4, 8 requests of 4096 in 8 splits 15.5 -> 14.9 us, one in 16 9.5 -> 9.0;
+    // 14 of 64 over 2, 32 of 700 in 4 7.2 -> 6.6, one of 1500 in 8 6.9 -> 6.3).
     const float2* ml = reinterpret_cast<const float2*>(part_ml) + part_row * n_splits;
-    float top = -INFINITY;
-    for (int base = 0; base < n_splits; base += 8) {
-        float2 pair[8];
-#pragma unroll
-        for (int j = 0; j < 8; ++j) pair[j] = ml[min(base + j, n_splits - 1)];
-#pragma unroll
-        for (int j = 0; j < 8; ++j) top = fmaxf(top, pair[j].x);
-    }
+    const float* o_row = part_o + part_row * n_splits * head_dim;
     const bool with_sink = EXTRA && extras.sink != nullptr;
     const float sink = with_sink ? extras.sink[blockIdx.x % heads] : 0.0f;
+    float2 first_pair[kJoinAtATime];
+    float first_part[kJoinAtATime];
+    const int first_dim = min(static_cast<int>(threadIdx.x), head_dim - 1);
+#pragma unroll
+    for (int j = 0; j < kJoinAtATime; ++j) first_pair[j] = ml[min(j, n_splits - 1)];
+#pragma unroll
+    for (int j = 0; j < kJoinAtATime; ++j) first_part[j] = o_row[min(j, n_splits - 1) * head_dim + first_dim];
+    if (token < 0) return;      // an entry that only pads the list to a fixed length
+    const int64_t row = static_cast<int64_t>(token) * heads + blockIdx.x % heads;
+    float top = -INFINITY;
+#pragma unroll
+    for (int j = 0; j < kJoinAtATime; ++j) top = fmaxf(top, first_pair[j].x);
+    for (int base = kJoinAtATime; base < n_splits; base += kJoinAtATime) {
+        float2 pair[kJoinAtATime];
+#pragma unroll
+        for (int j = 0; j < kJoinAtATime; ++j) pair[j] = ml[min(base + j, n_splits - 1)];
+#pragma unroll
+        for (int j = 0; j < kJoinAtATime; ++j) top = fmaxf(top, pair[j].x);
+    }
     if (with_sink) top = fmaxf(top, sink);
-    for (int dim = threadIdx.x; dim < head_dim; dim += blockDim.x) {
+    const int dim = threadIdx.x;        // a block has a thread a dim at least
+    if (dim < head_dim) {
         float total = 0.0f, weight_sum = 0.0f;
-        for (int base = 0; base < n_splits; base += 8) {
-            float2 pair[8];
-            float part[8];
+        const auto add = [&](int base, const float2 (&pair)[kJoinAtATime], const float (&part)[kJoinAtATime]) {
 #pragma unroll
-            for (int j = 0; j < 8; ++j) {
-                const int split = min(base + j, n_splits - 1);
-                pair[j] = ml[split];
-                part[j] = part_o[(part_row * n_splits + split) * head_dim + dim];
-            }
-#pragma unroll
-            for (int j = 0; j < 8; ++j) {
+            for (int j = 0; j < kJoinAtATime; ++j) {
                 if (base + j >= n_splits || pair[j].x == -INFINITY) continue;   // past the end, or a split without keys
                 const float weight = __expf(pair[j].x - top);
                 total += weight * part[j];
                 weight_sum += weight * pair[j].y;
             }
+        };
+        add(0, first_pair, first_part);
+        for (int base = kJoinAtATime; base < n_splits; base += kJoinAtATime) {
+            float2 pair[kJoinAtATime];
+            float part[kJoinAtATime];
+#pragma unroll
+            for (int j = 0; j < kJoinAtATime; ++j) {
+                const int split = min(base + j, n_splits - 1);
+                pair[j] = ml[split];
+                part[j] = o_row[static_cast<int64_t>(split) * head_dim + dim];
+            }
+            add(base, pair, part);
         }
         if (with_sink) weight_sum += __expf(sink - top);
         if (EXTRA) store_result(extras, out, token, (blockIdx.x % heads) * head_dim + dim, total / weight_sum * extras.out_scale * result_gate(extras, token, blockIdx.x % heads, head_dim, dim));

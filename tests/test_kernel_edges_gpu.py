@@ -869,3 +869,17 @@ def test_queries_keys_and_values_in_pairs_have_the_bits_of_any_number_of_parts(h
         q = k.qkv_rope_store(given, bias, pos, *stored, heads, kv_heads, hd, page_size, torch.bfloat16, pair_order=True, cos_sin=cos_sin)
         results.append([q, *pages])
     assert all(torch.equal(a, b) for a, b in zip(*results))
+
+
+@pytest.mark.parametrize("splits", [2, 8, 9, 17])
+def test_joined_splits_of_a_step_padded_to_a_fixed_length(splits):
+    """Eight splits are asked for before an entry's token is known, whatever it is: none of a padded list's other rows is written."""
+    rng, heads, kv_heads, hd = np.random.default_rng(splits), 6, 2, 80
+    lengths = [517, 1, 33, 960, 40, 7]
+    t, q_exact, ek, ev, seq, pos = build_paged_case(rng, torch.bfloat16, lengths, [1] * len(lengths), heads, kv_heads, hd, 16)
+    some = torch.tensor([3, -1, 0, -1, -1, 1], dtype=torch.int32, device=DEVICE)
+    out = torch.full_like(t["q"], 7.0)
+    kernels().paged_attention_decode(t["q"], t["k"], t["v"], t["table"], t["seq"], t["pos"], hd ** -0.5, 0, heads, kv_heads, hd, splits, out=out, token_ids=some)
+    want = reference_attention(q_exact, ek, ev, seq, pos, heads, kv_heads, hd, hd ** -0.5, 0)
+    np.testing.assert_allclose(out.float().cpu().numpy()[[0, 1, 3]], want[[0, 1, 3]], **tolerance(torch.bfloat16))
+    assert bool((out[[2, 4, 5]] == 7.0).all())
