@@ -493,7 +493,11 @@ __global__ void __launch_bounds__(kPairThreads) qkv_rope_store_pairs_kernel(
 
 // The same for float32 projections in the ordinary column order whose heads rotate whole (2 n_freq = head_dim, a
 // multiple of 8) with the step's table of cos and sin: a thread takes four pairs of a query or key head, or eight
-// dims of a value head, with 16-byte loads. out is bfloat16 or float32.
+// dims of a value head, with 16-byte loads. out is bfloat16 or float32. A wave takes eight items of eight tokens: in a page eight positions of eight dims of a
+// key, and of a dim of a value, lie side by side, so that tokens which follow each other fill whole lines from one place (an item after the
+// other over a token's heads: 2048 rows of 14 heads of 64 over 2 6.5 -> 4.6 us, of 28 of 128 over 4 16.3 -> 12.8, 16301 rows 135 -> 96, 300 4.2 -> 3.4).
+constexpr int kStoreThreads = 256, kStoreItems = kStoreThreads / 8;     // items of a token in a block
+
 template <typename T>
 __global__ void qkv_rope_store_vec4_kernel(const float* __restrict__ qkv, int n_partials, int64_t partial_stride,
                                            const float* __restrict__ bias, const int32_t* __restrict__ slot_mapping,
@@ -502,10 +506,11 @@ __global__ void qkv_rope_store_vec4_kernel(const float* __restrict__ qkv, int n_
                                            int kv_heads, int head_dim, int page_size) {
     const int groups = head_dim / 8;                       // items per head
     const int total_heads = heads + 2 * kv_heads;
-    const int64_t item = static_cast<int64_t>(blockIdx.x) * blockDim.x + threadIdx.x;
-    if (item >= static_cast<int64_t>(n_tokens) * total_heads * groups) return;
-    const int token = static_cast<int>(item / (total_heads * groups));
-    const int rest = static_cast<int>(item % (total_heads * groups));
+    const int runs = (total_heads * groups + kStoreItems - 1) / kStoreItems;      // blocks for eight tokens
+    const int token = static_cast<int>(blockIdx.x / runs) * 8 + threadIdx.x % kWave / 8;
+    const int rest = static_cast<int>(blockIdx.x % runs) * kStoreItems + threadIdx.x / kWave * 8 + threadIdx.x % 8;
+    if (token >= n_tokens || rest >= total_heads * groups) return;
+    const int slot = slot_mapping ? slot_mapping[token] : -1;
     const int head = rest / groups, group = rest % groups;
     const bool is_value = head >= heads + kv_heads;
     const int half = head_dim / 2;
@@ -542,7 +547,6 @@ __global__ void qkv_rope_store_vec4_kernel(const float* __restrict__ qkv, int n_
         store_four<T>(q_row + second, y2.x, y2.y, y2.z, y2.w);
         return;
     }
-    const int slot = slot_mapping ? slot_mapping[token] : -1;
     if (slot < 0) return;
     const CacheLayout layout(kv_heads, page_size, head_dim);
     const int64_t page = slot / page_size;
@@ -750,15 +754,15 @@ int mll_qkv_rope_store(const void* qkv, int in_dtype, int n_partials, int64_t pa
                       reinterpret_cast<uintptr_t>(cos_sin) % 16 == 0 && (bias == nullptr || reinterpret_cast<uintptr_t>(bias) % 16 == 0) &&
                       reinterpret_cast<uintptr_t>(q_out) % 16 == 0 && reinterpret_cast<uintptr_t>(k_cache) % 16 == 0;
     if (wide) {
-        const int64_t items = static_cast<int64_t>(n_tokens) * (heads + 2 * kv_heads) * (head_dim / 8);
-        const unsigned blocks = static_cast<unsigned>((items + 255) / 256);
+        const int64_t runs = ((heads + 2 * kv_heads) * (head_dim / 8) + kStoreItems - 1) / kStoreItems;
+        const unsigned blocks = static_cast<unsigned>((n_tokens + 7) / 8 * runs);
         if (dtype == kF32)
-            qkv_rope_store_vec4_kernel<float><<<blocks, 256, 0, stream>>>(
+            qkv_rope_store_vec4_kernel<float><<<blocks, kStoreThreads, 0, stream>>>(
                 static_cast<const float*>(qkv), n_partials, partial_stride, bias, slot_mapping, static_cast<const float2*>(cos_sin),
                 static_cast<float*>(q_out), static_cast<float*>(k_cache), static_cast<float*>(v_cache), n_tokens, heads, kv_heads,
                 head_dim, page_size);
         else
-            qkv_rope_store_vec4_kernel<bf16><<<blocks, 256, 0, stream>>>(
+            qkv_rope_store_vec4_kernel<bf16><<<blocks, kStoreThreads, 0, stream>>>(
                 static_cast<const float*>(qkv), n_partials, partial_stride, bias, slot_mapping, static_cast<const float2*>(cos_sin),
                 static_cast<bf16*>(q_out), static_cast<bf16*>(k_cache), static_cast<bf16*>(v_cache), n_tokens, heads, kv_heads,
                 head_dim, page_size);

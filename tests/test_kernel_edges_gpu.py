@@ -883,3 +883,29 @@ def test_joined_splits_of_a_step_padded_to_a_fixed_length(splits):
     want = reference_attention(q_exact, ek, ev, seq, pos, heads, kv_heads, hd, hd ** -0.5, 0)
     np.testing.assert_allclose(out.float().cpu().numpy()[[0, 1, 3]], want[[0, 1, 3]], **tolerance(torch.bfloat16))
     assert bool((out[[2, 4, 5]] == 7.0).all())
+
+
+@pytest.mark.parametrize("heads,kv_heads,hd,page_size,tokens", [(14, 2, 64, 16, 65), (3, 1, 16, 32, 72), (5, 5, 48, 16, 71), (28, 4, 128, 16, 130), (2, 0, 256, 16, 66), (2, 1, 80, 48, 200)])
+@pytest.mark.parametrize("parts,dtype", [(1, torch.bfloat16), (3, torch.bfloat16), (1, torch.float32)])
+def test_queries_keys_and_values_of_eight_tokens_a_wave_have_the_bits_of_a_block_a_token(heads, kv_heads, hd, page_size, tokens, parts, dtype):
+    """More than 64 tokens against the same tokens 64 at a time, which another kernel takes: tokens beyond the last eight, items beyond a block's, places in any order
+    and tokens without one."""
+    k, generator = kernels(), torch.Generator(device=DEVICE).manual_seed(heads + hd + tokens)
+    total, pages = (heads + 2 * kv_heads) * hd, -(-tokens // page_size) + 1
+    draw = lambda *shape: torch.randn(shape, generator=generator, device=DEVICE)
+    qkv, bias, angle = draw(parts, tokens, total), draw(total), draw(tokens, hd // 2)
+    cos_sin = torch.stack([angle.cos(), angle.sin()], dim=2).contiguous()
+    slots = torch.arange(tokens, device=DEVICE, dtype=torch.int32) + 3
+    slots[20:60] = slots[20:60].flip(0)
+    slots[[2, tokens - 1]] = -1
+    pos, results = torch.arange(tokens, device=DEVICE, dtype=torch.int32), []
+    for step in (tokens, 64):
+        stored = [torch.full(shape(pages, max(kv_heads, 1), page_size, hd), 5.0, dtype=dtype, device=DEVICE) for shape in (key_page_shape, value_page_shape)]
+        q = []
+        for first in range(0, tokens, step):
+            rows = slice(first, min(first + step, tokens))
+            given = qkv[:, rows].contiguous() if parts > 1 else qkv[0, rows]
+            places = (slots[rows], None, *stored) if kv_heads else (None, None, None, None)
+            q.append(k.qkv_rope_store(given, bias, pos[rows], *places, heads, kv_heads, hd, page_size, dtype, cos_sin=cos_sin[rows]))
+        results.append([torch.cat(q), *stored])
+    assert all(torch.equal(a, b) for a, b in zip(*results))
