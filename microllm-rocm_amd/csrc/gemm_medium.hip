@@ -35,6 +35,7 @@ constexpr int kMostTiles = 16;       // two a wave of 8
 constexpr unsigned kPast = 0x40000000;   // an offset past the end of every descriptor here
 constexpr int kMostSteps = static_cast<int>(kPast) / (kMostTiles * 1024);      // so that a workgroup's tiles end before it
 constexpr int kNonTemporal = 2;      // W is read once a step: past the caches
+constexpr int kArithmetic = 0xf;     // to sched_barrier: vector, scalar and matrix instructions
 
 union Piece {
     bf16x8 v;
@@ -117,6 +118,8 @@ __global__ __launch_bounds__(kWaves * kWave) void gemm_medium_kernel(
                 __builtin_amdgcn_raw_ptr_buffer_load_lds(a_rsrc, place, 16, at, 0, 0, 0);
             }
         }
+        // share_landed counts what was issued after the share: only arithmetic may pass from one side of this place to the other.
+        __builtin_amdgcn_sched_barrier(kArithmetic);
     };
     // The share that was asked for before the last `LATER` loads has landed, the wave's reads of the other buffer have arrived, and the workgroup meets.
     auto share_landed = [&]() __attribute__((always_inline)) {
