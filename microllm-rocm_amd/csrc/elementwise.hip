@@ -30,6 +30,36 @@ __global__ void embedding_kernel(const W* __restrict__ table, const int32_t* __r
     for (int column = threadIdx.x; column < width; column += blockDim.x) row_out[column] = to_float(row[column]) * scale;
 }
 
+// The same with four columns a thread, where the width and the addresses allow it: a step begins with this kernel, and a column a load makes a row of 3584
+// fourteen waits for memory, one behind the other (rows of 3584
+// in bfloat16, one 3.1 -> 2.1 us, 64 3.4 -> 2.3, 300 6.6 -> 3.1, 16301 110 -> 75; of 896 one 1.97 -> 2.05, 2048 4.3 -> 3.7, 16301 25 -> 19).
+template <typename W>
+__global__ void embedding_vec4_kernel(const W* __restrict__ table, const int32_t* __restrict__ ids, float* __restrict__ out, int width, int vocab,
+                                      float scale) {
+    struct alignas(4 * sizeof(W)) Four { W element[4]; };
+    const int token = blockIdx.x;
+    const int id = ids[token];
+    const bool known = id >= 0 && id < vocab;
+    const Four* row = reinterpret_cast<const Four*>(table + static_cast<int64_t>(known ? id : 0) * width);
+    float4* row_out = reinterpret_cast<float4*>(out + static_cast<int64_t>(token) * width);
+    for (int quad = threadIdx.x; quad < width / 4; quad += blockDim.x) {
+        const Four four = row[quad];
+        row_out[quad] = known ? make_float4(to_float(four.element[0]) * scale, to_float(four.element[1]) * scale, to_float(four.element[2]) * scale,
+                                            to_float(four.element[3]) * scale)
+                              : make_float4(NAN, NAN, NAN, NAN);
+    }
+}
+
+template <typename W>
+static void launch_embedding(const W* table, const int32_t* ids, float* out, int n_tokens, int width, int vocab, float scale, hipStream_t stream) {
+    if (width % 4 == 0 && reinterpret_cast<uintptr_t>(table) % (4 * sizeof(W)) == 0 && reinterpret_cast<uintptr_t>(out) % 16 == 0) {
+        const int threads = min(1024, (width / 4 + kWave - 1) / kWave * kWave);
+        embedding_vec4_kernel<W><<<n_tokens, threads, 0, stream>>>(table, ids, out, width, vocab, scale);
+    } else {
+        embedding_kernel<W><<<n_tokens, 256, 0, stream>>>(table, ids, out, width, vocab, scale);
+    }
+}
+
 // ---------------------------------------------------------------------------------------------
 // One block per output row. The sum of squares is taken in float32: per-thread strided partial
 // sums, a butterfly inside each wave, then the waves in ascending order.
@@ -647,9 +677,9 @@ int mll_embedding(const void* table, int table_dtype, const int32_t* ids, float*
     MLL_REQUIRE(n_tokens >= 0 && width > 0 && vocab > 0, "embedding: sizes must be positive");
     if (n_tokens == 0) return 0;
     if (table_dtype == kF32) {
-        embedding_kernel<float><<<n_tokens, 256, 0, stream>>>(static_cast<const float*>(table), ids, out, width, vocab, scale);
+        launch_embedding(static_cast<const float*>(table), ids, out, n_tokens, width, vocab, scale, stream);
     } else if (table_dtype == kBF16) {
-        embedding_kernel<bf16><<<n_tokens, 256, 0, stream>>>(static_cast<const bf16*>(table), ids, out, width, vocab, scale);
+        launch_embedding(static_cast<const bf16*>(table), ids, out, n_tokens, width, vocab, scale, stream);
     } else {
         return fail("embedding: unknown table dtype");
     }

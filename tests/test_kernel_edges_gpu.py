@@ -909,3 +909,15 @@ def test_queries_keys_and_values_of_eight_tokens_a_wave_have_the_bits_of_a_block
             q.append(k.qkv_rope_store(given, bias, pos[rows], *places, heads, kv_heads, hd, page_size, dtype, cos_sin=cos_sin[rows]))
         results.append([torch.cat(q), *stored])
     assert all(torch.equal(a, b) for a, b in zip(*results))
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("width,offset", [(4, 0), (252, 0), (3584, 0), (4100, 0), (896, 1), (1002, 0)])
+def test_embedding_rows_of_every_width_and_address(width, offset, dtype):
+    """Four columns a thread, in one round and in two, and the rows that begin at no whole four of them; ids outside the table."""
+    generator = torch.Generator(device=DEVICE).manual_seed(width)
+    flat = torch.randn(37 * width + offset, generator=generator, device=DEVICE).to(dtype)
+    table, ids = flat[offset:].view(37, width), torch.tensor([36, 0, -1, 5, 37, 5], dtype=torch.int32, device=DEVICE)
+    out = kernels().embedding(table, ids, scale=1.5)
+    known = [0, 1, 3, 5]
+    assert torch.equal(out[known], table[ids[known].long()].float() * 1.5) and bool(out[[2, 4]].isnan().all())
