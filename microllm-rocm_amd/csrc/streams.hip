@@ -21,6 +21,8 @@ inline int norm_threads(int width) { return width >= 2048 ? 1024 : (width >= 102
 // The same where a thread takes four columns at a time.
 inline int group_threads(int width) { return width >= 2048 ? 512 : (width >= 1024 ? 256 : (width > 256 ? 128 : 64)); }
 
+// A thread takes the two columns of an angle: bound by sine and cosine in float64, of which a column a thread makes every lane of a wave take both.
+// Rows of 2048: two 6.1 -> 2.8 us, 300 8.0 -> 4.4, 3117 33 -> 22; of 1024: two 3.8 -> 2.4, 3117 17.7 -> 11.3.
 template <typename T>
 __global__ void embedding_sinusoid_kernel(const T* __restrict__ table, const int32_t* __restrict__ ids,
                                           const int32_t* __restrict__ positions, const double* __restrict__ rates,
@@ -31,11 +33,14 @@ __global__ void embedding_sinusoid_kernel(const T* __restrict__ table, const int
     const double position = static_cast<double>(positions[token]);
     const T* row = table + static_cast<int64_t>(valid ? id : 0) * width;
     float* to = out + static_cast<int64_t>(token) * width;
-    for (int column = threadIdx.x; column < width; column += blockDim.x) {
+    for (int pair = threadIdx.x; 2 * pair < width; pair += blockDim.x) {
         // entry 2i: sin(p * rates[i]), entry 2i + 1: cos of the same angle; the angle in float64
-        const double angle = position * rates[column / 2];
-        const float wave = static_cast<float>((column & 1) ? cos(angle) : sin(angle));
-        to[column] = valid ? to_float(row[column]) + wave : __builtin_nanf("");
+        const int column = 2 * pair;
+        const bool both = column + 1 < width;
+        const float first = to_float(row[column]), second = to_float(row[both ? column + 1 : column]);
+        const double angle = position * rates[pair];
+        to[column] = valid ? first + static_cast<float>(sin(angle)) : __builtin_nanf("");
+        if (both) to[column + 1] = valid ? second + static_cast<float>(cos(angle)) : __builtin_nanf("");
     }
 }
 
@@ -246,11 +251,12 @@ int mll_embedding_sinusoid(const void* table, int table_dtype, const int32_t* id
                            const double* rates, float* out, int n_tokens, int width, int vocab, hipStream_t stream) {
     MLL_REQUIRE(n_tokens >= 0 && width > 0 && vocab > 0 && rates != nullptr, "embedding_sinusoid: sizes must be positive");
     if (n_tokens == 0) return 0;
+    const int threads = min(1024, ((width + 1) / 2 + kWave - 1) / kWave * kWave);
     if (table_dtype == kF32) {
-        embedding_sinusoid_kernel<float><<<n_tokens, 256, 0, stream>>>(static_cast<const float*>(table), ids, positions, rates,
+        embedding_sinusoid_kernel<float><<<n_tokens, threads, 0, stream>>>(static_cast<const float*>(table), ids, positions, rates,
                                                                       out, width, vocab);
     } else if (table_dtype == kBF16) {
-        embedding_sinusoid_kernel<bf16><<<n_tokens, 256, 0, stream>>>(static_cast<const bf16*>(table), ids, positions, rates,
+        embedding_sinusoid_kernel<bf16><<<n_tokens, threads, 0, stream>>>(static_cast<const bf16*>(table), ids, positions, rates,
                                                                      out, width, vocab);
     } else {
         return fail("embedding_sinusoid: unknown table dtype");

@@ -921,3 +921,18 @@ def test_embedding_rows_of_every_width_and_address(width, offset, dtype):
     out = kernels().embedding(table, ids, scale=1.5)
     known = [0, 1, 3, 5]
     assert torch.equal(out[known], table[ids[known].long()].float() * 1.5) and bool(out[[2, 4]].isnan().all())
+
+
+@pytest.mark.parametrize("width", [1, 2, 129, 2048, 2051])
+def test_position_waves_of_every_width(width):
+    """Two columns a thread: the last one alone, one round and two, ids outside the table. One rounding of the wave (2^-24 at most) and one of the sum."""
+    generator = torch.Generator(device=DEVICE).manual_seed(width)
+    table = torch.randn((11, width), generator=generator, device=DEVICE)
+    ids, pos = torch.tensor([10, 0, -1, 11, 3], dtype=torch.int32, device=DEVICE), torch.tensor([0, 1, 5, 7, 31999], dtype=torch.int32, device=DEVICE)
+    rates = 10000.0 ** (-torch.arange((width + 1) // 2, dtype=torch.float64, device=DEVICE) * 2 / width)
+    got = kernels().embedding_sinusoid(table, ids, pos, rates)
+    angle = (pos.double()[:, None] * rates).repeat_interleave(2, 1)[:, :width]
+    wave = torch.where(torch.arange(width, device=DEVICE) % 2 == 0, angle.sin(), angle.cos())
+    want = table[ids.clamp(0, 10).long()].double() + wave
+    assert bool(got[[2, 3]].isnan().all())
+    assert float((got - want)[[0, 1, 4]].abs().max()) <= 2 ** -24 * (1 + float(want.abs().max()))
