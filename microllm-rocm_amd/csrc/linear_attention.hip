@@ -339,6 +339,60 @@ gla_gate_kernel(const float* __restrict__ o, const float* __restrict__ proj, int
     }
 }
 
+// The same for heads of up to 64 CHUNKS values, which a wave holds: the gate and the weight are asked for with the row, not behind its sum, and a workgroup takes
+// blockDim.x / 64 rows (8 heads of 128: two tokens 2.47 -> 2.21 us, 3117 11.2 -> 8.8; 16 heads 21.0 -> 15.7; 4 of 64: two 2.11 -> 2.19, 3117 5.4 -> 4.6).
+constexpr int kGateWaves = 4, kGateRowsTogether = 2048;      // rows from which a workgroup takes several
+
+template <typename T, int CHUNKS>
+__global__ void __launch_bounds__(kGateWaves * kWave)
+gla_gate_held_kernel(const float* __restrict__ o, const float* __restrict__ proj, int64_t proj_stride, int gate_offset,
+                     const float* __restrict__ weight, float eps, T* __restrict__ out, int64_t out_stride, int rows, int heads,
+                     int value_dim, float out_scale) {
+    const int index = blockIdx.x * (blockDim.x / kWave) + __builtin_amdgcn_readfirstlane(threadIdx.x / kWave);
+    if (index >= rows) return;
+    const int token = index / heads, head = index % heads, lane = threadIdx.x % kWave;
+    const float* row = o + static_cast<int64_t>(index) * value_dim;
+    const float* gate = proj + static_cast<int64_t>(token) * proj_stride + gate_offset + head * value_dim;
+    float value[CHUNKS], g[CHUNKS], w[CHUNKS];
+#pragma unroll
+    for (int i = 0; i < CHUNKS; ++i) {
+        const int c = min(lane + i * kWave, value_dim - 1);
+        value[i] = row[c];
+        g[i] = gate[c];
+        w[i] = weight ? weight[c] : 1.0f;
+    }
+    float squares = 0.0f;
+#pragma unroll
+    for (int i = 0; i < CHUNKS; ++i)
+        if (lane + i * kWave < value_dim) squares += value[i] * value[i];
+    const float factor = 1.0f / sqrtf(wave_sum(squares) / static_cast<float>(value_dim) + eps);
+    T* to = out + static_cast<int64_t>(token) * out_stride + head * value_dim;
+#pragma unroll
+    for (int i = 0; i < CHUNKS; ++i) {
+        const int c = lane + i * kWave;
+        if (c >= value_dim) continue;
+        const float silu = g[i] / (1.0f + expf(-g[i]));
+        to[c] = from_float<T>((weight ? value[i] * factor * w[i] : value[i] * factor) * silu * out_scale);
+    }
+}
+
+template <typename T>
+static void launch_gla_gate(const float* o, const float* proj, int64_t proj_stride, int gate_offset, const float* weight, float eps, T* out,
+                            int64_t out_stride, int rows, int heads, int value_dim, float out_scale, hipStream_t stream) {
+    const int waves = rows >= kGateRowsTogether ? kGateWaves : 1;
+    const unsigned blocks = static_cast<unsigned>((static_cast<int64_t>(rows) + waves - 1) / waves);
+    const auto held = [&](auto chunks) {
+        gla_gate_held_kernel<T, decltype(chunks)::value><<<blocks, waves * kWave, 0, stream>>>(o, proj, proj_stride, gate_offset, weight, eps, out, out_stride,
+                                                                                              rows, heads, value_dim, out_scale);
+    };
+    if (value_dim <= kWave) held(std::integral_constant<int, 1>{});
+    else if (value_dim <= 2 * kWave) held(std::integral_constant<int, 2>{});
+    else if (value_dim <= 4 * kWave) held(std::integral_constant<int, 4>{});
+    else
+        gla_gate_kernel<T><<<static_cast<unsigned>(rows), kWave, 0, stream>>>(o, proj, proj_stride, gate_offset, weight, eps, out, out_stride, heads, value_dim,
+                                                                             out_scale);
+}
+
 }  // namespace mll
 
 using namespace mll;
@@ -426,11 +480,11 @@ int mll_gla_gate(const float* o, const float* proj, int64_t proj_stride, int gat
     const int64_t blocks = static_cast<int64_t>(n_tokens) * heads;
     MLL_REQUIRE(blocks < (1ll << 31), "gla_gate: too many rows for one launch");
     if (dtype == kF32) {
-        gla_gate_kernel<float><<<static_cast<unsigned>(blocks), kWave, 0, stream>>>(o, proj, proj_stride, gate_offset, weight, eps,
-                                                                                   static_cast<float*>(out), out_stride, heads, value_dim, out_scale);
+        launch_gla_gate(o, proj, proj_stride, gate_offset, weight, eps, static_cast<float*>(out), out_stride, static_cast<int>(blocks), heads, value_dim,
+                        out_scale, stream);
     } else if (dtype == kBF16) {
-        gla_gate_kernel<bf16><<<static_cast<unsigned>(blocks), kWave, 0, stream>>>(o, proj, proj_stride, gate_offset, weight, eps,
-                                                                                  static_cast<bf16*>(out), out_stride, heads, value_dim, out_scale);
+        launch_gla_gate(o, proj, proj_stride, gate_offset, weight, eps, static_cast<bf16*>(out), out_stride, static_cast<int>(blocks), heads, value_dim,
+                        out_scale, stream);
     } else {
         return fail("gla_gate: unknown dtype");
     }

@@ -936,3 +936,19 @@ def test_position_waves_of_every_width(width):
     want = table[ids.clamp(0, 10).long()].double() + wave
     assert bool(got[[2, 3]].isnan().all())
     assert float((got - want)[[0, 1, 4]].abs().max()) <= 2 ** -24 * (1 + float(want.abs().max()))
+
+
+@pytest.mark.parametrize("value_dim", [1, 63, 64, 65, 128, 200, 256, 257])
+@pytest.mark.parametrize("weighted", [False, True])
+def test_gated_heads_of_every_size(value_dim, weighted):
+    """One, two and four values a lane, and those a wave does not hold; a row a workgroup and four, the last of which have none, with the same bits."""
+    k, generator = kernels(), torch.Generator(device=DEVICE).manual_seed(value_dim)
+    heads, tokens, before = 3, 701, 5
+    draw = lambda *shape: torch.randn(shape, generator=generator, device=DEVICE)
+    o, proj, weight = draw(tokens, heads * value_dim), draw(tokens, before + heads * value_dim + 2), draw(value_dim) if weighted else None
+    run = lambda rows: k.gla_gate(o[:rows], proj[:rows], before, weight, 1e-5, heads, value_dim, 1.5, torch.float32)
+    got = run(tokens)
+    assert torch.equal(got[:7], run(7))
+    v, g = o.double().view(tokens, heads, value_dim), proj[:, before:before + heads * value_dim].double().view(tokens, heads, value_dim)
+    want = v / torch.sqrt((v * v).mean(2, keepdim=True) + 1e-5) * (weight.double() if weighted else 1.0) * g * torch.sigmoid(g) * 1.5
+    assert float((got.double().view_as(want) - want).norm() / want.norm()) < 1e-6      # some ten roundings of 2^-24
