@@ -319,9 +319,9 @@ __global__ __launch_bounds__(kSliceThreads) void sample_histogram_kernel(
     const int begin = min(static_cast<int>(blockIdx.y) * layout.slice, vocab);
     const int end = min(begin + layout.slice, vocab);
     float value[kLogitsAtOnce];
-    auto ask = [&](int base) {
+    auto ask = [&](int base) {      // (in unsigned numbers: what is asked for behind the end of a vocabulary near 2^31 is not below zero)
 #pragma unroll
-        for (int j = 0; j < kLogitsAtOnce; ++j) value[j] = row[min(base + j * kSliceThreads + static_cast<int>(threadIdx.x), vocab - 1)];
+        for (int j = 0; j < kLogitsAtOnce; ++j) value[j] = row[min(static_cast<unsigned>(base) + j * kSliceThreads + threadIdx.x, static_cast<unsigned>(vocab - 1))];
     };
     ask(begin);
     Counters counters[kRadixPasses - 1];
@@ -355,11 +355,11 @@ __global__ __launch_bounds__(kSliceThreads) void sample_histogram_kernel(
         }
         if ((todo >> lane) & 1ull) atomicAdd(&histogram[bin], 1);
     };
-    for (int base = begin; base < end; base += kLogitsAtOnce * kSliceThreads) {
-        if (base > begin) ask(base);
+    for (int done = 0; done < end - begin; done += kLogitsAtOnce * kSliceThreads) {
+        if (done > 0) ask(begin + done);
 #pragma unroll
         for (int j = 0; j < kLogitsAtOnce; ++j)
-            if (base + j * kSliceThreads < end) count_in(base + j * kSliceThreads + static_cast<int>(threadIdx.x), value[j]);
+            if (done + j * kSliceThreads < end - begin) count_in(begin + done + j * kSliceThreads + static_cast<int>(threadIdx.x), value[j]);
     }
     __syncthreads();
     for (int index = threadIdx.x; index < bins; index += kSliceThreads)

@@ -792,6 +792,18 @@ def test_tokens_of_vocabularies_up_to_and_beyond_what_a_thread_asks_for_at_once(
     assert k.argmax(logits)[4] == -1 and k.sample(logits, values[0], None, values[1])[4] == -1
 
 
+def test_the_best_tokens_of_the_longest_vocabulary():
+    """2^31 - 2048 logits (8.6 GB): what a thread asks for behind the last one lies beyond 2^31. Two thirds of the weight are the last token's."""
+    if torch.cuda.mem_get_info()[0] < 12 << 30:
+        pytest.skip("needs 12 GB")
+    vocab = 2 ** 31 - 2048
+    logits = torch.full((1, vocab), -3.0, device=DEVICE)
+    logits[0, vocab - 1], logits[0, 5] = math.log(2.0), 0.0
+    one = torch.ones(1, device=DEVICE)
+    chosen = [int(kernels().sample(logits, one, torch.full((1,), top, dtype=torch.int32, device=DEVICE), draw * one)) for top in (2, 1) for draw in (0.0, 0.3, 0.4, 0.99)]
+    assert chosen == [5, 5, vocab - 1, vocab - 1] + [vocab - 1] * 4
+
+
 @pytest.mark.parametrize("m", [17, 32, 33, 48, 49, 64])
 @pytest.mark.parametrize("n,k,splits", [(40, 8, 1), (300, 40, 1), (260, 264, 2), (1000, 1032, 3), (4112, 520, 1), (200, 2312, 4)])
 def test_activations_that_are_not_finite_stay_in_their_row(m, n, k, splits):
