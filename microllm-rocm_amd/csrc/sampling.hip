@@ -234,11 +234,15 @@ __global__ __launch_bounds__(kSliceThreads) void sample_slices_kernel(const floa
 // The row's maximum (first index) and whether any slice saw a non-finite value; every thread gets the same. A lane a slice: there are at most
 // 64, and the first maximum does not depend on the order in which they are compared.
 static_assert(kWave == 64, "a lane a slice");
+// Four words of the scratch in one load. The caller's scratch begins at any word, and so does what is read here.
+typedef int32_t Words __attribute__((ext_vector_type(4)));
+typedef Words WordsAnywhere __attribute__((aligned(4)));
+static_assert(alignof(WordsAnywhere) == 4, "the scratch is aligned to its words only");
 struct SlicePart {      // the lane's, asked for early
     ArgmaxPart part;
 };
 __device__ inline SlicePart ask_for_part(const int32_t* mine, const SampleLayout& layout, int lane) {
-    const int4 words = reinterpret_cast<const int4*>(mine + layout.parts)[min(lane, layout.slices - 1)];
+    const Words words = reinterpret_cast<const WordsAnywhere*>(mine + layout.parts)[min(lane, layout.slices - 1)];
     return SlicePart{ArgmaxPart{__int_as_float(words.x), words.y, words.z, words.w}};
 }
 __device__ inline Best row_best(const SlicePart& of_lane, bool* bad) {
@@ -259,9 +263,9 @@ struct Counters {
 };
 __device__ inline Counters ask_for_counters(const int32_t* histogram, int pass) {
     const int per = radix_bins(pass) / kSliceThreads;
-    const int4* words = reinterpret_cast<const int4*>(histogram + radix_bins(pass) - per * (static_cast<int>(threadIdx.x) + 1));
-    const int4 upper = words[per / 4 - 1];
-    int4 lower = make_int4(0, 0, 0, 0);
+    const WordsAnywhere* words = reinterpret_cast<const WordsAnywhere*>(histogram + radix_bins(pass) - per * (static_cast<int>(threadIdx.x) + 1));
+    const Words upper = words[per / 4 - 1];
+    Words lower = {0, 0, 0, 0};
     if (per == 8) lower = words[0];
     return Counters{{upper.w, upper.z, upper.y, upper.x, lower.w, lower.z, lower.y, lower.x}};
 }
@@ -462,8 +466,8 @@ __global__ __launch_bounds__(kWave) void sample_draw_kernel(
     // The pieces' sums in order: lane l holds pieces 4l .. 4l + 3. (What a row that is not drawn from left there is not used.)
     const int pieces = layout.slices * kSliceWaves;       // at most 256
     const int last_words = layout.slices - 1;             // four pieces to a slice
-    const int4 sum_words = reinterpret_cast<const int4*>(mine + layout.sums)[min(lane, last_words)];
-    const int4 equal_words = reinterpret_cast<const int4*>(mine + layout.equals)[min(lane, last_words)];
+    const Words sum_words = reinterpret_cast<const WordsAnywhere*>(mine + layout.sums)[min(lane, last_words)];
+    const Words equal_words = reinterpret_cast<const WordsAnywhere*>(mine + layout.equals)[min(lane, last_words)];
     const int select_key = mine[layout.select], select_equal = mine[layout.select + 1];
     const float row_uniform = uniform[row_index];
     bool bad;

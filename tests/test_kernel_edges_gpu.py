@@ -792,6 +792,19 @@ def test_tokens_of_vocabularies_up_to_and_beyond_what_a_thread_asks_for_at_once(
     assert k.argmax(logits)[4] == -1 and k.sample(logits, values[0], None, values[1])[4] == -1
 
 
+@pytest.mark.parametrize("words", [1, 2, 3])
+def test_the_scratch_of_a_draw_begins_at_any_word(words):
+    """It is promised four bytes of alignment, not the sixteen that a load of four words takes: the same tokens from every word on."""
+    k, lib, generator = kernels(), library.load(), torch.Generator(device=DEVICE).manual_seed(words)
+    rows, vocab = 7, 9001
+    logits, uniform = torch.randn((rows, vocab), generator=generator, device=DEVICE), torch.rand(rows, generator=generator, device=DEVICE)
+    temperature, top_k = torch.full((rows,), 0.9, device=DEVICE), torch.tensor([0, 1, 40, 3000, 0, 2, 9001], dtype=torch.int32, device=DEVICE)
+    scratch, out = torch.empty(lib.mll_sample_workspace(rows, vocab) // 4 + words, dtype=torch.int32, device=DEVICE), torch.empty(rows, dtype=torch.int32, device=DEVICE)
+    for restricted in (top_k, None):
+        k._check(lib.mll_sample(k._ptr(logits), k._ptr(temperature), k._ptr(restricted), k._ptr(uniform), k._ptr(out), k._ptr(scratch[words:]), rows, vocab, k._stream()), lib)
+        assert torch.equal(out, k.sample(logits, temperature, restricted, uniform))
+
+
 def test_the_best_tokens_of_the_longest_vocabulary():
     """2^31 - 2048 logits (8.6 GB): what a thread asks for behind the last one lies beyond 2^31. Two thirds of the weight are the last token's."""
     if torch.cuda.mem_get_info()[0] < 12 << 30:
