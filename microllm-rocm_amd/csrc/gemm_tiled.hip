@@ -96,7 +96,6 @@ __global__ __launch_bounds__(kTiledThreads, 1) void gemm_tiled_kernel(const bf16
     constexpr int kNowhere = 0x7fffffff;        // past what the descriptors hold
     __amdgpu_buffer_rsrc_t a_rsrc, w_rsrc;
     int a_offset[A_TURNS], w_offset[kWTurns / 2];    // of the lane's 16 bytes from the block's first row or tile, at stage 0, in bytes
-    const bool single = k_steps == 1;
     auto describe = [&](Place at) __attribute__((always_inline)) {
         const int m0 = at.m_block * TILE_M, n_tile0 = at.n_block * (kTileN / 16);
         a_rsrc = __builtin_amdgcn_make_buffer_rsrc(const_cast<bf16*>(a) + static_cast<int64_t>(m0) * k, 0, kNowhere, kBufferFlags);
@@ -105,8 +104,7 @@ __global__ __launch_bounds__(kTiledThreads, 1) void gemm_tiled_kernel(const bf16
             const int load = a_load(t);
             const int row_in_piece = 8 * (load % 2) + lane / 8;
             const int row = min((load / 2) * 16 + row_in_piece, m - 1 - m0);           // rows past the end repeat the last one
-            const int chunk = (lane % 8) ^ (row_in_piece / 2);
-            a_offset[t] = (row * k + (single ? chunk % 4 : chunk) * 8) * 2;
+            a_offset[t] = (row * k + ((lane % 8) ^ (row_in_piece / 2)) * 8) * 2;
         }
         w_rsrc = __builtin_amdgcn_make_buffer_rsrc(const_cast<bf16*>(w_packed) + static_cast<int64_t>(n_tile0) * k_steps * kPieceElements, 0, kNowhere,
                                                    kBufferFlags);
@@ -118,21 +116,27 @@ __global__ __launch_bounds__(kTiledThreads, 1) void gemm_tiled_kernel(const bf16
     const int stages_per_split = (all_stages + gridDim.y - 1) / gridDim.y;
     const int first_stage = blockIdx.y * stages_per_split;
     const int stages = min(all_stages, first_stage + stages_per_split);
-    // The last stage of an odd number of k steps is the last 64 of k, its first step with zeros for W (that step has been multiplied by the stage
-    // before; of a single step the second has zeros).
     auto copy_a = [&](int turn, int stage, unsigned slot) __attribute__((always_inline)) {
         // (arguments are worked out before the call: with a captured array's subscript in it the host pass drops the kernel's stub without a word)
         bf16* place = slots + slot * kSlotElements + a_load(turn) * 512;
-        const int at = a_offset[turn], from = max(0, min(stage * 128, (k_steps - 2) * 64));
-        __builtin_amdgcn_raw_ptr_buffer_load_lds(a_rsrc, place, 16, at, from, 0, 0);
+        const int at = a_offset[turn];
+        __builtin_amdgcn_raw_ptr_buffer_load_lds(a_rsrc, place, 16, at, stage * 128, 0, 0);
     };
     auto copy_w = [&](int turn, int stage, unsigned slot) __attribute__((always_inline)) {      // turn: which of the wave's two tiles and k steps
         const int p = turn / 2, h = turn % 2;
         bf16* place = slots + (kASlots + slot) * kSlotElements + (wave * (kWTurns / 2) + p) * 1024 + h * 512;
-        const bool last_alone = 2 * stage + 1 == k_steps;      // the stage has one step of its own
-        const int step = last_alone && !single ? k_steps - 1 : 2 * stage + h;
-        const int at = w_offset[p], from = last_alone && (h == 0) != single ? kNowhere : step * (kPieceElements * 2);
+        const int at = w_offset[p], from = 2 * stage + h < k_steps ? (2 * stage + h) * (kPieceElements * 2) : kNowhere;
         __builtin_amdgcn_raw_ptr_buffer_load_lds(w_rsrc, place, 16, at, from, 0, 0);
+    };
+    // The stage of an odd number's last k step has no second one: the lanes that would bring its half of a row of A ask past the descriptor's end from
+    // then on, as the loads of its pieces of W do, and get zeros. (Zeros on both sides: an infinity in a row's last elements times a zero would be no
+    // number.) Once a tile, by asm so that it stays a branch: a choice at every load is four vector instructions a stage (2048 x 37888 x 3584 gated 425 -> 431 us).
+    auto last_comes = [&]() __attribute__((always_inline)) {
+        if (2 * stages - 1 != k_steps) return;
+        const bool second_half = ((lane % 8) ^ (4 * (wave % 2) + lane / 16)) >= 4;      // the lane's chunk, the same in every load of the wave
+        const int past = second_half ? static_cast<int>(0x80000000u) : 0;
+#pragma unroll
+        for (int t = 0; t < A_TURNS; ++t) asm volatile("v_or_b32 %0, %0, %1" : "+v"(a_offset[t]) : "v"(past));
     };
     // Where the lane reads its operands: row `col` of a piece, chunk 4 step + quad at its place.
     const unsigned base = lds_address(slots);
@@ -148,7 +152,7 @@ __global__ __launch_bounds__(kTiledThreads, 1) void gemm_tiled_kernel(const bf16
     const bool any = EPILOGUE != 0 || first_stage < stages;      // a part of the reduction may be empty
     if (any) {
         describe(at);
-        begin_stages<A_TURNS>(first_stage, stages, copy_a, copy_w);
+        begin_stages<A_TURNS>(first_stage, stages, copy_a, copy_w, last_comes);
     }
     bool stored = false;      // whether the wave issued STORES stores after the tile's first loads
     for (;; at = next) {
@@ -157,11 +161,11 @@ __global__ __launch_bounds__(kTiledThreads, 1) void gemm_tiled_kernel(const bf16
         const int m0 = at.m_block * TILE_M, n_tile0 = at.n_block * (kTileN / 16), n_block = at.n_block;
         floatx4 acc[kWaveTilesN][WM];     // acc[nt][mt][i] = C[m = mt*16 + col][n = nt*16 + quad*4 + i] of the wave's part
         if (any) {
-            multiply_stages<kPackedStep, WM, A_TURNS, STORES>(acc, first_stage, stages, stored, a_step0, a_step1, w_lane, w_lane, copy_a, copy_w);
+            multiply_stages<kPackedStep, WM, A_TURNS, STORES>(acc, first_stage, stages, stored, a_step0, a_step1, w_lane, w_lane, copy_a, copy_w, last_comes);
             if (GATED || next.m_block >= 0) workgroup_meets();        // every wave is done with the slots
             if (next.m_block >= 0) {
                 describe(next);
-                begin_stages<A_TURNS>(first_stage, stages, copy_a, copy_w);
+                begin_stages<A_TURNS>(first_stage, stages, copy_a, copy_w, last_comes);
             }
         } else {
 #pragma unroll

@@ -143,8 +143,9 @@ __device__ __attribute__((always_inline)) inline void tile_products(bf16* slots,
     const unsigned a_at = base + wave_m * WM * 2048, w_at = base + kASlots * kSlotBytes + wave_n * kWaveTilesN * 2048;
 
     floatx4 acc[kWaveTilesN][WM];     // acc[nt][mt][i] = C[pair mt*16 + col][weight row nt*16 + quad*4 + i] of the wave's part
-    begin_stages<A_TURNS>(0, k / 64, copy_a, copy_w);
-    multiply_stages<0, WM, A_TURNS, 0>(acc, 0, k / 64, false, a_at + step0, a_at + step1, w_at + step0, w_at + step1, copy_a, copy_w);
+    const auto last_comes = [] {};      // reductions are whole stages
+    begin_stages<A_TURNS>(0, k / 64, copy_a, copy_w, last_comes);
+    multiply_stages<0, WM, A_TURNS, 0>(acc, 0, k / 64, false, a_at + step0, a_at + step1, w_at + step0, w_at + step1, copy_a, copy_w, last_comes);
 
     if constexpr (GATED) {
         workgroup_meets();

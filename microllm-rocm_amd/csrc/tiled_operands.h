@@ -92,14 +92,17 @@ __device__ __attribute__((always_inline)) inline void operands_arrived(TiledOper
 }
 
 // The loads of a tile's first two stages, from `first` to before `stages`, go out: copy_a(turn, stage, slot) and copy_w(turn, stage, slot) issue one of a
-// wave's A_TURNS and kWTurns loads of a stage, every wave all of them. The slots are free: the workgroup has met since they were read.
-template <int A_TURNS, typename CopyA, typename CopyW>
-__device__ __attribute__((always_inline)) inline void begin_stages(int first, int stages, const CopyA& copy_a, const CopyW& copy_w) {
+// wave's A_TURNS and kWTurns loads of a stage, every wave all of them. The slots are free: the workgroup has met since they were read. last_comes() is
+// called once, before the loads of the last stage go out.
+template <int A_TURNS, typename CopyA, typename CopyW, typename LastComes>
+__device__ __attribute__((always_inline)) inline void begin_stages(int first, int stages, const CopyA& copy_a, const CopyW& copy_w, const LastComes& last_comes) {
+    if (first + 1 == stages) last_comes();
 #pragma unroll
     for (int t = 0; t < A_TURNS; ++t) copy_a(t, first, 0);
 #pragma unroll
     for (int t = 0; t < kWTurns; ++t) copy_w(t, first, 0);
     if (first + 1 < stages) {
+        if (first + 2 == stages) last_comes();
 #pragma unroll
         for (int t = 0; t < A_TURNS; ++t) copy_a(t, first + 1, 1);
 #pragma unroll
@@ -114,10 +117,10 @@ __device__ __attribute__((always_inline)) inline void begin_stages(int first, in
 // stage nothing is copied, and what is read then is multiplied by nobody.
 // STORES: how many stores to memory the wave has issued since begin_stages, at least, if `stored`: loads and stores are counted together as they
 // were issued, and a wait that names the stores lets them go on while the first stages are multiplied.
-template <int W_STEP, int WM, int A_TURNS, int STORES, typename CopyA, typename CopyW>
+template <int W_STEP, int WM, int A_TURNS, int STORES, typename CopyA, typename CopyW, typename LastComes>
 __device__ __attribute__((always_inline)) inline void multiply_stages(floatx4 (&acc)[kWaveTilesN][WM], int first, int stages, bool stored, unsigned a_step0,
                                                                       unsigned a_step1, unsigned w_step0, unsigned w_step1, const CopyA& copy_a,
-                                                                      const CopyW& copy_w) {
+                                                                      const CopyW& copy_w, const LastComes& last_comes) {
     constexpr std::make_integer_sequence<int, WM> row_tiles{};
     constexpr int kStage = A_TURNS + kWTurns, kMostCounted = 63;
     constexpr int kStageAndStores = kStage + STORES < kMostCounted ? kStage + STORES : kMostCounted;
@@ -158,9 +161,15 @@ __device__ __attribute__((always_inline)) inline void multiply_stages(floatx4 (&
         w_now = w_next, w_next = w_after, w_after = w;
     };
     int stage = first;
-    if (STORES > 0 && stored && stage + 2 < stages) multiply_stage(stage++, std::true_type{}, std::integral_constant<int, kTurnsAndStores>{});
+    if (STORES > 0 && stored && stage + 2 < stages) {
+        if (stage + 3 == stages) last_comes();
+        multiply_stage(stage++, std::true_type{}, std::integral_constant<int, kTurnsAndStores>{});
+    }
 #pragma clang loop unroll(disable)
-    for (; stage + 2 < stages; ++stage) multiply_stage(stage, std::true_type{}, std::integral_constant<int, kWTurns>{});
+    for (; stage + 2 < stages; ++stage) {
+        if (stage + 3 == stages) last_comes();
+        multiply_stage(stage, std::true_type{}, std::integral_constant<int, kWTurns>{});
+    }
 #pragma clang loop unroll(disable)
     for (; stage < stages; ++stage) multiply_stage(stage, std::false_type{}, std::integral_constant<int, 0>{});
     // No load is on its way into LDS now and no read into registers; the last products must have written their results before these are read (the

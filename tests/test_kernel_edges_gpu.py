@@ -506,6 +506,29 @@ def test_tiles_whose_loads_go_out_before_the_tile_before_is_stored(m, n, k):
     assert float((ka.gemm_tiled(x, packed, n, "f32") - x.float() @ w.float().T).abs().max()) < 1e-5 * k ** 0.5 + 1e-4      # sums of at most 352 products of size 1 / sqrt(k)
 
 
+@pytest.mark.parametrize("k", [32, 64, 96, 160, 352])
+@pytest.mark.parametrize("tile_rows", [128, 160, 256])
+def test_infinities_at_the_end_of_a_reduction_stay_infinities(k, tile_rows):
+    """A stage takes two steps of 32: one that has only one multiplies nothing by the zeros of the other. One infinity in a row is that of its sign and the
+    weight's in every column, other rows keep their bits."""
+    ka, generator = kernels(), torch.Generator(device=DEVICE).manual_seed(k)
+    m, n = 300, 520
+    x, w = (torch.randn(shape, generator=generator, device=DEVICE).to(torch.bfloat16) for shape in ((m, k), (n, k)))
+    w = torch.where(w == 0, torch.ones_like(w), w)
+    packed, spoilt = ka.pack_weight(w), x.clone()
+    places = {row: place for row, place in ((1, k - 1), (2, k - 32), (130, k - 33), (4, k - 64), (5, 0), (m - 1, k - 1)) if place >= 0}
+    for row, place in places.items():
+        spoilt[row, place] = math.inf if row % 2 else -math.inf
+    kept = torch.tensor([row for row in range(m) if row not in places], device=DEVICE)
+    for epilogue, splits in (("f32", 1), ("bf16", 1), ("f32", 2)):
+        options = dict(epilogue=epilogue, splits=splits, tile_rows=tile_rows)
+        whole, got = (ka.gemm_tiled(rows, packed, n, **options) for rows in (x, spoilt))
+        assert torch.equal(got[..., kept, :], whole[..., kept, :])
+        total = got.sum(0) if splits > 1 else got.float()
+        for row, place in places.items():
+            assert torch.equal(total[row], w[:, place].float().sign() * float(spoilt[row, place])), (epilogue, splits, row)
+
+
 @pytest.mark.parametrize("heads,kv_heads,hd,window", [(14, 2, 64, 0), (4, 2, 48, 100), (4, 1, 128, 0), (2, 1, 256, 33)])
 def test_prompts_in_tiles_of_half_the_queries_have_the_same_bits(heads, kv_heads, hd, window):
     """Tiles of 64 queries, whose second one in a workgroup goes to the waves from the last on, against tiles of 128."""
