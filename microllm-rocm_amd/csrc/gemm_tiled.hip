@@ -56,7 +56,7 @@ __global__ __launch_bounds__(kTiledThreads, 1) void gemm_tiled_kernel(const bf16
     // Two slots of A, each [2 WM pieces of 16 rows][row][8 places of 16 bytes], the row's chunk c of 8 elements at place c ^ (row / 2); then three of W, each
     // [16 tiles][2 k steps][1 KB in MFMA operand order]. While stages are multiplied the direct loads alone write this memory and the asm reads alone read
     // it. Gated results pass through the last slot as rows, while the next tile's first two stages are on their way into the others.
-    __shared__ __align__(16) bf16 slots[kStageElements];
+    __shared__ __align__(kSlotsAlign) bf16 slots[kStageElements];
 
     const int lane = threadIdx.x % kWave;
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave);

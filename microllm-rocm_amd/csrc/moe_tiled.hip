@@ -218,7 +218,7 @@ __global__ __launch_bounds__(kTiledThreads, 1) void moe_tiled_kernel(const bf16*
                                                                      const float* __restrict__ weights, int n_out, int k, void* __restrict__ out,
                                                                      int top, int n_tokens, int weight_on_input, int from_tokens,
                                                                      const bf16* __restrict__ x, MllExpertForm form) {
-    __shared__ __align__(16) bf16 slots[kStageElements];
+    __shared__ __align__(kSlotsAlign) bf16 slots[kStageElements];
     constexpr int kOutputsATile = FORM == 1 ? kTileCols / 2 : kTileCols;
     const int lane = threadIdx.x % kWave;
     const int n_blocks = (n_out + kOutputsATile - 1) / kOutputsATile;

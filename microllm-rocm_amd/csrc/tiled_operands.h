@@ -192,6 +192,9 @@ __device__ __attribute__((always_inline)) inline void workgroup_meets() {
 constexpr int kResultColumns = 128;      // of a tile
 constexpr int kResultRows = 64;          // of a wave at a time, 16 a store
 constexpr int kResultBytes = 64;         // of a wave's row
+// The kernels exchange a row's chunks in the LDS address itself, whose lower bits must be the place in the row's alone wherever the compiler puts the slots.
+constexpr int kSlotsAlign = 128;
+static_assert(kSlotsAlign % kResultBytes == 0 && kSlotBytes % kResultBytes == 0, "a wave's rows of results begin at multiples of their length");
 template <int OFFSET> __device__ __attribute__((always_inline)) inline void put_result(unsigned address, unsigned word) {
     asm volatile("ds_write_b32 %0, %1 offset:%2" ::"v"(address), "v"(word), "n"(OFFSET) : "memory");
 }
