@@ -1258,18 +1258,18 @@ def tiled_gated_pays(rows: int, k: int, from_float: bool = False, n: int = TILED
     those over this one's), from 256 rows on:
 
     k up to 1024 from ``rows * n`` of 3700 k on: 512 x 512 at 1024, 3072 and 4096 rows 0.78, 0.99 and 1.07; 2816 x 1024 at 512, 1024, 1536 and 4096
-    0.76, 0.91, 1.06 and 1.51; 9728 x 896 at 192, 512, 2048 and 4096 0.91, 1.24, 1.39 and 1.21. Up to 2048 from 3000 k on: 1408 x 2048 at 1024
-    and 3072 0.61 and 0.91; 4096 x 2048 at 1024, 1536 and 2048 0.86, 1.02 and 1.13; 16384 x 2048 at 256, 512, 1024, 2048, 3072 and 4096 0.95,
-    1.10, 1.12, 1.01, 0.96 and 0.96 (at 3072, 4096, 8192 and 16384 with the loads between the products 1.10, 1.13, 1.11 and 1.11). Longer reductions: the library's rate jumps with the shape, this one's only where the last round of
-    workgroups leaves units idle; from 3584 to 6144 where they are nine tenths filled: 37888 x 3584 at 1280, 1536 (0.87 filled), 2048 and 3072
-    1.32, 0.92, 1.15 and 1.10; 22016 x 4096 at 1024 (0.67), 1536, 2048 and 2560 (0.84) 0.85, 1.35, 1.48 and 0.94; but 17920 x 2560 at 1536, 2560, 3072
-    and 3584 0.92, 1.39, 0.85 and 0.92, 59136 x 8192 at 1024 to 4096 0.88 to 0.99, 8192 x 8192 0.85 to 0.99. Above 3072 rows timed alone the
-    tiled kernel is faster there by now (37888 x 3584 at 4096, 8192 and 16384 1.07, 1.12 and 1.05), but a pass of 16301 tokens runs at the power cap
-    and takes 75.4 ms with it and 74.0 with the library. 9728 x 896 at 4096, 8192 and 16384 1.47, 1.48 and 1.44.
+    0.76, 0.91, 1.06 and 1.51; 9728 x 896 at 192, 512, 2048 and 4096 0.91, 1.24, 1.39 and 1.21, at 8192 and 16384 1.48 and 1.44. Up to 2048 from
+    3000 k on: 1408 x 2048 at 1024 and 3072 0.61 and 0.91; 4096 x 2048 at 1024, 1536 and 2048 0.86, 1.02 and 1.13; 16384 x 2048 at 256, 512, 1024, 2048, 3072
+    and 4096 0.95, 1.10, 1.12, 1.01, 0.96 and 0.96 (at 3072, 4096, 8192 and 16384 with the loads between the products 1.10, 1.13, 1.11 and 1.11).
+
+    Longer reductions, up to 6144 (``_tiled_gated_pays_in_long_reductions``): the library's rate jumps with the shape, this one's only where the last round
+    of workgroups leaves units idle. Beyond, 28672 x 7168 0.93 to 1.12, 59136 x 8192 0.94 to 1.09: the library's.
 
     Where the activation takes the float32 sums (``from_float``: clamped gates), the library's way writes and reads twice as much and has no
     upper line: 16384 x 2048 at 256, 512, 3584 and 8192 rows 0.97, 1.15, 1.22 and 1.30; 4096 x 2048 at 1024, 1536 and 8192 0.90, 1.05 and 1.18; 37888 x 3584
     at 768, 1024, 3072 and 8192 1.07, 1.12, 1.24 and 1.22; 4096 x 4096 at 1024, 1536 and 2048 0.77, 0.96 and 1.10; 59136 x 8192 at 1024 to 6144 0.97 to 1.07.
+    From 8192 columns on those of longer reductions are also the tiled kernel's where the rounded ones are (six weights from 8192 x 2304 to 37888 x 3584
+    at 256 to 896 rows: the gain is that of the rounded ones within 0.1, but for 320 and 384 rows of 8192 x 2304, which neither takes).
 
     A tuned library is 3 to 8 % faster than the tiled kernel where it matters most and keeps the product. Steps are padded to
     multiples of 64 rows, above 1024 of 256: the line is drawn at the padded number, so that both are on one side of it."""
@@ -1280,29 +1280,34 @@ def tiled_gated_pays(rows: int, k: int, from_float: bool = False, n: int = TILED
     if rows < 256:
         return False
     work = rows * n
-    if from_float:
-        return work >= 3500 * k if k <= 1024 else work >= 2800 * k if k <= 2048 else rows > 960 and work >= 1650 * k
     if k <= 1024:
-        return work >= 3700 * k
+        return work >= (3500 if from_float else 3700) * k
     if k <= 2048:
-        return work >= 3000 * k
-    return 3584 <= k <= 6144 and 960 < rows <= 3072 and _tiled_fill_of(rows, n) >= 0.9
+        return work >= (2800 if from_float else 3000) * k
+    if from_float and rows > 960 and work >= 1650 * k:
+        return True
+    return k <= 6144 and (n >= 8192 or not from_float) and _tiled_gated_pays_in_long_reductions(rows, k, n)
 
 
-def tiled_gated_pays_in_long_reductions(rows: int, k: int, n: int) -> bool:
-    """The same for reductions of more than 2048 and up to 6144 since the tiled kernel's loads go through descriptors and a workgroup's next tile is
-    on its way while one is stored: it is the faster one wherever its tiles fill three quarters of their rounds, and up to 768 rows, where the
-    library's tiles fill no more, always (14 weights from 13824 x 2304 to 32768 x 6144 at 19 numbers of rows from 256 to 8192, library and activation over
-    this kernel: 1.12 on the mean, 0.96 at the least; 37888 x 3584 at 384, 768, 1024, 2048, 4096, 8192 and 16384 rows 1.16, 1.04, 1.30, 1.34, 1.06, 1.11
-    and 1.06; 27648 x 5120 at 512 to 8192 1.10 to 1.29). Left out: 14336 x 4096 at 2560 rows (0.73 filled) 0.97, 13824 x 5120 at 320 and 1792 (0.63, 0.74) 0.96 and
-    0.95, 37888 x 3584 at 256 (0.58) 0.88; beyond, 28672 x 7168 0.93 to 1.12, 59136 x 8192 0.94 to 1.09. A tuned library keeps the product."""
-    if library_tuning() or k % 32 != 0 or not 2048 < k <= 6144:
-        return False
-    multiple = 64 if rows <= 1024 else 256
-    rows = -(-rows // multiple) * multiple
-    if rows < 256 or n < 8192:      # fewer columns were not measured
-        return False
-    return 384 <= rows <= 768 or _tiled_fill_of(rows, n) >= (0.8 if rows < 384 else 0.76)
+def _tiled_gated_pays_in_long_reductions(rows: int, k: int, n: int) -> bool:
+    """For 2048 < k <= 6144 and a padded number of rows, where the tiles fill their rounds (the library and the activation over the tiled kernel):
+
+    From 8192 columns on where three quarters are filled, 0.8 below 384 rows (25 weights from 8192 x 2304 to 13824 x 6144 at 16 numbers of rows from 256 to
+    4096: 1.15 on the mean of the 280 sizes it takes, 0.98 at the least; 14 from 13824 x 2304 to 32768 x 6144 at 19 from 256 to 8192 1.12 and
+    0.96; 37888 x 3584 at 1024, 2048, 4096, 8192 and 16384 rows 1.30, 1.34, 1.06, 1.11 and 1.06). From 384 to
+    768 rows, where the library's tiles fill no more, from 13824 columns on always (1.01 at the least; 37888 x 3584 at 384 1.16) and below where 0.65 are
+    filled: 8192 x 4096 at 384, 512, 640 and 704 (0.38, 0.50, 0.62 and 0.75 filled) 0.78, 0.87, 0.95 and 1.06, 9728 x 4096 at 384, 512 and 576 (0.45, 0.59 and 0.74) 0.86,
+    1.00 and 1.02, 11008 x 6144 at 384 and 448 (0.50 and 0.67) 0.97 and 1.05. Left out: 14336 x 4096 at 2560 rows (0.73) 0.97, 13824 x 5120 at 320 and
+    1792 (0.63 and 0.74) 0.96 and 0.95, 37888 x 3584 at 256 (0.58) 0.88.
+
+    Fewer columns: from 3584 and from 1024 to 3072 rows where nine tenths are filled (4096 to 7680 columns at 3584 to 6144, 68 sizes: 1.12 on the mean,
+    0.98 at the least); others were not measured."""
+    fill = _tiled_fill_of(rows, n)
+    if n < 8192:
+        return k >= 3584 and 960 < rows <= 3072 and fill >= 0.9
+    if 384 <= rows <= 768:
+        return n >= 13824 or fill >= 0.65
+    return fill >= (0.8 if rows < 384 else 0.76)
 
 
 def gemm_tiled(x: torch.Tensor, packed: torch.Tensor, n: int, epilogue: str = "f32", splits: int = 1,

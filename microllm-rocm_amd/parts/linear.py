@@ -112,11 +112,10 @@ def takes_packed(weight: "Weight", rows: int, gated: bool = False, address: int 
 
 def takes_tiled(x: torch.Tensor, weight: "Weight", from_float: bool = False) -> bool:
     """Whether a gated product of these rows is the tiled kernel's, although the weight is also kept as stored: where
-    ``kernels.tiled_gated_pays`` or ``tiled_gated_pays_in_long_reductions`` and the rows, as many as a tile has at least, lie at a 16-byte boundary, as its loads need (the
+    ``kernels.tiled_gated_pays`` and the rows, as many as a tile has at least, lie at a 16-byte boundary, as its loads need (the
     library takes any)."""
     return (x.dtype == torch.bfloat16 and weight.packed is not None and weight.gated and x.data_ptr() % 16 == 0
-            and (kernels.tiled_gated_pays(x.shape[0], weight.in_features, from_float, weight.out_features)
-                 or kernels.tiled_gated_pays_in_long_reductions(x.shape[0], weight.in_features, weight.out_features)))
+            and kernels.tiled_gated_pays(x.shape[0], weight.in_features, from_float, weight.out_features))
 
 
 def linear_clamped_glu(x: torch.Tensor, weight: "Weight", limit: float, slope: float) -> torch.Tensor:
