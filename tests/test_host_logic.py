@@ -106,7 +106,7 @@ def test_parts_take_their_tensors_out_of_the_dict_as_they_bind():
         assert set(untouched) == names
 
 
-def test_which_product_a_linear_takes():
+def test_which_product_a_linear_takes(monkeypatch):
     plain = Weight(torch.zeros((64, 32), dtype=torch.bfloat16))          # on the host nothing is packed
     assert plain.packed is None and not takes_packed(plain, 1) and not takes_unscaled(plain, 1)
     packed = Weight(torch.zeros((64, 32), dtype=torch.bfloat16), pack=False)
@@ -119,7 +119,17 @@ def test_which_product_a_linear_takes():
     assert takes_packed(packed, 5000) and takes_packed(packed, 40, gated=True)
     wide = Weight(torch.zeros((16, 8), dtype=torch.bfloat16), pack=False)
     wide.packed, wide.out_features = packed.packed, 2048 * 16
-    assert takes_packed(wide, 40) and not takes_packed(wide, 41), "weights with many tiles go to the library from 41 rows on"
+    assert takes_packed(wide, 40) and not takes_packed(wide, 41), "many tiles and a short reduction: the library's from 41 rows on"
+    for reduction, taken in ((504, False), (512, True)):                    # the head of a model
+        head = Weight(torch.zeros((16, reduction), dtype=torch.bfloat16), pack=False)
+        head.packed, head.out_features = packed.packed, 2048 * 16
+        assert takes_packed(head, 40, address=2) and takes_packed(head, 41) == takes_packed(head, 64) == taken and not takes_packed(head, 65)
+        assert not takes_packed(head, 41, address=2), "rows at no 16-byte boundary are the library's"
+        monkeypatch.setattr(kernels, "library_tuning", lambda: True)
+        assert takes_packed(head, 40) and not takes_packed(head, 41), "and so are those of a tuned one"
+        monkeypatch.undo()
+        head.out_features -= 16                                              # a tile fewer
+        assert takes_packed(head, 64, address=2)
 
 
 def test_percentile_interpolates_between_the_two_nearest_sorted_values():

@@ -1000,3 +1000,28 @@ def test_gated_heads_of_every_size(value_dim, weighted):
     v, g = o.double().view(tokens, heads, value_dim), proj[:, before:before + heads * value_dim].double().view(tokens, heads, value_dim)
     want = v / torch.sqrt((v * v).mean(2, keepdim=True) + 1e-5) * (weight.double() if weighted else 1.0) * g * torch.sigmoid(g) * 1.5
     assert float((got.double().view_as(want) - want).norm() / want.norm()) < 1e-6      # some ten roundings of 2^-24
+
+
+@pytest.mark.parametrize("dtype", [np.float32, np.int64])
+def test_uploads_hold_what_was_given_while_the_device_is_busy(dtype):
+    """The host goes on, writes over its array and gives the pinned copies back before the device has read any: a hundred uploads of some sizes behind 50 ms and
+    more of other work, from arrays in any order of their dims."""
+    from microllm_rocm_amd.ops.transfers import on_device_later
+    target = torch.device(DEVICE)
+    shapes = [(3, 97), (1,), (2, 0), (5, 4)]
+    for busy in (False, True):      # the first round makes the pinned memory, which may wait
+        torch.cuda.synchronize()
+        done, got = torch.cuda.Event(), []
+        if busy:
+            torch.cuda._sleep(100_000_000)
+        done.record()
+        for number in range(100):
+            rows, columns = (shapes[number % 4] + (1,))[:2]
+            array = np.empty((columns, rows), dtype=dtype).T
+            array[...] = number + np.arange(rows * columns).reshape(rows, columns) / 1
+            got.append(on_device_later(array, target))
+            array[...] = -1
+        assert not busy or not done.query()
+        for number, tensor in enumerate(got):
+            rows, columns = (shapes[number % 4] + (1,))[:2]
+            assert tensor.device.type == "cuda" and tensor.cpu().tolist() == (number + np.arange(rows * columns).reshape(rows, columns)).tolist()
