@@ -31,8 +31,9 @@ __global__ void embedding_kernel(const W* __restrict__ table, const int32_t* __r
 }
 
 // The same with four columns a thread, where the width and the addresses allow it: a step begins with this kernel, and a column a load makes a row of 3584
-// fourteen waits for memory, one behind the other (rows of 3584
-// in bfloat16, one 3.1 -> 2.1 us, 64 3.4 -> 2.3, 300 6.6 -> 3.1, 16301 110 -> 75; of 896 one 1.97 -> 2.05, 2048 4.3 -> 3.7, 16301 25 -> 19).
+// fourteen waits for memory, one behind the other (rows of 3584 in bfloat16, launch after launch, one 2.88 -> 1.86 us, 64 3.20 -> 2.10, 300 3.80 -> 2.59, 16301
+// 110 -> 75). Rows that a block of 256 reads in a few columns a thread gain nothing in steps of few tokens and lose nothing: of 896 one 1.86 both ways, 64
+// 2.05 and 2.08 (runs differ by that), 300 2.19 -> 2.11, 2048 3.52 -> 3.20; of 256 one 1.87 both ways, 2048 2.51 -> 2.34.
 template <typename W>
 __global__ void embedding_vec4_kernel(const W* __restrict__ table, const int32_t* __restrict__ ids, float* __restrict__ out, int width, int vocab,
                                       float scale) {
@@ -233,7 +234,8 @@ __global__ void rms_norm_vec4_kernel(float* __restrict__ h, const D* __restrict_
 // the weight and the delta's PARTS parts (0: no delta) are all asked for before the first is used, without a branch between them; threads past
 // the row ask for its last four again. The same additions in the same order. Against the kernel above, which has the weight behind the block's sum and a branch
 // before every part (MI355X, launch after launch): 32 rows of 896 in 16 parts 3.00 -> 2.46 us, in 4 2.76 -> 2.17, 64 of 3584 in 16 5.90 -> 5.22, 32 of
-// 2048 in 8 3.04 -> 2.65, 500 of 3584 7.25 -> 5.68; without a delta one row of 3584 2.07 -> 1.97, of 896 1.88 -> 1.92.
+// 2048 in 8 3.04 -> 2.65, 500 of 3584 7.25 -> 5.68; without a delta the same within 0.03 us up to 64 rows (one row of 896 1.89 both ways, of 3584 2.05 and
+// 2.08), 300 of 3584 3.41 -> 3.06, 2048 of 896 3.42 -> 3.19.
 template <typename T, typename D, int PARTS>
 __global__ void rms_norm_row_kernel(float* __restrict__ h, const D* __restrict__ delta, int64_t partial_stride,
                                     const int32_t* __restrict__ rows, const float* __restrict__ weight,

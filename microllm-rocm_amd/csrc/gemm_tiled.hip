@@ -19,7 +19,9 @@
 // while a tile's results are made and stored. Gated, before and after, 1.03 to 1.05 times as fast: 8192 x 37888 x 3584 1633 -> 1575 us (1.41 PFLOP/s), 16301 rows
 // 3230 -> 3109, 2048 rows 439 -> 418, 8192 x 16384 x 2048 425 -> 404, 3584 rows 199 -> 189, 2048 x 9728 x 896 37.0 -> 35.2; float32, 2048 x 3584 x 18944 in two
 // parts 225 -> 210. Four waves of 128 x 128, accumulators in the other half of the registers: the stages 5 % faster still, a tile's start and
-// end, with nothing beside a wave that waits, 2 us longer (2048 x 9728 x 896 39.0).
+// end, with nothing beside a wave that waits, 2 us longer (2048 x 9728 x 896 39.0). Two tiles at a time are more than the scalar registers hold: 16 to 30 of
+// them wait in lanes of a vector register in the gated forms, 38 to 42 in that of queries, keys and values, 0 to 4 in the others; three are read back in the
+// block of a tile's first stage, the others between tiles, none in the loop of the stages.
 // Workgroups are numbered so that the 32 that run together on one of the 8 XCDs (each with a second-level cache of
 // its own) own about 4 x 8 neighbouring tiles of C, and so share their rows of A and of W there, and so that every
 // XCD gets the same number of tiles.
@@ -354,9 +356,12 @@ static int launch_tiled_rows(const void* a, const void* w_packed, void* out, int
     return check_launch("gemm_tiled");
 }
 
-// How many rows a workgroup's tile gets: the height that is done first, if every round of 256 workgroups takes as
-// long as a tile's loads (a stage of A and W: rows + 256 columns), which is what bounds this kernel. 2048 x 4608
-// in tiles of 256 rows is 144 tiles, a round in which 112 compute units have none; in tiles of 160 rows 234.
+// How many rows a workgroup's tile gets: the height that is done first, if every round of 256 workgroups takes a time of rows + 256. 2048 x 4608
+// in tiles of 256 rows is 144 tiles, a round in which 112 compute units have none; in tiles of 160 rows 234. The model is that of a stage's loads, which
+// bounded this kernel when it was drawn; the products that bound it now would say rows plus less. It is kept because what it chooses was measured again and
+// because the rules of who takes a product (how full its rounds are) are drawn by it: over 8 weights from 1152 x 896 to 37888 x 3584 and 16 numbers of rows
+// from 128 to 8192 its height takes 1.005 times the best one's time on the mean gated, 1.003 in float32, and in 8 of the 128 sizes 1.04 to 1.10 times (2560 x 9728 x
+// 896, 1792 x 13824 x 4096, 8192 x 4608 x 3584); rows + 64 would be within 1.02 everywhere.
 // Every output's additions are the same whatever the height.
 static int choose_tile_rows(int m, int n, int splits) {
     const int n_blocks = (n + kTileN - 1) / kTileN;

@@ -340,7 +340,8 @@ gla_gate_kernel(const float* __restrict__ o, const float* __restrict__ proj, int
 }
 
 // The same for heads of up to 64 CHUNKS values, which a wave holds: the gate and the weight are asked for with the row, not behind its sum, and a workgroup takes
-// blockDim.x / 64 rows (8 heads of 128: two tokens 2.47 -> 2.21 us, 3117 11.2 -> 8.8; 16 heads 21.0 -> 15.7; 4 of 64: two 2.11 -> 2.19, 3117 5.4 -> 4.6).
+// blockDim.x / 64 rows (launch after launch: 8 heads of 128, two tokens 2.37 -> 2.03 us, 3117 11.9 -> 8.3; 16 heads 20.2 -> 15.3; 8 of 256 19.3 -> 13.0; 4 of 64,
+// two 2.03 -> 1.91, 3117 5.1 -> 4.4; 4 of 32, two 2.03 -> 1.93. Of a pass with two prompts and eight tokens each, 5.6 ms, that is 25 us: less than its runs differ by).
 constexpr int kGateWaves = 4, kGateRowsTogether = 2048;      // rows from which a workgroup takes several
 
 template <typename T, int CHUNKS>

@@ -23,8 +23,9 @@ LIBRARY_NAME = "libmicrollm_hip.so"
 ARCH = "gfx950"
 # Packed float32 instructions are switched off for every kernel of this library. Kernel arguments come in registers, as many of the first ones
 # as there are user registers for: a wave then asks for its data at once, where it would wait for a read of its arguments first. Against
-# reads (MI355X): generation and mixed steps of a 0.5B model, thousands of launches of 4 to 8 us, 1.8 to 2.1 % faster, a float32 decode step 1.2 %, no
-# step slower; where the arguments' use comes late anyway (streaming products at 8 requests and fewer) 0.0 to 0.4 %.
+# reads (MI355X): generation and mixed steps of a 0.5B model, thousands of launches of 3 to 7 us, 2.9 and 1.5 % faster, a float32 decode step 1.2 %, the other
+# passes 0.0 to 0.9 %, none slower. A loop over one short kernel shows the other side, since it finds its arguments in the caches: the embedding of one
+# row 1.72 -> 1.87 us a launch.
 HIPCC_FLAGS = ["-O3", "-std=c++17", "-fPIC", f"--offload-arch={ARCH}",
                "-Xclang", "-target-feature", "-Xclang", "-packed-fp32-ops",
                "-mllvm", "-amdgpu-kernarg-preload-count=16",
